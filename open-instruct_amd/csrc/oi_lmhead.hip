@@ -39,31 +39,32 @@ static_assert(256 * STAGE_STRIDE <= LDS_ELEMS, "the dZ staging tile must fit");
 typedef f32x16 AccTile[2][4];
 
 // XCD-aware tile order.  Consecutive workgroup ids go round-robin to the 8 XCDs, each with its own
-// L2; the 32 workgroups resident on one XCD form an 8 (m) x 4 (n) super-tile so that they share
-// operand slabs in that L2.  The 8 XCDs take super-tiles that are neighbours along n and the sweep
-// over n completes before m advances: the chip as a whole then works on one slab of A (the larger
-// operand: lm_head rows, dZ rows) at a time, which stays in the memory-side cache while every n
-// tile passes over it, instead of streaming all of A from HBM once per n super-tile.  Measured:
-// +4 to +7 % on every shape of the lm_head path (the kernel runs at the chip's power limit, and
-// HBM traffic costs power).
-__device__ __forceinline__ bool tile_of_pid(int64_t pid, int64_t tiles_m, int64_t tiles_n, int64_t* tm, int64_t* tn) {
-    const int64_t xcd = pid & 7, local = pid >> 3;
-    const int64_t nsn = (tiles_n + 3) / 4;
-    const int64_t st = (local >> 5) * 8 + xcd, inner = local & 31;
-    *tm = (st / nsn) * 8 + (inner & 7);
-    *tn = (st % nsn) * 4 + (inner >> 3);
-    return *tm < tiles_m && *tn < tiles_n;
+// L2.  The tiles of a launch are numbered in bands of 8 rows, n outermost inside a band, so that 32
+// consecutive numbers are an 8 (m) x 4 (n) super-tile (wider where there are fewer than 8 rows); the ids
+// of an XCD come in runs of 32 such numbers, which its 32 workgroups share operand slabs of in that L2,
+// and the 8 XCDs take neighbouring runs along n.  The sweep over n completes before m advances: the chip
+// as a whole then works on one slab of A (the larger operand: lm_head rows, dZ rows) at a time, which
+// stays in the memory-side cache while every n tile passes over it, instead of streaming all of A from
+// HBM once per n super-tile.  Measured: +4 to +7 % on every shape of the lm_head path (the kernel runs at
+// the chip's power limit, and HBM traffic costs power).  Every number is a tile, whatever the counts.
+__device__ __forceinline__ uint32_t item_of_pid(uint32_t pid) {
+    const uint32_t xcd = pid & 7, local = pid >> 3;
+    return ((local >> 5) * 8 + xcd) * 32 + (local & 31);
 }
-// number of ids to enumerate (whole super-tiles, a multiple of 256)
-__host__ __device__ inline int64_t pids_for_tiles(int64_t tiles_m, int64_t tiles_n) {
-    const int64_t nst = ((tiles_m + 7) / 8) * ((tiles_n + 3) / 4);
-    return ((nst + 7) / 8) * 8 * 32;
+__device__ __forceinline__ void tile_of_item(uint32_t item, uint32_t tiles_m, uint32_t tiles_n, int64_t* tm, int64_t* tn) {
+    const uint32_t band = item / (8 * tiles_n), in_band = item - band * 8 * tiles_n;
+    const uint32_t left = tiles_m - band * 8, rows = left < 8 ? left : 8;
+    const uint32_t col = in_band / rows;
+    *tm = band * 8 + (in_band - col * rows);
+    *tn = col;
 }
+// number of ids to enumerate (whole runs for every XCD, a multiple of 256)
+__host__ __device__ inline int64_t pids_for_items(int64_t items) { return (items + 255) / 256 * 256; }
 
 // Work queue.  A launch of the tile kernels is one workgroup per CU (the LDS ring leaves room for
 // no second one) that stays for the whole launch and draws tile ids from a counter, rather than
 // one short-lived workgroup per tile.  There is one counter per XCD (workgroup b is taken to run
-// on XCD b mod 8, as the tile order assumes), so the ids an XCD draws are the ones tile_of_pid
+// on XCD b mod 8, as the tile order assumes), so the ids an XCD draws are the ones item_of_pid
 // maps onto shared operand slabs; a wrong guess costs cache hits, never correctness.  The XCDs do
 // not finish their shares together (measured on the forward: 1.7 ms apart in an 18 ms launch), so
 // a workgroup whose own queue has run dry goes on with the queues of the other XCDs, one after the
@@ -82,10 +83,9 @@ __device__ __forceinline__ int opaque_tid() {
     return t;
 }
 template <class Body>
-__device__ __forceinline__ void for_each_tile(uint32_t* __restrict__ counters, int64_t tiles_m, int64_t tiles_n,
-                                              uint16_t* lds, Body&& body) {
+__device__ __forceinline__ void for_each_item(uint32_t* __restrict__ counters, uint32_t items, uint16_t* lds, Body&& body) {
     const uint32_t xcd = blockIdx.x & 7;
-    const uint32_t locals = (uint32_t)(pids_for_tiles(tiles_m, tiles_n) >> 3);  // ids per queue
+    const uint32_t locals = (uint32_t)(pids_for_items(items) >> 3);  // ids per queue
     // the word sits in the fifth ring slot, which the main loop first writes after its first barrier
     volatile uint32_t* mailbox = reinterpret_cast<volatile uint32_t*>(lds + 4 * BM * BK);
     constexpr uint32_t NONE = 0xffffffffu;
@@ -111,20 +111,32 @@ __device__ __forceinline__ void for_each_tile(uint32_t* __restrict__ counters, i
     while (pid != NONE) {
         // in flight while the tile is computed
         if (threadIdx.x == 0 && dry < 8) drawn = atomicAdd(&counters[(xcd + dry) & 7], 1u);
-        int64_t tm, tn;
-        if (tile_of_pid((int64_t)pid, tiles_m, tiles_n, &tm, &tn)) body(tm, tn);
+        const uint32_t item = item_of_pid(pid);
+        if (item < items) body(item);
         __syncthreads();  // the tile's last use of the LDS is over
         if (threadIdx.x == 0) *mailbox = dry < 8 ? resolve() : NONE;
         __syncthreads();
         pid = __builtin_amdgcn_readfirstlane(*mailbox);
     }
 }
+template <class Body>
+__device__ __forceinline__ void for_each_tile(uint32_t* __restrict__ counters, int64_t tiles_m, int64_t tiles_n,
+                                              uint16_t* lds, Body&& body) {
+    for_each_item(counters, (uint32_t)(tiles_m * tiles_n), lds, [&](uint32_t item) {
+        int64_t tm, tn;
+        tile_of_item(item, (uint32_t)tiles_m, (uint32_t)tiles_n, &tm, &tn);
+        body(tm, tn);
+    });
+}
 // fallback used by the stand-alone GEMM entry point, which has no workspace for a counter: one
 // workgroup per tile id
 __device__ __forceinline__ bool tile_of_block(int64_t tiles_m, int64_t tiles_n, int64_t* tm, int64_t* tn) {
-    return tile_of_pid(blockIdx.x, tiles_m, tiles_n, tm, tn);
+    const uint32_t item = item_of_pid(blockIdx.x);
+    if (item >= tiles_m * tiles_n) return false;
+    tile_of_item(item, (uint32_t)tiles_m, (uint32_t)tiles_n, tm, tn);
+    return true;
 }
-inline unsigned grid_for_tiles(int64_t tiles_m, int64_t tiles_n) { return (unsigned)pids_for_tiles(tiles_m, tiles_n); }
+inline unsigned grid_for_tiles(int64_t tiles_m, int64_t tiles_n) { return (unsigned)pids_for_items(tiles_m * tiles_n); }
 
 // LDS tile layout: row r of an operand tile holds its 64 k-values as eight 16-byte chunks; chunk c
 // is stored at position c ^ swz(r).  With that permutation the 16-byte fragment reads of 16
@@ -873,20 +885,140 @@ __device__ __forceinline__ void quad_transpose(float (&v)[4], int lane) {
     v[3] = b1 ? t3 : rb;
 }
 
+// Where a tile product goes.
 // mode 0: out_f32  = acc          mode 1: out_f32 += acc
 // mode 2: out_bf16 = acc          mode 3: out_bf16 = out_f32 + acc   (last chunk of d_hidden)
 // mode 4: out_bf16 += acc         (rows added to a d_weight that was already rounded)
-// A, B: operands without their tile origin (r0 is filled in here); the product has M x N
-// entries, of which rows below m_valid are stored.  K == 0 stores zeros.  With `out_rows`, row r
-// of a bf16 result goes to row out_rows[r] of out_bf16 (the fp32 accumulator stays compact).
+// Rows below m_valid and columns below N are stored.  With `out_rows`, row r of a bf16 result goes to row
+// out_rows[r] of out_bf16 (the fp32 accumulator stays compact).  scale_a / scale_b: factors of row r, see
+// DynRows.
+struct StoreTo {
+    int mode;
+    float* out_f32;
+    uint16_t* out_bf16;
+    int64_t ldo, N, m_valid;
+    const int32_t* out_rows;
+    const float *scale_a, *scale_b;
+};
+// 16-byte pieces (8 bytes of bf16) need whole groups of four columns
+__device__ __forceinline__ bool stores_in_pieces(const StoreTo& st) {
+    return ((st.N | st.ldo) & 3) == 0 && (reinterpret_cast<uintptr_t>(st.out_f32) & 15) == 0 &&
+           (reinterpret_cast<uintptr_t>(st.out_bf16) & 7) == 0;
+}
+// the four rows (one per group of 8) of a 32-row block that a lane stores pieces of
+struct LaneRows {
+    int64_t row[4], dst[4];
+    bool ok[4];
+    float sa[4], sb[4];
+};
+__device__ __forceinline__ LaneRows lane_rows(const StoreTo& st, int64_t row0, int lane) {
+    LaneRows r;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        r.row[q] = row0 + q * 8 + (lane >> 5) * 4 + (lane & 3);
+        r.ok[q] = r.row[q] < st.m_valid;
+        r.dst[q] = (r.ok[q] && st.out_rows) ? (int64_t)st.out_rows[r.row[q]] : r.row[q];
+        r.sa[q] = (r.ok[q] && st.scale_a) ? st.scale_a[r.row[q]] : 1.f;
+        r.sb[q] = (r.ok[q] && st.scale_a) ? st.scale_b[r.row[q]] : 1.f;
+    }
+    return r;
+}
+// Stores a 32-row x 64-column block whose entry (jj, q, e) of a lane is row q * 8 + (lane / 32) * 4 + e,
+// column jj * 32 + lane % 32 (the layout the MFMA leaves).  Every store and load as a 16-byte piece
+// (8 bytes of bf16): after a 4 x 4 transpose inside each quad of lanes a lane holds four consecutive
+// columns of one row.  A quarter of the memory instructions of the one-value-per-lane form, whose
+// address processing is what an epilogue of 128 values per lane waits for.  The fp32 sum of the
+// accumulating modes is requested before the transposes and added with plain loads and stores: every
+// element has one writer per launch and the launches follow each other on the stream, so no atomic is
+// needed.  32 registers of sums in flight.
+template <class Get>
+__device__ __forceinline__ void store_block(const StoreTo& st, const LaneRows& r, int64_t col0, int lane, Get&& get) {
+    const int mode = st.mode, g = (lane & 31) >> 2;
+    oi_f32x4 part[2][4];
+    uint2 part16[2][4];
+    if (mode == 1 || mode == 3) {
+#pragma unroll
+        for (int jj = 0; jj < 2; ++jj)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const int64_t col = col0 + jj * 32 + 4 * g;
+                part[jj][q] = (r.ok[q] && col < st.N)
+                                  ? *reinterpret_cast<const oi_f32x4*>(st.out_f32 + r.row[q] * st.ldo + col)
+                                  : oi_f32x4{0.f, 0.f, 0.f, 0.f};
+            }
+    } else if (mode == 4) {
+#pragma unroll
+        for (int jj = 0; jj < 2; ++jj)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const int64_t col = col0 + jj * 32 + 4 * g;
+                part16[jj][q] = (r.ok[q] && col < st.N)
+                                    ? *reinterpret_cast<const uint2*>(st.out_bf16 + r.dst[q] * st.ldo + col)
+                                    : make_uint2(0u, 0u);
+            }
+    }
+#pragma unroll
+    for (int jj = 0; jj < 2; ++jj) {
+        const int64_t col = col0 + jj * 32 + 4 * g;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            float v[4] = {get(jj, q, 0), get(jj, q, 1), get(jj, q, 2), get(jj, q, 3)};
+            quad_transpose(v, lane);
+            if (!r.ok[q] || col >= st.N) continue;
+            if (st.scale_a) {
+                // a row whose factor is exactly 0 is 0 whatever its sum holds (the sums of
+                // rows that were taken out may have left the fp32 range)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) v[e] = r.sb[q] == 0.f ? 0.f : v[e] * r.sa[q] * r.sb[q];
+            }
+            if (mode == 1 || mode == 3) {
+                v[0] += part[jj][q].x;
+                v[1] += part[jj][q].y;
+                v[2] += part[jj][q].z;
+                v[3] += part[jj][q].w;
+            } else if (mode == 4) {
+                v[0] += oi_bf16lo_to_f32(part16[jj][q].x);
+                v[1] += oi_bf16hi_to_f32(part16[jj][q].x);
+                v[2] += oi_bf16lo_to_f32(part16[jj][q].y);
+                v[3] += oi_bf16hi_to_f32(part16[jj][q].y);
+            }
+            if (mode <= 1)
+                *reinterpret_cast<oi_f32x4*>(st.out_f32 + r.row[q] * st.ldo + col) = oi_f32x4{v[0], v[1], v[2], v[3]};
+            else
+                *reinterpret_cast<uint2*>(st.out_bf16 + r.dst[q] * st.ldo + col) =
+                    make_uint2(oi_pack_bf16x2(v[0], v[1]), oi_pack_bf16x2(v[2], v[3]));
+        }
+    }
+}
+
+// A piece of a tile product that is one of several along k: the fp32 tile in the order in which the
+// accumulators lie in the registers (16 bytes per lane, consecutive lanes together).
+constexpr int PART_FLOATS = BM * BN;
+__device__ __forceinline__ void store_part(const AccTile& acc, float* part, int tid) {
+    asm volatile("" : "+v"(tid));
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+                *reinterpret_cast<oi_f32x4*>(part + (((i * 4 + j) * 4 + q) * NTHREADS + tid) * 4) =
+                    oi_f32x4{acc[i][j][q * 4], acc[i][j][q * 4 + 1], acc[i][j][q * 4 + 2], acc[i][j][q * 4 + 3]};
+}
+
+// A, B: operands without their tile origin (r0 is filled in here).  K == 0 stores zeros.  With `part`
+// the fp32 tile goes there and nowhere else.
 template <bool A_KM, bool B_KM>
-__device__ __forceinline__ void gemm_store_tile(Operand A, int64_t M, Operand B, int64_t N, int64_t K, int mode,
-                                                float* out_f32, uint16_t* out_bf16, int64_t ldo, int64_t m_valid,
-                                                const int32_t* __restrict__ out_rows,
-                                                const float* __restrict__ scale_a, const float* __restrict__ scale_b,
-                                                int64_t tm, int64_t tn, uint16_t* lds) {
+__device__ __forceinline__ void gemm_store_tile(Operand A, Operand B, int64_t K, const StoreTo& st, int64_t tm,
+                                                int64_t tn, float* part, uint16_t* lds) {
     const int tid = opaque_tid(), lane = tid & 63, wave = tid >> 6, wm = wave & 3, wn = wave >> 2;
     const int64_t m0 = tm * BM, n0 = tn * BN;
+    const int mode = st.mode;
+    float* out_f32 = st.out_f32;
+    uint16_t* out_bf16 = st.out_bf16;
+    const int64_t ldo = st.ldo, m_valid = st.m_valid, N = st.N;
+    const int32_t* out_rows = st.out_rows;
+    const float *scale_a = st.scale_a, *scale_b = st.scale_b;
     A.r0 = m0;
     B.r0 = n0;
     AccTile acc;
@@ -901,89 +1033,18 @@ __device__ __forceinline__ void gemm_store_tile(Operand A, int64_t M, Operand B,
 #pragma unroll
                 for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
     }
-    if (((N | ldo) & 3) == 0 && (reinterpret_cast<uintptr_t>(out_f32) & 15) == 0 &&
-        (reinterpret_cast<uintptr_t>(out_bf16) & 7) == 0) {
-        // Every store and load of the epilogue as a 16-byte piece (8 bytes of bf16): after a 4 x 4
-        // transpose inside each quad of lanes a lane holds four consecutive columns of one row.  A
-        // quarter of the memory instructions of the one-value-per-lane form, whose address
-        // processing is what an epilogue of 128 values per lane waits for.  The fp32 sum of the
-        // accumulating modes is requested before the transposes of the half tile it belongs to and
-        // added with plain loads and stores: every element has one writer per launch and the
-        // launches follow each other on the stream, so no atomic is needed.
-        const int kq = lane & 3, g = (lane & 31) >> 2, hl = lane >> 5;
+    if (part) {
+        store_part(acc, part, tid);
+        return;
+    }
+    if (stores_in_pieces(st)) {
 #pragma unroll
         for (int i = 0; i < 2; ++i) {
-            int64_t row[4], dst[4];
-            bool ok[4];
-            float sa[4], sb[4];
+            const LaneRows r = lane_rows(st, m0 + wm * 64 + i * 32, lane);
 #pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                row[q] = m0 + wm * 64 + i * 32 + q * 8 + hl * 4 + kq;
-                ok[q] = row[q] < m_valid;
-                dst[q] = (ok[q] && out_rows) ? (int64_t)out_rows[row[q]] : row[q];
-                sa[q] = (ok[q] && scale_a) ? scale_a[row[q]] : 1.f;
-                sb[q] = (ok[q] && scale_a) ? scale_b[row[q]] : 1.f;
-            }
-            // two of the four 32-column blocks at a time: 32 registers of sums in flight
-#pragma unroll
-            for (int jh = 0; jh < 2; ++jh) {
-                oi_f32x4 part[2][4];
-                uint2 part16[2][4];
-                if (mode == 1 || mode == 3) {
-#pragma unroll
-                    for (int jj = 0; jj < 2; ++jj)
-#pragma unroll
-                        for (int q = 0; q < 4; ++q) {
-                            const int64_t col = n0 + wn * 128 + (2 * jh + jj) * 32 + 4 * g;
-                            part[jj][q] = (ok[q] && col < N)
-                                              ? *reinterpret_cast<const oi_f32x4*>(out_f32 + row[q] * ldo + col)
-                                              : oi_f32x4{0.f, 0.f, 0.f, 0.f};
-                        }
-                } else if (mode == 4) {
-#pragma unroll
-                    for (int jj = 0; jj < 2; ++jj)
-#pragma unroll
-                        for (int q = 0; q < 4; ++q) {
-                            const int64_t col = n0 + wn * 128 + (2 * jh + jj) * 32 + 4 * g;
-                            part16[jj][q] = (ok[q] && col < N)
-                                                ? *reinterpret_cast<const uint2*>(out_bf16 + dst[q] * ldo + col)
-                                                : make_uint2(0u, 0u);
-                        }
-                }
-#pragma unroll
-                for (int jj = 0; jj < 2; ++jj) {
-                    const int j = 2 * jh + jj;
-                    const int64_t col = n0 + wn * 128 + j * 32 + 4 * g;
-#pragma unroll
-                    for (int q = 0; q < 4; ++q) {
-                        float v[4] = {acc[i][j][q * 4], acc[i][j][q * 4 + 1], acc[i][j][q * 4 + 2], acc[i][j][q * 4 + 3]};
-                        quad_transpose(v, lane);
-                        if (!ok[q] || col >= N) continue;
-                        if (scale_a) {
-                            // a row whose factor is exactly 0 is 0 whatever its sum holds (the sums of
-                            // rows that were taken out may have left the fp32 range)
-#pragma unroll
-                            for (int e = 0; e < 4; ++e) v[e] = sb[q] == 0.f ? 0.f : v[e] * sa[q] * sb[q];
-                        }
-                        if (mode == 1 || mode == 3) {
-                            v[0] += part[jj][q].x;
-                            v[1] += part[jj][q].y;
-                            v[2] += part[jj][q].z;
-                            v[3] += part[jj][q].w;
-                        } else if (mode == 4) {
-                            v[0] += oi_bf16lo_to_f32(part16[jj][q].x);
-                            v[1] += oi_bf16hi_to_f32(part16[jj][q].x);
-                            v[2] += oi_bf16lo_to_f32(part16[jj][q].y);
-                            v[3] += oi_bf16hi_to_f32(part16[jj][q].y);
-                        }
-                        if (mode <= 1)
-                            *reinterpret_cast<oi_f32x4*>(out_f32 + row[q] * ldo + col) = oi_f32x4{v[0], v[1], v[2], v[3]};
-                        else
-                            *reinterpret_cast<uint2*>(out_bf16 + dst[q] * ldo + col) =
-                                make_uint2(oi_pack_bf16x2(v[0], v[1]), oi_pack_bf16x2(v[2], v[3]));
-                    }
-                }
-            }
+            for (int jh = 0; jh < 2; ++jh)
+                store_block(st, r, n0 + wn * 128 + jh * 64, lane,
+                            [&](int jj, int q, int e) { return acc[i][2 * jh + jj][q * 4 + e]; });
         }
         return;
     }
@@ -1084,43 +1145,148 @@ struct DynRows {
     const int32_t* mode_dev;
 };
 
+// A launch of resident workgroups computes its tiles in rounds of one per workgroup, and a last round
+// that is half empty takes as long as a full one; with fewer tiles than workgroups most of the chip idles
+// from the start (200 token rows at a hidden size of 4096 are 16 tiles of the d_hidden product for 256 CUs,
+// each running over the whole vocabulary).  The tiles past the last whole round are therefore cut along
+// k into `parts` pieces each, which fill the workgroups evenly; a piece leaves its fp32 tile in scratch and
+// gemm_reduce_kernel adds the pieces of a tile in order (the result does not depend on who ran when).
+// The number of parts is the one with the lowest estimate, in k-tiles of 64 (about 1.5 us): rounds of
+// pieces, 4 k-tiles of prologue and drain per piece, and 3/32 of a k-tile for writing and reading back the
+// 256 KB of a piece.  Pieces are at least 16 k-tiles long.  All from sizes, on the device, where the row
+// count lives; the reduce kernel comes to the same numbers.
+// Measured (whole policy-loss step, before -> after): 268 rows, hidden 4096, vocabulary 100352 (32 tiles):
+// 2.94 -> 1.55 ms; 2400 rows, 3584, 151665 (140 tiles): 8.85 -> 7.46 ms; 22942 rows in three slabs of 480
+// tiles, 4096, 128256: unchanged (a last round that is 7/8 full is left alone).
+struct TailSplit {
+    uint32_t whole, rest, parts;  // tiles [0, whole) in one piece, the `rest` after them in `parts` pieces
+};
+constexpr uint32_t SPLIT_MIN_KTILES = 16, SPLIT_MAX_PARTS = 32, SPLIT_MAX_ITEMS = 1024;
+__host__ __device__ inline TailSplit plan_tail(uint32_t tiles, uint32_t grid, uint32_t ktiles) {
+    TailSplit t = {tiles, 0, 1};
+    const uint32_t rest = tiles % grid;
+    if (rest == 0) return t;
+    uint32_t best = 32 * (ktiles + 4);
+    for (uint32_t parts = 2; parts <= SPLIT_MAX_PARTS; ++parts) {
+        if (rest * parts > SPLIT_MAX_ITEMS || ktiles < SPLIT_MIN_KTILES * parts) break;
+        const uint32_t rounds = (rest * parts + grid - 1) / grid;
+        const uint32_t cost = rounds * (32 * ktiles / parts + 32 * 4) + 3 * rest * parts;
+        if (cost < best) {
+            best = cost;
+            t = {tiles - rest, rest, parts};
+        }
+    }
+    return t;
+}
+// scratch for the pieces of a product of at most `tiles` tiles with at most `ktiles` k-tiles
+inline size_t split_bytes(int64_t tiles, int64_t ktiles) {
+    int64_t parts = ktiles / SPLIT_MIN_KTILES;
+    parts = parts < SPLIT_MAX_PARTS ? parts : SPLIT_MAX_PARTS;
+    if (parts < 2) return 0;
+    const int64_t items = tiles * parts;
+    return (size_t)(items < SPLIT_MAX_ITEMS ? items : SPLIT_MAX_ITEMS) * PART_FLOATS * sizeof(float);
+}
+
+// The sizes of a product that only the device knows, filled in from dyn
+struct ProductSizes {
+    int64_t M, K, m_valid;
+};
+__device__ __forceinline__ ProductSizes product_sizes(int64_t M, int64_t K, int64_t m_valid, const DynRows& dyn) {
+    ProductSizes z = {M, K, m_valid};
+    if (dyn.n_dev) {
+        const int64_t n = *dyn.n_dev;
+        if (dyn.role == 1) {
+            z.M = (n + BM - 1) / BM * BM;
+            z.m_valid = n;
+        } else if (dyn.role == 2) {
+            z.K = (n + BK - 1) / BK * BK;
+        }
+    }
+    return z;
+}
+
 // `queue` null: one workgroup per tile id (blockIdx); otherwise a launch of resident workgroups
-// that draw their tiles from the queue
+// that draw their tiles from the queue.  `parts` (with a queue only): scratch for the pieces of split tiles.
 template <bool A_KM, bool B_KM>
 __global__ void __launch_bounds__(NTHREADS)
     gemm_store_kernel(Operand A, int64_t M, Operand B, int64_t N, int64_t K, int mode, float* out_f32,
-                      uint16_t* out_bf16, int64_t ldo, int64_t m_valid, DynRows dyn, uint32_t* __restrict__ queue) {
+                      uint16_t* out_bf16, int64_t ldo, int64_t m_valid, DynRows dyn, uint32_t* __restrict__ queue,
+                      float* __restrict__ parts) {
     __shared__ __align__(16) uint16_t lds[LDS_ELEMS];
     if (dyn.mode_dev) {
         mode = *dyn.mode_dev;
         if (mode < 0) return;
     }
-    if (dyn.n_dev) {
+    const ProductSizes z = product_sizes(M, K, m_valid, dyn);
+    if (dyn.n_dev && dyn.role == 1) A.extent = z.M;
+    if (dyn.n_dev && dyn.role == 2) {
         const int64_t n = *dyn.n_dev;
-        if (dyn.role == 1) {
-            M = (n + BM - 1) / BM * BM;
-            m_valid = n;
-            A.extent = M;
-        } else if (dyn.role == 2) {
-            K = (n + BK - 1) / BK * BK;
-            A.k_valid = (n + BM - 1) / BM * BM;
-            B.k_valid = n;
-        }
+        A.k_valid = (n + BM - 1) / BM * BM;
+        B.k_valid = n;
     }
+    K = z.K;
     // a product without terms that would only be added changes nothing: no tile is drawn at all
     if (K <= 0 && (mode == 1 || mode == 4)) return;
-    const int64_t tiles_m = (M + BM - 1) / BM, tiles_n = (N + BN - 1) / BN;
+    const StoreTo st = {mode, out_f32, out_bf16, ldo, N, z.m_valid, dyn.out_rows, dyn.scale_a, dyn.scale_b};
+    const int64_t tiles_m = (z.M + BM - 1) / BM, tiles_n = (N + BN - 1) / BN;
     if (queue) {
-        for_each_tile(queue, tiles_m, tiles_n, lds, [&](int64_t tm, int64_t tn) {
-            gemm_store_tile<A_KM, B_KM>(A, M, B, N, K, mode, out_f32, out_bf16, ldo, m_valid, dyn.out_rows, dyn.scale_a,
-                                        dyn.scale_b, tm, tn, lds);
+        const uint32_t tiles = (uint32_t)(tiles_m * tiles_n), ktiles = (uint32_t)(K / BK);
+        TailSplit ts = {tiles, 0, 1};
+        if (parts && stores_in_pieces(st)) ts = plan_tail(tiles, gridDim.x, ktiles);
+        for_each_item(queue, ts.whole + ts.rest * ts.parts, lds, [&](uint32_t item) {
+            uint32_t tile = item, k0 = 0, k1 = ktiles;
+            float* piece = nullptr;
+            if (item >= ts.whole) {
+                const uint32_t r = item - ts.whole, p = r / ts.rest;
+                tile = ts.whole + (r - p * ts.rest);
+                k0 = ktiles * p / ts.parts;
+                k1 = ktiles * (p + 1) / ts.parts;
+                piece = parts + (int64_t)r * PART_FLOATS;
+            }
+            int64_t tm, tn;
+            tile_of_item(tile, (uint32_t)tiles_m, (uint32_t)tiles_n, &tm, &tn);
+            Operand a = A, b = B;
+            const int64_t k_begin = (int64_t)k0 * BK;
+            a.p += A_KM ? k_begin * A.ld : k_begin;
+            b.p += B_KM ? k_begin * B.ld : k_begin;
+            a.k_valid -= k_begin;
+            b.k_valid -= k_begin;
+            gemm_store_tile<A_KM, B_KM>(a, b, (int64_t)(k1 - k0) * BK, st, tm, tn, piece, lds);
         });
     } else {
         int64_t tm, tn;
-        if (tile_of_block(tiles_m, tiles_n, &tm, &tn))
-            gemm_store_tile<A_KM, B_KM>(A, M, B, N, K, mode, out_f32, out_bf16, ldo, m_valid, dyn.out_rows, dyn.scale_a,
-                                        dyn.scale_b, tm, tn, lds);
+        if (tile_of_block(tiles_m, tiles_n, &tm, &tn)) gemm_store_tile<A_KM, B_KM>(A, B, K, st, tm, tn, nullptr, lds);
     }
+}
+
+// Adds the pieces of the split tiles of a gemm_store_kernel launch over `grid` workgroups and stores the
+// sums as that kernel stores a tile.  One wave per 32-row x 64-column block (32 blocks to a tile), four
+// waves to a workgroup; bound by reading the pieces once.
+__global__ void __launch_bounds__(256)
+    gemm_reduce_kernel(const float* __restrict__ parts, uint32_t grid, int64_t M, int64_t N, int64_t K, int mode,
+                       float* out_f32, uint16_t* out_bf16, int64_t ldo, int64_t m_valid, DynRows dyn) {
+    const ProductSizes z = product_sizes(M, K, m_valid, dyn);
+    const StoreTo st = {mode, out_f32, out_bf16, ldo, N, z.m_valid, dyn.out_rows, dyn.scale_a, dyn.scale_b};
+    if (!stores_in_pieces(st)) return;
+    const int64_t tiles_m = (z.M + BM - 1) / BM, tiles_n = (N + BN - 1) / BN;
+    const TailSplit ts = plan_tail((uint32_t)(tiles_m * tiles_n), grid, (uint32_t)(z.K / BK));
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const uint32_t unit = blockIdx.x * 4 + wave, tile = unit >> 5;
+    if (tile >= ts.rest) return;
+    const int w = (unit >> 2) & 7, i = (unit >> 1) & 1, jh = unit & 1;
+    const float* src = parts + (int64_t)tile * PART_FLOATS + ((i * 4 + jh * 2) * 4 * NTHREADS + w * 64 + lane) * 4;
+    oi_f32x4 sum[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) sum[k] = *reinterpret_cast<const oi_f32x4*>(src + k * NTHREADS * 4);
+    for (uint32_t p = 1; p < ts.parts; ++p) {
+        src += (int64_t)ts.rest * PART_FLOATS;
+#pragma unroll
+        for (int k = 0; k < 8; ++k) sum[k] += *reinterpret_cast<const oi_f32x4*>(src + k * NTHREADS * 4);
+    }
+    int64_t tm, tn;
+    tile_of_item(ts.whole + tile, (uint32_t)tiles_m, (uint32_t)tiles_n, &tm, &tn);
+    const LaneRows r = lane_rows(st, tm * BM + (w & 3) * 64 + i * 32, lane);
+    store_block(st, r, tn * BN + (w >> 2) * 128 + jh * 64, lane, [&](int jj, int q, int e) { return sum[jj * 4 + q][e]; });
 }
 
 inline int64_t round_up(int64_t x, int64_t m) { return (x + m - 1) / m * m; }
@@ -1350,7 +1516,7 @@ struct ProbeScope {
 unsigned resident_grid(int64_t tiles_m, int64_t tiles_n) {
     const int cus = oi_cu_count();
     const int64_t grid = (cus + 7) / 8 * 8;
-    const int64_t pids = pids_for_tiles(tiles_m, tiles_n);
+    const int64_t pids = pids_for_items(tiles_m * tiles_n);
     return (unsigned)(pids < grid ? pids : grid);
 }
 
@@ -1395,7 +1561,8 @@ struct KeepPlan {
 struct FwdPlan {
     int64_t token_tiles, vocab_tiles, n_splits, tiles_per_split, long_splits, n_pad;
     int64_t chunk, n_chunks;  // chunked flavour only
-    size_t off_partial, off_zy, off_queue, off_chunk, off_xref, total;
+    size_t off_partial, off_zy, off_queue, off_chunk, off_parts, total;
+    size_t parts_bytes;  // chunked flavour: scratch for the pieces of the products
     SelectionPlan sel;
 };
 // `chunked`: the launch covers one backward-sized vocabulary chunk at a time (the forward that also
@@ -1433,7 +1600,8 @@ FwdPlan plan_fwd(int64_t n_tokens, int64_t hdim, int64_t vocab, bool with_select
     p.off_queue = cv.take((chunked ? (size_t)p.n_chunks * (FWD_QUEUE_WORDS + QUEUE_WORDS) : (size_t)FWD_QUEUE_WORDS) *
                           sizeof(uint32_t));
     p.off_chunk = chunked ? cv.take((size_t)p.n_pad * p.chunk * 2) : 0;
-    p.off_xref = 0;
+    p.parts_bytes = chunked ? split_bytes(p.token_tiles * ((hdim + BN - 1) / BN), p.chunk / BK) : 0;
+    p.off_parts = cv.take(p.parts_bytes);
     if (with_selection) p.sel = plan_selection(cv, p.n_pad, hdim, false);
     p.total = cv.off;
     return p;
@@ -1441,10 +1609,12 @@ FwdPlan plan_fwd(int64_t n_tokens, int64_t hdim, int64_t vocab, bool with_select
 
 struct BwdPlan {
     int64_t n_pad, v_pad, chunk, n_chunks;
-    size_t off_dz, off_dh32, off_queues, total;
+    size_t off_dz, off_dh32, off_queues, off_parts, total;
+    size_t parts_bytes;
     SelectionPlan sel;
 };
-BwdPlan plan_bwd(int64_t n_tokens, int64_t hdim, int64_t vocab, bool with_selection) {
+// `few_rows`: for a call that normally finds no rows (its products are not split)
+BwdPlan plan_bwd(int64_t n_tokens, int64_t hdim, int64_t vocab, bool with_selection, bool few_rows = false) {
     BwdPlan p;
     p.n_pad = round_up(n_tokens, 256);
     p.v_pad = round_up(vocab, 256);
@@ -1455,6 +1625,8 @@ BwdPlan plan_bwd(int64_t n_tokens, int64_t hdim, int64_t vocab, bool with_select
     p.off_dh32 = cv.take((size_t)n_tokens * hdim * 4);
     // one set of work-queue counters per tile-kernel launch (three per vocabulary chunk)
     p.off_queues = cv.take((size_t)(3 * p.n_chunks) * QUEUE_WORDS * sizeof(uint32_t));
+    p.parts_bytes = few_rows ? 0 : split_bytes(p.n_pad / BM * ((hdim + BN - 1) / BN), p.chunk / BK);
+    p.off_parts = cv.take(p.parts_bytes);
     if (with_selection) p.sel = plan_selection(cv, p.n_pad, hdim, true);
     p.total = cv.off;
     return p;
@@ -1550,6 +1722,21 @@ void enqueue_fwd(const FwdPlan& p, char* ws, const RowInputs& in, const uint8_t*
                        keep.buf ? keep.unsafe : static_cast<uint8_t*>(nullptr));
 }
 
+// A product of token rows with W (k-contiguous x k-major, rows counted on the device): the tile kernel and,
+// where its tiles may be split along k, the addition of their pieces.
+void launch_rows_product(unsigned grid, const Operand& a, int64_t M, const Operand& b, int64_t N, int64_t K, int mode,
+                         float* out_f32, void* out_bf16, int64_t ldo, int64_t m_valid, const DynRows& dyn,
+                         uint32_t* queue, float* parts, hipStream_t s) {
+    uint16_t* o16 = static_cast<uint16_t*>(out_bf16);
+    hipLaunchKernelGGL((gemm_store_kernel<false, true>), dim3(grid), dim3(NTHREADS), 0, s, a, M, b, N, K, mode, out_f32,
+                       o16, ldo, m_valid, dyn, queue, parts);
+    if (!parts) return;
+    const int64_t tiles = (M + BM - 1) / BM * ((N + BN - 1) / BN);
+    const int64_t most = tiles < (int64_t)grid ? tiles : (int64_t)grid - 1;  // tiles past the last whole round
+    hipLaunchKernelGGL(gemm_reduce_kernel, dim3((unsigned)(most * 8)), dim3(256), 0, s, parts, grid, M, N, K, mode,
+                       out_f32, o16, ldo, m_valid, dyn);
+}
+
 // The forward that also prepares d_hidden.  With x = z c in the log2 domain and a per-token
 // reference exponent ref_n (the scaled logit of the token's own label),
 //   d_hidden[n] = sum_v dZ[n, v] W[v]
@@ -1568,6 +1755,7 @@ void enqueue_fwd_wsum(const FwdPlan& p, char* ws, const RowInputs& in, const uin
     float* zy = reinterpret_cast<float*>(ws + p.off_zy);
     uint32_t* queues = reinterpret_cast<uint32_t*>(ws + p.off_queue);
     uint16_t* chunk_buf = reinterpret_cast<uint16_t*>(ws + p.off_chunk);
+    float* parts = p.parts_bytes ? reinterpret_cast<float*>(ws + p.off_parts) : nullptr;
     const float c = inv_temperature * OI_LOG2E;
     const uint16_t* Wp = static_cast<const uint16_t*>(weight);
     const int64_t h_tiles = (hidden_dim + BN - 1) / BN;
@@ -1589,9 +1777,8 @@ void enqueue_fwd_wsum(const FwdPlan& p, char* ws, const RowInputs& in, const uin
         const Operand a = {chunk_buf, cols, 0, p.n_pad, cols};
         const Operand b = {Wp + v_begin * hidden_dim, hidden_dim, 0, hidden_dim, valid};
         const DynRows dyn = {in.n_dev, 1, nullptr, nullptr, nullptr, nullptr};
-        hipLaunchKernelGGL((gemm_store_kernel<false, true>), dim3(resident_grid(p.n_pad / BM, h_tiles)), dim3(NTHREADS), 0,
-                           s, a, p.n_pad, b, hidden_dim, round_up(valid, BK), ci == 0 ? 0 : 1, wsum,
-                           static_cast<uint16_t*>(nullptr), hidden_dim, n_tokens, dyn, q + FWD_QUEUE_WORDS);
+        launch_rows_product(resident_grid(p.n_pad / BM, h_tiles), a, p.n_pad, b, hidden_dim, round_up(valid, BK),
+                            ci == 0 ? 0 : 1, wsum, nullptr, hidden_dim, n_tokens, dyn, q + FWD_QUEUE_WORDS, parts, s);
     }
     hipLaunchKernelGGL(lmhead_fwd_combine_kernel, dim3((unsigned)((n_tokens + COMBINE_TOKENS - 1) / COMBINE_TOKENS)), dim3(256), 0, s, partial,
                        zy, n_tokens, in.n_dev, in.rows, row_mask, n_tokens, p.n_splits, p.n_pad, inv_temperature, c, logprob,
@@ -1656,6 +1843,7 @@ void enqueue_bwd(const BwdPlan& p, char* ws, const RowInputs& in, const void* we
     };
     uint16_t* dz = reinterpret_cast<uint16_t*>(ws + p.off_dz);
     float* dh32 = reinterpret_cast<float*>(ws + p.off_dh32);
+    float* parts = p.parts_bytes ? reinterpret_cast<float*>(ws + p.off_parts) : nullptr;
     uint32_t* queues = reinterpret_cast<uint32_t*>(ws + p.off_queues);
     const uint16_t* Wp = static_cast<const uint16_t*>(weight);
     const float c = inv_temperature * OI_LOG2E;
@@ -1675,9 +1863,8 @@ void enqueue_bwd(const BwdPlan& p, char* ws, const RowInputs& in, const void* we
             const Operand a = {dz, cols, 0, p.n_pad, cols};
             const Operand b = {Wp + v_begin * hidden_dim, hidden_dim, 0, hidden_dim, valid};
             const DynRows dyn = {in.n_dev, 1, in.rows, nullptr, nullptr, nullptr};
-            hipLaunchKernelGGL((gemm_store_kernel<false, true>), grid_of(p.n_pad / BM, h_tiles),
-                               dim3(NTHREADS), 0, s, a, p.n_pad, b, hidden_dim, round_up(valid, BK), mode, dh32,
-                               static_cast<uint16_t*>(d_hidden), hidden_dim, n_tokens, dyn, q + QUEUE_WORDS);
+            launch_rows_product(grid_of(p.n_pad / BM, h_tiles).x, a, p.n_pad, b, hidden_dim, round_up(valid, BK), mode,
+                                dh32, d_hidden, hidden_dim, n_tokens, dyn, q + QUEUE_WORDS, parts, s);
         }
         if (d_weight) {
             const Operand a = {dz, cols, 0, cols, p.n_pad};
@@ -1687,7 +1874,7 @@ void enqueue_bwd(const BwdPlan& p, char* ws, const RowInputs& in, const void* we
                                dim3(NTHREADS), 0, s, a, cols, b, hidden_dim, round_up(n_tokens, BK), dw_mode,
                                dw32 ? dw32 + v_begin * hidden_dim : static_cast<float*>(nullptr),
                                static_cast<uint16_t*>(d_weight) + v_begin * hidden_dim, hidden_dim, valid, dyn,
-                               q + 2 * QUEUE_WORDS);
+                               q + 2 * QUEUE_WORDS, static_cast<float*>(nullptr));
         }
     }
 }
@@ -1701,7 +1888,8 @@ void enqueue_products_from_exponentials(const uint16_t* ecache, int64_t cache_ld
                                         const int32_t* count, const int32_t* rows_s, const float* scale_a,
                                         const float* scale_b, const uint16_t* scaled_hidden, const void* weight,
                                         int64_t hidden_dim, int64_t vocab, void* d_hidden, void* d_weight,
-                                        const int32_t* dw_mode_dev, float* dw32, uint32_t* queues, hipStream_t s) {
+                                        const int32_t* dw_mode_dev, float* dw32, uint32_t* queues, float* parts,
+                                        hipStream_t s) {
     const uint16_t* Wp = static_cast<const uint16_t*>(weight);
     const int64_t h_tiles = (hidden_dim + BN - 1) / BN;
     {
@@ -1709,10 +1897,8 @@ void enqueue_products_from_exponentials(const uint16_t* ecache, int64_t cache_ld
         const Operand a = {ecache, cache_ld, 0, slab_pad, cache_ld};
         const Operand b = {Wp, hidden_dim, 0, hidden_dim, vocab};
         const DynRows dyn = {count, 1, rows_s, scale_a, scale_b, nullptr};
-        hipLaunchKernelGGL((gemm_store_kernel<false, true>), dim3(resident_grid(slab_pad / BM, h_tiles)),
-                           dim3(NTHREADS), 0, s, a, slab_pad, b, hidden_dim, round_up(vocab, BK), 2,
-                           static_cast<float*>(nullptr), static_cast<uint16_t*>(d_hidden), hidden_dim, slab_pad, dyn,
-                           queues);
+        launch_rows_product(resident_grid(slab_pad / BM, h_tiles), a, slab_pad, b, hidden_dim, round_up(vocab, BK), 2,
+                            nullptr, d_hidden, hidden_dim, slab_pad, dyn, queues, parts, s);
     }
     if (d_weight) {
         const ProbeScope probe(2, s);
@@ -1721,7 +1907,8 @@ void enqueue_products_from_exponentials(const uint16_t* ecache, int64_t cache_ld
         const DynRows dyn = {count, 2, nullptr, nullptr, nullptr, dw_mode_dev};
         hipLaunchKernelGGL((gemm_store_kernel<true, true>), dim3(resident_grid(cache_ld / BM, h_tiles)),
                            dim3(NTHREADS), 0, s, a, cache_ld, b, hidden_dim, round_up(slab_pad, BK), 2, dw32,
-                           static_cast<uint16_t*>(d_weight), hidden_dim, vocab, dyn, queues + QUEUE_WORDS);
+                           static_cast<uint16_t*>(d_weight), hidden_dim, vocab, dyn, queues + QUEUE_WORDS,
+                           static_cast<float*>(nullptr));
     }
 }
 
@@ -1771,7 +1958,8 @@ struct SlabPlan {
     BwdPlan repair;  // the recomputing backward over all rows (for the flagged ones)
     size_t off_fwd, off_order, off_count, off_meta, off_unsafe, off_keep, off_repair, off_hidden_s, off_labels_s,
         off_rows_s, off_xref_s, off_scale_a, off_scale_b, off_scaled_hidden, off_queues, off_dw32, off_stats, off_lse,
-        off_grad, off_denoms, total;
+        off_grad, off_denoms, off_parts, total;
+    size_t parts_bytes;
 };
 SlabPlan plan_slabs(int64_t n, int64_t stats_rows, int64_t stats_cols, int64_t hdim, int64_t vocab, bool want_dw,
                     int64_t slab_tokens, int64_t n_passes_override = 0) {
@@ -1782,7 +1970,7 @@ SlabPlan plan_slabs(int64_t n, int64_t stats_rows, int64_t stats_cols, int64_t h
     p.cap = p.n_pad < cap ? p.n_pad : cap;
     p.n_passes = n_passes_override > 0 ? n_passes_override : (p.n_pad + p.cap - 1) / p.cap;
     p.fwd = plan_fwd(p.cap, hdim, vocab, false);
-    p.repair = plan_bwd(n, hdim, vocab, true);
+    p.repair = plan_bwd(n, hdim, vocab, true, true);
     Carver cv;
     p.off_fwd = cv.take(p.fwd.total);
     p.off_order = cv.take((size_t)p.n_pad * sizeof(int32_t));
@@ -1805,6 +1993,8 @@ SlabPlan plan_slabs(int64_t n, int64_t stats_rows, int64_t stats_cols, int64_t h
     p.off_lse = cv.take((size_t)n * sizeof(float));
     p.off_grad = cv.take((size_t)n * sizeof(float));
     p.off_denoms = cv.take((size_t)stats_rows * sizeof(float));
+    p.parts_bytes = split_bytes(p.cap / BM * ((hdim + BN - 1) / BN), p.v_pad / BK);
+    p.off_parts = cv.take(p.parts_bytes);
     p.total = cv.off;
     return p;
 }
@@ -1888,6 +2078,7 @@ int run_slab_passes(const SlabPlan& p, char* ws, const SlabStep& st, hipStream_t
     float* dw32 = st.d_weight && p.n_passes > 1 ? reinterpret_cast<float*>(ws + p.off_dw32) : nullptr;
     float* lse = reinterpret_cast<float*>(ws + p.off_lse);
     float* grad = reinterpret_cast<float*>(ws + p.off_grad);
+    float* parts = p.parts_bytes ? reinterpret_cast<float*>(ws + p.off_parts) : nullptr;
     const uint16_t* hid = static_cast<const uint16_t*>(st.hidden);
 
     hipLaunchKernelGGL(zero_words_kernel, dim3((unsigned)((p.n_pad / 4 + 255) / 256)), dim3(256), 0, s,
@@ -1918,7 +2109,7 @@ int run_slab_passes(const SlabPlan& p, char* ws, const SlabStep& st, hipStream_t
                            hidden_s, scale_a, scale_b, scaled_hidden);
         enqueue_products_from_exponentials(keep_buf, p.v_pad, p.cap, cnt, rows_s, scale_a, scale_b, scaled_hidden,
                                            st.weight, hdim, vocab, st.d_hidden, st.d_weight, &meta[i].dw_mode, dw32,
-                                           queues + FWD_QUEUE_WORDS, s);
+                                           queues + FWD_QUEUE_WORDS, parts, s);
     }
     // the flagged rows, if any: one recomputing backward over them (its workspace takes the place of
     // the exponentials), added to what the slabs left in d_weight
@@ -2017,7 +2208,7 @@ struct DhPlan {
 };
 DhPlan plan_dh(int64_t n_tokens, int64_t hdim, int64_t vocab) {
     DhPlan p;
-    p.repair = plan_bwd(n_tokens, hdim, vocab, true);
+    p.repair = plan_bwd(n_tokens, hdim, vocab, true, true);
     Carver cv;
     p.off_rows = cv.take((size_t)round_up(n_tokens, 256) * sizeof(int32_t));
     p.off_count = cv.take(sizeof(int32_t));
@@ -2527,7 +2718,7 @@ extern "C" int oi_gemm_bf16_tn(const void* A, int64_t lda, int64_t M, const void
     const Operand b = {static_cast<const uint16_t*>(B), ldb, 0, N, K};
     hipLaunchKernelGGL((gemm_store_kernel<false, false>), dim3(grid_for_tiles((M + BM - 1) / BM, (N + BN - 1) / BN)),
                        dim3(NTHREADS), 0, static_cast<hipStream_t>(stream), a, M, b, N, K, mode, out_f32,
-                       static_cast<uint16_t*>(out_bf16), ldo, M, DynRows{nullptr, 0, nullptr, nullptr, nullptr, nullptr}, static_cast<uint32_t*>(nullptr));
+                       static_cast<uint16_t*>(out_bf16), ldo, M, DynRows{nullptr, 0, nullptr, nullptr, nullptr, nullptr}, static_cast<uint32_t*>(nullptr), static_cast<float*>(nullptr));
     return oi_launch_status();
 }
 
@@ -2551,18 +2742,19 @@ extern "C" int oi_gemm_bf16_layouts(const void* A, int64_t lda, int a_k_major, c
     hipStream_t s = static_cast<hipStream_t>(stream);
     uint16_t* o16 = static_cast<uint16_t*>(out_bf16);
     uint32_t* no_queue = nullptr;
+    float* no_parts = nullptr;
     const DynRows fixed = {nullptr, 0, nullptr, nullptr, nullptr, nullptr};
     if (a_k_major && b_k_major)
         hipLaunchKernelGGL((gemm_store_kernel<true, true>), grid, dim3(NTHREADS), 0, s, a, M, b, N, K, mode, out_f32, o16,
-                           ldo, M, fixed, no_queue);
+                           ldo, M, fixed, no_queue, no_parts);
     else if (a_k_major)
         hipLaunchKernelGGL((gemm_store_kernel<true, false>), grid, dim3(NTHREADS), 0, s, a, M, b, N, K, mode, out_f32,
-                           o16, ldo, M, fixed, no_queue);
+                           o16, ldo, M, fixed, no_queue, no_parts);
     else if (b_k_major)
         hipLaunchKernelGGL((gemm_store_kernel<false, true>), grid, dim3(NTHREADS), 0, s, a, M, b, N, K, mode, out_f32,
-                           o16, ldo, M, fixed, no_queue);
+                           o16, ldo, M, fixed, no_queue, no_parts);
     else
         hipLaunchKernelGGL((gemm_store_kernel<false, false>), grid, dim3(NTHREADS), 0, s, a, M, b, N, K, mode, out_f32,
-                           o16, ldo, M, fixed, no_queue);
+                           o16, ldo, M, fixed, no_queue, no_parts);
     return oi_launch_status();
 }

@@ -1,0 +1,94 @@
+"""GPU parity of the tile kernels at the sizes where their work is divided differently: products cut along
+the vocabulary, one vocabulary chunk or several, against fp32 autograd on the same bf16 inputs.
+
+Gradients are held to 2 % of their norm and, per entry, to one bf16 rounding (2**-8) of the entry plus 2**-7
+of the largest one: an entry is a sum of products with bf16 factors (dZ or the kept exponentials, 2**-9
+each), rounded once to bf16.
+"""
+
+import types
+
+import pytest
+import torch
+
+from open_instruct_amd import grpo_utils, lm_head
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+TOL = 2e-3
+
+
+def _inputs(n, h, v, seed):
+    g = torch.Generator(device=DEV).manual_seed(seed)
+    hidden = torch.randn(n, h, generator=g, device=DEV).bfloat16()
+    weight = (torch.randn(v, h, generator=g, device=DEV) * (2.0 / h**0.5)).bfloat16()
+    labels = torch.randint(0, v, (n,), generator=g, device=DEV)
+    mask = torch.rand(n, generator=g, device=DEV) < 0.8
+    upstream = torch.randn(n, generator=g, device=DEV)
+    return hidden, weight, labels, mask, upstream
+
+
+def _reference(hidden, weight, labels, mask, upstream):
+    """logprobs and both gradients in fp32, 2048 rows at a time."""
+    h32, w32 = hidden.float(), weight.float()
+    lp = torch.zeros(hidden.shape[0], device=DEV)
+    dh, dw = torch.zeros_like(h32), torch.zeros_like(w32)
+    for a in range(0, hidden.shape[0], 2048):
+        rows = slice(a, a + 2048)
+        z = h32[rows] @ w32.t()
+        logp = z.log_softmax(1)
+        lp[rows] = logp.gather(1, labels[rows, None])[:, 0] * mask[rows]
+        dz = logp.exp_().neg_()
+        dz[torch.arange(dz.shape[0], device=DEV), labels[rows]] += 1.0
+        dz *= (upstream * mask)[rows, None]
+        dh[rows] = dz @ w32
+        dw += dz.t() @ h32[rows]
+    return lp, dh, dw
+
+
+def _close(got, exp, name):
+    err = (got.float() - exp).abs()
+    bound = TOL * exp.abs().max() + exp.abs() * 2**-8 + exp.abs().max() * 2**-7
+    assert (err <= bound).all(), (name, err.max().item(), exp.abs().max().item())
+    rel = ((got.float() - exp).norm() / exp.norm()).item()
+    assert rel <= 2e-2, (name, rel)
+
+
+@pytest.mark.parametrize(
+    "n,h,v",
+    [
+        (70, 64, 1984),  # 31 k-tiles: too short to cut
+        (70, 64, 2048),  # 32 k-tiles: the shortest product that is cut, in two
+        (1, 64, 2049),  # one row, 33 k-tiles, the last of one vocabulary row
+        (300, 320, 9001),  # four tiles in eight pieces
+        (600, 1088, 33000),  # pieces bounded by the scratch, ragged last hidden tile
+        (16500, 1088, 2300),  # a whole round of tiles and a cut rest
+        (9000, 64, 120000),  # two vocabulary chunks
+    ],
+)
+@pytest.mark.parametrize("route", ["d_weight", "d_hidden_in_forward", "slabs"])
+def test_products_cut_along_the_vocabulary(n, h, v, route):
+    print(f"case N={n} H={h} V={v} route={route}", flush=True)
+    hidden, weight, labels, mask, upstream = _inputs(n, h, v, seed=n + v)
+    mask[0] = True
+    if route == "slabs":
+        # the policy loss whose gradient to a logprob is -advantage / count: ratio 1, no KL term
+        upstream = -upstream / mask.sum()
+        adv = -upstream * mask.sum()
+    lp, dh, dw = _reference(hidden, weight, labels, mask, upstream)
+    hid, w = hidden.requires_grad_(True), weight.requires_grad_(route != "d_hidden_in_forward")
+    if route == "slabs":
+        cfg = types.SimpleNamespace(loss_fn="cispo", clip_lower=0.2, clip_higher=0.2, beta=0.0, kl_estimator=2)
+        loss, _, out, _ = grpo_utils.grpo_loss_on_hidden(
+            hid[None], w, labels[None], None, None, adv[None], mask[None], cfg, token_slabs=4096
+        )
+        loss.backward()
+        out = out[0]
+    else:
+        out, _ = lm_head.fused_lm_head_logprobs(hid, w, labels, mask=mask)
+        out.backward(upstream)
+    assert (out.detach() - lp).abs().max().item() <= TOL
+    _close(hid.grad, dh, "d_hidden")
+    assert (hid.grad[~mask] == 0).all()
+    if w.requires_grad:
+        _close(w.grad, dw, "d_weight")
