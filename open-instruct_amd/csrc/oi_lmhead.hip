@@ -718,11 +718,13 @@ constexpr float KEEP_MAX_LOG2 = 64.f;
 // `unsafe` (one byte per caller row, optional, cleared by the caller beforehand): set for a token
 // whose kept exponentials cannot be trusted (its maximum is too far above xref[n], or is not a
 // number); never cleared here, so marks that the caller has put there survive.
-// Launch: 256 threads = 4 waves; a workgroup handles 64 tokens (lane = token, so the 16-byte partials
-// of a split are read as one contiguous piece per wave), wave w merges the splits w, w + 4, ... and
-// the four results meet in the LDS.
-constexpr int COMBINE_TOKENS = 64;
-__global__ void __launch_bounds__(256)
+// Launch: a workgroup handles 64 tokens (lane = token, so the 16-byte partials of a split are read as one
+// contiguous piece per wave), wave w merges the splits w, w + 16, ... and the results meet in the LDS.
+// Bound by the latency of the reads, since a call has few workgroups: hence 16 waves with four reads each in
+// flight.  One wave in four with one read in flight took 50 us for 268 tokens x 392 splits (10 us now),
+// 30 us for 1432 x 275 (9 us).
+constexpr int COMBINE_TOKENS = 64, COMBINE_WAVES = 16, COMBINE_THREADS = COMBINE_WAVES * OI_WAVE;
+__global__ void __launch_bounds__(COMBINE_THREADS)
     lmhead_fwd_combine_kernel(const float4* __restrict__ partial, const float* __restrict__ zy, int64_t n_tokens,
                               const int32_t* __restrict__ n_dev, const int32_t* __restrict__ rows,
                               const uint8_t* __restrict__ row_mask, int64_t n_total, int64_t n_splits, int64_t n_pad,
@@ -730,20 +732,31 @@ __global__ void __launch_bounds__(256)
                               float* __restrict__ lse_out, const float* __restrict__ xref,
                               uint8_t* __restrict__ unsafe) {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int64_t n = (int64_t)blockIdx.x * COMBINE_TOKENS + lane;
+    const int64_t first = (int64_t)blockIdx.x * COMBINE_TOKENS, n = first + lane;
     if (n_dev) n_tokens = *n_dev;
     if (wave == 0 && row_mask && n < n_total && !row_mask[n]) {
         logprob[n] = 0.f;
         if (entropy) entropy[n] = 0.f;
         if (lse_out) lse_out[n] = 0.f;
     }
+    if (first >= n_tokens) return;
     float m = OI_NEG_BIG, s = 0.f, t = 0.f;
-    if (n < n_tokens)
-        for (int64_t sp = wave; sp < n_splits; sp += 4) {
-            const float4 p = partial[sp * n_pad + n];
-            merge_stats(m, s, t, p.x, p.y, p.z, &m, &s, &t);
+    if (n < n_tokens) {
+        const float4* p = partial + n;
+        int64_t sp = wave;
+        for (; sp + 3 * COMBINE_WAVES < n_splits; sp += 4 * COMBINE_WAVES) {
+            float4 q[4];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) q[u] = p[(sp + u * COMBINE_WAVES) * n_pad];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) merge_stats(m, s, t, q[u].x, q[u].y, q[u].z, &m, &s, &t);
         }
-    __shared__ float red[3][3][COMBINE_TOKENS];
+        for (; sp < n_splits; sp += COMBINE_WAVES) {
+            const float4 q = p[sp * n_pad];
+            merge_stats(m, s, t, q.x, q.y, q.z, &m, &s, &t);
+        }
+    }
+    __shared__ float red[COMBINE_WAVES - 1][3][COMBINE_TOKENS];
     if (wave > 0) {
         red[wave - 1][0][lane] = m;
         red[wave - 1][1][lane] = s;
@@ -751,8 +764,8 @@ __global__ void __launch_bounds__(256)
     }
     __syncthreads();
     if (wave != 0 || n >= n_tokens) return;
-#pragma unroll
-    for (int w = 0; w < 3; ++w) merge_stats(m, s, t, red[w][0][lane], red[w][1][lane], red[w][2][lane], &m, &s, &t);
+    const int merged = n_splits < COMBINE_WAVES ? (int)n_splits : COMBINE_WAVES;
+    for (int w = 0; w < merged - 1; ++w) merge_stats(m, s, t, red[w][0][lane], red[w][1][lane], red[w][2][lane], &m, &s, &t);
     const double ln2 = 0.69314718055994530942;
     const double log2s = log2((double)s);
     // the statistics are in units of x = z * c with the fp32 constant c the tile kernel multiplied by:
@@ -1731,7 +1744,8 @@ void enqueue_fwd(const FwdPlan& p, char* ws, const RowInputs& in, const uint8_t*
     } else
         hipLaunchKernelGGL(lmhead_fwd_kernel<false>, grid, dim3(NTHREADS), 0, s, Wp, in.hidden, in.labels, n_tokens,
                            in.n_dev, hidden_dim, vocab, c, fl, p.n_pad, partial, zy, queue);
-    hipLaunchKernelGGL(lmhead_fwd_combine_kernel, dim3((unsigned)((n_tokens + COMBINE_TOKENS - 1) / COMBINE_TOKENS)), dim3(256), 0, s, partial,
+    hipLaunchKernelGGL(lmhead_fwd_combine_kernel, dim3((unsigned)((n_tokens + COMBINE_TOKENS - 1) / COMBINE_TOKENS)),
+                       dim3(COMBINE_THREADS), 0, s, partial,
                        zy, n_tokens, in.n_dev, in.rows, row_mask, n_tokens, p.n_splits, p.n_pad, inv_temperature, c, logprob,
                        entropy, lse, keep.buf ? keep.xref : static_cast<const float*>(nullptr),
                        keep.buf ? keep.unsafe : static_cast<uint8_t*>(nullptr));
@@ -1795,7 +1809,8 @@ void enqueue_fwd_wsum(const FwdPlan& p, char* ws, const RowInputs& in, const uin
         launch_rows_product(resident_grid(p.n_pad / BM, h_tiles), a, p.n_pad, b, hidden_dim, round_up(valid, BK),
                             ci == 0 ? 0 : 1, wsum, nullptr, hidden_dim, n_tokens, dyn, q + FWD_QUEUE_WORDS, parts, s);
     }
-    hipLaunchKernelGGL(lmhead_fwd_combine_kernel, dim3((unsigned)((n_tokens + COMBINE_TOKENS - 1) / COMBINE_TOKENS)), dim3(256), 0, s, partial,
+    hipLaunchKernelGGL(lmhead_fwd_combine_kernel, dim3((unsigned)((n_tokens + COMBINE_TOKENS - 1) / COMBINE_TOKENS)),
+                       dim3(COMBINE_THREADS), 0, s, partial,
                        zy, n_tokens, in.n_dev, in.rows, row_mask, n_tokens, p.n_splits, p.n_pad, inv_temperature, c, logprob,
                        entropy, lse, static_cast<const float*>(xref), unsafe);
 }
