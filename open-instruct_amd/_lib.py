@@ -63,6 +63,11 @@ SIGNATURES: dict[str, tuple] = {
     "oi_lmhead_logp_fwd": (_I, [_P, _P, _P, _P, _I64, _I64, _I64, _F, _P, _P, _P, _P, _SZ, _P]),
     "oi_lmhead_bwd_workspace_bytes": (_SZ, [_I64, _I64, _I64, _I, _I]),
     "oi_lmhead_logp_bwd": (_I, [_P, _P, _P, _P, _P, _P, _I, _I64, _I64, _I64, _F, _P, _P, _P, _P, _SZ, _P]),
+    "oi_lmhead_kept_bytes": (_SZ, [_I64, _I64]),
+    "oi_lmhead_logp_fwd_kept": (_I, [_P, _P, _P, _P, _I64, _I64, _I64, _F, _P, _P, _P, _P, _SZ, _P, _SZ, _P]),
+    "oi_lmhead_logp_bwd_kept": (
+        _I, [_P] * 6 + [_I64, _I64, _I64, _F, _P, _P, _SZ, _P, _P, _P, _SZ, _P],
+    ),
     "oi_lmhead_fwd_wsum_workspace_bytes": (_SZ, [_I64, _I64, _I64, _I]),
     "oi_lmhead_logp_fwd_wsum": (_I, [_P, _P, _P, _P, _I64, _I64, _I64, _F, _P, _P, _P, _P, _P, _P, _P, _SZ, _P]),
     "oi_lmhead_dh_workspace_bytes": (_SZ, [_I64, _I64, _I64]),

@@ -455,6 +455,23 @@ __device__ __forceinline__ int acc_row(int wm, int i, int r, int lane) {
 }
 __device__ __forceinline__ int acc_col(int wn, int j, int lane) { return wn * 128 + j * 32 + (lane & 31); }
 
+// A fp32 tile that another kernel picks up: in the order in which the accumulators lie in the registers
+// (16 bytes per lane, consecutive lanes together, groups of PART_GROUP floats), so that neither side
+// rearranges anything.
+constexpr int PART_FLOATS = BM * BN, PART_GROUP = NTHREADS * 4;
+__device__ __forceinline__ int part_group(int i, int j, int q) { return (i * 4 + j) * 4 + q; }
+__device__ __forceinline__ void store_part(const AccTile& acc, float* part, int tid) {
+    asm volatile("" : "+v"(tid));
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+                *reinterpret_cast<oi_f32x4*>(part + part_group(i, j, q) * PART_GROUP + tid * 4) =
+                    oi_f32x4{acc[i][j][q * 4], acc[i][j][q * 4 + 1], acc[i][j][q * 4 + 2], acc[i][j][q * 4 + 3]};
+}
+
 // Online softmax statistics in the log2 domain of the scaled logits x = z * c:
 //   m = max x,  s = sum 2^(x - m),  t = sum 2^(x - m) * (x - m)
 // (entropy = ln2 * (log2 s - t / s), logsumexp = ln2 * (m + log2 s)).
@@ -558,6 +575,8 @@ __device__ __forceinline__ void copy_staged_group(const uint16_t* stage, uint16_
 // ---------------------------------------------------------------------------------------------
 // CACHE: the vocabulary tiles [cache_tile0, cache_tile0 + cache_tiles) also leave 2^(z c - xref[n])
 // behind as bf16, token-major [n_pad, cache_ld]; rows of tokens past the end are zero.
+// LOGITS: every tile leaves its fp32 logits behind (store_part), tile (vt, tt) at logits +
+// (vt * logits_tiles + tt) * PART_FLOATS.
 // What a forward launch covers and where its exponentials go.  Splits [0, long_splits) take
 // tiles_per_split vocabulary tiles each, the others one.  A launch hands out the long splits
 // [first, first + n_first) from one set of queues and then the short splits
@@ -570,14 +589,18 @@ struct FwdLaunch {
     int64_t cache_ld, cache_tile0, cache_tiles;
     int skip_label;
     const float* xref;  // per token: the exponent that the kept exponentials are relative to (null: 0)
+    float* logits;
+    int64_t logits_tiles;
 };
+enum FwdKeep { FWD_PLAIN, FWD_EXPONENTIALS, FWD_LOGITS };
 
-template <bool CACHE>
+template <FwdKeep KEEP>
 __device__ __forceinline__ void lmhead_fwd_item(const uint16_t* __restrict__ W, const uint16_t* __restrict__ hidden,
                                                 const int64_t* __restrict__ labels, int64_t n_tokens, int64_t hdim,
                                                 int64_t vocab, float c, const FwdLaunch& fl, int64_t n_pad,
                                                 float4* __restrict__ partial, float* __restrict__ zy, int64_t split,
                                                 int64_t tt, uint16_t* lds) {
+    constexpr bool CACHE = KEEP == FWD_EXPONENTIALS;
     const int64_t tiles_per_split = fl.tiles_per_split, long_splits = fl.long_splits;
     const int64_t vocab_tiles = (vocab + BM - 1) / BM;
     // the first long_splits splits take tiles_per_split vocabulary tiles each, the others one
@@ -606,6 +629,8 @@ __device__ __forceinline__ void lmhead_fwd_item(const uint16_t* __restrict__ W, 
         AccTile acc;
         const int64_t m0 = vt * BM;
         gemm_tile(acc, W, hdim, m0, vocab, hidden, hdim, n0, n_tokens, hdim, lds);
+        // leaves while the statistics are computed
+        if (KEEP == FWD_LOGITS) store_part(acc, fl.logits + (vt * fl.logits_tiles + tt) * PART_FLOATS, tid);
         const bool partial_tile = m0 + BM > vocab;
         const bool keep_tile = CACHE && vt >= fl.cache_tile0 && vt < fl.cache_tile0 + fl.cache_tiles;
         const int wave_row0 = (int)m0 + wm * 64;
@@ -684,7 +709,7 @@ __device__ __forceinline__ void lmhead_fwd_item(const uint16_t* __restrict__ W, 
     }
 }
 
-template <bool CACHE>
+template <FwdKeep KEEP>
 __global__ void __launch_bounds__(NTHREADS)
     lmhead_fwd_kernel(const uint16_t* __restrict__ W, const uint16_t* __restrict__ hidden,
                       const int64_t* __restrict__ labels, int64_t n_tokens, const int32_t* __restrict__ n_dev,
@@ -696,12 +721,12 @@ __global__ void __launch_bounds__(NTHREADS)
     // every long item of every XCD's queue is taken before the first short one: the short items are
     // there to fill the end of the launch
     for_each_tile(queue, fl.n_first, token_tiles, lds, [&](int64_t split, int64_t tt) {
-        lmhead_fwd_item<CACHE>(W, hidden, labels, n_tokens, hdim, vocab, c, fl, n_pad, partial, zy, fl.first + split, tt,
-                               lds);
+        lmhead_fwd_item<KEEP>(W, hidden, labels, n_tokens, hdim, vocab, c, fl, n_pad, partial, zy, fl.first + split, tt,
+                              lds);
     });
     for_each_tile(queue + QUEUE_WORDS, fl.n_second, token_tiles, lds, [&](int64_t split, int64_t tt) {
-        lmhead_fwd_item<CACHE>(W, hidden, labels, n_tokens, hdim, vocab, c, fl, n_pad, partial, zy,
-                               fl.long_splits + split, tt, lds);
+        lmhead_fwd_item<KEEP>(W, hidden, labels, n_tokens, hdim, vocab, c, fl, n_pad, partial, zy,
+                              fl.long_splits + split, tt, lds);
     });
 }
 
@@ -780,69 +805,80 @@ __global__ void __launch_bounds__(COMBINE_THREADS)
 }
 
 // ---------------------------------------------------------------------------------------------
-// backward step 1: dZ tile = g * inv_T * (onehot - softmax), bf16, both orientations
+// backward step 1: dZ tile = g * inv_T * (onehot - softmax), bf16
 // ---------------------------------------------------------------------------------------------
+// What a dZ tile is made from besides its logits (per-token vectors in the order of the multiplied rows)
+struct DzInputs {
+    const int64_t* labels;
+    const float *lse, *grad, *logprob;
+    int64_t n_tokens, vocab;
+    float c, inv_t;
+};
+// One lane's 32 logits z0, z1 (rows acc_row(wm, 0 / 1, r, lane) of the tile's 256 vocabulary rows from m0)
+// of token n to bf16 entries of dZ in the staging row srow, whose bit 3 is that of the lane.
+//
+// stage[row][v]: rows = tokens, 256 (+8 pad) vocabulary columns.  A lane stores 8 bytes (4 vocabulary
+// entries of one token) and consecutive lanes store to consecutive rows, 132 words apart: the stores of
+// rows 8 apart meet on the same banks (measured: 1000 conflict cycles per tile).  Rows 8..15 of every 16
+// therefore swap the two 8-byte halves of each 16-byte piece (0 conflict cycles); the copy-out swaps them
+// back.
+__device__ __forceinline__ void dz_column(const f32x16& z0, const f32x16& z1, const DzInputs& in, int64_t n, int64_t m0,
+                                          int wm, int lane, uint16_t* srow, int row_bit3) {
+    const int rows_left = (int)(in.vocab - m0 < BM ? in.vocab - m0 : BM);  // real vocabulary rows of the tile
+    const int wave_row0 = wm * 64;
+    const bool live = n < in.n_tokens;
+    const float g = live ? in.grad[n] * in.inv_t : 0.f;
+    // a token without gradient gets an exponent of -huge: every entry becomes -0 * 0
+    const float l2 = g != 0.f ? in.lse[n] * OI_LOG2E : 3.0e38f;
+    int64_t y = live ? in.labels[n] : -1;
+    if (live) y = y < 0 ? 0 : (y >= in.vocab ? in.vocab - 1 : y);
+    // The label's entry is g (1 - p_label) = - g expm1(logprob), taken from the forward's result
+    // (exact also where p_label is close to 1) and written over the entry that the sweep below
+    // leaves there: the sweep itself then treats all entries alike.
+    const int rel = (live && y >= m0 && y < m0 + BM) ? (int)(y - m0) - wave_row0 : -1;
+    const bool mine = rel >= 0 && rel < 64 && (((rel & 31) >> 2) & 1) == (lane >> 5);
+    const float ng = -g;
+    auto sweep = [&](auto last_tile_tag) {
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                float d[4];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const int r = q * 4 + e;
+                    float val = ng * __builtin_amdgcn_exp2f(fmaf(i == 0 ? z0[r] : z1[r], in.c, -l2));
+                    if (decltype(last_tile_tag)::value && acc_row(wm, i, r, lane) >= rows_left) val = 0.f;
+                    d[e] = val;
+                }
+                const int vl = acc_row(wm, i, q * 4, lane) ^ (row_bit3 << 2);
+                uint2 pk = make_uint2(oi_pack_bf16x2(d[0], d[1]), oi_pack_bf16x2(d[2], d[3]));
+                *reinterpret_cast<uint2*>(srow + vl) = pk;
+            }
+    };
+    if (rows_left < BM) sweep(std::true_type{});  // the last vocabulary tile: rows past the vocabulary hold 0
+    else sweep(std::false_type{});
+    if (mine) {
+        // same lane, same LDS word as the store above: program order keeps them apart
+        const float val = ng * expm1f(in.logprob[n]);
+        srow[(wave_row0 + rel) ^ (row_bit3 << 2)] = (uint16_t)oi_f32_to_bf16_bits(val);
+    }
+}
+
 __device__ __forceinline__ void lmhead_dz_tile(const uint16_t* __restrict__ W, const uint16_t* __restrict__ hidden,
-                                               const int64_t* __restrict__ labels, const float* __restrict__ lse,
-                                               const float* __restrict__ grad, const float* __restrict__ logprob,
-                                               int64_t n_tokens, int64_t hdim, int64_t vocab, float c, float inv_t,
-                                               int64_t v_begin, int64_t chunk_cols, int64_t n_pad,
+                                               const DzInputs& in, int64_t hdim, int64_t v_begin, int64_t chunk_cols,
                                                uint16_t* __restrict__ dz, int64_t vt, int64_t tt, uint16_t* lds) {
     const int tid = opaque_tid(), lane = tid & 63, wave = tid >> 6, wm = wave & 3, wn = wave >> 2;
     const int64_t n0 = tt * BN, m0 = v_begin + vt * BM;
 
     AccTile acc;
-    gemm_tile(acc, W, hdim, m0, vocab, hidden, hdim, n0, n_tokens, hdim, lds);
+    gemm_tile(acc, W, hdim, m0, in.vocab, hidden, hdim, n0, in.n_tokens, hdim, lds);
 
-    // stage[n][v]: rows = tokens of the tile, 256 (+8 pad) vocabulary columns.  A lane stores 8 bytes
-    // (4 vocabulary entries of one token) and consecutive lanes store to consecutive rows, 132 words
-    // apart: the stores of rows 8 apart meet on the same banks (measured: 1000 conflict cycles per
-    // tile).  Rows 8..15 of every 16 therefore swap the two 8-byte halves of each 16-byte piece
-    // (0 conflict cycles); the copy-out swaps them back.
     uint16_t* stage = lds;
-    const int rows_left = (int)(vocab - m0 < BM ? vocab - m0 : BM);  // real vocabulary rows of the tile
-    const int wave_row0 = wm * 64;
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
         const int nl = acc_col(wn, j, lane);
-        const int64_t n = n0 + nl;
-        const bool live = n < n_tokens;
-        const float g = live ? grad[n] * inv_t : 0.f;
-        // a token without gradient gets an exponent of -huge: every entry becomes -0 * 0
-        const float l2 = g != 0.f ? lse[n] * OI_LOG2E : 3.0e38f;
-        int64_t y = live ? labels[n] : -1;
-        if (live) y = y < 0 ? 0 : (y >= vocab ? vocab - 1 : y);
-        // The label's entry is g (1 - p_label) = - g expm1(logprob), taken from the forward's result
-        // (exact also where p_label is close to 1) and written over the entry that the sweep below
-        // leaves there: the sweep itself then treats all entries alike.
-        const int rel = (live && y >= m0 && y < m0 + BM) ? (int)(y - m0) - wave_row0 : -1;
-        const bool mine = rel >= 0 && rel < 64 && (((rel & 31) >> 2) & 1) == (lane >> 5);
-        const float ng = -g;
-        auto sweep = [&](auto last_tile_tag) {
-#pragma unroll
-            for (int i = 0; i < 2; ++i)
-#pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                    float d[4];
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) {
-                        const int r = q * 4 + e;
-                        float val = ng * __builtin_amdgcn_exp2f(fmaf(acc[i][j][r], c, -l2));
-                        if (decltype(last_tile_tag)::value && acc_row(wm, i, r, lane) >= rows_left) val = 0.f;
-                        d[e] = val;
-                    }
-                    const int vl = acc_row(wm, i, q * 4, lane) ^ (((nl >> 3) & 1) << 2);
-                    uint2 pk = make_uint2(oi_pack_bf16x2(d[0], d[1]), oi_pack_bf16x2(d[2], d[3]));
-                    *reinterpret_cast<uint2*>(stage + nl * STAGE_STRIDE + vl) = pk;
-                }
-        };
-        if (rows_left < BM) sweep(std::true_type{});  // the last vocabulary tile: rows past the vocabulary hold 0
-        else sweep(std::false_type{});
-        if (mine) {
-            // same lane, same LDS word as the store above: program order keeps them apart
-            const float val = ng * expm1f(logprob[n]);
-            stage[nl * STAGE_STRIDE + ((wave_row0 + rel) ^ (((nl >> 3) & 1) << 2))] = (uint16_t)oi_f32_to_bf16_bits(val);
-        }
+        dz_column(acc[0][j], acc[1][j], in, n0 + nl, m0, wm, lane, stage + nl * STAGE_STRIDE, (nl >> 3) & 1);
     }
     __syncthreads();
     const int64_t vcol0 = vt * BM;  // column of this tile inside the chunk
@@ -858,21 +894,56 @@ __device__ __forceinline__ void lmhead_dz_tile(const uint16_t* __restrict__ W, c
 }
 
 __global__ void __launch_bounds__(NTHREADS)
-    lmhead_dz_kernel(const uint16_t* __restrict__ W, const uint16_t* __restrict__ hidden,
-                     const int64_t* __restrict__ labels, const float* __restrict__ lse,
-                     const float* __restrict__ grad, const float* __restrict__ logprob, int64_t n_tokens,
-                     const int32_t* __restrict__ n_dev, int64_t hdim, int64_t vocab, float c, float inv_t,
-                     int64_t v_begin, int64_t chunk_cols, int64_t n_pad, uint16_t* __restrict__ dz,
-                     uint32_t* __restrict__ queue) {
+    lmhead_dz_kernel(const uint16_t* __restrict__ W, const uint16_t* __restrict__ hidden, DzInputs in,
+                     const int32_t* __restrict__ n_dev, int64_t hdim, int64_t v_begin, int64_t chunk_cols, int64_t n_pad,
+                     uint16_t* __restrict__ dz, uint32_t* __restrict__ queue) {
     __shared__ __align__(16) uint16_t lds[LDS_ELEMS];
     if (n_dev) {
-        n_tokens = *n_dev;
-        n_pad = (n_tokens + BN - 1) / BN * BN;
+        in.n_tokens = *n_dev;
+        n_pad = (in.n_tokens + BN - 1) / BN * BN;
     }
     for_each_tile(queue, chunk_cols / BM, n_pad / BN, lds, [&](int64_t vt, int64_t tt) {
-        lmhead_dz_tile(W, hidden, labels, lse, grad, logprob, n_tokens, hdim, vocab, c, inv_t, v_begin, chunk_cols, n_pad, dz,
-                       vt, tt, lds);
+        lmhead_dz_tile(W, hidden, in, hdim, v_begin, chunk_cols, dz, vt, tt, lds);
     });
+}
+
+// The same dZ (to the bit) from the logits that the forward left behind as fp32 tiles, whole vocabulary at
+// once.  Workgroup (j, tt, vt) takes column group j of tile (vt, tt): 64 tokens (wn * 128 + j * 32 + 0..31 of
+// both wn halves) x 256 vocabulary columns, 64 KB in and 32 KB out.  A quarter of a tile per workgroup so that
+// four of them share a CU and one's stores run beside another's loads.
+constexpr int KEPT_ROWS = 64;
+__global__ void __launch_bounds__(NTHREADS)
+    lmhead_dz_kept_kernel(const float* __restrict__ logits, int64_t logits_tiles, DzInputs in,
+                          const int32_t* __restrict__ n_dev, int64_t cols, uint16_t* __restrict__ dz) {
+    __shared__ __align__(16) uint16_t stage[KEPT_ROWS * STAGE_STRIDE];
+    if (n_dev) in.n_tokens = *n_dev;
+    const int j = blockIdx.x & 3;
+    const int64_t tt = blockIdx.x >> 2, vt = blockIdx.y, n0 = tt * BN;
+    if (n0 >= in.n_tokens) return;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, wm = wave & 3, wn = wave >> 2;
+    const float* tile = logits + (vt * logits_tiles + tt) * PART_FLOATS;
+    oi_f32x4 z4[2][4];
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+            z4[i][q] = *reinterpret_cast<const oi_f32x4*>(tile + part_group(i, j, q) * PART_GROUP + tid * 4);
+    f32x16 z[2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) z[i][r] = z4[i][r >> 2][r & 3];
+    const int row = wn * 32 + (lane & 31);
+    dz_column(z[0], z[1], in, n0 + acc_col(wn, j, lane), vt * BM, wm, lane, stage + row * STAGE_STRIDE, (row >> 3) & 1);
+    __syncthreads();
+#pragma unroll
+    for (int it = 0; it < KEPT_ROWS * (BM / 8) / NTHREADS; ++it) {
+        const int cidx = tid + it * NTHREADS;
+        const int r = cidx >> 5, ch = cidx & 31;
+        oi_u32x4 v = *reinterpret_cast<const oi_u32x4*>(stage + r * STAGE_STRIDE + ch * 8);
+        if (r & 8) v = oi_u32x4{v.z, v.w, v.x, v.y};
+        *reinterpret_cast<oi_u32x4*>(dz + (n0 + (r >> 5) * 128 + j * 32 + (r & 31)) * cols + vt * BM + ch * 8) = v;
+    }
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -1002,21 +1073,6 @@ __device__ __forceinline__ void store_block(const StoreTo& st, const LaneRows& r
                     make_uint2(oi_pack_bf16x2(v[0], v[1]), oi_pack_bf16x2(v[2], v[3]));
         }
     }
-}
-
-// A piece of a tile product that is one of several along k: the fp32 tile in the order in which the
-// accumulators lie in the registers (16 bytes per lane, consecutive lanes together).
-constexpr int PART_FLOATS = BM * BN;
-__device__ __forceinline__ void store_part(const AccTile& acc, float* part, int tid) {
-    asm volatile("" : "+v"(tid));
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-#pragma unroll
-            for (int q = 0; q < 4; ++q)
-                *reinterpret_cast<oi_f32x4*>(part + (((i * 4 + j) * 4 + q) * NTHREADS + tid) * 4) =
-                    oi_f32x4{acc[i][j][q * 4], acc[i][j][q * 4 + 1], acc[i][j][q * 4 + 2], acc[i][j][q * 4 + 3]};
 }
 
 // A, B: operands without their tile origin (r0 is filled in here).  K == 0 stores zeros.  With `part`
@@ -1578,12 +1634,13 @@ SelectionPlan plan_selection(Carver& cv, int64_t n_pad, int64_t hdim, bool backw
     return p;
 }
 
-// Where the forward leaves the exponentials it computes anyway (all null / 0: nowhere)
+// Where the forward leaves the exponentials it computes anyway, or its logits (all null / 0: nowhere)
 struct KeepPlan {
     uint16_t* buf;        // bf16 [n_pad, ld], token-major
     int64_t ld, tiles;    // columns of the buffer, and as vocabulary tiles
     const float* xref;    // per token: the exponent the kept numbers are relative to
     uint8_t* unsafe;      // per caller row: set when the kept numbers of that token cannot be used
+    float* logits;        // or the fp32 logits themselves, tile by tile (buf null)
 };
 
 struct FwdPlan {
@@ -1633,6 +1690,18 @@ FwdPlan plan_fwd(int64_t n_tokens, int64_t hdim, int64_t vocab, bool with_select
     if (with_selection) p.sel = plan_selection(cv, p.n_pad, hdim, false);
     p.total = cv.off;
     return p;
+}
+
+// Bytes of the forward's logits, tile by tile, for a backward that reads them instead of computing them
+// again; 0 where they are not to be kept.  Keeping them takes the recomputation (a quarter of the matrix
+// work of a step with a trained head) out of the step and costs 4 bytes per row and column between the passes:
+// cross-entropy of 3072 rows, hidden 4096, vocabulary 128256: dZ 2460 -> 430 us (5.5 TB/s), forward 2350 -> 2770 us
+// with its stores, step 10.9 -> 8.65 ms.  The line is where the recomputing backward begins to take the vocabulary in chunks, i.e. 4 GiB: a larger batch is a
+// large part of a card's memory, and its step is better made slab by slab.
+size_t kept_bytes(int64_t n_tokens, int64_t vocab) {
+    const int64_t n_pad = round_up(n_tokens, BN), v_pad = round_up(vocab, BM);
+    if (v_pad > CHUNK_BUDGET / n_pad / 1024 * 1024) return 0;
+    return (size_t)n_pad * v_pad * sizeof(float);
 }
 
 struct BwdPlan {
@@ -1736,13 +1805,16 @@ void enqueue_fwd(const FwdPlan& p, char* ws, const RowInputs& in, const uint8_t*
     const dim3 grid(resident_grid(p.n_splits, p.token_tiles));
     const uint16_t* Wp = static_cast<const uint16_t*>(weight);
     const FwdLaunch fl = {p.tiles_per_split, p.long_splits, 0, p.long_splits, p.n_splits - p.long_splits,
-                          keep.buf, keep.ld, 0, keep.buf ? keep.tiles : 0, 0, keep.xref};
+                          keep.buf, keep.ld, 0, keep.buf ? keep.tiles : 0, 0, keep.xref, keep.logits, p.token_tiles};
     if (keep.buf) {
         const ProbeScope probe(0, s);
-        hipLaunchKernelGGL(lmhead_fwd_kernel<true>, grid, dim3(NTHREADS), 0, s, Wp, in.hidden, in.labels, n_tokens,
+        hipLaunchKernelGGL(lmhead_fwd_kernel<FWD_EXPONENTIALS>, grid, dim3(NTHREADS), 0, s, Wp, in.hidden, in.labels, n_tokens,
                            in.n_dev, hidden_dim, vocab, c, fl, p.n_pad, partial, zy, queue);
-    } else
-        hipLaunchKernelGGL(lmhead_fwd_kernel<false>, grid, dim3(NTHREADS), 0, s, Wp, in.hidden, in.labels, n_tokens,
+    } else if (keep.logits)
+        hipLaunchKernelGGL(lmhead_fwd_kernel<FWD_LOGITS>, grid, dim3(NTHREADS), 0, s, Wp, in.hidden, in.labels, n_tokens,
+                           in.n_dev, hidden_dim, vocab, c, fl, p.n_pad, partial, zy, queue);
+    else
+        hipLaunchKernelGGL(lmhead_fwd_kernel<FWD_PLAIN>, grid, dim3(NTHREADS), 0, s, Wp, in.hidden, in.labels, n_tokens,
                            in.n_dev, hidden_dim, vocab, c, fl, p.n_pad, partial, zy, queue);
     hipLaunchKernelGGL(lmhead_fwd_combine_kernel, dim3((unsigned)((n_tokens + COMBINE_TOKENS - 1) / COMBINE_TOKENS)),
                        dim3(COMBINE_THREADS), 0, s, partial,
@@ -1800,8 +1872,8 @@ void enqueue_fwd_wsum(const FwdPlan& p, char* ws, const RowInputs& in, const uin
         const int64_t n_first = p.n_splits - first < splits_per_chunk ? p.n_splits - first : splits_per_chunk;
         uint32_t* q = queues + ci * (FWD_QUEUE_WORDS + QUEUE_WORDS);
         const FwdLaunch fl = {p.tiles_per_split, p.long_splits, first, n_first, 0, chunk_buf, cols, v_begin / BM,
-                              cols / BM, 1, xref};
-        hipLaunchKernelGGL(lmhead_fwd_kernel<true>, dim3(resident_grid(n_first, p.token_tiles)), dim3(NTHREADS), 0, s, Wp,
+                              cols / BM, 1, xref, nullptr, 0};
+        hipLaunchKernelGGL(lmhead_fwd_kernel<FWD_EXPONENTIALS>, dim3(resident_grid(n_first, p.token_tiles)), dim3(NTHREADS), 0, s, Wp,
                            in.hidden, in.labels, n_tokens, in.n_dev, hidden_dim, vocab, c, fl, p.n_pad, partial, zy, q);
         const Operand a = {chunk_buf, cols, 0, p.n_pad, cols};
         const Operand b = {Wp + v_begin * hidden_dim, hidden_dim, 0, hidden_dim, valid};
@@ -1860,13 +1932,15 @@ __global__ void __launch_bounds__(256)
 // first call's product (0) and adds the following ones (1; a call without tokens adds nothing and
 // costs nothing); the caller rounds dw32 to bf16 when the last call is through.  4: the product is
 // added to bf16 rows that an earlier call wrote.
+// logits: the forward's logits (kept_bytes), read instead of recomputed.
 // max_grid > 0 caps the number of resident workgroups of every launch (the queues work with any
 // number): the launches that serve flagged rows normally find none, and a launch over a few CUs that
 // finds nothing costs a fraction of one over all of them.
 constexpr unsigned REPAIR_GRID = 32;
 void enqueue_bwd(const BwdPlan& p, char* ws, const RowInputs& in, const void* weight, int64_t n_tokens,
                  int64_t hidden_dim, int64_t vocab, float inv_temperature, void* d_hidden, void* d_weight,
-                 hipStream_t s, int dw_mode = 2, float* dw32 = nullptr, unsigned max_grid = 0) {
+                 hipStream_t s, int dw_mode = 2, float* dw32 = nullptr, unsigned max_grid = 0,
+                 const float* logits = nullptr) {
     auto grid_of = [&](int64_t tiles_m, int64_t tiles_n) {
         const unsigned g = resident_grid(tiles_m, tiles_n);
         return dim3(max_grid > 0 && g > max_grid ? max_grid : g);
@@ -1884,9 +1958,13 @@ void enqueue_bwd(const BwdPlan& p, char* ws, const RowInputs& in, const void* we
         const int64_t cols = v_end - v_begin;                                   // multiple of 256
         const int64_t valid = vocab - v_begin < cols ? vocab - v_begin : cols;  // real rows of W
         uint32_t* q = queues + ci * 3 * QUEUE_WORDS;
-        hipLaunchKernelGGL(lmhead_dz_kernel, grid_of(cols / BM, p.n_pad / BN), dim3(NTHREADS), 0, s, Wp,
-                           in.hidden, in.labels, in.lse, in.grad, in.logprob, n_tokens, in.n_dev, hidden_dim, vocab, c,
-                           inv_temperature, v_begin, cols, p.n_pad, dz, q);
+        const DzInputs di = {in.labels, in.lse, in.grad, in.logprob, n_tokens, vocab, c, inv_temperature};
+        if (logits)
+            hipLaunchKernelGGL(lmhead_dz_kept_kernel, dim3((unsigned)(p.n_pad / BN * 4), (unsigned)(cols / BM)),
+                               dim3(NTHREADS), 0, s, logits, p.n_pad / BN, di, in.n_dev, cols, dz);
+        else
+            hipLaunchKernelGGL(lmhead_dz_kernel, grid_of(cols / BM, p.n_pad / BN), dim3(NTHREADS), 0, s, Wp, in.hidden, di,
+                               in.n_dev, hidden_dim, v_begin, cols, p.n_pad, dz, q);
         const bool first = ci == 0, last = ci == p.n_chunks - 1;
         const int mode = last ? (first ? 2 : 3) : (first ? 0 : 1);
         {
@@ -2126,7 +2204,7 @@ int run_slab_passes(const SlabPlan& p, char* ws, const SlabStep& st, hipStream_t
                            static_cast<float*>(nullptr), static_cast<float*>(nullptr), static_cast<float*>(nullptr));
         const RowInputs in = {hidden_s, labels_s, nullptr, nullptr, rows_s, cnt, nullptr};
         launch_label_ref(in, st.weight, p.cap, hdim, vocab, st.inv_temperature, xref_s, s);
-        const KeepPlan keep = {keep_buf, p.v_pad, p.v_pad / BM, xref_s, unsafe};
+        const KeepPlan keep = {keep_buf, p.v_pad, p.v_pad / BM, xref_s, unsafe, nullptr};
         // the forward's own queue words are the first FWD_QUEUE_WORDS of `queues`
         FwdPlan fp = p.fwd;
         fp.off_queue = (size_t)(reinterpret_cast<char*>(queues) - ws_fwd);
@@ -2168,15 +2246,11 @@ extern "C" size_t oi_lmhead_fwd_workspace_bytes(int64_t n_tokens, int64_t hidden
     return plan_fwd(n_tokens, hidden_dim, vocab, with_row_mask != 0).total;
 }
 
-extern "C" int oi_lmhead_logp_fwd(const void* hidden, const void* weight, const int64_t* labels,
-                                  const uint8_t* row_mask, int64_t n_tokens, int64_t hidden_dim, int64_t vocab,
-                                  float inv_temperature, float* logprob, float* entropy, float* lse, void* workspace,
-                                  size_t workspace_bytes, void* stream) {
-    int rc = check_lmhead(hidden, weight, labels, n_tokens, hidden_dim, vocab, inv_temperature);
-    if (rc != OI_OK) return rc;
-    if (n_tokens == 0) return OI_OK;
-    OI_RETURN_IF(!logprob || !workspace, OI_ENULL);
-    OI_RETURN_IF(!oi_aligned(workspace, 256), OI_EALIGN);
+namespace {
+// `logits`: null, or kept_bytes of memory for the backward that follows
+int lmhead_forward(const void* hidden, const void* weight, const int64_t* labels, const uint8_t* row_mask,
+                   int64_t n_tokens, int64_t hidden_dim, int64_t vocab, float inv_temperature, float* logprob,
+                   float* entropy, float* lse, float* logits, void* workspace, size_t workspace_bytes, void* stream) {
     const FwdPlan p = plan_fwd(n_tokens, hidden_dim, vocab, row_mask != nullptr);
     OI_RETURN_IF(workspace_bytes < p.total, OI_EWORKSPACE);
     char* ws = static_cast<char*>(workspace);
@@ -2188,9 +2262,44 @@ extern "C" int oi_lmhead_logp_fwd(const void* hidden, const void* weight, const 
                               FWD_QUEUE_WORDS, s);
     else
         hipLaunchKernelGGL(zero_words_kernel, dim3(1), dim3(64), 0, s, queue, FWD_QUEUE_WORDS);
-    enqueue_fwd(p, ws, in, row_mask, weight, n_tokens, hidden_dim, vocab, inv_temperature, logprob, entropy, lse,
-                KeepPlan{nullptr, 0, 0, nullptr, nullptr}, s);
+    KeepPlan keep = {};
+    keep.logits = logits;
+    enqueue_fwd(p, ws, in, row_mask, weight, n_tokens, hidden_dim, vocab, inv_temperature, logprob, entropy, lse, keep, s);
     return oi_launch_status();
+}
+}  // namespace
+
+extern "C" int oi_lmhead_logp_fwd(const void* hidden, const void* weight, const int64_t* labels,
+                                  const uint8_t* row_mask, int64_t n_tokens, int64_t hidden_dim, int64_t vocab,
+                                  float inv_temperature, float* logprob, float* entropy, float* lse, void* workspace,
+                                  size_t workspace_bytes, void* stream) {
+    int rc = check_lmhead(hidden, weight, labels, n_tokens, hidden_dim, vocab, inv_temperature);
+    if (rc != OI_OK) return rc;
+    if (n_tokens == 0) return OI_OK;
+    OI_RETURN_IF(!logprob || !workspace, OI_ENULL);
+    OI_RETURN_IF(!oi_aligned(workspace, 256), OI_EALIGN);
+    return lmhead_forward(hidden, weight, labels, row_mask, n_tokens, hidden_dim, vocab, inv_temperature, logprob, entropy,
+                          lse, nullptr, workspace, workspace_bytes, stream);
+}
+
+extern "C" size_t oi_lmhead_kept_bytes(int64_t n_tokens, int64_t vocab) {
+    if (n_tokens <= 0 || vocab <= 0 || n_tokens > MAX_LD || vocab > MAX_LD) return 0;
+    return kept_bytes(n_tokens, vocab);
+}
+
+extern "C" int oi_lmhead_logp_fwd_kept(const void* hidden, const void* weight, const int64_t* labels,
+                                       const uint8_t* row_mask, int64_t n_tokens, int64_t hidden_dim, int64_t vocab,
+                                       float inv_temperature, float* logprob, float* entropy, float* lse, float* logits,
+                                       size_t logits_bytes, void* workspace, size_t workspace_bytes, void* stream) {
+    int rc = check_lmhead(hidden, weight, labels, n_tokens, hidden_dim, vocab, inv_temperature);
+    if (rc != OI_OK) return rc;
+    if (n_tokens == 0) return OI_OK;
+    OI_RETURN_IF(!logprob || !lse || !logits || !workspace, OI_ENULL);
+    OI_RETURN_IF(!oi_aligned(workspace, 256) || !oi_aligned(logits, 16), OI_EALIGN);
+    const size_t need = kept_bytes(n_tokens, vocab);
+    OI_RETURN_IF(need == 0 || logits_bytes < need, OI_EWORKSPACE);
+    return lmhead_forward(hidden, weight, labels, row_mask, n_tokens, hidden_dim, vocab, inv_temperature, logprob, entropy,
+                          lse, logits, workspace, workspace_bytes, stream);
 }
 
 extern "C" size_t oi_lmhead_fwd_wsum_workspace_bytes(int64_t n_tokens, int64_t hidden_dim, int64_t vocab,
@@ -2303,11 +2412,12 @@ extern "C" size_t oi_lmhead_bwd_workspace_bytes(int64_t n_tokens, int64_t hidden
     return plan_bwd(n_tokens, hidden_dim, vocab, with_row_selection != 0).total;
 }
 
-extern "C" int oi_lmhead_logp_bwd(const void* hidden, const void* weight, const int64_t* labels, const float* lse,
-                                  const float* grad_logprob, const uint8_t* row_mask, int skip_zero_grad_rows,
-                                  int64_t n_tokens, int64_t hidden_dim, int64_t vocab, float inv_temperature,
-                                  const float* logprob, void* d_hidden, void* d_weight, void* workspace,
-                                  size_t workspace_bytes, void* stream) {
+namespace {
+// `logits`: null, or what the forward over the same rows (the same mask, no rows skipped) left behind
+int lmhead_backward(const void* hidden, const void* weight, const int64_t* labels, const float* lse,
+                    const float* grad_logprob, const uint8_t* row_mask, int skip_zero_grad_rows, int64_t n_tokens,
+                    int64_t hidden_dim, int64_t vocab, float inv_temperature, const float* logprob, const float* logits,
+                    void* d_hidden, void* d_weight, void* workspace, size_t workspace_bytes, void* stream) {
     int rc = check_lmhead(hidden, weight, labels, n_tokens, hidden_dim, vocab, inv_temperature);
     if (rc != OI_OK) return rc;
     if (n_tokens == 0) return OI_OK;
@@ -2334,9 +2444,37 @@ extern "C" int oi_lmhead_logp_bwd(const void* hidden, const void* weight, const 
         hipLaunchKernelGGL(zero_unselected_rows_kernel, dim3((unsigned)n_tokens), dim3(256), 0, s, row_mask,
                            zero_grad_probe, hidden_dim, static_cast<uint16_t*>(d_hidden));
     }
-    enqueue_bwd(p, ws, in, weight, n_tokens, hidden_dim, vocab, inv_temperature, d_hidden, d_weight, s);
+    enqueue_bwd(p, ws, in, weight, n_tokens, hidden_dim, vocab, inv_temperature, d_hidden, d_weight, s, 2,
+                nullptr, 0, logits);
     return oi_launch_status();
 }
+}  // namespace
+
+extern "C" int oi_lmhead_logp_bwd(const void* hidden, const void* weight, const int64_t* labels, const float* lse,
+                                  const float* grad_logprob, const uint8_t* row_mask, int skip_zero_grad_rows,
+                                  int64_t n_tokens, int64_t hidden_dim, int64_t vocab, float inv_temperature,
+                                  const float* logprob, void* d_hidden, void* d_weight, void* workspace,
+                                  size_t workspace_bytes, void* stream) {
+    return lmhead_backward(hidden, weight, labels, lse, grad_logprob, row_mask, skip_zero_grad_rows, n_tokens, hidden_dim,
+                           vocab, inv_temperature, logprob, nullptr, d_hidden, d_weight, workspace, workspace_bytes,
+                           stream);
+}
+
+extern "C" int oi_lmhead_logp_bwd_kept(const void* hidden, const void* weight, const int64_t* labels, const float* lse,
+                                       const float* grad_logprob, const uint8_t* row_mask, int64_t n_tokens,
+                                       int64_t hidden_dim, int64_t vocab, float inv_temperature, const float* logprob,
+                                       const float* logits, size_t logits_bytes, void* d_hidden, void* d_weight,
+                                       void* workspace, size_t workspace_bytes, void* stream) {
+    if (n_tokens > 0) {
+        OI_RETURN_IF(!logits, OI_ENULL);
+        OI_RETURN_IF(!oi_aligned(logits, 16), OI_EALIGN);
+        const size_t need = oi_lmhead_kept_bytes(n_tokens, vocab);
+        OI_RETURN_IF(need == 0 || logits_bytes < need, OI_EWORKSPACE);
+    }
+    return lmhead_backward(hidden, weight, labels, lse, grad_logprob, row_mask, 0, n_tokens, hidden_dim, vocab,
+                           inv_temperature, logprob, logits, d_hidden, d_weight, workspace, workspace_bytes, stream);
+}
+
 
 extern "C" size_t oi_lmhead_grpo_workspace_bytes(int64_t rows, int64_t cols, int64_t hidden_dim, int64_t vocab,
                                                  int want_d_weight, int64_t slab_tokens) {
@@ -2440,7 +2578,7 @@ extern "C" int oi_lmhead_grpo_fwd_bwd(const void* hidden, const void* weight, co
     RowInputs in = launch_selection(p.bwd.sel, ws_bwd, hidden, labels, nullptr, nullptr, mask, false, n_tokens,
                                     hidden_dim, bwd_queues, select_clears_queues ? n_queue_words : 0, s);
     enqueue_fwd(p.fwd, ws_fwd, in, mask, weight, n_tokens, hidden_dim, vocab, inv_temperature, logprob, entropy, lse,
-                KeepPlan{nullptr, 0, 0, nullptr, nullptr}, s);
+                KeepPlan{}, s);
 
     // loss and statistics from the logprobs, then every token's d loss / d logprob (upstream gradient 1)
     rc = oi_grpo_fused_fwd(logprob, old_logprobs, ref_logprobs, advantages, mask, rho_weights, entropy, nullptr, nullptr,

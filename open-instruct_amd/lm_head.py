@@ -20,7 +20,7 @@ from . import _lib
 class _FusedLMHead(torch.autograd.Function):
     @staticmethod
     def forward(ctx, hidden, weight, labels, mask, inv_temperature, want_entropy, compact_backward=False,
-                dhidden_in_forward="auto"):
+                dhidden_in_forward="auto", keep_logits=False):
         dev = _lib.require_gpu(hidden, weight, labels, mask)
         if hidden.dtype != torch.bfloat16 or weight.dtype != torch.bfloat16:
             raise ValueError("fused lm_head expects bf16 hidden states and weight")
@@ -48,7 +48,7 @@ class _FusedLMHead(torch.autograd.Function):
         wsum_mode = bool(dhidden_in_forward) and ctx.needs_input_grad[0] and not ctx.needs_input_grad[1] and n > 0
         if wsum_mode and compact_backward:
             raise ValueError("dhidden_in_forward cannot be combined with compact_backward")
-        wsum = xref = unsafe = None
+        wsum = xref = unsafe = logits = None
         if wsum_mode:
             lib = _lib.load()
             wsum = torch.empty(n, h, dtype=torch.float32, device=dev)
@@ -65,12 +65,21 @@ class _FusedLMHead(torch.autograd.Function):
             lib = _lib.load()
             ws_bytes = lib.oi_lmhead_fwd_workspace_bytes(n, h, v, int(m is not None))
             ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
-            _lib.call(
-                "oi_lmhead_logp_fwd", hid.data_ptr(), w.data_ptr(), lab.data_ptr(), _lib.ptr(m), n, h, v,
-                inv_temperature, logprob.data_ptr(), _lib.ptr(entropy), lse.data_ptr(), ws.data_ptr(), ws_bytes,
-                _lib.stream_of(hid),
-            )  # fmt: skip
-        ctx.save_for_backward(hid, w, lab, lse, m, logprob, wsum, xref, unsafe)
+            if keep_logits and ctx.needs_input_grad[1] and not compact_backward:
+                logits = _kept_logits(n, v, dev)
+            if logits is not None:
+                _lib.call(
+                    "oi_lmhead_logp_fwd_kept", hid.data_ptr(), w.data_ptr(), lab.data_ptr(), _lib.ptr(m), n, h, v,
+                    inv_temperature, logprob.data_ptr(), _lib.ptr(entropy), lse.data_ptr(), logits.data_ptr(),
+                    logits.numel() * 4, ws.data_ptr(), ws_bytes, _lib.stream_of(hid),
+                )  # fmt: skip
+            else:
+                _lib.call(
+                    "oi_lmhead_logp_fwd", hid.data_ptr(), w.data_ptr(), lab.data_ptr(), _lib.ptr(m), n, h, v,
+                    inv_temperature, logprob.data_ptr(), _lib.ptr(entropy), lse.data_ptr(), ws.data_ptr(), ws_bytes,
+                    _lib.stream_of(hid),
+                )  # fmt: skip
+        ctx.save_for_backward(hid, w, lab, lse, m, logprob, wsum, xref, unsafe, logits)
         ctx.inv_temperature = inv_temperature
         ctx.compact_backward = bool(compact_backward)
         if want_entropy:
@@ -79,12 +88,12 @@ class _FusedLMHead(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, grad_logprob, _grad_entropy):
-        hid, w, lab, lse, m, logprob, wsum, xref, unsafe = ctx.saved_tensors
+        hid, w, lab, lse, m, logprob, wsum, xref, unsafe, logits = ctx.saved_tensors
         n, h = hid.shape
         v = w.shape[0]
         need_h, need_w = ctx.needs_input_grad[0], ctx.needs_input_grad[1]
         if grad_logprob is None or not (need_h or need_w):
-            return (None,) * 8
+            return (None,) * 9
         g = _lib.f32c(grad_logprob)
         d_hidden = torch.empty_like(hid)
         if wsum is not None:
@@ -95,12 +104,19 @@ class _FusedLMHead(torch.autograd.Function):
                 logprob.data_ptr(), g.data_ptr(), _lib.ptr(m), wsum.data_ptr(), xref.data_ptr(), unsafe.data_ptr(), n, h,
                 v, ctx.inv_temperature, d_hidden.data_ptr(), ws.data_ptr(), ws_bytes, _lib.stream_of(hid),
             )  # fmt: skip
-            return (d_hidden,) + (None,) * 7
+            return (d_hidden,) + (None,) * 8
         d_weight = torch.empty_like(w) if need_w else None
         if n > 0:
             selecting = m is not None or ctx.compact_backward
             ws_bytes = _lib.load().oi_lmhead_bwd_workspace_bytes(n, h, v, int(need_w), int(selecting))
             ws = torch.empty(ws_bytes, dtype=torch.uint8, device=hid.device)
+            if logits is not None:
+                _lib.call(
+                    "oi_lmhead_logp_bwd_kept", hid.data_ptr(), w.data_ptr(), lab.data_ptr(), lse.data_ptr(), g.data_ptr(),
+                    _lib.ptr(m), n, h, v, ctx.inv_temperature, logprob.data_ptr(), logits.data_ptr(), logits.numel() * 4,
+                    d_hidden.data_ptr(), _lib.ptr(d_weight), ws.data_ptr(), ws_bytes, _lib.stream_of(hid),
+                )  # fmt: skip
+                return (d_hidden if need_h else None), d_weight, None, None, None, None, None, None, None
             _lib.call(
                 "oi_lmhead_logp_bwd", hid.data_ptr(), w.data_ptr(), lab.data_ptr(), lse.data_ptr(), g.data_ptr(),
                 _lib.ptr(m), int(ctx.compact_backward), n, h, v, ctx.inv_temperature, _lib.ptr(logprob),
@@ -108,7 +124,19 @@ class _FusedLMHead(torch.autograd.Function):
             )  # fmt: skip
         elif d_weight is not None:
             d_weight.zero_()
-        return (d_hidden if need_h else None), d_weight, None, None, None, None, None, None
+        return (d_hidden if need_h else None), d_weight, None, None, None, None, None, None, None
+
+
+def _kept_logits(n, v, dev):
+    """Memory for the forward's logits where they are kept for the backward, else None (the backward then
+    computes them again, with the same results): too many of them, or none of that size to be had."""
+    kept = _lib.load().oi_lmhead_kept_bytes(n, v)
+    if not kept:
+        return None
+    try:
+        return torch.empty(kept // 4, dtype=torch.float32, device=dev)
+    except torch.cuda.OutOfMemoryError:
+        return None
 
 
 def fused_lm_head_logprobs(
@@ -134,8 +162,10 @@ def fused_lm_head_logprobs(
     upstream gradient is exactly zero (zero-advantage completions, clipped ratios without a KL
     term) out of the backward products; it changes no result.
 
-    Nothing of size ``[tokens, vocab]`` ever exists.  When ``weight`` takes a gradient the backward
-    recomputes the logits one vocabulary chunk at a time (for a step without that recomputation see
+    When ``weight`` takes a gradient the forward of a small batch keeps its logits for the backward (fp32, at most
+    4 GiB: 8192 rows at a vocabulary of 131072; memory permitting).  Above that nothing of size
+    ``[tokens, vocab]`` ever exists: the backward recomputes the logits one vocabulary chunk at a time, with the
+    same results (for a step of any size without that recomputation see
     :func:`open_instruct_amd.grpo_utils.grpo_loss_on_hidden` and
     :func:`open_instruct_amd.dpo_utils.dpo_loss_on_hidden`, which know the loss and can therefore
     finish a slab of tokens before they start the next).
@@ -163,8 +193,9 @@ def fused_lm_head_logprobs(
         dhidden_in_forward = not compact_backward
     # without a backward pass to come (torch.no_grad(): scoring passes, the reference-logprob cache) there is
     # nothing to prepare; inside an autograd Function the grad mode is off, so it is read here
-    dhidden_in_forward = bool(dhidden_in_forward) and torch.is_grad_enabled()
-    lp, ent = _FusedLMHead.apply(hid2, weight, lab1, mask, inv_t, return_entropy, compact_backward, dhidden_in_forward)
+    grad = torch.is_grad_enabled()
+    dhidden_in_forward = bool(dhidden_in_forward) and grad
+    lp, ent = _FusedLMHead.apply(hid2, weight, lab1, mask, inv_t, return_entropy, compact_backward, dhidden_in_forward, grad)
     return lp.reshape(lead), (ent.reshape(lead) if ent is not None else None)
 
 
