@@ -7,8 +7,8 @@
 //   forward   a = W [V, H],  b = hidden [N, H]   both k-contiguous -> online (max, sum-exp,
 //             sum exp*z) per token, merged over the vocabulary tiles of a work item
 //   dz        a = W,         b = hidden          -> dZ = g * (onehot - softmax), bf16 [N, Vc]
-//   d_hidden  a = dZ [N, Vc] k-contiguous, b = W [Vc, H] k-major -> fp32 accumulate over chunks
-//   d_weight  a = dZ [N, Vc] k-major,      b = hidden [N, H] k-major -> bf16 rows of dW
+//   d_hidden  a = W [Vc, H] k-major,      b = dZ [N, Vc] k-contiguous -> fp32 accumulate over chunks
+//   d_weight  a = hidden [N, H] k-major,  b = dZ [N, Vc] k-major      -> bf16 rows of dW
 //
 // so the backward reads W, hidden and dZ where they lie: no transposed copies.
 //
@@ -82,41 +82,76 @@ __device__ __forceinline__ int opaque_tid() {
     asm volatile("" : "+v"(t));
     return t;
 }
+__device__ __forceinline__ void lds_barrier();
+struct ItemQueue {
+    static constexpr uint32_t NONE = 0xffffffffu;
+    uint32_t* counters;
+    // the word sits in the fifth ring slot, which the main loop first writes after its first barrier
+    volatile uint32_t* mailbox;
+    uint32_t items, locals, xcd;
+    // thread 0 only: the queues of XCDs xcd .. xcd + dry - 1 (mod 8) are known to be empty, `drawn` came from
+    // the queue of XCD xcd + dry, `next` is the id it stands for
+    uint32_t dry, drawn, next;
+
+    __device__ __forceinline__ ItemQueue(uint32_t* counters_, uint32_t items_, uint16_t* lds)
+        : counters(counters_),
+          mailbox(reinterpret_cast<volatile uint32_t*>(lds + 4 * BM * BK)),
+          items(items_),
+          locals((uint32_t)(pids_for_items(items_) >> 3)),  // ids per queue
+          xcd(blockIdx.x & 7),
+          dry(0),
+          drawn(0),
+          next(NONE) {
+        // a kernel may run several queues one after the other over the same word: every wave must have
+        // read the previous one's last value before thread 0 writes this one's first
+        __syncthreads();
+    }
+    // asks for an id; in flight until settle()
+    __device__ __forceinline__ void request() {
+        if (threadIdx.x == 0 && dry < 8) drawn = atomicAdd(&counters[(xcd + dry) & 7], 1u);
+    }
+    __device__ __forceinline__ void settle() {
+        if (threadIdx.x != 0) return;
+        next = NONE;
+        while (dry < 8) {
+            if (drawn < locals) {
+                next = drawn * 8 + ((xcd + dry) & 7);
+                return;
+            }
+            if (++dry < 8) drawn = atomicAdd(&counters[(xcd + dry) & 7], 1u);
+        }
+    }
+    // the settled id, for every thread.  The LDS must be free.
+    __device__ __forceinline__ uint32_t take() {
+        lds_barrier();
+        if (threadIdx.x == 0) *mailbox = next;
+        lds_barrier();
+        return __builtin_amdgcn_readfirstlane(*mailbox);
+    }
+    // its item; ids without one are passed over
+    __device__ __forceinline__ uint32_t take_item() {
+        for (;;) {
+            const uint32_t pid = take();
+            if (pid == NONE) return NONE;
+            const uint32_t item = item_of_pid(pid);
+            if (item < items) return item;
+            request();
+            settle();
+        }
+    }
+};
 template <class Body>
 __device__ __forceinline__ void for_each_item(uint32_t* __restrict__ counters, uint32_t items, uint16_t* lds, Body&& body) {
-    const uint32_t xcd = blockIdx.x & 7;
-    const uint32_t locals = (uint32_t)(pids_for_items(items) >> 3);  // ids per queue
-    // the word sits in the fifth ring slot, which the main loop first writes after its first barrier
-    volatile uint32_t* mailbox = reinterpret_cast<volatile uint32_t*>(lds + 4 * BM * BK);
-    constexpr uint32_t NONE = 0xffffffffu;
-    // thread 0 only: the queues of XCDs xcd .. xcd + dry - 1 (mod 8) are known to be empty and
-    // `drawn` came from the queue of XCD xcd + dry
-    uint32_t dry = 0, drawn = 0;
-    // a kernel may run several of these loops back to back over the same word: every wave must have
-    // read the previous loop's last value before thread 0 writes this loop's first one
-    __syncthreads();
-    auto resolve = [&]() -> uint32_t {
-        for (;;) {
-            if (drawn < locals) return drawn * 8 + ((xcd + dry) & 7);
-            if (++dry == 8) return NONE;
-            drawn = atomicAdd(&counters[(xcd + dry) & 7], 1u);
-        }
-    };
-    if (threadIdx.x == 0) {
-        drawn = atomicAdd(&counters[xcd], 1u);
-        *mailbox = resolve();
-    }
-    __syncthreads();
-    uint32_t pid = __builtin_amdgcn_readfirstlane(*mailbox);
-    while (pid != NONE) {
-        // in flight while the tile is computed
-        if (threadIdx.x == 0 && dry < 8) drawn = atomicAdd(&counters[(xcd + dry) & 7], 1u);
+    ItemQueue queue(counters, items, lds);
+    queue.request();
+    queue.settle();
+    uint32_t pid = queue.take();
+    while (pid != ItemQueue::NONE) {
+        queue.request();
         const uint32_t item = item_of_pid(pid);
         if (item < items) body(item);
-        __syncthreads();  // the tile's last use of the LDS is over
-        if (threadIdx.x == 0) *mailbox = dry < 8 ? resolve() : NONE;
-        __syncthreads();
-        pid = __builtin_amdgcn_readfirstlane(*mailbox);
+        queue.settle();
+        pid = queue.take();
     }
 }
 template <class Body>
@@ -128,14 +163,7 @@ __device__ __forceinline__ void for_each_tile(uint32_t* __restrict__ counters, i
         body(tm, tn);
     });
 }
-// fallback used by the stand-alone GEMM entry point, which has no workspace for a counter: one
-// workgroup per tile id
-__device__ __forceinline__ bool tile_of_block(int64_t tiles_m, int64_t tiles_n, int64_t* tm, int64_t* tn) {
-    const uint32_t item = item_of_pid(blockIdx.x);
-    if (item >= tiles_m * tiles_n) return false;
-    tile_of_item(item, (uint32_t)tiles_m, (uint32_t)tiles_n, tm, tn);
-    return true;
-}
+// stand-alone products have no workspace for counters: one workgroup per id
 inline unsigned grid_for_tiles(int64_t tiles_m, int64_t tiles_n) { return (unsigned)pids_for_items(tiles_m * tiles_n); }
 
 // LDS tile layout: row r of an operand tile holds its 64 k-values as eight 16-byte chunks; chunk c
@@ -157,21 +185,14 @@ __device__ __forceinline__ void wait_loads_and_barrier() {
     asm volatile("" ::: "memory");
 }
 
-// acc = A[m0 : m0+256, :K] * B[n0 : n0+256, :K]^T.  Rows past M / N are clamped onto the last
-// valid row (their results are discarded by the epilogues); K must be a multiple of 64.
-//
-// Operand tiles reach the LDS by direct global->LDS loads (no VGPR staging, no LDS store
-// instructions).  Eight consecutive lanes fetch the eight 16-byte chunks of one 128-byte row
-// segment, i.e. whole cache lines.  The path from L2 into the LDS delivers a 64 KB k-tile to a CU
-// in about the time the matrix pipe needs to multiply it, so the loads must be in flight all the
-// time: issued in one burst per k-tile they back up in the load unit and hold the issuing waves
-// (and their MFMAs) for twice the MFMA time of that k-step.  Spreading them needs a free
-// destination throughout the k-tile, which two full stages cannot give (the stage being read is
-// the only candidate), hence a ring of FIVE operand slots of 32 KB, all of a CU's 160 KB:
-// k-tile t reads A_t and B_t from two slots, A_(t+1) and B_(t+1) are landing in two more,
-// A_(t+2) goes into the fifth at any time, and B_(t+2) takes A_t's slot once the barrier near the
-// end of k-tile t has passed.
-// Wave w owns rows [32 w, 32 w + 32) of both operand tiles: 4 + 4 loads of 1 KB per k-tile.
+// Meets the other waves once this wave's LDS accesses are done.  __syncthreads() also waits for every global
+// store and load of the wave, which in an epilogue is the round trip of its stores at each barrier.
+__device__ __forceinline__ void lds_barrier() {
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+}
+
 constexpr int NSLOT = 5;
 constexpr int64_t MAX_LD = (int64_t)1 << 22;  // 255 rows * ld * 2 bytes must fit 32 bits
 __device__ __forceinline__ int ring_slot(int s) { return s >= NSLOT ? s - NSLOT : s; }
@@ -214,12 +235,102 @@ typedef short v4i16 __attribute__((ext_vector_type(4)));
 // 4 (s % 4)) and lane i receives column i at k0 .. k0 + 3, which is the MFMA operand layout (row
 // per lane, consecutive k per register).  The permutation puts the four k rows of such a read on
 // different banks.
+//
+// The product comes in two halves: begin_loads requests the first two k-tiles into slots 0 .. 3 (all but the
+// last block), gemm_loop waits for them and does the rest.  A caller may do other work in between that
+// touches slot 4 only.
+//
+// Loader side.  Addresses are a uniform 64-bit base (tile origin + k offset) plus a 32-bit byte
+// offset per lane; for a k-major operand the lanes' offsets of the last k-tile differ (its k
+// rows may end early), `last` holds those.
+struct Loader {
+    const char* tile;    // origin of the tile in global memory
+    int64_t k_step;      // bytes from one k-tile to the next
+    uint32_t off[4];     // per-lane byte offsets of the four loads
+    uint32_t last[4];    // the same for the last k-tile
+    int lds_block;       // elements between the LDS destinations of consecutive loads
+    int lds_wave;        // element offset of this wave's first load inside a slot
+};
+template <bool KM>
+__device__ __forceinline__ Loader make_loader(const Operand& op, int64_t ktiles, int lane, int wave) {
+    Loader L;
+    if constexpr (!KM) {
+        L.tile = reinterpret_cast<const char*>(op.p + op.r0 * op.ld);
+        L.k_step = BK * 2;
+        const int last_row = (int)((op.extent - 1 - op.r0) < 255 ? (op.extent - 1 - op.r0) : 255);
+#pragma unroll
+        for (int b = 0; b < 4; ++b) {
+            const int r = wave * 32 + b * 8 + (lane >> 3);
+            const int c = (lane & 7) ^ swz(r);
+            L.off[b] = (uint32_t)(r < last_row ? r : last_row) * (uint32_t)(op.ld * 2) + c * 16;
+            L.last[b] = L.off[b];
+        }
+        L.lds_block = 8 * BK;
+        L.lds_wave = wave * 32 * BK;
+    } else {
+        L.tile = reinterpret_cast<const char*>(op.p);
+        L.k_step = BK * op.ld * 2;
+        const int last_k = (int)(op.k_valid - 1 - (ktiles - 1) * BK);  // inside the last k-tile
+#pragma unroll
+        for (int b = 0; b < 4; ++b) {
+            const int kk = wave * 8 + b * 2 + (lane >> 5);
+            const int c = (lane & 31) ^ (4 * (kk & 3));
+            int64_t col = op.r0 + c * 8;
+            col = col + 8 <= op.extent ? col : op.extent - 8;
+            L.off[b] = (uint32_t)kk * (uint32_t)(op.ld * 2) + (uint32_t)(col * 2);
+            L.last[b] = (uint32_t)(kk < last_k ? kk : last_k) * (uint32_t)(op.ld * 2) + (uint32_t)(col * 2);
+        }
+        L.lds_block = 2 * 256;
+        L.lds_wave = wave * 8 * 256;
+    }
+    return L;
+}
+// k-tiles past the end are never requested by the main loop; begin_loads may ask for k-tile 1
+// of a one-k-tile product and then re-reads k-tile 0 into a slot nobody reads
+__device__ __forceinline__ const char* k_src(const Loader& L, int64_t kt, int64_t ktiles) {
+    const uint64_t v = reinterpret_cast<uint64_t>(L.tile + (kt < ktiles ? kt : ktiles - 1) * L.k_step);
+    const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)v);
+    const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)(v >> 32));
+    return reinterpret_cast<const char*>(((uint64_t)hi << 32) | lo);
+}
+// one 1 KB load: block b of this wave's share of an operand k-tile into ring slot `slot`
+__device__ __forceinline__ void load_block(const Loader& L, const char* src, uint32_t off, int slot, int b, uint16_t* lds) {
+    __builtin_amdgcn_global_load_lds(OI_GLOBAL_PTR(src + off),
+                                     OI_LDS_PTR(lds + slot * TILE_ELEMS + L.lds_wave + b * L.lds_block), 16, 0, 0);
+}
+// ring slots: A_t -> (2 t) mod 5, B_t -> (2 t + 1) mod 5
 template <bool A_KM, bool B_KM>
-__device__ __forceinline__ void gemm_tile(AccTile& acc, const Operand& A, const Operand& B, int64_t K, uint16_t* lds) {
+__device__ __forceinline__ void begin_loads(const Operand& A, const Operand& B, int64_t K, uint16_t* lds) {
     const int tid = opaque_tid();
     // the wave index as a scalar: the LDS destinations of the loads (M0) then take no VALU work
     const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int64_t ktiles = K / BK;
+    const Loader la = make_loader<A_KM>(A, ktiles, lane, wave), lb = make_loader<B_KM>(B, ktiles, lane, wave);
+    const char* a_k0 = k_src(la, 0, ktiles);
+    const char* b_k0 = k_src(lb, 0, ktiles);
+    const char* a_k1 = k_src(la, 1, ktiles);
+    const char* b_k1 = k_src(lb, 1, ktiles);
+    const bool t0_last = ktiles == 1, t1_last = ktiles <= 2;
+#pragma unroll
+    for (int b = 0; b < 4; ++b) load_block(la, a_k0, t0_last ? la.last[b] : la.off[b], 0, b, lds);
+#pragma unroll
+    for (int b = 0; b < 4; ++b) load_block(lb, b_k0, t0_last ? lb.last[b] : lb.off[b], 1, b, lds);
+#pragma unroll
+    for (int b = 0; b < 4; ++b) load_block(la, a_k1, t1_last ? la.last[b] : la.off[b], 2, b, lds);
+#pragma unroll
+    for (int b = 0; b < 3; ++b) load_block(lb, b_k1, t1_last ? lb.last[b] : lb.off[b], 3, b, lds);
+}
+
+// `__restrict__` here and in store_tile is what tells the compiler that the LDS accesses of these functions carry
+// alias information; without any it waits for every global->LDS load in flight before each LDS access
+// (d_weight of 3072 rows: 2.7 -> 4.9 ms).
+template <bool A_KM, bool B_KM>
+__device__ __forceinline__ void gemm_loop(AccTile& __restrict__ acc, const Operand& A, const Operand& B, int64_t K, uint16_t* lds) {
+    const int tid = opaque_tid();
+    const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wm = wave & 3, wn = wave >> 2;
+    const int64_t ktiles = K / BK;
+    const Loader la = make_loader<A_KM>(A, ktiles, lane, wave), lb = make_loader<B_KM>(B, ktiles, lane, wave);
 
 #pragma unroll
     for (int i = 0; i < 2; ++i)
@@ -227,84 +338,6 @@ __device__ __forceinline__ void gemm_tile(AccTile& acc, const Operand& A, const 
         for (int j = 0; j < 4; ++j)
 #pragma unroll
             for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
-
-    const int64_t ktiles = K / BK;
-    // loader side.  Addresses are a uniform 64-bit base (tile origin + k offset) plus a 32-bit byte
-    // offset per lane; for a k-major operand the lanes' offsets of the last k-tile differ (its k
-    // rows may end early), `last` holds those.
-    struct Loader {
-        const char* tile;    // origin of the tile in global memory
-        int64_t k_step;      // bytes from one k-tile to the next
-        uint32_t off[4];     // per-lane byte offsets of the four loads
-        uint32_t last[4];    // the same for the last k-tile
-        int lds_block;       // elements between the LDS destinations of consecutive loads
-        int lds_wave;        // element offset of this wave's first load inside a slot
-    };
-    auto make_loader = [&](const Operand& op, auto km_tag) {
-        constexpr bool KM = decltype(km_tag)::value;
-        Loader L;
-        if constexpr (!KM) {
-            L.tile = reinterpret_cast<const char*>(op.p + op.r0 * op.ld);
-            L.k_step = BK * 2;
-            const int last_row = (int)((op.extent - 1 - op.r0) < 255 ? (op.extent - 1 - op.r0) : 255);
-#pragma unroll
-            for (int b = 0; b < 4; ++b) {
-                const int r = wave * 32 + b * 8 + (lane >> 3);
-                const int c = (lane & 7) ^ swz(r);
-                L.off[b] = (uint32_t)(r < last_row ? r : last_row) * (uint32_t)(op.ld * 2) + c * 16;
-                L.last[b] = L.off[b];
-            }
-            L.lds_block = 8 * BK;
-            L.lds_wave = wave * 32 * BK;
-        } else {
-            L.tile = reinterpret_cast<const char*>(op.p);
-            L.k_step = BK * op.ld * 2;
-            const int last_k = (int)(op.k_valid - 1 - (ktiles - 1) * BK);  // inside the last k-tile
-#pragma unroll
-            for (int b = 0; b < 4; ++b) {
-                const int kk = wave * 8 + b * 2 + (lane >> 5);
-                const int c = (lane & 31) ^ (4 * (kk & 3));
-                int64_t col = op.r0 + c * 8;
-                col = col + 8 <= op.extent ? col : op.extent - 8;
-                L.off[b] = (uint32_t)kk * (uint32_t)(op.ld * 2) + (uint32_t)(col * 2);
-                L.last[b] = (uint32_t)(kk < last_k ? kk : last_k) * (uint32_t)(op.ld * 2) + (uint32_t)(col * 2);
-            }
-            L.lds_block = 2 * 256;
-            L.lds_wave = wave * 8 * 256;
-        }
-        return L;
-    };
-    const Loader la = make_loader(A, std::integral_constant<bool, A_KM>{});
-    const Loader lb = make_loader(B, std::integral_constant<bool, B_KM>{});
-    // k-tiles past the end are never requested by the loop below; the prologue may ask for k-tile 1
-    // of a one-k-tile product and then re-reads k-tile 0 into a slot nobody reads
-    auto k_src = [&](const Loader& L, int64_t kt) {
-        const uint64_t v = reinterpret_cast<uint64_t>(L.tile + (kt < ktiles ? kt : ktiles - 1) * L.k_step);
-        const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)v);
-        const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)(v >> 32));
-        return reinterpret_cast<const char*>(((uint64_t)hi << 32) | lo);
-    };
-    // one 1 KB load: block b of this wave's share of an operand k-tile into ring slot `slot`
-    auto load_block = [&](const Loader& L, const char* src, uint32_t off, int slot, int b) {
-        __builtin_amdgcn_global_load_lds(OI_GLOBAL_PTR(src + off),
-                                         OI_LDS_PTR(lds + slot * TILE_ELEMS + L.lds_wave + b * L.lds_block), 16, 0, 0);
-    };
-    // ring slots: A_t -> (2 t) mod 5, B_t -> (2 t + 1) mod 5
-    {
-        const char* a_k0 = k_src(la, 0);
-        const char* b_k0 = k_src(lb, 0);
-        const char* a_k1 = k_src(la, 1);
-        const char* b_k1 = k_src(lb, 1);
-        const bool t0_last = ktiles == 1, t1_last = ktiles <= 2;
-#pragma unroll
-        for (int b = 0; b < 4; ++b) load_block(la, a_k0, t0_last ? la.last[b] : la.off[b], 0, b);
-#pragma unroll
-        for (int b = 0; b < 4; ++b) load_block(lb, b_k0, t0_last ? lb.last[b] : lb.off[b], 1, b);
-#pragma unroll
-        for (int b = 0; b < 4; ++b) load_block(la, a_k1, t1_last ? la.last[b] : la.off[b], 2, b);
-#pragma unroll
-        for (int b = 0; b < 3; ++b) load_block(lb, b_k1, t1_last ? lb.last[b] : lb.off[b], 3, b);
-    }
 
     // consumer side: element offsets of this lane's fragments inside a slot
     const int lr = lane & 31, h = lane >> 5;
@@ -363,20 +396,20 @@ __device__ __forceinline__ void gemm_tile(AccTile& acc, const Operand& A, const 
     // the 8 loads of a k-tile iteration, as evenly spread as the slot hand-over allows; OFF selects
     // the lanes' offsets (off, or last when the k-tile being fetched is the last one)
 #define OI_LOADS_KS0(q)                                         \
-    if (q == 1) load_block(lb, b_n1, lb.off[3], s_b1, 3);       \
-    if (q == 5) load_block(la, a_n2, la.OFF2[0], s_a2, 0);
+    if (q == 1) load_block(lb, b_n1, lb.off[3], s_b1, 3, lds);       \
+    if (q == 5) load_block(la, a_n2, la.OFF2[0], s_a2, 0, lds);
 #define OI_LOADS_KS1(q) \
-    if (q == 3) load_block(la, a_n2, la.OFF2[1], s_a2, 1);
+    if (q == 3) load_block(la, a_n2, la.OFF2[1], s_a2, 1, lds);
 #define OI_LOADS_KS2(q)                                         \
-    if (q == 1) load_block(la, a_n2, la.OFF2[2], s_a2, 2);      \
-    if (q == 5) load_block(la, a_n2, la.OFF2[3], s_a2, 3);
+    if (q == 1) load_block(la, a_n2, la.OFF2[2], s_a2, 2, lds);      \
+    if (q == 5) load_block(la, a_n2, la.OFF2[3], s_a2, 3, lds);
 #define OI_LOADS_KS3(q)                                         \
-    if (q == 0) load_block(lb, b_n2, lb.OFF2[0], s_a, 0);       \
-    if (q == 3) load_block(lb, b_n2, lb.OFF2[1], s_a, 1);       \
-    if (q == 6) load_block(lb, b_n2, lb.OFF2[2], s_a, 2);
+    if (q == 0) load_block(lb, b_n2, lb.OFF2[0], s_a, 0, lds);       \
+    if (q == 3) load_block(lb, b_n2, lb.OFF2[1], s_a, 1, lds);       \
+    if (q == 6) load_block(lb, b_n2, lb.OFF2[2], s_a, 2, lds);
 #define OI_LOADS_NONE(q)
 #define OI_LOADS_KS0_ONLY_B(q) \
-    if (q == 1) load_block(lb, b_n1, lb.last[3], s_b1, 3);
+    if (q == 1) load_block(lb, b_n1, lb.last[3], s_b1, 3, lds);
 
     // A_0 and B_0 must have landed.  The wait is for everything in flight, not for "all but the 7
     // younger loads": a workgroup that runs several tiles may still have the previous tile's
@@ -394,9 +427,9 @@ __device__ __forceinline__ void gemm_tile(AccTile& acc, const Operand& A, const 
         const int s_a = sa, s_b = ring_slot(sa + 1);                  /* being read */                          \
         const int s_a1 = ring_slot(sa + 2), s_b1 = ring_slot(sa + 3); /* k-tile kt+1 */                         \
         const int s_a2 = ring_slot(sa + 4);                           /* free all along: takes A_(kt+2) */      \
-        const char* b_n1 = k_src(lb, kt + 1);                                                                    \
-        const char* a_n2 = k_src(la, kt + 2);                                                                    \
-        const char* b_n2 = k_src(lb, kt + 2);                                                                    \
+        const char* b_n1 = k_src(lb, kt + 1, ktiles);                                                                    \
+        const char* a_n2 = k_src(la, kt + 2, ktiles);                                                                    \
+        const char* b_n2 = k_src(lb, kt + 2, ktiles);                                                                    \
         (void)s_a2; (void)s_b1; (void)b_n1; (void)a_n2; (void)b_n2;                                              \
         OI_KSTEP(a0, b0, a1, b1, s_a, s_b, 1, L0)                                                                \
         OI_KSTEP(a1, b1, a0, b0, s_a, s_b, 2, L1)                                                                \
@@ -438,6 +471,11 @@ __device__ __forceinline__ void gemm_tile(AccTile& acc, const Operand& A, const 
     // every wave is done reading before the caller reuses the LDS (epilogue staging, next tile)
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
+}
+template <bool A_KM, bool B_KM>
+__device__ __forceinline__ void gemm_tile(AccTile& acc, const Operand& A, const Operand& B, int64_t K, uint16_t* lds) {
+    begin_loads<A_KM, B_KM>(A, B, K, lds);
+    gemm_loop<A_KM, B_KM>(acc, A, B, K, lds);
 }
 // both operands k-contiguous: C[m, n] = sum_k A[m0 + m, k] * B[n0 + n, k]
 __device__ __forceinline__ void gemm_tile(AccTile& acc, const uint16_t* __restrict__ A, int64_t lda, int64_t m0,
@@ -670,7 +708,7 @@ __device__ __forceinline__ void lmhead_fwd_item(const uint16_t* __restrict__ W, 
                 // of the image, so one barrier per group (written -> read out) is all they need
                 __builtin_amdgcn_sched_barrier(0);
                 stage_group_bf16(acc, lds, wm, wn, lane, j);
-                __syncthreads();
+                lds_barrier();
                 const int64_t left = n_tokens - n0;
                 copy_staged_group(lds, fl.ecache + n0 * fl.cache_ld + (vt - fl.cache_tile0) * BM, fl.cache_ld, tid,
                                   (int)(left < BN ? left : BN), j);
@@ -678,7 +716,7 @@ __device__ __forceinline__ void lmhead_fwd_item(const uint16_t* __restrict__ W, 
             }
         }
         // the next tile's first loads must wait until the image has been read out again
-        if (CACHE && keep_tile) __syncthreads();
+        if (CACHE && keep_tile) lds_barrier();
     }
 
     // merge the two lane halves (same token, other rows), then the four m-waves through LDS
@@ -949,33 +987,14 @@ __global__ void __launch_bounds__(NTHREADS)
 // ---------------------------------------------------------------------------------------------
 // backward steps 2 and 3: plain tile products with a store epilogue
 // ---------------------------------------------------------------------------------------------
-// Transposes the 4 x 4 block that a quad of lanes holds: on entry lane k of the quad has v[e] = M[e][k]
-// (one column, four consecutive rows, which is how the MFMA leaves its results), on return
-// v[f] = M[k][f] (one row, four consecutive columns, which is what a 16-byte store wants).  Two
-// exchange steps inside the quad (DPP), every lane of the wave must take part.
-__device__ __forceinline__ float quad_swap(float x, bool far) {
-    const int i = __float_as_int(x);
-    return __int_as_float(far ? __builtin_amdgcn_mov_dpp(i, 0x4E /* quad_perm 2,3,0,1 */, 0xF, 0xF, true)
-                              : __builtin_amdgcn_mov_dpp(i, 0xB1 /* quad_perm 1,0,3,2 */, 0xF, 0xF, true));
-}
-__device__ __forceinline__ void quad_transpose(float (&v)[4], int lane) {
-    const bool b0 = lane & 1, b1 = lane & 2;
-    const float r01 = quad_swap(b0 ? v[0] : v[1], false), r23 = quad_swap(b0 ? v[2] : v[3], false);
-    const float t0 = b0 ? r01 : v[0], t1 = b0 ? v[1] : r01, t2 = b0 ? r23 : v[2], t3 = b0 ? v[3] : r23;
-    const float ra = quad_swap(b1 ? t0 : t2, true), rb = quad_swap(b1 ? t1 : t3, true);
-    v[0] = b1 ? ra : t0;
-    v[1] = b1 ? rb : t1;
-    v[2] = b1 ? t2 : ra;
-    v[3] = b1 ? t3 : rb;
-}
-
 // Where a tile product goes.
 // mode 0: out_f32  = acc          mode 1: out_f32 += acc
 // mode 2: out_bf16 = acc          mode 3: out_bf16 = out_f32 + acc   (last chunk of d_hidden)
 // mode 4: out_bf16 += acc         (rows added to a d_weight that was already rounded)
 // Rows below m_valid and columns below N are stored.  With `out_rows`, row r of a bf16 result goes to row
 // out_rows[r] of out_bf16 (the fp32 accumulator stays compact).  scale_a / scale_b: factors of row r, see
-// DynRows.
+// DynRows.  Every element has one writer per launch and the launches follow each other on the stream, so the
+// sums of modes 1, 3 and 4 are plain loads and stores.
 struct StoreTo {
     int mode;
     float* out_f32;
@@ -984,220 +1003,216 @@ struct StoreTo {
     const int32_t* out_rows;
     const float *scale_a, *scale_b;
 };
-// 16-byte pieces (8 bytes of bf16) need whole groups of four columns
+// whole 16-byte pieces (8 bytes for the bf16 results of modes 3 and 4) can be stored and loaded
 __device__ __forceinline__ bool stores_in_pieces(const StoreTo& st) {
-    return ((st.N | st.ldo) & 3) == 0 && (reinterpret_cast<uintptr_t>(st.out_f32) & 15) == 0 &&
-           (reinterpret_cast<uintptr_t>(st.out_bf16) & 7) == 0;
+    return ((st.N | st.ldo) & 7) == 0 &&
+           ((reinterpret_cast<uintptr_t>(st.out_f32) | reinterpret_cast<uintptr_t>(st.out_bf16)) & 15) == 0;
 }
-// the four rows (one per group of 8) of a 32-row block that a lane stores pieces of
-struct LaneRows {
-    int64_t row[4], dst[4];
-    bool ok[4];
-    float sa[4], sb[4];
+
+// Column group j of a finished tile is its rows row0 + wn * 128 + j * 32 + (0..31) of both wn halves with all 256
+// columns from col0.  z0, z1: the lane's accumulators, row acc_col(wn, j, lane), columns acc_row(wm, 0 / 1, r,
+// lane), i.e. groups of four consecutive columns of one row.  They meet in the LDS region `stage` (64 rows) and
+// leave as whole rows, 512 bytes of bf16 or 1 KB of fp32 at a time.  Every thread of the workgroup takes part.
+//
+// What bounds the epilogue is that nothing is multiplied meanwhile (one workgroup per CU), so few instructions
+// and whole lines.  Registers transposed in quads of lanes and stored from there in 64-byte pieces, with a wait
+// for the stores of the tile before the next tile's first load: d_weight of 268 rows (100352 x 4096, 6272
+// tiles of 5 k-tiles) 606 us; through the LDS 544; without waiting for stores at its barriers 504; with the next tile's
+// first loads ahead of it 478.
+constexpr int STAGE_F32 = BM + 4;                            // floats per row: rows 4 banks apart
+constexpr int GROUP_ROWS = 64;
+constexpr int GROUP_F32 = GROUP_ROWS * STAGE_F32 * 2;        // LDS elements of an fp32 region
+static_assert(2 * GROUP_F32 <= LDS_ELEMS, "the epilogue's regions fit the ring");
+constexpr int GROUP_BF16_AT = 4 * TILE_ELEMS;                // the bf16 region is ring slot 4
+static_assert(GROUP_ROWS * BM <= TILE_ELEMS, "a bf16 group fits one ring slot");
+struct RowScale {
+    float a, b;
+    bool on;
+    // a row whose factor is exactly 0 is 0 whatever its sum holds (the sums of rows that were taken out may
+    // have left the fp32 range)
+    __device__ __forceinline__ float operator()(float v) const { return on ? (b == 0.f ? 0.f : v * a * b) : v; }
 };
-__device__ __forceinline__ LaneRows lane_rows(const StoreTo& st, int64_t row0, int lane) {
-    LaneRows r;
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-        r.row[q] = row0 + q * 8 + (lane >> 5) * 4 + (lane & 3);
-        r.ok[q] = r.row[q] < st.m_valid;
-        r.dst[q] = (r.ok[q] && st.out_rows) ? (int64_t)st.out_rows[r.row[q]] : r.row[q];
-        r.sa[q] = (r.ok[q] && st.scale_a) ? st.scale_a[r.row[q]] : 1.f;
-        r.sb[q] = (r.ok[q] && st.scale_a) ? st.scale_b[r.row[q]] : 1.f;
+__device__ __forceinline__ RowScale row_scale(const StoreTo& st, int64_t row) {
+    RowScale s = {1.f, 1.f, st.scale_a != nullptr};
+    if (s.on && row < st.m_valid) {
+        s.a = st.scale_a[row];
+        s.b = st.scale_b[row];
     }
-    return r;
+    return s;
 }
-// Stores a 32-row x 64-column block whose entry (jj, q, e) of a lane is row q * 8 + (lane / 32) * 4 + e,
-// column jj * 32 + lane % 32 (the layout the MFMA leaves).  Every store and load as a 16-byte piece
-// (8 bytes of bf16): after a 4 x 4 transpose inside each quad of lanes a lane holds four consecutive
-// columns of one row.  A quarter of the memory instructions of the one-value-per-lane form, whose
-// address processing is what an epilogue of 128 values per lane waits for.  The fp32 sum of the
-// accumulating modes is requested before the transposes and added with plain loads and stores: every
-// element has one writer per launch and the launches follow each other on the stream, so no atomic is
-// needed.  32 registers of sums in flight.
-template <class Get>
-__device__ __forceinline__ void store_block(const StoreTo& st, const LaneRows& r, int64_t col0, int lane, Get&& get) {
-    const int mode = st.mode, g = (lane & 31) >> 2;
-    oi_f32x4 part[2][4];
-    uint2 part16[2][4];
-    if (mode == 1 || mode == 3) {
+__device__ __forceinline__ int64_t group_row(int64_t row0, int j, int r) { return row0 + (r >> 5) * 128 + j * 32 + (r & 31); }
+
+// mode 2 in whole pieces
+__device__ __forceinline__ void store_group_bf16(const f32x16& z0, const f32x16& z1, const StoreTo& st, int64_t row0,
+                                                 int64_t col0, int j, uint16_t* stage, int tid) {
+    asm volatile("" : "+v"(tid));  // addresses are formed here, not ahead of the tile's main loop
+    const int lane = tid & 63, wave = tid >> 6, wm = wave & 3, wn = wave >> 2;
+    const int srow = wn * 32 + (lane & 31);
+    const RowScale sc = row_scale(st, group_row(row0, j, srow));
+    // 64 rows of 512 bytes, unpadded; the 16-byte pieces of a row at c ^ (row mod 32) and their halves swapped in
+    // rows 16 .. 31 of every 32, which puts the 8-byte stores of 32 lanes on all 64 banks
 #pragma unroll
-        for (int jj = 0; jj < 2; ++jj)
-#pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                const int64_t col = col0 + jj * 32 + 4 * g;
-                part[jj][q] = (r.ok[q] && col < st.N)
-                                  ? *reinterpret_cast<const oi_f32x4*>(st.out_f32 + r.row[q] * st.ldo + col)
-                                  : oi_f32x4{0.f, 0.f, 0.f, 0.f};
-            }
-    } else if (mode == 4) {
-#pragma unroll
-        for (int jj = 0; jj < 2; ++jj)
-#pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                const int64_t col = col0 + jj * 32 + 4 * g;
-                part16[jj][q] = (r.ok[q] && col < st.N)
-                                    ? *reinterpret_cast<const uint2*>(st.out_bf16 + r.dst[q] * st.ldo + col)
-                                    : make_uint2(0u, 0u);
-            }
-    }
-#pragma unroll
-    for (int jj = 0; jj < 2; ++jj) {
-        const int64_t col = col0 + jj * 32 + 4 * g;
+    for (int i = 0; i < 2; ++i)
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
-            float v[4] = {get(jj, q, 0), get(jj, q, 1), get(jj, q, 2), get(jj, q, 3)};
-            quad_transpose(v, lane);
-            if (!r.ok[q] || col >= st.N) continue;
-            if (st.scale_a) {
-                // a row whose factor is exactly 0 is 0 whatever its sum holds (the sums of
-                // rows that were taken out may have left the fp32 range)
+            const f32x16& z = i == 0 ? z0 : z1;
+            const int piece = (wm * 8 + i * 4 + q) ^ (srow & 31), half = (lane >> 5) ^ ((srow >> 4) & 1);
+            *reinterpret_cast<uint2*>(stage + srow * BM + piece * 8 + half * 4) =
+                make_uint2(oi_pack_bf16x2(sc(z[q * 4]), sc(z[q * 4 + 1])), oi_pack_bf16x2(sc(z[q * 4 + 2]), sc(z[q * 4 + 3])));
+        }
+    lds_barrier();
+    constexpr int ITERS = GROUP_ROWS * (BM / 8) / NTHREADS;
+    oi_u32x4 v[ITERS];
 #pragma unroll
-                for (int e = 0; e < 4; ++e) v[e] = r.sb[q] == 0.f ? 0.f : v[e] * r.sa[q] * r.sb[q];
-            }
-            if (mode == 1 || mode == 3) {
-                v[0] += part[jj][q].x;
-                v[1] += part[jj][q].y;
-                v[2] += part[jj][q].z;
-                v[3] += part[jj][q].w;
-            } else if (mode == 4) {
-                v[0] += oi_bf16lo_to_f32(part16[jj][q].x);
-                v[1] += oi_bf16hi_to_f32(part16[jj][q].x);
-                v[2] += oi_bf16lo_to_f32(part16[jj][q].y);
-                v[3] += oi_bf16hi_to_f32(part16[jj][q].y);
-            }
-            if (mode <= 1)
-                *reinterpret_cast<oi_f32x4*>(st.out_f32 + r.row[q] * st.ldo + col) = oi_f32x4{v[0], v[1], v[2], v[3]};
-            else
-                *reinterpret_cast<uint2*>(st.out_bf16 + r.dst[q] * st.ldo + col) =
-                    make_uint2(oi_pack_bf16x2(v[0], v[1]), oi_pack_bf16x2(v[2], v[3]));
+    for (int it = 0; it < ITERS; ++it) {
+        const int cidx = tid + it * NTHREADS, r = cidx >> 5, ch = cidx & 31;
+        v[it] = *reinterpret_cast<const oi_u32x4*>(stage + r * BM + (ch ^ (r & 31)) * 8);
+    }
+    lds_barrier();  // the region is free for the next group
+#pragma unroll
+    for (int it = 0; it < ITERS; ++it) {
+        const int cidx = tid + it * NTHREADS, r = cidx >> 5, ch = cidx & 31;
+        const int64_t row = group_row(row0, j, r), col = col0 + ch * 8;
+        if (row >= st.m_valid || col >= st.N) continue;
+        const int64_t dst = st.out_rows ? (int64_t)st.out_rows[row] : row;
+        *reinterpret_cast<oi_u32x4*>(st.out_bf16 + dst * st.ldo + col) =
+            (r & 16) ? oi_u32x4{v[it].z, v[it].w, v[it].x, v[it].y} : v[it];
+    }
+}
+
+// every mode, any pitch, any alignment of the element type
+__device__ __forceinline__ void store_group_f32(const f32x16& z0, const f32x16& z1, const StoreTo& st, bool pieces,
+                                                int64_t row0, int64_t col0, int j, uint16_t* stage, int tid) {
+    asm volatile("" : "+v"(tid));
+    const int lane = tid & 63, wave = tid >> 6, wm = wave & 3, wn = wave >> 2;
+    const int mode = st.mode, srow = wn * 32 + (lane & 31);
+    float* stage32 = reinterpret_cast<float*>(stage);
+    constexpr int ITERS = GROUP_ROWS * (BM / 4) / NTHREADS;
+    const int ch = tid & 63, r_first = tid >> 6;  // piece `it` of a thread: row r_first + 8 it, columns 4 ch ..
+    const int64_t col = col0 + ch * 4;
+    const bool adds = pieces && (mode == 1 || mode == 3);
+    // the sum so far is requested before the tile goes through the LDS; rows and columns past the end read the last
+    // valid piece and store nothing
+    oi_f32x4 sum[ITERS];
+    if (adds) {
+        const int64_t c = col < st.N ? col : st.N - 4;
+#pragma unroll
+        for (int it = 0; it < ITERS; ++it) {
+            int64_t row = group_row(row0, j, r_first + it * 8);
+            row = row < st.m_valid ? row : st.m_valid - 1;
+            sum[it] = *reinterpret_cast<const oi_f32x4*>(st.out_f32 + row * st.ldo + c);
+        }
+    }
+    const RowScale sc = row_scale(st, group_row(row0, j, srow));
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const f32x16& z = i == 0 ? z0 : z1;
+            *reinterpret_cast<oi_f32x4*>(stage32 + srow * STAGE_F32 + acc_row(wm, i, q * 4, lane)) =
+                oi_f32x4{sc(z[q * 4]), sc(z[q * 4 + 1]), sc(z[q * 4 + 2]), sc(z[q * 4 + 3])};
+        }
+    lds_barrier();
+    const float* from = stage32 + r_first * STAGE_F32 + ch * 4;
+    if (pieces && mode <= 1) {
+#pragma unroll
+        for (int it = 0; it < ITERS; ++it) {
+            const int64_t row = group_row(row0, j, r_first + it * 8);
+            oi_f32x4 v = *reinterpret_cast<const oi_f32x4*>(from + it * 8 * STAGE_F32);
+            if (adds) v += sum[it];
+            if (row < st.m_valid && col < st.N) *reinterpret_cast<oi_f32x4*>(st.out_f32 + row * st.ldo + col) = v;
+        }
+        return;
+    }
+    if (adds) {
+#pragma unroll
+        for (int it = 0; it < ITERS; ++it) {
+            const int64_t row = group_row(row0, j, r_first + it * 8);
+            const oi_f32x4 v = *reinterpret_cast<const oi_f32x4*>(from + it * 8 * STAGE_F32) + sum[it];
+            if (row >= st.m_valid || col >= st.N) continue;
+            const int64_t dst = st.out_rows ? (int64_t)st.out_rows[row] : row;
+            *reinterpret_cast<uint2*>(st.out_bf16 + dst * st.ldo + col) =
+                make_uint2(oi_pack_bf16x2(v.x, v.y), oi_pack_bf16x2(v.z, v.w));
+        }
+        return;
+    }
+    if (col >= st.N) return;
+    const int n = st.N - col < 4 ? (int)(st.N - col) : 4;
+#pragma unroll 1
+    for (int it = 0; it < ITERS; ++it) {
+        const int64_t row = group_row(row0, j, r_first + it * 8);
+        if (row >= st.m_valid) break;
+        const oi_f32x4 v = *reinterpret_cast<const oi_f32x4*>(from + it * 8 * STAGE_F32);
+        float e[4] = {v.x, v.y, v.z, v.w};
+        if (mode <= 1) {
+            float* f = st.out_f32 + row * st.ldo + col;
+#pragma unroll
+            for (int k = 0; k < 4; ++k)
+                if (k < n) f[k] = mode == 1 ? f[k] + e[k] : e[k];
+            continue;
+        }
+        uint16_t* b = st.out_bf16 + (st.out_rows ? (int64_t)st.out_rows[row] : row) * st.ldo + col;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            if (k >= n) continue;
+            if (mode == 3) e[k] += st.out_f32[row * st.ldo + col + k];
+            if (mode == 4) e[k] += oi_bf16lo_to_f32((uint32_t)b[k]);
+        }
+        if (n == 4 && (reinterpret_cast<uintptr_t>(b) & 3) == 0) {
+            reinterpret_cast<uint32_t*>(b)[0] = oi_pack_bf16x2(e[0], e[1]);
+            reinterpret_cast<uint32_t*>(b)[1] = oi_pack_bf16x2(e[2], e[3]);
+        } else {
+#pragma unroll
+            for (int k = 0; k < 4; ++k)
+                if (k < n) b[k] = (uint16_t)oi_f32_to_bf16_bits(e[k]);
         }
     }
 }
 
-// A, B: operands without their tile origin (r0 is filled in here).  K == 0 stores zeros.  With `part`
-// the fp32 tile goes there and nowhere else.
-template <bool A_KM, bool B_KM>
-__device__ __forceinline__ void gemm_store_tile(Operand A, Operand B, int64_t K, const StoreTo& st, int64_t tm,
-                                                int64_t tn, float* part, uint16_t* lds) {
-    const int tid = opaque_tid(), lane = tid & 63, wave = tid >> 6, wm = wave & 3, wn = wave >> 2;
-    const int64_t m0 = tm * BM, n0 = tn * BN;
-    const int mode = st.mode;
-    float* out_f32 = st.out_f32;
-    uint16_t* out_bf16 = st.out_bf16;
-    const int64_t ldo = st.ldo, m_valid = st.m_valid, N = st.N;
-    const int32_t* out_rows = st.out_rows;
-    const float *scale_a = st.scale_a, *scale_b = st.scale_b;
-    A.r0 = m0;
-    B.r0 = n0;
-    AccTile acc;
-    if (K <= 0 && (mode == 1 || mode == 4)) return;  // nothing to add
-    if (K > 0) {
-        gemm_tile<A_KM, B_KM>(acc, A, B, K, lds);
-    } else {
-#pragma unroll
-        for (int i = 0; i < 2; ++i)
-#pragma unroll
-            for (int j = 0; j < 4; ++j)
-#pragma unroll
-                for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
-    }
-    if (part) {
-        store_part(acc, part, tid);
-        return;
-    }
-    if (stores_in_pieces(st)) {
-#pragma unroll
-        for (int i = 0; i < 2; ++i) {
-            const LaneRows r = lane_rows(st, m0 + wm * 64 + i * 32, lane);
-#pragma unroll
-            for (int jh = 0; jh < 2; ++jh)
-                store_block(st, r, n0 + wn * 128 + jh * 64, lane,
-                            [&](int jj, int q, int e) { return acc[i][2 * jh + jj][q * 4 + e]; });
-        }
-        return;
-    }
-    if (mode >= 2 && (ldo & 1) == 0) {
-        // bf16 output: neighbouring lanes hold neighbouring columns of the same rows; after one DPP
-        // swap per pair of rows every lane stores two columns of one row as a 4-byte word (half as
-        // many, twice as wide stores as one bf16 per lane)
-        const bool odd = lane & 1;
-#pragma unroll
-        for (int i = 0; i < 2; ++i)
-#pragma unroll
-            for (int t = 0; t < 8; ++t) {
-                const int64_t row = m0 + acc_row(wm, i, 2 * t, lane) + (odd ? 1 : 0);
-                // a lane past the last row still takes part in the exchange below: its neighbour
-                // holds the row before it and needs this lane's half of that row
-                const bool row_ok = row < m_valid;
-                const int64_t dst_row = (row_ok && out_rows) ? (int64_t)out_rows[row] : row;
-                const float sa = (row_ok && scale_a) ? scale_a[row] : 1.f, sb = (row_ok && scale_a) ? scale_b[row] : 1.f;
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    const int64_t col = n0 + (acc_col(wn, j, lane) & ~1);
-                    const float own0 = acc[i][j][2 * t], own1 = acc[i][j][2 * t + 1];
-                    const float send = odd ? own0 : own1;
-                    const float recv = __int_as_float(
-                        __builtin_amdgcn_mov_dpp(__float_as_int(send), 0xB1 /* quad_perm 1,0,3,2 */, 0xF, 0xF, true));
-                    float lo = odd ? recv : own0, hi = odd ? own1 : recv;
-                    if (!row_ok || col >= N) continue;
-                    if (scale_a) {
-                        // a row whose factor is exactly 0 is 0 whatever its sum holds (the sums of
-                        // rows that were taken out may have left the fp32 range)
-                        lo = sb == 0.f ? 0.f : lo * sa * sb;
-                        hi = sb == 0.f ? 0.f : hi * sa * sb;
-                    }
-                    const int64_t o = row * ldo + col, d = dst_row * ldo + col;
-                    if (col + 1 < N) {
-                        if (mode == 3) {
-                            const float2 part = *reinterpret_cast<const float2*>(out_f32 + o);
-                            lo += part.x;
-                            hi += part.y;
-                        } else if (mode == 4) {
-                            const uint32_t prev = *reinterpret_cast<const uint32_t*>(out_bf16 + d);
-                            lo += oi_bf16lo_to_f32(prev);
-                            hi += oi_bf16hi_to_f32(prev);
-                        }
-                        *reinterpret_cast<uint32_t*>(out_bf16 + d) = oi_pack_bf16x2(lo, hi);
-                    } else {
-                        if (mode == 3) lo += out_f32[o];
-                        else if (mode == 4) lo += oi_bf16lo_to_f32((uint32_t)out_bf16[d]);
-                        out_bf16[d] = (uint16_t)oi_f32_to_bf16_bits(lo);
-                    }
-                }
-            }
-        return;
-    }
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
+// out[row, col] = sum_k R(row, k) * C(col, k).  R's rows (token or vocabulary rows of the result) are the tile
+// product's n dimension and C's (the result's columns) its m dimension, because a lane's consecutive
+// accumulators are consecutive in m: four columns of one row, which the epilogue stores without a transpose.
+// One tile, or with `part` a piece of one along k whose fp32 tile goes there and nowhere else.
+struct ProductTile {
+    Operand R, C;
+    int64_t K;
+    float* part;
+};
+// In mode 2 with whole pieces this leaves the ring slots 0 .. 3 alone.
+__device__ __forceinline__ void store_tile(const AccTile& __restrict__ acc, const ProductTile& t, const StoreTo& st, bool pieces,
+                                           uint16_t* lds) {
+    const int tid = opaque_tid();
+    if (t.part) {
+        store_part(acc, t.part, tid);
+    } else if (st.mode == 2 && pieces) {
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
-            const int64_t col = n0 + acc_col(wn, j, lane);
-            if (col >= N) continue;
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const int64_t row = m0 + acc_row(wm, i, r, lane);
-                if (row >= m_valid) continue;
-                const int64_t o = row * ldo + col;
-                float v = acc[i][j][r];
-                if (scale_a) v = scale_b[row] == 0.f ? 0.f : v * scale_a[row] * scale_b[row];
-                if (mode == 1) {
-                    // the addition is done by the L2 (no load to wait for: 8.2 -> 6.9 ms per d_weight slab product);
-                    // every element has one writer per launch and the launches follow each other on
-                    // the stream, so the sum is the one a load + add + store would give, to the bit
-                    unsafeAtomicAdd(out_f32 + o, v);
-                    continue;
-                }
-                if (mode == 3) v += out_f32[o];
-                if (mode == 0) {
-                    out_f32[o] = v;
-                    continue;
-                }
-                const int64_t d = (out_rows ? (int64_t)out_rows[row] : row) * ldo + col;
-                if (mode == 4) v += oi_bf16lo_to_f32((uint32_t)out_bf16[d]);
-                out_bf16[d] = (uint16_t)oi_f32_to_bf16_bits(v);
-            }
+            __builtin_amdgcn_sched_barrier(0);
+            store_group_bf16(acc[0][j], acc[1][j], st, t.R.r0, t.C.r0, j, lds + GROUP_BF16_AT, tid);
+            __builtin_amdgcn_sched_barrier(0);
         }
+    } else {
+        // two regions in turn: one is written again only after the barrier of the group in between, by which
+        // every wave has read it out
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            __builtin_amdgcn_sched_barrier(0);
+            store_group_f32(acc[0][j], acc[1][j], st, pieces, t.R.r0, t.C.r0, j, lds + (j & 1) * GROUP_F32, tid);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    }
+}
+// a product without terms (no rows selected): zeros, or what the earlier launches summed up
+__device__ __forceinline__ void store_no_terms(const StoreTo& st) {
+    if (st.mode == 1 || st.mode == 4) return;
+    for (int64_t row = blockIdx.x; row < st.m_valid; row += gridDim.x) {
+        const int64_t dst = (st.mode >= 2 && st.out_rows) ? (int64_t)st.out_rows[row] : row;
+        for (int64_t col = threadIdx.x; col < st.N; col += NTHREADS) {
+            if (st.mode == 0) st.out_f32[row * st.ldo + col] = 0.f;
+            else st.out_bf16[dst * st.ldo + col] =
+                st.mode == 3 ? (uint16_t)oi_f32_to_bf16_bits(st.out_f32[row * st.ldo + col]) : (uint16_t)0;
+        }
+    }
 }
 
 // Sizes that depend on a row count which only the device knows (rows selected by a mask).
@@ -1276,9 +1291,9 @@ __device__ __forceinline__ ProductSizes product_sizes(int64_t M, int64_t K, int6
 
 // `queue` null: one workgroup per tile id (blockIdx); otherwise a launch of resident workgroups
 // that draw their tiles from the queue.  `parts` (with a queue only): scratch for the pieces of split tiles.
-template <bool A_KM, bool B_KM>
+template <bool R_KM, bool C_KM>
 __global__ void __launch_bounds__(NTHREADS)
-    gemm_store_kernel(Operand A, int64_t M, Operand B, int64_t N, int64_t K, int mode, float* out_f32,
+    gemm_store_kernel(Operand R, int64_t M, Operand C, int64_t N, int64_t K, int mode, float* out_f32,
                       uint16_t* out_bf16, int64_t ldo, int64_t m_valid, DynRows dyn, uint32_t* __restrict__ queue,
                       float* __restrict__ parts) {
     __shared__ __align__(16) uint16_t lds[LDS_ELEMS];
@@ -1287,75 +1302,125 @@ __global__ void __launch_bounds__(NTHREADS)
         if (mode < 0) return;
     }
     const ProductSizes z = product_sizes(M, K, m_valid, dyn);
-    if (dyn.n_dev && dyn.role == 1) A.extent = z.M;
+    if (dyn.n_dev && dyn.role == 1) R.extent = z.M;
     if (dyn.n_dev && dyn.role == 2) {
         const int64_t n = *dyn.n_dev;
-        A.k_valid = (n + BM - 1) / BM * BM;
-        B.k_valid = n;
+        R.k_valid = (n + BM - 1) / BM * BM;
+        C.k_valid = n;
     }
     K = z.K;
-    // a product without terms that would only be added changes nothing: no tile is drawn at all
-    if (K <= 0 && (mode == 1 || mode == 4)) return;
     const StoreTo st = {mode, out_f32, out_bf16, ldo, N, z.m_valid, dyn.out_rows, dyn.scale_a, dyn.scale_b};
-    const int64_t tiles_m = (z.M + BM - 1) / BM, tiles_n = (N + BN - 1) / BN;
-    if (queue) {
-        const uint32_t tiles = (uint32_t)(tiles_m * tiles_n), ktiles = (uint32_t)(K / BK);
-        TailSplit ts = {tiles, 0, 1};
-        if (parts && stores_in_pieces(st)) ts = plan_tail(tiles, gridDim.x, ktiles);
-        for_each_item(queue, ts.whole + ts.rest * ts.parts, lds, [&](uint32_t item) {
-            uint32_t tile = item, k0 = 0, k1 = ktiles;
-            float* piece = nullptr;
-            if (item >= ts.whole) {
-                const uint32_t r = item - ts.whole, p = r / ts.rest;
-                tile = ts.whole + (r - p * ts.rest);
-                k0 = ktiles * p / ts.parts;
-                k1 = ktiles * (p + 1) / ts.parts;
-                piece = parts + (int64_t)r * PART_FLOATS;
-            }
-            int64_t tm, tn;
-            tile_of_item(tile, (uint32_t)tiles_m, (uint32_t)tiles_n, &tm, &tn);
-            Operand a = A, b = B;
+    const bool pieces = stores_in_pieces(st);
+    if (K <= 0) {
+        store_no_terms(st);
+        return;
+    }
+    const uint32_t tiles_r = (uint32_t)((z.M + BN - 1) / BN), tiles_c = (uint32_t)((N + BM - 1) / BM);
+    const uint32_t tiles = tiles_r * tiles_c, ktiles = (uint32_t)(K / BK);
+    TailSplit ts = {tiles, 0, 1};
+    if (parts) ts = plan_tail(tiles, gridDim.x, ktiles);
+    auto tile_at = [&](uint32_t item) {
+        ProductTile t = {R, C, K, nullptr};
+        uint32_t tile = item;
+        if (item >= ts.whole) {
+            const uint32_t r = item - ts.whole, p = r / ts.rest;
+            tile = ts.whole + (r - p * ts.rest);
+            const uint32_t k0 = ktiles * p / ts.parts, k1 = ktiles * (p + 1) / ts.parts;
             const int64_t k_begin = (int64_t)k0 * BK;
-            a.p += A_KM ? k_begin * A.ld : k_begin;
-            b.p += B_KM ? k_begin * B.ld : k_begin;
-            a.k_valid -= k_begin;
-            b.k_valid -= k_begin;
-            gemm_store_tile<A_KM, B_KM>(a, b, (int64_t)(k1 - k0) * BK, st, tm, tn, piece, lds);
-        });
-    } else {
-        int64_t tm, tn;
-        if (tile_of_block(tiles_m, tiles_n, &tm, &tn)) gemm_store_tile<A_KM, B_KM>(A, B, K, st, tm, tn, nullptr, lds);
+            t.R.p += R_KM ? k_begin * R.ld : k_begin;
+            t.C.p += C_KM ? k_begin * C.ld : k_begin;
+            t.R.k_valid -= k_begin;
+            t.C.k_valid -= k_begin;
+            t.K = (int64_t)(k1 - k0) * BK;
+            t.part = parts + (int64_t)r * PART_FLOATS;
+        }
+        int64_t tr, tc;
+        tile_of_item(tile, tiles_r, tiles_c, &tr, &tc);
+        t.R.r0 = tr * BN;
+        t.C.r0 = tc * BM;
+        return t;
+    };
+    if (!queue) {
+        const uint32_t item = item_of_pid(blockIdx.x);
+        if (item >= tiles) return;
+        const ProductTile t = tile_at(item);
+        AccTile acc;
+        gemm_tile<C_KM, R_KM>(acc, t.C, t.R, t.K, lds);
+        store_tile(acc, t, st, pieces, lds);
+        return;
+    }
+    // Whole bf16 pieces leave through slot 4 while the next tile's first loads go to slots 0 .. 3: a tile of
+    // few k-tiles (d_weight of a short batch) otherwise spends more time between its main loops than in them.
+    // The fp32 modes need more LDS than one slot and belong to batches of several slabs, whose tiles are long.
+    const bool ahead = mode == 2 && pieces;
+    ItemQueue q(queue, ts.whole + ts.rest * ts.parts, lds);
+    q.request();
+    q.settle();
+    uint32_t item = q.take_item();
+    if (item == ItemQueue::NONE) return;
+    ProductTile t = tile_at(item);
+    begin_loads<C_KM, R_KM>(t.C, t.R, t.K, lds);
+    for (;;) {
+        AccTile acc;
+        q.request();
+        gemm_loop<C_KM, R_KM>(acc, t.C, t.R, t.K, lds);
+        q.settle();
+        if (!ahead) {
+            store_tile(acc, t, st, pieces, lds);
+            item = q.take_item();
+            if (item == ItemQueue::NONE) return;
+            t = tile_at(item);
+            begin_loads<C_KM, R_KM>(t.C, t.R, t.K, lds);
+            continue;
+        }
+        item = q.take_item();
+        const ProductTile done = t;
+        if (item != ItemQueue::NONE) {
+            t = tile_at(item);
+            begin_loads<C_KM, R_KM>(t.C, t.R, t.K, lds);
+        }
+        lds_barrier();  // every wave has read the queue's word, which lies in slot 4
+        store_tile(acc, done, st, pieces, lds);
+        if (item == ItemQueue::NONE) return;
     }
 }
 
 // Adds the pieces of the split tiles of a gemm_store_kernel launch over `grid` workgroups and stores the
-// sums as that kernel stores a tile.  One wave per 32-row x 64-column block (32 blocks to a tile), four
-// waves to a workgroup; bound by reading the pieces once.
-__global__ void __launch_bounds__(256)
+// sums as that kernel stores a tile.  One workgroup per column group of a tile (as in lmhead_dz_kept_kernel);
+// bound by reading the pieces once.
+__global__ void __launch_bounds__(NTHREADS)
     gemm_reduce_kernel(const float* __restrict__ parts, uint32_t grid, int64_t M, int64_t N, int64_t K, int mode,
                        float* out_f32, uint16_t* out_bf16, int64_t ldo, int64_t m_valid, DynRows dyn) {
+    __shared__ __align__(16) uint16_t stage[GROUP_F32];
     const ProductSizes z = product_sizes(M, K, m_valid, dyn);
     const StoreTo st = {mode, out_f32, out_bf16, ldo, N, z.m_valid, dyn.out_rows, dyn.scale_a, dyn.scale_b};
-    if (!stores_in_pieces(st)) return;
-    const int64_t tiles_m = (z.M + BM - 1) / BM, tiles_n = (N + BN - 1) / BN;
-    const TailSplit ts = plan_tail((uint32_t)(tiles_m * tiles_n), grid, (uint32_t)(z.K / BK));
-    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
-    const uint32_t unit = blockIdx.x * 4 + wave, tile = unit >> 5;
+    const int64_t tiles_r = (z.M + BN - 1) / BN, tiles_c = (N + BM - 1) / BM;
+    const TailSplit ts = plan_tail((uint32_t)(tiles_r * tiles_c), grid, (uint32_t)(z.K / BK));
+    const uint32_t tile = blockIdx.x >> 2;
+    const int j = blockIdx.x & 3, tid = threadIdx.x;
     if (tile >= ts.rest) return;
-    const int w = (unit >> 2) & 7, i = (unit >> 1) & 1, jh = unit & 1;
-    const float* src = parts + (int64_t)tile * PART_FLOATS + ((i * 4 + jh * 2) * 4 * NTHREADS + w * 64 + lane) * 4;
-    oi_f32x4 sum[8];
+    const float* src = parts + (int64_t)tile * PART_FLOATS + tid * 4;
+    oi_f32x4 sum[2][4];
 #pragma unroll
-    for (int k = 0; k < 8; ++k) sum[k] = *reinterpret_cast<const oi_f32x4*>(src + k * NTHREADS * 4);
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) sum[i][q] = *reinterpret_cast<const oi_f32x4*>(src + part_group(i, j, q) * PART_GROUP);
     for (uint32_t p = 1; p < ts.parts; ++p) {
         src += (int64_t)ts.rest * PART_FLOATS;
 #pragma unroll
-        for (int k = 0; k < 8; ++k) sum[k] += *reinterpret_cast<const oi_f32x4*>(src + k * NTHREADS * 4);
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+                sum[i][q] += *reinterpret_cast<const oi_f32x4*>(src + part_group(i, j, q) * PART_GROUP);
     }
-    int64_t tm, tn;
-    tile_of_item(ts.whole + tile, (uint32_t)tiles_m, (uint32_t)tiles_n, &tm, &tn);
-    const LaneRows r = lane_rows(st, tm * BM + (w & 3) * 64 + i * 32, lane);
-    store_block(st, r, tn * BN + (w >> 2) * 128 + jh * 64, lane, [&](int jj, int q, int e) { return sum[jj * 4 + q][e]; });
+    f32x16 acc[2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[i][r] = sum[i][r >> 2][r & 3];
+    int64_t tr, tc;
+    tile_of_item(ts.whole + tile, (uint32_t)tiles_r, (uint32_t)tiles_c, &tr, &tc);
+    store_group_f32(acc[0], acc[1], st, stores_in_pieces(st), tr * BN, tc * BM, j, stage, tid);
 }
 
 inline int64_t round_up(int64_t x, int64_t m) { return (x + m - 1) / m * m; }
@@ -1834,7 +1899,7 @@ void launch_rows_product(unsigned grid, const Operand& a, int64_t M, const Opera
     if (!parts) return;
     const int64_t tiles = (M + BM - 1) / BM * ((N + BN - 1) / BN);
     const int64_t most = tiles < (int64_t)grid ? tiles : (int64_t)grid - 1;  // tiles past the last whole round
-    hipLaunchKernelGGL(gemm_reduce_kernel, dim3((unsigned)(most * 8)), dim3(256), 0, s, parts, grid, M, N, K, mode,
+    hipLaunchKernelGGL(gemm_reduce_kernel, dim3((unsigned)(most * 4)), dim3(NTHREADS), 0, s, parts, grid, M, N, K, mode,
                        out_f32, o16, ldo, m_valid, dyn);
 }
 

@@ -92,3 +92,35 @@ def test_products_cut_along_the_vocabulary(n, h, v, route):
     assert (hid.grad[~mask] == 0).all()
     if w.requires_grad:
         _close(w.grad, dw, "d_weight")
+
+
+@pytest.mark.parametrize("n,h,v", [(70, 64, 301), (300, 320, 513)])
+def test_gradients_off_16_byte_boundaries(n, h, v):
+    """Gradients that lie on 4-byte boundaries only are stored by another route of the same epilogue."""
+    print("case unaligned gradients", n, h, v, flush=True)
+    g = torch.Generator().manual_seed(n)
+    hidden = torch.randn(n, h, generator=g).bfloat16().to(DEV)
+    weight = (torch.randn(v, h, generator=g) * 0.2).bfloat16().to(DEV)
+    labels = torch.randint(0, v, (n,), generator=g).to(DEV)
+    up = torch.rand(n, generator=g).to(DEV)
+    lib = _lib.load()
+    stream = torch.cuda.current_stream().cuda_stream
+    lp, lse = torch.empty(n, device=DEV), torch.empty(n, device=DEV)
+    ws_bytes = max(lib.oi_lmhead_fwd_workspace_bytes(n, h, v, 0), lib.oi_lmhead_bwd_workspace_bytes(n, h, v, 1, 0))
+    ws = torch.empty(ws_bytes, dtype=torch.uint8, device=DEV)
+    p = lambda t: t.data_ptr()  # noqa: E731
+    assert lib.oi_lmhead_logp_fwd(p(hidden), p(weight), p(labels), None, n, h, v, 1.0, p(lp), None, p(lse), p(ws), ws_bytes, stream) == 0
+    got = []
+    for shift in (0, 2):
+        dh = torch.full((n * h + 16,), 7.0, dtype=torch.bfloat16, device=DEV)
+        dw = torch.full((v * h + 16,), 7.0, dtype=torch.bfloat16, device=DEV)
+        rc = lib.oi_lmhead_logp_bwd(
+            p(hidden), p(weight), p(labels), p(lse), p(up), None, 0, n, h, v, 1.0, p(lp), p(dh[shift:]), p(dw[shift:]),
+            p(ws), ws_bytes, stream,
+        )  # fmt: skip
+        assert rc == 0
+        for t, size in ((dh, n * h), (dw, v * h)):  # nothing written around them
+            assert (t[:shift] == 7).all() and (t[shift + size :] == 7).all()
+        got.append((dh[shift : shift + n * h], dw[shift : shift + v * h]))
+    for a, b in zip(*got):
+        assert a.float().abs().max() > 0 and torch.equal(a, b)
