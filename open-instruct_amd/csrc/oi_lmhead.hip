@@ -534,7 +534,7 @@ __device__ __forceinline__ void merge_stats(float ma, float sa, float ta, float 
 // binary orders above its label's (tokens beyond that are flagged by the merge kernel and take the
 // recomputing backward).
 template <bool PARTIAL, bool KEEP>
-__device__ __forceinline__ void stats_update(AccTile& acc, int j, int wm, int lane, int64_t m0, int64_t vocab, float c,
+__device__ __forceinline__ void stats_update(f32x16 (&z)[2], int wm, int lane, int64_t m0, int64_t vocab, float c,
                                              float ref, float& st_m, float& st_s, float& st_t) {
     // the maximum is taken over the unscaled logits (c > 0) and every exponent is one fma: the new
     // maximum is the rounded product max(z) * c while the exponents are rounded once, so the largest
@@ -544,7 +544,7 @@ __device__ __forceinline__ void stats_update(AccTile& acc, int j, int wm, int la
     for (int i = 0; i < 2; ++i)
 #pragma unroll
         for (int r = 0; r < 16; ++r)
-            if (!PARTIAL || m0 + acc_row(wm, i, r, lane) < vocab) zmax = fmaxf(zmax, acc[i][j][r]);
+            if (!PARTIAL || m0 + acc_row(wm, i, r, lane) < vocab) zmax = fmaxf(zmax, z[i][r]);
     const float mn = fmaxf(st_m, fmaxf(zmax * c, OI_NEG_BIG));
     const float shift = st_m - mn;
     const float alpha = __builtin_amdgcn_exp2f(shift);
@@ -555,7 +555,7 @@ __device__ __forceinline__ void stats_update(AccTile& acc, int j, int wm, int la
     for (int i = 0; i < 2; ++i)
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
-            float d = fmaf(acc[i][j][r], c, -mn);
+            float d = fmaf(z[i][r], c, -mn);
             float e = __builtin_amdgcn_exp2f(d);
             if (PARTIAL && m0 + acc_row(wm, i, r, lane) >= vocab) {
                 d = 0.f;
@@ -563,49 +563,36 @@ __device__ __forceinline__ void stats_update(AccTile& acc, int j, int wm, int la
             }
             s += e;
             t = fmaf(e, d, t);
-            if (KEEP) acc[i][j][r] = e * pow2_max;
+            if (KEEP) z[i][r] = e * pow2_max;
         }
     st_m = mn;
     st_s = s;
     st_t = t;
 }
 
-// A finished tile leaves as a bf16 image [256 tokens][256 vocabulary columns] through the LDS (rows of
-// STAGE_STRIDE entries; the two 8-byte halves of every 16-byte piece swapped in rows 8..15 of each
-// 16, which keeps the 8-byte stores of a wave off each other's banks), and from there to global
-// memory in 16-byte pieces of whole 512-byte rows.  Rows at or past rows_valid are written as zeros.
-// It leaves one column group at a time: group j holds the 64 tokens wn*128 + j*32 + (0..31) of both
-// wn halves with all 256 vocabulary columns (every m-wave contributes its 64), i.e. 64 whole rows of
-// the image, and goes to global memory while the next group's statistics are still being computed
-// (forward per slab at the Llama-3.1-8B shape: 6.32 -> 6.28 ms against the whole image at the end, and
-// fewer live registers).
-__device__ __forceinline__ void stage_group_bf16(const AccTile& acc, uint16_t* stage, int wm, int wn, int lane, int j) {
-    asm volatile("" : "+v"(lane));
-    const int nl = acc_col(wn, j, lane);
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            const int vl = acc_row(wm, i, q * 4, lane) ^ (((nl >> 3) & 1) << 2);
-            const uint2 pk = make_uint2(oi_pack_bf16x2(acc[i][j][q * 4], acc[i][j][q * 4 + 1]),
-                                        oi_pack_bf16x2(acc[i][j][q * 4 + 2], acc[i][j][q * 4 + 3]));
-            *reinterpret_cast<uint2*>(stage + nl * STAGE_STRIDE + vl) = pk;
-        }
+// A finished tile leaves as bf16 rows of 256 columns one column group at a time: group j holds the 64 rows
+// (tokens, or rows of a product) wn * 128 + j * 32 + (0..31) of both wn halves with all 256 columns (every m-wave
+// contributes its 64).  A lane holds groups of four consecutive columns of one row; they meet in a region of one
+// ring slot and go to global memory in 16-byte pieces of whole 512-byte rows, while the next group's work is being
+// done (forward per slab at the Llama-3.1-8B shape: 6.32 -> 6.28 ms against the whole image at the end).
+//
+// The region: 64 rows of 512 bytes, unpadded; the 16-byte pieces of a row at c ^ (row mod 32) and their halves
+// swapped in rows 16 .. 31 of every 32, which puts the 8-byte stores of 32 lanes on all 64 banks.
+constexpr int GROUP_ROWS = 64;
+constexpr int GROUP_BF16_AT = 4 * TILE_ELEMS;  // ring slot 4: slots 0 .. 3 may be filling for the next tile
+static_assert(GROUP_ROWS * BM <= TILE_ELEMS, "a bf16 group fits one ring slot");
+__device__ __forceinline__ int64_t group_row(int64_t row0, int j, int r) { return row0 + (r >> 5) * 128 + j * 32 + (r & 31); }
+// columns acc_row(wm, i, 4 q .. 4 q + 3, lane) of the lane's row
+__device__ __forceinline__ void stage_bf16x4(uint16_t* stage, int wm, int wn, int lane, int i, int q, float a, float b, float c,
+                                             float d) {
+    const int srow = wn * 32 + (lane & 31);
+    const int piece = (wm * 8 + i * 4 + q) ^ (srow & 31), half = (lane >> 5) ^ ((srow >> 4) & 1);
+    *reinterpret_cast<uint2*>(stage + srow * BM + piece * 8 + half * 4) = make_uint2(oi_pack_bf16x2(a, b), oi_pack_bf16x2(c, d));
 }
-__device__ __forceinline__ void copy_staged_group(const uint16_t* stage, uint16_t* __restrict__ dst, int64_t ld, int tid,
-                                                  int rows_valid, int j) {
-    // the lane's addresses are formed here, where they are used, not ahead of the tile's main loop
-    asm volatile("" : "+v"(tid));
-#pragma unroll 1
-    for (int it = 0; it < 4; ++it) {
-        const int cidx = tid + it * NTHREADS;
-        const int r = cidx >> 5, ch = cidx & 31;                 // r: 0..63 within the group
-        const int row = (r >> 5) * 128 + j * 32 + (r & 31);      // row of the image = token of the tile
-        oi_u32x4 v = *reinterpret_cast<const oi_u32x4*>(stage + row * STAGE_STRIDE + ch * 8);
-        if (row & 8) v = oi_u32x4{v.z, v.w, v.x, v.y};
-        if (row >= rows_valid) v = oi_u32x4{0u, 0u, 0u, 0u};
-        *reinterpret_cast<oi_u32x4*>(dst + (int64_t)row * ld + ch * 8) = v;
-    }
+constexpr int GROUP_PIECES = GROUP_ROWS * (BM / 8) / NTHREADS;  // 16-byte pieces per thread
+__device__ __forceinline__ oi_u32x4 staged_piece(const uint16_t* stage, int r, int ch) {
+    const oi_u32x4 v = *reinterpret_cast<const oi_u32x4*>(stage + r * BM + (ch ^ (r & 31)) * 8);
+    return (r & 16) ? oi_u32x4{v.z, v.w, v.x, v.y} : v;
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -632,140 +619,177 @@ struct FwdLaunch {
 };
 enum FwdKeep { FWD_PLAIN, FWD_EXPONENTIALS, FWD_LOGITS };
 
+// what a forward tile is folded into, and from
+struct FwdArgs {
+    const uint16_t *W, *hidden;
+    const int64_t* labels;
+    int64_t n_tokens, hdim, vocab;
+    float c;
+    int64_t n_pad;
+    float4* partial;
+    float* zy;
+};
+// running statistics of one token column of a lane, its reference exponent and its label (vocabulary ids fit
+// 32 bits: vocab <= 2^22)
+struct FwdColumn {
+    float m, s, t, ref;
+    int lab;
+};
+__device__ __forceinline__ FwdColumn fwd_column(const FwdArgs& a, const float* xref, int64_t n) {
+    FwdColumn col = {OI_NEG_BIG, 0.f, 0.f, (xref && n < a.n_tokens) ? xref[n] : 0.f, 0};
+    const int64_t y = n < a.n_tokens ? a.labels[n] : 0;
+    col.lab = (int)(y < 0 ? 0 : (y >= a.vocab ? a.vocab - 1 : y));
+    // in a register now: a wait for these loads later on would also wait for whatever was requested since
+    asm volatile("" : "+v"(col.lab), "+v"(col.ref));
+    return col;
+}
+// Column group j of vocabulary tile vt: the label's logit, the statistics and, where they are kept, the
+// exponentials (through `stage`; every thread of the workgroup takes part).
 template <FwdKeep KEEP>
-__device__ __forceinline__ void lmhead_fwd_item(const uint16_t* __restrict__ W, const uint16_t* __restrict__ hidden,
-                                                const int64_t* __restrict__ labels, int64_t n_tokens, int64_t hdim,
-                                                int64_t vocab, float c, const FwdLaunch& fl, int64_t n_pad,
-                                                float4* __restrict__ partial, float* __restrict__ zy, int64_t split,
-                                                int64_t tt, uint16_t* lds) {
+__device__ __forceinline__ void fwd_fold(f32x16 (&__restrict__ z)[2], FwdColumn& col, const FwdArgs& a, const FwdLaunch& fl,
+                                         int64_t vt, int64_t n0, int j, int tid, uint16_t* stage) {
     constexpr bool CACHE = KEEP == FWD_EXPONENTIALS;
-    const int64_t tiles_per_split = fl.tiles_per_split, long_splits = fl.long_splits;
-    const int64_t vocab_tiles = (vocab + BM - 1) / BM;
+    asm volatile("" : "+v"(tid));  // addresses are formed here, not ahead of the tile's main loop
+    const int lane = tid & 63, wave = tid >> 6, wm = wave & 3, wn = wave >> 2;
+    const int64_t m0 = vt * BM;
+    // the target logit, when its row falls into this wave's 64 rows
+    const int rel = col.lab - ((int)m0 + wm * 64);
+    // register of this lane that holds the label's row, -1 when another lane or wave does
+    int label_reg = -1;
+    if (rel >= 0 && rel < 64) {
+        const int rr = rel & 31;
+        if (((rr >> 2) & 1) == (lane >> 5)) label_reg = (rel >> 5) * 16 + (rr >> 3) * 4 + (rr & 3);
+    }
+    if (label_reg >= 0) {
+        float v = 0.f;
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int r = 0; r < 16; ++r)
+                if (i * 16 + r == label_reg) v = z[i][r];
+        const int64_t n = n0 + acc_col(wn, j, lane);
+        if (n < a.n_tokens) a.zy[n] = v;
+    }
+    if (m0 + BM > a.vocab)
+        stats_update<true, CACHE>(z, wm, lane, m0, a.vocab, a.c, col.ref, col.m, col.s, col.t);
+    else
+        stats_update<false, CACHE>(z, wm, lane, m0, a.vocab, a.c, col.ref, col.m, col.s, col.t);
+    if constexpr (CACHE) {
+        if (fl.skip_label && label_reg >= 0) {
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+#pragma unroll
+                for (int r = 0; r < 16; ++r)
+                    if (i * 16 + r == label_reg) z[i][r] = 0.f;
+        }
+        if (vt < fl.cache_tile0 || vt >= fl.cache_tile0 + fl.cache_tiles) return;
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+                stage_bf16x4(stage, wm, wn, lane, i, q, z[i][q * 4], z[i][q * 4 + 1], z[i][q * 4 + 2],
+                             z[i][q * 4 + 3]);
+        lds_barrier();
+        uint16_t* dst = fl.ecache + n0 * fl.cache_ld + (vt - fl.cache_tile0) * BM;
+#pragma unroll 1
+        for (int it = 0; it < GROUP_PIECES; ++it) {
+            const int r = (tid >> 5) + it * (NTHREADS / 32);
+            const int64_t row = group_row(0, j, r);  // token of the tile
+            const oi_u32x4 v = staged_piece(stage, r, tid & 31);
+            *reinterpret_cast<oi_u32x4*>(dst + row * fl.cache_ld + (tid & 31) * 8) =
+                n0 + row < a.n_tokens ? v : oi_u32x4{0u, 0u, 0u, 0u};
+        }
+        lds_barrier();  // the region is free for the next group
+        __builtin_amdgcn_sched_barrier(0);
+    }
+}
+// the statistics of the lane's column meet those of the other lane half (same token, other rows), which leaves
+// them in lanes 0 .. 31
+__device__ __forceinline__ void fwd_merge_halves(FwdColumn& col) {
+    const float om = __shfl_xor(col.m, 32, OI_WAVE), os = __shfl_xor(col.s, 32, OI_WAVE), ot = __shfl_xor(col.t, 32, OI_WAVE);
+    float m, s, t;
+    merge_stats(col.m, col.s, col.t, om, os, ot, &m, &s, &t);
+    col.m = m;
+    col.s = s;
+    col.t = t;
+}
+// of `columns` tokens, red [4 m-waves][columns][3] to the partial statistics of a split (tid < columns)
+__device__ __forceinline__ float4 fwd_merge_waves(const float* red, int columns, int tid) {
+    float m = red[tid * 3], s = red[tid * 3 + 1], t = red[tid * 3 + 2];
+#pragma unroll
+    for (int w = 1; w < 4; ++w) {
+        const float* p = red + (w * columns + tid) * 3;
+        merge_stats(m, s, t, p[0], p[1], p[2], &m, &s, &t);
+    }
+    return make_float4(m, s, t, 0.f);
+}
+
+template <FwdKeep KEEP>
+__device__ __forceinline__ void lmhead_fwd_item(const FwdArgs& a, const FwdLaunch& fl, int64_t split, int64_t tt,
+                                                uint16_t* lds) {
+    const int64_t vocab_tiles = (a.vocab + BM - 1) / BM;
     // the first long_splits splits take tiles_per_split vocabulary tiles each, the others one
-    const bool long_item = split < long_splits;
-    const int64_t vt_begin = long_item ? split * tiles_per_split : long_splits * tiles_per_split + (split - long_splits);
-    int64_t vt_end = vt_begin + (long_item ? tiles_per_split : 1);
+    const bool long_item = split < fl.long_splits;
+    const int64_t vt_begin =
+        long_item ? split * fl.tiles_per_split : fl.long_splits * fl.tiles_per_split + (split - fl.long_splits);
+    int64_t vt_end = vt_begin + (long_item ? fl.tiles_per_split : 1);
     vt_end = vt_end < vocab_tiles ? vt_end : vocab_tiles;
 
     const int tid = opaque_tid(), lane = tid & 63, wave = tid >> 6, wm = wave & 3, wn = wave >> 2;
     const int64_t n0 = tt * BN;
+    const Operand tokens = {a.hidden, a.hdim, n0, a.n_tokens, a.hdim};
+    Operand rows = {a.W, a.hdim, vt_begin * BM, a.vocab, a.hdim};
 
-    float st_m[4], st_s[4], st_t[4], ref[4];
-    int lab[4];  // vocabulary ids fit 32 bits (vocab <= 2^22)
+    FwdColumn col[4];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        st_m[j] = OI_NEG_BIG;
-        st_s[j] = 0.f;
-        st_t[j] = 0.f;
-        const int64_t n = n0 + acc_col(wn, j, lane);
-        int64_t y = n < n_tokens ? labels[n] : 0;
-        lab[j] = (int)(y < 0 ? 0 : (y >= vocab ? vocab - 1 : y));
-        ref[j] = (CACHE && fl.xref && n < n_tokens) ? fl.xref[n] : 0.f;
-    }
+    for (int j = 0; j < 4; ++j)
+        col[j] = fwd_column(a, KEEP == FWD_EXPONENTIALS ? fl.xref : nullptr, n0 + acc_col(wn, j, lane));
 
+    begin_loads<false, false>(rows, tokens, a.hdim, lds);
     for (int64_t vt = vt_begin; vt < vt_end; ++vt) {
         AccTile acc;
-        const int64_t m0 = vt * BM;
-        gemm_tile(acc, W, hdim, m0, vocab, hidden, hdim, n0, n_tokens, hdim, lds);
+        gemm_loop<false, false>(acc, rows, tokens, a.hdim, lds);
+        // the next tile's first loads run beside this tile's statistics, which leave slots 0 .. 3 alone (scoring
+        // pass of 1432 rows, 4096 x 128256: 1.435 -> 1.40 ms; steps 0.2 to 0.6 %)
+        rows.r0 += BM;
+        if (vt + 1 < vt_end) begin_loads<false, false>(rows, tokens, a.hdim, lds);
         // leaves while the statistics are computed
         if (KEEP == FWD_LOGITS) store_part(acc, fl.logits + (vt * fl.logits_tiles + tt) * PART_FLOATS, tid);
-        const bool partial_tile = m0 + BM > vocab;
-        const bool keep_tile = CACHE && vt >= fl.cache_tile0 && vt < fl.cache_tile0 + fl.cache_tiles;
-        const int wave_row0 = (int)m0 + wm * 64;
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
-            // the target logit, when its row falls into this wave's 64 rows
-            const int rel = lab[j] - wave_row0;
-            // register of this lane that holds the label's row, -1 when another lane or wave does
-            int label_reg = -1;
-            if (rel >= 0 && rel < 64) {
-                const int rr = rel & 31;
-                if (((rr >> 2) & 1) == (lane >> 5)) label_reg = (rel >> 5) * 16 + (rr >> 3) * 4 + (rr & 3);
-            }
-            if (label_reg >= 0) {
-                float v = 0.f;
-#pragma unroll
-                for (int i = 0; i < 2; ++i)
-#pragma unroll
-                    for (int r = 0; r < 16; ++r)
-                        if (i * 16 + r == label_reg) v = acc[i][j][r];
-                const int64_t n = n0 + acc_col(wn, j, lane);
-                if (n < n_tokens) zy[n] = v;
-            }
-            if (partial_tile)
-                stats_update<true, CACHE>(acc, j, wm, lane, m0, vocab, c, ref[j], st_m[j], st_s[j], st_t[j]);
-            else
-                stats_update<false, CACHE>(acc, j, wm, lane, m0, vocab, c, ref[j], st_m[j], st_s[j], st_t[j]);
-            if (CACHE && fl.skip_label && label_reg >= 0) {
-#pragma unroll
-                for (int i = 0; i < 2; ++i)
-#pragma unroll
-                    for (int r = 0; r < 16; ++r)
-                        if (i * 16 + r == label_reg) acc[i][j][r] = 0.f;
-            }
-            if (CACHE && keep_tile) {
-                // the operand ring is free (the product ended with a barrier); the groups use disjoint rows
-                // of the image, so one barrier per group (written -> read out) is all they need
-                __builtin_amdgcn_sched_barrier(0);
-                stage_group_bf16(acc, lds, wm, wn, lane, j);
-                lds_barrier();
-                const int64_t left = n_tokens - n0;
-                copy_staged_group(lds, fl.ecache + n0 * fl.cache_ld + (vt - fl.cache_tile0) * BM, fl.cache_ld, tid,
-                                  (int)(left < BN ? left : BN), j);
-                __builtin_amdgcn_sched_barrier(0);
-            }
+            f32x16 z[2] = {acc[0][j], acc[1][j]};
+            fwd_fold<KEEP>(z, col[j], a, fl, vt, n0, j, tid, lds + GROUP_BF16_AT);
         }
-        // the next tile's first loads must wait until the image has been read out again
-        if (CACHE && keep_tile) lds_barrier();
     }
 
-    // merge the two lane halves (same token, other rows), then the four m-waves through LDS
     float* red = reinterpret_cast<float*>(lds);  // [4 wm][256 tokens][3]
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-        const float om = __shfl_xor(st_m[j], 32, OI_WAVE), os = __shfl_xor(st_s[j], 32, OI_WAVE),
-                    ot = __shfl_xor(st_t[j], 32, OI_WAVE);
-        float mn, s, t;
-        merge_stats(st_m[j], st_s[j], st_t[j], om, os, ot, &mn, &s, &t);
+        fwd_merge_halves(col[j]);
         if (lane < 32) {
             float* p = red + (wm * 256 + acc_col(wn, j, lane)) * 3;
-            p[0] = mn;
-            p[1] = s;
-            p[2] = t;
+            p[0] = col[j].m;
+            p[1] = col[j].s;
+            p[2] = col[j].t;
         }
     }
-    __syncthreads();
-    if (tid < 256) {
-        float m = red[tid * 3], s = red[tid * 3 + 1], t = red[tid * 3 + 2];
-#pragma unroll
-        for (int w = 1; w < 4; ++w) {
-            const float* p = red + (w * 256 + tid) * 3;
-            merge_stats(m, s, t, p[0], p[1], p[2], &m, &s, &t);
-        }
-        const int64_t n = n0 + tid;
-        if (n < n_tokens) partial[split * n_pad + n] = make_float4(m, s, t, 0.f);
-    }
+    lds_barrier();
+    if (tid < 256 && n0 + tid < a.n_tokens) a.partial[split * a.n_pad + n0 + tid] = fwd_merge_waves(red, 256, tid);
 }
 
 template <FwdKeep KEEP>
 __global__ void __launch_bounds__(NTHREADS)
-    lmhead_fwd_kernel(const uint16_t* __restrict__ W, const uint16_t* __restrict__ hidden,
-                      const int64_t* __restrict__ labels, int64_t n_tokens, const int32_t* __restrict__ n_dev,
-                      int64_t hdim, int64_t vocab, float c, FwdLaunch fl, int64_t n_pad, float4* __restrict__ partial,
-                      float* __restrict__ zy, uint32_t* __restrict__ queue) {
+    lmhead_fwd_kernel(FwdArgs a, const int32_t* __restrict__ n_dev, FwdLaunch fl, uint32_t* __restrict__ queue) {
     __shared__ __align__(16) uint16_t lds[LDS_ELEMS];
-    if (n_dev) n_tokens = *n_dev;  // rows selected on the device: the host only knows an upper bound
-    const int64_t token_tiles = (n_tokens + BN - 1) / BN;
+    if (n_dev) a.n_tokens = *n_dev;  // rows selected on the device: the host only knows an upper bound
+    const int64_t token_tiles = (a.n_tokens + BN - 1) / BN;
     // every long item of every XCD's queue is taken before the first short one: the short items are
     // there to fill the end of the launch
-    for_each_tile(queue, fl.n_first, token_tiles, lds, [&](int64_t split, int64_t tt) {
-        lmhead_fwd_item<KEEP>(W, hidden, labels, n_tokens, hdim, vocab, c, fl, n_pad, partial, zy, fl.first + split, tt,
-                              lds);
-    });
-    for_each_tile(queue + QUEUE_WORDS, fl.n_second, token_tiles, lds, [&](int64_t split, int64_t tt) {
-        lmhead_fwd_item<KEEP>(W, hidden, labels, n_tokens, hdim, vocab, c, fl, n_pad, partial, zy,
-                              fl.long_splits + split, tt, lds);
-    });
+    for_each_tile(queue, fl.n_first, token_tiles, lds,
+                  [&](int64_t split, int64_t tt) { lmhead_fwd_item<KEEP>(a, fl, fl.first + split, tt, lds); });
+    for_each_tile(queue + QUEUE_WORDS, fl.n_second, token_tiles, lds,
+                  [&](int64_t split, int64_t tt) { lmhead_fwd_item<KEEP>(a, fl, fl.long_splits + split, tt, lds); });
 }
 
 // A token whose largest scaled logit lies more than this many binary orders above its reference
@@ -1020,11 +1044,8 @@ __device__ __forceinline__ bool stores_in_pieces(const StoreTo& st) {
 // tiles of 5 k-tiles) 606 us; through the LDS 544; without waiting for stores at its barriers 504; with the next tile's
 // first loads ahead of it 478.
 constexpr int STAGE_F32 = BM + 4;                            // floats per row: rows 4 banks apart
-constexpr int GROUP_ROWS = 64;
 constexpr int GROUP_F32 = GROUP_ROWS * STAGE_F32 * 2;        // LDS elements of an fp32 region
 static_assert(2 * GROUP_F32 <= LDS_ELEMS, "the epilogue's regions fit the ring");
-constexpr int GROUP_BF16_AT = 4 * TILE_ELEMS;                // the bf16 region is ring slot 4
-static_assert(GROUP_ROWS * BM <= TILE_ELEMS, "a bf16 group fits one ring slot");
 struct RowScale {
     float a, b;
     bool on;
@@ -1040,8 +1061,6 @@ __device__ __forceinline__ RowScale row_scale(const StoreTo& st, int64_t row) {
     }
     return s;
 }
-__device__ __forceinline__ int64_t group_row(int64_t row0, int j, int r) { return row0 + (r >> 5) * 128 + j * 32 + (r & 31); }
-
 // mode 2 in whole pieces
 __device__ __forceinline__ void store_group_bf16(const f32x16& z0, const f32x16& z1, const StoreTo& st, int64_t row0,
                                                  int64_t col0, int j, uint16_t* stage, int tid) {
@@ -1049,34 +1068,25 @@ __device__ __forceinline__ void store_group_bf16(const f32x16& z0, const f32x16&
     const int lane = tid & 63, wave = tid >> 6, wm = wave & 3, wn = wave >> 2;
     const int srow = wn * 32 + (lane & 31);
     const RowScale sc = row_scale(st, group_row(row0, j, srow));
-    // 64 rows of 512 bytes, unpadded; the 16-byte pieces of a row at c ^ (row mod 32) and their halves swapped in
-    // rows 16 .. 31 of every 32, which puts the 8-byte stores of 32 lanes on all 64 banks
 #pragma unroll
     for (int i = 0; i < 2; ++i)
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
             const f32x16& z = i == 0 ? z0 : z1;
-            const int piece = (wm * 8 + i * 4 + q) ^ (srow & 31), half = (lane >> 5) ^ ((srow >> 4) & 1);
-            *reinterpret_cast<uint2*>(stage + srow * BM + piece * 8 + half * 4) =
-                make_uint2(oi_pack_bf16x2(sc(z[q * 4]), sc(z[q * 4 + 1])), oi_pack_bf16x2(sc(z[q * 4 + 2]), sc(z[q * 4 + 3])));
+            stage_bf16x4(stage, wm, wn, lane, i, q, sc(z[q * 4]), sc(z[q * 4 + 1]), sc(z[q * 4 + 2]), sc(z[q * 4 + 3]));
         }
     lds_barrier();
-    constexpr int ITERS = GROUP_ROWS * (BM / 8) / NTHREADS;
-    oi_u32x4 v[ITERS];
+    oi_u32x4 v[GROUP_PIECES];
 #pragma unroll
-    for (int it = 0; it < ITERS; ++it) {
-        const int cidx = tid + it * NTHREADS, r = cidx >> 5, ch = cidx & 31;
-        v[it] = *reinterpret_cast<const oi_u32x4*>(stage + r * BM + (ch ^ (r & 31)) * 8);
-    }
+    for (int it = 0; it < GROUP_PIECES; ++it) v[it] = staged_piece(stage, (tid >> 5) + it * (NTHREADS / 32), tid & 31);
     lds_barrier();  // the region is free for the next group
+    const int64_t col = col0 + (tid & 31) * 8;
 #pragma unroll
-    for (int it = 0; it < ITERS; ++it) {
-        const int cidx = tid + it * NTHREADS, r = cidx >> 5, ch = cidx & 31;
-        const int64_t row = group_row(row0, j, r), col = col0 + ch * 8;
+    for (int it = 0; it < GROUP_PIECES; ++it) {
+        const int64_t row = group_row(row0, j, (tid >> 5) + it * (NTHREADS / 32));
         if (row >= st.m_valid || col >= st.N) continue;
         const int64_t dst = st.out_rows ? (int64_t)st.out_rows[row] : row;
-        *reinterpret_cast<oi_u32x4*>(st.out_bf16 + dst * st.ldo + col) =
-            (r & 16) ? oi_u32x4{v[it].z, v[it].w, v[it].x, v[it].y} : v[it];
+        *reinterpret_cast<oi_u32x4*>(st.out_bf16 + dst * st.ldo + col) = v[it];
     }
 }
 
@@ -1868,19 +1878,17 @@ void enqueue_fwd(const FwdPlan& p, char* ws, const RowInputs& in, const uint8_t*
     uint32_t* queue = reinterpret_cast<uint32_t*>(ws + p.off_queue);
     const float c = inv_temperature * OI_LOG2E;
     const dim3 grid(resident_grid(p.n_splits, p.token_tiles));
-    const uint16_t* Wp = static_cast<const uint16_t*>(weight);
+    const FwdArgs fa = {static_cast<const uint16_t*>(weight), in.hidden, in.labels, n_tokens, hidden_dim, vocab, c,
+                        p.n_pad, partial, zy};
     const FwdLaunch fl = {p.tiles_per_split, p.long_splits, 0, p.long_splits, p.n_splits - p.long_splits,
                           keep.buf, keep.ld, 0, keep.buf ? keep.tiles : 0, 0, keep.xref, keep.logits, p.token_tiles};
     if (keep.buf) {
         const ProbeScope probe(0, s);
-        hipLaunchKernelGGL(lmhead_fwd_kernel<FWD_EXPONENTIALS>, grid, dim3(NTHREADS), 0, s, Wp, in.hidden, in.labels, n_tokens,
-                           in.n_dev, hidden_dim, vocab, c, fl, p.n_pad, partial, zy, queue);
+        hipLaunchKernelGGL(lmhead_fwd_kernel<FWD_EXPONENTIALS>, grid, dim3(NTHREADS), 0, s, fa, in.n_dev, fl, queue);
     } else if (keep.logits)
-        hipLaunchKernelGGL(lmhead_fwd_kernel<FWD_LOGITS>, grid, dim3(NTHREADS), 0, s, Wp, in.hidden, in.labels, n_tokens,
-                           in.n_dev, hidden_dim, vocab, c, fl, p.n_pad, partial, zy, queue);
+        hipLaunchKernelGGL(lmhead_fwd_kernel<FWD_LOGITS>, grid, dim3(NTHREADS), 0, s, fa, in.n_dev, fl, queue);
     else
-        hipLaunchKernelGGL(lmhead_fwd_kernel<FWD_PLAIN>, grid, dim3(NTHREADS), 0, s, Wp, in.hidden, in.labels, n_tokens,
-                           in.n_dev, hidden_dim, vocab, c, fl, p.n_pad, partial, zy, queue);
+        hipLaunchKernelGGL(lmhead_fwd_kernel<FWD_PLAIN>, grid, dim3(NTHREADS), 0, s, fa, in.n_dev, fl, queue);
     hipLaunchKernelGGL(lmhead_fwd_combine_kernel, dim3((unsigned)((n_tokens + COMBINE_TOKENS - 1) / COMBINE_TOKENS)),
                        dim3(COMBINE_THREADS), 0, s, partial,
                        zy, n_tokens, in.n_dev, in.rows, row_mask, n_tokens, p.n_splits, p.n_pad, inv_temperature, c, logprob,
@@ -1927,6 +1935,7 @@ void enqueue_fwd_wsum(const FwdPlan& p, char* ws, const RowInputs& in, const uin
     const int64_t h_tiles = (hidden_dim + BN - 1) / BN;
     const int64_t v_pad = p.vocab_tiles * BM;
     const int64_t splits_per_chunk = (p.chunk / BM + p.tiles_per_split - 1) / p.tiles_per_split;
+    const FwdArgs fa = {Wp, in.hidden, in.labels, n_tokens, hidden_dim, vocab, c, p.n_pad, partial, zy};
     launch_label_ref(in, weight, n_tokens, hidden_dim, vocab, inv_temperature, xref, s);
     for (int64_t ci = 0; ci < p.n_chunks; ++ci) {
         const int64_t v_begin = ci * p.chunk;
@@ -1938,8 +1947,8 @@ void enqueue_fwd_wsum(const FwdPlan& p, char* ws, const RowInputs& in, const uin
         uint32_t* q = queues + ci * (FWD_QUEUE_WORDS + QUEUE_WORDS);
         const FwdLaunch fl = {p.tiles_per_split, p.long_splits, first, n_first, 0, chunk_buf, cols, v_begin / BM,
                               cols / BM, 1, xref, nullptr, 0};
-        hipLaunchKernelGGL(lmhead_fwd_kernel<FWD_EXPONENTIALS>, dim3(resident_grid(n_first, p.token_tiles)), dim3(NTHREADS), 0, s, Wp,
-                           in.hidden, in.labels, n_tokens, in.n_dev, hidden_dim, vocab, c, fl, p.n_pad, partial, zy, q);
+        hipLaunchKernelGGL(lmhead_fwd_kernel<FWD_EXPONENTIALS>, dim3(resident_grid(n_first, p.token_tiles)), dim3(NTHREADS), 0, s, fa,
+                           in.n_dev, fl, q);
         const Operand a = {chunk_buf, cols, 0, p.n_pad, cols};
         const Operand b = {Wp + v_begin * hidden_dim, hidden_dim, 0, hidden_dim, valid};
         const DynRows dyn = {in.n_dev, 1, nullptr, nullptr, nullptr, nullptr};

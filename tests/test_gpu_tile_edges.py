@@ -11,7 +11,7 @@ import types
 import pytest
 import torch
 
-from open_instruct_amd import grpo_utils, lm_head
+from open_instruct_amd import _lib, grpo_utils, lm_head
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
