@@ -1510,6 +1510,16 @@ __global__ void __launch_bounds__(256)
     }
 }
 
+__device__ __forceinline__ float dot_bf16x8(const oi_u32x4& a, const oi_u32x4& b, float acc) {
+    const uint32_t aw[4] = {a.x, a.y, a.z, a.w}, bw[4] = {b.x, b.y, b.z, b.w};
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        acc = fmaf(oi_bf16lo_to_f32(aw[k]), oi_bf16lo_to_f32(bw[k]), acc);
+        acc = fmaf(oi_bf16hi_to_f32(aw[k]), oi_bf16hi_to_f32(bw[k]), acc);
+    }
+    return acc;
+}
+
 // xref[j] = c * <hidden[j, :], W[label_j, :]>: the scaled logit of token j's own label, the exponent
 // that the token's kept exponentials are relative to.  It needs to be close to the token's largest
 // scaled logit, not equal to it (the same number is taken out again wherever the exponentials are
@@ -1528,13 +1538,7 @@ __global__ void __launch_bounds__(256)
     const oi_u32x4* b = reinterpret_cast<const oi_u32x4*>(W + y * hdim);
     float acc = 0.f;
     for (int64_t p = lane; p < hdim / 8; p += OI_WAVE) {  // hdim is a multiple of 64
-        const oi_u32x4 av = a[p], bv = b[p];
-        const uint32_t aw[4] = {av.x, av.y, av.z, av.w}, bw[4] = {bv.x, bv.y, bv.z, bv.w};
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            acc = fmaf(oi_bf16lo_to_f32(aw[k]), oi_bf16lo_to_f32(bw[k]), acc);
-            acc = fmaf(oi_bf16hi_to_f32(aw[k]), oi_bf16hi_to_f32(bw[k]), acc);
-        }
+        acc = dot_bf16x8(a[p], b[p], acc);
     }
     acc = oi_wave_sum(acc);
     if (lane == 0) xref[j] = acc * c;
@@ -1551,27 +1555,33 @@ struct SlabMeta {
 };
 
 // Workgroup j copies row order[meta->offset + j] into the slab's own buffers: the hidden-state row
-// (hdim bf16, 16-byte pieces), its label, its row number and, when given, its logsumexp, upstream
-// gradient and logprob.
+// (hdim bf16, 16-byte pieces), its label and its row number, and leaves the token's reference exponent
+// (see label_ref_kernel) on the way.
 __global__ void __launch_bounds__(256)
-    gather_slab_kernel(const uint16_t* __restrict__ hidden, const int64_t* __restrict__ labels,
-                       const float* __restrict__ lse, const float* __restrict__ grad,
-                       const float* __restrict__ logprob, const int32_t* __restrict__ order,
-                       const SlabMeta* __restrict__ meta, int64_t hdim, uint16_t* __restrict__ hidden_s,
-                       int64_t* __restrict__ labels_s, int32_t* __restrict__ rows_s, float* __restrict__ lse_s,
-                       float* __restrict__ grad_s, float* __restrict__ logprob_s) {
+    gather_slab_kernel(const uint16_t* __restrict__ hidden, const uint16_t* __restrict__ W,
+                       const int64_t* __restrict__ labels, const int32_t* __restrict__ order,
+                       const SlabMeta* __restrict__ meta, int64_t hdim, int64_t vocab, float c,
+                       uint16_t* __restrict__ hidden_s, int64_t* __restrict__ labels_s, int32_t* __restrict__ rows_s,
+                       float* __restrict__ xref_s) {
     const int64_t j = blockIdx.x;
     if (j >= meta->count) return;
-    const int64_t src = order[meta->offset + j];
+    const int64_t src = order[meta->offset + j], label = labels[src];
+    const int64_t y = label < 0 ? 0 : (label >= vocab ? vocab - 1 : label);
     const oi_u32x4* from = reinterpret_cast<const oi_u32x4*>(hidden + src * hdim);
+    const oi_u32x4* wy = reinterpret_cast<const oi_u32x4*>(W + y * hdim);
     oi_u32x4* to = reinterpret_cast<oi_u32x4*>(hidden_s + j * hdim);
-    for (int64_t c = threadIdx.x; c < hdim / 8; c += blockDim.x) to[c] = from[c];
+    float acc = 0.f;
+    for (int64_t p = threadIdx.x; p < hdim / 8; p += blockDim.x) {
+        const oi_u32x4 a = from[p], b = wy[p];
+        to[p] = a;
+        acc = dot_bf16x8(a, b, acc);
+    }
+    __shared__ float scratch[16];
+    acc = oi_block_sum(acc, scratch);
     if (threadIdx.x == 0) {
-        labels_s[j] = labels[src];
+        labels_s[j] = label;
         rows_s[j] = (int32_t)src;
-        if (lse_s) lse_s[j] = lse[src];
-        if (grad_s) grad_s[j] = grad[src];
-        if (logprob_s) logprob_s[j] = logprob[src];
+        xref_s[j] = acc * c;
     }
 }
 
@@ -2169,7 +2179,7 @@ SlabPlan plan_slabs(int64_t n, int64_t stats_rows, int64_t stats_cols, int64_t h
     p.off_scale_a = cv.take((size_t)p.cap * sizeof(float));
     p.off_scale_b = cv.take((size_t)p.cap * sizeof(float));
     p.off_scaled_hidden = cv.take(want_dw ? (size_t)p.cap * hdim * 2 : 0);
-    p.off_queues = cv.take((size_t)SLAB_QUEUE_WORDS * sizeof(uint32_t));
+    p.off_queues = cv.take((size_t)p.n_passes * SLAB_QUEUE_WORDS * sizeof(uint32_t));
     p.off_dw32 = cv.take(want_dw && p.n_passes > 1 ? (size_t)vocab * hdim * sizeof(float) : 0);
     p.off_stats = cv.take(oi_grpo_fused_workspace_bytes(stats_rows, stats_cols));
     p.off_lse = cv.take((size_t)n * sizeof(float));
@@ -2213,15 +2223,23 @@ __global__ void plan_slabs_kernel(const int32_t* __restrict__ count, int cap, in
     meta[i].reserved = 0;
 }
 
-// The per-token outputs start at zero: rows that take no part stay there, and the passes that look
+// What a step starts from, in one launch (a small launch is 5 us of the stream, and the step of a short batch has 19 of
+// them beside its three products; it had 25): the queue words of every pass and the marks of the rows (n_pad bytes) are
+// cleared, and the per-token outputs are zero: rows that take no part stay there, and the passes that look
 // at every row before its own slab has run (the upstream gradient of a slab is computed for all rows)
 // read zeros rather than whatever the caller's buffers held.
-__global__ void zero_f32_kernel(int64_t n, float* __restrict__ a, float* __restrict__ b, float* __restrict__ c) {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    a[i] = 0.f;
-    if (b) b[i] = 0.f;
-    if (c) c[i] = 0.f;
+__global__ void __launch_bounds__(256)
+    slab_setup_kernel(int64_t n, int64_t n_pad, int64_t queue_words, float* __restrict__ logprob,
+                      float* __restrict__ entropy, float* __restrict__ lse, uint32_t* __restrict__ unsafe,
+                      uint32_t* __restrict__ queues) {
+    const int64_t first = (int64_t)blockIdx.x * blockDim.x + threadIdx.x, stride = (int64_t)gridDim.x * blockDim.x;
+    for (int64_t i = first; i < n; i += stride) {
+        logprob[i] = 0.f;
+        if (entropy) entropy[i] = 0.f;
+        lse[i] = 0.f;
+    }
+    for (int64_t i = first; i < n_pad / 4; i += stride) unsafe[i] = 0u;
+    for (int64_t i = first; i < queue_words; i += stride) queues[i] = 0u;
 }
 
 // What a slab-wise step is made of besides the passes themselves
@@ -2236,9 +2254,9 @@ struct SlabStep {
 };
 
 // Runs the slab passes of `st` over the row index order[0 .. *count) that `plan_rows` leaves in the
-// workspace together with the passes' SlabMeta.  `upstream(final)` must enqueue kernels that leave
+// workspace together with the passes' SlabMeta.  `upstream()` must enqueue kernels that leave
 // every caller row's d loss / d logprob in the workspace's grad vector, given the logprobs computed
-// so far (the rows of the slabs up to the current one; with `final` set, all rows).
+// so far (the rows of the slabs up to the current one; in the last pass, all rows).
 template <class PlanRows, class Upstream>
 int run_slab_passes(const SlabPlan& p, char* ws, const SlabStep& st, hipStream_t s, PlanRows&& plan_rows,
                     Upstream&& upstream) {
@@ -2263,41 +2281,38 @@ int run_slab_passes(const SlabPlan& p, char* ws, const SlabStep& st, hipStream_t
     float* parts = p.parts_bytes ? reinterpret_cast<float*>(ws + p.off_parts) : nullptr;
     const uint16_t* hid = static_cast<const uint16_t*>(st.hidden);
 
-    hipLaunchKernelGGL(zero_words_kernel, dim3((unsigned)((p.n_pad / 4 + 255) / 256)), dim3(256), 0, s,
-                       reinterpret_cast<uint32_t*>(unsafe), (int)(p.n_pad / 4));
+    hipLaunchKernelGGL(slab_setup_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, n, p.n_pad,
+                       p.n_passes * SLAB_QUEUE_WORDS, st.logprob, st.entropy, lse, reinterpret_cast<uint32_t*>(unsafe),
+                       queues);
     plan_rows(order, count, meta);
-    hipLaunchKernelGGL(zero_f32_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, n, st.logprob, st.entropy, lse);
     hipLaunchKernelGGL(zero_unselected_rows_kernel, dim3((unsigned)n), dim3(256), 0, s, st.mask,
                        static_cast<const float*>(nullptr), hdim, static_cast<uint16_t*>(st.d_hidden));
     for (int64_t i = 0; i < p.n_passes; ++i) {
         const int32_t* cnt = &meta[i].count;
-        hipLaunchKernelGGL(zero_words_kernel, dim3(1), dim3(64), 0, s, queues, SLAB_QUEUE_WORDS);
-        hipLaunchKernelGGL(gather_slab_kernel, dim3((unsigned)p.cap), dim3(256), 0, s, hid, st.labels,
-                           static_cast<const float*>(nullptr), static_cast<const float*>(nullptr),
-                           static_cast<const float*>(nullptr), order, meta + i, hdim, hidden_s, labels_s, rows_s,
-                           static_cast<float*>(nullptr), static_cast<float*>(nullptr), static_cast<float*>(nullptr));
+        uint32_t* pass_queues = queues + i * SLAB_QUEUE_WORDS;
+        hipLaunchKernelGGL(gather_slab_kernel, dim3((unsigned)p.cap), dim3(256), 0, s, hid,
+                           static_cast<const uint16_t*>(st.weight), st.labels, order, meta + i, hdim, vocab,
+                           st.inv_temperature * OI_LOG2E, hidden_s, labels_s, rows_s, xref_s);
         const RowInputs in = {hidden_s, labels_s, nullptr, nullptr, rows_s, cnt, nullptr};
-        launch_label_ref(in, st.weight, p.cap, hdim, vocab, st.inv_temperature, xref_s, s);
         const KeepPlan keep = {keep_buf, p.v_pad, p.v_pad / BM, xref_s, unsafe, nullptr};
-        // the forward's own queue words are the first FWD_QUEUE_WORDS of `queues`
+        // the forward's own queue words are the first FWD_QUEUE_WORDS of the pass
         FwdPlan fp = p.fwd;
-        fp.off_queue = (size_t)(reinterpret_cast<char*>(queues) - ws_fwd);
+        fp.off_queue = (size_t)(reinterpret_cast<char*>(pass_queues) - ws_fwd);
         enqueue_fwd(fp, ws_fwd, in, nullptr, st.weight, p.cap, hdim, vocab, st.inv_temperature, st.logprob, st.entropy,
                     lse, keep, s);
-        const int rc = upstream(false);
+        const int rc = upstream();
         if (rc != OI_OK) return rc;
         hipLaunchKernelGGL(slab_prepare_kernel, dim3((unsigned)p.cap), dim3(256), 0, s, lse, grad, st.logprob, unsafe,
                            rows_s, labels_s, xref_s, meta + i, st.inv_temperature, vocab, hdim, keep_buf, p.v_pad,
                            hidden_s, scale_a, scale_b, scaled_hidden);
         enqueue_products_from_exponentials(keep_buf, p.v_pad, p.cap, cnt, rows_s, scale_a, scale_b, scaled_hidden,
                                            st.weight, hdim, vocab, st.d_hidden, st.d_weight, &meta[i].dw_mode, dw32,
-                                           queues + FWD_QUEUE_WORDS, parts, s);
+                                           pass_queues + FWD_QUEUE_WORDS, parts, s);
     }
     // the flagged rows, if any: one recomputing backward over them (its workspace takes the place of
-    // the exponentials), added to what the slabs left in d_weight
+    // the exponentials), added to what the slabs left in d_weight; the upstream gradients are those of the last
+    // pass, which saw every logprob
     {
-        const int rc = upstream(true);
-        if (rc != OI_OK) return rc;
         char* ws_rep = ws + p.off_repair;
         uint32_t* rq = reinterpret_cast<uint32_t*>(ws_rep + p.repair.off_queues);
         const int n_words = (int)(3 * p.repair.n_chunks * QUEUE_WORDS);
@@ -2573,14 +2588,7 @@ int grpo_step_in_slabs(const void* hidden, const void* weight, const int64_t* la
     char* ws = static_cast<char*>(workspace);
     float* grad = reinterpret_cast<float*>(ws + p.off_grad);
     float* row_denoms = reinterpret_cast<float*>(ws + p.off_denoms);
-    // the denominators come from the mask alone: a first pass of the statistics over logprobs that are
-    // not there yet (zeros) leaves them in row_denoms (its other results are overwritten at the end)
-    hipLaunchKernelGGL(zero_f32_kernel, dim3((unsigned)((n_tokens + 255) / 256)), dim3(256), 0, s, n_tokens, logprob, entropy,
-                       static_cast<float*>(nullptr));
-    int rc = oi_grpo_fused_fwd(logprob, old_logprobs, ref_logprobs, advantages, mask, rho_weights, entropy, nullptr, nullptr,
-                               nullptr, nullptr, rows, cols, loss_fn, ratio_lo, ratio_hi, kl_estimator, beta, axis_mode,
-                               denominator, scale, out_stats, row_denoms, ws + p.off_stats,
-                               oi_grpo_fused_workspace_bytes(rows, cols), stream);
+    int rc = oi_check_grpo(rows, cols, axis_mode, loss_fn, kl_estimator);
     if (rc != OI_OK) return rc;
     const SlabStep st = {hidden, weight, labels, mask, n_tokens, hidden_dim, vocab, inv_temperature, logprob, entropy,
                          d_hidden, d_weight};
@@ -2593,8 +2601,10 @@ int grpo_step_in_slabs(const void* hidden, const void* weight, const int64_t* la
             const int64_t h_tiles = (hidden_dim + BN - 1) / BN;
             hipLaunchKernelGGL(plan_slabs_kernel, dim3((unsigned)((p.n_passes + 63) / 64)), dim3(64), 0, s, count,
                                (int)p.cap, (int)p.n_passes, (int)h_tiles, (int)resident_grid(p.cap / BM, h_tiles), meta);
+            // the denominators come from the mask alone
+            (void)oi_launch_grpo_denoms(mask, count, rows, cols, axis_mode, denominator, row_denoms, s);
         },
-        [&](bool) {
+        [&]() {
             // every token's d loss / d logprob from its own logprob; tokens of later slabs hold numbers
             // that nobody reads before their own slab has overwritten them
             return oi_grpo_fused_bwd(logprob, old_logprobs, ref_logprobs, advantages, mask, rho_weights, rows, cols,
@@ -2891,7 +2901,7 @@ extern "C" int oi_lmhead_dpo_fwd_bwd(const void* hidden, const void* weight, con
                          nullptr, d_hidden, d_weight};
     // per-sequence sums of the logprobs computed so far, the loss derivative of every pair, and from it
     // every token's d loss / d logprob (right for the pairs whose tokens are all there)
-    auto upstream = [&](bool) {
+    auto upstream = [&]() {
         int r = oi_seq_logp_fwd(per_token_logps, labels, cu_seq_lens, n_seqs, total, average_log_prob, seq_logps, counts,
                                 stream);
         if (r != OI_OK) return r;
