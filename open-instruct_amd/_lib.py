@@ -88,7 +88,16 @@ SIGNATURES: dict[str, tuple] = {
     "oi_gemm_bf16_layouts": (_I, [_P, _I64, _I, _P, _I64, _I, _I64, _I64, _I64, _P, _P, _I64, _I, _P]),
 }
 
+PYLISTS_PATH = os.path.join(_HERE, "csrc", "liboi_pylists.so")
+PYLISTS_SIGNATURES: dict[str, list] = {
+    "oi_py_offsets": [ctypes.py_object, _I64, _P],
+    "oi_py_flatten_ints": [ctypes.py_object, _I64, _P, _I64, _P, _P],
+    "oi_py_flatten_flags": [ctypes.py_object, _I64, _P, _P],
+    "oi_py_flatten_floats": [ctypes.py_object, _I64, _P, _P],
+}
+
 _lib: ctypes.CDLL | None = None
+_pylists: ctypes.PyDLL | None = None
 
 
 class KernelError(RuntimeError):
@@ -111,6 +120,21 @@ def load() -> ctypes.CDLL:
             fn.argtypes = argtypes
         _lib = lib
     return _lib
+
+
+def pylists() -> ctypes.PyDLL:
+    """The host library that reads Python lists, loaded once; its functions run under the interpreter lock."""
+    global _pylists
+    if _pylists is None:
+        if not os.path.exists(PYLISTS_PATH):
+            raise RuntimeError(f"{PYLISTS_PATH} is missing: build it with `python -m open_instruct_amd.build`")
+        lib = ctypes.PyDLL(PYLISTS_PATH)
+        for name, argtypes in PYLISTS_SIGNATURES.items():
+            fn = getattr(lib, name)
+            fn.restype = _I
+            fn.argtypes = argtypes
+        _pylists = lib
+    return _pylists
 
 
 def ptr(t: torch.Tensor | None) -> int | None:

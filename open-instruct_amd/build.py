@@ -1,6 +1,8 @@
-"""Build ``csrc/liboi_kernels.so`` for gfx950 with hipcc (``python -m open_instruct_amd.build``).
+"""Build ``csrc/liboi_kernels.so`` for gfx950 with hipcc (``python -m open_instruct_amd.build``), and beside it
+``csrc/liboi_pylists.so``, host code that reads Python lists and is kept apart because it needs an interpreter
+around it (the kernel library does not).
 
-The shared object is built in-tree so that it travels with the source tree; nothing is compiled
+The shared objects are built in-tree so that they travel with the source tree; nothing is compiled
 at import time.
 """
 
@@ -9,12 +11,15 @@ from __future__ import annotations
 import os
 import subprocess
 import sys
+import sysconfig
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 INCLUDE = os.path.join(os.path.dirname(HERE), "include")
 SOURCES = ["oi_rowwise.hip", "oi_loss.hip", "oi_pack.hip", "oi_lmhead.hip"]
 OUTPUT = os.path.join(CSRC, "liboi_kernels.so")
+PYLISTS_SOURCE = os.path.join(CSRC, "oi_pylists.cpp")
+PYLISTS_OUTPUT = os.path.join(CSRC, "liboi_pylists.so")
 
 HIPCC_FLAGS = [
     "--offload-arch=gfx950",
@@ -57,6 +62,11 @@ def build(verbose: bool = False) -> str:
         raise RuntimeError(f"link failed:\n{res.stderr}")
     for obj in objs:
         os.remove(obj)
+    include = sysconfig.get_paths()["include"]
+    cmd = [_hipcc(), "-x", "c++", "-O3", "-std=c++17", "-fPIC", "-shared", f"-I{include}", PYLISTS_SOURCE, "-o", PYLISTS_OUTPUT]
+    res = subprocess.run(cmd, capture_output=True, text=True)
+    if res.returncode != 0:
+        raise RuntimeError(f"compiling {PYLISTS_SOURCE} failed:\n{res.stderr}")
     return OUTPUT
 
 

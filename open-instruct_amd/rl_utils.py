@@ -121,12 +121,64 @@ class PackedSequences:
     rewards: list[torch.Tensor] | None = None
 
 
-def _csr(seqs: list, dtype) -> tuple[np.ndarray, np.ndarray]:
-    lens = np.fromiter((len(x) for x in seqs), dtype=np.int64, count=len(seqs))
-    offsets = np.zeros(len(seqs) + 1, dtype=np.int64)
-    np.cumsum(lens, out=offsets[1:])
-    flat = np.fromiter(itertools.chain.from_iterable(seqs), dtype=dtype, count=int(offsets[-1]))
-    return flat, offsets
+_INT64 = range(-(2**63), 2**63)
+
+
+def _offsets(seqs) -> np.ndarray:
+    """Where each sequence starts in the flat array, and the end."""
+    n = len(seqs)
+    offsets = np.empty(n + 1, dtype=np.int64)
+    if _lib.pylists().oi_py_offsets(seqs, n, offsets.ctypes.data):
+        offsets[0] = 0
+        np.cumsum(np.fromiter((len(x) for x in seqs), dtype=np.int64, count=n), out=offsets[1:])
+    return offsets
+
+
+def _walk(seqs, offsets: np.ndarray, dtype) -> np.ndarray:
+    """Sequences of any kind, flattened element by element."""
+    return np.fromiter(itertools.chain.from_iterable(seqs), dtype=dtype, count=int(offsets[-1]))
+
+
+def _fill_ints(seqs, offsets: np.ndarray, out: np.ndarray, skip) -> np.ndarray:
+    """Flattens integer sequences into ``out``; returns how many elements of each differ from ``skip``."""
+    n = len(offsets) - 1
+    others = np.empty(n, dtype=np.int64)
+    if type(skip) is int and skip in _INT64:
+        if not _lib.pylists().oi_py_flatten_ints(seqs, n, offsets.ctypes.data, skip, out.ctypes.data, others.ctypes.data):
+            return others
+    out[:] = _walk(seqs, offsets, np.int64)
+    before = np.zeros(len(out) + 1, dtype=np.int64)
+    np.cumsum(out != skip, out=before[1:])
+    return before[offsets[1:]] - before[offsets[:-1]]
+
+
+def _fill_flags(seqs, offsets: np.ndarray, out: np.ndarray) -> None:
+    if _lib.pylists().oi_py_flatten_flags(seqs, len(offsets) - 1, offsets.ctypes.data, out.ctypes.data):
+        out[:] = _walk(seqs, offsets, np.int64) != 0
+
+
+def _fill_floats(seqs, offsets: np.ndarray, out: np.ndarray) -> None:
+    if _lib.pylists().oi_py_flatten_floats(seqs, len(offsets) - 1, offsets.ctypes.data, out.ctypes.data):
+        out[:] = _walk(seqs, offsets, np.float32)
+
+
+class _Staging:
+    """Arrays that go to the device together: sections of one pinned buffer, 16-byte aligned, and one copy."""
+
+    def __init__(self, sizes: list[tuple[int, type]]):
+        self.at, end = [], 0
+        for count, dtype in sizes:
+            self.at.append(end)
+            end += (count * np.dtype(dtype).itemsize + 15) // 16 * 16
+        self.host = torch.empty(max(end, 16), dtype=torch.uint8, pin_memory=True)
+        raw = self.host.numpy()
+        self.arrays = [
+            raw[at : at + count * np.dtype(dtype).itemsize].view(dtype) for at, (count, dtype) in zip(self.at, sizes)
+        ]
+
+    def upload(self, dev) -> torch.Tensor:
+        # the allocator of pinned memory hands the buffer out again only when the copy is through
+        return self.host.to(dev, non_blocking=True)
 
 
 def pack_sequences(
@@ -154,25 +206,40 @@ def pack_sequences(
     n = len(queries)
     if not (len(responses) == len(masks) == len(vllm_logprobs) == n):
         raise ValueError("queries, responses, masks and vllm_logprobs must have one length")
-    assert not any(pad_token_id in query for query in queries)
-    for i in range(n):
+    q_off = _offsets(queries)
+    r_off = _offsets(responses)
+    dev = torch.device(device)
+    with_adv = advantages is not None
+    # queries, responses, tool mask, logprobs, their offsets, destinations, row bases, advantages, lengths
+    staging = None
+    if dev.type == "cuda" and n:
+        n_q, n_r = int(q_off[-1]), int(r_off[-1])
+        staging = _Staging(
+            [(n_q, np.int64), (n_r, np.int64), (n_r if mask_tool_use else 0, np.uint8), (n_r, np.float32), (n + 1, np.int64),
+             (n + 1, np.int64), (n, np.int64), (n, np.int32), (n if with_adv else 0, np.float32), (2 * n, np.int64)]
+        )  # fmt: skip
+        q_flat, r_flat, tool, lp_flat, q_off_s, r_off_s, dst_s, mask_base, adv_s, lens = staging.arrays
+    else:
+        q_flat = np.empty(int(q_off[-1]), dtype=np.int64)
+    others = _fill_ints(queries, q_off, q_flat, pad_token_id)
+    q_len = q_off[1:] - q_off[:-1]
+    assert (others == q_len).all()  # no padding token in a query
+    lp_off, m_off = _offsets(vllm_logprobs), _offsets(masks)
+    for i in np.flatnonzero((np.diff(lp_off) != np.diff(r_off)) | (np.diff(m_off) != np.diff(r_off))):
         assert len(vllm_logprobs[i]) == len(responses[i]), (
             f"Response {i}: logprobs length ({len(vllm_logprobs[i])}) != response length ({len(responses[i])})"
         )
-        if len(masks[i]) != len(responses[i]):
-            raise ValueError(f"Response {i}: mask length ({len(masks[i])}) != response length ({len(responses[i])})")
-    dev = torch.device(device)
+        raise ValueError(f"Response {i}: mask length ({len(masks[i])}) != response length ({len(responses[i])})")
     if dev.type != "cuda":
         raise RuntimeError("pack_sequences writes its outputs on an AMD GPU; there is no CPU implementation")
-    q_flat, q_off = _csr(queries, np.int64)
-    r_flat, r_off = _csr(responses, np.int64)
-    m_flat = _csr(masks, np.int64)[0] if mask_tool_use else None  # only read when tool tokens are masked out
-    lp_flat, _ = _csr(vllm_logprobs, np.float32)
-    kept = r_flat != pad_token_id
-    kept_before = np.zeros(len(r_flat) + 1, dtype=np.int64)
-    np.cumsum(kept, out=kept_before[1:])
-    r_len = kept_before[r_off[1:]] - kept_before[r_off[:-1]]
-    seq_len = (q_off[1:] - q_off[:-1]) + r_len
+    if n:
+        r_len = _fill_ints(responses, r_off, r_flat, pad_token_id)
+        if mask_tool_use:  # only read when tool tokens are masked out
+            _fill_flags(masks, r_off, tool)
+        _fill_floats(vllm_logprobs, r_off, lp_flat)
+    else:
+        r_len = np.zeros(0, dtype=np.int64)
+    seq_len = q_len + r_len
     if n and int(seq_len.min()) < 1:
         raise ValueError("every sequence needs at least one token")
     total_tokens = int(seq_len.sum())
@@ -182,39 +249,40 @@ def pack_sequences(
         effective = pack_length
     # greedy row assignment: O(n) scalar work
     row_first = [0] if n else []  # index of the first sequence of each row
-    mask_base = np.zeros(n, dtype=np.int32)
+    bases = []
     cur = 0
     for i, length in enumerate(seq_len.tolist()):
         if length + cur > effective and cur > 0:
             row_first.append(i)
             cur = 0
-        mask_base[i] = row_first[-1]
+        bases.append(row_first[-1])
         cur += length
     dst = np.zeros(n + 1, dtype=np.int64)
     np.cumsum(seq_len, out=dst[1:])
 
-    def up(a):
-        return torch.from_numpy(np.ascontiguousarray(a)).to(dev)
-
     out_i64 = torch.empty(5, max(total_tokens, 1), dtype=torch.int64, device=dev)
     out_f32 = torch.empty(2, max(total_tokens, 1), dtype=torch.float32, device=dev)
-    adv_dev = None
-    if advantages is not None:
+    if with_adv:
         adv_np = np.asarray(advantages, dtype=np.float32).reshape(-1)
         if adv_np.shape[0] != n:
             raise ValueError(f"advantages has {adv_np.shape[0]} entries for {n} sequences")
-        adv_dev = up(adv_np)
-    lens_dev = up(np.stack([r_len, seq_len])) if n else torch.zeros(2, 0, dtype=torch.int64, device=dev)
+    lens_dev = torch.zeros(2, 0, dtype=torch.int64, device=dev)
     if n:
-        tool = up(m_flat != 0).view(torch.uint8) if mask_tool_use else None
-        ins = [up(q_flat), up(q_off), up(r_flat), up(r_off), tool, up(lp_flat), up(dst[:-1]), up(mask_base)]
+        q_off_s[:], r_off_s[:], dst_s[:], mask_base[:] = q_off, r_off, dst[:-1], bases
+        lens[:n], lens[n:] = r_len, seq_len
+        if with_adv:
+            adv_s[:] = adv_np
+        ins = staging.upload(dev)
+        q_p, r_p, tool_p, lp_p, qo_p, ro_p, dst_p, base_p, adv_p, _ = (ins.data_ptr() + at for at in staging.at)
         _lib.call(
-            "oi_pack_sequences", ins[0].data_ptr(), ins[1].data_ptr(), ins[2].data_ptr(), ins[3].data_ptr(),
-            _lib.ptr(ins[4]), ins[5].data_ptr(), _lib.ptr(adv_dev), ins[6].data_ptr(), ins[7].data_ptr(), n,
-            int(pad_token_id), int(bool(mask_tool_use)), out_i64[0].data_ptr(), out_i64[1].data_ptr(),
+            "oi_pack_sequences", q_p if n_q else None, qo_p, r_p if n_r else None, ro_p, tool_p if mask_tool_use else None,
+            lp_p, adv_p if with_adv else None,
+            dst_p, base_p, n, int(pad_token_id), int(bool(mask_tool_use)), out_i64[0].data_ptr(), out_i64[1].data_ptr(),
             out_i64[2].data_ptr(), out_i64[3].data_ptr(), out_i64[4].data_ptr(), out_f32[0].data_ptr(),
-            out_f32[1].data_ptr() if adv_dev is not None else None, torch.cuda.current_stream(dev).cuda_stream,
+            out_f32[1].data_ptr() if with_adv else None, torch.cuda.current_stream(dev).cuda_stream,
         )  # fmt: skip
+        # a tensor of their own: the caller keeps the lengths, not the inputs
+        lens_dev = ins[staging.at[-1] : staging.at[-1] + 16 * n].view(torch.int64).view(2, n).clone()
     bounds = [int(dst[i]) for i in row_first] + [total_tokens]
     seq_bounds = row_first + [n]
 
@@ -234,5 +302,5 @@ def pack_sequences(
         packed_seq_lens=seq_rows(lens_dev[1]),
         dones=rows(out_i64[4]),
         vllm_logprobs=rows(out_f32[0]),
-        advantages=rows(out_f32[1]) if adv_dev is not None else None,
+        advantages=rows(out_f32[1]) if with_adv else None,
     )

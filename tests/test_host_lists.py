@@ -1,0 +1,58 @@
+"""The native readers of ragged Python lists against numpy's element by element walk, over what they take
+themselves (exact lists of exact numbers), what they leave to that walk, and what nothing takes."""
+
+import numpy as np
+import pytest
+
+from open_instruct_amd import rl_utils
+
+BIG = 2**63 - 1
+INTS = [
+    [[1, 2, 3], [], [0, -7, BIG, -BIG - 1]],
+    [[], [], []],
+    [[True, False], [5]],
+    [np.arange(4), [1, 2]],  # left to the walk
+    [(1, 0), [2]],
+    ([1, 0], [0, 0, 0]),
+    [list(range(300)), [0] * 17],
+]
+
+
+@pytest.mark.parametrize("seqs", INTS)
+@pytest.mark.parametrize("skip", [0, 2, BIG, 2**64, 0.0, None])
+def test_integers(seqs, skip):
+    offsets = rl_utils._offsets(seqs)
+    assert offsets.tolist() == [0] + np.cumsum([len(s) for s in seqs]).tolist()
+    out = np.full(offsets[-1], 77, dtype=np.int64)
+    others = rl_utils._fill_ints(seqs, offsets, out, skip)
+    assert out.tolist() == [int(x) for s in seqs for x in s]
+    assert others.tolist() == [sum(int(x) != skip for x in s) for s in seqs]
+    flags = np.full(offsets[-1], 77, dtype=np.uint8)
+    rl_utils._fill_flags(seqs, offsets, flags)
+    assert flags.tolist() == [int(x != 0) for s in seqs for x in s]
+
+
+@pytest.mark.parametrize(
+    "seqs", [[[-0.5, 1e-45, 3.4e38], [], [float("nan"), float("inf"), 0.1]], [[1, 2.5]], [np.array([0.25], np.float32)], [[]]]
+)
+def test_floats(seqs):
+    offsets = rl_utils._offsets(seqs)
+    out = np.full(offsets[-1], 7, dtype=np.float32)
+    rl_utils._fill_floats(seqs, offsets, out)
+    np.testing.assert_array_equal(out, np.array([x for s in seqs for x in s], dtype=np.float32))
+
+
+@pytest.mark.parametrize("bad,error", [([["a"]], ValueError), ([[2**63]], OverflowError), ([[None]], TypeError), ([3], TypeError)])
+def test_refused(bad, error):
+    with pytest.raises(error):
+        offsets = rl_utils._offsets(bad)
+        rl_utils._fill_ints(bad, offsets, np.empty(offsets[-1], dtype=np.int64), 0)
+
+
+def test_a_list_that_changed_since_its_length_was_taken():
+    seqs = [[1, 2], [3]]
+    offsets = rl_utils._offsets(seqs)
+    seqs[1].append(4)
+    lib = rl_utils._lib.pylists()
+    out, others = np.empty(3, dtype=np.int64), np.empty(2, dtype=np.int64)
+    assert lib.oi_py_flatten_ints(seqs, 2, offsets.ctypes.data, 0, out.ctypes.data, others.ctypes.data) == -1
