@@ -212,6 +212,9 @@ def pack_sequences(
     with_adv = advantages is not None
     # queries, responses, tool mask, logprobs, their offsets, destinations, row bases, advantages, lengths
     staging = None
+    if dev.type == "cuda" and n and torch.cuda.is_current_stream_capturing():
+        # a recorded copy would read the pinned buffer at every replay, when it has long been handed out again
+        raise RuntimeError("pack_sequences reads Python lists and cannot be captured into a graph")
     if dev.type == "cuda" and n:
         n_q, n_r = int(q_off[-1]), int(r_off[-1])
         staging = _Staging(

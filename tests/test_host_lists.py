@@ -3,6 +3,7 @@ themselves (exact lists of exact numbers), what they leave to that walk, and wha
 
 import numpy as np
 import pytest
+import torch
 
 from open_instruct_amd import rl_utils
 
@@ -56,3 +57,10 @@ def test_a_list_that_changed_since_its_length_was_taken():
     lib = rl_utils._lib.pylists()
     out, others = np.empty(3, dtype=np.int64), np.empty(2, dtype=np.int64)
     assert lib.oi_py_flatten_ints(seqs, 2, offsets.ctypes.data, 0, out.ctypes.data, others.ctypes.data) == -1
+
+
+def test_packing_is_refused_while_a_stream_captures(monkeypatch):
+    # its inputs are read from host lists: a graph would replay the copy of a buffer that is no longer theirs
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: True)
+    with pytest.raises(RuntimeError, match="captured"):
+        rl_utils.pack_sequences([[1, 2]], [[3]], [[1]], 8, 0, [[-0.5]], device="cuda")
