@@ -134,19 +134,54 @@ __device__ __forceinline__ double block_sum_f64(double v, double* scratch) {
 
 // One workgroup: per-row totals in fp64 in chunk order, then the loss and the statistics.
 // Statistic q goes to out_stats[q * out_stride] when bit q of write_mask is set.
-// Thread (slice, q) adds up sum q of the rows slice, slice + 16, ...: the sums run side by side and meet at one
-// barrier (fifteen sums one after the other, a barrier pair each, and sixteen divisions in one thread: 12 us for 2 rows, 5.4 us now, of which a launch is 4.5).
-constexpr int FINAL_SLICES = 16;
+// Thread (slice, q) adds up sum q of the rows slice, slice + SLICES, ...: the sums run side by side and meet at one
+// barrier (fifteen sums one after the other, a barrier pair each, and sixteen divisions in one thread: 12 us for 2
+// rows, 5.4 us now, of which a launch is 4.5).  Many short rows are bound by the latency of their one read each: 64
+// slices with FINAL_ROWS reads in flight per thread.  Statistics of [4096, 128], mean per row, both launches: 87 us with 16
+// slices, 68 with 64, 54 with a lane per row for the divisions; 54 with the rows over 256 threads and the sums one
+// after the other, where [16, 1024] took 21 us (now 14) and [1024, 256] 34 (now 29 to 31).
+constexpr int FINAL_ROWS = 4;
+constexpr int64_t FINAL_FEW_ROWS = 64;
 static_assert(NSUM < 16 && OI_GRPO_NUM_STATS == 16, "a sum and a statistic per lane of a group of 16");
+template <int FINAL_SLICES>
 __global__ void __launch_bounds__(16 * FINAL_SLICES)
     grpo_stats_final_kernel(const float* __restrict__ partial, int64_t rows, int64_t nchunks, int axis_mode,
                             float denominator, float scale, float beta, int kl_est, float* __restrict__ out_stats,
                             int64_t out_stride, uint32_t write_mask, float* __restrict__ row_denoms) {
     __shared__ double part[FINAL_SLICES][16];
     const int q = threadIdx.x & 15, slice = threadIdx.x >> 4;
-    // lane 15 of a group has no sum of its own: it adds up the per-row means of axis_mode 1
-    double tot = 0.0;
-    for (int64_t r0 = 0; r0 < rows; r0 += FINAL_SLICES) {  // the same trip count for every thread: lanes exchange below
+    double tot = 0.0, means = 0.0;
+    auto row_mean = [&](int64_t r, double loss, double tokens) {
+        const double den = denominator > 0.f ? (double)denominator : tokens;
+        const double inv = den > 0.0 ? 1.0 / den : 0.0;
+        if (row_denoms) row_denoms[r] = (float)(inv / (double)rows);
+        means += loss * inv;
+    };
+    int64_t r0 = 0;  // the same trip counts for every thread: lanes exchange below
+    for (; r0 + FINAL_SLICES * FINAL_ROWS <= rows; r0 += FINAL_SLICES * FINAL_ROWS) {
+        double rt[FINAL_ROWS];
+#pragma unroll
+        for (int u = 0; u < FINAL_ROWS; ++u) rt[u] = 0.0;
+        if (q < NSUM)
+            for (int64_t ch = 0; ch < nchunks; ++ch) {
+#pragma unroll
+                for (int u = 0; u < FINAL_ROWS; ++u)
+                    rt[u] += (double)partial[((r0 + u * FINAL_SLICES + slice) * nchunks + ch) * NSUM + q];
+            }
+#pragma unroll
+        for (int u = 0; u < FINAL_ROWS; ++u) tot += rt[u];
+        if (axis_mode == 1) {  // lane u divides for row u
+            double loss = 0.0, tokens = 0.0;
+#pragma unroll
+            for (int u = 0; u < FINAL_ROWS; ++u) {
+                const double l = __shfl(rt[u], 0, 16), t = __shfl(rt[u], 9, 16);
+                loss = q == u ? l : loss;
+                tokens = q == u ? t : tokens;
+            }
+            if (q < FINAL_ROWS) row_mean(r0 + q * FINAL_SLICES + slice, loss, tokens);
+        }
+    }
+    for (; r0 < rows; r0 += FINAL_SLICES) {
         const int64_t r = r0 + slice;
         double rt = 0.0;
         if (r < rows && q < NSUM) {
@@ -154,16 +189,16 @@ __global__ void __launch_bounds__(16 * FINAL_SLICES)
 #pragma unroll 4
             for (int64_t ch = 0; ch < nchunks; ++ch) rt += (double)p[ch * NSUM];
         }
+        tot += rt;
         if (axis_mode == 1) {
             const double loss = __shfl(rt, 0, 16), tokens = __shfl(rt, 9, 16);
-            if (q == 15 && r < rows) {
-                const double den = denominator > 0.f ? (double)denominator : tokens;
-                const double inv = den > 0.0 ? 1.0 / den : 0.0;
-                rt = loss * inv;
-                if (row_denoms) row_denoms[r] = (float)(inv / (double)rows);
-            }
+            if (q == 0 && r < rows) row_mean(r, loss, tokens);
         }
-        tot += rt;
+    }
+    if (axis_mode == 1) {  // lane 15 of a group has no sum of its own: it takes the per-row means
+#pragma unroll
+        for (int off = 8; off > 0; off >>= 1) means += __shfl_xor(means, off, 16);
+        if (q == 15) tot = means;
     }
     part[slice][q] = tot;
     __syncthreads();
@@ -623,7 +658,8 @@ int launch_grpo_stats(const StatIn& in, int64_t rows, int64_t cols, const GrpoCf
     const int64_t nchunks = (cols + FUSED_CHUNK - 1) / FUSED_CHUNK;
     hipLaunchKernelGGL(grpo_stats_partial_kernel, dim3((unsigned)(rows * nchunks)), dim3(FUSED_THREADS), 0, s, in,
                        cols, nchunks, c, beta, partial);
-    hipLaunchKernelGGL(grpo_stats_final_kernel, dim3(1), dim3(16 * FINAL_SLICES), 0, s, partial, rows, nchunks, axis_mode,
+    auto final_kernel = rows > FINAL_FEW_ROWS ? grpo_stats_final_kernel<64> : grpo_stats_final_kernel<16>;
+    hipLaunchKernelGGL(final_kernel, dim3(1), dim3(rows > FINAL_FEW_ROWS ? 1024 : 256), 0, s, partial, rows, nchunks, axis_mode,
                        denominator, scale, beta, c.kl_est, out_stats, out_stride, write_mask, row_denoms);
     return oi_launch_status();
 }
