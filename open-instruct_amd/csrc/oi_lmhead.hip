@@ -46,10 +46,14 @@ typedef f32x16 AccTile[2][4];
 // as a whole then works on one slab of A (the larger operand: lm_head rows, dZ rows) at a time, which
 // stays in the memory-side cache while every n tile passes over it, instead of streaming all of A from
 // HBM once per n super-tile.  Measured: +4 to +7 % on every shape of the lm_head path (the kernel runs at
-// the chip's power limit, and HBM traffic costs power).  Every number is a tile, whatever the counts.
-__device__ __forceinline__ uint32_t item_of_pid(uint32_t pid) {
-    const uint32_t xcd = pid & 7, local = pid >> 3;
-    return ((local >> 5) * 8 + xcd) * 32 + (local & 31);
+// the chip's power limit, and HBM traffic costs power).  Every number is a tile, whatever the counts, and the
+// numbers past the last whole 256 are dealt out evenly: runs of 32 would leave whole XCDs to take tiles from
+// the others' queues, out of the runs that share slabs.  d_hidden of 7648 rows (480 tiles, 4096 x 128256): 7.03 ms in
+// runs of 32, 6.61 evenly; scoring pass of 1432 rows 1.258 -> 1.223 ms.  Ids without a number give one >= items.
+__device__ __forceinline__ uint32_t item_of_pid(uint32_t pid, uint32_t items) {
+    const uint32_t xcd = pid & 7, local = pid >> 3, first = (local >> 5) * 256, at = local & 31;
+    const uint32_t left = first < items ? items - first : 0, run = left >= 256 ? 32 : (left + 7) / 8;
+    return at < run ? first + xcd * run + at : 0xffffffffu;
 }
 __device__ __forceinline__ void tile_of_item(uint32_t item, uint32_t tiles_m, uint32_t tiles_n, int64_t* tm, int64_t* tn) {
     const uint32_t band = item / (8 * tiles_n), in_band = item - band * 8 * tiles_n;
@@ -133,7 +137,7 @@ struct ItemQueue {
         for (;;) {
             const uint32_t pid = take();
             if (pid == NONE) return NONE;
-            const uint32_t item = item_of_pid(pid);
+            const uint32_t item = item_of_pid(pid, items);
             if (item < items) return item;
             request();
             settle();
@@ -148,7 +152,7 @@ __device__ __forceinline__ void for_each_item(uint32_t* __restrict__ counters, u
     uint32_t pid = queue.take();
     while (pid != ItemQueue::NONE) {
         queue.request();
-        const uint32_t item = item_of_pid(pid);
+        const uint32_t item = item_of_pid(pid, items);
         if (item < items) body(item);
         queue.settle();
         pid = queue.take();
@@ -1351,7 +1355,7 @@ __global__ void __launch_bounds__(NTHREADS)
         return t;
     };
     if (!queue) {
-        const uint32_t item = item_of_pid(blockIdx.x);
+        const uint32_t item = item_of_pid(blockIdx.x, tiles);
         if (item >= tiles) return;
         const ProductTile t = tile_at(item);
         AccTile acc;
