@@ -12,6 +12,9 @@ causal-LM cross-entropy that the reference obtains from the model's own forward
 
 from __future__ import annotations
 
+import threading
+import weakref
+
 import torch
 
 from . import _lib
@@ -66,7 +69,7 @@ class _FusedLMHead(torch.autograd.Function):
             ws_bytes = lib.oi_lmhead_fwd_workspace_bytes(n, h, v, int(m is not None))
             ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
             if keep_logits and ctx.needs_input_grad[1] and not compact_backward:
-                logits = _kept_logits(n, v, dev)
+                logits = _kept_logits(n, h, v, dev, m is not None)
             if logits is not None:
                 _lib.call(
                     "oi_lmhead_logp_fwd_kept", hid.data_ptr(), w.data_ptr(), lab.data_ptr(), _lib.ptr(m), n, h, v,
@@ -127,16 +130,49 @@ class _FusedLMHead(torch.autograd.Function):
         return (d_hidden if need_h else None), d_weight, None, None, None, None, None, None, None
 
 
-def _kept_logits(n, v, dev):
+# Bytes of kept logits that may be alive on one device at a time, over all graphs: as many as the largest call that
+# keeps any (oi_lmhead_kept_bytes), so two forwards before one backward do not hold twice that.
+KEPT_BUDGET = 4 << 30
+# Device memory that has to be free for each byte of kept logits, once the backward's own needs are taken off.
+KEPT_SHARE = 8
+_kept_lock = threading.Lock()
+_kept_alive: list[weakref.ref] = []
+
+
+def _free_bytes(dev) -> int:
+    """Device memory that this process has not reserved so far, at the peak of its steps, and still may.  What the
+    allocator holds unused is left out: it is there because a step needed it."""
+    free, total = torch.cuda.mem_get_info(dev)
+    fraction = torch.cuda.get_per_process_memory_fraction(dev)
+    return free if fraction >= 1.0 else min(free, int(total * fraction) - torch.cuda.memory_reserved(dev))
+
+
+def _kept_logits(n, h, v, dev, selecting):
     """Memory for the forward's logits where they are kept for the backward, else None (the backward then
-    computes them again, with the same results): too many of them, or none of that size to be had."""
-    kept = _lib.load().oi_lmhead_kept_bytes(n, v)
-    if not kept:
+    computes them again, with the same results).  Kept only where nothing else has to give way for them:
+    not more than one call's largest share over all live graphs, and only out of plenty; not where saved tensors
+    are packed (checkpointing counts them and would compute them twice, offloading would copy them), and not into
+    the private pool of a graph, which would hold them as long as the graph lives."""
+    lib = _lib.load()
+    kept = lib.oi_lmhead_kept_bytes(n, v)
+    if not kept or torch._C._autograd._top_saved_tensors_default_hooks(True) is not None:
         return None
-    try:
-        return torch.empty(kept // 4, dtype=torch.float32, device=dev)
-    except torch.cuda.OutOfMemoryError:
+    if torch.cuda.is_current_stream_capturing():
         return None
+    backward = lib.oi_lmhead_bwd_workspace_bytes(n, h, v, 1, int(selecting)) + 2 * h * (n + v)
+    with _kept_lock:
+        alive = [(r, t) for r, t in ((r, r()) for r in _kept_alive) if t is not None]
+        _kept_alive[:] = [r for r, _ in alive]
+        if kept + sum(t.numel() * 4 for _, t in alive if t.device == dev) > KEPT_BUDGET:
+            return None
+        if _free_bytes(dev) < KEPT_SHARE * kept + backward:
+            return None
+        try:
+            logits = torch.empty(kept // 4, dtype=torch.float32, device=dev)
+        except torch.cuda.OutOfMemoryError:
+            return None
+        _kept_alive.append(weakref.ref(logits))
+        return logits
 
 
 def fused_lm_head_logprobs(
@@ -148,6 +184,7 @@ def fused_lm_head_logprobs(
     return_entropy: bool = False,
     compact_backward: bool = False,
     dhidden_in_forward: bool | str = "auto",
+    keep_logits: bool = True,
 ) -> tuple[torch.Tensor, torch.Tensor | None]:
     """``log_softmax(hidden @ weight.T / temperature)[labels]`` (+ entropy) per token, fp32.
 
@@ -163,9 +200,13 @@ def fused_lm_head_logprobs(
     term) out of the backward products; it changes no result.
 
     When ``weight`` takes a gradient the forward of a small batch keeps its logits for the backward (fp32, at most
-    4 GiB: 8192 rows at a vocabulary of 131072; memory permitting).  Above that nothing of size
-    ``[tokens, vocab]`` ever exists: the backward recomputes the logits one vocabulary chunk at a time, with the
-    same results (for a step of any size without that recomputation see
+    4 GiB: 8192 rows at a vocabulary of 131072), where memory is plentiful: at most 4 GiB over all live graphs of a
+    device, and an eighth of its free memory besides the backward's own needs.  Otherwise, with
+    ``keep_logits=False``, under saved-tensor hooks (activation checkpointing, offloading) and while a stream
+    captures, nothing of size ``[tokens, vocab]`` lives between the passes: the backward recomputes the logits one
+    vocabulary chunk at a time, with the same results.  A forward that never gets its backward pays the stores of
+    the kept logits for nothing (3072 rows, 4096 x 128256: 2.35 -> 2.77 ms): run it under ``torch.no_grad()`` or
+    with ``keep_logits=False``.  (For a step of any size without recomputation see
     :func:`open_instruct_amd.grpo_utils.grpo_loss_on_hidden` and
     :func:`open_instruct_amd.dpo_utils.dpo_loss_on_hidden`, which know the loss and can therefore
     finish a slab of tokens before they start the next).
@@ -195,7 +236,8 @@ def fused_lm_head_logprobs(
     # nothing to prepare; inside an autograd Function the grad mode is off, so it is read here
     grad = torch.is_grad_enabled()
     dhidden_in_forward = bool(dhidden_in_forward) and grad
-    lp, ent = _FusedLMHead.apply(hid2, weight, lab1, mask, inv_t, return_entropy, compact_backward, dhidden_in_forward, grad)
+    lp, ent = _FusedLMHead.apply(hid2, weight, lab1, mask, inv_t, return_entropy, compact_backward, dhidden_in_forward,
+                                 bool(keep_logits) and grad)
     return lp.reshape(lead), (ent.reshape(lead) if ent is not None else None)
 
 
@@ -208,6 +250,7 @@ def fused_linear_cross_entropy(
     num_items_in_batch: torch.Tensor | int | float | None = None,
     ignore_index: int = -100,
     token_slabs: bool | int = False,
+    keep_logits: bool = True,
 ) -> torch.Tensor:
     """Causal-LM cross-entropy of ``hidden @ weight.T`` against next-token labels, scalar fp32.
 
@@ -223,7 +266,8 @@ def fused_linear_cross_entropy(
     constant ``-1 / count``, so the step can run slab by slab like
     :func:`open_instruct_amd.grpo_utils.grpo_loss_on_hidden` (whose ``loss_fn="cispo"`` term with
     unit advantages, ratio 1 and no KL term *is* the negative log-likelihood); the gradients are
-    handed out by ``loss.backward()``.  Needs a 2-D ``[B, T]`` batch.
+    handed out by ``loss.backward()``.  Needs a 2-D ``[B, T]`` batch.  ``keep_logits``: see
+    :func:`fused_lm_head_logprobs` (without ``token_slabs``).
     """
     if (labels is None) == (shift_labels is None):
         raise ValueError("pass exactly one of labels / shift_labels")
@@ -250,7 +294,7 @@ def fused_linear_cross_entropy(
             loss_denominator=denominator, token_slabs=token_slabs,
         )  # fmt: skip
         return loss
-    logps, _ = fused_lm_head_logprobs(hidden, weight, shift_labels, mask=keep)
+    logps, _ = fused_lm_head_logprobs(hidden, weight, shift_labels, mask=keep, keep_logits=keep_logits)
     total = -logps.sum()
     if num_items_in_batch is None:
         return total / keep.sum().clamp(min=1)

@@ -42,6 +42,8 @@ class DPOLMHead(torch.nn.Module):
     """
 
     score_ignored_positions = False
+    # False: nothing of size [tokens, vocab] is held between the passes (lm_head.fused_lm_head_logprobs)
+    keep_logits = True
     # Set for the duration of one model call by open_instruct_amd.dpo_utils.fused_loss_olmo: the keyword
     # arguments of dpo_loss_on_hidden.  The head then computes the preference loss and both gradients in the
     # same call as the logps (nothing recomputed) and leaves the result in `fused_result`.
@@ -83,7 +85,9 @@ class DPOLMHead(torch.nn.Module):
             return LMOutputWithLoss(logits=None, loss=logps, ce_loss=logps.clone(), z_loss=None)
         shifted = padding_free_collator.shift_labels(labels)
         keep = None if self.score_ignored_positions else shifted != ignore_index
-        per_token_logps, _ = lm_head.fused_lm_head_logprobs(h, self.w_out.weight, shifted, mask=keep)
+        per_token_logps, _ = lm_head.fused_lm_head_logprobs(
+            h, self.w_out.weight, shifted, mask=keep, keep_logits=self.keep_logits
+        )
         return LMOutputWithLoss(
             logits=None, loss=per_token_logps, ce_loss=per_token_logps.detach().clone(), z_loss=None
         )
