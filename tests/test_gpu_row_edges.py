@@ -111,3 +111,25 @@ def test_statistics_of_few_and_many_rows(rows, cols, axis):
     assert stats["num_response_tokens"].item() == float(mask.sum())
     mean_pg = (e_pg.detach() * mask).sum().item() / mask.sum().item()
     assert abs(stats["loss/policy_avg"].item() - mean_pg) <= 1e-5 * max(1.0, abs(mean_pg))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("shift", [0, 1])
+def test_scaling_by_a_device_scalar(dtype, shift):
+    """Every element once, at the ends of the pieces that a thread takes two at a time (768 x 256 threads on 256 CUs).
+    A product is rounded to fp32 and then to the dtype, or to the dtype at once (the compiler's choice): half a unit
+    in the last place of either, and half the smallest fp16 number."""
+    vec, threads = 16 // dtype.itemsize, 3 * torch.cuda.get_device_properties(0).multi_processor_count * 256
+    tag = _lib.DTYPE_TAGS[dtype]
+    for n in (1, vec - 1, vec * threads - 1, vec * threads, vec * (threads + 1) + 1, 2 * vec * threads, vec * (3 * threads - 1) + 3):
+        print("case scale", dtype, shift, n, flush=True)
+        x = torch.randn(n + 2, device=DEV).to(dtype)
+        for value in (1.0, -0.3):
+            scale = torch.tensor([value], device=DEV)
+            got = x.clone()
+            _lib.call("oi_scale_by_device_scalar", got[shift:].data_ptr(), tag, n, scale.data_ptr(), _lib.stream_of(got))
+            exp = x.double()
+            exp[shift : shift + n] *= scale.double()
+            bound = exp.abs() * (torch.finfo(dtype).eps / 2 + 2**-24) + 2**-25
+            assert ((got.double() - exp).abs() <= (bound if value != 1.0 else 0.0)).all()
+            assert torch.equal(got[:shift], x[:shift]) and torch.equal(got[shift + n :], x[shift + n :])
