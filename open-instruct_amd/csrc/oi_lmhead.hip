@@ -1399,6 +1399,170 @@ __global__ void __launch_bounds__(NTHREADS)
     }
 }
 
+// ---- products whose rows are not whole 16-byte pieces --------------------------------------------------------
+// The stand-alone products take any pitch and any alignment of the element type (modes 0, 1 and 2, no row index, no
+// factors); the others' rows are hidden_dim (a multiple of 64) columns.  Kept out of gemm_store_kernel, whose main
+// loop comes out 0.3 to 1.6 % slower with either this code or less code in it.
+//
+// Widest access of a row: 8 columns (16 bytes of bf16), 4 (16 bytes of fp32, 8 of bf16), 2 (4 bytes of bf16) or 1;
+// `out` is the buffer that the mode touches
+__host__ __device__ inline int store_width(int mode, const void* out, int64_t N, int64_t ldo) {
+    const uintptr_t p = reinterpret_cast<uintptr_t>(out), element = mode <= 1 ? 4 : 2;
+    if (((N | ldo) & 7) == 0 && (p & 15) == 0) return 8;
+    if (((N | ldo) & 3) == 0 && (p & (4 * element - 1)) == 0) return 4;
+    return mode == 2 && (ldo & 1) == 0 && (p & 3) == 0 ? 2 : 1;
+}
+
+// A staged group whose rows cannot be stored four columns at a time: a lane takes W columns every 64 W, so that a
+// wave's access is one run of a row; four rows at a time, whose sums so far (clamped onto valid entries) and LDS
+// reads are all under way before the first is used.
+// Four neighbouring columns per lane, stored one by one, against this: bf16 [8192, 8190] x 256 113 -> 76 us, fp32 130
+// -> 91, added to fp32 243 -> 135; added to fp32 [300, 1001] x 512 49 -> 25.
+template <int W>
+__device__ __forceinline__ void store_group_by_columns(const StoreTo& st, int64_t row0, int64_t col0, int j, const float* stage32,
+                                                       int tid) {
+    constexpr int PER = BM / (64 * W), ROWS = 4;
+    const int mode = st.mode, lane = tid & 63, left = (int)(st.N - col0 < BM ? st.N - col0 : BM);
+#pragma unroll 1
+    for (int r0 = tid >> 6; r0 < GROUP_ROWS; r0 += 8 * ROWS) {
+        float v[ROWS][PER][W];
+        int64_t row[ROWS], dst[ROWS];
+#pragma unroll
+        for (int u = 0; u < ROWS; ++u) {
+            row[u] = group_row(row0, j, r0 + 8 * u);
+            const int64_t r = row[u] < st.m_valid ? row[u] : st.m_valid - 1;
+            dst[u] = (mode >= 2 && st.out_rows ? (int64_t)st.out_rows[r] : r) * st.ldo + col0;
+        }
+        if (mode == 1) {
+#pragma unroll
+            for (int u = 0; u < ROWS; ++u)
+#pragma unroll
+                for (int k = 0; k < PER; ++k)
+#pragma unroll
+                    for (int w = 0; w < W; ++w) {
+                        const int c = (lane + 64 * k) * W + w;
+                        v[u][k][w] = st.out_f32[dst[u] + (c < left ? c : left - 1)];
+                    }
+        }
+#pragma unroll
+        for (int u = 0; u < ROWS; ++u)
+#pragma unroll
+            for (int k = 0; k < PER; ++k)
+#pragma unroll
+                for (int w = 0; w < W; ++w) {
+                    const float z = stage32[(r0 + 8 * u) * STAGE_F32 + (lane + 64 * k) * W + w];
+                    v[u][k][w] = mode == 1 ? v[u][k][w] + z : z;
+                }
+#pragma unroll
+        for (int u = 0; u < ROWS; ++u) {
+            if (row[u] >= st.m_valid) return;
+#pragma unroll
+            for (int k = 0; k < PER; ++k) {
+                const int c = (lane + 64 * k) * W;
+                if (c >= left) continue;
+                if (W == 2 && c + 1 < left) {
+                    *reinterpret_cast<uint32_t*>(st.out_bf16 + dst[u] + c) = oi_pack_bf16x2(v[u][k][0], v[u][k][W - 1]);
+                } else if (mode <= 1) {
+                    st.out_f32[dst[u] + c] = v[u][k][0];
+                } else {
+                    st.out_bf16[dst[u] + c] = (uint16_t)oi_f32_to_bf16_bits(v[u][k][0]);
+                }
+            }
+        }
+    }
+}
+
+// Column group j of a tile through the LDS region `stage`, as store_group_f32
+__device__ __forceinline__ void store_group_any(const f32x16& z0, const f32x16& z1, const StoreTo& st, int width, int64_t row0,
+                                                int64_t col0, int j, uint16_t* stage, int tid) {
+    asm volatile("" : "+v"(tid));
+    const int lane = tid & 63, wave = tid >> 6, wm = wave & 3, wn = wave >> 2;
+    const int mode = st.mode, srow = wn * 32 + (lane & 31);
+    float* stage32 = reinterpret_cast<float*>(stage);
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const f32x16& z = i == 0 ? z0 : z1;
+            *reinterpret_cast<oi_f32x4*>(stage32 + srow * STAGE_F32 + acc_row(wm, i, q * 4, lane)) =
+                oi_f32x4{z[q * 4], z[q * 4 + 1], z[q * 4 + 2], z[q * 4 + 3]};
+        }
+    lds_barrier();
+    if (width == 2) return store_group_by_columns<2>(st, row0, col0, j, stage32, tid);
+    if (width == 1) return store_group_by_columns<1>(st, row0, col0, j, stage32, tid);
+    // four columns at once (added to fp32 [128256, 4092] x 256: one by one 1857 us, so 945; bf16 901 -> 561)
+    constexpr int ITERS = GROUP_ROWS * (BM / 4) / NTHREADS;
+    const int ch = tid & 63, r_first = tid >> 6;
+    const int64_t col = col0 + ch * 4;
+    if (col >= st.N) return;
+    oi_f32x4 v[ITERS];
+    if (mode == 1) {
+#pragma unroll
+        for (int it = 0; it < ITERS; ++it) {
+            int64_t row = group_row(row0, j, r_first + it * 8);
+            row = row < st.m_valid ? row : st.m_valid - 1;
+            v[it] = *reinterpret_cast<const oi_f32x4*>(st.out_f32 + row * st.ldo + col);
+        }
+    }
+#pragma unroll
+    for (int it = 0; it < ITERS; ++it) {
+        const oi_f32x4 z = *reinterpret_cast<const oi_f32x4*>(stage32 + (r_first + it * 8) * STAGE_F32 + ch * 4);
+        v[it] = mode == 1 ? v[it] + z : z;
+    }
+#pragma unroll
+    for (int it = 0; it < ITERS; ++it) {
+        const int64_t row = group_row(row0, j, r_first + it * 8);
+        if (row >= st.m_valid) return;
+        if (mode <= 1)
+            *reinterpret_cast<oi_f32x4*>(st.out_f32 + row * st.ldo + col) = v[it];
+        else
+            *reinterpret_cast<uint2*>(st.out_bf16 + row * st.ldo + col) =
+                make_uint2(oi_pack_bf16x2(v[it].x, v[it].y), oi_pack_bf16x2(v[it].z, v[it].w));
+    }
+}
+
+// one workgroup per tile id, width < 8
+template <bool R_KM, bool C_KM>
+__global__ void __launch_bounds__(NTHREADS)
+    gemm_any_kernel(Operand R, int64_t M, Operand C, int64_t N, int64_t K, int mode, float* out_f32, uint16_t* out_bf16,
+                    int64_t ldo, int width) {
+    __shared__ __align__(16) uint16_t lds[LDS_ELEMS];
+    const StoreTo st = {mode, out_f32, out_bf16, ldo, N, M, nullptr, nullptr, nullptr};
+    const uint32_t tiles_r = (uint32_t)((M + BN - 1) / BN), tiles_c = (uint32_t)((N + BM - 1) / BM);
+    const uint32_t item = item_of_pid(blockIdx.x, tiles_r * tiles_c);
+    if (item >= tiles_r * tiles_c) return;
+    int64_t tr, tc;
+    tile_of_item(item, tiles_r, tiles_c, &tr, &tc);
+    R.r0 = tr * BN;
+    C.r0 = tc * BM;
+    AccTile acc;
+    gemm_tile<C_KM, R_KM>(acc, C, R, K, lds);
+    const int tid = opaque_tid();
+    // two regions in turn, as in store_tile
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        __builtin_amdgcn_sched_barrier(0);
+        store_group_any(acc[0][j], acc[1][j], st, width, R.r0, C.r0, j, lds + (j & 1) * GROUP_F32, tid);
+        __builtin_amdgcn_sched_barrier(0);
+    }
+}
+
+template <bool R_KM, bool C_KM>
+int launch_product(const Operand& a, int64_t M, const Operand& b, int64_t N, int64_t K, float* out_f32, void* out_bf16, int64_t ldo,
+                   int accumulate, hipStream_t s) {
+    const int mode = out_f32 ? (accumulate ? 1 : 0) : 2;
+    const int width = store_width(mode, out_f32 ? static_cast<void*>(out_f32) : out_bf16, N, ldo);
+    const dim3 grid(grid_for_tiles((M + BM - 1) / BM, (N + BN - 1) / BN));
+    uint16_t* o16 = static_cast<uint16_t*>(out_bf16);
+    if (width == 8)
+        hipLaunchKernelGGL((gemm_store_kernel<R_KM, C_KM>), grid, dim3(NTHREADS), 0, s, a, M, b, N, K, mode, out_f32, o16, ldo, M,
+                           DynRows{}, static_cast<uint32_t*>(nullptr), static_cast<float*>(nullptr));
+    else
+        hipLaunchKernelGGL((gemm_any_kernel<R_KM, C_KM>), grid, dim3(NTHREADS), 0, s, a, M, b, N, K, mode, out_f32, o16, ldo,
+                           width);
+    return oi_launch_status();
+}
+
 // Adds the pieces of the split tiles of a gemm_store_kernel launch over `grid` workgroups and stores the
 // sums as that kernel stores a tile.  One workgroup per column group of a tile (as in lmhead_dz_kept_kernel);
 // bound by reading the pieces once.
@@ -2971,13 +3135,9 @@ extern "C" int oi_gemm_bf16_tn(const void* A, int64_t lda, int64_t M, const void
     OI_RETURN_IF(!oi_aligned(A, 16) || !oi_aligned(B, 16), OI_EALIGN);
     // bf16 rows of even pitch are written as pairs (4-byte words), fp32 results as single words
     OI_RETURN_IF(!oi_aligned(out_f32, 4) || !oi_aligned(out_bf16, (ldo & 1) ? 2 : 4), OI_EALIGN);
-    const int mode = out_f32 ? (accumulate ? 1 : 0) : 2;
     const Operand a = {static_cast<const uint16_t*>(A), lda, 0, M, K};
     const Operand b = {static_cast<const uint16_t*>(B), ldb, 0, N, K};
-    hipLaunchKernelGGL((gemm_store_kernel<false, false>), dim3(grid_for_tiles((M + BM - 1) / BM, (N + BN - 1) / BN)),
-                       dim3(NTHREADS), 0, static_cast<hipStream_t>(stream), a, M, b, N, K, mode, out_f32,
-                       static_cast<uint16_t*>(out_bf16), ldo, M, DynRows{nullptr, 0, nullptr, nullptr, nullptr, nullptr}, static_cast<uint32_t*>(nullptr), static_cast<float*>(nullptr));
-    return oi_launch_status();
+    return launch_product<false, false>(a, M, b, N, K, out_f32, out_bf16, ldo, accumulate, static_cast<hipStream_t>(stream));
 }
 
 extern "C" int oi_gemm_bf16_layouts(const void* A, int64_t lda, int a_k_major, const void* B, int64_t ldb,
@@ -2993,26 +3153,11 @@ extern "C" int oi_gemm_bf16_layouts(const void* A, int64_t lda, int a_k_major, c
     OI_RETURN_IF(!oi_aligned(A, 16) || !oi_aligned(B, 16), OI_EALIGN);
     // bf16 rows of even pitch are written as pairs (4-byte words), fp32 results as single words
     OI_RETURN_IF(!oi_aligned(out_f32, 4) || !oi_aligned(out_bf16, (ldo & 1) ? 2 : 4), OI_EALIGN);
-    const int mode = out_f32 ? (accumulate ? 1 : 0) : 2;
     const Operand a = {static_cast<const uint16_t*>(A), lda, 0, M, K};
     const Operand b = {static_cast<const uint16_t*>(B), ldb, 0, N, K};
-    const dim3 grid(grid_for_tiles((M + BM - 1) / BM, (N + BN - 1) / BN));
     hipStream_t s = static_cast<hipStream_t>(stream);
-    uint16_t* o16 = static_cast<uint16_t*>(out_bf16);
-    uint32_t* no_queue = nullptr;
-    float* no_parts = nullptr;
-    const DynRows fixed = {nullptr, 0, nullptr, nullptr, nullptr, nullptr};
-    if (a_k_major && b_k_major)
-        hipLaunchKernelGGL((gemm_store_kernel<true, true>), grid, dim3(NTHREADS), 0, s, a, M, b, N, K, mode, out_f32, o16,
-                           ldo, M, fixed, no_queue, no_parts);
-    else if (a_k_major)
-        hipLaunchKernelGGL((gemm_store_kernel<true, false>), grid, dim3(NTHREADS), 0, s, a, M, b, N, K, mode, out_f32,
-                           o16, ldo, M, fixed, no_queue, no_parts);
-    else if (b_k_major)
-        hipLaunchKernelGGL((gemm_store_kernel<false, true>), grid, dim3(NTHREADS), 0, s, a, M, b, N, K, mode, out_f32,
-                           o16, ldo, M, fixed, no_queue, no_parts);
-    else
-        hipLaunchKernelGGL((gemm_store_kernel<false, false>), grid, dim3(NTHREADS), 0, s, a, M, b, N, K, mode, out_f32,
-                           o16, ldo, M, fixed, no_queue, no_parts);
-    return oi_launch_status();
+    if (a_k_major && b_k_major) return launch_product<true, true>(a, M, b, N, K, out_f32, out_bf16, ldo, accumulate, s);
+    if (a_k_major) return launch_product<true, false>(a, M, b, N, K, out_f32, out_bf16, ldo, accumulate, s);
+    if (b_k_major) return launch_product<false, true>(a, M, b, N, K, out_f32, out_bf16, ldo, accumulate, s);
+    return launch_product<false, false>(a, M, b, N, K, out_f32, out_bf16, ldo, accumulate, s);
 }

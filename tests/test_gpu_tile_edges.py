@@ -94,7 +94,7 @@ def test_products_cut_along_the_vocabulary(n, h, v, route):
         _close(w.grad, dw, "d_weight")
 
 
-@pytest.mark.parametrize("n,h,v", [(70, 64, 301), (300, 320, 513)])
+@pytest.mark.parametrize("n,h,v", [(70, 64, 301), (300, 320, 513), (16500, 64, 66000)])  # the last: three chunks
 def test_gradients_off_16_byte_boundaries(n, h, v):
     """Gradients that lie on 4-byte boundaries only are stored by another route of the same epilogue."""
     print("case unaligned gradients", n, h, v, flush=True)
@@ -124,3 +124,38 @@ def test_gradients_off_16_byte_boundaries(n, h, v):
         got.append((dh[shift : shift + n * h], dw[shift : shift + v * h]))
     for a, b in zip(*got):
         assert a.float().abs().max() > 0 and torch.equal(a, b)
+
+
+@pytest.mark.parametrize(
+    "m,n,k,ldo,shift",
+    [
+        (257, 264, 64, 272, 0),  # whole 16-byte pieces
+        (300, 260, 128, 260, 0),  # four columns at a time
+        (64, 300, 192, 308, 4),  # the same, results off 16-byte boundaries
+        (130, 258, 64, 262, 2),  # pairs of bf16
+        (66, 517, 64, 518, 0),  # pairs and a last single column
+        (5, 1001, 128, 1001, 0),  # one column at a time
+        (513, 3, 64, 7, 0),
+    ],
+)
+def test_products_of_any_pitch(m, n, k, ldo, shift):
+    """Small whole numbers: every sum is exact in fp32 and is rounded once to bf16, so nothing may differ, and
+    nothing may be written around the result."""
+    print("case product", m, n, k, ldo, shift, flush=True)
+    lib = _lib.load()
+    stream = torch.cuda.current_stream().cuda_stream
+    g = torch.Generator().manual_seed(m + n)
+    a = torch.randint(-4, 5, (m, k), generator=g).bfloat16().to(DEV)
+    b = torch.randint(-4, 5, (n, k), generator=g).bfloat16().to(DEV)
+    exact = a.float() @ b.float().t()
+    for dtype, accumulate in ((torch.float32, 0), (torch.float32, 1), (torch.bfloat16, 0)):
+        out = torch.full((m * ldo + shift + 8,), 3.0, dtype=dtype, device=DEV)
+        rows = out[shift : shift + m * ldo].view(m, ldo)
+        o = rows.data_ptr()
+        rc = lib.oi_gemm_bf16_tn(
+            a.data_ptr(), k, m, b.data_ptr(), k, n, k, o if dtype == torch.float32 else None,
+            o if dtype == torch.bfloat16 else None, ldo, accumulate, stream,
+        )  # fmt: skip
+        assert rc == 0
+        assert torch.equal(rows[:, :n], (exact + 3.0 * accumulate).to(dtype)), (dtype, accumulate)
+        assert (rows[:, n:] == 3).all() and (out[:shift] == 3).all() and (out[shift + m * ldo :] == 3).all()
