@@ -1276,14 +1276,6 @@ __host__ __device__ inline TailSplit plan_tail(uint32_t tiles, uint32_t grid, ui
     }
     return t;
 }
-// scratch for the pieces of a product of at most `tiles` tiles with at most `ktiles` k-tiles
-inline size_t split_bytes(int64_t tiles, int64_t ktiles) {
-    int64_t parts = ktiles / SPLIT_MIN_KTILES;
-    parts = parts < SPLIT_MAX_PARTS ? parts : SPLIT_MAX_PARTS;
-    if (parts < 2) return 0;
-    const int64_t items = tiles * parts;
-    return (size_t)(items < SPLIT_MAX_ITEMS ? items : SPLIT_MAX_ITEMS) * PART_FLOATS * sizeof(float);
-}
 
 // The sizes of a product that only the device knows, filled in from dyn
 struct ProductSizes {
@@ -1842,6 +1834,26 @@ unsigned resident_grid(int64_t tiles_m, int64_t tiles_n) {
     return (unsigned)(pids < grid ? pids : grid);
 }
 
+// Scratch for the pieces of the rows products of a call, as launch_rows_product starts them: at most `row_tiles` x
+// `h_tiles` tiles, the vocabulary in chunks of `chunk` columns.  The row count is known on the device only, so it is
+// the most that plan_tail asks for at any count up to there: 256 pieces of 256 KB for one or two row tiles of 4096
+// columns, 1008 for seven and more.
+size_t split_bytes(int64_t row_tiles, int64_t h_tiles, int64_t chunk, int64_t vocab) {
+    const uint32_t grid = resident_grid(row_tiles, h_tiles);
+    const int64_t columns[2] = {chunk < vocab ? chunk : vocab, (vocab - 1) % chunk + 1};  // of the first and last chunk
+    uint32_t most = 0;
+    for (int64_t c : columns) {
+        const uint32_t ktiles = (uint32_t)(round_up(c, BK) / BK);
+        // what is left of whole rounds repeats after `grid` row tiles
+        for (int64_t r = 1; r <= row_tiles && r <= (int64_t)grid && ktiles >= 2 * SPLIT_MIN_KTILES; ++r) {
+            const TailSplit t = plan_tail((uint32_t)(r * h_tiles), grid, ktiles);
+            if (t.rest * t.parts > most) most = t.rest * t.parts;
+        }
+        if (columns[0] == columns[1]) break;
+    }
+    return (size_t)most * PART_FLOATS * sizeof(float);
+}
+
 // Vocabulary columns that the recomputing backward takes at a time.  At 32768 token rows 32768, 65536 and
 // the whole vocabulary measured the same and 16384 columns 1.3-2.5 % slower, so the scratch (2 bytes per
 // token row and column) decides; fewer rows take as many more columns as the same scratch holds, up to the
@@ -1938,7 +1950,7 @@ FwdPlan plan_fwd(int64_t n_tokens, int64_t hdim, int64_t vocab, bool with_select
     p.off_queue = cv.take((chunked ? (size_t)p.n_chunks * (FWD_QUEUE_WORDS + QUEUE_WORDS) : (size_t)FWD_QUEUE_WORDS) *
                           sizeof(uint32_t));
     p.off_chunk = chunked ? cv.take((size_t)p.n_pad * p.chunk * 2) : 0;
-    p.parts_bytes = chunked ? split_bytes(p.token_tiles * ((hdim + BN - 1) / BN), p.chunk / BK) : 0;
+    p.parts_bytes = chunked ? split_bytes(p.token_tiles, (hdim + BN - 1) / BN, p.chunk, vocab) : 0;
     p.off_parts = cv.take(p.parts_bytes);
     if (with_selection) p.sel = plan_selection(cv, p.n_pad, hdim, false);
     p.total = cv.off;
@@ -1975,7 +1987,7 @@ BwdPlan plan_bwd(int64_t n_tokens, int64_t hdim, int64_t vocab, bool with_select
     p.off_dh32 = cv.take((size_t)n_tokens * hdim * 4);
     // one set of work-queue counters per tile-kernel launch (three per vocabulary chunk)
     p.off_queues = cv.take((size_t)(3 * p.n_chunks) * QUEUE_WORDS * sizeof(uint32_t));
-    p.parts_bytes = few_rows ? 0 : split_bytes(p.n_pad / BM * ((hdim + BN - 1) / BN), p.chunk / BK);
+    p.parts_bytes = few_rows ? 0 : split_bytes(p.n_pad / BM, (hdim + BN - 1) / BN, p.chunk, vocab);
     p.off_parts = cv.take(p.parts_bytes);
     if (with_selection) p.sel = plan_selection(cv, p.n_pad, hdim, true);
     p.total = cv.off;
@@ -2353,7 +2365,7 @@ SlabPlan plan_slabs(int64_t n, int64_t stats_rows, int64_t stats_cols, int64_t h
     p.off_lse = cv.take((size_t)n * sizeof(float));
     p.off_grad = cv.take((size_t)n * sizeof(float));
     p.off_denoms = cv.take((size_t)stats_rows * sizeof(float));
-    p.parts_bytes = split_bytes(p.cap / BM * ((hdim + BN - 1) / BN), p.v_pad / BK);
+    p.parts_bytes = split_bytes(p.cap / BM, (hdim + BN - 1) / BN, p.v_pad, vocab);
     p.off_parts = cv.take(p.parts_bytes);
     p.total = cv.off;
     return p;

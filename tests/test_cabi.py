@@ -141,3 +141,36 @@ def test_missing_library_is_an_error(monkeypatch):
     monkeypatch.setattr(_lib, "LIB_PATH", "/nonexistent/liboi_kernels.so")
     with pytest.raises(RuntimeError, match="no fallback"):
         _lib.load()
+
+
+def _pieces(tiles, ktiles, grid=256):
+    """Pieces into which the tiles past the last whole round are cut: rounds of pieces, 4 k-tiles of prologue and drain
+    per piece and 3/32 of a k-tile for writing and reading one, against a round of whole tiles."""
+    rest = tiles % grid
+    best, pieces = 32 * (ktiles + 4), 0
+    for parts in range(2, 33):
+        if rest == 0 or rest * parts > 1024 or ktiles < 16 * parts:
+            break
+        cost = -(-rest * parts // grid) * (32 * ktiles // parts + 128) + 3 * rest * parts
+        if cost < best:
+            best, pieces = cost, rest * parts
+    return pieces
+
+
+@pytest.mark.parametrize(
+    "n,h,v",
+    [(1, 64, 300), (70, 64, 2048), (382, 4096, 100352), (2048, 8192, 128256), (3072, 4096, 128256), (2400, 3584, 151665),
+     (9000, 64, 120000), (70000, 192, 5000)],
+)  # fmt: skip
+def test_backward_scratch_holds_the_pieces_of_any_row_count_and_no_more(n, h, v):
+    up = lambda x, m: -(-x // m) * m  # noqa: E731
+    n_pad, v_pad = up(n, 256), up(v, 256)
+    most = max((1 << 30) // n_pad // 1024 * 1024, 32768)
+    chunks = -(-v_pad // most)
+    chunk = v_pad if chunks == 1 else up(-(-v_pad // chunks), 1024)
+    chunks = -(-v_pad // chunk)
+    h_tiles = -(-h // 256)
+    ktiles = {up(min(chunk, v), 64) // 64, up((v - 1) % chunk + 1, 64) // 64}
+    pieces = max(_pieces(r * h_tiles, k) for r in range(1, n_pad // 256 + 1) for k in ktiles)
+    parts = [n_pad * chunk * 2, n * h * 4, 3 * chunks * 32, pieces * 256 * 1024]
+    assert _lib.load().oi_lmhead_bwd_workspace_bytes(n, h, v, 1, 0) == sum(up(b, 256) for b in parts)
