@@ -8,6 +8,8 @@ from __future__ import annotations
 
 import ctypes
 import os
+import sysconfig
+import warnings
 from ctypes import c_char_p, c_double, c_float, c_int, c_int64, c_size_t, c_uint32, c_void_p
 
 import torch
@@ -88,7 +90,8 @@ SIGNATURES: dict[str, tuple] = {
     "oi_gemm_bf16_layouts": (_I, [_P, _I64, _I, _P, _I64, _I, _I64, _I64, _I64, _P, _P, _I64, _I, _P]),
 }
 
-PYLISTS_PATH = os.path.join(_HERE, "csrc", "liboi_pylists.so")
+# reads the storage of list and float objects, so it belongs to one interpreter version
+PYLISTS_PATH = os.path.join(_HERE, "csrc", "liboi_pylists" + sysconfig.get_config_var("EXT_SUFFIX"))
 PYLISTS_SIGNATURES: dict[str, list] = {
     "oi_py_offsets": [ctypes.py_object, _I64, _P],
     "oi_py_flatten_ints": [ctypes.py_object, _I64, _P, _I64, _P, _P],
@@ -97,7 +100,7 @@ PYLISTS_SIGNATURES: dict[str, list] = {
 }
 
 _lib: ctypes.CDLL | None = None
-_pylists: ctypes.PyDLL | None = None
+_pylists: ctypes.PyDLL | bool | None = None  # False: looked for and not there
 
 
 class KernelError(RuntimeError):
@@ -122,19 +125,25 @@ def load() -> ctypes.CDLL:
     return _lib
 
 
-def pylists() -> ctypes.PyDLL:
-    """The host library that reads Python lists, loaded once; its functions run under the interpreter lock."""
+def pylists() -> ctypes.PyDLL | None:
+    """The host library that reads Python lists, loaded once; its functions run under the interpreter lock.  None,
+    with one warning, where it was not built for this interpreter: the caller then walks the lists with numpy."""
     global _pylists
     if _pylists is None:
         if not os.path.exists(PYLISTS_PATH):
-            raise RuntimeError(f"{PYLISTS_PATH} is missing: build it with `python -m open_instruct_amd.build`")
+            warnings.warn(
+                f"{PYLISTS_PATH} is missing: lists are read element by element (build it with "
+                "`python -m open_instruct_amd.build`)", RuntimeWarning, stacklevel=2,
+            )  # fmt: skip
+            _pylists = False
+            return None
         lib = ctypes.PyDLL(PYLISTS_PATH)
         for name, argtypes in PYLISTS_SIGNATURES.items():
             fn = getattr(lib, name)
             fn.restype = _I
             fn.argtypes = argtypes
         _pylists = lib
-    return _pylists
+    return _pylists or None
 
 
 def ptr(t: torch.Tensor | None) -> int | None:

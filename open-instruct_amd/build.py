@@ -1,6 +1,7 @@
 """Build ``csrc/liboi_kernels.so`` for gfx950 with hipcc (``python -m open_instruct_amd.build``), and beside it
-``csrc/liboi_pylists.so``, host code that reads Python lists and is kept apart because it needs an interpreter
-around it (the kernel library does not).
+``csrc/liboi_pylists.<interpreter>.so``, host code that reads Python lists and is kept apart because it needs an
+interpreter around it, and one of the version that it was compiled for (the kernel library does not).  Without the
+interpreter's headers it is left out: its callers have a general path.
 
 The shared objects are built in-tree so that they travel with the source tree; nothing is compiled
 at import time.
@@ -19,7 +20,7 @@ INCLUDE = os.path.join(os.path.dirname(HERE), "include")
 SOURCES = ["oi_rowwise.hip", "oi_loss.hip", "oi_pack.hip", "oi_lmhead.hip"]
 OUTPUT = os.path.join(CSRC, "liboi_kernels.so")
 PYLISTS_SOURCE = os.path.join(CSRC, "oi_pylists.cpp")
-PYLISTS_OUTPUT = os.path.join(CSRC, "liboi_pylists.so")
+PYLISTS_OUTPUT = os.path.join(CSRC, "liboi_pylists" + sysconfig.get_config_var("EXT_SUFFIX"))
 
 HIPCC_FLAGS = [
     "--offload-arch=gfx950",
@@ -63,6 +64,9 @@ def build(verbose: bool = False) -> str:
     for obj in objs:
         os.remove(obj)
     include = sysconfig.get_paths()["include"]
+    if not os.path.exists(os.path.join(include, "Python.h")):
+        print(f"no Python.h in {include}: {os.path.basename(PYLISTS_OUTPUT)} is not built", file=sys.stderr)
+        return OUTPUT
     cmd = [_hipcc(), "-x", "c++", "-O3", "-std=c++17", "-fPIC", "-shared", f"-I{include}", PYLISTS_SOURCE, "-o", PYLISTS_OUTPUT]
     res = subprocess.run(cmd, capture_output=True, text=True)
     if res.returncode != 0:

@@ -124,11 +124,17 @@ class PackedSequences:
 _INT64 = range(-(2**63), 2**63)
 
 
+def _native(name: str, *args) -> bool:
+    """Whether the native reader took these lists (otherwise its outputs mean nothing)."""
+    lib = _lib.pylists()
+    return lib is not None and getattr(lib, name)(*args) == 0
+
+
 def _offsets(seqs) -> np.ndarray:
     """Where each sequence starts in the flat array, and the end."""
     n = len(seqs)
     offsets = np.empty(n + 1, dtype=np.int64)
-    if _lib.pylists().oi_py_offsets(seqs, n, offsets.ctypes.data):
+    if not _native("oi_py_offsets", seqs, n, offsets.ctypes.data):
         offsets[0] = 0
         np.cumsum(np.fromiter((len(x) for x in seqs), dtype=np.int64, count=n), out=offsets[1:])
     return offsets
@@ -144,7 +150,7 @@ def _fill_ints(seqs, offsets: np.ndarray, out: np.ndarray, skip) -> np.ndarray:
     n = len(offsets) - 1
     others = np.empty(n, dtype=np.int64)
     if type(skip) is int and skip in _INT64:
-        if not _lib.pylists().oi_py_flatten_ints(seqs, n, offsets.ctypes.data, skip, out.ctypes.data, others.ctypes.data):
+        if _native("oi_py_flatten_ints", seqs, n, offsets.ctypes.data, skip, out.ctypes.data, others.ctypes.data):
             return others
     out[:] = _walk(seqs, offsets, np.int64)
     before = np.zeros(len(out) + 1, dtype=np.int64)
@@ -153,12 +159,12 @@ def _fill_ints(seqs, offsets: np.ndarray, out: np.ndarray, skip) -> np.ndarray:
 
 
 def _fill_flags(seqs, offsets: np.ndarray, out: np.ndarray) -> None:
-    if _lib.pylists().oi_py_flatten_flags(seqs, len(offsets) - 1, offsets.ctypes.data, out.ctypes.data):
+    if not _native("oi_py_flatten_flags", seqs, len(offsets) - 1, offsets.ctypes.data, out.ctypes.data):
         out[:] = _walk(seqs, offsets, np.int64) != 0
 
 
 def _fill_floats(seqs, offsets: np.ndarray, out: np.ndarray) -> None:
-    if _lib.pylists().oi_py_flatten_floats(seqs, len(offsets) - 1, offsets.ctypes.data, out.ctypes.data):
+    if not _native("oi_py_flatten_floats", seqs, len(offsets) - 1, offsets.ctypes.data, out.ctypes.data):
         out[:] = _walk(seqs, offsets, np.float32)
 
 

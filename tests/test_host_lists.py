@@ -1,6 +1,8 @@
 """The native readers of ragged Python lists against numpy's element by element walk, over what they take
 themselves (exact lists of exact numbers), what they leave to that walk, and what nothing takes."""
 
+import os
+
 import numpy as np
 import pytest
 import torch
@@ -48,6 +50,32 @@ def test_refused(bad, error):
     with pytest.raises(error):
         offsets = rl_utils._offsets(bad)
         rl_utils._fill_ints(bad, offsets, np.empty(offsets[-1], dtype=np.int64), 0)
+
+
+def test_without_the_native_reader_every_list_takes_the_walk(monkeypatch, tmp_path):
+    with_reader = [(rl_utils._offsets(s).tolist(), s) for s in INTS]
+    monkeypatch.setattr(rl_utils._lib, "PYLISTS_PATH", str(tmp_path / "none.so"))
+    monkeypatch.setattr(rl_utils._lib, "_pylists", None)
+    with pytest.warns(RuntimeWarning, match="missing") as caught:
+        for expected, seqs in with_reader:
+            offsets = rl_utils._offsets(seqs)
+            assert offsets.tolist() == expected
+            out, flags = np.empty(offsets[-1], dtype=np.int64), np.empty(offsets[-1], dtype=np.uint8)
+            others = rl_utils._fill_ints(seqs, offsets, out, 0)
+            rl_utils._fill_flags(seqs, offsets, flags)
+            assert out.tolist() == [int(x) for s in seqs for x in s] and flags.tolist() == [int(x != 0) for x in out]
+            assert others.tolist() == [sum(int(x) != 0 for x in s) for s in seqs]
+        floats = np.empty(2, dtype=np.float32)
+        rl_utils._fill_floats([[0.5], [2.0]], np.array([0, 1, 2]), floats)
+        assert floats.tolist() == [0.5, 2.0]
+    assert len(caught) == 1  # one warning, not one per call
+
+
+def test_the_reader_is_named_after_the_interpreter_it_was_built_for():
+    import sysconfig
+
+    assert os.path.basename(rl_utils._lib.PYLISTS_PATH) == "liboi_pylists" + sysconfig.get_config_var("EXT_SUFFIX")
+    assert rl_utils._lib.pylists() is not None
 
 
 def test_a_list_that_changed_since_its_length_was_taken():
