@@ -135,6 +135,9 @@ class _FusedLMHead(torch.autograd.Function):
 KEPT_BUDGET = 4 << 30
 # Device memory that has to be free for each byte of kept logits, once the backward's own needs are taken off.
 KEPT_SHARE = 8
+# Up to this many bytes over all live graphs are kept without a look at the free memory: the look takes 25 us of the
+# host, which calls with few logits do not hide (64 x 300, forward and backward: 155 us without it, 181 with it).
+KEPT_UNASKED = 256 << 20
 _kept_lock = threading.Lock()
 _kept_alive: list[weakref.ref] = []
 
@@ -150,7 +153,7 @@ def _free_bytes(dev) -> int:
 def _kept_logits(n, h, v, dev, selecting):
     """Memory for the forward's logits where they are kept for the backward, else None (the backward then
     computes them again, with the same results).  Kept only where nothing else has to give way for them:
-    not more than one call's largest share over all live graphs, and only out of plenty; not where saved tensors
+    not more than one call's largest share over all live graphs, and more than a little only out of plenty; not where saved tensors
     are packed (checkpointing counts them and would compute them twice, offloading would copy them), and not into
     the private pool of a graph, which would hold them as long as the graph lives."""
     lib = _lib.load()
@@ -159,14 +162,16 @@ def _kept_logits(n, h, v, dev, selecting):
         return None
     if torch.cuda.is_current_stream_capturing():
         return None
-    backward = lib.oi_lmhead_bwd_workspace_bytes(n, h, v, 1, int(selecting)) + 2 * h * (n + v)
     with _kept_lock:
         alive = [(r, t) for r, t in ((r, r()) for r in _kept_alive) if t is not None]
         _kept_alive[:] = [r for r, _ in alive]
-        if kept + sum(t.numel() * 4 for _, t in alive if t.device == dev) > KEPT_BUDGET:
+        together = kept + sum(t.numel() * 4 for _, t in alive if t.device == dev)
+        if together > KEPT_BUDGET:
             return None
-        if _free_bytes(dev) < KEPT_SHARE * kept + backward:
-            return None
+        if together > KEPT_UNASKED:
+            backward = lib.oi_lmhead_bwd_workspace_bytes(n, h, v, 1, int(selecting)) + 2 * h * (n + v)
+            if _free_bytes(dev) < KEPT_SHARE * kept + backward:
+                return None
         try:
             logits = torch.empty(kept // 4, dtype=torch.float32, device=dev)
         except torch.cuda.OutOfMemoryError:
@@ -201,7 +206,7 @@ def fused_lm_head_logprobs(
 
     When ``weight`` takes a gradient the forward of a small batch keeps its logits for the backward (fp32, at most
     4 GiB: 8192 rows at a vocabulary of 131072), where memory is plentiful: at most 4 GiB over all live graphs of a
-    device, and an eighth of its free memory besides the backward's own needs.  Otherwise, with
+    device and, beyond 256 MiB, an eighth of its free memory besides the backward's own needs.  Otherwise, with
     ``keep_logits=False``, under saved-tensor hooks (activation checkpointing, offloading) and while a stream
     captures, nothing of size ``[tokens, vocab]`` lives between the passes: the backward recomputes the logits one
     vocabulary chunk at a time, with the same results.  A forward that never gets its backward pays the stores of

@@ -79,6 +79,9 @@ def test_live_graphs_share_one_budget(plenty, monkeypatch):
 def test_kept_only_out_of_plenty(plenty, monkeypatch):
     lib = _lib.load()
     n, h, v = 300, 64, 1000
+    monkeypatch.setattr(lm_head, "_free_bytes", lambda dev: 0)
+    assert _ask(n, h, v) is not None  # a little is kept without asking
+    monkeypatch.setattr(lm_head, "KEPT_UNASKED", 0)
     needs = 8 * lib.oi_lmhead_kept_bytes(n, v) + lib.oi_lmhead_bwd_workspace_bytes(n, h, v, 1, 0) + 2 * h * (n + v)
     monkeypatch.setattr(lm_head, "_free_bytes", lambda dev: needs - 1)
     assert _ask(n, h, v) is None
@@ -128,6 +131,7 @@ def test_calls_without_kept_logits_give_the_same_bits(n, h, v, monkeypatch):
     kept = run(True)
     others = [run(False, keep_logits=False), run(False, call=checkpointed)]
     with monkeypatch.context() as m:
+        m.setattr(lm_head, "KEPT_UNASKED", 0)
         m.setattr(lm_head, "_free_bytes", lambda dev: 0)
         others.append(run(False))
     with monkeypatch.context() as m:
