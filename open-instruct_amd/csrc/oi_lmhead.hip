@@ -1018,11 +1018,10 @@ __global__ void __launch_bounds__(NTHREADS)
 // Where a tile product goes.
 // mode 0: out_f32  = acc          mode 1: out_f32 += acc
 // mode 2: out_bf16 = acc          mode 3: out_bf16 = out_f32 + acc   (last chunk of d_hidden)
-// mode 4: out_bf16 += acc         (rows added to a d_weight that was already rounded)
 // Rows below m_valid and columns below N are stored.  With `out_rows`, row r of a bf16 result goes to row
 // out_rows[r] of out_bf16 (the fp32 accumulator stays compact).  scale_a / scale_b: factors of row r, see
 // DynRows.  Every element has one writer per launch and the launches follow each other on the stream, so the
-// sums of modes 1, 3 and 4 are plain loads and stores.
+// sums of modes 1 and 3 are plain loads and stores.
 struct StoreTo {
     int mode;
     float* out_f32;
@@ -1031,10 +1030,10 @@ struct StoreTo {
     const int32_t* out_rows;
     const float *scale_a, *scale_b;
 };
-// whole 16-byte pieces (8 bytes for the bf16 results of modes 3 and 4) can be stored and loaded
+// Whole 16-byte pieces (8 bytes for the bf16 results of mode 3) can be stored and loaded.  Rows are whole pieces here
+// (products that are not have gemm_any_kernel) and fp32 buffers are aligned; bf16 rows may lie on 4-byte boundaries.
 __device__ __forceinline__ bool stores_in_pieces(const StoreTo& st) {
-    return ((st.N | st.ldo) & 7) == 0 &&
-           ((reinterpret_cast<uintptr_t>(st.out_f32) | reinterpret_cast<uintptr_t>(st.out_bf16)) & 15) == 0;
+    return st.mode <= 1 || (reinterpret_cast<uintptr_t>(st.out_bf16) & 15) == 0;
 }
 
 // Column group j of a finished tile is its rows row0 + wn * 128 + j * 32 + (0..31) of both wn halves with all 256
@@ -1150,36 +1149,17 @@ __device__ __forceinline__ void store_group_f32(const f32x16& z0, const f32x16& 
         }
         return;
     }
+    // bf16 rows off 8-byte boundaries
     if (col >= st.N) return;
-    const int n = st.N - col < 4 ? (int)(st.N - col) : 4;
 #pragma unroll 1
     for (int it = 0; it < ITERS; ++it) {
         const int64_t row = group_row(row0, j, r_first + it * 8);
         if (row >= st.m_valid) break;
-        const oi_f32x4 v = *reinterpret_cast<const oi_f32x4*>(from + it * 8 * STAGE_F32);
-        float e[4] = {v.x, v.y, v.z, v.w};
-        if (mode <= 1) {
-            float* f = st.out_f32 + row * st.ldo + col;
-#pragma unroll
-            for (int k = 0; k < 4; ++k)
-                if (k < n) f[k] = mode == 1 ? f[k] + e[k] : e[k];
-            continue;
-        }
-        uint16_t* b = st.out_bf16 + (st.out_rows ? (int64_t)st.out_rows[row] : row) * st.ldo + col;
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            if (k >= n) continue;
-            if (mode == 3) e[k] += st.out_f32[row * st.ldo + col + k];
-            if (mode == 4) e[k] += oi_bf16lo_to_f32((uint32_t)b[k]);
-        }
-        if (n == 4 && (reinterpret_cast<uintptr_t>(b) & 3) == 0) {
-            reinterpret_cast<uint32_t*>(b)[0] = oi_pack_bf16x2(e[0], e[1]);
-            reinterpret_cast<uint32_t*>(b)[1] = oi_pack_bf16x2(e[2], e[3]);
-        } else {
-#pragma unroll
-            for (int k = 0; k < 4; ++k)
-                if (k < n) b[k] = (uint16_t)oi_f32_to_bf16_bits(e[k]);
-        }
+        oi_f32x4 v = *reinterpret_cast<const oi_f32x4*>(from + it * 8 * STAGE_F32);
+        if (mode == 3) v += *reinterpret_cast<const oi_f32x4*>(st.out_f32 + row * st.ldo + col);
+        uint32_t* b = reinterpret_cast<uint32_t*>(st.out_bf16 + (st.out_rows ? (int64_t)st.out_rows[row] : row) * st.ldo + col);
+        b[0] = oi_pack_bf16x2(v.x, v.y);
+        b[1] = oi_pack_bf16x2(v.z, v.w);
     }
 }
 
@@ -1218,7 +1198,7 @@ __device__ __forceinline__ void store_tile(const AccTile& __restrict__ acc, cons
 }
 // a product without terms (no rows selected): zeros, or what the earlier launches summed up
 __device__ __forceinline__ void store_no_terms(const StoreTo& st) {
-    if (st.mode == 1 || st.mode == 4) return;
+    if (st.mode == 1) return;
     for (int64_t row = blockIdx.x; row < st.m_valid; row += gridDim.x) {
         const int64_t dst = (st.mode >= 2 && st.out_rows) ? (int64_t)st.out_rows[row] : row;
         for (int64_t col = threadIdx.x; col < st.N; col += NTHREADS) {
@@ -1394,7 +1374,7 @@ __global__ void __launch_bounds__(NTHREADS)
 // ---- products whose rows are not whole 16-byte pieces --------------------------------------------------------
 // The stand-alone products take any pitch and any alignment of the element type (modes 0, 1 and 2, no row index, no
 // factors); the others' rows are hidden_dim (a multiple of 64) columns.  Kept out of gemm_store_kernel, whose main
-// loop comes out 0.3 to 1.6 % slower with either this code or less code in it.
+// loop comes out 0.3 % slower with this code in it.
 //
 // Widest access of a row: 8 columns (16 bytes of bf16), 4 (16 bytes of fp32, 8 of bf16), 2 (4 bytes of bf16) or 1;
 // `out` is the buffer that the mode touches
@@ -1553,6 +1533,69 @@ int launch_product(const Operand& a, int64_t M, const Operand& b, int64_t N, int
         hipLaunchKernelGGL((gemm_any_kernel<R_KM, C_KM>), grid, dim3(NTHREADS), 0, s, a, M, b, N, K, mode, out_f32, o16, ldo,
                            width);
     return oi_launch_status();
+}
+
+// A product added to bf16 rows that are there already: out[row, col] += sum over the n selected tokens (n on the
+// device; none: nothing happens).  It serves the d_weight of flagged rows, of which there are normally none, so it is
+// kept out of gemm_store_kernel's main loop; the few k-tiles of a call that has some leave it bound by reading and
+// writing d_weight.  Policy-loss step of 3000 rows, 4096 x 128256, one of them flagged: 22.8 ms with the entries read
+// and added one by one, 15.5 ms so.
+__global__ void __launch_bounds__(NTHREADS)
+    gemm_add_kernel(Operand R, int64_t M, Operand C, int64_t N, uint16_t* out, int64_t ldo, const int32_t* __restrict__ n_dev,
+                    uint32_t* __restrict__ queue) {
+    __shared__ __align__(16) uint16_t lds[LDS_ELEMS];
+    const int64_t n = *n_dev;
+    if (n <= 0) return;
+    R.k_valid = (n + BM - 1) / BM * BM;
+    C.k_valid = n;
+    const int64_t K = (n + BK - 1) / BK * BK;
+    for_each_tile(queue, (M + BN - 1) / BN, (N + BM - 1) / BM, lds, [&](int64_t tr, int64_t tc) {
+        R.r0 = tr * BN;
+        C.r0 = tc * BM;
+        AccTile acc;
+        gemm_tile<true, true>(acc, C, R, K, lds);
+        const int tid = opaque_tid(), lane = tid & 63, wave = tid >> 6, wm = wave & 3, wn = wave >> 2;
+        constexpr int ITERS = GROUP_ROWS * (BM / 4) / NTHREADS;
+        const int ch = tid & 63, r_first = tid >> 6, srow = wn * 32 + (lane & 31);
+        const int64_t col = C.r0 + ch * 4;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            __builtin_amdgcn_sched_barrier(0);
+            // what is there already is requested before the tile goes through the LDS; rows and columns past the
+            // end read the last valid entries and store nothing.  N and ldo are multiples of 64, out is 4-byte aligned.
+            uint32_t there[ITERS][2];
+            const int64_t c = col < N ? col : N - 4;
+#pragma unroll
+            for (int it = 0; it < ITERS; ++it) {
+                int64_t row = group_row(R.r0, j, r_first + it * 8);
+                row = row < M ? row : M - 1;
+                const uint32_t* b = reinterpret_cast<const uint32_t*>(out + row * ldo + c);
+                there[it][0] = b[0];
+                there[it][1] = b[1];
+            }
+            // two regions in turn, as in store_tile
+            float* stage32 = reinterpret_cast<float*>(lds + (j & 1) * GROUP_F32);
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+#pragma unroll
+                for (int q = 0; q < 4; ++q)
+                    *reinterpret_cast<oi_f32x4*>(stage32 + srow * STAGE_F32 + acc_row(wm, i, q * 4, lane)) =
+                        oi_f32x4{acc[i][j][q * 4], acc[i][j][q * 4 + 1], acc[i][j][q * 4 + 2], acc[i][j][q * 4 + 3]};
+            lds_barrier();
+#pragma unroll
+            for (int it = 0; it < ITERS; ++it) {
+                const int64_t row = group_row(R.r0, j, r_first + it * 8);
+                oi_f32x4 v = *reinterpret_cast<const oi_f32x4*>(stage32 + (r_first + it * 8) * STAGE_F32 + ch * 4);
+                v += oi_f32x4{oi_bf16lo_to_f32(there[it][0]), oi_bf16hi_to_f32(there[it][0]), oi_bf16lo_to_f32(there[it][1]),
+                              oi_bf16hi_to_f32(there[it][1])};
+                if (row >= M || col >= N) continue;
+                uint32_t* b = reinterpret_cast<uint32_t*>(out + row * ldo + col);
+                b[0] = oi_pack_bf16x2(v.x, v.y);
+                b[1] = oi_pack_bf16x2(v.z, v.w);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    });
 }
 
 // Adds the pieces of the split tiles of a gemm_store_kernel launch over `grid` workgroups and stores the
@@ -2191,11 +2234,8 @@ __global__ void __launch_bounds__(256)
 //   d_weight[v_begin + v, h] = sum_n dZ[n, v] * hidden[n, h]    A k-major,      B k-major
 // The sums stop at the last real vocabulary row / token (rounded up to a k-tile, whose missing
 // rows are read from the last real one and meet zeros of dZ).  The queue words must be zeroed.
-// dw_mode / dw32: how d_weight is stored.  2 (default): this call holds every token, bf16 rows are
-// written directly.  0 / 1: the tokens come in several calls; dw32 (fp32 [vocab, hidden]) takes the
-// first call's product (0) and adds the following ones (1; a call without tokens adds nothing and
-// costs nothing); the caller rounds dw32 to bf16 when the last call is through.  4: the product is
-// added to bf16 rows that an earlier call wrote.
+// dw_adds: the product is added to the bf16 rows of d_weight that an earlier call wrote, instead of stored there; a call
+// without tokens then changes nothing and costs nothing (the rows must be selected on the device).
 // logits: the forward's logits (kept_bytes), read instead of recomputed.
 // max_grid > 0 caps the number of resident workgroups of every launch (the queues work with any
 // number): the launches that serve flagged rows normally find none, and a launch over a few CUs that
@@ -2203,7 +2243,7 @@ __global__ void __launch_bounds__(256)
 constexpr unsigned REPAIR_GRID = 32;
 void enqueue_bwd(const BwdPlan& p, char* ws, const RowInputs& in, const void* weight, int64_t n_tokens,
                  int64_t hidden_dim, int64_t vocab, float inv_temperature, void* d_hidden, void* d_weight,
-                 hipStream_t s, int dw_mode = 2, float* dw32 = nullptr, unsigned max_grid = 0,
+                 hipStream_t s, bool dw_adds = false, unsigned max_grid = 0,
                  const float* logits = nullptr) {
     auto grid_of = [&](int64_t tiles_m, int64_t tiles_n) {
         const unsigned g = resident_grid(tiles_m, tiles_n);
@@ -2241,12 +2281,16 @@ void enqueue_bwd(const BwdPlan& p, char* ws, const RowInputs& in, const void* we
         if (d_weight) {
             const Operand a = {dz, cols, 0, cols, p.n_pad};
             const Operand b = {in.hidden, hidden_dim, 0, hidden_dim, n_tokens};
-            const DynRows dyn = {in.n_dev, 2, nullptr, nullptr, nullptr, nullptr};
-            hipLaunchKernelGGL((gemm_store_kernel<true, true>), grid_of(cols / BM, h_tiles),
-                               dim3(NTHREADS), 0, s, a, cols, b, hidden_dim, round_up(n_tokens, BK), dw_mode,
-                               dw32 ? dw32 + v_begin * hidden_dim : static_cast<float*>(nullptr),
-                               static_cast<uint16_t*>(d_weight) + v_begin * hidden_dim, hidden_dim, valid, dyn,
-                               q + 2 * QUEUE_WORDS, static_cast<float*>(nullptr));
+            uint16_t* dw = static_cast<uint16_t*>(d_weight) + v_begin * hidden_dim;
+            const dim3 grid = grid_of(cols / BM, h_tiles);
+            if (dw_adds)
+                hipLaunchKernelGGL(gemm_add_kernel, grid, dim3(NTHREADS), 0, s, a, valid, b, hidden_dim, dw, hidden_dim, in.n_dev,
+                                   q + 2 * QUEUE_WORDS);
+            else
+                hipLaunchKernelGGL((gemm_store_kernel<true, true>), grid, dim3(NTHREADS), 0, s, a, cols, b, hidden_dim,
+                                   round_up(n_tokens, BK), 2, static_cast<float*>(nullptr), dw, hidden_dim, valid,
+                                   DynRows{in.n_dev, 2, nullptr, nullptr, nullptr, nullptr}, q + 2 * QUEUE_WORDS,
+                                   static_cast<float*>(nullptr));
         }
     }
 }
@@ -2501,8 +2545,8 @@ int run_slab_passes(const SlabPlan& p, char* ws, const SlabStep& st, hipStream_t
             hipLaunchKernelGGL(zero_words_kernel, dim3((unsigned)((n_words + 255) / 256)), dim3(256), 0, s, rq, n_words);
         const RowInputs in = launch_selection(p.repair.sel, ws_rep, st.hidden, st.labels, lse, grad, unsafe, false, n,
                                               hdim, rq, select_clears ? n_words : 0, s, st.logprob);
-        enqueue_bwd(p.repair, ws_rep, in, st.weight, n, hdim, vocab, st.inv_temperature, st.d_hidden, st.d_weight, s, 4,
-                    nullptr, REPAIR_GRID);
+        enqueue_bwd(p.repair, ws_rep, in, st.weight, n, hdim, vocab, st.inv_temperature, st.d_hidden, st.d_weight, s, true,
+                    REPAIR_GRID);
     }
     return oi_launch_status();
 }
@@ -2669,7 +2713,7 @@ extern "C" int oi_lmhead_dh_from_wsum(const void* hidden, const void* weight, co
         hipLaunchKernelGGL(zero_words_kernel, dim3((unsigned)((n_words + 255) / 256)), dim3(256), 0, s, rq, n_words);
     const RowInputs in = launch_selection(p.repair.sel, ws_rep, hidden, labels, lse, grad_logprob, unsafe, false,
                                           n_tokens, hidden_dim, rq, select_clears ? n_words : 0, s, logprob);
-    enqueue_bwd(p.repair, ws_rep, in, weight, n_tokens, hidden_dim, vocab, inv_temperature, d_hidden, nullptr, s, 2, nullptr,
+    enqueue_bwd(p.repair, ws_rep, in, weight, n_tokens, hidden_dim, vocab, inv_temperature, d_hidden, nullptr, s, false,
                 REPAIR_GRID);
     return oi_launch_status();
 }
@@ -2713,8 +2757,8 @@ int lmhead_backward(const void* hidden, const void* weight, const int64_t* label
         hipLaunchKernelGGL(zero_unselected_rows_kernel, dim3((unsigned)n_tokens), dim3(256), 0, s, row_mask,
                            zero_grad_probe, hidden_dim, static_cast<uint16_t*>(d_hidden));
     }
-    enqueue_bwd(p, ws, in, weight, n_tokens, hidden_dim, vocab, inv_temperature, d_hidden, d_weight, s, 2,
-                nullptr, 0, logits);
+    enqueue_bwd(p, ws, in, weight, n_tokens, hidden_dim, vocab, inv_temperature, d_hidden, d_weight, s, false,
+                0, logits);
     return oi_launch_status();
 }
 }  // namespace

@@ -159,3 +159,28 @@ def test_products_of_any_pitch(m, n, k, ldo, shift):
         assert rc == 0
         assert torch.equal(rows[:, :n], (exact + 3.0 * accumulate).to(dtype)), (dtype, accumulate)
         assert (rows[:, n:] == 3).all() and (out[:shift] == 3).all() and (out[shift + m * ldo :] == 3).all()
+
+
+@pytest.mark.parametrize("n,h,v,flagged,slabs", [(1, 64, 300, 1, 4096), (300, 64, 301, 70, 4096), (600, 320, 513, 257, 256)])
+def test_flagged_rows_are_added_to_d_weight(n, h, v, flagged, slabs):
+    """Rows whose label lies more than 44 nats below the largest logit are recomputed and added to the bf16 d_weight
+    of the others (which rounds its entries once more: within the bound of _close, half of which is one rounding)."""
+    print("case flagged", n, h, v, flagged, slabs, flush=True)
+    hidden, weight, labels, mask, upstream = _inputs(n, h, v, seed=n + v)
+    labels = labels % (v - 1) + 1
+    weight[0] = 0.5
+    hidden[:flagged] = 1.5
+    weight[labels[:flagged]] = -0.5
+    mask[:flagged] = True
+    upstream = -upstream / mask.sum()
+    lp, dh, dw = _reference(hidden, weight, labels, mask, upstream)
+    cfg = types.SimpleNamespace(loss_fn="cispo", clip_lower=0.2, clip_higher=0.2, beta=0.0, kl_estimator=2)
+    hid, w = hidden.requires_grad_(True), weight.requires_grad_(True)
+    adv = -upstream * mask.sum()
+    loss, _, out, _ = grpo_utils.grpo_loss_on_hidden(
+        hid[None], w, labels[None], None, None, adv[None], mask[None], cfg, token_slabs=slabs
+    )
+    loss.backward()
+    assert lp[:flagged].max() < -44 and (out[0].detach() - lp).abs().max() <= 1e-5 * lp.abs().max() + TOL
+    _close(hid.grad, dh, "d_hidden")
+    _close(w.grad, dw, "d_weight")
