@@ -2478,7 +2478,7 @@ struct SlabStep {
 };
 
 // Runs the slab passes of `st` over the row index order[0 .. *count) that `plan_rows` leaves in the
-// workspace together with the passes' SlabMeta.  `upstream()` must enqueue kernels that leave
+// workspace together with the passes' SlabMeta (it returns a status: reading one clears it).  `upstream()` must enqueue kernels that leave
 // every caller row's d loss / d logprob in the workspace's grad vector, given the logprobs computed
 // so far (the rows of the slabs up to the current one; in the last pass, all rows).
 template <class PlanRows, class Upstream>
@@ -2508,7 +2508,8 @@ int run_slab_passes(const SlabPlan& p, char* ws, const SlabStep& st, hipStream_t
     hipLaunchKernelGGL(slab_setup_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, n, p.n_pad,
                        p.n_passes * SLAB_QUEUE_WORDS, st.logprob, st.entropy, lse, reinterpret_cast<uint32_t*>(unsafe),
                        queues);
-    plan_rows(order, count, meta);
+    const int planned = plan_rows(order, count, meta);
+    if (planned != OI_OK) return planned;
     hipLaunchKernelGGL(zero_unselected_rows_kernel, dim3((unsigned)n), dim3(256), 0, s, st.mask,
                        static_cast<const float*>(nullptr), hdim, static_cast<uint16_t*>(st.d_hidden));
     for (int64_t i = 0; i < p.n_passes; ++i) {
@@ -2826,7 +2827,7 @@ int grpo_step_in_slabs(const void* hidden, const void* weight, const int64_t* la
             hipLaunchKernelGGL(plan_slabs_kernel, dim3((unsigned)((p.n_passes + 63) / 64)), dim3(64), 0, s, count,
                                (int)p.cap, (int)p.n_passes, (int)h_tiles, (int)resident_grid(p.cap / BM, h_tiles), meta);
             // the denominators come from the mask alone
-            (void)oi_launch_grpo_denoms(mask, count, rows, cols, axis_mode, denominator, row_denoms, s);
+            return oi_launch_grpo_denoms(mask, count, rows, cols, axis_mode, denominator, row_denoms, s);
         },
         [&]() {
             // every token's d loss / d logprob from its own logprob; tokens of later slabs hold numbers
@@ -3141,6 +3142,7 @@ extern "C" int oi_lmhead_dpo_fwd_bwd(const void* hidden, const void* weight, con
                                (int)p.slabs.n_passes, off, seq_unsafe, count, meta);
             hipLaunchKernelGGL(dpo_order_kernel, dim3((unsigned)n_seqs), dim3(256), 0, s, mask, cu_seq_lens, n_seqs, total,
                                off, seq_unsafe, order, unsafe);
+            return oi_launch_status();
         },
         upstream);
     if (rc != OI_OK) return rc;
