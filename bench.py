@@ -61,7 +61,7 @@ MEASURED_TRAFFIC_BYTES = {
     # lmhead_fwd_kernel: L2 misses of the tiled operand re-reads (1.24 GB of unique operands at c3) + the partials
     "c3-recompute": 42.57e9 + 0.20e9,
     "c4-recompute": 40.24e9 + 0.20e9,
-    # oi_lmhead_logp_fwd_wsum: two launches of lmhead_fwd_kernel<true> and two of gemm_store_kernel<false, true>
+    # oi_lmhead_logp_fwd_wsum: two launches of lmhead_fwd_kernel and two of gemm_store_kernel<false, true>
     "c5": 2 * (44.80e9 + 3.09e9) + 2 * (40.44e9 + 0.75e9),
     # lsg_grpo_fused_kernel: one read of the logits (the row waits on the CU for the gradient pass) + one write of
     # dlogits
@@ -271,7 +271,7 @@ def make_fused(torch, oi, n_tokens, hdim, vocab, w_std, dpo=False, route="slabs"
         # the weight takes no gradient: the forward call also accumulates the weighted sum of weight rows that
         # the backward to hidden needs (per vocabulary chunk: statistics + exponentials, then E_chunk @ W_chunk)
         info["kernel"] = (
-            "oi_lmhead_logp_fwd_wsum (per vocabulary chunk: lmhead_fwd_kernel<true> + gemm_store_kernel<false, true>; "
+            "oi_lmhead_logp_fwd_wsum (per vocabulary chunk: lmhead_fwd_kernel + gemm_store_kernel<false, true>; "
             "all of the step's matrix work, nothing is recomputed)"
         )
         info["alg_per_launch"] = 2.0 * flops_fwd
@@ -885,7 +885,8 @@ def main():
     if isinstance(info["timer"], KernelProbe) and not args.one_kernel:
         # the other tile kernels of the slab-wise call, each timed over three more steps (outside the timed region)
         probe, timed_kernel = info["timer"], info["timer"].kernel
-        names = {0: "lmhead_fwd_kernel<true> (forward that keeps its exponentials)", 1: "gemm_store_kernel<false, true> (d_hidden product)",
+        names = {0: "lmhead_fwd_kernel (forward that keeps its exponentials)",
+                 1: "gemm_store_kernel<false, true> + gemm_reduce_kernel (d_hidden product)",
                  2: "gemm_store_kernel<true, true> (d_weight product)"}
         per_kernel = {names[timed_kernel]: {"ms_per_launch": kernel_ms, "frac": achieved / peak}}
         for k in (0, 1, 2):

@@ -331,7 +331,8 @@ int oi_pack_sequences(const int64_t* q_tokens, const int64_t* q_offsets, const i
                       float* out_advantages, void* stream);
 
 /* ------------------------------------------------------------------------------------------
- * Fused lm_head projection + per-token logprob / entropy, logits never materialised.
+ * Fused lm_head projection + per-token logprob / entropy.  No [tokens, vocab] logits leave the chip, except in the
+ * pair that keeps them for its backward (oi_lmhead_logp_fwd_kept).
  *
  * Replaces the pair "lm_head GEMM -> calculate_per_token_logps" of
  * open_instruct/olmo_core_train_modules.py:71-76 (DPOLMHead.forward) and
@@ -360,8 +361,11 @@ int oi_lmhead_logp_fwd(const void* hidden, const void* weight, const int64_t* la
  *   dZ[n, v] = grad_logprob[n] * inv_T * (1[v == label_n] - exp(z[n,v] * inv_T - lse[n])),
  *   d_hidden = dZ @ weight   (bf16 [n_tokens, hidden_dim]),
  *   d_weight = dZ^T @ hidden (bf16 [vocab, hidden_dim]; NULL skips it).
- * Vocabulary is processed in chunks of 32768 columns; only one chunk of dZ (bf16, token-major)
- * lives in the workspace at a time, next to the fp32 accumulator of d_hidden.  Both products
+ * One vocabulary chunk of dZ (bf16, token-major) lives in the workspace at a time, next to the fp32 accumulator
+ * of d_hidden.  With N and V rounded up to 256 a chunk is the whole vocabulary while N * V <= 2^30 (2 GiB of dZ),
+ * and beyond that equal chunks of at most max(2^30 / N, 32768) columns.  Where the last round of tiles of the
+ * d_hidden product would leave most of the chip idle its tiles are cut along the vocabulary, and their pieces take
+ * up to 252 MiB more (64 MiB for 512 rows at hidden_dim 4096).  Both products
  * read weight, hidden and dZ where they lie (no transposed copies), so the workspace is the same
  * with and without d_weight.  row_mask as in the forward (rows left out get a zero d_hidden row
  * and add nothing to d_weight); skip_zero_grad_rows != 0 also leaves out rows whose grad_logprob is
@@ -381,8 +385,9 @@ int oi_lmhead_logp_bwd(const void* hidden, const void* weight, const int64_t* la
  * The same pair with the logits kept in between (for a backward that wants d_weight): the forward also leaves
  * its fp32 logits in `logits` (16-byte aligned, oi_lmhead_kept_bytes bytes, in an order of its own), and the
  * backward reads them instead of computing them again: 6 N H V of matrix work instead of 8 N H V, results
- * identical to the bit.  oi_lmhead_kept_bytes is 0 where the logits are not to be kept (more than 4 GiB of them, i.e.
- * where the recomputing backward takes the vocabulary in chunks): the kept calls then return OI_EWORKSPACE.
+ * identical to the bit.  oi_lmhead_kept_bytes is 0 where the logits are not to be kept, i.e. where there are
+ * more than 4 GiB of them (N * V > 2^30 with both rounded up to 256, and the columns that fit counted in whole
+ * 1024s): the kept calls then return OI_EWORKSPACE.
  * The backward takes the forward's row_mask and skips no further rows; it leaves `logits` as it is.
  * Workspaces as for the pair above (oi_lmhead_fwd_workspace_bytes, oi_lmhead_bwd_workspace_bytes).
  */
@@ -419,8 +424,9 @@ int oi_lmhead_logp_bwd_kept(const void* hidden, const void* weight, const int64_
  * any d_weight == NULL use of oi_lmhead_logp_bwd).  With e' and xref as above,
  *   d_hidden[n] = s_n * sum_{v != label_n} e'[n,v] * weight[v]  -  g_n * inv_T * expm1(logprob_n) * weight[label_n],
  * and the sum does not depend on the upstream gradient g: oi_lmhead_logp_fwd_wsum computes it together
- * with logprob / entropy / lse while the logits exist (one chunk of 65536 vocabulary columns at a
- * time: the chunk's exponentials as bf16 in the workspace, then wsum (+)= E_chunk @ weight_chunk in
+ * with logprob / entropy / lse while the logits exist (one vocabulary chunk at a time, as
+ * wide as in the recomputing backward but at least 65536 columns: the chunk's exponentials as bf16 in the
+ * workspace, then wsum (+)= E_chunk @ weight_chunk in
  * fp32), and oi_lmhead_dh_from_wsum turns it into d_hidden in one pass over [n_tokens, hidden_dim].
  * Matrix work of forward + backward: 4 N H V instead of 6 N H V, nothing is recomputed, nothing of size
  * [tokens, vocab] exists.
@@ -530,8 +536,9 @@ int oi_lmhead_dpo_fwd_bwd(const void* hidden, const void* weight, const int64_t*
  * Timing probe of the slab-wise entry points (no reference counterpart; it exists for the
  * measurement harness, which has to time one kernel inside a call that launches several).  Between
  * oi_lmhead_probe_arm(kernel) and oi_lmhead_probe_read the slab-wise calls of this process record a
- * pair of HIP events, on the stream of the call, around every launch of the chosen tile kernel:
- * 0 = the forward that keeps its exponentials, 1 = the d_hidden product, 2 = the d_weight product
+ * pair of HIP events, on the stream of the call, around the chosen tile kernel of every pass:
+ * 0 = the forward that keeps its exponentials, 1 = the d_hidden product (with the launch that adds the pieces of
+ * cut tiles), 2 = the d_weight product
  * (at most 1024 launches; later ones are not recorded).  oi_lmhead_probe_read waits for the recorded
  * events, writes the duration of each recorded launch in milliseconds to ms[0 .. min(n, capacity)),
  * the number of recorded launches to *n_launches, and disarms the probe.  Launches whose slab is

@@ -1,4 +1,5 @@
-// Fused lm_head projection + per-token logprob / entropy for gfx950, logits never materialised.
+// Fused lm_head projection + per-token logprob / entropy for gfx950.  The logits stay on the chip, except where the
+// forward leaves them for its backward (lmhead_dz_kept_kernel).
 //
 // One bf16 MFMA main loop, C[m, n] = sum_k a(m, k) * b(n, k), serves four kernels that differ in
 // what they do with the fp32 tile and in the memory order of their operands (k-contiguous: the k
@@ -1751,7 +1752,7 @@ __global__ void __launch_bounds__(256)
 // on the device.  Written by a planning kernel, read by every kernel of the pass.
 struct SlabMeta {
     int32_t offset, count;
-    // how the slab's d_weight product is stored (the modes of gemm_store_tile): the only slab writes
+    // how the slab's d_weight product is stored (the modes of StoreTo): the only slab writes
     // bf16 rows (2); of several, the first stores fp32 (0), the middle ones add to it (1) and the last
     // one adds the fp32 sum to its own product and writes bf16 rows (3); a pass without rows: -1
     int32_t dw_mode, reserved;
@@ -1847,8 +1848,9 @@ __global__ void __launch_bounds__(256)
 }
 
 // Timing probe for the measurement harness: while armed, the slab-wise entry points record a pair
-// of HIP events around every launch of one of their three tile kernels (which one is chosen when the
-// probe is armed), on the stream of the call.  Off by default and between arm / read; not meant for
+// of HIP events around one of their three products in every pass (which one is chosen when the probe is
+// armed; d_hidden: the tile kernel and the launch that adds the pieces of its cut tiles, which finds none where no tile
+// is cut), on the stream of the call.  Off by default and between arm / read; not meant for
 // calls that are being captured into a graph.
 struct Probe {
     int kernel = -1;  // 0 forward with kept exponentials, 1 d_hidden product, 2 d_weight product; -1 = off
@@ -2004,8 +2006,8 @@ FwdPlan plan_fwd(int64_t n_tokens, int64_t hdim, int64_t vocab, bool with_select
 // again; 0 where they are not to be kept.  Keeping them takes the recomputation (a quarter of the matrix
 // work of a step with a trained head) out of the step and costs 4 bytes per row and column between the passes:
 // cross-entropy of 3072 rows, hidden 4096, vocabulary 128256: dZ 2460 -> 430 us (5.5 TB/s), forward 2350 -> 2770 us
-// with its stores, step 10.9 -> 8.65 ms.  The line is where the recomputing backward begins to take the vocabulary in chunks, i.e. 4 GiB: a larger batch is a
-// large part of a card's memory, and its step is better made slab by slab.
+// with its stores, step 10.9 -> 8.65 ms.  The line is 4 GiB, twice the scratch of the backward's dZ at the same sizes:
+// a larger batch would hold a large part of a card's memory, and its step is better made slab by slab.
 size_t kept_bytes(int64_t n_tokens, int64_t vocab) {
     const int64_t n_pad = round_up(n_tokens, BN), v_pad = round_up(vocab, BM);
     if (v_pad > CHUNK_BUDGET / n_pad / 1024 * 1024) return 0;
@@ -2419,8 +2421,10 @@ SlabPlan plan_slabs(int64_t n, int64_t stats_rows, int64_t stats_cols, int64_t h
 // 256 rows, the last one takes what is left), or, when that takes fewer rounds of tiles, full slabs of
 // `cap` rows and a last one with the remainder.  What is counted is the slab's d_hidden product, the one
 // tile kernel whose work items are long (a tile runs over the whole vocabulary): it has
-// ceil(rows / 256) * h_tiles tiles for `grid` resident workgroups, and a round of tiles takes the same
-// time whether it is full or not.  Passes past the last slab are empty.
+// ceil(rows / 256) * h_tiles tiles for `grid` resident workgroups, in whole rounds.  A last round that is
+// mostly empty is cut along the vocabulary (plan_tail) and costs less than that, so the choice matters little:
+// steps at 4096 x 128256, full slabs of 8192 against equal ones, 12288 rows 31.1 to 31.3 against 31.3 to 31.4 ms, 9472
+// rows 24.6 against 24.6, 16640 rows 43.2 against 43.1.  Passes past the last slab are empty.
 __global__ void plan_slabs_kernel(const int32_t* __restrict__ count, int cap, int n_passes, int h_tiles, int grid,
                                   SlabMeta* __restrict__ meta) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;

@@ -239,8 +239,8 @@ def concatenated_forward(
     HuggingFace interface: ``model(**inputs).logits``; with ``output_router_logits`` the model is
     asked for its router logits and the ``aux_loss`` of its output is passed through.  Returns
     ``(chosen_logps, rejected_logps, aux_loss)``.  ``fused_head=True`` (not in the reference) runs
-    the model's trunk only and sends its hidden states through the fused lm_head, so the ``[B, T, V]``
-    logits are never formed and prompt / padding positions are not multiplied; same results.
+    the model's trunk only and sends its hidden states through the fused lm_head, so the model never forms
+    its ``[B, T, V]`` logits and prompt / padding positions are not multiplied; same results.
     """
     if packing:
         concat, bs = padding_free_collator.concatenated_inputs(batch)
@@ -317,7 +317,7 @@ def concatenated_forward_olmo(
     open_instruct/dpo_utils.py:959-1019.
 
     The labels go INTO the model: its LM head (:class:`~open_instruct_amd.olmo_core_train_modules.DPOLMHead`)
-    returns the per-token logps as ``output.loss`` and never forms the ``[tokens, vocab]`` logits.
+    returns the per-token logps as ``output.loss`` instead of logits.
     Packed batches pass ``position_ids`` and the document lengths derived from ``cu_seq_lens_k``.
     ``output_router_logits`` is accepted and unused, ``aux_loss`` is always None, as in the reference.
     """
@@ -351,7 +351,9 @@ def separate_forward_olmo(model, batch: dict, average_log_prob: bool = False, ou
     :class:`~open_instruct_amd.olmo_core_train_modules.DPOLMHead` returns the per-token logps as
     ``output.loss``; only one side's activations are alive at a time.  ``output_router_logits`` is accepted
     and unused, ``aux_loss`` is always None, as in the reference.  (The reference empties the allocator's
-    cache after each side; the fused head leaves no ``[tokens, vocab]`` block behind to give back.)
+    cache after each side, to give back a side's logits.  Here no block of that kind is free between the sides: what a
+    trained head may keep, at most 4 GiB over both, is in use until the backward; its ``keep_logits = False`` keeps
+    nothing.)
     """
     del output_router_logits
     sides = []
@@ -409,7 +411,7 @@ def dpo_loss_on_hidden(
     slab of token rows can be finished (forward, upstream gradient, ``d_hidden``, its share of ``d_weight``)
     before the next one starts, so a trainable lm_head costs 6·N·H·V of matrix work instead of the 8·N·H·V of
     the differentiable route through :class:`~open_instruct_amd.olmo_core_train_modules.DPOLMHead`, whose
-    backward has to recompute the logits.  The ``[tokens, vocab]`` logits never exist; the scratch is a
+    backward recomputes the logits of all but small batches.  The ``[tokens, vocab]`` logits never exist; the scratch is a
     ``[slab, vocab]`` bf16 buffer and an fp32 ``[vocab, hidden]``.
 
     ``hidden`` is ``[2 * bs, T, H]`` bf16 with ``labels`` ``[2 * bs, T]`` (padded; chosen rows first:

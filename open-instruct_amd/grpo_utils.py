@@ -605,12 +605,13 @@ def grpo_loss_on_hidden(
     that buffer before the next slab overwrites it (``d_weight`` accumulates in fp32 over the
     slabs).  6·N·H·V of matrix work instead of 8·N·H·V; the scratch is ``[slab, vocab]`` bf16 plus an
     fp32 ``[vocab, hidden]``, never ``[tokens, vocab]``.  The slab size hardly matters for the time of the step
-    (8192 to 32768 tokens measured within 1 %); smaller slabs need less scratch.  The route has no limit on the size of the logits or on the
-    temperature: a token whose label is extremely unlikely (largest logit more than 44 nats above the
-    label's) or whose logits hold a NaN is flagged on the device and served by a recomputing backward
-    over the flagged rows inside the same call.  ``token_slabs=False`` is the recomputing step: one
+    (8192 to 32768 tokens measured within 1 %); smaller slabs need less scratch.  The route has no limit on the
+    size of the logits or on the temperature: a token whose label is extremely unlikely (largest logit more
+    than 44 nats above the label's) or whose logits hold a NaN is flagged on the device and served by a
+    recomputing backward over the flagged rows inside the same call.  ``token_slabs=False`` is the recomputing step: one
     forward over all selected rows, then a backward that recomputes the logits one vocabulary chunk at
-    a time (8·N·H·V, scratch ``[tokens, 32768]`` bf16).
+    a time (8·N·H·V; scratch: the bf16 gradient of one chunk of the logits, 2 GiB or ``[tokens, 32768]``, whichever
+    is more).
 
     ``loss.backward()`` may be called once per call of this function.
     """

@@ -1,4 +1,5 @@
-"""Fused lm_head projection + per-token logprob / entropy (no ``[tokens, vocab]`` logits tensor).
+"""Fused lm_head projection + per-token logprob / entropy (no ``[tokens, vocab]`` logits tensor, except for the fp32
+block that the forward of a small batch with a trained head may leave for its backward, see ``_kept_logits``).
 
 There is no single counterpart in the reference: this replaces the pair "lm_head GEMM, then
 ``calculate_per_token_logps`` / ``log_softmax_and_gather`` (+ ``entropy_from_logits``)" at
@@ -153,9 +154,9 @@ def _free_bytes(dev) -> int:
 def _kept_logits(n, h, v, dev, selecting):
     """Memory for the forward's logits where they are kept for the backward, else None (the backward then
     computes them again, with the same results).  Kept only where nothing else has to give way for them:
-    not more than one call's largest share over all live graphs, and more than a little only out of plenty; not where saved tensors
-    are packed (checkpointing counts them and would compute them twice, offloading would copy them), and not into
-    the private pool of a graph, which would hold them as long as the graph lives."""
+    not more than one call's largest share over all live graphs, and more than a little only out of plenty; not
+    where saved tensors are packed (checkpointing counts them and would compute them twice, offloading would copy
+    them), and not into the private pool of a graph, which would hold them as long as the graph lives."""
     lib = _lib.load()
     kept = lib.oi_lmhead_kept_bytes(n, v)
     if not kept or torch._C._autograd._top_saved_tensors_default_hooks(True) is not None:

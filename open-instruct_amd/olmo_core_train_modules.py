@@ -31,7 +31,8 @@ class DPOLMHead(torch.nn.Module):
 
     ``output.loss[b, i] = log p(labels[b, i+1] | x[b, i])`` with the label shift done internally,
     as ``calculate_per_token_logps`` does (open_instruct/padding_free_collator.py:10-16).  The
-    ``[B, T, V]`` logits are never formed when labels are given.
+    ``[B, T, V]`` logits of the model are never formed when labels are given (``keep_logits`` below is about a
+    block that a small batch with a trained head may hold between the passes).
 
     Positions whose next label is ``ignore_index`` (prompt and padding tokens, the last position)
     are not multiplied at all: their entry of ``output.loss`` is 0 and they receive no gradient.
