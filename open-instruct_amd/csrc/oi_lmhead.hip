@@ -2423,8 +2423,9 @@ SlabPlan plan_slabs(int64_t n, int64_t stats_rows, int64_t stats_cols, int64_t h
 // tile kernel whose work items are long (a tile runs over the whole vocabulary): it has
 // ceil(rows / 256) * h_tiles tiles for `grid` resident workgroups, in whole rounds.  A last round that is
 // mostly empty is cut along the vocabulary (plan_tail) and costs less than that, so the choice matters little:
-// steps at 4096 x 128256, full slabs of 8192 against equal ones, 12288 rows 31.1 to 31.3 against 31.3 to 31.4 ms, 9472
-// rows 24.6 against 24.6, 16640 rows 43.2 against 43.1.  Passes past the last slab are empty.
+// steps at 4096 x 128256, full slabs of 8192 against equal ones, 8500 rows 21.6 to 21.8 against 22.0 ms, 9472 rows 24.6
+// against 24.6, 12288 rows 30.5 to 31.3 against 30.6 to 31.4, 16640 rows 43.2 against 43.1.  Passes past the last slab
+// are empty.
 __global__ void plan_slabs_kernel(const int32_t* __restrict__ count, int cap, int n_passes, int h_tiles, int grid,
                                   SlabMeta* __restrict__ meta) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
