@@ -60,8 +60,9 @@ def _close(got, exp, name):
         (70, 64, 1984),  # 31 k-tiles: too short to cut
         (70, 64, 2048),  # 32 k-tiles: the shortest product that is cut, in two
         (1, 64, 2049),  # one row, 33 k-tiles, the last of one vocabulary row
-        (300, 320, 9001),  # four tiles in eight pieces
-        (600, 1088, 33000),  # pieces bounded by the scratch, ragged last hidden tile
+        (300, 320, 9001),  # two tiles (about 240 rows are selected) in eight pieces
+        (600, 1088, 33000),  # ten tiles in 25 pieces, ragged last hidden tile
+        (2100, 4096, 128256),  # 112 tiles in nine pieces: 1008, the most scratch there is
         (16500, 1088, 2300),  # a whole round of tiles and a cut rest
         (9000, 64, 120000),  # two vocabulary chunks
     ],
