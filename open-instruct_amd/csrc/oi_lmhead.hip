@@ -14,9 +14,8 @@
 // so the backward reads W, hidden and dZ where they lie: no transposed copies.
 //
 // Tile: 256 x 256 x 64 per 512-thread workgroup, 8 waves as 4 (m) x 2 (n), each wave 64 x 128 =
-// 2 x 4 MFMA 32x32x16 accumulators.  With vocabulary as the m dim a lane's 16 accumulator
-// registers of one MFMA tile belong to ONE token (column), so the softmax statistics reduce
-// inside the lane.  LDS: a ring of five 32 KB operand slots (k-tiles of A and of B) filled by
+// 4 x 8 MFMA 16x16x32 accumulators.  With vocabulary as the m dim a lane's accumulators of a
+// column of tiles belong to ONE token, so the softmax statistics reduce inside the lane.  LDS: a ring of five 32 KB operand slots (k-tiles of A and of B) filled by
 // direct global->LDS loads of whole 128-byte line segments; the 16-byte chunks of a row are
 // XOR-permuted so that fragment reads (16-byte reads of a k-contiguous image, transposing 8-byte
 // reads of a k-major image) stay free of bank conflicts.  A launch is one resident workgroup per
@@ -28,6 +27,7 @@
 namespace {
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
 constexpr int BM = 256, BN = 256, BK = 64;
@@ -37,7 +37,7 @@ constexpr int STAGE_STRIDE = 256 + 8;           // bf16 per row of the dZ stagin
 constexpr int LDS_ELEMS = 5 * TILE_ELEMS;       // 163840 B: the five-slot operand ring, all of a CU's LDS
 static_assert(256 * STAGE_STRIDE <= LDS_ELEMS, "the dZ staging tile must fit");
 
-typedef f32x16 AccTile[2][4];
+typedef f32x4 AccTile[4][8];
 
 // XCD-aware tile order.  Consecutive workgroup ids go round-robin to the 8 XCDs, each with its own
 // L2.  The tiles of a launch are numbered in bands of 8 rows, n outermost inside a band, so that 32
@@ -198,9 +198,22 @@ __device__ __forceinline__ void lds_barrier() {
     asm volatile("" ::: "memory");
 }
 
-constexpr int NSLOT = 5;
+// A count in device memory, in a scalar register: sizes and base addresses that follow from it then take no vector
+// registers and no vector instructions in the main loops.
+__device__ __forceinline__ int device_count(const int32_t* p) { return __builtin_amdgcn_readfirstlane(*p); }
+// The same for 64-bit values that every lane holds alike
+__device__ __forceinline__ int64_t scalar(int64_t v) {
+    const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)v);
+    const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)((uint64_t)v >> 32));
+    return (int64_t)(((uint64_t)hi << 32) | lo);
+}
+template <class T>
+__device__ __forceinline__ const T* scalar(const T* p) {
+    return reinterpret_cast<const T*>(scalar((int64_t)reinterpret_cast<uint64_t>(p)));
+}
+
+constexpr int SLOT_BYTES = TILE_ELEMS * 2;
 constexpr int64_t MAX_LD = (int64_t)1 << 22;  // 255 rows * ld * 2 bytes must fit 32 bits
-__device__ __forceinline__ int ring_slot(int s) { return s >= NSLOT ? s - NSLOT : s; }
 
 // One operand of a tile product, in either of two memory layouts.
 //   k-contiguous (KM = false): element (row, k) at p[row * ld + k]; the tile takes rows
@@ -216,10 +229,19 @@ struct Operand {
     const uint16_t* p;
     int64_t ld, r0, extent, k_valid;
 };
+__device__ __forceinline__ Operand scalar(const Operand& o) {
+    return {scalar(o.p), o.ld, scalar(o.r0), scalar(o.extent), scalar(o.k_valid)};
+}
 
 typedef short v4i16 __attribute__((ext_vector_type(4)));
 
 // acc = A_tile * B_tile^T over k in [0, K), K a multiple of 64.
+//
+// What bounds it is power: the chip runs these loops at its limit, so the clock follows the energy of an operation.
+// Hence v_mfma_f32_16x16x32_bf16 and not 32x32x16, whose accumulators are read and written twice as often per
+// operation: MFMAs alone on random data, eight waves per CU, sustain 2.01 against 1.74 PFLOP/s.  Products of
+// 16384 x 8192 x 4096 in the four layouts, 1.31 -> 1.40 to 1.45 PFLOP/s; the vendor's kernel 1.38 to 1.42 (all on
+// one box); policy-loss step of 22942 rows, 4096 x 128256: 55.8 -> 50.9 ms.
 //
 // Operand tiles reach the LDS by direct global->LDS loads (no VGPR staging, no LDS store
 // instructions), whole 128-byte cache-line segments per 8 lanes.  The path from L2 into the LDS
@@ -235,243 +257,238 @@ typedef short v4i16 __attribute__((ext_vector_type(4)));
 // LDS image of a k-contiguous operand tile: [256 rows][64 k], the eight 16-byte chunks of a row
 // stored at c ^ swz(row); wave w loads rows [32 w, 32 w + 32); fragments are 16-byte reads.
 // LDS image of a k-major operand tile: [64 k][256 columns], the 32 chunks of a k row stored at
-// c ^ 4 (k & 3); wave w loads k rows [8 w, 8 w + 8); fragments come through the transposing read
+// c ^ 4 (k & 3) ^ 2 (k / 8 & 1); wave w loads k rows [8 w, 8 w + 8); fragments come through the transposing read
 // ds_read_b64_tr_b16: in a group of 16 lanes, lane s points at (k0 + s / 4, 4 columns from
 // 4 (s % 4)) and lane i receives column i at k0 .. k0 + 3, which is the MFMA operand layout (row
-// per lane, consecutive k per register).  The permutation puts the four k rows of such a read on
+// per lane, consecutive k per register).  The permutation puts the k rows that 32 lanes read together on
 // different banks.
 //
 // The product comes in two halves: begin_loads requests the first two k-tiles into slots 0 .. 3 (all but the
 // last block), gemm_loop waits for them and does the rest.  A caller may do other work in between that
 // touches slot 4 only.
 //
-// Loader side.  Addresses are a uniform 64-bit base (tile origin + k offset) plus a 32-bit byte
-// offset per lane; for a k-major operand the lanes' offsets of the last k-tile differ (its k
-// rows may end early), `last` holds those.
-struct Loader {
-    const char* tile;    // origin of the tile in global memory
-    int64_t k_step;      // bytes from one k-tile to the next
-    uint32_t off[4];     // per-lane byte offsets of the four loads
-    uint32_t last[4];    // the same for the last k-tile
-    int lds_block;       // elements between the LDS destinations of consecutive loads
-    int lds_wave;        // element offset of this wave's first load inside a slot
-};
+// Loader side: direct global->LDS loads in their buffer form, which takes a uniform 64-bit base (that of a k-tile) and
+// a uniform byte offset in scalar registers and 32 bits per lane in one vector register.  (With 64-bit lane addresses
+// the loads of a k-tile held 32 vector registers, and the compiler waited for every LDS access in flight before it used
+// any fragment, because it counts such a load among them.)  Lanes clamp their offsets onto valid rows and columns, so
+// no bounds are set; a load of a k-tile past the last one gets a buffer of no bytes and fetches nothing.
+//
+// A loader stands at one k-tile and moves on to the next with advance().
 template <bool KM>
-__device__ __forceinline__ Loader make_loader(const Operand& op, int64_t ktiles, int lane, int wave) {
-    Loader L;
-    if constexpr (!KM) {
-        L.tile = reinterpret_cast<const char*>(op.p + op.r0 * op.ld);
-        L.k_step = BK * 2;
-        const int last_row = (int)((op.extent - 1 - op.r0) < 255 ? (op.extent - 1 - op.r0) : 255);
+struct Loader {
+    const char* base;   // of the operand, for k-major of the k-tile
+    uint32_t plus;      // bytes from there to the k-tile (k-contiguous)
+    uint32_t off[4];    // per-lane byte offsets of the four loads
+    int lds_wave;       // bytes to this wave's first load inside a slot
+    int tiles_left;     // from this k-tile on, negated
+    int bytes;          // of the buffer: all there are, or none past the last k-tile
+    int rows_left;      // k rows from this k-tile's first on, without that one (k-major)
+    static constexpr int LDS_BLOCK = KM ? 2 * 256 * 2 : 8 * BK * 2;  // bytes between the LDS destinations of loads
+
+    __device__ __forceinline__ Loader(const Operand& op, int ktiles, int lane, int wave) {
+        tiles_left = -ktiles;
+        bytes = -1;
+        plus = 0;
+        rows_left = (int)op.k_valid - 1;
+        if constexpr (!KM) {
+            base = reinterpret_cast<const char*>(op.p + op.r0 * op.ld);
+            const int last_row = (int)((op.extent - 1 - op.r0) < 255 ? (op.extent - 1 - op.r0) : 255);
 #pragma unroll
-        for (int b = 0; b < 4; ++b) {
-            const int r = wave * 32 + b * 8 + (lane >> 3);
-            const int c = (lane & 7) ^ swz(r);
-            L.off[b] = (uint32_t)(r < last_row ? r : last_row) * (uint32_t)(op.ld * 2) + c * 16;
-            L.last[b] = L.off[b];
+            for (int b = 0; b < 4; ++b) {
+                const int r = wave * 32 + b * 8 + (lane >> 3);
+                const int c = (lane & 7) ^ swz(r);
+                off[b] = __umul24(r < last_row ? r : last_row, pitch(op)) + c * 16;
+            }
+            lds_wave = wave * 32 * BK * 2;
+        } else {
+            base = reinterpret_cast<const char*>(op.p);
+            set_rows(op, lane, wave);
+            lds_wave = wave * 8 * 256 * 2;
         }
-        L.lds_block = 8 * BK;
-        L.lds_wave = wave * 32 * BK;
-    } else {
-        L.tile = reinterpret_cast<const char*>(op.p);
-        L.k_step = BK * op.ld * 2;
-        const int last_k = (int)(op.k_valid - 1 - (ktiles - 1) * BK);  // inside the last k-tile
+    }
+    // at most 2^23; rows inside a tile are at most 255
+    static __device__ __forceinline__ uint32_t pitch(const Operand& op) { return (uint32_t)(op.ld * 2); }
+    // k-major: this k-tile's k rows, which may end inside it
+    __device__ __forceinline__ void set_rows(const Operand& op, int lane, int wave) {
+        const int last_k = rows_left < BK - 1 ? (rows_left < 0 ? 0 : rows_left) : BK - 1;
+        const int r0 = (int)op.r0, extent = (int)op.extent;
 #pragma unroll
         for (int b = 0; b < 4; ++b) {
             const int kk = wave * 8 + b * 2 + (lane >> 5);
-            const int c = (lane & 31) ^ (4 * (kk & 3));
-            int64_t col = op.r0 + c * 8;
-            col = col + 8 <= op.extent ? col : op.extent - 8;
-            L.off[b] = (uint32_t)kk * (uint32_t)(op.ld * 2) + (uint32_t)(col * 2);
-            L.last[b] = (uint32_t)(kk < last_k ? kk : last_k) * (uint32_t)(op.ld * 2) + (uint32_t)(col * 2);
+            const int c = r0 + ((lane & 31) ^ (4 * (kk & 3)) ^ (2 * ((kk >> 3) & 1))) * 8;
+            off[b] = __umul24(kk < last_k ? kk : last_k, pitch(op)) + (uint32_t)((c + 8 <= extent ? c : extent - 8) * 2);
         }
-        L.lds_block = 2 * 256;
-        L.lds_wave = wave * 8 * 256;
     }
-    return L;
+    __device__ __forceinline__ void advance(const Operand& op, int lane, int wave) {
+        ++tiles_left;
+        // in assembly, or the compiler makes a compare of it whose result it puts into a vector register
+        asm("s_ashr_i32 %0, %1, 31" : "=s"(bytes) : "s"(tiles_left) : "scc");
+        if constexpr (KM) {
+            base += (int64_t)BK * 2 * op.ld;  // k rows can lie more than 32 bits apart
+            rows_left -= BK;
+            if (rows_left < BK - 1) set_rows(op, lane, wave);
+        } else {
+            plus += BK * 2;
+        }
+    }
+};
+// 16 bytes per lane from base + off (lane) + plus, 1 KB of consecutive LDS per wave
+__device__ __forceinline__ void load_to_lds(const char* base, int bytes, uint32_t off, uint32_t plus, char* to) {
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(__builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(base), 0, bytes, 0x00027000),
+                                             OI_LDS_PTR(to), 16, off, plus, 0, 0);
 }
-// k-tiles past the end are never requested by the main loop; begin_loads may ask for k-tile 1
-// of a one-k-tile product and then re-reads k-tile 0 into a slot nobody reads
-__device__ __forceinline__ const char* k_src(const Loader& L, int64_t kt, int64_t ktiles) {
-    const uint64_t v = reinterpret_cast<uint64_t>(L.tile + (kt < ktiles ? kt : ktiles - 1) * L.k_step);
-    const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)v);
-    const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)(v >> 32));
-    return reinterpret_cast<const char*>(((uint64_t)hi << 32) | lo);
-}
-// one 1 KB load: block b of this wave's share of an operand k-tile into ring slot `slot`
-__device__ __forceinline__ void load_block(const Loader& L, const char* src, uint32_t off, int slot, int b, uint16_t* lds) {
-    __builtin_amdgcn_global_load_lds(OI_GLOBAL_PTR(src + off),
-                                     OI_LDS_PTR(lds + slot * TILE_ELEMS + L.lds_wave + b * L.lds_block), 16, 0, 0);
+// one 1 KB load: block b of this wave's share of an operand k-tile into the ring slot at byte offset `slot`
+template <bool KM>
+__device__ __forceinline__ void load_block(const Loader<KM>& L, int slot, int b, uint16_t* lds) {
+    load_to_lds(L.base, L.bytes, L.off[b], L.plus, reinterpret_cast<char*>(lds) + slot + L.lds_wave + b * L.LDS_BLOCK);
 }
 // ring slots: A_t -> (2 t) mod 5, B_t -> (2 t + 1) mod 5
 template <bool A_KM, bool B_KM>
-__device__ __forceinline__ void begin_loads(const Operand& A, const Operand& B, int64_t K, uint16_t* lds) {
+__device__ __forceinline__ void begin_loads(const Operand& A_, const Operand& B_, int64_t K, uint16_t* lds) {
+    const Operand A = scalar(A_), B = scalar(B_);
     const int tid = opaque_tid();
     // the wave index as a scalar: the LDS destinations of the loads (M0) then take no VALU work
     const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int64_t ktiles = K / BK;
-    const Loader la = make_loader<A_KM>(A, ktiles, lane, wave), lb = make_loader<B_KM>(B, ktiles, lane, wave);
-    const char* a_k0 = k_src(la, 0, ktiles);
-    const char* b_k0 = k_src(lb, 0, ktiles);
-    const char* a_k1 = k_src(la, 1, ktiles);
-    const char* b_k1 = k_src(lb, 1, ktiles);
-    const bool t0_last = ktiles == 1, t1_last = ktiles <= 2;
+    const int ktiles = __builtin_amdgcn_readfirstlane((int)(K / BK));
+    Loader<A_KM> la(A, ktiles, lane, wave);
+    Loader<B_KM> lb(B, ktiles, lane, wave);
 #pragma unroll
-    for (int b = 0; b < 4; ++b) load_block(la, a_k0, t0_last ? la.last[b] : la.off[b], 0, b, lds);
+    for (int b = 0; b < 4; ++b) load_block(la, 0, b, lds);
 #pragma unroll
-    for (int b = 0; b < 4; ++b) load_block(lb, b_k0, t0_last ? lb.last[b] : lb.off[b], 1, b, lds);
+    for (int b = 0; b < 4; ++b) load_block(lb, SLOT_BYTES, b, lds);
+    la.advance(A, lane, wave);
+    lb.advance(B, lane, wave);
 #pragma unroll
-    for (int b = 0; b < 4; ++b) load_block(la, a_k1, t1_last ? la.last[b] : la.off[b], 2, b, lds);
+    for (int b = 0; b < 4; ++b) load_block(la, 2 * SLOT_BYTES, b, lds);
 #pragma unroll
-    for (int b = 0; b < 3; ++b) load_block(lb, b_k1, t1_last ? lb.last[b] : lb.off[b], 3, b, lds);
+    for (int b = 0; b < 3; ++b) load_block(lb, 3 * SLOT_BYTES, b, lds);
 }
 
 // `__restrict__` here and in store_tile is what tells the compiler that the LDS accesses of these functions carry
 // alias information; without any it waits for every global->LDS load in flight before each LDS access
 // (d_weight of 3072 rows: 2.7 -> 4.9 ms).
 template <bool A_KM, bool B_KM>
-__device__ __forceinline__ void gemm_loop(AccTile& __restrict__ acc, const Operand& A, const Operand& B, int64_t K, uint16_t* lds) {
+__device__ __forceinline__ void gemm_loop(AccTile& __restrict__ acc, const Operand& A_, const Operand& B_, int64_t K, uint16_t* lds) {
+    const Operand A = scalar(A_), B = scalar(B_);
     const int tid = opaque_tid();
     const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wm = wave & 3, wn = wave >> 2;
-    const int64_t ktiles = K / BK;
-    const Loader la = make_loader<A_KM>(A, ktiles, lane, wave), lb = make_loader<B_KM>(B, ktiles, lane, wave);
+    const int ktiles = __builtin_amdgcn_readfirstlane((int)(K / BK));
+    Loader<A_KM> la(A, ktiles, lane, wave);  // at k-tile kt+2
+    Loader<B_KM> lb(B, ktiles, lane, wave);  // at k-tile kt+1 in group 0, kt+2 from group 12 on
+    la.advance(A, lane, wave);
+    la.advance(A, lane, wave);
+    lb.advance(B, lane, wave);
 
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
+    for (int i = 0; i < 4; ++i)
 #pragma unroll
-        for (int j = 0; j < 4; ++j)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
+        for (int j = 0; j < 8; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-    // consumer side: element offsets of this lane's fragments inside a slot
-    const int lr = lane & 31, h = lane >> 5;
-    // k-contiguous image: k-step ks flips the stored chunk by (2 ks); rows 32 apart share the
-    // same permutation
-    const int pg = h ^ swz(lr);
-    const int a_base = (wm * 64 + lr) * BK + pg * 8, b_base = (wn * 128 + lr) * BK + pg * 8;
-    // k-major image: source lane s of a 16-lane group points at k row (s >> 2) of the lane's
-    // half-k-step and at 4 columns from 4 (s & 3) of the group's 16; one address per 32-row tile
-    // because the column permutation reaches the bits that select the tile
-    const int s16 = lane & 15, e4 = s16 >> 2, g16 = (lane >> 4) & 1;
-    int a_km[2], b_km[4];
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-        a_km[i] = (h * 8 + e4) * 256 + (((wm * 8 + i * 4 + g16 * 2 + ((s16 & 3) >> 1)) ^ (4 * e4)) * 8) + 4 * (s16 & 1);
-#pragma unroll
-    for (int j = 0; j < 4; ++j)
-        b_km[j] = (h * 8 + e4) * 256 + (((wn * 16 + j * 4 + g16 * 2 + ((s16 & 3) >> 1)) ^ (4 * e4)) * 8) + 4 * (s16 & 1);
-    auto read_tr = [&](const uint16_t* p) {
-        // rows k0 .. k0 + 3 and k0 + 4 .. k0 + 7 of the lane's half-k-step
+    // consumer side: byte offsets of this lane's fragments inside a slot; a lane holds row lr of a 16-row
+    // fragment at the k values 8 g .. 8 g + 7 of a k-step
+    const int lr = lane & 15, g = lane >> 4;
+    // k-contiguous image: the second k-step flips bit 2 of the stored chunk; rows 16 apart share the same
+    // permutation
+    const int pg = (g ^ swz(lr)) * 16;
+    const int a_base = (wm * 64 + lr) * (BK * 2) + pg, b_base = (wn * 128 + lr) * (BK * 2) + pg;
+    // k-major image: source lane lr of a 16-lane group points at k row (lr >> 2) of the group's 8 and at 4
+    // columns from 4 (lr & 3) of the fragment's 16; fragments are two chunks apart, which flips the chunk bits
+    // that the permutation reaches
+    const int e4 = lr >> 2, km_row = (g * 8 + e4) * 512 + 8 * (lr & 1), km_perm = (4 * e4) ^ (2 * (g & 1));
+    const int a_km = km_row + ((wm * 8 + ((lr & 3) >> 1)) ^ km_perm) * 16;
+    const int b_km = km_row + ((wn * 16 + ((lr & 3) >> 1)) ^ km_perm) * 16;
+    const char* ring = reinterpret_cast<const char*>(lds);
+    auto read_tr = [&](int at) {
+        // k rows 0 .. 3 and 4 .. 7 of the lane's 8
         const v4i16 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-            (__attribute__((address_space(3))) v4i16*)OI_LDS_PTR(const_cast<uint16_t*>(p)));
+            (__attribute__((address_space(3))) v4i16*)OI_LDS_PTR(const_cast<char*>(ring + at)));
         const v4i16 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-            (__attribute__((address_space(3))) v4i16*)OI_LDS_PTR(const_cast<uint16_t*>(p + 4 * 256)));
+            (__attribute__((address_space(3))) v4i16*)OI_LDS_PTR(const_cast<char*>(ring + at + 4 * 512)));
         const short __attribute__((ext_vector_type(8))) both = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
         return __builtin_bit_cast(bf16x8, both);
     };
     auto read_a = [&](int slot, int ks, int i) {
-        if constexpr (A_KM) return read_tr(lds + slot * TILE_ELEMS + ks * 16 * 256 + a_km[i]);
-        else return *reinterpret_cast<const bf16x8*>(lds + slot * TILE_ELEMS + (a_base ^ (ks * 16)) + i * 32 * BK);
+        if constexpr (A_KM) return read_tr(((slot + a_km) ^ (i * 32)) + ks * 32 * 512);
+        else return *reinterpret_cast<const bf16x8*>(ring + slot + (a_base ^ (ks * 64)) + i * 16 * (BK * 2));
     };
     auto read_b = [&](int slot, int ks, int j) {
-        if constexpr (B_KM) return read_tr(lds + slot * TILE_ELEMS + ks * 16 * 256 + b_km[j]);
-        else return *reinterpret_cast<const bf16x8*>(lds + slot * TILE_ELEMS + (b_base ^ (ks * 16)) + j * 32 * BK);
+        if constexpr (B_KM) return read_tr(((slot + b_km) ^ (j * 32)) + ks * 32 * 512);
+        else return *reinterpret_cast<const bf16x8*>(ring + slot + (b_base ^ (ks * 64)) + j * 16 * (BK * 2));
     };
 
-    // One k-step: 8 MFMAs on (ac, bc) with the 6 fragment reads of the following k-step (from slots
-    // sa_n / sb_n at k-step ks_n) and this k-step's share of the global->LDS loads placed between
-    // them one by one.  Nothing may move across the scheduling barriers: loads issued back to back
-    // hold up the wave's MFMA issue, and a fragment read issued ahead of the first MFMA would be
-    // waited for together with the current fragments (a full LDS round trip with the matrix pipe
-    // idle).
-    bf16x8 a0[2], b0[4], a1[2], b1[4];
-#define OI_KSTEP(ac, bc, an, bn, sa_n, sb_n, ks_n, LOADS_AT)                                                     \
-    {                                                                                                            \
-        _Pragma("unroll") for (int q = 0; q < 8; ++q) {                                                          \
-            acc[q >> 2][q & 3] =                                                                                 \
-                __builtin_amdgcn_mfma_f32_32x32x16_bf16(ac[q >> 2], bc[q & 3], acc[q >> 2][q & 3], 0, 0, 0);     \
-            __builtin_amdgcn_sched_barrier(0);                                                                   \
-            LOADS_AT(q)                                                                                          \
-            if (q < 2) an[q] = read_a(sa_n, ks_n, q);                                                            \
-            else if (q < 6) bn[q - 2] = read_b(sb_n, ks_n, q - 2);                                               \
-            __builtin_amdgcn_sched_barrier(0);                                                                   \
-        }                                                                                                        \
-    }
-    // the 8 loads of a k-tile iteration, as evenly spread as the slot hand-over allows; OFF selects
-    // the lanes' offsets (off, or last when the k-tile being fetched is the last one)
-#define OI_LOADS_KS0(q)                                         \
-    if (q == 1) load_block(lb, b_n1, lb.off[3], s_b1, 3, lds);       \
-    if (q == 5) load_block(la, a_n2, la.OFF2[0], s_a2, 0, lds);
-#define OI_LOADS_KS1(q) \
-    if (q == 3) load_block(la, a_n2, la.OFF2[1], s_a2, 1, lds);
-#define OI_LOADS_KS2(q)                                         \
-    if (q == 1) load_block(la, a_n2, la.OFF2[2], s_a2, 2, lds);      \
-    if (q == 5) load_block(la, a_n2, la.OFF2[3], s_a2, 3, lds);
-#define OI_LOADS_KS3(q)                                         \
-    if (q == 0) load_block(lb, b_n2, lb.OFF2[0], s_a, 0, lds);       \
-    if (q == 3) load_block(lb, b_n2, lb.OFF2[1], s_a, 1, lds);       \
-    if (q == 6) load_block(lb, b_n2, lb.OFF2[2], s_a, 2, lds);
-#define OI_LOADS_NONE(q)
-#define OI_LOADS_KS0_ONLY_B(q) \
-    if (q == 1) load_block(lb, b_n1, lb.last[3], s_b1, 3, lds);
-
+    // A k-tile is two k-steps of 32, each eight groups of four MFMAs: group u of the sixteen multiplies B fragment
+    // u (u mod 8 of its k-step) with the four A fragments, up and down in turn, so that one operand of an MFMA is
+    // always that of the one before (power is what limits the loop).  A fragments have two sets of registers, B
+    // fragments a ring of eight; the 24 fragment reads and the 8 global->LDS loads stand one by one between the
+    // MFMAs.  Nothing may move across the scheduling barriers: loads issued back to back hold up the wave's MFMA
+    // issue, and a fragment read issued ahead of the MFMAs before it would be waited for together with the
+    // current fragments (a full LDS round trip with the matrix pipe idle).
+    bf16x8 a[2][4], b[16];
     // A_0 and B_0 must have landed.  The wait is for everything in flight, not for "all but the 7
     // younger loads": a workgroup that runs several tiles may still have the previous tile's
     // stores outstanding, and stores complete out of order with loads.
     wait_loads_and_barrier<0>();
 #pragma unroll
-    for (int i = 0; i < 2; ++i) a0[i] = read_a(0, 0, i);
+    for (int i = 0; i < 4; ++i) {
+        a[0][i] = read_a(0, 0, i);
+        __builtin_amdgcn_sched_barrier(0);
+    }
 #pragma unroll
-    for (int j = 0; j < 4; ++j) b0[j] = read_b(1, 0, j);
+    for (int j = 0; j < 4; ++j) {
+        b[j] = read_b(SLOT_BYTES, 0, j);
+        __builtin_amdgcn_sched_barrier(0);
+    }
 
-    // One k-tile iteration.  The last two iterations have no later k-tiles to fetch: they run
-    // without those loads (no wasted traffic, nothing to drain before the epilogue).
-#define OI_KTILE(L0, L1, L2, L3, PENDING)                                                                       \
-    {                                                                                                            \
-        const int s_a = sa, s_b = ring_slot(sa + 1);                  /* being read */                          \
-        const int s_a1 = ring_slot(sa + 2), s_b1 = ring_slot(sa + 3); /* k-tile kt+1 */                         \
-        const int s_a2 = ring_slot(sa + 4);                           /* free all along: takes A_(kt+2) */      \
-        const char* b_n1 = k_src(lb, kt + 1, ktiles);                                                                    \
-        const char* a_n2 = k_src(la, kt + 2, ktiles);                                                                    \
-        const char* b_n2 = k_src(lb, kt + 2, ktiles);                                                                    \
-        (void)s_a2; (void)s_b1; (void)b_n1; (void)a_n2; (void)b_n2;                                              \
-        OI_KSTEP(a0, b0, a1, b1, s_a, s_b, 1, L0)                                                                \
-        OI_KSTEP(a1, b1, a0, b0, s_a, s_b, 2, L1)                                                                \
-        OI_KSTEP(a0, b0, a1, b1, s_a, s_b, 3, L2)                                                                \
-        /* k-tile kt+1 must have landed (its last load was issued in the first k-step above; the  */            \
-        /* PENDING younger ones may stay in flight) and this wave's reads of k-tile kt must be     */            \
-        /* complete: after the barrier A_kt's slot is overwritten with B_(kt+2)                    */            \
-        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(PENDING) : "memory");                                \
-        __builtin_amdgcn_s_barrier();                                                                            \
-        asm volatile("" ::: "memory");                                                                           \
-        OI_KSTEP(a1, b1, a0, b0, s_a1, s_b1, 0, L3)                                                              \
-        sa = s_a1;                                                                                               \
+    // Fragments: at the start of a k-tile the A fragments of the first k-step and B fragments 0 .. 3 are there or under
+    // way; groups 0 .. 11 read the rest.  Before group 12 goes on, k-tile kt+1 must have landed (its last load was
+    // issued in group 0; the 4 younger ones may stay in flight) and this wave's reads of k-tile kt must be complete:
+    // after the barrier A_kt's slot is overwritten with B_(kt+2), and groups 12 .. 15 read the first fragments of
+    // k-tile kt+1 (past the last k-tile: of slots that hold nothing, for nobody).
+    // The scalar work of a k-tile (loaders, slots) is spread as well: in one place it is a gap between MFMAs.
+    // slots of A_kt, B_kt (being read), A_(kt+1), B_(kt+1), and the one that is free all along: takes A_(kt+2)
+    int s_a = 0, s_b = SLOT_BYTES, s_a1 = 2 * SLOT_BYTES, s_b1 = 3 * SLOT_BYTES, s_a2 = 4 * SLOT_BYTES;
+#pragma unroll 1
+    for (int left = ktiles; left > 0; --left) {
+#pragma unroll
+        for (int u = 0; u < 16; ++u) {
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const int i = (u & 1) ? 3 - q : q, j = u & 7;
+                acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[u >> 3][i], b[u], acc[i][j], 0, 0, 0);
+                __builtin_amdgcn_sched_barrier(0);
+                if (u == 12 && q == 1) {
+                    asm volatile("s_waitcnt vmcnt(4) lgkmcnt(0)" ::: "memory");
+                    __builtin_amdgcn_s_barrier();
+                    asm volatile("" ::: "memory");
+                }
+                // one of the loads, as evenly spread as the slot hand-over allows
+                if (u == 0 && q == 1) load_block(lb, s_b1, 3, lds);
+                if ((u == 2 || u == 5 || u == 7 || u == 10) && q == 1) load_block(la, s_a2, u == 2 ? 0 : u == 5 ? 1 : u == 7 ? 2 : 3, lds);
+                if ((u == 12 || u == 13) && q == 3) load_block(lb, s_a, u - 12, lds);
+                if (u == 15 && q == 1) load_block(lb, s_a, 2, lds);
+                if (u == 11 && q == 2) la.advance(A, lane, wave);
+                if (u == 10 && q == 2) lb.advance(B, lane, wave);
+                // fragments
+                if (u < 12 && q == 0) b[u + 4] = read_b(s_b, (u + 4) >> 3, (u + 4) & 7);
+                if (u >= 2 && u < 6 && q == 2) a[1][u - 2] = read_a(s_a, 1, u - 2);
+                if (u == 12 && q >= 1) a[0][q - 1] = read_a(s_a1, 0, q - 1);
+                if (u == 13 && q == 0) a[0][3] = read_a(s_a1, 0, 3);
+                if (u == 13 && q >= 1 && q <= 2) b[q - 1] = read_b(s_b1, 0, q - 1);
+                if (u == 14 && q == 1) b[2] = read_b(s_b1, 0, 2);
+                if (u == 15 && q == 0) b[3] = read_b(s_b1, 0, 3);
+                if (u == 15 && q == 2) {
+                    const int was_a = s_a, was_b = s_b;
+                    s_a = s_a1;
+                    s_b = s_b1;
+                    s_a1 = s_a2;
+                    s_b1 = was_a;
+                    s_a2 = was_b;
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
     }
-    int sa = 0;  // slot of A_kt
-    int64_t kt = 0;
-#define OFF2 off
-    for (; kt + 3 < ktiles; ++kt) OI_KTILE(OI_LOADS_KS0, OI_LOADS_KS1, OI_LOADS_KS2, OI_LOADS_KS3, 4)
-#undef OFF2
-#define OFF2 last
-    if (kt + 2 < ktiles) {  // this iteration fetches the last k-tile
-        OI_KTILE(OI_LOADS_KS0, OI_LOADS_KS1, OI_LOADS_KS2, OI_LOADS_KS3, 4)
-        ++kt;
-    }
-#undef OFF2
-    if (kt + 1 < ktiles) {
-        OI_KTILE(OI_LOADS_KS0_ONLY_B, OI_LOADS_NONE, OI_LOADS_NONE, OI_LOADS_NONE, 0)
-        ++kt;
-    }
-    OI_KTILE(OI_LOADS_NONE, OI_LOADS_NONE, OI_LOADS_NONE, OI_LOADS_NONE, 0)
-#undef OI_KTILE
-#undef OI_KSTEP
-#undef OI_LOADS_KS0
-#undef OI_LOADS_KS1
-#undef OI_LOADS_KS2
-#undef OI_LOADS_KS3
-#undef OI_LOADS_NONE
-#undef OI_LOADS_KS0_ONLY_B
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     // every wave is done reading before the caller reuses the LDS (epilogue staging, next tile)
     __builtin_amdgcn_s_barrier();
@@ -490,29 +507,62 @@ __device__ __forceinline__ void gemm_tile(AccTile& acc, const uint16_t* __restri
     gemm_tile<false, false>(acc, a, b, K, lds);
 }
 
-// Accumulator geometry of one wave: element (i, j, r) of lane `lane` is
-//   m (row, vocabulary in the logits kernels) = wm*64 + i*32 + (r/4)*8 + (lane/32)*4 + r%4
+// An MFMA leaves lane l with rows 4 (l / 16) .. + 3 of column l % 16 of a 16 x 16 tile (acc[i][j]: rows 16 i, columns
+// 16 j of the wave's 64 x 128).  The epilogues take column groups of 32: swapping the odd quarters of the lanes of one
+// column tile with the even ones of the next gives a lane one column and eight consecutive rows of every 16.
+// Element (i, r) of lane `lane` of column group j is then
+//   m (row, vocabulary in the logits kernels) = wm*64 + i*32 + (r/8)*16 + (lane/32)*8 + r%8
 //   n (column, token in the logits kernels)   = wn*128 + j*32 + lane%32
+__device__ __forceinline__ void swap_quarters(const f32x4& x, const f32x4& y, f32x16& z, int r0) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        const auto w = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(uint32_t, (float)x[e]),
+                                                        __builtin_bit_cast(uint32_t, (float)y[e]), false, false);
+        z[r0 + e] = __builtin_bit_cast(float, (uint32_t)w[0]);
+        z[r0 + 4 + e] = __builtin_bit_cast(float, (uint32_t)w[1]);
+    }
+}
+struct Columns {
+    f32x16 z[2];  // not an array of floats: the search for the label's register would put that into memory
+};
+__device__ __forceinline__ Columns tile_columns(const AccTile& acc, int j) {
+    Columns c;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) swap_quarters(acc[i][2 * j], acc[i][2 * j + 1], c.z[i >> 1], (i & 1) * 8);
+    return c;
+}
 __device__ __forceinline__ int acc_row(int wm, int i, int r, int lane) {
-    return wm * 64 + i * 32 + (r >> 2) * 8 + (lane >> 5) * 4 + (r & 3);
+    return wm * 64 + i * 32 + (r >> 3) * 16 + (lane >> 5) * 8 + (r & 7);
 }
 __device__ __forceinline__ int acc_col(int wn, int j, int lane) { return wn * 128 + j * 32 + (lane & 31); }
 
-// A fp32 tile that another kernel picks up: in the order in which the accumulators lie in the registers
+// A fp32 tile that another kernel picks up: in the order in which its column groups lie in the registers
 // (16 bytes per lane, consecutive lanes together, groups of PART_GROUP floats), so that neither side
 // rearranges anything.
 constexpr int PART_FLOATS = BM * BN, PART_GROUP = NTHREADS * 4;
 __device__ __forceinline__ int part_group(int i, int j, int q) { return (i * 4 + j) * 4 + q; }
-__device__ __forceinline__ void store_part(const AccTile& acc, float* part, int tid) {
+__device__ __forceinline__ void store_part(const Columns& c, float* part, int j, int tid) {
     asm volatile("" : "+v"(tid));
 #pragma unroll
     for (int i = 0; i < 2; ++i)
 #pragma unroll
-        for (int j = 0; j < 4; ++j)
+        for (int q = 0; q < 4; ++q)
+            *reinterpret_cast<oi_f32x4*>(part + part_group(i, j, q) * PART_GROUP + tid * 4) =
+                oi_f32x4{c.z[i][q * 4], c.z[i][q * 4 + 1], c.z[i][q * 4 + 2], c.z[i][q * 4 + 3]};
+}
+__device__ __forceinline__ Columns load_part(const float* part, int j, int tid) {
+    oi_f32x4 v[2][4];
 #pragma unroll
-            for (int q = 0; q < 4; ++q)
-                *reinterpret_cast<oi_f32x4*>(part + part_group(i, j, q) * PART_GROUP + tid * 4) =
-                    oi_f32x4{acc[i][j][q * 4], acc[i][j][q * 4 + 1], acc[i][j][q * 4 + 2], acc[i][j][q * 4 + 3]};
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+            v[i][q] = *reinterpret_cast<const oi_f32x4*>(part + part_group(i, j, q) * PART_GROUP + tid * 4);
+    Columns c;
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) c.z[i][r] = v[i][r >> 2][r & 3];
+    return c;
 }
 
 // Online softmax statistics in the log2 domain of the scaled logits x = z * c:
@@ -577,27 +627,28 @@ __device__ __forceinline__ void stats_update(f32x16 (&z)[2], int wm, int lane, i
 
 // A finished tile leaves as bf16 rows of 256 columns one column group at a time: group j holds the 64 rows
 // (tokens, or rows of a product) wn * 128 + j * 32 + (0..31) of both wn halves with all 256 columns (every m-wave
-// contributes its 64).  A lane holds groups of four consecutive columns of one row; they meet in a region of one
+// contributes its 64).  A lane holds groups of eight consecutive columns of one row; they meet in a region of one
 // ring slot and go to global memory in 16-byte pieces of whole 512-byte rows, while the next group's work is being
 // done (forward per slab at the Llama-3.1-8B shape: 6.32 -> 6.28 ms against the whole image at the end).
 //
-// The region: 64 rows of 512 bytes, unpadded; the 16-byte pieces of a row at c ^ (row mod 32) and their halves
-// swapped in rows 16 .. 31 of every 32, which puts the 8-byte stores of 32 lanes on all 64 banks.
+// The region: 64 rows of 512 bytes, unpadded; the 16-byte pieces of a row at c ^ piece_perm(row), which puts the
+// 16-byte stores of 16 rows, and those of 8 rows and two neighbouring pieces, on all 64 banks.
+__device__ __forceinline__ int piece_perm(int row) { return (row & 7) << 1 | (row >> 3 & 1) | (row & 16); }
 constexpr int GROUP_ROWS = 64;
 constexpr int GROUP_BF16_AT = 4 * TILE_ELEMS;  // ring slot 4: slots 0 .. 3 may be filling for the next tile
 static_assert(GROUP_ROWS * BM <= TILE_ELEMS, "a bf16 group fits one ring slot");
 __device__ __forceinline__ int64_t group_row(int64_t row0, int j, int r) { return row0 + (r >> 5) * 128 + j * 32 + (r & 31); }
-// columns acc_row(wm, i, 4 q .. 4 q + 3, lane) of the lane's row
-__device__ __forceinline__ void stage_bf16x4(uint16_t* stage, int wm, int wn, int lane, int i, int q, float a, float b, float c,
-                                             float d) {
-    const int srow = wn * 32 + (lane & 31);
-    const int piece = (wm * 8 + i * 4 + q) ^ (srow & 31), half = (lane >> 5) ^ ((srow >> 4) & 1);
-    *reinterpret_cast<uint2*>(stage + srow * BM + piece * 8 + half * 4) = make_uint2(oi_pack_bf16x2(a, b), oi_pack_bf16x2(c, d));
+// columns acc_row(wm, i, 8 p .. 8 p + 7, lane) of the lane's row, which value(r) gives
+template <class Value>
+__device__ __forceinline__ void stage_bf16x8(uint16_t* stage, int wm, int wn, int lane, int i, int p, Value&& value) {
+    const int srow = wn * 32 + (lane & 31), piece = (wm * 8 + i * 4 + p * 2 + (lane >> 5)) ^ piece_perm(srow);
+    *reinterpret_cast<oi_u32x4*>(stage + srow * BM + piece * 8) =
+        oi_u32x4{oi_pack_bf16x2(value(p * 8), value(p * 8 + 1)), oi_pack_bf16x2(value(p * 8 + 2), value(p * 8 + 3)),
+                 oi_pack_bf16x2(value(p * 8 + 4), value(p * 8 + 5)), oi_pack_bf16x2(value(p * 8 + 6), value(p * 8 + 7))};
 }
 constexpr int GROUP_PIECES = GROUP_ROWS * (BM / 8) / NTHREADS;  // 16-byte pieces per thread
 __device__ __forceinline__ oi_u32x4 staged_piece(const uint16_t* stage, int r, int ch) {
-    const oi_u32x4 v = *reinterpret_cast<const oi_u32x4*>(stage + r * BM + (ch ^ (r & 31)) * 8);
-    return (r & 16) ? oi_u32x4{v.z, v.w, v.x, v.y} : v;
+    return *reinterpret_cast<const oi_u32x4*>(stage + r * BM + (ch ^ piece_perm(r)) * 8);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -652,7 +703,7 @@ __device__ __forceinline__ FwdColumn fwd_column(const FwdArgs& a, const float* x
 // exponentials (through `stage`; every thread of the workgroup takes part).
 template <FwdKeep KEEP>
 __device__ __forceinline__ void fwd_fold(f32x16 (&__restrict__ z)[2], FwdColumn& col, const FwdArgs& a, const FwdLaunch& fl,
-                                         int64_t vt, int64_t n0, int j, int tid, uint16_t* stage) {
+                                         int64_t vt, int64_t n0, int j, int tid, uint16_t* __restrict__ stage) {
     constexpr bool CACHE = KEEP == FWD_EXPONENTIALS;
     asm volatile("" : "+v"(tid));  // addresses are formed here, not ahead of the tile's main loop
     const int lane = tid & 63, wave = tid >> 6, wm = wave & 3, wn = wave >> 2;
@@ -663,7 +714,7 @@ __device__ __forceinline__ void fwd_fold(f32x16 (&__restrict__ z)[2], FwdColumn&
     int label_reg = -1;
     if (rel >= 0 && rel < 64) {
         const int rr = rel & 31;
-        if (((rr >> 2) & 1) == (lane >> 5)) label_reg = (rel >> 5) * 16 + (rr >> 3) * 4 + (rr & 3);
+        if (((rr >> 3) & 1) == (lane >> 5)) label_reg = (rel >> 5) * 16 + (rr >> 4) * 8 + (rr & 7);
     }
     if (label_reg >= 0) {
         float v = 0.f;
@@ -692,9 +743,7 @@ __device__ __forceinline__ void fwd_fold(f32x16 (&__restrict__ z)[2], FwdColumn&
 #pragma unroll
         for (int i = 0; i < 2; ++i)
 #pragma unroll
-            for (int q = 0; q < 4; ++q)
-                stage_bf16x4(stage, wm, wn, lane, i, q, z[i][q * 4], z[i][q * 4 + 1], z[i][q * 4 + 2],
-                             z[i][q * 4 + 3]);
+            for (int p = 0; p < 2; ++p) stage_bf16x8(stage, wm, wn, lane, i, p, [&](int r) { return z[i][r]; });
         lds_barrier();
         uint16_t* dst = fl.ecache + n0 * fl.cache_ld + (vt - fl.cache_tile0) * BM;
 #pragma unroll 1
@@ -759,12 +808,13 @@ __device__ __forceinline__ void lmhead_fwd_item(const FwdArgs& a, const FwdLaunc
         // pass of 1432 rows, 4096 x 128256: 1.435 -> 1.40 ms; steps 0.2 to 0.6 %)
         rows.r0 += BM;
         if (vt + 1 < vt_end) begin_loads<false, false>(rows, tokens, a.hdim, lds);
-        // leaves while the statistics are computed
-        if (KEEP == FWD_LOGITS) store_part(acc, fl.logits + (vt * fl.logits_tiles + tt) * PART_FLOATS, tid);
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
-            f32x16 z[2] = {acc[0][j], acc[1][j]};
-            fwd_fold<KEEP>(z, col[j], a, fl, vt, n0, j, tid, lds + GROUP_BF16_AT);
+            Columns c = tile_columns(acc, j);
+            // leaves while the statistics are computed
+            if (KEEP == FWD_LOGITS) store_part(c, fl.logits + (vt * fl.logits_tiles + tt) * PART_FLOATS, j, tid);
+            fwd_fold<KEEP>(c.z, col[j], a, fl, vt, n0, j, tid, lds + GROUP_BF16_AT);
+            __builtin_amdgcn_sched_barrier(0);
         }
     }
 
@@ -787,7 +837,7 @@ template <FwdKeep KEEP>
 __global__ void __launch_bounds__(NTHREADS)
     lmhead_fwd_kernel(FwdArgs a, const int32_t* __restrict__ n_dev, FwdLaunch fl, uint32_t* __restrict__ queue) {
     __shared__ __align__(16) uint16_t lds[LDS_ELEMS];
-    if (n_dev) a.n_tokens = *n_dev;  // rows selected on the device: the host only knows an upper bound
+    if (n_dev) a.n_tokens = device_count(n_dev);  // rows selected on the device: the host only knows an upper bound
     const int64_t token_tiles = (a.n_tokens + BN - 1) / BN;
     // every long item of every XCD's queue is taken before the first short one: the short items are
     // there to fill the end of the launch
@@ -882,15 +932,12 @@ struct DzInputs {
     float c, inv_t;
 };
 // One lane's 32 logits z0, z1 (rows acc_row(wm, 0 / 1, r, lane) of the tile's 256 vocabulary rows from m0)
-// of token n to bf16 entries of dZ in the staging row srow, whose bit 3 is that of the lane.
+// of token n to bf16 entries of dZ in the staging row srow.
 //
-// stage[row][v]: rows = tokens, 256 (+8 pad) vocabulary columns.  A lane stores 8 bytes (4 vocabulary
-// entries of one token) and consecutive lanes store to consecutive rows, 132 words apart: the stores of
-// rows 8 apart meet on the same banks (measured: 1000 conflict cycles per tile).  Rows 8..15 of every 16
-// therefore swap the two 8-byte halves of each 16-byte piece (0 conflict cycles); the copy-out swaps them
-// back.
+// stage[row][v]: rows = tokens, 256 (+8 pad) vocabulary columns.  A lane stores 16 bytes (8 vocabulary entries of
+// one token) and consecutive lanes store to consecutive rows, 132 words apart: 16 of them meet all 64 banks.
 __device__ __forceinline__ void dz_column(const f32x16& z0, const f32x16& z1, const DzInputs& in, int64_t n, int64_t m0,
-                                          int wm, int lane, uint16_t* srow, int row_bit3) {
+                                          int wm, int lane, uint16_t* srow) {
     const int rows_left = (int)(in.vocab - m0 < BM ? in.vocab - m0 : BM);  // real vocabulary rows of the tile
     const int wave_row0 = wm * 64;
     const bool live = n < in.n_tokens;
@@ -903,32 +950,32 @@ __device__ __forceinline__ void dz_column(const f32x16& z0, const f32x16& z1, co
     // (exact also where p_label is close to 1) and written over the entry that the sweep below
     // leaves there: the sweep itself then treats all entries alike.
     const int rel = (live && y >= m0 && y < m0 + BM) ? (int)(y - m0) - wave_row0 : -1;
-    const bool mine = rel >= 0 && rel < 64 && (((rel & 31) >> 2) & 1) == (lane >> 5);
+    const bool mine = rel >= 0 && rel < 64 && (((rel & 31) >> 3) & 1) == (lane >> 5);
     const float ng = -g;
     auto sweep = [&](auto last_tile_tag) {
 #pragma unroll
         for (int i = 0; i < 2; ++i)
 #pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                float d[4];
+            for (int p = 0; p < 2; ++p) {
+                float d[8];
 #pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    const int r = q * 4 + e;
+                for (int e = 0; e < 8; ++e) {
+                    const int r = p * 8 + e;
                     float val = ng * __builtin_amdgcn_exp2f(fmaf(i == 0 ? z0[r] : z1[r], in.c, -l2));
                     if (decltype(last_tile_tag)::value && acc_row(wm, i, r, lane) >= rows_left) val = 0.f;
                     d[e] = val;
                 }
-                const int vl = acc_row(wm, i, q * 4, lane) ^ (row_bit3 << 2);
-                uint2 pk = make_uint2(oi_pack_bf16x2(d[0], d[1]), oi_pack_bf16x2(d[2], d[3]));
-                *reinterpret_cast<uint2*>(srow + vl) = pk;
+                *reinterpret_cast<oi_u32x4*>(srow + acc_row(wm, i, p * 8, lane)) =
+                    oi_u32x4{oi_pack_bf16x2(d[0], d[1]), oi_pack_bf16x2(d[2], d[3]), oi_pack_bf16x2(d[4], d[5]),
+                             oi_pack_bf16x2(d[6], d[7])};
             }
     };
     if (rows_left < BM) sweep(std::true_type{});  // the last vocabulary tile: rows past the vocabulary hold 0
     else sweep(std::false_type{});
     if (mine) {
-        // same lane, same LDS word as the store above: program order keeps them apart
+        // same lane, same LDS piece as the store above: program order keeps them apart
         const float val = ng * expm1f(in.logprob[n]);
-        srow[(wave_row0 + rel) ^ (row_bit3 << 2)] = (uint16_t)oi_f32_to_bf16_bits(val);
+        srow[wave_row0 + rel] = (uint16_t)oi_f32_to_bf16_bits(val);
     }
 }
 
@@ -945,7 +992,8 @@ __device__ __forceinline__ void lmhead_dz_tile(const uint16_t* __restrict__ W, c
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
         const int nl = acc_col(wn, j, lane);
-        dz_column(acc[0][j], acc[1][j], in, n0 + nl, m0, wm, lane, stage + nl * STAGE_STRIDE, (nl >> 3) & 1);
+        const Columns c = tile_columns(acc, j);
+        dz_column(c.z[0], c.z[1], in, n0 + nl, m0, wm, lane, stage + nl * STAGE_STRIDE);
     }
     __syncthreads();
     const int64_t vcol0 = vt * BM;  // column of this tile inside the chunk
@@ -954,9 +1002,8 @@ __device__ __forceinline__ void lmhead_dz_tile(const uint16_t* __restrict__ W, c
     for (int it = 0; it < 16; ++it) {
         const int cidx = tid + it * NTHREADS;
         const int row = cidx >> 5, ch = cidx & 31;
-        oi_u32x4 v = *reinterpret_cast<const oi_u32x4*>(stage + row * STAGE_STRIDE + ch * 8);
-        if (row & 8) v = oi_u32x4{v.z, v.w, v.x, v.y};
-        *reinterpret_cast<oi_u32x4*>(dz + (n0 + row) * chunk_cols + vcol0 + ch * 8) = v;
+        *reinterpret_cast<oi_u32x4*>(dz + (n0 + row) * chunk_cols + vcol0 + ch * 8) =
+            *reinterpret_cast<const oi_u32x4*>(stage + row * STAGE_STRIDE + ch * 8);
     }
 }
 
@@ -966,7 +1013,7 @@ __global__ void __launch_bounds__(NTHREADS)
                      uint16_t* __restrict__ dz, uint32_t* __restrict__ queue) {
     __shared__ __align__(16) uint16_t lds[LDS_ELEMS];
     if (n_dev) {
-        in.n_tokens = *n_dev;
+        in.n_tokens = device_count(n_dev);
         n_pad = (in.n_tokens + BN - 1) / BN * BN;
     }
     for_each_tile(queue, chunk_cols / BM, n_pad / BN, lds, [&](int64_t vt, int64_t tt) {
@@ -989,27 +1036,16 @@ __global__ void __launch_bounds__(NTHREADS)
     if (n0 >= in.n_tokens) return;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, wm = wave & 3, wn = wave >> 2;
     const float* tile = logits + (vt * logits_tiles + tt) * PART_FLOATS;
-    oi_f32x4 z4[2][4];
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int q = 0; q < 4; ++q)
-            z4[i][q] = *reinterpret_cast<const oi_f32x4*>(tile + part_group(i, j, q) * PART_GROUP + tid * 4);
-    f32x16 z[2];
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) z[i][r] = z4[i][r >> 2][r & 3];
+    const Columns c = load_part(tile, j, tid);
     const int row = wn * 32 + (lane & 31);
-    dz_column(z[0], z[1], in, n0 + acc_col(wn, j, lane), vt * BM, wm, lane, stage + row * STAGE_STRIDE, (row >> 3) & 1);
+    dz_column(c.z[0], c.z[1], in, n0 + acc_col(wn, j, lane), vt * BM, wm, lane, stage + row * STAGE_STRIDE);
     __syncthreads();
 #pragma unroll
     for (int it = 0; it < KEPT_ROWS * (BM / 8) / NTHREADS; ++it) {
         const int cidx = tid + it * NTHREADS;
         const int r = cidx >> 5, ch = cidx & 31;
-        oi_u32x4 v = *reinterpret_cast<const oi_u32x4*>(stage + r * STAGE_STRIDE + ch * 8);
-        if (r & 8) v = oi_u32x4{v.z, v.w, v.x, v.y};
-        *reinterpret_cast<oi_u32x4*>(dz + (n0 + (r >> 5) * 128 + j * 32 + (r & 31)) * cols + vt * BM + ch * 8) = v;
+        *reinterpret_cast<oi_u32x4*>(dz + (n0 + (r >> 5) * 128 + j * 32 + (r & 31)) * cols + vt * BM + ch * 8) =
+            *reinterpret_cast<const oi_u32x4*>(stage + r * STAGE_STRIDE + ch * 8);
     }
 }
 
@@ -1067,7 +1103,7 @@ __device__ __forceinline__ RowScale row_scale(const StoreTo& st, int64_t row) {
 }
 // mode 2 in whole pieces
 __device__ __forceinline__ void store_group_bf16(const f32x16& z0, const f32x16& z1, const StoreTo& st, int64_t row0,
-                                                 int64_t col0, int j, uint16_t* stage, int tid) {
+                                                 int64_t col0, int j, uint16_t* __restrict__ stage, int tid) {
     asm volatile("" : "+v"(tid));  // addresses are formed here, not ahead of the tile's main loop
     const int lane = tid & 63, wave = tid >> 6, wm = wave & 3, wn = wave >> 2;
     const int srow = wn * 32 + (lane & 31);
@@ -1075,9 +1111,9 @@ __device__ __forceinline__ void store_group_bf16(const f32x16& z0, const f32x16&
 #pragma unroll
     for (int i = 0; i < 2; ++i)
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
+        for (int p = 0; p < 2; ++p) {
             const f32x16& z = i == 0 ? z0 : z1;
-            stage_bf16x4(stage, wm, wn, lane, i, q, sc(z[q * 4]), sc(z[q * 4 + 1]), sc(z[q * 4 + 2]), sc(z[q * 4 + 3]));
+            stage_bf16x8(stage, wm, wn, lane, i, p, [&](int r) { return sc(z[r]); });
         }
     lds_barrier();
     oi_u32x4 v[GROUP_PIECES];
@@ -1096,7 +1132,7 @@ __device__ __forceinline__ void store_group_bf16(const f32x16& z0, const f32x16&
 
 // every mode, any pitch, any alignment of the element type
 __device__ __forceinline__ void store_group_f32(const f32x16& z0, const f32x16& z1, const StoreTo& st, bool pieces,
-                                                int64_t row0, int64_t col0, int j, uint16_t* stage, int tid) {
+                                                int64_t row0, int64_t col0, int j, uint16_t* __restrict__ stage, int tid) {
     asm volatile("" : "+v"(tid));
     const int lane = tid & 63, wave = tid >> 6, wm = wave & 3, wn = wave >> 2;
     const int mode = st.mode, srow = wn * 32 + (lane & 31);
@@ -1178,12 +1214,14 @@ __device__ __forceinline__ void store_tile(const AccTile& __restrict__ acc, cons
                                            uint16_t* lds) {
     const int tid = opaque_tid();
     if (t.part) {
-        store_part(acc, t.part, tid);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) store_part(tile_columns(acc, j), t.part, j, tid);
     } else if (st.mode == 2 && pieces) {
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
             __builtin_amdgcn_sched_barrier(0);
-            store_group_bf16(acc[0][j], acc[1][j], st, t.R.r0, t.C.r0, j, lds + GROUP_BF16_AT, tid);
+            const Columns c = tile_columns(acc, j);
+            store_group_bf16(c.z[0], c.z[1], st, t.R.r0, t.C.r0, j, lds + GROUP_BF16_AT, tid);
             __builtin_amdgcn_sched_barrier(0);
         }
     } else {
@@ -1192,7 +1230,8 @@ __device__ __forceinline__ void store_tile(const AccTile& __restrict__ acc, cons
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
             __builtin_amdgcn_sched_barrier(0);
-            store_group_f32(acc[0][j], acc[1][j], st, pieces, t.R.r0, t.C.r0, j, lds + (j & 1) * GROUP_F32, tid);
+            const Columns c = tile_columns(acc, j);
+            store_group_f32(c.z[0], c.z[1], st, pieces, t.R.r0, t.C.r0, j, lds + (j & 1) * GROUP_F32, tid);
             __builtin_amdgcn_sched_barrier(0);
         }
     }
@@ -1265,7 +1304,7 @@ struct ProductSizes {
 __device__ __forceinline__ ProductSizes product_sizes(int64_t M, int64_t K, int64_t m_valid, const DynRows& dyn) {
     ProductSizes z = {M, K, m_valid};
     if (dyn.n_dev) {
-        const int64_t n = *dyn.n_dev;
+        const int64_t n = device_count(dyn.n_dev);
         if (dyn.role == 1) {
             z.M = (n + BM - 1) / BM * BM;
             z.m_valid = n;
@@ -1285,13 +1324,13 @@ __global__ void __launch_bounds__(NTHREADS)
                       float* __restrict__ parts) {
     __shared__ __align__(16) uint16_t lds[LDS_ELEMS];
     if (dyn.mode_dev) {
-        mode = *dyn.mode_dev;
+        mode = device_count(dyn.mode_dev);
         if (mode < 0) return;
     }
     const ProductSizes z = product_sizes(M, K, m_valid, dyn);
     if (dyn.n_dev && dyn.role == 1) R.extent = z.M;
     if (dyn.n_dev && dyn.role == 2) {
-        const int64_t n = *dyn.n_dev;
+        const int64_t n = device_count(dyn.n_dev);
         R.k_valid = (n + BM - 1) / BM * BM;
         C.k_valid = n;
     }
@@ -1306,7 +1345,8 @@ __global__ void __launch_bounds__(NTHREADS)
     const uint32_t tiles = tiles_r * tiles_c, ktiles = (uint32_t)(K / BK);
     TailSplit ts = {tiles, 0, 1};
     if (parts) ts = plan_tail(tiles, gridDim.x, ktiles);
-    auto tile_at = [&](uint32_t item) {
+    auto tile_at = [&](uint32_t any_item) {
+        const uint32_t item = __builtin_amdgcn_readfirstlane(any_item);
         ProductTile t = {R, C, K, nullptr};
         uint32_t tile = item;
         if (item >= ts.whole) {
@@ -1447,7 +1487,7 @@ __device__ __forceinline__ void store_group_by_columns(const StoreTo& st, int64_
 
 // Column group j of a tile through the LDS region `stage`, as store_group_f32
 __device__ __forceinline__ void store_group_any(const f32x16& z0, const f32x16& z1, const StoreTo& st, int width, int64_t row0,
-                                                int64_t col0, int j, uint16_t* stage, int tid) {
+                                                int64_t col0, int j, uint16_t* __restrict__ stage, int tid) {
     asm volatile("" : "+v"(tid));
     const int lane = tid & 63, wave = tid >> 6, wm = wave & 3, wn = wave >> 2;
     const int mode = st.mode, srow = wn * 32 + (lane & 31);
@@ -1515,7 +1555,8 @@ __global__ void __launch_bounds__(NTHREADS)
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
         __builtin_amdgcn_sched_barrier(0);
-        store_group_any(acc[0][j], acc[1][j], st, width, R.r0, C.r0, j, lds + (j & 1) * GROUP_F32, tid);
+        const Columns c = tile_columns(acc, j);
+        store_group_any(c.z[0], c.z[1], st, width, R.r0, C.r0, j, lds + (j & 1) * GROUP_F32, tid);
         __builtin_amdgcn_sched_barrier(0);
     }
 }
@@ -1545,7 +1586,7 @@ __global__ void __launch_bounds__(NTHREADS)
     gemm_add_kernel(Operand R, int64_t M, Operand C, int64_t N, uint16_t* out, int64_t ldo, const int32_t* __restrict__ n_dev,
                     uint32_t* __restrict__ queue) {
     __shared__ __align__(16) uint16_t lds[LDS_ELEMS];
-    const int64_t n = *n_dev;
+    const int64_t n = device_count(n_dev);
     if (n <= 0) return;
     R.k_valid = (n + BM - 1) / BM * BM;
     C.k_valid = n;
@@ -1565,23 +1606,24 @@ __global__ void __launch_bounds__(NTHREADS)
             // what is there already is requested before the tile goes through the LDS; rows and columns past the
             // end read the last valid entries and store nothing.  N and ldo are multiples of 64, out is 4-byte aligned.
             uint32_t there[ITERS][2];
-            const int64_t c = col < N ? col : N - 4;
+            const int64_t from = col < N ? col : N - 4;
 #pragma unroll
             for (int it = 0; it < ITERS; ++it) {
                 int64_t row = group_row(R.r0, j, r_first + it * 8);
                 row = row < M ? row : M - 1;
-                const uint32_t* b = reinterpret_cast<const uint32_t*>(out + row * ldo + c);
+                const uint32_t* b = reinterpret_cast<const uint32_t*>(out + row * ldo + from);
                 there[it][0] = b[0];
                 there[it][1] = b[1];
             }
             // two regions in turn, as in store_tile
             float* stage32 = reinterpret_cast<float*>(lds + (j & 1) * GROUP_F32);
+            const Columns c = tile_columns(acc, j);
 #pragma unroll
             for (int i = 0; i < 2; ++i)
 #pragma unroll
                 for (int q = 0; q < 4; ++q)
                     *reinterpret_cast<oi_f32x4*>(stage32 + srow * STAGE_F32 + acc_row(wm, i, q * 4, lane)) =
-                        oi_f32x4{acc[i][j][q * 4], acc[i][j][q * 4 + 1], acc[i][j][q * 4 + 2], acc[i][j][q * 4 + 3]};
+                        oi_f32x4{c.z[i][q * 4], c.z[i][q * 4 + 1], c.z[i][q * 4 + 2], c.z[i][q * 4 + 3]};
             lds_barrier();
 #pragma unroll
             for (int it = 0; it < ITERS; ++it) {
@@ -1613,28 +1655,19 @@ __global__ void __launch_bounds__(NTHREADS)
     const uint32_t tile = blockIdx.x >> 2;
     const int j = blockIdx.x & 3, tid = threadIdx.x;
     if (tile >= ts.rest) return;
-    const float* src = parts + (int64_t)tile * PART_FLOATS + tid * 4;
-    oi_f32x4 sum[2][4];
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int q = 0; q < 4; ++q) sum[i][q] = *reinterpret_cast<const oi_f32x4*>(src + part_group(i, j, q) * PART_GROUP);
+    const float* src = parts + (int64_t)tile * PART_FLOATS;
+    Columns c = load_part(src, j, tid);
     for (uint32_t p = 1; p < ts.parts; ++p) {
         src += (int64_t)ts.rest * PART_FLOATS;
+        const Columns more = load_part(src, j, tid);
 #pragma unroll
         for (int i = 0; i < 2; ++i)
 #pragma unroll
-            for (int q = 0; q < 4; ++q)
-                sum[i][q] += *reinterpret_cast<const oi_f32x4*>(src + part_group(i, j, q) * PART_GROUP);
+            for (int r = 0; r < 16; ++r) c.z[i][r] += more.z[i][r];
     }
-    f32x16 acc[2];
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) acc[i][r] = sum[i][r >> 2][r & 3];
     int64_t tr, tc;
     tile_of_item(ts.whole + tile, (uint32_t)tiles_r, (uint32_t)tiles_c, &tr, &tc);
-    store_group_f32(acc[0], acc[1], st, stores_in_pieces(st), tr * BN, tc * BM, j, stage, tid);
+    store_group_f32(c.z[0], c.z[1], st, stores_in_pieces(st), tr * BN, tc * BM, j, stage, tid);
 }
 
 inline int64_t round_up(int64_t x, int64_t m) { return (x + m - 1) / m * m; }

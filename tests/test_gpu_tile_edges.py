@@ -185,3 +185,25 @@ def test_flagged_rows_are_added_to_d_weight(n, h, v, flagged, slabs):
     assert lp[:flagged].max() < -44 and (out[0].detach() - lp).abs().max() <= 1e-5 * lp.abs().max() + TOL
     _close(hid.grad, dh, "d_hidden")
     _close(w.grad, dw, "d_weight")
+
+
+@pytest.mark.parametrize("k_tiles", [1, 2, 3, 4, 5, 6, 11])  # around the ring of five slots, once and twice
+@pytest.mark.parametrize("a_km,b_km", [(0, 0), (0, 1), (1, 0), (1, 1)])
+def test_products_of_whole_numbers_are_exact(k_tiles, a_km, b_km):
+    """Entries in -4 .. 4: every sum is a whole number below 2**24, so any order of the additions gives it."""
+    for m, n in ((8, 8), (256, 264), (296, 520)):  # one fragment; one tile; ragged in both directions
+        k = 64 * k_tiles
+        print(f"case M={m} N={n} K={k} k-major {a_km} {b_km}", flush=True)
+        g = torch.Generator(device=DEV).manual_seed(m + k)
+        a = torch.randint(-4, 5, (m, k), generator=g, device=DEV).bfloat16()
+        b = torch.randint(-4, 5, (n, k), generator=g, device=DEV).bfloat16()
+        exp = (a.double() @ b.double().t()).float()
+        at = a.t().contiguous() if a_km else a
+        bt = b.t().contiguous() if b_km else b
+        out = torch.full((m, n), -1.0, device=DEV)
+        rc = _lib.load().oi_gemm_bf16_layouts(
+            at.data_ptr(), m if a_km else k, a_km, bt.data_ptr(), n if b_km else k, b_km, m, n, k, out.data_ptr(), None,
+            n, 0, torch.cuda.current_stream().cuda_stream,
+        )  # fmt: skip
+        assert rc == 0
+        assert torch.equal(out, exp)
