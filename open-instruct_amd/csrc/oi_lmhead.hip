@@ -271,9 +271,12 @@ typedef short v4i16 __attribute__((ext_vector_type(4)));
 // a uniform byte offset in scalar registers and 32 bits per lane in one vector register.  (With 64-bit lane addresses
 // the loads of a k-tile held 32 vector registers, and the compiler waited for every LDS access in flight before it used
 // any fragment, because it counts such a load among them.)  Lanes clamp their offsets onto valid rows and columns, so
-// no bounds are set; a load of a k-tile past the last one gets a buffer of no bytes and fetches nothing.
+// no bounds are set.
 //
-// A loader stands at one k-tile and moves on to the next with advance().
+// A loader stands at one k-tile and moves on to the next with advance().  Past the last one it stays there and all lanes
+// fetch the same 16 bytes, into slots that nobody reads: the waits of the loop count loads, so one has to be issued and
+// has to come back in its turn.  (A load outside the bounds of its buffer does not: it is counted off at once, ahead of
+// older loads that are still under way.)
 template <bool KM>
 struct Loader {
     const char* base;   // of the operand, for k-major of the k-tile
@@ -281,13 +284,13 @@ struct Loader {
     uint32_t off[4];    // per-lane byte offsets of the four loads
     int lds_wave;       // bytes to this wave's first load inside a slot
     int tiles_left;     // from this k-tile on, negated
-    int bytes;          // of the buffer: all there are, or none past the last k-tile
+    int live;           // all ones, or 0 past the last k-tile
     int rows_left;      // k rows from this k-tile's first on, without that one (k-major)
     static constexpr int LDS_BLOCK = KM ? 2 * 256 * 2 : 8 * BK * 2;  // bytes between the LDS destinations of loads
 
     __device__ __forceinline__ Loader(const Operand& op, int ktiles, int lane, int wave) {
         tiles_left = -ktiles;
-        bytes = -1;
+        live = -1;
         plus = 0;
         rows_left = (int)op.k_valid - 1;
         if constexpr (!KM) {
@@ -316,31 +319,35 @@ struct Loader {
         for (int b = 0; b < 4; ++b) {
             const int kk = wave * 8 + b * 2 + (lane >> 5);
             const int c = r0 + ((lane & 31) ^ (4 * (kk & 3)) ^ (2 * ((kk >> 3) & 1))) * 8;
-            off[b] = __umul24(kk < last_k ? kk : last_k, pitch(op)) + (uint32_t)((c + 8 <= extent ? c : extent - 8) * 2);
+            off[b] = (__umul24(kk < last_k ? kk : last_k, pitch(op)) + (uint32_t)((c + 8 <= extent ? c : extent - 8) * 2)) & live;
         }
     }
     __device__ __forceinline__ void advance(const Operand& op, int lane, int wave) {
         ++tiles_left;
         // in assembly, or the compiler makes a compare of it whose result it puts into a vector register
-        asm("s_ashr_i32 %0, %1, 31" : "=s"(bytes) : "s"(tiles_left) : "scc");
+        asm("s_ashr_i32 %0, %1, 31" : "=s"(live) : "s"(tiles_left) : "scc");
         if constexpr (KM) {
-            base += (int64_t)BK * 2 * op.ld;  // k rows can lie more than 32 bits apart
+            base += (int64_t)BK * 2 * op.ld & (int64_t)live;  // k rows can lie more than 32 bits apart
             rows_left -= BK;
             if (rows_left < BK - 1) set_rows(op, lane, wave);
         } else {
-            plus += BK * 2;
+            plus += BK * 2 & live;
+            if (!live) {
+#pragma unroll
+                for (int b = 0; b < 4; ++b) off[b] = 0;
+            }
         }
     }
 };
 // 16 bytes per lane from base + off (lane) + plus, 1 KB of consecutive LDS per wave
-__device__ __forceinline__ void load_to_lds(const char* base, int bytes, uint32_t off, uint32_t plus, char* to) {
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(__builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(base), 0, bytes, 0x00027000),
+__device__ __forceinline__ void load_to_lds(const char* base, uint32_t off, uint32_t plus, char* to) {
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(__builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(base), 0, -1, 0x00027000),
                                              OI_LDS_PTR(to), 16, off, plus, 0, 0);
 }
 // one 1 KB load: block b of this wave's share of an operand k-tile into the ring slot at byte offset `slot`
 template <bool KM>
 __device__ __forceinline__ void load_block(const Loader<KM>& L, int slot, int b, uint16_t* lds) {
-    load_to_lds(L.base, L.bytes, L.off[b], L.plus, reinterpret_cast<char*>(lds) + slot + L.lds_wave + b * L.LDS_BLOCK);
+    load_to_lds(L.base, L.off[b], L.plus, reinterpret_cast<char*>(lds) + slot + L.lds_wave + b * L.LDS_BLOCK);
 }
 // ring slots: A_t -> (2 t) mod 5, B_t -> (2 t + 1) mod 5
 template <bool A_KM, bool B_KM>
@@ -444,7 +451,7 @@ __device__ __forceinline__ void gemm_loop(AccTile& __restrict__ acc, const Opera
     // way; groups 0 .. 11 read the rest.  Before group 12 goes on, k-tile kt+1 must have landed (its last load was
     // issued in group 0; the 4 younger ones may stay in flight) and this wave's reads of k-tile kt must be complete:
     // after the barrier A_kt's slot is overwritten with B_(kt+2), and groups 12 .. 15 read the first fragments of
-    // k-tile kt+1 (past the last k-tile: of slots that hold nothing, for nobody).
+    // k-tile kt+1 (past the last k-tile: of slots that hold nothing of use, for nobody).
     // The scalar work of a k-tile (loaders, slots) is spread as well: in one place it is a gap between MFMAs.
     // slots of A_kt, B_kt (being read), A_(kt+1), B_(kt+1), and the one that is free all along: takes A_(kt+2)
     int s_a = 0, s_b = SLOT_BYTES, s_a1 = 2 * SLOT_BYTES, s_b1 = 3 * SLOT_BYTES, s_a2 = 4 * SLOT_BYTES;
