@@ -104,7 +104,7 @@ struct ItemQueue {
           items(items_),
           locals((uint32_t)(pids_for_items(items_) >> 3)),  // ids per queue
           xcd(blockIdx.x & 7),
-          dry(0),
+          dry(counters_ ? 0 : 8),  // without counters there is nothing to draw
           drawn(0),
           next(NONE) {
         // a kernel may run several queues one after the other over the same word: every wave must have
@@ -1089,38 +1089,64 @@ __device__ __forceinline__ bool stores_in_pieces(const StoreTo& st) {
 // and whole lines.  Registers transposed in quads of lanes and stored from there in 64-byte pieces, with a wait
 // for the stores of the tile before the next tile's first load: d_weight of 268 rows (100352 x 4096, 6272
 // tiles of 5 k-tiles) 606 us; through the LDS 544; without waiting for stores at its barriers 504; with the next tile's
-// first loads ahead of it 478.
+// first loads ahead of it 478; without waiting for each store before the next 382 (with the tile engine's other changes).
 constexpr int STAGE_F32 = BM + 4;                            // floats per row: rows 4 banks apart
 constexpr int GROUP_F32 = GROUP_ROWS * STAGE_F32 * 2;        // LDS elements of an fp32 region
 static_assert(2 * GROUP_F32 <= LDS_ELEMS, "the epilogue's regions fit the ring");
-struct RowScale {
-    float a, b;
-    bool on;
+//
+// A wave's loads and stores leave its counter in the order in which they were issued, so a load behind a group's stores
+// is not there before those have reached memory.  PLAIN products (no factors of rows, no row index) therefore have no
+// such loads in their code (behind a branch, their waits stand in everybody's way: each store of d_weight waited for the
+// one before), and what they are added to is requested one group ahead.  d_weight of 268 rows 430 -> 382 us, of 3072
+// rows (128256 x 4096) 2.22 -> 2.16 ms.
+//
+// Rows and columns past the end read what the last valid ones do, and store nothing.
+template <bool PLAIN, int PIECES>
+struct GroupRows {
+    float a, b;       // factors of the lane's accumulator row
+    int dst[PIECES];  // result rows of the thread's pieces
+
+    // srow: group row of the lane's accumulators; r_first: that of the thread's piece 0, the others `step` apart
+    __device__ __forceinline__ void request(const StoreTo& st, int64_t row0, int j, int srow, int r_first, int step) {
+        if constexpr (!PLAIN) {
+            const int64_t last = st.m_valid - 1;
+            if (st.scale_a) {
+                const int64_t row = group_row(row0, j, srow);
+                a = st.scale_a[row < last ? row : last];
+                b = st.scale_b[row < last ? row : last];
+            }
+#pragma unroll
+            for (int it = 0; it < PIECES; ++it) {
+                const int64_t row = group_row(row0, j, r_first + it * step);
+                dst[it] = (int)row;
+                if (st.mode >= 2 && st.out_rows) dst[it] = st.out_rows[row < last ? row : last];
+            }
+        }
+    }
     // a row whose factor is exactly 0 is 0 whatever its sum holds (the sums of rows that were taken out may
     // have left the fp32 range)
-    __device__ __forceinline__ float operator()(float v) const { return on ? (b == 0.f ? 0.f : v * a * b) : v; }
-};
-__device__ __forceinline__ RowScale row_scale(const StoreTo& st, int64_t row) {
-    RowScale s = {1.f, 1.f, st.scale_a != nullptr};
-    if (s.on && row < st.m_valid) {
-        s.a = st.scale_a[row];
-        s.b = st.scale_b[row];
+    __device__ __forceinline__ float scale(const StoreTo& st, float v) const {
+        return !PLAIN && st.scale_a ? (b == 0.f ? 0.f : v * a * b) : v;
     }
-    return s;
-}
+    // element offset of column col of piece it, group row r
+    __device__ __forceinline__ int64_t at(const StoreTo& st, int64_t row0, int64_t col, int j, int r, int it) const {
+        return (PLAIN ? group_row(row0, j, r) : (int64_t)dst[it]) * st.ldo + col;
+    }
+};
 // mode 2 in whole pieces
+template <bool PLAIN>
 __device__ __forceinline__ void store_group_bf16(const f32x16& z0, const f32x16& z1, const StoreTo& st, int64_t row0,
                                                  int64_t col0, int j, uint16_t* __restrict__ stage, int tid) {
     asm volatile("" : "+v"(tid));  // addresses are formed here, not ahead of the tile's main loop
     const int lane = tid & 63, wave = tid >> 6, wm = wave & 3, wn = wave >> 2;
-    const int srow = wn * 32 + (lane & 31);
-    const RowScale sc = row_scale(st, group_row(row0, j, srow));
+    GroupRows<PLAIN, GROUP_PIECES> rows;
+    rows.request(st, row0, j, wn * 32 + (lane & 31), tid >> 5, NTHREADS / 32);
 #pragma unroll
     for (int i = 0; i < 2; ++i)
 #pragma unroll
         for (int p = 0; p < 2; ++p) {
             const f32x16& z = i == 0 ? z0 : z1;
-            stage_bf16x8(stage, wm, wn, lane, i, p, [&](int r) { return sc(z[r]); });
+            stage_bf16x8(stage, wm, wn, lane, i, p, [&](int r) { return rows.scale(st, z[r]); });
         }
     lds_barrier();
     oi_u32x4 v[GROUP_PIECES];
@@ -1130,65 +1156,83 @@ __device__ __forceinline__ void store_group_bf16(const f32x16& z0, const f32x16&
     const int64_t col = col0 + (tid & 31) * 8;
 #pragma unroll
     for (int it = 0; it < GROUP_PIECES; ++it) {
-        const int64_t row = group_row(row0, j, (tid >> 5) + it * (NTHREADS / 32));
-        if (row >= st.m_valid || col >= st.N) continue;
-        const int64_t dst = st.out_rows ? (int64_t)st.out_rows[row] : row;
-        *reinterpret_cast<oi_u32x4*>(st.out_bf16 + dst * st.ldo + col) = v[it];
+        const int r = (tid >> 5) + it * (NTHREADS / 32);
+        if (group_row(row0, j, r) >= st.m_valid || col >= st.N) continue;
+        *reinterpret_cast<oi_u32x4*>(st.out_bf16 + rows.at(st, row0, col, j, r, it)) = v[it];
     }
 }
 
-// every mode, any pitch, any alignment of the element type
+// Every other mode, any pitch, any alignment of the element type.  ADDS: modes 1 and 3 in whole pieces.
+// Piece `it` of a thread is row (thread / 64) + 8 it of the group, columns 4 (thread mod 64) ..
+constexpr int F32_PIECES = GROUP_ROWS * (BM / 4) / NTHREADS;
+template <bool PLAIN, bool ADDS>
+struct F32Rows {
+    GroupRows<PLAIN, F32_PIECES> rows;
+    oi_f32x4 sum[F32_PIECES];
+
+    __device__ __forceinline__ void request(const StoreTo& st, int64_t row0, int64_t col0, int j, int tid) {
+        asm volatile("" : "+v"(tid));
+        rows.request(st, row0, j, (tid >> 8) * 32 + (tid & 31), tid >> 6, NTHREADS / 64);
+        if constexpr (ADDS) {
+            // offsets inside the tile fit 32 bits (255 rows of at most MAX_LD columns)
+            const float* tile = st.out_f32 + row0 * st.ldo + col0;
+            const int last = (int)(st.m_valid - 1 - row0 < BN - 1 ? st.m_valid - 1 - row0 : BN - 1);
+            const int c = (tid & 63) * 4, last_c = (int)(st.N - 4 - col0 < BM - 4 ? st.N - 4 - col0 : BM - 4);
+#pragma unroll
+            for (int it = 0; it < F32_PIECES; ++it) {
+                const int row = (int)group_row(0, j, (tid >> 6) + it * 8);
+                const uint32_t off = __umul24(row < last ? row : last, (uint32_t)st.ldo) + (c < last_c ? c : last_c);
+                sum[it] = *reinterpret_cast<const oi_f32x4*>(tile + off);
+            }
+        }
+    }
+};
+// `staged` is called when the accumulators are in the LDS.
+template <bool PLAIN, bool ADDS, class Staged>
 __device__ __forceinline__ void store_group_f32(const f32x16& z0, const f32x16& z1, const StoreTo& st, bool pieces,
-                                                int64_t row0, int64_t col0, int j, uint16_t* __restrict__ stage, int tid) {
+                                                const F32Rows<PLAIN, ADDS>& in, int64_t row0, int64_t col0, int j,
+                                                uint16_t* __restrict__ stage, int tid, Staged&& staged) {
     asm volatile("" : "+v"(tid));
     const int lane = tid & 63, wave = tid >> 6, wm = wave & 3, wn = wave >> 2;
     const int mode = st.mode, srow = wn * 32 + (lane & 31);
     float* stage32 = reinterpret_cast<float*>(stage);
-    constexpr int ITERS = GROUP_ROWS * (BM / 4) / NTHREADS;
-    const int ch = tid & 63, r_first = tid >> 6;  // piece `it` of a thread: row r_first + 8 it, columns 4 ch ..
+    const int ch = tid & 63, r_first = tid >> 6;
     const int64_t col = col0 + ch * 4;
-    const bool adds = pieces && (mode == 1 || mode == 3);
-    // the sum so far is requested before the tile goes through the LDS; rows and columns past the end read the last
-    // valid piece and store nothing
-    oi_f32x4 sum[ITERS];
-    if (adds) {
-        const int64_t c = col < st.N ? col : st.N - 4;
-#pragma unroll
-        for (int it = 0; it < ITERS; ++it) {
-            int64_t row = group_row(row0, j, r_first + it * 8);
-            row = row < st.m_valid ? row : st.m_valid - 1;
-            sum[it] = *reinterpret_cast<const oi_f32x4*>(st.out_f32 + row * st.ldo + c);
-        }
-    }
-    const RowScale sc = row_scale(st, group_row(row0, j, srow));
+    const auto& rows = in.rows;
 #pragma unroll
     for (int i = 0; i < 2; ++i)
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
             const f32x16& z = i == 0 ? z0 : z1;
             *reinterpret_cast<oi_f32x4*>(stage32 + srow * STAGE_F32 + acc_row(wm, i, q * 4, lane)) =
-                oi_f32x4{sc(z[q * 4]), sc(z[q * 4 + 1]), sc(z[q * 4 + 2]), sc(z[q * 4 + 3])};
+                oi_f32x4{rows.scale(st, z[q * 4]), rows.scale(st, z[q * 4 + 1]), rows.scale(st, z[q * 4 + 2]),
+                         rows.scale(st, z[q * 4 + 3])};
         }
+    __builtin_amdgcn_sched_barrier(0);
+    staged();
     lds_barrier();
     const float* from = stage32 + r_first * STAGE_F32 + ch * 4;
-    if (pieces && mode <= 1) {
+    auto piece = [&](int it) {
+        oi_f32x4 v = *reinterpret_cast<const oi_f32x4*>(from + it * 8 * STAGE_F32);
+        if constexpr (ADDS) v += in.sum[it];
+        return v;
+    };
+    if (mode <= 1 && (ADDS || pieces)) {
 #pragma unroll
-        for (int it = 0; it < ITERS; ++it) {
+        for (int it = 0; it < F32_PIECES; ++it) {
             const int64_t row = group_row(row0, j, r_first + it * 8);
-            oi_f32x4 v = *reinterpret_cast<const oi_f32x4*>(from + it * 8 * STAGE_F32);
-            if (adds) v += sum[it];
+            const oi_f32x4 v = piece(it);
             if (row < st.m_valid && col < st.N) *reinterpret_cast<oi_f32x4*>(st.out_f32 + row * st.ldo + col) = v;
         }
         return;
     }
-    if (adds) {
+    if (ADDS) {
 #pragma unroll
-        for (int it = 0; it < ITERS; ++it) {
-            const int64_t row = group_row(row0, j, r_first + it * 8);
-            const oi_f32x4 v = *reinterpret_cast<const oi_f32x4*>(from + it * 8 * STAGE_F32) + sum[it];
-            if (row >= st.m_valid || col >= st.N) continue;
-            const int64_t dst = st.out_rows ? (int64_t)st.out_rows[row] : row;
-            *reinterpret_cast<uint2*>(st.out_bf16 + dst * st.ldo + col) =
+        for (int it = 0; it < F32_PIECES; ++it) {
+            const int r = r_first + it * 8;
+            const oi_f32x4 v = piece(it);
+            if (group_row(row0, j, r) >= st.m_valid || col >= st.N) continue;
+            *reinterpret_cast<uint2*>(st.out_bf16 + rows.at(st, row0, col, j, r, it)) =
                 make_uint2(oi_pack_bf16x2(v.x, v.y), oi_pack_bf16x2(v.z, v.w));
         }
         return;
@@ -1196,7 +1240,7 @@ __device__ __forceinline__ void store_group_f32(const f32x16& z0, const f32x16& 
     // bf16 rows off 8-byte boundaries
     if (col >= st.N) return;
 #pragma unroll 1
-    for (int it = 0; it < ITERS; ++it) {
+    for (int it = 0; it < F32_PIECES; ++it) {
         const int64_t row = group_row(row0, j, r_first + it * 8);
         if (row >= st.m_valid) break;
         oi_f32x4 v = *reinterpret_cast<const oi_f32x4*>(from + it * 8 * STAGE_F32);
@@ -1206,6 +1250,8 @@ __device__ __forceinline__ void store_group_f32(const f32x16& z0, const f32x16& 
         b[1] = oi_pack_bf16x2(v.z, v.w);
     }
 }
+__device__ __forceinline__ bool plain_rows(const StoreTo& st) { return !st.scale_a && !(st.mode >= 2 && st.out_rows); }
+__device__ __forceinline__ bool adds_in_pieces(const StoreTo& st, bool pieces) { return pieces && (st.mode == 1 || st.mode == 3); }
 
 // out[row, col] = sum_k R(row, k) * C(col, k).  R's rows (token or vocabulary rows of the result) are the tile
 // product's n dimension and C's (the result's columns) its m dimension, because a lane's consecutive
@@ -1216,6 +1262,42 @@ struct ProductTile {
     int64_t K;
     float* part;
 };
+// all but mode 2 in whole pieces: two regions in turn; one is written again only after the barrier of the group in
+// between, by which every wave has read it out
+template <bool PLAIN, bool ADDS>
+__device__ __forceinline__ void store_tile_f32(const AccTile& acc, const ProductTile& t, const StoreTo& st, bool pieces,
+                                               uint16_t* lds, int tid) {
+    constexpr bool AHEAD = PLAIN && ADDS;
+    F32Rows<PLAIN, ADDS> in[2];
+    if (AHEAD) in[0].request(st, t.R.r0, t.C.r0, 0, tid);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        __builtin_amdgcn_sched_barrier(0);
+        if (!AHEAD) in[j & 1].request(st, t.R.r0, t.C.r0, j, tid);
+        const Columns c = tile_columns(acc, j);
+        store_group_f32<PLAIN, ADDS>(c.z[0], c.z[1], st, pieces, in[j & 1], t.R.r0, t.C.r0, j, lds + (j & 1) * GROUP_F32, tid, [&] {
+            if (AHEAD && j < 3) in[(j + 1) & 1].request(st, t.R.r0, t.C.r0, j + 1, tid);
+        });
+        __builtin_amdgcn_sched_barrier(0);
+    }
+}
+template <bool PLAIN>
+__device__ __forceinline__ void store_tile_as(const AccTile& acc, const ProductTile& t, const StoreTo& st, bool pieces,
+                                              uint16_t* lds, int tid) {
+    if (st.mode == 2 && pieces) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            __builtin_amdgcn_sched_barrier(0);
+            const Columns c = tile_columns(acc, j);
+            store_group_bf16<PLAIN>(c.z[0], c.z[1], st, t.R.r0, t.C.r0, j, lds + GROUP_BF16_AT, tid);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    } else if (adds_in_pieces(st, pieces)) {
+        store_tile_f32<PLAIN, true>(acc, t, st, pieces, lds, tid);
+    } else {
+        store_tile_f32<PLAIN, false>(acc, t, st, pieces, lds, tid);
+    }
+}
 // In mode 2 with whole pieces this leaves the ring slots 0 .. 3 alone.
 __device__ __forceinline__ void store_tile(const AccTile& __restrict__ acc, const ProductTile& t, const StoreTo& st, bool pieces,
                                            uint16_t* lds) {
@@ -1223,24 +1305,10 @@ __device__ __forceinline__ void store_tile(const AccTile& __restrict__ acc, cons
     if (t.part) {
 #pragma unroll
         for (int j = 0; j < 4; ++j) store_part(tile_columns(acc, j), t.part, j, tid);
-    } else if (st.mode == 2 && pieces) {
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            __builtin_amdgcn_sched_barrier(0);
-            const Columns c = tile_columns(acc, j);
-            store_group_bf16(c.z[0], c.z[1], st, t.R.r0, t.C.r0, j, lds + GROUP_BF16_AT, tid);
-            __builtin_amdgcn_sched_barrier(0);
-        }
+    } else if (plain_rows(st)) {
+        store_tile_as<true>(acc, t, st, pieces, lds, tid);
     } else {
-        // two regions in turn: one is written again only after the barrier of the group in between, by which
-        // every wave has read it out
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            __builtin_amdgcn_sched_barrier(0);
-            const Columns c = tile_columns(acc, j);
-            store_group_f32(c.z[0], c.z[1], st, pieces, t.R.r0, t.C.r0, j, lds + (j & 1) * GROUP_F32, tid);
-            __builtin_amdgcn_sched_barrier(0);
-        }
+        store_tile_as<false>(acc, t, st, pieces, lds, tid);
     }
 }
 // a product without terms (no rows selected): zeros, or what the earlier launches summed up
@@ -1374,15 +1442,6 @@ __global__ void __launch_bounds__(NTHREADS)
         t.C.r0 = tc * BM;
         return t;
     };
-    if (!queue) {
-        const uint32_t item = item_of_pid(blockIdx.x, tiles);
-        if (item >= tiles) return;
-        const ProductTile t = tile_at(item);
-        AccTile acc;
-        gemm_tile<C_KM, R_KM>(acc, t.C, t.R, t.K, lds);
-        store_tile(acc, t, st, pieces, lds);
-        return;
-    }
     // Whole bf16 pieces leave through slot 4 while the next tile's first loads go to slots 0 .. 3: a tile of
     // few k-tiles (d_weight of a short batch) otherwise spends more time between its main loops than in them.
     // The fp32 modes need more LDS than one slot and belong to batches of several slabs, whose tiles are long.
@@ -1390,8 +1449,8 @@ __global__ void __launch_bounds__(NTHREADS)
     ItemQueue q(queue, ts.whole + ts.rest * ts.parts, lds);
     q.request();
     q.settle();
-    uint32_t item = q.take_item();
-    if (item == ItemQueue::NONE) return;
+    uint32_t item = queue ? q.take_item() : item_of_pid(blockIdx.x, tiles);
+    if (item >= q.items) return;
     ProductTile t = tile_at(item);
     begin_loads<C_KM, R_KM>(t.C, t.R, t.K, lds);
     for (;;) {
@@ -1399,23 +1458,19 @@ __global__ void __launch_bounds__(NTHREADS)
         q.request();
         gemm_loop<C_KM, R_KM>(acc, t.C, t.R, t.K, lds);
         q.settle();
-        if (!ahead) {
-            store_tile(acc, t, st, pieces, lds);
-            item = q.take_item();
-            if (item == ItemQueue::NONE) return;
-            t = tile_at(item);
-            begin_loads<C_KM, R_KM>(t.C, t.R, t.K, lds);
-            continue;
-        }
         item = q.take_item();
         const ProductTile done = t;
         if (item != ItemQueue::NONE) {
             t = tile_at(item);
-            begin_loads<C_KM, R_KM>(t.C, t.R, t.K, lds);
+            if (ahead) begin_loads<C_KM, R_KM>(t.C, t.R, t.K, lds);
         }
         lds_barrier();  // every wave has read the queue's word, which lies in slot 4
         store_tile(acc, done, st, pieces, lds);
         if (item == ItemQueue::NONE) return;
+        if (!ahead) {
+            lds_barrier();
+            begin_loads<C_KM, R_KM>(t.C, t.R, t.K, lds);
+        }
     }
 }
 
@@ -1674,7 +1729,17 @@ __global__ void __launch_bounds__(NTHREADS)
     }
     int64_t tr, tc;
     tile_of_item(ts.whole + tile, (uint32_t)tiles_r, (uint32_t)tiles_c, &tr, &tc);
-    store_group_f32(c.z[0], c.z[1], st, stores_in_pieces(st), tr * BN, tc * BM, j, stage, tid);
+    const bool pieces = stores_in_pieces(st);
+    const int64_t row0 = tr * BN, col0 = tc * BM;
+    if (adds_in_pieces(st, pieces)) {
+        F32Rows<false, true> in;
+        in.request(st, row0, col0, j, tid);
+        store_group_f32<false, true>(c.z[0], c.z[1], st, pieces, in, row0, col0, j, stage, tid, [] {});
+    } else {
+        F32Rows<false, false> in;
+        in.request(st, row0, col0, j, tid);
+        store_group_f32<false, false>(c.z[0], c.z[1], st, pieces, in, row0, col0, j, stage, tid, [] {});
+    }
 }
 
 inline int64_t round_up(int64_t x, int64_t m) { return (x + m - 1) / m * m; }
