@@ -192,6 +192,8 @@ __device__ __forceinline__ void wait_loads_and_barrier() {
 
 // Meets the other waves once this wave's LDS accesses are done.  __syncthreads() also waits for every global
 // store and load of the wave, which in an epilogue is the round trip of its stores at each barrier.
+// No pointer to a region that is handed over at a barrier is `__restrict__`: nothing but its own accesses would
+// touch the region then, and a read whose value is first used in a branch behind the barrier is moved there.
 __device__ __forceinline__ void lds_barrier() {
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     __builtin_amdgcn_s_barrier();
@@ -710,7 +712,7 @@ __device__ __forceinline__ FwdColumn fwd_column(const FwdArgs& a, const float* x
 // exponentials (through `stage`; every thread of the workgroup takes part).
 template <FwdKeep KEEP>
 __device__ __forceinline__ void fwd_fold(f32x16 (&__restrict__ z)[2], FwdColumn& col, const FwdArgs& a, const FwdLaunch& fl,
-                                         int64_t vt, int64_t n0, int j, int tid, uint16_t* __restrict__ stage) {
+                                         int64_t vt, int64_t n0, int j, int tid, uint16_t* stage) {
     constexpr bool CACHE = KEEP == FWD_EXPONENTIALS;
     asm volatile("" : "+v"(tid));  // addresses are formed here, not ahead of the tile's main loop
     const int lane = tid & 63, wave = tid >> 6, wm = wave & 3, wn = wave >> 2;
@@ -1136,7 +1138,7 @@ struct GroupRows {
 // mode 2 in whole pieces
 template <bool PLAIN>
 __device__ __forceinline__ void store_group_bf16(const f32x16& z0, const f32x16& z1, const StoreTo& st, int64_t row0,
-                                                 int64_t col0, int j, uint16_t* __restrict__ stage, int tid) {
+                                                 int64_t col0, int j, uint16_t* stage, int tid) {
     asm volatile("" : "+v"(tid));  // addresses are formed here, not ahead of the tile's main loop
     const int lane = tid & 63, wave = tid >> 6, wm = wave & 3, wn = wave >> 2;
     GroupRows<PLAIN, GROUP_PIECES> rows;
@@ -1191,7 +1193,7 @@ struct F32Rows {
 template <bool PLAIN, bool ADDS, class Staged>
 __device__ __forceinline__ void store_group_f32(const f32x16& z0, const f32x16& z1, const StoreTo& st, bool pieces,
                                                 const F32Rows<PLAIN, ADDS>& in, int64_t row0, int64_t col0, int j,
-                                                uint16_t* __restrict__ stage, int tid, Staged&& staged) {
+                                                uint16_t* stage, int tid, Staged&& staged) {
     asm volatile("" : "+v"(tid));
     const int lane = tid & 63, wave = tid >> 6, wm = wave & 3, wn = wave >> 2;
     const int mode = st.mode, srow = wn * 32 + (lane & 31);
@@ -1549,7 +1551,7 @@ __device__ __forceinline__ void store_group_by_columns(const StoreTo& st, int64_
 
 // Column group j of a tile through the LDS region `stage`, as store_group_f32
 __device__ __forceinline__ void store_group_any(const f32x16& z0, const f32x16& z1, const StoreTo& st, int width, int64_t row0,
-                                                int64_t col0, int j, uint16_t* __restrict__ stage, int tid) {
+                                                int64_t col0, int j, uint16_t* stage, int tid) {
     asm volatile("" : "+v"(tid));
     const int lane = tid & 63, wave = tid >> 6, wm = wave & 3, wn = wave >> 2;
     const int mode = st.mode, srow = wn * 32 + (lane & 31);

@@ -207,3 +207,21 @@ def test_products_of_whole_numbers_are_exact(k_tiles, a_km, b_km):
         )  # fmt: skip
         assert rc == 0
         assert torch.equal(out, exp)
+
+
+@pytest.mark.parametrize("n", [64, 65, 128, 129, 192, 193, 256, 320, 321])  # last rows of each group of 64 token rows and the first of the next
+@pytest.mark.parametrize("keep_logits", [True, False])
+def test_last_tile_of_token_rows(n, keep_logits):
+    h, v = 192, 700  # three k-tiles, a ragged vocabulary tile; one tile of d_hidden columns, short of its last group
+    print(f"case N={n} keep_logits={keep_logits}", flush=True)
+    hidden, weight, labels, _, upstream = _inputs(n, h, v, seed=n)
+    lp, dh, dw = _reference(hidden, weight, labels, torch.ones_like(labels, dtype=torch.bool), upstream)
+    for frozen in (False, True):  # logits or statistics alone; kept exponentials and their weighted sum
+        hid, w = hidden.clone().requires_grad_(True), weight.clone().requires_grad_(not frozen)
+        out = lm_head.fused_lm_head_logprobs(hid, w, labels, keep_logits=keep_logits)
+        out = out[0] if isinstance(out, tuple) else out
+        assert (out.detach() - lp).abs().max().item() <= TOL
+        out.backward(upstream)
+        _close(hid.grad, dh, "d_hidden")
+        if not frozen:
+            _close(w.grad, dw, "d_weight")
