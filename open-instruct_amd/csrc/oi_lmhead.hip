@@ -37,7 +37,11 @@ constexpr int STAGE_STRIDE = 256 + 8;           // bf16 per row of the dZ stagin
 constexpr int LDS_ELEMS = 5 * TILE_ELEMS;       // 163840 B: the five-slot operand ring, all of a CU's LDS
 static_assert(256 * STAGE_STRIDE <= LDS_ELEMS, "the dZ staging tile must fit");
 
-typedef f32x4 AccTile[4][8];
+// A workgroup's tile is 256 (m) x 32 NJ (n): each wave 64 x 16 NJ, NJ column tiles.  NJ is 8, or less for the last tile
+// of token rows of a forward pass (tile_width).
+constexpr int WIDE = 8;
+template <int NJ = WIDE>
+using AccTile = f32x4[4][NJ];
 
 // XCD-aware tile order.  Consecutive workgroup ids go round-robin to the 8 XCDs, each with its own
 // L2.  The tiles of a launch are numbered in bands of 8 rows, n outermost inside a band, so that 32
@@ -279,11 +283,12 @@ typedef short v4i16 __attribute__((ext_vector_type(4)));
 // fetch the same 16 bytes, into slots that nobody reads: the waits of the loop count loads, so one has to be issued and
 // has to come back in its turn.  (A load outside the bounds of its buffer does not: it is counted off at once, ahead of
 // older loads that are still under way.)
-template <bool KM>
+template <bool KM, int LOADS>
 struct Loader {
+    static_assert(LOADS == 4 || !KM, "k-major operands are whole tiles");
     const char* base;   // of the operand, for k-major of the k-tile
     uint32_t plus;      // bytes from there to the k-tile (k-contiguous)
-    uint32_t off[4];    // per-lane byte offsets of the four loads
+    uint32_t off[LOADS];  // per-lane byte offsets of the loads
     int lds_wave;       // bytes to this wave's first load inside a slot
     int tiles_left;     // from this k-tile on, negated
     int live;           // all ones, or 0 past the last k-tile
@@ -299,16 +304,16 @@ struct Loader {
             base = reinterpret_cast<const char*>(op.p + op.r0 * op.ld);
             const int last_row = (int)((op.extent - 1 - op.r0) < 255 ? (op.extent - 1 - op.r0) : 255);
 #pragma unroll
-            for (int b = 0; b < 4; ++b) {
-                const int r = wave * 32 + b * 8 + (lane >> 3);
+            for (int b = 0; b < LOADS; ++b) {
+                const int r = (wave * LOADS + b) * 8 + (lane >> 3);
                 const int c = (lane & 7) ^ swz(r);
                 off[b] = __umul24(r < last_row ? r : last_row, pitch(op)) + c * 16;
             }
-            lds_wave = wave * 32 * BK * 2;
+            lds_wave = wave * LOADS * LDS_BLOCK;
         } else {
             base = reinterpret_cast<const char*>(op.p);
             set_rows(op, lane, wave);
-            lds_wave = wave * 8 * 256 * 2;
+            lds_wave = wave * LOADS * LDS_BLOCK;
         }
     }
     // at most 2^23; rows inside a tile are at most 255
@@ -336,7 +341,7 @@ struct Loader {
             plus += BK * 2 & live;
             if (!live) {
 #pragma unroll
-                for (int b = 0; b < 4; ++b) off[b] = 0;
+                for (int b = 0; b < LOADS; ++b) off[b] = 0;
             }
         }
     }
@@ -347,44 +352,46 @@ __device__ __forceinline__ void load_to_lds(const char* base, uint32_t off, uint
                                              OI_LDS_PTR(to), 16, off, plus, 0, 0);
 }
 // one 1 KB load: block b of this wave's share of an operand k-tile into the ring slot at byte offset `slot`
-template <bool KM>
-__device__ __forceinline__ void load_block(const Loader<KM>& L, int slot, int b, uint16_t* lds) {
+template <bool KM, int LOADS>
+__device__ __forceinline__ void load_block(const Loader<KM, LOADS>& L, int slot, int b, uint16_t* lds) {
     load_to_lds(L.base, L.off[b], L.plus, reinterpret_cast<char*>(lds) + slot + L.lds_wave + b * L.LDS_BLOCK);
 }
 // ring slots: A_t -> (2 t) mod 5, B_t -> (2 t + 1) mod 5
-template <bool A_KM, bool B_KM>
+template <bool A_KM, bool B_KM, int NJ = WIDE>
 __device__ __forceinline__ void begin_loads(const Operand& A_, const Operand& B_, int64_t K, uint16_t* lds) {
     const Operand A = scalar(A_), B = scalar(B_);
     const int tid = opaque_tid();
     // the wave index as a scalar: the LDS destinations of the loads (M0) then take no VALU work
     const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int ktiles = __builtin_amdgcn_readfirstlane((int)(K / BK));
-    Loader<A_KM> la(A, ktiles, lane, wave);
-    Loader<B_KM> lb(B, ktiles, lane, wave);
+    constexpr int B_LOADS = NJ / 2;
+    Loader<A_KM, 4> la(A, ktiles, lane, wave);
+    Loader<B_KM, B_LOADS> lb(B, ktiles, lane, wave);
 #pragma unroll
     for (int b = 0; b < 4; ++b) load_block(la, 0, b, lds);
 #pragma unroll
-    for (int b = 0; b < 4; ++b) load_block(lb, SLOT_BYTES, b, lds);
+    for (int b = 0; b < B_LOADS; ++b) load_block(lb, SLOT_BYTES, b, lds);
     la.advance(A, lane, wave);
     lb.advance(B, lane, wave);
 #pragma unroll
     for (int b = 0; b < 4; ++b) load_block(la, 2 * SLOT_BYTES, b, lds);
 #pragma unroll
-    for (int b = 0; b < 3; ++b) load_block(lb, 3 * SLOT_BYTES, b, lds);
+    for (int b = 0; b < B_LOADS - 1; ++b) load_block(lb, 3 * SLOT_BYTES, b, lds);
 }
 
 // `__restrict__` here and in store_tile is what tells the compiler that the LDS accesses of these functions carry
 // alias information; without any it waits for every global->LDS load in flight before each LDS access
 // (d_weight of 3072 rows: 2.7 -> 4.9 ms).
-template <bool A_KM, bool B_KM>
-__device__ __forceinline__ void gemm_loop(AccTile& __restrict__ acc, const Operand& A_, const Operand& B_, int64_t K, uint16_t* lds) {
+template <bool A_KM, bool B_KM, int NJ>
+__device__ __forceinline__ void gemm_loop(AccTile<NJ>& __restrict__ acc, const Operand& A_, const Operand& B_, int64_t K, uint16_t* lds) {
     const Operand A = scalar(A_), B = scalar(B_);
     const int tid = opaque_tid();
     const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wm = wave & 3, wn = wave >> 2;
     const int ktiles = __builtin_amdgcn_readfirstlane((int)(K / BK));
-    Loader<A_KM> la(A, ktiles, lane, wave);  // at k-tile kt+2
-    Loader<B_KM> lb(B, ktiles, lane, wave);  // at k-tile kt+1 in group 0, kt+2 from group 12 on
+    constexpr int B_LOADS = NJ / 2;
+    Loader<A_KM, 4> la(A, ktiles, lane, wave);        // at k-tile kt+2
+    Loader<B_KM, B_LOADS> lb(B, ktiles, lane, wave);  // at k-tile kt+1 in group 0, kt+2 behind the barrier
     la.advance(A, lane, wave);
     la.advance(A, lane, wave);
     lb.advance(B, lane, wave);
@@ -392,7 +399,7 @@ __device__ __forceinline__ void gemm_loop(AccTile& __restrict__ acc, const Opera
 #pragma unroll
     for (int i = 0; i < 4; ++i)
 #pragma unroll
-        for (int j = 0; j < 8; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+        for (int j = 0; j < NJ; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
 
     // consumer side: byte offsets of this lane's fragments inside a slot; a lane holds row lr of a 16-row
     // fragment at the k values 8 g .. 8 g + 7 of a k-step
@@ -400,7 +407,7 @@ __device__ __forceinline__ void gemm_loop(AccTile& __restrict__ acc, const Opera
     // k-contiguous image: the second k-step flips bit 2 of the stored chunk; rows 16 apart share the same
     // permutation
     const int pg = (g ^ swz(lr)) * 16;
-    const int a_base = (wm * 64 + lr) * (BK * 2) + pg, b_base = (wn * 128 + lr) * (BK * 2) + pg;
+    const int a_base = (wm * 64 + lr) * (BK * 2) + pg, b_base = (wn * 16 * NJ + lr) * (BK * 2) + pg;
     // k-major image: source lane lr of a 16-lane group points at k row (lr >> 2) of the group's 8 and at 4
     // columns from 4 (lr & 3) of the fragment's 16; fragments are two chunks apart, which flips the chunk bits
     // that the permutation reaches
@@ -426,14 +433,14 @@ __device__ __forceinline__ void gemm_loop(AccTile& __restrict__ acc, const Opera
         else return *reinterpret_cast<const bf16x8*>(ring + slot + (b_base ^ (ks * 64)) + j * 16 * (BK * 2));
     };
 
-    // A k-tile is two k-steps of 32, each eight groups of four MFMAs: group u of the sixteen multiplies B fragment
-    // u (u mod 8 of its k-step) with the four A fragments, up and down in turn, so that one operand of an MFMA is
-    // always that of the one before (power is what limits the loop).  A fragments have two sets of registers, B
-    // fragments a ring of eight; the 24 fragment reads and the 8 global->LDS loads stand one by one between the
-    // MFMAs.  Nothing may move across the scheduling barriers: loads issued back to back hold up the wave's MFMA
-    // issue, and a fragment read issued ahead of the MFMAs before it would be waited for together with the
-    // current fragments (a full LDS round trip with the matrix pipe idle).
-    bf16x8 a[2][4], b[16];
+    // A k-tile is two k-steps of 32, each NJ groups of four MFMAs: group u of the 2 NJ multiplies B fragment
+    // u (u mod NJ of its k-step) with the four A fragments, up and down in turn, so that one operand of an MFMA is
+    // always that of the one before (power is what limits the loop).  The fragment reads and the global->LDS loads (24
+    // and 8 of a wide tile) stand one by one between the MFMAs.  Nothing may move across the scheduling barriers: loads
+    // issued back to back hold up the wave's MFMA issue, and a fragment read issued ahead of the MFMAs before it would
+    // be waited for together with the current fragments (a full LDS round trip with the matrix pipe idle).
+    constexpr int GROUPS = 2 * NJ, BARRIER = NJ == 2 ? 2 : GROUPS * 3 / 4;
+    bf16x8 a[2][4], b[GROUPS];
     // A_0 and B_0 must have landed.  The wait is for everything in flight, not for "all but the 7
     // younger loads": a workgroup that runs several tiles may still have the previous tile's
     // stores outstanding, and stores complete out of order with loads.
@@ -445,14 +452,14 @@ __device__ __forceinline__ void gemm_loop(AccTile& __restrict__ acc, const Opera
     }
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-        b[j] = read_b(SLOT_BYTES, 0, j);
+        b[j] = read_b(SLOT_BYTES, j / NJ, j % NJ);
         __builtin_amdgcn_sched_barrier(0);
     }
 
     // Fragments: at the start of a k-tile the A fragments of the first k-step and B fragments 0 .. 3 are there or under
-    // way; groups 0 .. 11 read the rest.  Before group 12 goes on, k-tile kt+1 must have landed (its last load was
+    // way; the groups ahead of the barrier read the rest.  At the barrier k-tile kt+1 must have landed (its last load was
     // issued in group 0; the 4 younger ones may stay in flight) and this wave's reads of k-tile kt must be complete:
-    // after the barrier A_kt's slot is overwritten with B_(kt+2), and groups 12 .. 15 read the first fragments of
+    // behind it A_kt's slot is overwritten with B_(kt+2), and the last quarter of the groups reads the first fragments of
     // k-tile kt+1 (past the last k-tile: of slots that hold nothing of use, for nobody).
     // The scalar work of a k-tile (loaders, slots) is spread as well: in one place it is a gap between MFMAs.
     // slots of A_kt, B_kt (being read), A_(kt+1), B_(kt+1), and the one that is free all along: takes A_(kt+2)
@@ -460,33 +467,57 @@ __device__ __forceinline__ void gemm_loop(AccTile& __restrict__ acc, const Opera
 #pragma unroll 1
     for (int left = ktiles; left > 0; --left) {
 #pragma unroll
-        for (int u = 0; u < 16; ++u) {
+        for (int u = 0; u < GROUPS; ++u) {
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
-                const int i = (u & 1) ? 3 - q : q, j = u & 7;
-                acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[u >> 3][i], b[u], acc[i][j], 0, 0, 0);
+                const int i = (u & 1) ? 3 - q : q, j = u % NJ;
+                acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[u / NJ][i], b[u], acc[i][j], 0, 0, 0);
                 __builtin_amdgcn_sched_barrier(0);
-                if (u == 12 && q == 1) {
+                if (u == BARRIER && q == 1) {
                     asm volatile("s_waitcnt vmcnt(4) lgkmcnt(0)" ::: "memory");
                     __builtin_amdgcn_s_barrier();
                     asm volatile("" ::: "memory");
                 }
                 // one of the loads, as evenly spread as the slot hand-over allows
-                if (u == 0 && q == 1) load_block(lb, s_b1, 3, lds);
-                if ((u == 2 || u == 5 || u == 7 || u == 10) && q == 1) load_block(la, s_a2, u == 2 ? 0 : u == 5 ? 1 : u == 7 ? 2 : 3, lds);
-                if ((u == 12 || u == 13) && q == 3) load_block(lb, s_a, u - 12, lds);
-                if (u == 15 && q == 1) load_block(lb, s_a, 2, lds);
-                if (u == 11 && q == 2) la.advance(A, lane, wave);
-                if (u == 10 && q == 2) lb.advance(B, lane, wave);
+                if (u == 0 && q == 1) load_block(lb, s_b1, B_LOADS - 1, lds);
+                if constexpr (NJ == 8) {
+                    if ((u == 2 || u == 5 || u == 7 || u == 10) && q == 1) load_block(la, s_a2, u == 2 ? 0 : u == 5 ? 1 : u == 7 ? 2 : 3, lds);
+                    if ((u == 12 || u == 13) && q == 3) load_block(lb, s_a, u - 12, lds);
+                    if (u == 15 && q == 1) load_block(lb, s_a, 2, lds);
+                } else if constexpr (NJ == 6) {
+                    if (u < 8 && u % 2 == 1 && q == 1) load_block(la, s_a2, u / 2, lds);
+                    if (u >= 10 && q == 1) load_block(lb, s_a, u - 10, lds);
+                } else if constexpr (NJ == 4) {
+                    if (u >= 1 && u <= 4 && q == 1) load_block(la, s_a2, u - 1, lds);
+                    if (u == 7 && q == 0) load_block(lb, s_a, 0, lds);
+                } else {
+                    if (u == 0 && q >= 2) load_block(la, s_a2, q - 2, lds);
+                    if (u == 1 && (q == 0 || q == 2)) load_block(la, s_a2, 2 + q / 2, lds);
+                }
+                if (u == (NJ == 2 ? 2 : BARRIER - 1) && q == 2) la.advance(A, lane, wave);
+                if (u == (NJ == 2 ? 1 : BARRIER - 2) && q == 2) lb.advance(B, lane, wave);
                 // fragments
-                if (u < 12 && q == 0) b[u + 4] = read_b(s_b, (u + 4) >> 3, (u + 4) & 7);
-                if (u >= 2 && u < 6 && q == 2) a[1][u - 2] = read_a(s_a, 1, u - 2);
-                if (u == 12 && q >= 1) a[0][q - 1] = read_a(s_a1, 0, q - 1);
-                if (u == 13 && q == 0) a[0][3] = read_a(s_a1, 0, 3);
-                if (u == 13 && q >= 1 && q <= 2) b[q - 1] = read_b(s_b1, 0, q - 1);
-                if (u == 14 && q == 1) b[2] = read_b(s_b1, 0, 2);
-                if (u == 15 && q == 0) b[3] = read_b(s_b1, 0, 3);
-                if (u == 15 && q == 2) {
+                if (u < BARRIER && u + 4 < GROUPS && q == 0) b[u + 4] = read_b(s_b, (u + 4) / NJ, (u + 4) % NJ);
+                if constexpr (NJ >= 6) {
+                    if (u >= NJ / 4 && u < NJ / 4 + 4 && q == 2) a[1][u - NJ / 4] = read_a(s_a, 1, u - NJ / 4);
+                } else if constexpr (NJ == 4) {
+                    if (u < 2 && q >= 2) a[1][2 * u + q - 2] = read_a(s_a, 1, 2 * u + q - 2);
+                } else {
+                    if (u == 0) a[1][q] = read_a(s_a, 1, q);
+                }
+                if constexpr (NJ == 2) {
+                    if (u == 2 && q >= 1) a[0][q - 1] = read_a(s_a1, 0, q - 1);
+                    if (u == 3 && q == 0) a[0][3] = read_a(s_a1, 0, 3);
+                    if (u == 3 && q >= 1) b[q - 1] = read_b(s_b1, (q - 1) / NJ, (q - 1) % NJ);
+                    if (u == 3 && q == 3) b[3] = read_b(s_b1, 1, 1);
+                } else {
+                    if (u == BARRIER && q >= 1) a[0][q - 1] = read_a(s_a1, 0, q - 1);
+                    if (u == BARRIER + 1 && q == 0) a[0][3] = read_a(s_a1, 0, 3);
+                    if (u == BARRIER + 1 && q >= 1 && q <= 2) b[q - 1] = read_b(s_b1, 0, q - 1);
+                    if (u == (NJ >= 6 ? BARRIER + 2 : BARRIER + 1) && q == (NJ >= 6 ? 1 : 3)) b[2] = read_b(s_b1, 0, 2);
+                    if (u == GROUPS - 1 && q == (NJ == 8 ? 0 : 3)) b[3] = read_b(s_b1, 0, 3);
+                }
+                if (u == GROUPS - 1 && q == 3) {
                     const int was_a = s_a, was_b = s_b;
                     s_a = s_a1;
                     s_b = s_b1;
@@ -504,12 +535,12 @@ __device__ __forceinline__ void gemm_loop(AccTile& __restrict__ acc, const Opera
     asm volatile("" ::: "memory");
 }
 template <bool A_KM, bool B_KM>
-__device__ __forceinline__ void gemm_tile(AccTile& acc, const Operand& A, const Operand& B, int64_t K, uint16_t* lds) {
+__device__ __forceinline__ void gemm_tile(AccTile<>& acc, const Operand& A, const Operand& B, int64_t K, uint16_t* lds) {
     begin_loads<A_KM, B_KM>(A, B, K, lds);
     gemm_loop<A_KM, B_KM>(acc, A, B, K, lds);
 }
 // both operands k-contiguous: C[m, n] = sum_k A[m0 + m, k] * B[n0 + n, k]
-__device__ __forceinline__ void gemm_tile(AccTile& acc, const uint16_t* __restrict__ A, int64_t lda, int64_t m0,
+__device__ __forceinline__ void gemm_tile(AccTile<>& acc, const uint16_t* __restrict__ A, int64_t lda, int64_t m0,
                                           int64_t M, const uint16_t* __restrict__ B, int64_t ldb, int64_t n0,
                                           int64_t N, int64_t K, uint16_t* lds) {
     const Operand a = {A, lda, m0, M, K}, b = {B, ldb, n0, N, K};
@@ -517,11 +548,11 @@ __device__ __forceinline__ void gemm_tile(AccTile& acc, const uint16_t* __restri
 }
 
 // An MFMA leaves lane l with rows 4 (l / 16) .. + 3 of column l % 16 of a 16 x 16 tile (acc[i][j]: rows 16 i, columns
-// 16 j of the wave's 64 x 128).  The epilogues take column groups of 32: swapping the odd quarters of the lanes of one
+// 16 j of the wave's 64 x 16 NJ).  The epilogues take column groups of 32: swapping the odd quarters of the lanes of one
 // column tile with the even ones of the next gives a lane one column and eight consecutive rows of every 16.
 // Element (i, r) of lane `lane` of column group j is then
 //   m (row, vocabulary in the logits kernels) = wm*64 + i*32 + (r/8)*16 + (lane/32)*8 + r%8
-//   n (column, token in the logits kernels)   = wn*128 + j*32 + lane%32
+//   n (column, token in the logits kernels)   = wn*16*NJ + j*32 + lane%32
 __device__ __forceinline__ void swap_quarters(const f32x4& x, const f32x4& y, f32x16& z, int r0) {
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
@@ -534,7 +565,8 @@ __device__ __forceinline__ void swap_quarters(const f32x4& x, const f32x4& y, f3
 struct Columns {
     f32x16 z[2];  // not an array of floats: the search for the label's register would put that into memory
 };
-__device__ __forceinline__ Columns tile_columns(const AccTile& acc, int j) {
+template <int NJ>
+__device__ __forceinline__ Columns tile_columns(const AccTile<NJ>& acc, int j) {
     Columns c;
 #pragma unroll
     for (int i = 0; i < 4; ++i) swap_quarters(acc[i][2 * j], acc[i][2 * j + 1], c.z[i >> 1], (i & 1) * 8);
@@ -543,7 +575,33 @@ __device__ __forceinline__ Columns tile_columns(const AccTile& acc, int j) {
 __device__ __forceinline__ int acc_row(int wm, int i, int r, int lane) {
     return wm * 64 + i * 32 + (r >> 3) * 16 + (lane >> 5) * 8 + (r & 7);
 }
-__device__ __forceinline__ int acc_col(int wn, int j, int lane) { return wn * 128 + j * 32 + (lane & 31); }
+template <int NJ = WIDE>
+__device__ __forceinline__ int acc_col(int wn, int j, int lane) { return wn * 16 * NJ + j * 32 + (lane & 31); }
+// Width of the forward's tile of token rows from row0.  Where tiles may be narrow, the last one is as wide as the rows
+// that are left need, in groups of 64: the loop is bound by the matrix cores, so products of rows that do not exist
+// cost what others do.  The line between: a narrow tile gets ahead of the tiles that multiply the same W rows, and is
+// worth that while an XCD's 4 MB L2 holds the 512 hidden_dim bytes of those rows and more, and while it is not one of
+// too many (vocabulary 128256, kept logits, us with whole and with narrow tiles: 300 rows x 2048 276, 234; 300 x 4096
+// 455, 386; 1900 x 3584 1513, 1477; 2940 x 4096 2445, 2387; 3900 x 6144 4666, 4590; across the line 900 x 8192 1691,
+// 1719; 2940 x 8192 4605, 4675; 5000 x 4096 4003, 4024, exponentials; 5000 x 8192 7652, 7983).  With up to two tiles
+// of rows there is little to be shared (300 x 8192 874, 851).  `rows` is all that the call has, selected or not: a
+// choice on the device keeps the other widths' code in every call's kernel (2940 x 8192 0.5 % longer for it).
+//
+// The products behind it have whole tiles only: among them narrow ones gain nothing, as the pieces that tiles are cut
+// into stop being alike (d_hidden of 268 rows 312, so 322).
+inline bool narrow_tiles(int64_t rows, int64_t hdim) { return rows <= 2 * BN || (rows <= 16 * BN && hdim <= 6144); }
+__device__ __forceinline__ int tile_width(int64_t rows, int64_t row0, bool narrow) {
+    const int64_t left = rows - row0;
+    if (!narrow || left > 192) return WIDE;
+    return left > 128 ? 6 : left > 64 ? 4 : 2;
+}
+template <class Body>
+__device__ __forceinline__ void with_width(int nj, Body&& body) {
+    if (nj == WIDE) body(std::integral_constant<int, WIDE>{});
+    else if (nj == 6) body(std::integral_constant<int, 6>{});
+    else if (nj == 4) body(std::integral_constant<int, 4>{});
+    else body(std::integral_constant<int, 2>{});
+}
 
 // A fp32 tile that another kernel picks up: in the order in which its column groups lie in the registers
 // (16 bytes per lane, consecutive lanes together, groups of PART_GROUP floats), so that neither side
@@ -635,7 +693,7 @@ __device__ __forceinline__ void stats_update(f32x16 (&z)[2], int wm, int lane, i
 }
 
 // A finished tile leaves as bf16 rows of 256 columns one column group at a time: group j holds the 64 rows
-// (tokens, or rows of a product) wn * 128 + j * 32 + (0..31) of both wn halves with all 256 columns (every m-wave
+// (tokens, or rows of a product) wn * 16 NJ + j * 32 + (0..31) of both wn halves with all 256 columns (every m-wave
 // contributes its 64).  A lane holds groups of eight consecutive columns of one row; they meet in a region of one
 // ring slot and go to global memory in 16-byte pieces of whole 512-byte rows, while the next group's work is being
 // done (forward per slab at the Llama-3.1-8B shape: 6.32 -> 6.28 ms against the whole image at the end).
@@ -646,7 +704,8 @@ __device__ __forceinline__ int piece_perm(int row) { return (row & 7) << 1 | (ro
 constexpr int GROUP_ROWS = 64;
 constexpr int GROUP_BF16_AT = 4 * TILE_ELEMS;  // ring slot 4: slots 0 .. 3 may be filling for the next tile
 static_assert(GROUP_ROWS * BM <= TILE_ELEMS, "a bf16 group fits one ring slot");
-__device__ __forceinline__ int64_t group_row(int64_t row0, int j, int r) { return row0 + (r >> 5) * 128 + j * 32 + (r & 31); }
+template <int NJ = WIDE>
+__device__ __forceinline__ int64_t group_row(int64_t row0, int j, int r) { return row0 + (r >> 5) * 16 * NJ + j * 32 + (r & 31); }
 // columns acc_row(wm, i, 8 p .. 8 p + 7, lane) of the lane's row, which value(r) gives
 template <class Value>
 __device__ __forceinline__ void stage_bf16x8(uint16_t* stage, int wm, int wn, int lane, int i, int p, Value&& value) {
@@ -710,7 +769,7 @@ __device__ __forceinline__ FwdColumn fwd_column(const FwdArgs& a, const float* x
 }
 // Column group j of vocabulary tile vt: the label's logit, the statistics and, where they are kept, the
 // exponentials (through `stage`; every thread of the workgroup takes part).
-template <FwdKeep KEEP>
+template <FwdKeep KEEP, int NJ>
 __device__ __forceinline__ void fwd_fold(f32x16 (&__restrict__ z)[2], FwdColumn& col, const FwdArgs& a, const FwdLaunch& fl,
                                          int64_t vt, int64_t n0, int j, int tid, uint16_t* stage) {
     constexpr bool CACHE = KEEP == FWD_EXPONENTIALS;
@@ -732,7 +791,7 @@ __device__ __forceinline__ void fwd_fold(f32x16 (&__restrict__ z)[2], FwdColumn&
 #pragma unroll
             for (int r = 0; r < 16; ++r)
                 if (i * 16 + r == label_reg) v = z[i][r];
-        const int64_t n = n0 + acc_col(wn, j, lane);
+        const int64_t n = n0 + acc_col<NJ>(wn, j, lane);
         if (n < a.n_tokens) a.zy[n] = v;
     }
     if (m0 + BM > a.vocab)
@@ -758,7 +817,7 @@ __device__ __forceinline__ void fwd_fold(f32x16 (&__restrict__ z)[2], FwdColumn&
 #pragma unroll 1
         for (int it = 0; it < GROUP_PIECES; ++it) {
             const int r = (tid >> 5) + it * (NTHREADS / 32);
-            const int64_t row = group_row(0, j, r);  // token of the tile
+            const int64_t row = group_row<NJ>(0, j, r);  // token of the tile
             const oi_u32x4 v = staged_piece(stage, r, tid & 31);
             *reinterpret_cast<oi_u32x4*>(dst + row * fl.cache_ld + (tid & 31) * 8) =
                 n0 + row < a.n_tokens ? v : oi_u32x4{0u, 0u, 0u, 0u};
@@ -788,7 +847,7 @@ __device__ __forceinline__ float4 fwd_merge_waves(const float* red, int columns,
     return make_float4(m, s, t, 0.f);
 }
 
-template <FwdKeep KEEP>
+template <FwdKeep KEEP, int NJ>
 __device__ __forceinline__ void lmhead_fwd_item(const FwdArgs& a, const FwdLaunch& fl, int64_t split, int64_t tt,
                                                 uint16_t* lds) {
     const int64_t vocab_tiles = (a.vocab + BM - 1) / BM;
@@ -804,45 +863,46 @@ __device__ __forceinline__ void lmhead_fwd_item(const FwdArgs& a, const FwdLaunc
     const Operand tokens = {a.hidden, a.hdim, n0, a.n_tokens, a.hdim};
     Operand rows = {a.W, a.hdim, vt_begin * BM, a.vocab, a.hdim};
 
-    FwdColumn col[4];
+    FwdColumn col[NJ / 2];
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
-        col[j] = fwd_column(a, KEEP == FWD_EXPONENTIALS ? fl.xref : nullptr, n0 + acc_col(wn, j, lane));
+    for (int j = 0; j < NJ / 2; ++j)
+        col[j] = fwd_column(a, KEEP == FWD_EXPONENTIALS ? fl.xref : nullptr, n0 + acc_col<NJ>(wn, j, lane));
 
-    begin_loads<false, false>(rows, tokens, a.hdim, lds);
+    begin_loads<false, false, NJ>(rows, tokens, a.hdim, lds);
     for (int64_t vt = vt_begin; vt < vt_end; ++vt) {
-        AccTile acc;
+        AccTile<NJ> acc;
         gemm_loop<false, false>(acc, rows, tokens, a.hdim, lds);
         // the next tile's first loads run beside this tile's statistics, which leave slots 0 .. 3 alone (scoring
         // pass of 1432 rows, 4096 x 128256: 1.435 -> 1.40 ms; steps 0.2 to 0.6 %)
         rows.r0 += BM;
-        if (vt + 1 < vt_end) begin_loads<false, false>(rows, tokens, a.hdim, lds);
+        if (vt + 1 < vt_end) begin_loads<false, false, NJ>(rows, tokens, a.hdim, lds);
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            Columns c = tile_columns(acc, j);
+        for (int j = 0; j < NJ / 2; ++j) {
+            Columns c = tile_columns<NJ>(acc, j);
             // leaves while the statistics are computed
             if (KEEP == FWD_LOGITS) store_part(c, fl.logits + (vt * fl.logits_tiles + tt) * PART_FLOATS, j, tid);
-            fwd_fold<KEEP>(c.z, col[j], a, fl, vt, n0, j, tid, lds + GROUP_BF16_AT);
+            fwd_fold<KEEP, NJ>(c.z, col[j], a, fl, vt, n0, j, tid, lds + GROUP_BF16_AT);
             __builtin_amdgcn_sched_barrier(0);
         }
     }
 
-    float* red = reinterpret_cast<float*>(lds);  // [4 wm][256 tokens][3]
+    constexpr int COLUMNS = 32 * NJ;
+    float* red = reinterpret_cast<float*>(lds);  // [4 wm][COLUMNS tokens][3]
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
+    for (int j = 0; j < NJ / 2; ++j) {
         fwd_merge_halves(col[j]);
         if (lane < 32) {
-            float* p = red + (wm * 256 + acc_col(wn, j, lane)) * 3;
+            float* p = red + (wm * COLUMNS + acc_col<NJ>(wn, j, lane)) * 3;
             p[0] = col[j].m;
             p[1] = col[j].s;
             p[2] = col[j].t;
         }
     }
     lds_barrier();
-    if (tid < 256 && n0 + tid < a.n_tokens) a.partial[split * a.n_pad + n0 + tid] = fwd_merge_waves(red, 256, tid);
+    if (tid < COLUMNS && n0 + tid < a.n_tokens) a.partial[split * a.n_pad + n0 + tid] = fwd_merge_waves(red, COLUMNS, tid);
 }
 
-template <FwdKeep KEEP>
+template <FwdKeep KEEP, bool NARROW>
 __global__ void __launch_bounds__(NTHREADS)
     lmhead_fwd_kernel(FwdArgs a, const int32_t* __restrict__ n_dev, FwdLaunch fl, uint32_t* __restrict__ queue) {
     __shared__ __align__(16) uint16_t lds[LDS_ELEMS];
@@ -850,10 +910,15 @@ __global__ void __launch_bounds__(NTHREADS)
     const int64_t token_tiles = (a.n_tokens + BN - 1) / BN;
     // every long item of every XCD's queue is taken before the first short one: the short items are
     // there to fill the end of the launch
-    for_each_tile(queue, fl.n_first, token_tiles, lds,
-                  [&](int64_t split, int64_t tt) { lmhead_fwd_item<KEEP>(a, fl, fl.first + split, tt, lds); });
-    for_each_tile(queue + QUEUE_WORDS, fl.n_second, token_tiles, lds,
-                  [&](int64_t split, int64_t tt) { lmhead_fwd_item<KEEP>(a, fl, fl.long_splits + split, tt, lds); });
+#pragma unroll 1
+    for (int pass = 0; pass < 2; ++pass) {
+        const int64_t first = pass ? fl.long_splits : fl.first, splits = pass ? fl.n_second : fl.n_first;
+        for_each_tile(queue + pass * QUEUE_WORDS, splits, token_tiles, lds, [&](int64_t split, int64_t tt) {
+            auto item = [&](auto nj) { lmhead_fwd_item<KEEP, decltype(nj)::value>(a, fl, first + split, tt, lds); };
+            if constexpr (NARROW) with_width(tile_width(a.n_tokens, tt * BN, true), item);
+            else item(std::integral_constant<int, WIDE>{});
+        });
+    }
 }
 
 // A token whose largest scaled logit lies more than this many binary orders above its reference
@@ -994,7 +1059,7 @@ __device__ __forceinline__ void lmhead_dz_tile(const uint16_t* __restrict__ W, c
     const int tid = opaque_tid(), lane = tid & 63, wave = tid >> 6, wm = wave & 3, wn = wave >> 2;
     const int64_t n0 = tt * BN, m0 = v_begin + vt * BM;
 
-    AccTile acc;
+    AccTile<> acc;
     gemm_tile(acc, W, hdim, m0, in.vocab, hidden, hdim, n0, in.n_tokens, hdim, lds);
 
     uint16_t* stage = lds;
@@ -1037,23 +1102,26 @@ __global__ void __launch_bounds__(NTHREADS)
 constexpr int KEPT_ROWS = 64;
 __global__ void __launch_bounds__(NTHREADS)
     lmhead_dz_kept_kernel(const float* __restrict__ logits, int64_t logits_tiles, DzInputs in,
-                          const int32_t* __restrict__ n_dev, int64_t cols, uint16_t* __restrict__ dz) {
+                          const int32_t* __restrict__ n_dev, bool narrow, int64_t cols, uint16_t* __restrict__ dz) {
     __shared__ __align__(16) uint16_t stage[KEPT_ROWS * STAGE_STRIDE];
     if (n_dev) in.n_tokens = *n_dev;
     const int j = blockIdx.x & 3;
     const int64_t tt = blockIdx.x >> 2, vt = blockIdx.y, n0 = tt * BN;
-    if (n0 >= in.n_tokens) return;
+    const int nj = tile_width(in.n_tokens, n0, narrow), half = 16 * nj;  // a group's rows: 32 at j * 32 of both halves
+    if (n0 >= in.n_tokens || j >= nj / 2) return;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, wm = wave & 3, wn = wave >> 2;
     const float* tile = logits + (vt * logits_tiles + tt) * PART_FLOATS;
     const Columns c = load_part(tile, j, tid);
     const int row = wn * 32 + (lane & 31);
-    dz_column(c.z[0], c.z[1], in, n0 + acc_col(wn, j, lane), vt * BM, wm, lane, stage + row * STAGE_STRIDE);
+    dz_column(c.z[0], c.z[1], in, n0 + wn * half + j * 32 + (lane & 31), vt * BM, wm, lane,
+              stage + row * STAGE_STRIDE);
     __syncthreads();
 #pragma unroll
     for (int it = 0; it < KEPT_ROWS * (BM / 8) / NTHREADS; ++it) {
         const int cidx = tid + it * NTHREADS;
         const int r = cidx >> 5, ch = cidx & 31;
-        *reinterpret_cast<oi_u32x4*>(dz + (n0 + (r >> 5) * 128 + j * 32 + (r & 31)) * cols + vt * BM + ch * 8) =
+        const int64_t n = n0 + (r >> 5) * half + j * 32 + (r & 31);
+        *reinterpret_cast<oi_u32x4*>(dz + n * cols + vt * BM + ch * 8) =
             *reinterpret_cast<const oi_u32x4*>(stage + r * STAGE_STRIDE + ch * 8);
     }
 }
@@ -1267,7 +1335,7 @@ struct ProductTile {
 // all but mode 2 in whole pieces: two regions in turn; one is written again only after the barrier of the group in
 // between, by which every wave has read it out
 template <bool PLAIN, bool ADDS>
-__device__ __forceinline__ void store_tile_f32(const AccTile& acc, const ProductTile& t, const StoreTo& st, bool pieces,
+__device__ __forceinline__ void store_tile_f32(const AccTile<>& acc, const ProductTile& t, const StoreTo& st, bool pieces,
                                                uint16_t* lds, int tid) {
     constexpr bool AHEAD = PLAIN && ADDS;
     F32Rows<PLAIN, ADDS> in[2];
@@ -1284,7 +1352,7 @@ __device__ __forceinline__ void store_tile_f32(const AccTile& acc, const Product
     }
 }
 template <bool PLAIN>
-__device__ __forceinline__ void store_tile_as(const AccTile& acc, const ProductTile& t, const StoreTo& st, bool pieces,
+__device__ __forceinline__ void store_tile_as(const AccTile<>& acc, const ProductTile& t, const StoreTo& st, bool pieces,
                                               uint16_t* lds, int tid) {
     if (st.mode == 2 && pieces) {
 #pragma unroll
@@ -1301,7 +1369,7 @@ __device__ __forceinline__ void store_tile_as(const AccTile& acc, const ProductT
     }
 }
 // In mode 2 with whole pieces this leaves the ring slots 0 .. 3 alone.
-__device__ __forceinline__ void store_tile(const AccTile& __restrict__ acc, const ProductTile& t, const StoreTo& st, bool pieces,
+__device__ __forceinline__ void store_tile(const AccTile<>& __restrict__ acc, const ProductTile& t, const StoreTo& st, bool pieces,
                                            uint16_t* lds) {
     const int tid = opaque_tid();
     if (t.part) {
@@ -1456,7 +1524,7 @@ __global__ void __launch_bounds__(NTHREADS)
     ProductTile t = tile_at(item);
     begin_loads<C_KM, R_KM>(t.C, t.R, t.K, lds);
     for (;;) {
-        AccTile acc;
+        AccTile<> acc;
         q.request();
         gemm_loop<C_KM, R_KM>(acc, t.C, t.R, t.K, lds);
         q.settle();
@@ -1612,7 +1680,7 @@ __global__ void __launch_bounds__(NTHREADS)
     tile_of_item(item, tiles_r, tiles_c, &tr, &tc);
     R.r0 = tr * BN;
     C.r0 = tc * BM;
-    AccTile acc;
+    AccTile<> acc;
     gemm_tile<C_KM, R_KM>(acc, C, R, K, lds);
     const int tid = opaque_tid();
     // two regions in turn, as in store_tile
@@ -1658,7 +1726,7 @@ __global__ void __launch_bounds__(NTHREADS)
     for_each_tile(queue, (M + BN - 1) / BN, (N + BM - 1) / BM, lds, [&](int64_t tr, int64_t tc) {
         R.r0 = tr * BN;
         C.r0 = tc * BM;
-        AccTile acc;
+        AccTile<> acc;
         gemm_tile<true, true>(acc, C, R, K, lds);
         const int tid = opaque_tid(), lane = tid & 63, wave = tid >> 6, wm = wave & 3, wn = wave >> 2;
         constexpr int ITERS = GROUP_ROWS * (BM / 4) / NTHREADS;
@@ -2224,13 +2292,15 @@ void enqueue_fwd(const FwdPlan& p, char* ws, const RowInputs& in, const uint8_t*
                         p.n_pad, partial, zy};
     const FwdLaunch fl = {p.tiles_per_split, p.long_splits, 0, p.long_splits, p.n_splits - p.long_splits,
                           keep.buf, keep.ld, 0, keep.buf ? keep.tiles : 0, 0, keep.xref, keep.logits, p.token_tiles};
+    const bool narrow = narrow_tiles(n_tokens, hidden_dim);
+    auto launch = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, dim3(NTHREADS), 0, s, fa, in.n_dev, fl, queue); };
     if (keep.buf) {
         const ProbeScope probe(0, s);
-        hipLaunchKernelGGL(lmhead_fwd_kernel<FWD_EXPONENTIALS>, grid, dim3(NTHREADS), 0, s, fa, in.n_dev, fl, queue);
+        launch(narrow ? lmhead_fwd_kernel<FWD_EXPONENTIALS, true> : lmhead_fwd_kernel<FWD_EXPONENTIALS, false>);
     } else if (keep.logits)
-        hipLaunchKernelGGL(lmhead_fwd_kernel<FWD_LOGITS>, grid, dim3(NTHREADS), 0, s, fa, in.n_dev, fl, queue);
+        launch(narrow ? lmhead_fwd_kernel<FWD_LOGITS, true> : lmhead_fwd_kernel<FWD_LOGITS, false>);
     else
-        hipLaunchKernelGGL(lmhead_fwd_kernel<FWD_PLAIN>, grid, dim3(NTHREADS), 0, s, fa, in.n_dev, fl, queue);
+        launch(narrow ? lmhead_fwd_kernel<FWD_PLAIN, true> : lmhead_fwd_kernel<FWD_PLAIN, false>);
     hipLaunchKernelGGL(lmhead_fwd_combine_kernel, dim3((unsigned)((n_tokens + COMBINE_TOKENS - 1) / COMBINE_TOKENS)),
                        dim3(COMBINE_THREADS), 0, s, partial,
                        zy, n_tokens, in.n_dev, in.rows, row_mask, n_tokens, p.n_splits, p.n_pad, inv_temperature, c, logprob,
@@ -2289,7 +2359,9 @@ void enqueue_fwd_wsum(const FwdPlan& p, char* ws, const RowInputs& in, const uin
         uint32_t* q = queues + ci * (FWD_QUEUE_WORDS + QUEUE_WORDS);
         const FwdLaunch fl = {p.tiles_per_split, p.long_splits, first, n_first, 0, chunk_buf, cols, v_begin / BM,
                               cols / BM, 1, xref, nullptr, 0};
-        hipLaunchKernelGGL(lmhead_fwd_kernel<FWD_EXPONENTIALS>, dim3(resident_grid(n_first, p.token_tiles)), dim3(NTHREADS), 0, s, fa,
+        hipLaunchKernelGGL((narrow_tiles(n_tokens, hidden_dim) ? lmhead_fwd_kernel<FWD_EXPONENTIALS, true>
+                                                                   : lmhead_fwd_kernel<FWD_EXPONENTIALS, false>),
+                           dim3(resident_grid(n_first, p.token_tiles)), dim3(NTHREADS), 0, s, fa,
                            in.n_dev, fl, q);
         const Operand a = {chunk_buf, cols, 0, p.n_pad, cols};
         const Operand b = {Wp + v_begin * hidden_dim, hidden_dim, 0, hidden_dim, valid};
@@ -2374,7 +2446,8 @@ void enqueue_bwd(const BwdPlan& p, char* ws, const RowInputs& in, const void* we
         const DzInputs di = {in.labels, in.lse, in.grad, in.logprob, n_tokens, vocab, c, inv_temperature};
         if (logits)
             hipLaunchKernelGGL(lmhead_dz_kept_kernel, dim3((unsigned)(p.n_pad / BN * 4), (unsigned)(cols / BM)),
-                               dim3(NTHREADS), 0, s, logits, p.n_pad / BN, di, in.n_dev, cols, dz);
+                               dim3(NTHREADS), 0, s, logits, p.n_pad / BN, di, in.n_dev,
+                               narrow_tiles(n_tokens, hidden_dim), cols, dz);
         else
             hipLaunchKernelGGL(lmhead_dz_kernel, grid_of(cols / BM, p.n_pad / BN), dim3(NTHREADS), 0, s, Wp, in.hidden, di,
                                in.n_dev, hidden_dim, v_begin, cols, p.n_pad, dz, q);

@@ -209,10 +209,11 @@ def test_products_of_whole_numbers_are_exact(k_tiles, a_km, b_km):
         assert torch.equal(out, exp)
 
 
-@pytest.mark.parametrize("n", [64, 65, 128, 129, 192, 193, 256, 320, 321])  # last rows of each group of 64 token rows and the first of the next
+# last rows of each group of 64 token rows and the first of the next: the widths of the forward's last tile
+@pytest.mark.parametrize("n", [64, 65, 128, 129, 192, 193, 256, 320, 321])
 @pytest.mark.parametrize("keep_logits", [True, False])
 def test_last_tile_of_token_rows(n, keep_logits):
-    h, v = 192, 700  # three k-tiles, a ragged vocabulary tile; one tile of d_hidden columns, short of its last group
+    h, v = 192, 700  # three k-tiles; ragged vocabulary tile and d_hidden columns
     print(f"case N={n} keep_logits={keep_logits}", flush=True)
     hidden, weight, labels, _, upstream = _inputs(n, h, v, seed=n)
     lp, dh, dw = _reference(hidden, weight, labels, torch.ones_like(labels, dtype=torch.bool), upstream)
