@@ -281,13 +281,15 @@ typedef short v4i16 __attribute__((ext_vector_type(4)));
 //
 // A loader stands at one k-tile and moves on to the next with advance().  Past the last one it stays there and all lanes
 // fetch the same 16 bytes, into slots that nobody reads: the waits of the loop count loads, so one has to be issued and
-// has to come back in its turn.  (A load outside the bounds of its buffer does not: it is counted off at once, ahead of
+// has to come back in its turn.  ROUND: the product begins at k-tile `start` and goes round.  (A load outside the bounds of its buffer does not: it is counted off at once, ahead of
 // older loads that are still under way.)
-template <bool KM, int LOADS>
+template <bool KM, int LOADS, bool ROUND = false>
 struct Loader {
+    static_assert(!(KM && ROUND), "the others begin at the first k-tile");
     static_assert(LOADS == 4 || !KM, "k-major operands are whole tiles");
     const char* base;   // of the operand, for k-major of the k-tile
     uint32_t plus;      // bytes from there to the k-tile (k-contiguous)
+    uint32_t plus_end;  // and to the end of the last one (ROUND)
     uint32_t off[LOADS];  // per-lane byte offsets of the loads
     int lds_wave;       // bytes to this wave's first load inside a slot
     int tiles_left;     // from this k-tile on, negated
@@ -295,10 +297,11 @@ struct Loader {
     int rows_left;      // k rows from this k-tile's first on, without that one (k-major)
     static constexpr int LDS_BLOCK = KM ? 2 * 256 * 2 : 8 * BK * 2;  // bytes between the LDS destinations of loads
 
-    __device__ __forceinline__ Loader(const Operand& op, int ktiles, int lane, int wave) {
+    __device__ __forceinline__ Loader(const Operand& op, int ktiles, int start, int lane, int wave) {
         tiles_left = -ktiles;
         live = -1;
-        plus = 0;
+        plus = ROUND ? (uint32_t)start * (BK * 2) : 0;
+        plus_end = (uint32_t)ktiles * (BK * 2);
         rows_left = (int)op.k_valid - 1;
         if constexpr (!KM) {
             base = reinterpret_cast<const char*>(op.p + op.r0 * op.ld);
@@ -339,6 +342,7 @@ struct Loader {
             if (rows_left < BK - 1) set_rows(op, lane, wave);
         } else {
             plus += BK * 2 & live;
+            if (ROUND && plus == plus_end) plus = 0;
             if (!live) {
 #pragma unroll
                 for (int b = 0; b < LOADS; ++b) off[b] = 0;
@@ -352,21 +356,22 @@ __device__ __forceinline__ void load_to_lds(const char* base, uint32_t off, uint
                                              OI_LDS_PTR(to), 16, off, plus, 0, 0);
 }
 // one 1 KB load: block b of this wave's share of an operand k-tile into the ring slot at byte offset `slot`
-template <bool KM, int LOADS>
-__device__ __forceinline__ void load_block(const Loader<KM, LOADS>& L, int slot, int b, uint16_t* lds) {
+template <bool KM, int LOADS, bool ROUND>
+__device__ __forceinline__ void load_block(const Loader<KM, LOADS, ROUND>& L, int slot, int b, uint16_t* lds) {
     load_to_lds(L.base, L.off[b], L.plus, reinterpret_cast<char*>(lds) + slot + L.lds_wave + b * L.LDS_BLOCK);
 }
 // ring slots: A_t -> (2 t) mod 5, B_t -> (2 t + 1) mod 5
-template <bool A_KM, bool B_KM, int NJ = WIDE>
-__device__ __forceinline__ void begin_loads(const Operand& A_, const Operand& B_, int64_t K, uint16_t* lds) {
+template <bool A_KM, bool B_KM, int NJ = WIDE, bool ROUND = false>
+__device__ __forceinline__ void begin_loads(const Operand& A_, const Operand& B_, int64_t K, uint16_t* lds,
+                                            int start = 0) {
     const Operand A = scalar(A_), B = scalar(B_);
     const int tid = opaque_tid();
     // the wave index as a scalar: the LDS destinations of the loads (M0) then take no VALU work
     const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int ktiles = __builtin_amdgcn_readfirstlane((int)(K / BK));
     constexpr int B_LOADS = NJ / 2;
-    Loader<A_KM, 4> la(A, ktiles, lane, wave);
-    Loader<B_KM, B_LOADS> lb(B, ktiles, lane, wave);
+    Loader<A_KM, 4, ROUND> la(A, ktiles, start, lane, wave);
+    Loader<B_KM, B_LOADS, ROUND> lb(B, ktiles, start, lane, wave);
 #pragma unroll
     for (int b = 0; b < 4; ++b) load_block(la, 0, b, lds);
 #pragma unroll
@@ -382,16 +387,17 @@ __device__ __forceinline__ void begin_loads(const Operand& A_, const Operand& B_
 // `__restrict__` here and in store_tile is what tells the compiler that the LDS accesses of these functions carry
 // alias information; without any it waits for every global->LDS load in flight before each LDS access
 // (d_weight of 3072 rows: 2.7 -> 4.9 ms).
-template <bool A_KM, bool B_KM, int NJ>
-__device__ __forceinline__ void gemm_loop(AccTile<NJ>& __restrict__ acc, const Operand& A_, const Operand& B_, int64_t K, uint16_t* lds) {
+template <bool A_KM, bool B_KM, bool ROUND = false, int NJ>
+__device__ __forceinline__ void gemm_loop(AccTile<NJ>& __restrict__ acc, const Operand& A_, const Operand& B_, int64_t K,
+                                          uint16_t* lds, int start = 0) {
     const Operand A = scalar(A_), B = scalar(B_);
     const int tid = opaque_tid();
     const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wm = wave & 3, wn = wave >> 2;
     const int ktiles = __builtin_amdgcn_readfirstlane((int)(K / BK));
     constexpr int B_LOADS = NJ / 2;
-    Loader<A_KM, 4> la(A, ktiles, lane, wave);        // at k-tile kt+2
-    Loader<B_KM, B_LOADS> lb(B, ktiles, lane, wave);  // at k-tile kt+1 in group 0, kt+2 behind the barrier
+    Loader<A_KM, 4, ROUND> la(A, ktiles, start, lane, wave);        // at k-tile kt+2
+    Loader<B_KM, B_LOADS, ROUND> lb(B, ktiles, start, lane, wave);  // at k-tile kt+1 in group 0, kt+2 behind the barrier
     la.advance(A, lane, wave);
     la.advance(A, lane, wave);
     lb.advance(B, lane, wave);
@@ -540,11 +546,13 @@ __device__ __forceinline__ void gemm_tile(AccTile<>& acc, const Operand& A, cons
     gemm_loop<A_KM, B_KM>(acc, A, B, K, lds);
 }
 // both operands k-contiguous: C[m, n] = sum_k A[m0 + m, k] * B[n0 + n, k]
+template <bool ROUND>
 __device__ __forceinline__ void gemm_tile(AccTile<>& acc, const uint16_t* __restrict__ A, int64_t lda, int64_t m0,
                                           int64_t M, const uint16_t* __restrict__ B, int64_t ldb, int64_t n0,
-                                          int64_t N, int64_t K, uint16_t* lds) {
+                                          int64_t N, int64_t K, uint16_t* lds, int start) {
     const Operand a = {A, lda, m0, M, K}, b = {B, ldb, n0, N, K};
-    gemm_tile<false, false>(acc, a, b, K, lds);
+    begin_loads<false, false, WIDE, ROUND>(a, b, K, lds, start);
+    gemm_loop<false, false, ROUND>(acc, a, b, K, lds, start);
 }
 
 // An MFMA leaves lane l with rows 4 (l / 16) .. + 3 of column l % 16 of a 16 x 16 tile (acc[i][j]: rows 16 i, columns
@@ -594,6 +602,21 @@ __device__ __forceinline__ int tile_width(int64_t rows, int64_t row0, bool narro
     const int64_t left = rows - row0;
     if (!narrow || left > 192) return WIDE;
     return left > 128 ? 6 : left > 64 ? 4 : 2;
+}
+// What a call has of token rows: up to one tile (narrow too), tiles of which the last may be narrow, whole tiles.
+enum RowTiles { ONE_TILE, NARROW_LAST, WHOLE_TILES };
+inline RowTiles row_tiles(int64_t rows, int64_t hdim) {
+    return rows <= BN ? ONE_TILE : narrow_tiles(rows, hdim) ? NARROW_LAST : WHOLE_TILES;
+}
+// The k-tile at which the product of vocabulary tile vt with ONE_TILE begins.  Such a call reads W once and little else,
+// 128 bytes of 256 rows at a time: with all workgroups at the same k-tile those lie hidden_dim * 2 bytes apart, on few of
+// the memory channels.  So each run of 32 vocabulary tiles, the ones that an XCD works on together and that share
+// hidden's k-tiles in its L2, begins at another eighth (vocabulary 128256, us before and after: 100 rows x 2048 160, 134;
+// 100 x 4096 260, 212; 256 x 4096 311, 247; 256 x 8192 560, 444; 30 x 8192 378, 382).  With more
+// tiles of rows W's k-tiles are shared as well and nothing is gained (300 x 4096 350, 360; 2940 x 4096 2205, 2195), while
+// going round costs 0.4 % (scoring pass of 1432 rows, step of 268).
+__device__ __forceinline__ int first_k_tile(int64_t vt, int64_t hdim) {
+    return __builtin_amdgcn_readfirstlane((int)(vt >> 5 & 7) * (int)(hdim / BK) / 8);
 }
 template <class Body>
 __device__ __forceinline__ void with_width(int nj, Body&& body) {
@@ -847,7 +870,7 @@ __device__ __forceinline__ float4 fwd_merge_waves(const float* red, int columns,
     return make_float4(m, s, t, 0.f);
 }
 
-template <FwdKeep KEEP, int NJ>
+template <FwdKeep KEEP, bool ROUND, int NJ>
 __device__ __forceinline__ void lmhead_fwd_item(const FwdArgs& a, const FwdLaunch& fl, int64_t split, int64_t tt,
                                                 uint16_t* lds) {
     const int64_t vocab_tiles = (a.vocab + BM - 1) / BM;
@@ -868,14 +891,15 @@ __device__ __forceinline__ void lmhead_fwd_item(const FwdArgs& a, const FwdLaunc
     for (int j = 0; j < NJ / 2; ++j)
         col[j] = fwd_column(a, KEEP == FWD_EXPONENTIALS ? fl.xref : nullptr, n0 + acc_col<NJ>(wn, j, lane));
 
-    begin_loads<false, false, NJ>(rows, tokens, a.hdim, lds);
+    auto start_of = [&](int64_t vt) { return ROUND ? first_k_tile(vt, a.hdim) : 0; };
+    begin_loads<false, false, NJ, ROUND>(rows, tokens, a.hdim, lds, start_of(vt_begin));
     for (int64_t vt = vt_begin; vt < vt_end; ++vt) {
         AccTile<NJ> acc;
-        gemm_loop<false, false>(acc, rows, tokens, a.hdim, lds);
+        gemm_loop<false, false, ROUND>(acc, rows, tokens, a.hdim, lds, start_of(vt));
         // the next tile's first loads run beside this tile's statistics, which leave slots 0 .. 3 alone (scoring
         // pass of 1432 rows, 4096 x 128256: 1.435 -> 1.40 ms; steps 0.2 to 0.6 %)
         rows.r0 += BM;
-        if (vt + 1 < vt_end) begin_loads<false, false, NJ>(rows, tokens, a.hdim, lds);
+        if (vt + 1 < vt_end) begin_loads<false, false, NJ, ROUND>(rows, tokens, a.hdim, lds, start_of(vt + 1));
 #pragma unroll
         for (int j = 0; j < NJ / 2; ++j) {
             Columns c = tile_columns<NJ>(acc, j);
@@ -902,7 +926,7 @@ __device__ __forceinline__ void lmhead_fwd_item(const FwdArgs& a, const FwdLaunc
     if (tid < COLUMNS && n0 + tid < a.n_tokens) a.partial[split * a.n_pad + n0 + tid] = fwd_merge_waves(red, COLUMNS, tid);
 }
 
-template <FwdKeep KEEP, bool NARROW>
+template <FwdKeep KEEP, RowTiles TILES>
 __global__ void __launch_bounds__(NTHREADS)
     lmhead_fwd_kernel(FwdArgs a, const int32_t* __restrict__ n_dev, FwdLaunch fl, uint32_t* __restrict__ queue) {
     __shared__ __align__(16) uint16_t lds[LDS_ELEMS];
@@ -914,8 +938,10 @@ __global__ void __launch_bounds__(NTHREADS)
     for (int pass = 0; pass < 2; ++pass) {
         const int64_t first = pass ? fl.long_splits : fl.first, splits = pass ? fl.n_second : fl.n_first;
         for_each_tile(queue + pass * QUEUE_WORDS, splits, token_tiles, lds, [&](int64_t split, int64_t tt) {
-            auto item = [&](auto nj) { lmhead_fwd_item<KEEP, decltype(nj)::value>(a, fl, first + split, tt, lds); };
-            if constexpr (NARROW) with_width(tile_width(a.n_tokens, tt * BN, true), item);
+            auto item = [&](auto nj) {
+                lmhead_fwd_item<KEEP, TILES == ONE_TILE, decltype(nj)::value>(a, fl, first + split, tt, lds);
+            };
+            if constexpr (TILES != WHOLE_TILES) with_width(tile_width(a.n_tokens, tt * BN, true), item);
             else item(std::integral_constant<int, WIDE>{});
         });
     }
@@ -1053,6 +1079,7 @@ __device__ __forceinline__ void dz_column(const f32x16& z0, const f32x16& z1, co
     }
 }
 
+template <bool ROUND>
 __device__ __forceinline__ void lmhead_dz_tile(const uint16_t* __restrict__ W, const uint16_t* __restrict__ hidden,
                                                const DzInputs& in, int64_t hdim, int64_t v_begin, int64_t chunk_cols,
                                                uint16_t* __restrict__ dz, int64_t vt, int64_t tt, uint16_t* lds) {
@@ -1060,7 +1087,9 @@ __device__ __forceinline__ void lmhead_dz_tile(const uint16_t* __restrict__ W, c
     const int64_t n0 = tt * BN, m0 = v_begin + vt * BM;
 
     AccTile<> acc;
-    gemm_tile(acc, W, hdim, m0, in.vocab, hidden, hdim, n0, in.n_tokens, hdim, lds);
+    // as the forward, so that the logits are its to the bit
+    gemm_tile<ROUND>(acc, W, hdim, m0, in.vocab, hidden, hdim, n0, in.n_tokens, hdim, lds,
+                     ROUND ? first_k_tile(m0 / BM, hdim) : 0);
 
     uint16_t* stage = lds;
 #pragma unroll
@@ -1081,6 +1110,7 @@ __device__ __forceinline__ void lmhead_dz_tile(const uint16_t* __restrict__ W, c
     }
 }
 
+template <bool ROUND>
 __global__ void __launch_bounds__(NTHREADS)
     lmhead_dz_kernel(const uint16_t* __restrict__ W, const uint16_t* __restrict__ hidden, DzInputs in,
                      const int32_t* __restrict__ n_dev, int64_t hdim, int64_t v_begin, int64_t chunk_cols, int64_t n_pad,
@@ -1091,7 +1121,7 @@ __global__ void __launch_bounds__(NTHREADS)
         n_pad = (in.n_tokens + BN - 1) / BN * BN;
     }
     for_each_tile(queue, chunk_cols / BM, n_pad / BN, lds, [&](int64_t vt, int64_t tt) {
-        lmhead_dz_tile(W, hidden, in, hdim, v_begin, chunk_cols, dz, vt, tt, lds);
+        lmhead_dz_tile<ROUND>(W, hidden, in, hdim, v_begin, chunk_cols, dz, vt, tt, lds);
     });
 }
 
@@ -2278,6 +2308,14 @@ void launch_label_ref(const RowInputs& in, const void* weight, int64_t n_tokens,
                        inv_temperature * OI_LOG2E, xref);
 }
 
+template <FwdKeep KEEP>
+auto fwd_kernel(int64_t n_tokens, int64_t hidden_dim) {
+    const RowTiles tiles = row_tiles(n_tokens, hidden_dim);
+    return tiles == ONE_TILE      ? lmhead_fwd_kernel<KEEP, ONE_TILE>
+           : tiles == NARROW_LAST ? lmhead_fwd_kernel<KEEP, NARROW_LAST>
+                                  : lmhead_fwd_kernel<KEEP, WHOLE_TILES>;
+}
+
 // forward launches: tile kernel + merge of the partial statistics.  `queue` must be zeroed.
 // `keep`: where the exponentials of every vocabulary tile go as well (buf null: nowhere).
 void enqueue_fwd(const FwdPlan& p, char* ws, const RowInputs& in, const uint8_t* row_mask, const void* weight,
@@ -2292,15 +2330,17 @@ void enqueue_fwd(const FwdPlan& p, char* ws, const RowInputs& in, const uint8_t*
                         p.n_pad, partial, zy};
     const FwdLaunch fl = {p.tiles_per_split, p.long_splits, 0, p.long_splits, p.n_splits - p.long_splits,
                           keep.buf, keep.ld, 0, keep.buf ? keep.tiles : 0, 0, keep.xref, keep.logits, p.token_tiles};
-    const bool narrow = narrow_tiles(n_tokens, hidden_dim);
-    auto launch = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, dim3(NTHREADS), 0, s, fa, in.n_dev, fl, queue); };
+    auto launch = [&](auto keep_as) {
+        hipLaunchKernelGGL(fwd_kernel<decltype(keep_as)::value>(n_tokens, hidden_dim), grid, dim3(NTHREADS), 0, s, fa, in.n_dev,
+                           fl, queue);
+    };
     if (keep.buf) {
         const ProbeScope probe(0, s);
-        launch(narrow ? lmhead_fwd_kernel<FWD_EXPONENTIALS, true> : lmhead_fwd_kernel<FWD_EXPONENTIALS, false>);
+        launch(std::integral_constant<FwdKeep, FWD_EXPONENTIALS>{});
     } else if (keep.logits)
-        launch(narrow ? lmhead_fwd_kernel<FWD_LOGITS, true> : lmhead_fwd_kernel<FWD_LOGITS, false>);
+        launch(std::integral_constant<FwdKeep, FWD_LOGITS>{});
     else
-        launch(narrow ? lmhead_fwd_kernel<FWD_PLAIN, true> : lmhead_fwd_kernel<FWD_PLAIN, false>);
+        launch(std::integral_constant<FwdKeep, FWD_PLAIN>{});
     hipLaunchKernelGGL(lmhead_fwd_combine_kernel, dim3((unsigned)((n_tokens + COMBINE_TOKENS - 1) / COMBINE_TOKENS)),
                        dim3(COMBINE_THREADS), 0, s, partial,
                        zy, n_tokens, in.n_dev, in.rows, row_mask, n_tokens, p.n_splits, p.n_pad, inv_temperature, c, logprob,
@@ -2359,8 +2399,7 @@ void enqueue_fwd_wsum(const FwdPlan& p, char* ws, const RowInputs& in, const uin
         uint32_t* q = queues + ci * (FWD_QUEUE_WORDS + QUEUE_WORDS);
         const FwdLaunch fl = {p.tiles_per_split, p.long_splits, first, n_first, 0, chunk_buf, cols, v_begin / BM,
                               cols / BM, 1, xref, nullptr, 0};
-        hipLaunchKernelGGL((narrow_tiles(n_tokens, hidden_dim) ? lmhead_fwd_kernel<FWD_EXPONENTIALS, true>
-                                                                   : lmhead_fwd_kernel<FWD_EXPONENTIALS, false>),
+        hipLaunchKernelGGL(fwd_kernel<FWD_EXPONENTIALS>(n_tokens, hidden_dim),
                            dim3(resident_grid(n_first, p.token_tiles)), dim3(NTHREADS), 0, s, fa,
                            in.n_dev, fl, q);
         const Operand a = {chunk_buf, cols, 0, p.n_pad, cols};
@@ -2447,10 +2486,10 @@ void enqueue_bwd(const BwdPlan& p, char* ws, const RowInputs& in, const void* we
         if (logits)
             hipLaunchKernelGGL(lmhead_dz_kept_kernel, dim3((unsigned)(p.n_pad / BN * 4), (unsigned)(cols / BM)),
                                dim3(NTHREADS), 0, s, logits, p.n_pad / BN, di, in.n_dev,
-                               narrow_tiles(n_tokens, hidden_dim), cols, dz);
+                               row_tiles(n_tokens, hidden_dim) != WHOLE_TILES, cols, dz);
         else
-            hipLaunchKernelGGL(lmhead_dz_kernel, grid_of(cols / BM, p.n_pad / BN), dim3(NTHREADS), 0, s, Wp, in.hidden, di,
-                               in.n_dev, hidden_dim, v_begin, cols, p.n_pad, dz, q);
+            hipLaunchKernelGGL((row_tiles(n_tokens, hidden_dim) == ONE_TILE ? lmhead_dz_kernel<true> : lmhead_dz_kernel<false>),
+                               grid_of(cols / BM, p.n_pad / BN), dim3(NTHREADS), 0, s, Wp, in.hidden, di, in.n_dev, hidden_dim, v_begin, cols, p.n_pad, dz, q);
         const bool first = ci == 0, last = ci == p.n_chunks - 1;
         const int mode = last ? (first ? 2 : 3) : (first ? 0 : 1);
         {

@@ -226,3 +226,22 @@ def test_last_tile_of_token_rows(n, keep_logits):
         _close(hid.grad, dh, "d_hidden")
         if not frozen:
             _close(w.grad, dw, "d_weight")
+
+
+@pytest.mark.parametrize("n,h", [(1, 64), (256, 192), (100, 576), (257, 576)])  # k-tiles fewer than eighths, and not a multiple
+def test_products_that_begin_at_another_k_tile(n, h):
+    v = 8 * 32 * 256 + 300  # vocabulary tiles of every eighth and of the first once more
+    print(f"case N={n} H={h}", flush=True)
+    hidden, weight, labels, _, upstream = _inputs(n, h, v, seed=n + h)
+    lp, dh, dw = _reference(hidden, weight, labels, torch.ones_like(labels, dtype=torch.bool), upstream)
+    grads = []
+    for keep_logits in (True, False):  # read back; computed again, by the same rule
+        hid, w = hidden.clone().requires_grad_(True), weight.clone().requires_grad_(True)
+        out = lm_head.fused_lm_head_logprobs(hid, w, labels, keep_logits=keep_logits)
+        out = out[0] if isinstance(out, tuple) else out
+        assert (out.detach() - lp).abs().max().item() <= TOL
+        out.backward(upstream)
+        _close(hid.grad, dh, "d_hidden")
+        _close(w.grad, dw, "d_weight")
+        grads.append(hid.grad)
+    assert torch.equal(*grads)
