@@ -15,8 +15,8 @@
 //
 // Tile: 256 x 256 x 64 per 512-thread workgroup, 8 waves as 4 (m) x 2 (n), each wave 64 x 128 =
 // 4 x 8 MFMA 16x16x32 accumulators.  With vocabulary as the m dim a lane's accumulators of a
-// column of tiles belong to ONE token, so the softmax statistics reduce inside the lane.  LDS: a ring of five 32 KB operand slots (k-tiles of A and of B) filled by
-// direct global->LDS loads of whole 128-byte line segments; the 16-byte chunks of a row are
+// column of tiles belong to ONE token, so the softmax statistics reduce inside the lane.  LDS: a ring of five 32 KB
+// operand slots (k-tiles of A and of B) filled by direct global->LDS loads of whole 128-byte line segments; the 16-byte chunks of a row are
 // XOR-permuted so that fragment reads (16-byte reads of a k-contiguous image, transposing 8-byte
 // reads of a k-major image) stay free of bank conflicts.  A launch is one resident workgroup per
 // CU that draws tile ids from per-XCD counters.
@@ -281,8 +281,8 @@ typedef short v4i16 __attribute__((ext_vector_type(4)));
 //
 // A loader stands at one k-tile and moves on to the next with advance().  Past the last one it stays there and all lanes
 // fetch the same 16 bytes, into slots that nobody reads: the waits of the loop count loads, so one has to be issued and
-// has to come back in its turn.  ROUND: the product begins at k-tile `start` and goes round.  (A load outside the bounds of its buffer does not: it is counted off at once, ahead of
-// older loads that are still under way.)
+// has to come back in its turn.  (A load outside the bounds of its buffer does not: it is counted off at once, ahead of
+// older loads that are still under way.)  ROUND: the product begins at k-tile `start` and goes round.
 template <bool KM, int LOADS, bool ROUND = false>
 struct Loader {
     static_assert(!(KM && ROUND), "the others begin at the first k-tile");
@@ -717,29 +717,37 @@ __device__ __forceinline__ void stats_update(f32x16 (&z)[2], int wm, int lane, i
 
 // A finished tile leaves as bf16 rows of 256 columns one column group at a time: group j holds the 64 rows
 // (tokens, or rows of a product) wn * 16 NJ + j * 32 + (0..31) of both wn halves with all 256 columns (every m-wave
-// contributes its 64).  A lane holds groups of eight consecutive columns of one row; they meet in a region of one
-// ring slot and go to global memory in 16-byte pieces of whole 512-byte rows, while the next group's work is being
-// done (forward per slab at the Llama-3.1-8B shape: 6.32 -> 6.28 ms against the whole image at the end).
+// contributes its 64).  A lane holds groups of eight consecutive columns of one row; a wave's meet in its share of one
+// ring slot and go to global memory as whole 128-byte lines, eight rows at a time.  The waves do not wait for each
+// other: with rows of 512 bytes that all waves fill there were two barriers per group (d_weight of 268 rows 404 us, now
+// 391, of 2340 rows x 128256 1934, now 1907; step of 268 rows 1117, now 1095).
 //
-// The region: 64 rows of 512 bytes, unpadded; the 16-byte pieces of a row at c ^ piece_perm(row), which puts the
-// 16-byte stores of 16 rows, and those of 8 rows and two neighbouring pieces, on all 64 banks.
-__device__ __forceinline__ int piece_perm(int row) { return (row & 7) << 1 | (row >> 3 & 1) | (row & 16); }
+// A share: 32 rows of 128 bytes, unpadded; the 16-byte pieces of a row at c ^ piece_perm(row), which puts the
+// 16-byte stores of 16 rows, and those of a row pair, on all 64 banks.
+__device__ __forceinline__ int piece_perm(int row) { return row >> 1 & 7; }
 constexpr int GROUP_ROWS = 64;
 constexpr int GROUP_BF16_AT = 4 * TILE_ELEMS;  // ring slot 4: slots 0 .. 3 may be filling for the next tile
 static_assert(GROUP_ROWS * BM <= TILE_ELEMS, "a bf16 group fits one ring slot");
 template <int NJ = WIDE>
 __device__ __forceinline__ int64_t group_row(int64_t row0, int j, int r) { return row0 + (r >> 5) * 16 * NJ + j * 32 + (r & 31); }
-// columns acc_row(wm, i, 8 p .. 8 p + 7, lane) of the lane's row, which value(r) gives
+// One wave's share: 32 rows of 64 columns (128 bytes), row lane % 32 from each lane.  Columns acc_row(wm, i, 8 p .. 8 p + 7,
+// lane) of the lane's row, which value(r) gives
+constexpr int SHARE_COLS = 64, SHARE_ELEMS = 32 * SHARE_COLS;
 template <class Value>
-__device__ __forceinline__ void stage_bf16x8(uint16_t* stage, int wm, int wn, int lane, int i, int p, Value&& value) {
-    const int srow = wn * 32 + (lane & 31), piece = (wm * 8 + i * 4 + p * 2 + (lane >> 5)) ^ piece_perm(srow);
-    *reinterpret_cast<oi_u32x4*>(stage + srow * BM + piece * 8) =
+__device__ __forceinline__ void stage_bf16x8(uint16_t* share, int lane, int i, int p, Value&& value) {
+    const int srow = lane & 31, piece = (i * 4 + p * 2 + (lane >> 5)) ^ piece_perm(srow);
+    *reinterpret_cast<oi_u32x4*>(share + srow * SHARE_COLS + piece * 8) =
         oi_u32x4{oi_pack_bf16x2(value(p * 8), value(p * 8 + 1)), oi_pack_bf16x2(value(p * 8 + 2), value(p * 8 + 3)),
                  oi_pack_bf16x2(value(p * 8 + 4), value(p * 8 + 5)), oi_pack_bf16x2(value(p * 8 + 6), value(p * 8 + 7))};
 }
-constexpr int GROUP_PIECES = GROUP_ROWS * (BM / 8) / NTHREADS;  // 16-byte pieces per thread
-__device__ __forceinline__ oi_u32x4 staged_piece(const uint16_t* stage, int r, int ch) {
-    return *reinterpret_cast<const oi_u32x4*>(stage + r * BM + (ch ^ piece_perm(r)) * 8);
+// between a wave's writes to its share and its reads: the LDS serves a wave in order, so this only holds the compiler
+__device__ __forceinline__ void share_staged() { asm volatile("" ::: "memory"); }
+// piece it of a lane: row it * 8 + lane / 8, columns 8 (lane % 8) ..
+constexpr int GROUP_PIECES = SHARE_ELEMS / 8 / OI_WAVE;
+__device__ __forceinline__ int piece_row(int lane, int it) { return it * 8 + (lane >> 3); }
+__device__ __forceinline__ oi_u32x4 staged_piece(const uint16_t* share, int lane, int it) {
+    const int r = piece_row(lane, it);
+    return *reinterpret_cast<const oi_u32x4*>(share + r * SHARE_COLS + ((lane & 7) ^ piece_perm(r)) * 8);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -798,6 +806,7 @@ __device__ __forceinline__ void fwd_fold(f32x16 (&__restrict__ z)[2], FwdColumn&
     constexpr bool CACHE = KEEP == FWD_EXPONENTIALS;
     asm volatile("" : "+v"(tid));  // addresses are formed here, not ahead of the tile's main loop
     const int lane = tid & 63, wave = tid >> 6, wm = wave & 3, wn = wave >> 2;
+    uint16_t* share = stage + wave * SHARE_ELEMS;
     const int64_t m0 = vt * BM;
     // the target logit, when its row falls into this wave's 64 rows
     const int rel = col.lab - ((int)m0 + wm * 64);
@@ -834,18 +843,15 @@ __device__ __forceinline__ void fwd_fold(f32x16 (&__restrict__ z)[2], FwdColumn&
 #pragma unroll
         for (int i = 0; i < 2; ++i)
 #pragma unroll
-            for (int p = 0; p < 2; ++p) stage_bf16x8(stage, wm, wn, lane, i, p, [&](int r) { return z[i][r]; });
-        lds_barrier();
-        uint16_t* dst = fl.ecache + n0 * fl.cache_ld + (vt - fl.cache_tile0) * BM;
+            for (int p = 0; p < 2; ++p) stage_bf16x8(share, lane, i, p, [&](int r) { return z[i][r]; });
+        share_staged();
+        uint16_t* dst = fl.ecache + n0 * fl.cache_ld + (vt - fl.cache_tile0) * BM + wm * SHARE_COLS + (lane & 7) * 8;
 #pragma unroll 1
         for (int it = 0; it < GROUP_PIECES; ++it) {
-            const int r = (tid >> 5) + it * (NTHREADS / 32);
-            const int64_t row = group_row<NJ>(0, j, r);  // token of the tile
-            const oi_u32x4 v = staged_piece(stage, r, tid & 31);
-            *reinterpret_cast<oi_u32x4*>(dst + row * fl.cache_ld + (tid & 31) * 8) =
-                n0 + row < a.n_tokens ? v : oi_u32x4{0u, 0u, 0u, 0u};
+            const int64_t row = group_row<NJ>(0, j, wn * 32 + piece_row(lane, it));  // token of the tile
+            const oi_u32x4 v = staged_piece(share, lane, it);
+            *reinterpret_cast<oi_u32x4*>(dst + row * fl.cache_ld) = n0 + row < a.n_tokens ? v : oi_u32x4{0u, 0u, 0u, 0u};
         }
-        lds_barrier();  // the region is free for the next group
         __builtin_amdgcn_sched_barrier(0);
     }
 }
@@ -1182,14 +1188,16 @@ __device__ __forceinline__ bool stores_in_pieces(const StoreTo& st) {
 
 // Column group j of a finished tile is its rows row0 + wn * 128 + j * 32 + (0..31) of both wn halves with all 256
 // columns from col0.  z0, z1: the lane's accumulators, row acc_col(wn, j, lane), columns acc_row(wm, 0 / 1, r,
-// lane), i.e. groups of four consecutive columns of one row.  They meet in the LDS region `stage` (64 rows) and
-// leave as whole rows, 512 bytes of bf16 or 1 KB of fp32 at a time.  Every thread of the workgroup takes part.
+// lane), i.e. groups of four consecutive columns of one row.  bf16 goes through the wave's share of the LDS and
+// leaves 128 bytes of a row at a time; fp32 meets in the LDS region `stage` (64 rows) and leaves as whole rows of 1 KB,
+// every thread of the workgroup taking part.
 //
 // What bounds the epilogue is that nothing is multiplied meanwhile (one workgroup per CU), so few instructions
 // and whole lines.  Registers transposed in quads of lanes and stored from there in 64-byte pieces, with a wait
 // for the stores of the tile before the next tile's first load: d_weight of 268 rows (100352 x 4096, 6272
 // tiles of 5 k-tiles) 606 us; through the LDS 544; without waiting for stores at its barriers 504; with the next tile's
-// first loads ahead of it 478; without waiting for each store before the next 382 (with the tile engine's other changes).
+// first loads ahead of it 478; without waiting for each store before the next 382 (with the tile engine's other changes);
+// without barriers 3 % less.
 constexpr int STAGE_F32 = BM + 4;                            // floats per row: rows 4 banks apart
 constexpr int GROUP_F32 = GROUP_ROWS * STAGE_F32 * 2;        // LDS elements of an fp32 region
 static_assert(2 * GROUP_F32 <= LDS_ELEMS, "the epilogue's regions fit the ring");
@@ -1239,26 +1247,24 @@ __device__ __forceinline__ void store_group_bf16(const f32x16& z0, const f32x16&
                                                  int64_t col0, int j, uint16_t* stage, int tid) {
     asm volatile("" : "+v"(tid));  // addresses are formed here, not ahead of the tile's main loop
     const int lane = tid & 63, wave = tid >> 6, wm = wave & 3, wn = wave >> 2;
+    uint16_t* share = stage + wave * SHARE_ELEMS;
     GroupRows<PLAIN, GROUP_PIECES> rows;
-    rows.request(st, row0, j, wn * 32 + (lane & 31), tid >> 5, NTHREADS / 32);
+    rows.request(st, row0, j, wn * 32 + (lane & 31), wn * 32 + (lane >> 3), 8);
 #pragma unroll
     for (int i = 0; i < 2; ++i)
 #pragma unroll
         for (int p = 0; p < 2; ++p) {
             const f32x16& z = i == 0 ? z0 : z1;
-            stage_bf16x8(stage, wm, wn, lane, i, p, [&](int r) { return rows.scale(st, z[r]); });
+            stage_bf16x8(share, lane, i, p, [&](int r) { return rows.scale(st, z[r]); });
         }
-    lds_barrier();
-    oi_u32x4 v[GROUP_PIECES];
-#pragma unroll
-    for (int it = 0; it < GROUP_PIECES; ++it) v[it] = staged_piece(stage, (tid >> 5) + it * (NTHREADS / 32), tid & 31);
-    lds_barrier();  // the region is free for the next group
-    const int64_t col = col0 + (tid & 31) * 8;
+    share_staged();
+    const int64_t col = col0 + wm * SHARE_COLS + (lane & 7) * 8;
 #pragma unroll
     for (int it = 0; it < GROUP_PIECES; ++it) {
-        const int r = (tid >> 5) + it * (NTHREADS / 32);
+        const oi_u32x4 v = staged_piece(share, lane, it);
+        const int r = wn * 32 + piece_row(lane, it);
         if (group_row(row0, j, r) >= st.m_valid || col >= st.N) continue;
-        *reinterpret_cast<oi_u32x4*>(st.out_bf16 + rows.at(st, row0, col, j, r, it)) = v[it];
+        *reinterpret_cast<oi_u32x4*>(st.out_bf16 + rows.at(st, row0, col, j, r, it)) = v;
     }
 }
 
