@@ -361,6 +361,68 @@ __global__ void __launch_bounds__(256)
     if (threadIdx.x == 0) out[e] = (float)(axis_mode == 0 ? num_tot * inv_global : mean_sum / (double)rows);
 }
 
+// Both of the above in one launch for few elements: one workgroup per e, fp64 sums.  Without axis_mode the waves share all
+// rows * cols elements; with it each has a row.  A call of this size is bound by its launches (about 4 us each on the
+// device).  Device time with two launches and with one, us: [4, 512] 7.6, 3.7; [8, 1024] 8.0, 4.5; [16, 1024] 8.8, 5.8;
+// means of rows [4, 512] 7.2, 3.5; [16, 1024] 7.7, 5.5; [1, 2048] 7.9, 6.7, which is as long as a wave's chain of reads
+// may be; several rows per wave take longer ([64, 256] 7.0, 7.9; [256, 64] 7.0, 21).
+constexpr int SMALL_THREADS = 1024, SMALL_WAVES = SMALL_THREADS / OI_WAVE;
+constexpr int64_t SMALL_ELEMS = 16384, SMALL_COLS = 2048;
+__global__ void __launch_bounds__(SMALL_THREADS)
+    masked_small_kernel(const float* __restrict__ values, const void* __restrict__ mask, int mask_is_float, int rows,
+                        int cols, int axis_mode, float denominator, float* __restrict__ out,
+                        float* __restrict__ row_denoms) {
+    __shared__ double part[3][SMALL_WAVES];
+    const int e = blockIdx.x, n = rows * cols, wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const float* v = values + (int64_t)e * n;
+    double num = 0.0, cnt = 0.0, means = 0.0;
+    if (axis_mode == 1) {
+        if (wave < rows) {
+            double rn = 0.0, rc = 0.0;
+#pragma unroll 4
+            for (int i = wave * cols + lane; i < (wave + 1) * cols; i += OI_WAVE) {
+                const float m = mask_at(mask, mask_is_float, i);
+                rn += (double)(v[i] * m);
+                rc += (double)m;
+            }
+            rn = oi_wave_sum(rn);
+            rc = oi_wave_sum(rc);
+            const double den = denominator > 0.f ? (double)denominator : rc;
+            const double inv = den > 0.0 ? 1.0 / den : 0.0;
+            means = rn * inv;
+            if (row_denoms && e == 0 && lane == 0) row_denoms[wave] = (float)(inv / (double)rows);
+        }
+    } else {
+#pragma unroll 4
+        for (int i = threadIdx.x; i < n; i += SMALL_THREADS) {
+            const float m = mask_at(mask, mask_is_float, i);
+            num += (double)(v[i] * m);
+            cnt += (double)m;
+        }
+        num = oi_wave_sum(num);
+        cnt = oi_wave_sum(cnt);
+    }
+    if (lane == 0) {
+        part[0][wave] = num;
+        part[1][wave] = cnt;
+        part[2][wave] = means;
+    }
+    __syncthreads();
+    double total[3] = {0.0, 0.0, 0.0};
+#pragma unroll
+    for (int w = 0; w < SMALL_WAVES; ++w)
+#pragma unroll
+        for (int k = 0; k < 3; ++k) total[k] += part[k][w];
+    double inv = 0.0;
+    if (axis_mode == 0) {
+        const double den = denominator > 0.f ? (double)denominator : total[1];
+        inv = den > 0.0 ? 1.0 / den : 0.0;
+        if (row_denoms && e == 0)
+            for (int r = threadIdx.x; r < rows; r += SMALL_THREADS) row_denoms[r] = (float)inv;
+    }
+    if (threadIdx.x == 0) out[e] = (float)(axis_mode == 0 ? total[0] * inv : total[2] / (double)rows);
+}
+
 __global__ void masked_bwd_kernel(const float* __restrict__ grad_out, const void* __restrict__ mask,
                                   int mask_is_float, const float* __restrict__ row_denoms, int64_t extra,
                                   int64_t rows, int64_t cols, float* __restrict__ d_values) {
@@ -825,6 +887,11 @@ extern "C" int oi_masked_mean_fwd(const float* values, const void* mask, int mas
     float* partial = static_cast<float*>(workspace);
     float* cnt = partial + extra * rows * nchunks;
     hipStream_t s = static_cast<hipStream_t>(stream);
+    if (rows <= SMALL_ELEMS / cols && (axis_mode == 0 || (rows <= SMALL_WAVES && cols <= SMALL_COLS))) {
+        hipLaunchKernelGGL(masked_small_kernel, dim3((unsigned)extra), dim3(SMALL_THREADS), 0, s, values, mask, mask_is_float,
+                           (int)rows, (int)cols, axis_mode, denominator, out, row_denoms);
+        return oi_launch_status();
+    }
     hipLaunchKernelGGL(masked_partial_kernel, dim3((unsigned)(extra * rows * nchunks)), dim3(FUSED_THREADS), 0, s,
                        values, mask, mask_is_float, rows, cols, nchunks, partial, cnt);
     hipLaunchKernelGGL(masked_final_kernel, dim3((unsigned)extra), dim3(256), 0, s, partial, cnt, rows, nchunks,

@@ -60,6 +60,29 @@ def test_masked_mean_random_and_gradient(axis, denominator, bool_mask):
     assert (dv.grad.cpu() - exp_grad).abs().max().item() <= 1e-7 + 1e-5 * exp_grad.abs().max().item()
 
 
+# both sides of the sizes that go in one launch: elements, rows and columns of a mean per row
+@pytest.mark.parametrize("rows,cols,axis", [(1, 1, None), (1, 16384, None), (1, 16385, None), (3, 5461, None), (1, 2048, 1),
+                                            (1, 2049, 1), (16, 1024, 1), (16, 1025, 1), (17, 900, 1), (15, 63, 1)])  # fmt: skip
+def test_masked_mean_sizes_of_one_launch(rows, cols, axis):
+    g = torch.Generator().manual_seed(rows * cols)
+    values = torch.randn(3, rows, cols, generator=g)
+    mask = torch.rand(rows, cols, generator=g) > 0.3
+    mask[rows // 2] = rows == 1  # an empty row where there is another
+    ref_v = values.double().requires_grad_(True)
+    if axis is None:
+        ref = (ref_v * mask).sum((1, 2)) / mask.sum()
+    else:
+        ref = ((ref_v * mask).sum(2) / mask.sum(1).clamp(min=1)).mean(1)
+    ref.sum().backward()
+    dv = values.to(DEV).requires_grad_(True)
+    out = rl_utils.masked_mean(dv, mask.to(DEV), axis)
+    out.sum().backward()
+    # chunks of 1024 in fp32 at most: 10 roundings of partial sums no larger than the sum of magnitudes
+    bound = 10 * 2.0**-24 * values.abs().amax().item()
+    assert (out.detach().cpu().double() - ref.detach()).abs().max().item() <= bound
+    assert (dv.grad.cpu().double() - ref_v.grad).abs().max().item() <= 2.0**-22 * ref_v.grad.abs().max().item()
+
+
 def test_masked_mean_scalar_cases():
     v = torch.tensor([[1.0, 2.0, 3.0], [4.0, 5.0, 6.0]], device=DEV)
     m = torch.tensor([[True, True, False], [True, False, False]], device=DEV)
