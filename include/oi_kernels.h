@@ -225,6 +225,10 @@ int oi_grpo_fused_bwd(const float* new_logprobs, const float* old_logprobs, cons
  *   drop outside (mask_lower, mask_upper), clamp to [clamp_lower, clamp_upper] (a bound of 0
  *   disables it); six fp32 [rows, cols] outputs: rho, weights, dropped, dropped-low,
  *   dropped-high, clamped-flag.
+ * oi_pick_values: out[0 .. *count) = the values whose mask byte is set, in order (out has room for n).  One workgroup:
+ *   meant for a few thousand values.
+ * oi_record_stats: one sample's column of a [OI_GRPO_NUM_STATS, columns] table of statistics: the rows whose bit in
+ *   row_mask is set from vector [OI_GRPO_NUM_STATS], and row loss_row from loss [1].
  * ------------------------------------------------------------------------------------------ */
 int oi_estimate_kl_fwd(const float* ref_logprobs_diff, const float* ratio, int64_t n, float* out, void* stream);
 int oi_estimate_kl_bwd(const float* ref_logprobs_diff, const float* ratio, const float* grad_out, int64_t n,
@@ -238,6 +242,9 @@ int oi_rho_correction(const float* old_logprobs, const float* vllm_logprobs, con
                       float mask_lower, float mask_upper, float clamp_lower, float clamp_upper, float* rho,
                       float* weights, float* drop_any, float* drop_low, float* drop_high, float* clipped,
                       void* stream);
+int oi_pick_values(const float* values, const uint8_t* mask, int64_t n, float* out, int32_t* count, void* stream);
+int oi_record_stats(const float* vector, uint32_t row_mask, const float* loss, int loss_row, float* table,
+                    int64_t columns, int64_t column, void* stream);
 
 /* Group-normalised advantages.  Carries open_instruct/data_loader.py:1472-1484: population std,
  * mode 0 "standard" (s - mean) / (std + 1e-8), mode 1 "centered" s - mean.  Computed in fp64 like

@@ -69,14 +69,15 @@ class _SigmoidPairLoss(torch.autograd.Function):
         ctx.meta = (beta, label_smoothing, margin, shape, pc.dtype, pr.dtype)
         losses, cr, rj = (t.reshape(shape) for t in out.unbind(0))
         ctx.mark_non_differentiable(cr, rj)
+        ctx.set_materialize_grads(False)  # of the rewards: two fills that nobody reads
         return losses, cr, rj
 
     @staticmethod
     def backward(ctx, g_losses, _g_cr, _g_rj):
         pc_c, pr_c, rc_c, rr_c, w_c = ctx.saved_tensors
         beta, ls, margin, shape, dt_c, dt_r = ctx.meta
-        g = _lib.f32c(g_losses).reshape(-1)
         n = pc_c.numel()
+        g = _lib.f32c(g_losses).reshape(-1) if g_losses is not None else torch.zeros_like(pc_c)
         d = torch.empty((2, n), dtype=torch.float32, device=g.device)
         _lib.call(
             "oi_dpo_sigmoid_bwd", pc_c.data_ptr(), pr_c.data_ptr(), _lib.ptr(rc_c), _lib.ptr(rr_c), _lib.ptr(w_c),

@@ -126,7 +126,7 @@ def compute_rho_correction(
             *[bufs[k].data_ptr() for k in range(6)], _lib.stream_of(old),
         )  # fmt: skip
         rho, weights, drop_any, drop_low, drop_high, clipped = bufs.unbind(0)
-        hist = {"val/rho_hist": rho[response_mask.bool()].detach().float()}
+        hist = {"val/rho_hist": _picked(rho, m)}
         if not use:
             return RhoCorrection(weights=torch.ones_like(rho), metrics={}, histogram_metrics=hist)
         metrics = {
@@ -137,6 +137,24 @@ def compute_rho_correction(
             "val/rho_clipfrac": clipped,
         }
         return RhoCorrection(weights=weights, metrics=metrics, histogram_metrics=hist)
+
+
+# Up to here one workgroup and the read of its count beat torch's selection, which waits for its size as well: 2047
+# values 38 us, now 21; 32768 41, now 32; 65536 40, would be 46.
+_PICK_MAX = 32768
+
+
+def _picked(values: torch.Tensor, mask_u8: torch.Tensor) -> torch.Tensor:
+    """``values[mask]`` as a new 1-D tensor."""
+    n = values.numel()
+    if not 0 < n <= _PICK_MAX:
+        return values[mask_u8.bool()]
+    out = torch.empty(n, dtype=torch.float32, device=values.device)
+    count = torch.empty(1, dtype=torch.int32, device=values.device)
+    _lib.call(
+        "oi_pick_values", values.data_ptr(), mask_u8.data_ptr(), n, out.data_ptr(), count.data_ptr(), _lib.stream_of(values)
+    )
+    return out[: count.item()]
 
 
 def accumulate_rho_histograms(acc: dict[str, list[torch.Tensor]], correction: RhoCorrection) -> None:
@@ -318,13 +336,14 @@ class _GrpoFused(torch.autograd.Function):
         ctx.in_dtype = new_logprobs.dtype
         loss = stats[0]
         ctx.mark_non_differentiable(stats)
+        ctx.set_materialize_grads(False)  # of stats: a fill that nobody reads
         return loss.clone(), stats
 
     @staticmethod
     def backward(ctx, g_loss, _g_stats):
         nl, old_c, ref_c, adv_c, m, rho_c, row_denoms = ctx.saved_tensors
         loss_fn, lo, hi, kl_estimator, beta, _axis_mode, _denominator, scale = ctx.cfg
-        g = _lib.f32c(g_loss).reshape(1)
+        g = _lib.f32c(g_loss).reshape(1) if g_loss is not None else nl.new_zeros(1)
         d_new = torch.empty_like(nl)
         rows, cols = nl.shape
         _lib.call(
@@ -925,6 +944,22 @@ def _rows_to_record(config, ref_logprobs, entropy, rho_metrics) -> list[int]:
     return sorted(set(rows))
 
 
+def _recorded_in_one(table, sample_idx, vec, loss, rows) -> bool:
+    """A sample's column of an intact table in one launch instead of four (20 us, now 13)."""
+    if table is None or type(sample_idx) is not int or not 0 <= sample_idx < table.shape[1]:
+        return False
+    for t in (vec, loss):
+        if not torch.is_tensor(t) or t.dtype != torch.float32 or t.device != table.device or not t.is_cuda:
+            return False
+    if vec.shape != (len(GRPO_STAT_NAMES),) or not vec.is_contiguous() or loss.numel() != 1 or loss.ndim:
+        return False
+    _lib.call(
+        "oi_record_stats", vec.data_ptr(), sum(1 << r for r in rows), loss.data_ptr(), _STAT_ROW["loss/total_avg"],
+        table.data_ptr(), table.shape[1], sample_idx, _lib.stream_of(table),
+    )  # fmt: skip
+    return True
+
+
 def populate_sample_loss_stats(
     loss_stats_B: dict[str, torch.Tensor],
     sample_idx: int,
@@ -986,6 +1021,8 @@ def populate_sample_loss_stats(
                 _lib.stream_of(pg_c),
             )  # fmt: skip
         if vec is not None:
+            if "loss/total_avg" in loss_stats_B and _recorded_in_one(table, sample_idx, vec, loss, rows):
+                return
             if table is not None:
                 sel = _row_selector(tuple(rows), table.device)
                 table[:, sample_idx].index_copy_(0, sel, vec.to(table.device).index_select(0, sel))

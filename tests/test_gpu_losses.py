@@ -841,3 +841,33 @@ def test_rho_correction_broadcast_advantages():
     _close(got.weights, exp.weights)
     for k, v in exp.metrics.items():
         _close(got.metrics[k], v)
+
+
+@pytest.mark.parametrize("shape", [(1, 1), (1, 255), (1, 257), (3, 1365), (1, 4096), (1, 4097), (2, 16384), (1, 32769)])
+@pytest.mark.parametrize("kept", [0.0, 0.6, 1.0])
+def test_rho_histogram_is_the_selection_in_order(shape, kept):
+    g = torch.Generator().manual_seed(shape[1])
+    old, vllm = torch.randn(shape, generator=g).to(DEV), torch.randn(shape, generator=g).to(DEV)
+    mask = (torch.rand(shape, generator=g) < kept).to(DEV)
+    cfg = make_grpo_config(use_rho_correction=True)
+    hist = grpo_utils.compute_rho_correction(old, vllm, mask, torch.ones(shape, device=DEV), cfg).histogram_metrics["val/rho_hist"]
+    expected = torch.exp((old - vllm).clamp(-10, 10))[mask]
+    assert hist.shape == expected.shape and torch.allclose(hist, expected, rtol=1e-5, atol=0)
+
+
+@pytest.mark.parametrize("sample_idx", [0, 6, -1])  # the last by the general way
+def test_recorded_column_equals_the_general_way(sample_idx):
+    g = torch.Generator().manual_seed(5)
+    t = lambda: torch.randn(2, 70, generator=g).to(DEV)  # noqa: E731
+    mask = (torch.rand(2, 70, generator=g) < 0.7).to(DEV)
+    cfg = make_grpo_config(load_ref_policy=True, beta=0.05)
+    new, old, ref, adv, ent = t(), t(), t(), t(), t()
+    loss, stats = grpo_utils.grpo_loss_fused(new, old, ref, adv, mask, cfg, entropy=ent)
+    tables = []
+    for recorded in (stats, {k: v for k, v in stats.items()}):
+        table = grpo_utils.create_loss_stats(7, DEV, record_entropy=True)
+        table.table.fill_(7.0)
+        total = loss if recorded is stats else loss.double()  # the general way
+        grpo_utils.populate_sample_loss_stats(table, sample_idx, None, None, None, total, mask, new, ref, ent, cfg, fused_stats=recorded)
+        tables.append(table.table)
+    assert torch.equal(*tables)
