@@ -1279,15 +1279,15 @@ struct F32Rows {
         asm volatile("" : "+v"(tid));
         rows.request(st, row0, j, (tid >> 8) * 32 + (tid & 31), tid >> 6, NTHREADS / 64);
         if constexpr (ADDS) {
-            // offsets inside the tile fit 32 bits (255 rows of at most MAX_LD columns)
-            const float* tile = st.out_f32 + row0 * st.ldo + col0;
-            const int last = (int)(st.m_valid - 1 - row0 < BN - 1 ? st.m_valid - 1 - row0 : BN - 1);
+            // a wave reads one row at a time, whose address is scalar; results have any pitch, so it is formed in 64 bits
+            const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+            const int64_t last = st.m_valid - 1;
             const int c = (tid & 63) * 4, last_c = (int)(st.N - 4 - col0 < BM - 4 ? st.N - 4 - col0 : BM - 4);
+            const uint32_t col = c < last_c ? c : last_c;
 #pragma unroll
             for (int it = 0; it < F32_PIECES; ++it) {
-                const int row = (int)group_row(0, j, (tid >> 6) + it * 8);
-                const uint32_t off = __umul24(row < last ? row : last, (uint32_t)st.ldo) + (c < last_c ? c : last_c);
-                sum[it] = *reinterpret_cast<const oi_f32x4*>(tile + off);
+                const int64_t row = group_row(row0, j, wave + it * (NTHREADS / 64));
+                sum[it] = *reinterpret_cast<const oi_f32x4*>(st.out_f32 + (row < last ? row : last) * st.ldo + col0 + col);
             }
         }
     }

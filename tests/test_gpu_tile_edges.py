@@ -162,6 +162,25 @@ def test_products_of_any_pitch(m, n, k, ldo, shift):
         assert (rows[:, n:] == 3).all() and (out[:shift] == 3).all() and (out[shift + m * ldo :] == 3).all()
 
 
+# pitches past 24 and past 32 bits; one column tile and two
+@pytest.mark.parametrize("m,n,ldo", [(3, 8, 1 << 24), (3, 264, (1 << 24) + 8), (2, 8, (1 << 32) + 8)])
+def test_products_added_to_rows_far_apart(m, n, ldo):
+    """Small whole numbers, exact in fp32."""
+    k = 64
+    print("case far rows", m, n, ldo, flush=True)
+    g = torch.Generator().manual_seed(n)
+    a = torch.randint(-4, 5, (m, k), generator=g).bfloat16().to(DEV)
+    b = torch.randint(-4, 5, (n, k), generator=g).bfloat16().to(DEV)
+    before = torch.randint(-9, 10, (m, n), generator=g).float().to(DEV)
+    out = torch.empty((m - 1) * ldo + n, device=DEV)
+    rows = out.as_strided((m, n), (ldo, 1))
+    rows.copy_(before)
+    rc = _lib.load().oi_gemm_bf16_tn(
+        a.data_ptr(), k, m, b.data_ptr(), k, n, k, out.data_ptr(), None, ldo, 1, torch.cuda.current_stream().cuda_stream
+    )
+    assert rc == 0 and torch.equal(rows, before + a.float() @ b.float().t())
+
+
 @pytest.mark.parametrize("n,h,v,flagged,slabs", [(1, 64, 300, 1, 4096), (300, 64, 301, 70, 4096), (600, 320, 513, 257, 256)])
 def test_flagged_rows_are_added_to_d_weight(n, h, v, flagged, slabs):
     """Rows whose label lies more than 44 nats below the largest logit are recomputed and added to the bf16 d_weight
