@@ -21,6 +21,7 @@
 // reads of a k-major image) stay free of bank conflicts.  A launch is one resident workgroup per
 // CU that draws tile ids from per-XCD counters.
 #include "oi_common.h"
+#include "oi_ktiles.h"
 
 #include <type_traits>
 
@@ -282,27 +283,25 @@ typedef short v4i16 __attribute__((ext_vector_type(4)));
 // A loader stands at one k-tile and moves on to the next with advance().  Past the last one it stays there and all lanes
 // fetch the same 16 bytes, into slots that nobody reads: the waits of the loop count loads, so one has to be issued and
 // has to come back in its turn.  (A load outside the bounds of its buffer does not: it is counted off at once, ahead of
-// older loads that are still under way.)  ROUND: the product begins at k-tile `start` and goes round.
-template <bool KM, int LOADS, bool ROUND = false>
+// older loads that are still under way.)  WALK: how it moves.  A k range that goes ROUND begins at k-tile `start`; a FAR
+// one may be longer than a row pitch (stand-alone products whose rows are all one).
+enum Walk { NEAR, ROUND, FAR };
+template <bool KM, int LOADS, Walk WALK = NEAR>
 struct Loader {
-    static_assert(!(KM && ROUND), "the others begin at the first k-tile");
+    static_assert(!KM || WALK != ROUND, "the others begin at the first k-tile");
     static_assert(LOADS == 4 || !KM, "k-major operands are whole tiles");
-    const char* base;   // of the operand, for k-major of the k-tile
-    uint32_t plus;      // bytes from there to the k-tile (k-contiguous)
+    static constexpr bool MOVES_BASE = KM || WALK == FAR;  // by more than 32 bits in all
+    const char* base;   // of the operand, or of the k-tile
+    uint32_t plus;      // bytes from there to the k-tile
     uint32_t plus_end;  // and to the end of the last one (ROUND)
     uint32_t off[LOADS];  // per-lane byte offsets of the loads
     int lds_wave;       // bytes to this wave's first load inside a slot
-    int tiles_left;     // from this k-tile on, negated
-    int live;           // all ones, or 0 past the last k-tile
-    int rows_left;      // k rows from this k-tile's first on, without that one (k-major)
+    KTiles<BK> k;
     static constexpr int LDS_BLOCK = KM ? 2 * 256 * 2 : 8 * BK * 2;  // bytes between the LDS destinations of loads
 
-    __device__ __forceinline__ Loader(const Operand& op, int ktiles, int start, int lane, int wave) {
-        tiles_left = -ktiles;
-        live = -1;
-        plus = ROUND ? (uint32_t)start * (BK * 2) : 0;
+    __device__ __forceinline__ Loader(const Operand& op, int ktiles, int start, int lane, int wave) : k(ktiles, op.k_valid) {
+        plus = WALK == ROUND ? (uint32_t)start * (BK * 2) : 0;
         plus_end = (uint32_t)ktiles * (BK * 2);
-        rows_left = (int)op.k_valid - 1;
         if constexpr (!KM) {
             base = reinterpret_cast<const char*>(op.p + op.r0 * op.ld);
             const int last_row = (int)((op.extent - 1 - op.r0) < 255 ? (op.extent - 1 - op.r0) : 255);
@@ -323,30 +322,25 @@ struct Loader {
     static __device__ __forceinline__ uint32_t pitch(const Operand& op) { return (uint32_t)(op.ld * 2); }
     // k-major: this k-tile's k rows, which may end inside it
     __device__ __forceinline__ void set_rows(const Operand& op, int lane, int wave) {
-        const int last_k = rows_left < BK - 1 ? (rows_left < 0 ? 0 : rows_left) : BK - 1;
+        const int last_k = k.end_row();
         const int r0 = (int)op.r0, extent = (int)op.extent;
 #pragma unroll
         for (int b = 0; b < 4; ++b) {
             const int kk = wave * 8 + b * 2 + (lane >> 5);
             const int c = r0 + ((lane & 31) ^ (4 * (kk & 3)) ^ (2 * ((kk >> 3) & 1))) * 8;
-            off[b] = (__umul24(kk < last_k ? kk : last_k, pitch(op)) + (uint32_t)((c + 8 <= extent ? c : extent - 8) * 2)) & live;
+            off[b] = (__umul24(kk < last_k ? kk : last_k, pitch(op)) + (uint32_t)((c + 8 <= extent ? c : extent - 8) * 2)) & k.live;
         }
     }
     __device__ __forceinline__ void advance(const Operand& op, int lane, int wave) {
-        ++tiles_left;
-        // in assembly, or the compiler makes a compare of it whose result it puts into a vector register
-        asm("s_ashr_i32 %0, %1, 31" : "=s"(live) : "s"(tiles_left) : "scc");
+        k.next();
+        if constexpr (MOVES_BASE) base += k.step(KM ? BK * 2 * op.ld : BK * 2);
+        else plus += BK * 2 & k.live;
+        if constexpr (WALK == ROUND) plus = plus == plus_end ? 0 : plus;
         if constexpr (KM) {
-            base += (int64_t)BK * 2 * op.ld & (int64_t)live;  // k rows can lie more than 32 bits apart
-            rows_left -= BK;
-            if (rows_left < BK - 1) set_rows(op, lane, wave);
-        } else {
-            plus += BK * 2 & live;
-            if (ROUND && plus == plus_end) plus = 0;
-            if (!live) {
+            if (k.ending()) set_rows(op, lane, wave);
+        } else if (!k.live) {
 #pragma unroll
-                for (int b = 0; b < LOADS; ++b) off[b] = 0;
-            }
+            for (int b = 0; b < LOADS; ++b) off[b] = 0;
         }
     }
 };
@@ -356,12 +350,12 @@ __device__ __forceinline__ void load_to_lds(const char* base, uint32_t off, uint
                                              OI_LDS_PTR(to), 16, off, plus, 0, 0);
 }
 // one 1 KB load: block b of this wave's share of an operand k-tile into the ring slot at byte offset `slot`
-template <bool KM, int LOADS, bool ROUND>
-__device__ __forceinline__ void load_block(const Loader<KM, LOADS, ROUND>& L, int slot, int b, uint16_t* lds) {
+template <bool KM, int LOADS, Walk WALK>
+__device__ __forceinline__ void load_block(const Loader<KM, LOADS, WALK>& L, int slot, int b, uint16_t* lds) {
     load_to_lds(L.base, L.off[b], L.plus, reinterpret_cast<char*>(lds) + slot + L.lds_wave + b * L.LDS_BLOCK);
 }
 // ring slots: A_t -> (2 t) mod 5, B_t -> (2 t + 1) mod 5
-template <bool A_KM, bool B_KM, int NJ = WIDE, bool ROUND = false>
+template <bool A_KM, bool B_KM, int NJ = WIDE, Walk WALK = NEAR>
 __device__ __forceinline__ void begin_loads(const Operand& A_, const Operand& B_, int64_t K, uint16_t* lds,
                                             int start = 0) {
     const Operand A = scalar(A_), B = scalar(B_);
@@ -370,8 +364,8 @@ __device__ __forceinline__ void begin_loads(const Operand& A_, const Operand& B_
     const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int ktiles = __builtin_amdgcn_readfirstlane((int)(K / BK));
     constexpr int B_LOADS = NJ / 2;
-    Loader<A_KM, 4, ROUND> la(A, ktiles, start, lane, wave);
-    Loader<B_KM, B_LOADS, ROUND> lb(B, ktiles, start, lane, wave);
+    Loader<A_KM, 4, WALK> la(A, ktiles, start, lane, wave);
+    Loader<B_KM, B_LOADS, WALK> lb(B, ktiles, start, lane, wave);
 #pragma unroll
     for (int b = 0; b < 4; ++b) load_block(la, 0, b, lds);
 #pragma unroll
@@ -387,7 +381,7 @@ __device__ __forceinline__ void begin_loads(const Operand& A_, const Operand& B_
 // `__restrict__` here and in store_tile is what tells the compiler that the LDS accesses of these functions carry
 // alias information; without any it waits for every global->LDS load in flight before each LDS access
 // (d_weight of 3072 rows: 2.7 -> 4.9 ms).
-template <bool A_KM, bool B_KM, bool ROUND = false, int NJ>
+template <bool A_KM, bool B_KM, Walk WALK = NEAR, int NJ>
 __device__ __forceinline__ void gemm_loop(AccTile<NJ>& __restrict__ acc, const Operand& A_, const Operand& B_, int64_t K,
                                           uint16_t* lds, int start = 0) {
     const Operand A = scalar(A_), B = scalar(B_);
@@ -396,8 +390,8 @@ __device__ __forceinline__ void gemm_loop(AccTile<NJ>& __restrict__ acc, const O
     const int wm = wave & 3, wn = wave >> 2;
     const int ktiles = __builtin_amdgcn_readfirstlane((int)(K / BK));
     constexpr int B_LOADS = NJ / 2;
-    Loader<A_KM, 4, ROUND> la(A, ktiles, start, lane, wave);        // at k-tile kt+2
-    Loader<B_KM, B_LOADS, ROUND> lb(B, ktiles, start, lane, wave);  // at k-tile kt+1 in group 0, kt+2 behind the barrier
+    Loader<A_KM, 4, WALK> la(A, ktiles, start, lane, wave);        // at k-tile kt+2
+    Loader<B_KM, B_LOADS, WALK> lb(B, ktiles, start, lane, wave);  // at k-tile kt+1 in group 0, kt+2 behind the barrier
     la.advance(A, lane, wave);
     la.advance(A, lane, wave);
     lb.advance(B, lane, wave);
@@ -539,19 +533,19 @@ __device__ __forceinline__ void gemm_loop(AccTile<NJ>& __restrict__ acc, const O
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
 }
-template <bool A_KM, bool B_KM>
+template <bool A_KM, bool B_KM, Walk WALK = NEAR>
 __device__ __forceinline__ void gemm_tile(AccTile<>& acc, const Operand& A, const Operand& B, int64_t K, uint16_t* lds) {
-    begin_loads<A_KM, B_KM>(A, B, K, lds);
-    gemm_loop<A_KM, B_KM>(acc, A, B, K, lds);
+    begin_loads<A_KM, B_KM, WIDE, WALK>(A, B, K, lds);
+    gemm_loop<A_KM, B_KM, WALK>(acc, A, B, K, lds);
 }
 // both operands k-contiguous: C[m, n] = sum_k A[m0 + m, k] * B[n0 + n, k]
-template <bool ROUND>
+template <Walk WALK>
 __device__ __forceinline__ void gemm_tile(AccTile<>& acc, const uint16_t* __restrict__ A, int64_t lda, int64_t m0,
                                           int64_t M, const uint16_t* __restrict__ B, int64_t ldb, int64_t n0,
                                           int64_t N, int64_t K, uint16_t* lds, int start) {
     const Operand a = {A, lda, m0, M, K}, b = {B, ldb, n0, N, K};
-    begin_loads<false, false, WIDE, ROUND>(a, b, K, lds, start);
-    gemm_loop<false, false, ROUND>(acc, a, b, K, lds, start);
+    begin_loads<false, false, WIDE, WALK>(a, b, K, lds, start);
+    gemm_loop<false, false, WALK>(acc, a, b, K, lds, start);
 }
 
 // An MFMA leaves lane l with rows 4 (l / 16) .. + 3 of column l % 16 of a 16 x 16 tile (acc[i][j]: rows 16 i, columns
@@ -875,7 +869,7 @@ __device__ __forceinline__ float4 fwd_merge_waves(const float* red, int columns,
     return make_float4(m, s, t, 0.f);
 }
 
-template <FwdKeep KEEP, bool ROUND, int NJ>
+template <FwdKeep KEEP, Walk WALK, int NJ>
 __device__ __forceinline__ void lmhead_fwd_item(const FwdArgs& a, const FwdLaunch& fl, int64_t split, int64_t tt,
                                                 uint16_t* lds) {
     const int64_t vocab_tiles = (a.vocab + BM - 1) / BM;
@@ -896,15 +890,15 @@ __device__ __forceinline__ void lmhead_fwd_item(const FwdArgs& a, const FwdLaunc
     for (int j = 0; j < NJ / 2; ++j)
         col[j] = fwd_column(a, KEEP == FWD_EXPONENTIALS ? fl.xref : nullptr, n0 + acc_col<NJ>(wn, j, lane));
 
-    auto start_of = [&](int64_t vt) { return ROUND ? first_k_tile(vt, a.hdim) : 0; };
-    begin_loads<false, false, NJ, ROUND>(rows, tokens, a.hdim, lds, start_of(vt_begin));
+    auto start_of = [&](int64_t vt) { return WALK == ROUND ? first_k_tile(vt, a.hdim) : 0; };
+    begin_loads<false, false, NJ, WALK>(rows, tokens, a.hdim, lds, start_of(vt_begin));
     for (int64_t vt = vt_begin; vt < vt_end; ++vt) {
         AccTile<NJ> acc;
-        gemm_loop<false, false, ROUND>(acc, rows, tokens, a.hdim, lds, start_of(vt));
+        gemm_loop<false, false, WALK>(acc, rows, tokens, a.hdim, lds, start_of(vt));
         // the next tile's first loads run beside this tile's statistics, which leave slots 0 .. 3 alone (scoring
         // pass of 1432 rows, 4096 x 128256: 1.435 -> 1.40 ms; steps 0.2 to 0.6 %)
         rows.r0 += BM;
-        if (vt + 1 < vt_end) begin_loads<false, false, NJ, ROUND>(rows, tokens, a.hdim, lds, start_of(vt + 1));
+        if (vt + 1 < vt_end) begin_loads<false, false, NJ, WALK>(rows, tokens, a.hdim, lds, start_of(vt + 1));
 #pragma unroll
         for (int j = 0; j < NJ / 2; ++j) {
             Columns c = tile_columns<NJ>(acc, j);
@@ -944,7 +938,7 @@ __global__ void __launch_bounds__(NTHREADS)
         const int64_t first = pass ? fl.long_splits : fl.first, splits = pass ? fl.n_second : fl.n_first;
         for_each_tile(queue + pass * QUEUE_WORDS, splits, token_tiles, lds, [&](int64_t split, int64_t tt) {
             auto item = [&](auto nj) {
-                lmhead_fwd_item<KEEP, TILES == ONE_TILE, decltype(nj)::value>(a, fl, first + split, tt, lds);
+                lmhead_fwd_item<KEEP, TILES == ONE_TILE ? ROUND : NEAR, decltype(nj)::value>(a, fl, first + split, tt, lds);
             };
             if constexpr (TILES != WHOLE_TILES) with_width(tile_width(a.n_tokens, tt * BN, true), item);
             else item(std::integral_constant<int, WIDE>{});
@@ -1084,7 +1078,7 @@ __device__ __forceinline__ void dz_column(const f32x16& z0, const f32x16& z1, co
     }
 }
 
-template <bool ROUND>
+template <Walk WALK>
 __device__ __forceinline__ void lmhead_dz_tile(const uint16_t* __restrict__ W, const uint16_t* __restrict__ hidden,
                                                const DzInputs& in, int64_t hdim, int64_t v_begin, int64_t chunk_cols,
                                                uint16_t* __restrict__ dz, int64_t vt, int64_t tt, uint16_t* lds) {
@@ -1093,8 +1087,8 @@ __device__ __forceinline__ void lmhead_dz_tile(const uint16_t* __restrict__ W, c
 
     AccTile<> acc;
     // as the forward, so that the logits are its to the bit
-    gemm_tile<ROUND>(acc, W, hdim, m0, in.vocab, hidden, hdim, n0, in.n_tokens, hdim, lds,
-                     ROUND ? first_k_tile(m0 / BM, hdim) : 0);
+    gemm_tile<WALK>(acc, W, hdim, m0, in.vocab, hidden, hdim, n0, in.n_tokens, hdim, lds,
+                    WALK == ROUND ? first_k_tile(m0 / BM, hdim) : 0);
 
     uint16_t* stage = lds;
 #pragma unroll
@@ -1115,7 +1109,7 @@ __device__ __forceinline__ void lmhead_dz_tile(const uint16_t* __restrict__ W, c
     }
 }
 
-template <bool ROUND>
+template <Walk WALK>
 __global__ void __launch_bounds__(NTHREADS)
     lmhead_dz_kernel(const uint16_t* __restrict__ W, const uint16_t* __restrict__ hidden, DzInputs in,
                      const int32_t* __restrict__ n_dev, int64_t hdim, int64_t v_begin, int64_t chunk_cols, int64_t n_pad,
@@ -1126,7 +1120,7 @@ __global__ void __launch_bounds__(NTHREADS)
         n_pad = (in.n_tokens + BN - 1) / BN * BN;
     }
     for_each_tile(queue, chunk_cols / BM, n_pad / BN, lds, [&](int64_t vt, int64_t tt) {
-        lmhead_dz_tile<ROUND>(W, hidden, in, hdim, v_begin, chunk_cols, dz, vt, tt, lds);
+        lmhead_dz_tile<WALK>(W, hidden, in, hdim, v_begin, chunk_cols, dz, vt, tt, lds);
     });
 }
 
@@ -1701,7 +1695,7 @@ __device__ __forceinline__ void store_group_any(const f32x16& z0, const f32x16& 
     }
 }
 
-// one workgroup per tile id, width < 8
+// one workgroup per tile id, any width
 template <bool R_KM, bool C_KM>
 __global__ void __launch_bounds__(NTHREADS)
     gemm_any_kernel(Operand R, int64_t M, Operand C, int64_t N, int64_t K, int mode, float* out_f32, uint16_t* out_bf16,
@@ -1716,7 +1710,7 @@ __global__ void __launch_bounds__(NTHREADS)
     R.r0 = tr * BN;
     C.r0 = tc * BM;
     AccTile<> acc;
-    gemm_tile<C_KM, R_KM>(acc, C, R, K, lds);
+    gemm_tile<C_KM, R_KM, FAR>(acc, C, R, K, lds);
     const int tid = opaque_tid();
     // two regions in turn, as in store_tile
 #pragma unroll
@@ -1735,7 +1729,9 @@ int launch_product(const Operand& a, int64_t M, const Operand& b, int64_t N, int
     const int width = store_width(mode, out_f32 ? static_cast<void*>(out_f32) : out_bf16, N, ldo);
     const dim3 grid(grid_for_tiles((M + BM - 1) / BM, (N + BN - 1) / BN));
     uint16_t* o16 = static_cast<uint16_t*>(out_bf16);
-    if (width == 8)
+    // both operands one row each (pitch 0): the only k-contiguous ones that can be longer than a pitch
+    const bool far = !R_KM && !C_KM && K > MAX_LD;
+    if (width == 8 && !far)
         hipLaunchKernelGGL((gemm_store_kernel<R_KM, C_KM>), grid, dim3(NTHREADS), 0, s, a, M, b, N, K, mode, out_f32, o16, ldo, M,
                            DynRows{}, static_cast<uint32_t*>(nullptr), static_cast<float*>(nullptr));
     else
@@ -2493,7 +2489,7 @@ void enqueue_bwd(const BwdPlan& p, char* ws, const RowInputs& in, const void* we
                                dim3(NTHREADS), 0, s, logits, p.n_pad / BN, di, in.n_dev,
                                row_tiles(n_tokens, hidden_dim) != WHOLE_TILES, cols, dz);
         else
-            hipLaunchKernelGGL((row_tiles(n_tokens, hidden_dim) == ONE_TILE ? lmhead_dz_kernel<true> : lmhead_dz_kernel<false>),
+            hipLaunchKernelGGL((row_tiles(n_tokens, hidden_dim) == ONE_TILE ? lmhead_dz_kernel<ROUND> : lmhead_dz_kernel<NEAR>),
                                grid_of(cols / BM, p.n_pad / BN), dim3(NTHREADS), 0, s, Wp, in.hidden, di, in.n_dev, hidden_dim, v_begin, cols, p.n_pad, dz, q);
         const bool first = ci == 0, last = ci == p.n_chunks - 1;
         const int mode = last ? (first ? 2 : 3) : (first ? 0 : 1);

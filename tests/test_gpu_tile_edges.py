@@ -181,6 +181,25 @@ def test_products_added_to_rows_far_apart(m, n, ldo):
     assert rc == 0 and torch.equal(rows, before + a.float() @ b.float().t())
 
 
+# operands of one row each (pitch 0), to and past the longest range that other operands have
+@pytest.mark.parametrize("k", [1 << 22, (1 << 22) + 64])
+@pytest.mark.parametrize("m,n", [(1, 1), (3, 264)])
+def test_products_of_one_long_row(m, n, k):
+    """Entries in -1 .. 1: every sum is a whole number below 2**24, so any order of the additions gives it."""
+    print("case one row", m, n, k, flush=True)
+    g = torch.Generator(device=DEV).manual_seed(n)
+    a, b = (torch.randint(-1, 2, (k,), generator=g, device=DEV).bfloat16() for _ in range(2))
+    exact = (a.float() * b.float()).double().sum().float()
+    for dtype, accumulate in ((torch.float32, 0), (torch.float32, 1), (torch.bfloat16, 0)):
+        out = torch.full((m, n), 3.0, dtype=dtype, device=DEV)
+        o = out.data_ptr()
+        rc = _lib.load().oi_gemm_bf16_tn(
+            a.data_ptr(), 0, m, b.data_ptr(), 0, n, k, o if dtype == torch.float32 else None,
+            o if dtype == torch.bfloat16 else None, n, accumulate, torch.cuda.current_stream().cuda_stream,
+        )  # fmt: skip
+        assert rc == 0 and (out == (exact + 3.0 * accumulate).to(dtype)).all(), (dtype, accumulate)
+
+
 @pytest.mark.parametrize("n,h,v,flagged,slabs", [(1, 64, 300, 1, 4096), (300, 64, 301, 70, 4096), (600, 320, 513, 257, 256)])
 def test_flagged_rows_are_added_to_d_weight(n, h, v, flagged, slabs):
     """Rows whose label lies more than 44 nats below the largest logit are recomputed and added to the bf16 d_weight
