@@ -421,6 +421,11 @@ __global__ void __launch_bounds__(256)
 // may be; several rows per wave take longer ([64, 256] 7.0, 7.9; [256, 64] 7.0, 21).
 constexpr int SMALL_THREADS = 1024, SMALL_WAVES = SMALL_THREADS / OI_WAVE;
 constexpr int64_t SMALL_ELEMS = 16384, SMALL_COLS = 2048;
+// So long as a CU holds all of its workgroups at once (two of 1024 threads), or has one where a mean per row leaves a
+// wave alone with a chain of reads.  Beyond, smaller workgroups come out ahead: [e, 1, 2048] 7.4 us here and 8.9 with two
+// launches at e = 512, 10.7 and 9.5 at 768, 0.88 and 0.45 ms at 65535; means of rows 8.2 and 8.4 at 256, 13.2 and 8.4 at
+// 257, 3.74 and 0.45 ms at 65535.
+constexpr int64_t SMALL_EXTRA = 512, SMALL_EXTRA_ROWS = 256;
 __global__ void __launch_bounds__(SMALL_THREADS)
     masked_small_kernel(const float* __restrict__ values, const void* __restrict__ mask, int mask_is_float, int rows,
                         int cols, int axis_mode, float denominator, float* __restrict__ out,
@@ -940,7 +945,8 @@ extern "C" int oi_masked_mean_fwd(const float* values, const void* mask, int mas
     float* partial = static_cast<float*>(workspace);
     float* cnt = partial + extra * rows * nchunks;
     hipStream_t s = static_cast<hipStream_t>(stream);
-    if (rows <= SMALL_ELEMS / cols && (axis_mode == 0 || (rows <= SMALL_WAVES && cols <= SMALL_COLS))) {
+    if (rows <= SMALL_ELEMS / cols && extra <= (axis_mode == 0 ? SMALL_EXTRA : SMALL_EXTRA_ROWS) &&
+        (axis_mode == 0 || (rows <= SMALL_WAVES && cols <= SMALL_COLS))) {
         hipLaunchKernelGGL(masked_small_kernel, dim3((unsigned)extra), dim3(SMALL_THREADS), 0, s, values, mask, mask_is_float,
                            (int)rows, (int)cols, axis_mode, denominator, out, row_denoms);
         return oi_launch_status();

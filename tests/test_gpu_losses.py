@@ -83,6 +83,19 @@ def test_masked_mean_sizes_of_one_launch(rows, cols, axis):
     assert (dv.grad.cpu().double() - ref_v.grad).abs().max().item() <= 2.0**-22 * ref_v.grad.abs().max().item()
 
 
+# both sides of the leading entries that go in one launch
+@pytest.mark.parametrize("extra,axis", [(512, None), (513, None), (256, 1), (257, 1), (65535, 1)])
+def test_masked_mean_of_many_leading_entries(extra, axis):
+    g = torch.Generator().manual_seed(extra)
+    values = torch.randn(extra, 2, 33, generator=g)
+    mask = torch.rand(2, 33, generator=g) > 0.3
+    kept = values.double() * mask
+    ref = kept.sum((1, 2)) / mask.sum() if axis is None else (kept.sum(2) / mask.sum(1)).mean(1)
+    out = rl_utils.masked_mean(values.to(DEV), mask.to(DEV), axis)
+    # fp32 at most: 6 roundings of a wave's sum, 3 of the four waves', and that of the result, none of more than the largest
+    assert (out.cpu().double() - ref).abs().max().item() <= 10 * 2.0**-24 * values.abs().amax().item()
+
+
 def test_masked_mean_scalar_cases():
     v = torch.tensor([[1.0, 2.0, 3.0], [4.0, 5.0, 6.0]], device=DEV)
     m = torch.tensor([[True, True, False], [True, False, False]], device=DEV)
