@@ -1198,8 +1198,10 @@ static_assert(2 * GROUP_F32 <= LDS_ELEMS, "the epilogue's regions fit the ring")
 // A wave's loads and stores leave its counter in the order in which they were issued, so a load behind a group's stores
 // is not there before those have reached memory.  PLAIN products (no factors of rows, no row index) therefore have no
 // such loads in their code (behind a branch, their waits stand in everybody's way: each store of d_weight waited for the
-// one before), and what they are added to is requested one group ahead.  d_weight of 268 rows 430 -> 382 us, of 3072
-// rows (128256 x 4096) 2.22 -> 2.16 ms.
+// one before).  d_weight of 268 rows 430 -> 382 us, of 3072 rows (128256 x 4096) 2.22 -> 2.16 ms.  What a product is
+// added to is read group by group all the same: requested one group ahead, reads meet the stores of the group before,
+// and sums of few k-tiles lose what those of many do not gain (100352 x 4096, us so and one group ahead: K = 320 791,
+// 843; K = 1024 1156, 1196; 128256 x 4096, K = 7680 6000, 6005).
 //
 // Rows and columns past the end read what the last valid ones do, and store nothing.
 template <bool PLAIN, int PIECES>
@@ -1286,11 +1288,10 @@ struct F32Rows {
         }
     }
 };
-// `staged` is called when the accumulators are in the LDS.
-template <bool PLAIN, bool ADDS, class Staged>
+template <bool PLAIN, bool ADDS>
 __device__ __forceinline__ void store_group_f32(const f32x16& z0, const f32x16& z1, const StoreTo& st, bool pieces,
                                                 const F32Rows<PLAIN, ADDS>& in, int64_t row0, int64_t col0, int j,
-                                                uint16_t* stage, int tid, Staged&& staged) {
+                                                uint16_t* stage, int tid) {
     asm volatile("" : "+v"(tid));
     const int lane = tid & 63, wave = tid >> 6, wm = wave & 3, wn = wave >> 2;
     const int mode = st.mode, srow = wn * 32 + (lane & 31);
@@ -1307,8 +1308,6 @@ __device__ __forceinline__ void store_group_f32(const f32x16& z0, const f32x16& 
                 oi_f32x4{rows.scale(st, z[q * 4]), rows.scale(st, z[q * 4 + 1]), rows.scale(st, z[q * 4 + 2]),
                          rows.scale(st, z[q * 4 + 3])};
         }
-    __builtin_amdgcn_sched_barrier(0);
-    staged();
     lds_barrier();
     const float* from = stage32 + r_first * STAGE_F32 + ch * 4;
     auto piece = [&](int it) {
@@ -1366,17 +1365,13 @@ struct ProductTile {
 template <bool PLAIN, bool ADDS>
 __device__ __forceinline__ void store_tile_f32(const AccTile<>& acc, const ProductTile& t, const StoreTo& st, bool pieces,
                                                uint16_t* lds, int tid) {
-    constexpr bool AHEAD = PLAIN && ADDS;
-    F32Rows<PLAIN, ADDS> in[2];
-    if (AHEAD) in[0].request(st, t.R.r0, t.C.r0, 0, tid);
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
         __builtin_amdgcn_sched_barrier(0);
-        if (!AHEAD) in[j & 1].request(st, t.R.r0, t.C.r0, j, tid);
+        F32Rows<PLAIN, ADDS> in;
+        in.request(st, t.R.r0, t.C.r0, j, tid);
         const Columns c = tile_columns(acc, j);
-        store_group_f32<PLAIN, ADDS>(c.z[0], c.z[1], st, pieces, in[j & 1], t.R.r0, t.C.r0, j, lds + (j & 1) * GROUP_F32, tid, [&] {
-            if (AHEAD && j < 3) in[(j + 1) & 1].request(st, t.R.r0, t.C.r0, j + 1, tid);
-        });
+        store_group_f32<PLAIN, ADDS>(c.z[0], c.z[1], st, pieces, in, t.R.r0, t.C.r0, j, lds + (j & 1) * GROUP_F32, tid);
         __builtin_amdgcn_sched_barrier(0);
     }
 }
@@ -1835,11 +1830,11 @@ __global__ void __launch_bounds__(NTHREADS)
     if (adds_in_pieces(st, pieces)) {
         F32Rows<false, true> in;
         in.request(st, row0, col0, j, tid);
-        store_group_f32<false, true>(c.z[0], c.z[1], st, pieces, in, row0, col0, j, stage, tid, [] {});
+        store_group_f32<false, true>(c.z[0], c.z[1], st, pieces, in, row0, col0, j, stage, tid);
     } else {
         F32Rows<false, false> in;
         in.request(st, row0, col0, j, tid);
-        store_group_f32<false, false>(c.z[0], c.z[1], st, pieces, in, row0, col0, j, stage, tid, [] {});
+        store_group_f32<false, false>(c.z[0], c.z[1], st, pieces, in, row0, col0, j, stage, tid);
     }
 }
 
