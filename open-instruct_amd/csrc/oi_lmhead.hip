@@ -591,6 +591,9 @@ __device__ __forceinline__ int acc_col(int wn, int j, int lane) { return wn * 16
 // The products behind it have whole tiles only: among them narrow ones gain nothing, as the pieces that tiles are cut
 // into stop being alike (d_hidden of 268 rows 312, so 322).
 inline bool narrow_tiles(int64_t rows, int64_t hdim) { return rows <= 2 * BN || (rows <= 16 * BN && hdim <= 6144); }
+// What a narrow tile leaves in memory ends with it.  d_weight's k-tiles, the only reader of rows past the last one, do so
+// at the same row or before.
+static_assert(32 * 2 % BK == 0, "rows past the end are written to the end of the last k-tile");
 __device__ __forceinline__ int tile_width(int64_t rows, int64_t row0, bool narrow) {
     const int64_t left = rows - row0;
     if (!narrow || left > 192) return WIDE;
@@ -747,7 +750,8 @@ __device__ __forceinline__ oi_u32x4 staged_piece(const uint16_t* share, int lane
 // forward: per-token softmax statistics over the vocabulary tiles of one split
 // ---------------------------------------------------------------------------------------------
 // CACHE: the vocabulary tiles [cache_tile0, cache_tile0 + cache_tiles) also leave 2^(z c - xref[n])
-// behind as bf16, token-major [n_pad, cache_ld]; rows of tokens past the end are zero.
+// behind as bf16, token-major [n_pad, cache_ld]; rows of tokens past the end are zero up to the next multiple of 64 and
+// not written behind it, where the last tile is narrow.
 // LOGITS: every tile leaves its fp32 logits behind (store_part), tile (vt, tt) at logits +
 // (vt * logits_tiles + tt) * PART_FLOATS.
 // What a forward launch covers and where its exponentials go.  Splits [0, long_splits) take
@@ -1500,7 +1504,7 @@ __global__ void __launch_bounds__(NTHREADS)
     if (dyn.n_dev && dyn.role == 1) R.extent = z.M;
     if (dyn.n_dev && dyn.role == 2) {
         const int64_t n = device_count(dyn.n_dev);
-        R.k_valid = (n + BM - 1) / BM * BM;
+        R.k_valid = z.K;  // rows of dZ behind these are not defined
         C.k_valid = n;
     }
     K = z.K;
@@ -1746,9 +1750,9 @@ __global__ void __launch_bounds__(NTHREADS)
     __shared__ __align__(16) uint16_t lds[LDS_ELEMS];
     const int64_t n = device_count(n_dev);
     if (n <= 0) return;
-    R.k_valid = (n + BM - 1) / BM * BM;
-    C.k_valid = n;
     const int64_t K = (n + BK - 1) / BK * BK;
+    R.k_valid = K;
+    C.k_valid = n;
     for_each_tile(queue, (M + BN - 1) / BN, (N + BM - 1) / BM, lds, [&](int64_t tr, int64_t tc) {
         R.r0 = tr * BN;
         C.r0 = tc * BM;
@@ -2444,8 +2448,8 @@ __global__ void __launch_bounds__(256)
 }
 
 // The recomputing backward.  Per vocabulary chunk: dZ [n_pad, cols] (token-major, bf16, zero in padded
-// rows and columns), then both products straight from W and the (selected) hidden rows, which enter
-// as k-major operands:
+// columns and in padded rows up to the next k-tile; rows behind it may never have been written), then both
+// products straight from W and the (selected) hidden rows, which enter as k-major operands:
 //   d_hidden[n, h] (+)= sum_v dZ[n, v] * W[v_begin + v, h]      A k-contiguous, B k-major
 //   d_weight[v_begin + v, h] = sum_n dZ[n, v] * hidden[n, h]    A k-major,      B k-major
 // The sums stop at the last real vocabulary row / token (rounded up to a k-tile, whose missing
@@ -2496,7 +2500,7 @@ void enqueue_bwd(const BwdPlan& p, char* ws, const RowInputs& in, const void* we
                                 dh32, d_hidden, hidden_dim, n_tokens, dyn, q + QUEUE_WORDS, parts, s);
         }
         if (d_weight) {
-            const Operand a = {dz, cols, 0, cols, p.n_pad};
+            const Operand a = {dz, cols, 0, cols, round_up(n_tokens, BK)};
             const Operand b = {in.hidden, hidden_dim, 0, hidden_dim, n_tokens};
             uint16_t* dw = static_cast<uint16_t*>(d_weight) + v_begin * hidden_dim;
             const dim3 grid = grid_of(cols / BM, h_tiles);

@@ -283,3 +283,42 @@ def test_products_that_begin_at_another_k_tile(n, h):
         _close(w.grad, dw, "d_weight")
         grads.append(hid.grad)
     assert torch.equal(*grads)
+
+
+# token counts in each width of the last tile; a narrow tile leaves the rows behind it as they were
+@pytest.mark.parametrize("n", [1, 64, 65, 100, 130, 193, 300])
+@pytest.mark.parametrize("masked", [False, True])
+def test_old_contents_of_scratch_memory_do_not_matter(n, masked, monkeypatch):
+    """Scratch memory full of NaN bits gives the results that other contents give, to the bit."""
+    h, v = 192, 700
+    hidden, weight, labels, mask, upstream = _inputs(n, h, v, seed=n)
+    mask[0] = True  # an empty selection has no mean
+    sel = mask if masked else None
+    empty, empty_like = torch.empty, torch.empty_like
+
+    def filled(t):
+        t.untyped_storage().fill_(255)
+        return t
+
+    def results():
+        out = []
+        for keep_logits, frozen in ((True, False), (False, False), (False, True)):
+            hid, w = hidden.clone().requires_grad_(True), weight.clone().requires_grad_(not frozen)
+            lp = lm_head.fused_lm_head_logprobs(hid, w, labels, mask=sel, keep_logits=keep_logits)
+            lp = lp[0] if isinstance(lp, tuple) else lp
+            lp.backward(upstream)
+            out += [lp.detach(), hid.grad] + ([] if frozen else [w.grad])
+        hid, w = hidden.clone().requires_grad_(True), weight.clone().requires_grad_(True)
+        y = labels.masked_fill(~mask, -100) if masked else labels
+        loss = lm_head.fused_linear_cross_entropy(hid[None], w, shift_labels=y[None], token_slabs=True)
+        loss.backward()
+        return out + [loss.detach(), hid.grad, w.grad]
+
+    print(f"case N={n} masked={masked}", flush=True)
+    exp = results()
+    monkeypatch.setattr(torch, "empty", lambda *a, **k: filled(empty(*a, **k)))
+    monkeypatch.setattr(torch, "empty_like", lambda *a, **k: filled(empty_like(*a, **k)))
+    got = results()
+    monkeypatch.undo()
+    for i, (a, b) in enumerate(zip(got, exp)):
+        assert torch.equal(a, b), i
