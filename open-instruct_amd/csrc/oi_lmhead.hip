@@ -715,11 +715,12 @@ __device__ __forceinline__ void stats_update(f32x16 (&z)[2], int wm, int lane, i
 // (tokens, or rows of a product) wn * 16 NJ + j * 32 + (0..31) of both wn halves with all 256 columns (every m-wave
 // contributes its 64).  A lane holds groups of eight consecutive columns of one row; a wave's meet in its share of one
 // ring slot and go to global memory as whole 128-byte lines, eight rows at a time.  The waves do not wait for each
-// other: with rows of 512 bytes that all waves fill there were two barriers per group (d_weight of 268 rows 404 us, now
-// 391, of 2340 rows x 128256 1934, now 1907; step of 268 rows 1117, now 1095).
+// other: with rows of 512 bytes that all waves fill there were two barriers per group (d_weight of 268 rows x 100352
+// 370 us, now 356, of 2340 rows x 128256 1983, now 1960; step of 268 rows 985, now 969).
 //
-// A share: 32 rows of 128 bytes, unpadded; the 16-byte pieces of a row at c ^ piece_perm(row), which puts the
-// 16-byte stores of 16 rows, and those of a row pair, on all 64 banks.
+// A share: 32 rows of 128 bytes, unpadded; the 16-byte pieces of a row at c ^ piece_perm(row), which spreads the
+// 16-byte accesses of 16 rows, and those of a row pair, over all 64 banks.  Counters still show 1000 conflict cycles per
+// tile of 256 x 256, four for each access; under 1 % of a tile of 64 k-tiles.
 __device__ __forceinline__ int piece_perm(int row) { return row >> 1 & 7; }
 constexpr int GROUP_ROWS = 64;
 constexpr int GROUP_BF16_AT = 4 * TILE_ELEMS;  // ring slot 4: slots 0 .. 3 may be filling for the next tile
@@ -796,7 +797,7 @@ __device__ __forceinline__ FwdColumn fwd_column(const FwdArgs& a, const float* x
     return col;
 }
 // Column group j of vocabulary tile vt: the label's logit, the statistics and, where they are kept, the
-// exponentials (through `stage`; every thread of the workgroup takes part).
+// exponentials (through the wave's share of `stage`; every lane of the wave takes part).
 template <FwdKeep KEEP, int NJ>
 __device__ __forceinline__ void fwd_fold(f32x16 (&__restrict__ z)[2], FwdColumn& col, const FwdArgs& a, const FwdLaunch& fl,
                                          int64_t vt, int64_t n0, int j, int tid, uint16_t* stage) {
@@ -1129,9 +1130,9 @@ __global__ void __launch_bounds__(NTHREADS)
 }
 
 // The same dZ (to the bit) from the logits that the forward left behind as fp32 tiles, whole vocabulary at
-// once.  Workgroup (j, tt, vt) takes column group j of tile (vt, tt): 64 tokens (wn * 128 + j * 32 + 0..31 of
-// both wn halves) x 256 vocabulary columns, 64 KB in and 32 KB out.  A quarter of a tile per workgroup so that
-// four of them share a CU and one's stores run beside another's loads.
+// once.  Workgroup (j, tt, vt) takes column group j of tile (vt, tt): 64 tokens (j * 32 + 0..31 of both halves of the
+// tile's width, which is the forward's) x 256 vocabulary columns, 64 KB in and 32 KB out.  A quarter of a whole tile per
+// workgroup so that four of them share a CU and one's stores run beside another's loads.
 constexpr int KEPT_ROWS = 64;
 __global__ void __launch_bounds__(NTHREADS)
     lmhead_dz_kept_kernel(const float* __restrict__ logits, int64_t logits_tiles, DzInputs in,
@@ -1183,9 +1184,9 @@ __device__ __forceinline__ bool stores_in_pieces(const StoreTo& st) {
     return st.mode <= 1 || (reinterpret_cast<uintptr_t>(st.out_bf16) & 15) == 0;
 }
 
-// Column group j of a finished tile is its rows row0 + wn * 128 + j * 32 + (0..31) of both wn halves with all 256
-// columns from col0.  z0, z1: the lane's accumulators, row acc_col(wn, j, lane), columns acc_row(wm, 0 / 1, r,
-// lane), i.e. groups of four consecutive columns of one row.  bf16 goes through the wave's share of the LDS and
+// Column group j of a finished tile (products have whole ones) is its rows row0 + wn * 128 + j * 32 + (0..31) of both wn
+// halves with all 256 columns from col0.  z0, z1: the lane's accumulators, row acc_col(wn, j, lane), columns acc_row(wm,
+// 0 / 1, r, lane), i.e. groups of eight consecutive columns of one row.  bf16 goes through the wave's share of the LDS and
 // leaves 128 bytes of a row at a time; fp32 meets in the LDS region `stage` (64 rows) and leaves as whole rows of 1 KB,
 // every thread of the workgroup taking part.
 //
@@ -1193,8 +1194,8 @@ __device__ __forceinline__ bool stores_in_pieces(const StoreTo& st) {
 // and whole lines.  Registers transposed in quads of lanes and stored from there in 64-byte pieces, with a wait
 // for the stores of the tile before the next tile's first load: d_weight of 268 rows (100352 x 4096, 6272
 // tiles of 5 k-tiles) 606 us; through the LDS 544; without waiting for stores at its barriers 504; with the next tile's
-// first loads ahead of it 478; without waiting for each store before the next 382 (with the tile engine's other changes);
-// without barriers 3 % less.
+// first loads ahead of it 478.  On a faster box that form took 417; without waiting for each store before the next (and
+// with the tile engine's other changes) 370; without barriers 356.
 constexpr int STAGE_F32 = BM + 4;                            // floats per row: rows 4 banks apart
 constexpr int GROUP_F32 = GROUP_ROWS * STAGE_F32 * 2;        // LDS elements of an fp32 region
 static_assert(2 * GROUP_F32 <= LDS_ELEMS, "the epilogue's regions fit the ring");
@@ -1202,10 +1203,10 @@ static_assert(2 * GROUP_F32 <= LDS_ELEMS, "the epilogue's regions fit the ring")
 // A wave's loads and stores leave its counter in the order in which they were issued, so a load behind a group's stores
 // is not there before those have reached memory.  PLAIN products (no factors of rows, no row index) therefore have no
 // such loads in their code (behind a branch, their waits stand in everybody's way: each store of d_weight waited for the
-// one before).  d_weight of 268 rows 430 -> 382 us, of 3072 rows (128256 x 4096) 2.22 -> 2.16 ms.  What a product is
-// added to is read group by group all the same: requested one group ahead, reads meet the stores of the group before,
-// and sums of few k-tiles lose what those of many do not gain (100352 x 4096, us so and one group ahead: K = 320 791,
-// 843; K = 1024 1156, 1196; 128256 x 4096, K = 7680 6000, 6005).
+// one before: an eighth of d_weight of 268 rows, 3 % of that of 3072).  What a product is added to is read group by
+// group all the same: requested one group ahead, reads meet the stores of the group before, and sums of few k-tiles lose
+// what those of many do not gain (100352 x 4096, us so and one group ahead: K = 320 791, 843; K = 1024 1156, 1196;
+// 128256 x 4096, K = 7680 6000, 6005).
 //
 // Rows and columns past the end read what the last valid ones do, and store nothing.
 template <bool PLAIN, int PIECES>
@@ -1339,7 +1340,7 @@ __device__ __forceinline__ void store_group_f32(const f32x16& z0, const f32x16& 
         }
         return;
     }
-    // bf16 rows off 8-byte boundaries
+    // bf16 in 4-byte words: rows off 16-byte boundaries, and every row of mode 2 that comes here (added pieces of tiles)
     if (col >= st.N) return;
 #pragma unroll 1
     for (int it = 0; it < F32_PIECES; ++it) {
@@ -1357,7 +1358,8 @@ __device__ __forceinline__ bool adds_in_pieces(const StoreTo& st, bool pieces) {
 
 // out[row, col] = sum_k R(row, k) * C(col, k).  R's rows (token or vocabulary rows of the result) are the tile
 // product's n dimension and C's (the result's columns) its m dimension, because a lane's consecutive
-// accumulators are consecutive in m: four columns of one row, which the epilogue stores without a transpose.
+// accumulators are consecutive in m: after the swap of lane quarters eight columns of one row, which the epilogue
+// stores without a transpose.
 // One tile, or with `part` a piece of one along k whose fp32 tile goes there and nowhere else.
 struct ProductTile {
     Operand R, C;

@@ -145,7 +145,7 @@ _PICK_MAX = 32768
 
 
 def _picked(values: torch.Tensor, mask_u8: torch.Tensor) -> torch.Tensor:
-    """``values[mask]`` as a new 1-D tensor."""
+    """``values[mask]``, 1-D; up to ``_PICK_MAX`` values the start of a buffer as long as ``values``."""
     n = values.numel()
     if not 0 < n <= _PICK_MAX:
         return values[mask_u8.bool()]

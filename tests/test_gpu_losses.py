@@ -869,18 +869,20 @@ def test_rho_histogram_is_the_selection_in_order(shape, kept):
 
 
 @pytest.mark.parametrize("sample_idx", [0, 6, -1])  # the last by the general way
-def test_recorded_column_equals_the_general_way(sample_idx):
+def test_recorded_column_equals_the_general_way(sample_idx, monkeypatch):
     g = torch.Generator().manual_seed(5)
     t = lambda: torch.randn(2, 70, generator=g).to(DEV)  # noqa: E731
     mask = (torch.rand(2, 70, generator=g) < 0.7).to(DEV)
     cfg = make_grpo_config(load_ref_policy=True, beta=0.05)
     new, old, ref, adv, ent = t(), t(), t(), t(), t()
     loss, stats = grpo_utils.grpo_loss_fused(new, old, ref, adv, mask, cfg, entropy=ent)
-    tables = []
+    tables, calls, call = [], [], _lib.call
+    monkeypatch.setattr(_lib, "call", lambda name, *args: (calls.append(name), call(name, *args))[1])
     for recorded in (stats, {k: v for k, v in stats.items()}):
         table = grpo_utils.create_loss_stats(7, DEV, record_entropy=True)
         table.table.fill_(7.0)
         total = loss if recorded is stats else loss.double()  # the general way
         grpo_utils.populate_sample_loss_stats(table, sample_idx, None, None, None, total, mask, new, ref, ent, cfg, fused_stats=recorded)
         tables.append(table.table)
+    assert calls.count("oi_record_stats") == (1 if sample_idx >= 0 else 0)
     assert torch.equal(*tables)
