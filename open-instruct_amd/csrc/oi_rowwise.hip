@@ -181,6 +181,33 @@ __device__ __forceinline__ int64_t row_head(const typename R::elem_t* p, int64_t
 constexpr int FWD_UNROLL = 4;
 constexpr int FWD_MAX_THREADS = 1024;
 
+// A forward whose backward will read the same logits (it is asked for lse) leaves the last rows in the memory-side cache
+// (256 MB), where the backward begins: it takes the rows from the last one down.  The rows ahead of them are read past the
+// cache as before: through it, they would push out the ones that matter and cost the forward 11 to 15 %.  Backward, us
+// before and after: bf16 2036 x 151665 193, 176; 800 x 128256 67, 53; 4096 x 100352 250, 237; 12000 x 128256 931, 906;
+// fp32 2000 x 32000 87, 71; 2048 x 151936 410, 378; the forwards within 2 %.
+constexpr int64_t CACHED_BYTES = (int64_t)224 << 20;
+
+// full groups of FWD_UNROLL vectors per lane from vector i on: all loads are issued before the first use.  Returns the
+// lane's first vector behind them.
+template <typename R, bool ENT, bool CACHED>
+__device__ __forceinline__ int64_t fwd_groups(RowStat& st, const typename R::elem_t* __restrict__ body, int64_t i, int64_t nvec,
+                                              int nthr, float c) {
+    constexpr int VEC = R::VEC;
+    for (; i + (int64_t)(FWD_UNROLL - 1) * nthr < nvec; i += (int64_t)FWD_UNROLL * nthr) {
+        float z[FWD_UNROLL][VEC];
+#pragma unroll
+        for (int u = 0; u < FWD_UNROLL; ++u) {
+            const typename R::elem_t* at = body + (i + (int64_t)u * nthr) * VEC;
+            if constexpr (CACHED) R::unpack(R::load_raw_cached(at), z[u]);
+            else R::load_vec(at, z[u]);
+        }
+#pragma unroll
+        for (int u = 0; u < FWD_UNROLL; ++u) stat_update<VEC, ENT>(st, z[u], c);
+    }
+    return i;
+}
+
 template <typename R, bool ENT>
 __global__ void __launch_bounds__(FWD_MAX_THREADS) lsg_entropy_fwd_kernel(const typename R::elem_t* __restrict__ logits,
                                                               int64_t n_inner, int64_t stride_outer,
@@ -199,14 +226,9 @@ __global__ void __launch_bounds__(FWD_MAX_THREADS) lsg_entropy_fwd_kernel(const 
     const typename R::elem_t* body = p + head;
     const int64_t nvec = (vocab - head) / VEC;
     int64_t i = tid;
-    // full groups of FWD_UNROLL vectors per lane: all loads are issued before the first use
-    for (; i + (int64_t)(FWD_UNROLL - 1) * nthr < nvec; i += (int64_t)FWD_UNROLL * nthr) {
-        float z[FWD_UNROLL][VEC];
-#pragma unroll
-        for (int u = 0; u < FWD_UNROLL; ++u) R::load_vec(body + (i + (int64_t)u * nthr) * VEC, z[u]);
-#pragma unroll
-        for (int u = 0; u < FWD_UNROLL; ++u) stat_update<VEC, ENT>(st, z[u], c);
-    }
+    const bool cached = lse_out && ((int64_t)gridDim.x - row) * vocab * (int64_t)sizeof(typename R::elem_t) <= CACHED_BYTES;
+    if (cached) i = fwd_groups<R, ENT, true>(st, body, i, nvec, nthr, c);
+    else i = fwd_groups<R, ENT, false>(st, body, i, nvec, nthr, c);
     for (; i < nvec; i += nthr) {
         float z[VEC];
         R::load_vec(body + i * VEC, z);
@@ -262,7 +284,7 @@ __global__ void __launch_bounds__(256) lsg_bwd_kernel(const typename R::elem_t* 
                                                       typename R::elem_t* dlogits, int64_t out_stride_outer,
                                                       int64_t out_stride_inner) {
     constexpr int VEC = R::VEC;
-    const int64_t row = blockIdx.x;
+    const int64_t row = (int64_t)gridDim.x - 1 - blockIdx.x;  // see CACHED_BYTES
     const typename R::elem_t* p = logits + row_offset(row, n_inner, stride_outer, stride_inner);
     typename R::elem_t* q = dlogits + row_offset(row, n_inner, out_stride_outer, out_stride_inner);
     const int tid = threadIdx.x, nthr = blockDim.x;
@@ -345,7 +367,7 @@ __global__ void __launch_bounds__(BURST_THREADS)
                          int64_t out_stride_outer, int64_t out_stride_inner) {
     constexpr int VEC = R::VEC;
     constexpr int U = BURST_U;
-    const int64_t row = blockIdx.x;
+    const int64_t row = (int64_t)gridDim.x - 1 - blockIdx.x;  // see CACHED_BYTES
     const typename R::elem_t* p = logits + row_offset(row, n_inner, stride_outer, stride_inner);
     typename R::elem_t* q = dlogits + row_offset(row, n_inner, out_stride_outer, out_stride_inner);
     const int tid = threadIdx.x;

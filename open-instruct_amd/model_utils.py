@@ -109,11 +109,12 @@ class _LogSoftmaxGather(torch.autograd.Function):
         rows = n_outer * n_inner
         logprob = torch.empty(index.shape, dtype=torch.float32, device=dev)
         entropy = torch.empty(index.shape, dtype=torch.float32, device=dev) if want_entropy else None
-        lse = torch.empty(index.shape, dtype=torch.float32, device=dev)
+        # for the backward only: a forward that leaves it also leaves the last rows in the memory-side cache
+        lse = torch.empty(index.shape, dtype=torch.float32, device=dev) if ctx.needs_input_grad[0] else None
         if rows > 0:
             _lib.call(
                 "oi_lsg_entropy_fwd", view.data_ptr(), _lib.DTYPE_TAGS[view.dtype], n_outer, n_inner, so, si, vocab,
-                index.data_ptr(), inv_temperature, logprob.data_ptr(), _lib.ptr(entropy), lse.data_ptr(),
+                index.data_ptr(), inv_temperature, logprob.data_ptr(), _lib.ptr(entropy), _lib.ptr(lse),
                 _lib.stream_of(view),
             )  # fmt: skip
         ctx.save_for_backward(logits, index, lse)

@@ -63,6 +63,32 @@ def test_rows_off_line_boundaries(rows, vocab, dtype):
     assert (leaf.grad[1] == 0).all()
 
 
+# 224 MB of logits from the last row up are read through the caches by a forward with a gradient, the others past them;
+# 895 and 1791 rows of these are as many; odd vocabularies lie off line boundaries
+@pytest.mark.parametrize("rows,vocab,dtype", [(893, 131101, torch.bfloat16), (900, 131101, torch.bfloat16), (1800, 32771, torch.float32)])
+def test_rows_read_through_the_caches_and_past_them(rows, vocab, dtype):
+    print(f"case rows={rows} V={vocab} {dtype}", flush=True)
+    g = torch.Generator(device=DEV).manual_seed(rows)
+    logits = torch.empty(rows, vocab, dtype=dtype, device=DEV).normal_(0, 3, generator=g)
+    index = torch.randint(0, vocab, (rows,), generator=g, device=DEV)
+    upstream = torch.randn(rows, generator=g, device=DEV)
+    leaf = logits.clone().requires_grad_(True)
+    lp, ent = model_utils.logprob_and_entropy(leaf, index)
+    lp.backward(upstream)
+    with torch.no_grad():  # nothing is kept for a backward
+        lp_n, ent_n = model_utils.logprob_and_entropy(logits, index)
+    assert torch.equal(lp, lp_n) and torch.equal(ent, ent_n)
+    edge = rows - (224 << 20) // (vocab * logits.element_size())  # first of the last rows
+    some = sorted({0, 1, max(edge - 1, 0), max(edge, 0), rows // 2, rows - 2, rows - 1})
+    lp_e, ent_e, grad_e = _reference(logits[some], index[some], upstream[some], 1.0)
+    tol = 1e-5 if dtype == torch.float32 else 2e-3
+    assert (lp[some].double() - lp_e).abs().max().item() <= tol and (ent[some].double() - ent_e).abs().max().item() <= tol
+    assert ((leaf.grad[some].double() - grad_e).abs() - (grad_e.abs() * STEP[dtype] + 1e-5)).max().item() <= 0
+    # a gradient row sums to 0 up to its rounding: every row was written, none twice
+    sums = leaf.grad.float().sum(1).abs()
+    assert (sums - upstream.abs() * 2e-2 - 1e-3).max().item() <= 0
+
+
 @pytest.mark.parametrize("shift_in,shift_out,pitch_out", [(0, 1, 0), (3, 3, 0), (5, 2, 0), (0, 0, 8), (0, 0, 3)])
 def test_gradient_rows_placed_otherwise_than_the_logits(shift_in, shift_out, pitch_out):
     """Logits and gradient that start at different places of a line, or have different pitches, through the
