@@ -246,6 +246,13 @@ int oi_pick_values(const float* values, const uint8_t* mask, int64_t n, float* o
 int oi_record_stats(const float* vector, uint32_t row_mask, const float* loss, int loss_row, float* table,
                     int64_t columns, int64_t column, void* stream);
 
+/* Factor of every token's loss in the masked mean of open_instruct/rl_utils.py:426-448:
+ * coef = scale / denominator on set mask bytes, 0 elsewhere (and where the denominator is 0).  axis_mode 0: one
+ * denominator for all rows, axis_mode 1: one per row (`scale` then holds the 1 / rows of the mean over rows); it is
+ * `denominator` if > 0, else the number of set bytes.  mask, coef: [rows, cols]; rows * cols < 2^31. */
+int oi_grpo_token_coef(const uint8_t* mask, int64_t rows, int64_t cols, int axis_mode, float denominator, float scale,
+                       float* coef, void* stream);
+
 /* Group-normalised advantages.  Carries open_instruct/data_loader.py:1472-1484: population std,
  * mode 0 "standard" (s - mean) / (std + 1e-8), mode 1 "centered" s - mean.  Computed in fp64 like
  * the reference's numpy, stored as fp32.  scores: fp64 [n_groups * group_size]. */

@@ -282,6 +282,51 @@ __global__ void __launch_bounds__(256)
     row_denoms[r] = (float)((den > 0.0 ? 1.0 / den : 0.0) / (double)rows);
 }
 
+// coef = scale / denominator on response tokens, 0 elsewhere; the denominator is the number of set mask bytes of the row
+// (axis_mode 1) or of all rows where none is given.  Without axis_mode every workgroup counts all of them itself, so that
+// one launch does (16384 tokens 6 us; as a chain of ten elementwise launches 47 us of the stream).
+constexpr int COEF_THREADS = 1024, COEF_MAX_BLOCKS = 64;
+__global__ void __launch_bounds__(COEF_THREADS)
+    grpo_token_coef_kernel(const uint8_t* __restrict__ mask, int64_t rows, int64_t cols, int axis_mode, float denominator,
+                           float scale, float* __restrict__ coef) {
+    const int64_t n = axis_mode == 0 ? rows * cols : cols;
+    const uint8_t* m = axis_mode == 0 ? mask : mask + blockIdx.x * cols;
+    float* out = axis_mode == 0 ? coef : coef + blockIdx.x * cols;
+    float den = denominator;
+    if (!(denominator > 0.f)) {
+        __shared__ int counts[COEF_THREADS / OI_WAVE];
+        int c = 0;
+        // bytes up to a 16-byte boundary, whole pieces, bytes after the last
+        int64_t head = (16 - (reinterpret_cast<uintptr_t>(m) & 15)) & 15;
+        head = head < n ? head : n;
+        const oi_u32x4* pieces = reinterpret_cast<const oi_u32x4*>(m + head);
+        const int64_t whole = (n - head) / 16;
+        auto set_bytes = [](uint32_t w) {  // non-zero bytes
+            return __popc(((((w & 0x7f7f7f7fu) + 0x7f7f7f7fu) | w) & 0x80808080u));
+        };
+        if ((int64_t)threadIdx.x < head) c += m[threadIdx.x] != 0;
+#pragma unroll 4
+        for (int64_t i = threadIdx.x; i < whole; i += COEF_THREADS) {
+            const oi_u32x4 v = pieces[i];
+            c += set_bytes(v.x) + set_bytes(v.y) + set_bytes(v.z) + set_bytes(v.w);
+        }
+        const int64_t rest = head + whole * 16 + threadIdx.x;
+        if (rest < n) c += m[rest] != 0;
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) c += __shfl_xor(c, off, OI_WAVE);
+        if ((threadIdx.x & 63) == 0) counts[threadIdx.x >> 6] = c;
+        __syncthreads();
+        c = 0;
+#pragma unroll
+        for (int w = 0; w < COEF_THREADS / OI_WAVE; ++w) c += counts[w];
+        den = (float)c;
+    }
+    const float value = (den > 0.f ? 1.f / fmaxf(den, 1e-30f) : 0.f) * scale;
+    const int64_t stride = axis_mode == 0 ? (int64_t)gridDim.x * COEF_THREADS : COEF_THREADS;
+    for (int64_t i = (axis_mode == 0 ? (int64_t)blockIdx.x * COEF_THREADS : 0) + threadIdx.x; i < n; i += stride)
+        out[i] = m[i] ? value : 0.f;
+}
+
 __global__ void grpo_fused_bwd_kernel(const float* __restrict__ nlp, const float* __restrict__ old,
                                       const float* __restrict__ ref, const float* __restrict__ adv,
                                       const uint8_t* __restrict__ mask, const float* __restrict__ rho, int64_t rows,
@@ -832,6 +877,21 @@ int oi_launch_grpo_denoms(const uint8_t* mask, const int32_t* count, int64_t row
                           float denominator, float* row_denoms, hipStream_t s) {
     hipLaunchKernelGGL(grpo_denoms_kernel, dim3((unsigned)(axis_mode == 0 ? 1 : rows)), dim3(256), 0, s, mask, count, rows,
                        cols, axis_mode, denominator, row_denoms);
+    return oi_launch_status();
+}
+
+extern "C" int oi_grpo_token_coef(const uint8_t* mask, int64_t rows, int64_t cols, int axis_mode, float denominator,
+                                  float scale, float* coef, void* stream) {
+    OI_RETURN_IF(rows < 0 || cols < 0 || rows > 0x7fffffffLL || cols > 0x7fffffffLL, OI_EINVAL);
+    OI_RETURN_IF(axis_mode != 0 && axis_mode != 1, OI_EINVAL);
+    const int64_t n = rows * cols;
+    OI_RETURN_IF(n > 0x7fffffffLL, OI_EINVAL);
+    if (n == 0) return OI_OK;
+    OI_RETURN_IF(!mask || !coef, OI_ENULL);
+    const int64_t blocks = (n + COEF_THREADS - 1) / COEF_THREADS;
+    const dim3 grid((unsigned)(axis_mode == 1 ? rows : blocks < COEF_MAX_BLOCKS ? blocks : COEF_MAX_BLOCKS));
+    hipLaunchKernelGGL(grpo_token_coef_kernel, grid, dim3(COEF_THREADS), 0, static_cast<hipStream_t>(stream), mask, rows, cols,
+                       axis_mode, denominator, scale, coef);
     return oi_launch_status();
 }
 

@@ -309,29 +309,43 @@ def _rho_indicator_ptrs(rho_metrics: dict[str, torch.Tensor] | None, shape) -> t
     return [_lib.ptr(t) for t in keep], keep
 
 
+def _fused_cfg(config, axis, loss_denominator, dp_scale) -> tuple:
+    lo, hi = _clip_bounds(config)
+    return (
+        _loss_fn_tag(config), lo, hi, int(config.kl_estimator), float(config.beta), 0 if axis is None else 1,
+        0.0 if loss_denominator is None else float(loss_denominator), float(dp_scale),
+    )  # fmt: skip
+
+
+def _fused_stats(new_logprobs, old, ref, adv, mask, rho, entropy, cfg, rho_metrics=None):
+    """The statistics vector of a micro-batch, and what a backward from its loss needs."""
+    dev = _lib.require_gpu(new_logprobs, old, ref, adv, mask, rho, entropy)
+    loss_fn, lo, hi, kl_estimator, beta, axis_mode, denominator, scale = cfg
+    nl = _lib.f32c(new_logprobs)
+    if nl.ndim != 2:
+        raise ValueError("grpo_loss_fused expects [rows, cols] tensors")
+    rows, cols = nl.shape
+    sides = [None if t is None else _lib.f32c(t.expand(rows, cols)) for t in (old, ref, adv, rho, entropy)]
+    old_c, ref_c, adv_c, rho_c, ent_c = sides
+    m = _lib.mask_u8(mask.expand(rows, cols))
+    stats = torch.empty(len(GRPO_STAT_NAMES), dtype=torch.float32, device=dev)
+    row_denoms = torch.empty(rows, dtype=torch.float32, device=dev)
+    ws_bytes = _lib.load().oi_grpo_fused_workspace_bytes(rows, cols)
+    ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
+    rho_ptrs, _alive = _rho_indicator_ptrs(rho_metrics, (rows, cols))
+    _lib.call(
+        "oi_grpo_fused_fwd", nl.data_ptr(), _lib.ptr(old_c), _lib.ptr(ref_c), adv_c.data_ptr(), m.data_ptr(),
+        _lib.ptr(rho_c), _lib.ptr(ent_c), *rho_ptrs, rows, cols, loss_fn, lo, hi, kl_estimator, beta, axis_mode,
+        denominator, scale, stats.data_ptr(), row_denoms.data_ptr(), ws.data_ptr(), ws_bytes, _lib.stream_of(nl),
+    )  # fmt: skip
+    return stats, (nl, old_c, ref_c, adv_c, m, rho_c, row_denoms)
+
+
 class _GrpoFused(torch.autograd.Function):
     @staticmethod
     def forward(ctx, new_logprobs, old, ref, adv, mask, rho, entropy, cfg, rho_metrics=None):
-        dev = _lib.require_gpu(new_logprobs, old, ref, adv, mask, rho, entropy)
-        loss_fn, lo, hi, kl_estimator, beta, axis_mode, denominator, scale = cfg
-        nl = _lib.f32c(new_logprobs)
-        if nl.ndim != 2:
-            raise ValueError("grpo_loss_fused expects [rows, cols] tensors")
-        rows, cols = nl.shape
-        sides = [None if t is None else _lib.f32c(t.expand(rows, cols)) for t in (old, ref, adv, rho, entropy)]
-        old_c, ref_c, adv_c, rho_c, ent_c = sides
-        m = _lib.mask_u8(mask.expand(rows, cols))
-        stats = torch.empty(len(GRPO_STAT_NAMES), dtype=torch.float32, device=dev)
-        row_denoms = torch.empty(rows, dtype=torch.float32, device=dev)
-        ws_bytes = _lib.load().oi_grpo_fused_workspace_bytes(rows, cols)
-        ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
-        rho_ptrs, _alive = _rho_indicator_ptrs(rho_metrics, (rows, cols))
-        _lib.call(
-            "oi_grpo_fused_fwd", nl.data_ptr(), _lib.ptr(old_c), _lib.ptr(ref_c), adv_c.data_ptr(), m.data_ptr(),
-            _lib.ptr(rho_c), _lib.ptr(ent_c), *rho_ptrs, rows, cols, loss_fn, lo, hi, kl_estimator, beta, axis_mode,
-            denominator, scale, stats.data_ptr(), row_denoms.data_ptr(), ws.data_ptr(), ws_bytes, _lib.stream_of(nl),
-        )  # fmt: skip
-        ctx.save_for_backward(nl, old_c, ref_c, adv_c, m, rho_c, row_denoms)
+        stats, saved = _fused_stats(new_logprobs, old, ref, adv, mask, rho, entropy, cfg, rho_metrics)
+        ctx.save_for_backward(*saved)
         ctx.cfg = cfg
         ctx.in_dtype = new_logprobs.dtype
         loss = stats[0]
@@ -385,15 +399,10 @@ def grpo_loss_fused(
         raise ValueError("axis must be None or the token axis (1)")
     if loss_denominator is not None and float(loss_denominator) <= 0.0:
         raise ValueError("loss_denominator must be positive when given")
-    lo, hi = _clip_bounds(config)
-    cfg = (
-        _loss_fn_tag(config), lo, hi, int(config.kl_estimator), float(config.beta), 0 if axis is None else 1,
-        0.0 if loss_denominator is None else float(loss_denominator), float(dp_scale),
-    )  # fmt: skip
     detach = lambda t: None if t is None else t.detach()  # noqa: E731
     loss, stats = _GrpoFused.apply(
         new_logprobs, detach(old_logprobs), detach(ref_logprobs), advantages.detach(), response_mask,
-        detach(rho_weights), detach(entropy), cfg, rho_metrics,
+        detach(rho_weights), detach(entropy), _fused_cfg(config, axis, loss_denominator, dp_scale), rho_metrics,
     )  # fmt: skip
     return loss, _StatsView(stats)
 
@@ -410,17 +419,17 @@ class _StatsView(dict):
 # ----------------------------------------------------------------------------------------------
 # GRPO on materialised logits: forward + gradient in one read and one write of the logits
 # ----------------------------------------------------------------------------------------------
-def _token_coef(mask: torch.Tensor, axis: int | None, loss_denominator: float | None, dp_scale: float) -> torch.Tensor:
+def _token_coef(mask_u8: torch.Tensor, axis: int | None, loss_denominator: float | None, dp_scale: float) -> torch.Tensor:
     """``scale / denominator`` on response tokens, 0 elsewhere: the factor that ``masked_mean``
-    (open_instruct/rl_utils.py:426-448) puts in front of every token's loss.  Device arithmetic only."""
-    m = mask.to(torch.float32)
-    if axis is None:
-        den = m.sum() if loss_denominator is None else torch.full((), float(loss_denominator), device=m.device)
-        inv = torch.where(den > 0, 1.0 / den.clamp(min=1e-30), torch.zeros_like(den))
-        return m * (inv * float(dp_scale))
-    den = m.sum(dim=1, keepdim=True) if loss_denominator is None else torch.full_like(m[:, :1], float(loss_denominator))
-    inv = torch.where(den > 0, 1.0 / den.clamp(min=1e-30), torch.zeros_like(den))
-    return m * (inv * (float(dp_scale) / m.shape[0]))
+    (open_instruct/rl_utils.py:426-448) puts in front of every token's loss."""
+    rows, cols = mask_u8.shape
+    coef = torch.empty((rows, cols), dtype=torch.float32, device=mask_u8.device)
+    scale = float(dp_scale) if axis is None else float(dp_scale) / max(rows, 1)
+    _lib.call(
+        "oi_grpo_token_coef", mask_u8.data_ptr(), rows, cols, 0 if axis is None else 1,
+        0.0 if loss_denominator is None else float(loss_denominator), scale, coef.data_ptr(), _lib.stream_of(coef),
+    )  # fmt: skip
+    return coef
 
 
 def _single_pass_ok(view: torch.Tensor, so: int, si: int) -> bool:
@@ -540,24 +549,21 @@ def grpo_loss_on_logits(
             entropy=entropy, loss_denominator=loss_denominator, axis=axis, dp_scale=dp_scale,
         )  # fmt: skip
         return loss, stats, logprob.detach(), entropy
-    lo, hi = _clip_bounds(config)
-    cfg = (_loss_fn_tag(config), lo, hi, int(config.kl_estimator), float(config.beta))
-    mask = response_mask if response_mask.dtype == torch.bool else response_mask != 0
-    coef = _token_coef(mask, None if axis is None else 1, loss_denominator, dp_scale).contiguous()
+    cfg = _fused_cfg(config, axis, loss_denominator, dp_scale)
     shape = tuple(labels.shape)
-    # the kernel indexes every side tensor per token: broadcastable inputs are expanded first
+    # the kernels index every side tensor per token: broadcastable inputs are expanded first
     f32 = lambda t, name: None if t is None else _lib.f32c(_expand_to(t.detach(), shape, name))  # noqa: E731
+    old, ref = f32(old_logprobs, "old_logprobs"), f32(ref_logprobs, "ref_logprobs")
+    adv, rho = f32(advantages, "advantages"), f32(rho_weights, "rho_weights")
+    _lib.require_gpu(logits, labels, old, ref, adv, rho, response_mask)
     with torch.no_grad():
+        coef = _token_coef(_lib.mask_u8(response_mask), axis, loss_denominator, dp_scale)
         logprob, entropy, dlogits = _grpo_on_logits_launch(
-            logits.detach(), labels.long().contiguous(), f32(old_logprobs, "old_logprobs"),
-            f32(ref_logprobs, "ref_logprobs"), f32(advantages, "advantages"), f32(rho_weights, "rho_weights"), coef,
-            inv_t, cfg, drop_last,
-        )  # fmt: skip
-        loss, stats = grpo_loss_fused(
-            logprob, old_logprobs, ref_logprobs, advantages, response_mask, config, rho_weights=rho_weights,
-            entropy=entropy, loss_denominator=loss_denominator, axis=axis, dp_scale=dp_scale,
-        )  # fmt: skip
-    return _AttachLogitsGrad.apply(loss, logits, dlogits), stats, logprob, entropy
+            logits.detach(), labels.long().contiguous(), old, ref, adv, rho, coef, inv_t, cfg[:5], drop_last
+        )
+        stats, _ = _fused_stats(logprob, old, ref, adv, response_mask, rho, entropy, cfg)
+    loss = _AttachLogitsGrad.apply(stats[0], logits, dlogits)
+    return loss, _StatsView(stats), logprob, entropy
 
 
 class _AttachHeadGrads(torch.autograd.Function):

@@ -139,6 +139,27 @@ def test_statistics_of_few_and_many_rows(rows, cols, axis):
     assert abs(stats["loss/policy_avg"].item() - mean_pg) <= 1e-5 * max(1.0, abs(mean_pg))
 
 
+# bytes in front of the first 16-byte boundary and behind the last, one workgroup and as many as count for themselves
+@pytest.mark.parametrize("rows,cols,shift", [(1, 1, 0), (1, 1, 3), (3, 5, 0), (3, 17, 1), (2, 1000, 13), (16, 1024, 0), (5, 13109, 7)])
+@pytest.mark.parametrize("axis,denominator", [(None, None), (1, None), (None, 37.5), (1, 37.5)])
+def test_token_coefficients(rows, cols, shift, axis, denominator):
+    g = torch.Generator(device=DEV).manual_seed(rows * cols + shift)
+    whole = torch.rand(rows * cols + shift, generator=g, device=DEV) < 0.6
+    mask = whole[shift:].view(rows, cols)
+    if rows > 1:
+        mask[0] = False  # a row without a response token
+    got = grpo_utils._token_coef(_lib.mask_u8(mask), axis, denominator, 1.5)
+    m = mask.cpu().float()
+    if axis is None:
+        den, scale = m.sum(), torch.tensor(1.5)
+    else:
+        den, scale = m.sum(1, keepdim=True), torch.tensor(1.5 / rows)
+    if denominator is not None:
+        den = torch.full_like(den, denominator)
+    want = m * (torch.where(den > 0, 1.0 / den.clamp(min=1e-30), torch.zeros_like(den)) * scale)
+    assert torch.equal(got.cpu(), want)
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
 @pytest.mark.parametrize("shift", [0, 1])
 def test_scaling_by_a_device_scalar(dtype, shift):
