@@ -122,6 +122,11 @@ int oi_lsg_grpo_fwd_bwd(const void* logits, int dtype, int64_t n_outer, int64_t 
  */
 int oi_scale_by_device_scalar(void* data, int dtype, int64_t n, const float* scale, void* stream);
 
+/* The same for two tensors of one dtype (n or n_second may be 0) in one launch: the gradients of the steps on hidden
+ * states. */
+int oi_scale_pair_by_device_scalar(void* data, int64_t n, void* second, int64_t n_second, int dtype, const float* scale,
+                                   void* stream);
+
 /* ------------------------------------------------------------------------------------------
  * Per-token GRPO loss terms.  Carries open_instruct/grpo_utils.py:504-538 (compute_grpo_loss)
  * with open_instruct/model_utils.py:793-818 (estimate_kl) for the selected estimator.

@@ -103,8 +103,8 @@ __device__ __forceinline__ float oi_block_sum(float v, float* scratch) {
 
 // ---- between the translation units of the library (oi_loss.hip) ------------------------------------
 int oi_check_grpo(int64_t rows, int64_t cols, int axis_mode, int loss_fn, int kl_estimator);
-int oi_launch_grpo_denoms(const uint8_t* mask, const int32_t* count, int64_t rows, int64_t cols, int axis_mode,
-                          float denominator, float* row_denoms, hipStream_t s);
+// of the rows' own means (axis_mode 1)
+int oi_launch_grpo_denoms(const uint8_t* mask, int64_t rows, int64_t cols, float denominator, float* row_denoms, hipStream_t s);
 
 // ---- per-sequence ranges of a batch of token positions ---------------------------------------------
 // cu != null: one packed row of `total` positions with sequence boundaries cu[0 .. n_seqs]

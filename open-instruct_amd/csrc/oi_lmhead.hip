@@ -21,6 +21,7 @@
 // reads of a k-major image) stay free of bank conflicts.  A launch is one resident workgroup per
 // CU that draws tile ids from per-XCD counters.
 #include "oi_common.h"
+#include "oi_grpo_math.h"
 #include "oi_ktiles.h"
 
 #include <type_traits>
@@ -1875,18 +1876,28 @@ __device__ __forceinline__ bool row_selected(const uint8_t* __restrict__ mask, c
 }
 
 constexpr int SELECT_THREADS = 1024;
-// One workgroup: rows[0 .. count) = positions of the selected rows in ascending order (a stable
-// compaction: count per thread segment, block scan, write).  Also clears `n_zero` (<= 1024) queue
-// words for the launches that follow.
-__global__ void __launch_bounds__(SELECT_THREADS)
-    select_rows_kernel(const uint8_t* __restrict__ mask, const float* __restrict__ grad, int64_t n,
-                       int32_t* __restrict__ rows, int32_t* __restrict__ count, uint32_t* __restrict__ zero_words,
-                       int n_zero) {
+// Of one workgroup: rows[0 .. count) = positions of the selected rows in ascending order (a stable
+// compaction: count per thread segment, block scan, write).  Returns the count to every thread.
+__device__ __forceinline__ int select_rows(const uint8_t* __restrict__ mask, const float* __restrict__ grad, int64_t n,
+                                           int32_t* __restrict__ rows) {
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
     const int64_t per = (n + SELECT_THREADS - 1) / SELECT_THREADS;
     const int64_t b = t * per, e = b + per < n ? b + per : n;
+    // up to 64 rows of a thread: their bits, read once
+    const bool few = per <= 64;
+    uint64_t bits = 0;
     int c = 0;
-    for (int64_t i = b; i < e; ++i) c += row_selected(mask, grad, i) ? 1 : 0;
+    if (few) {
+#pragma unroll 8
+        for (int k = 0; k < per; ++k) {
+            const int64_t i = b + k < e ? b + k : n - 1;
+            const bool set = row_selected(mask, grad, i);
+            bits |= (uint64_t)(set && b + k < e) << k;
+        }
+        c = __popcll(bits);
+    } else {
+        for (int64_t i = b; i < e; ++i) c += row_selected(mask, grad, i) ? 1 : 0;
+    }
     int incl = c;
 #pragma unroll
     for (int off = 1; off < OI_WAVE; off <<= 1) {
@@ -1896,13 +1907,29 @@ __global__ void __launch_bounds__(SELECT_THREADS)
     __shared__ int wave_total[SELECT_THREADS / OI_WAVE];
     if (lane == OI_WAVE - 1) wave_total[wave] = incl;
     __syncthreads();
-    int base = 0;
-    for (int w = 0; w < wave; ++w) base += wave_total[w];
+    int base = 0, total = 0;
+#pragma unroll
+    for (int w = 0; w < SELECT_THREADS / OI_WAVE; ++w) {
+        base += w < wave ? wave_total[w] : 0;
+        total += wave_total[w];
+    }
     int pos = base + incl - c;
-    for (int64_t i = b; i < e; ++i)
-        if (row_selected(mask, grad, i)) rows[pos++] = (int32_t)i;
-    if (t == SELECT_THREADS - 1) *count = base + incl;
-    if (t < n_zero) zero_words[t] = 0u;
+    if (few) {
+        for (; bits; bits &= bits - 1) rows[pos++] = (int32_t)(b + __ffsll((unsigned long long)bits) - 1);
+    } else {
+        for (int64_t i = b; i < e; ++i)
+            if (row_selected(mask, grad, i)) rows[pos++] = (int32_t)i;
+    }
+    return total;
+}
+// One workgroup.  Also clears `n_zero` (<= 1024) queue words for the launches that follow.
+__global__ void __launch_bounds__(SELECT_THREADS)
+    select_rows_kernel(const uint8_t* __restrict__ mask, const float* __restrict__ grad, int64_t n,
+                       int32_t* __restrict__ rows, int32_t* __restrict__ count, uint32_t* __restrict__ zero_words,
+                       int n_zero) {
+    const int total = select_rows(mask, grad, n, rows);
+    if (threadIdx.x == 0) *count = total;
+    if ((int)threadIdx.x < n_zero) zero_words[threadIdx.x] = 0u;
 }
 
 // Workgroup j copies selected row j: the hidden-state row (hdim bf16, 16-byte pieces), its label
@@ -2014,8 +2041,27 @@ __global__ void __launch_bounds__(256)
 // (exact where the label's probability is close to 1), and, when d_weight is wanted, the scaled
 // hidden row.  A token flagged in `unsafe` gets factors of exactly 0: it adds nothing to either
 // product here and takes the recomputing backward afterwards.
+// `upstream`: d loss / d logprob of a caller row, which GrpoUpstream derives here (a launch of its own for it took 5 us of
+// every slab) and leaves in `grad` for the flagged rows, and StoredUpstream reads there.
+struct StoredUpstream {
+    __device__ __forceinline__ float operator()(int64_t row, float* grad) const { return grad[row]; }
+};
+struct GrpoUpstream {  // as grpo_fused_bwd_kernel, without an upstream gradient of the loss
+    const float *logprob, *old, *ref, *adv, *rho, *row_denoms;
+    int64_t cols;
+    GrpoCfg cfg;
+    float beta, scale;
+    __device__ __forceinline__ float operator()(int64_t row, float* grad) const {
+        const float x = logprob[row], ratio = old ? expf(x - old[row]) : 1.f;
+        const float d = grpo_token_dnew(x, ratio, adv[row], ref != nullptr, ref ? ref[row] : 0.f, rho ? rho[row] : 1.f, cfg, beta);
+        const float g = scale * row_denoms[(uint32_t)row / (uint32_t)cols] * d;  // rows are at most 2^22
+        if (threadIdx.x == 0) grad[row] = g;
+        return g;
+    }
+};
+template <class Upstream>
 __global__ void __launch_bounds__(256)
-    slab_prepare_kernel(const float* __restrict__ lse, const float* __restrict__ grad,
+    slab_prepare_kernel(Upstream upstream, const float* __restrict__ lse, float* __restrict__ grad,
                         const float* __restrict__ logprob, const uint8_t* __restrict__ unsafe,
                         const int32_t* __restrict__ rows_s, const int64_t* __restrict__ labels_s,
                         const float* __restrict__ xref_s, const SlabMeta* __restrict__ meta, float inv_t,
@@ -2028,7 +2074,7 @@ __global__ void __launch_bounds__(256)
     const bool dead = unsafe[src] != 0;
     const float l2 = lse[src] * OI_LOG2E - xref_s[j];  // log2 of the sum of the kept numbers of this token
     const float half = dead ? 0.f : __builtin_amdgcn_exp2f(-0.5f * l2);
-    const float a = half, b = -grad[src] * inv_t * half;
+    const float a = half, b = -upstream(src, grad) * inv_t * half;
     if (threadIdx.x == 0) {
         scale_a[j] = a;
         scale_b[j] = b;
@@ -2654,11 +2700,14 @@ SlabPlan plan_slabs(int64_t n, int64_t stats_rows, int64_t stats_cols, int64_t h
 // steps at 4096 x 128256, full slabs of 8192 against equal ones, 8500 rows 21.6 to 21.8 against 22.0 ms, 9472 rows 24.6
 // against 24.6, 12288 rows 30.5 to 31.3 against 30.6 to 31.4, 16640 rows 43.2 against 43.1.  Passes past the last slab
 // are empty.
-__global__ void plan_slabs_kernel(const int32_t* __restrict__ count, int cap, int n_passes, int h_tiles, int grid,
-                                  SlabMeta* __restrict__ meta) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n_passes) return;
-    const int n = *count;
+struct SlabPlanning {
+    int cap, n_passes, h_tiles, grid;
+    SlabMeta* meta;
+};
+// of n selected rows, pass i
+__device__ __forceinline__ void plan_slab(const SlabPlanning& p, int n, int i) {
+    const int cap = p.cap, h_tiles = p.h_tiles, grid = p.grid;
+    SlabMeta* meta = p.meta;
     const int k = n > 0 ? (n + cap - 1) / cap : 1;
     int equal = ((n + k - 1) / k + 255) / 256 * 256;
     equal = equal > cap ? cap : equal;
@@ -2680,23 +2729,56 @@ __global__ void plan_slabs_kernel(const int32_t* __restrict__ count, int cap, in
     meta[i].reserved = 0;
 }
 
-// What a step starts from, in one launch (a small launch is 5 us of the stream, and the step of a short batch has 19 of
-// them beside its three products; it had 25): the queue words of every pass and the marks of the rows (n_pad bytes) are
+// What a step starts from: the queue words of every pass and the marks of the rows (n_pad bytes) are
 // cleared, and the per-token outputs are zero: rows that take no part stay there, and the passes that look
-// at every row before its own slab has run (the upstream gradient of a slab is computed for all rows)
-// read zeros rather than whatever the caller's buffers held.
-__global__ void __launch_bounds__(256)
-    slab_setup_kernel(int64_t n, int64_t n_pad, int64_t queue_words, float* __restrict__ logprob,
-                      float* __restrict__ entropy, float* __restrict__ lse, uint32_t* __restrict__ unsafe,
-                      uint32_t* __restrict__ queues) {
-    const int64_t first = (int64_t)blockIdx.x * blockDim.x + threadIdx.x, stride = (int64_t)gridDim.x * blockDim.x;
-    for (int64_t i = first; i < n; i += stride) {
-        logprob[i] = 0.f;
-        if (entropy) entropy[i] = 0.f;
-        lse[i] = 0.f;
+// at every row before its own slab has run (the upstream gradient of a slab's pairs) read zeros rather than whatever the
+// caller's buffers held.  d_hidden rows of tokens that take no part are zero.
+struct SlabSetup {
+    const uint8_t* mask;
+    int64_t n, n_pad, queue_words, hdim;
+    float *logprob, *entropy, *lse;
+    uint32_t *unsafe, *queues;
+    uint16_t* d_hidden;
+};
+// The share of workgroup `block` of `blocks` of 1024 threads, four rows of d_hidden at a time
+constexpr int SETUP_THREADS = 1024, SETUP_ROWS = 4;
+__device__ __forceinline__ void slab_setup(const SlabSetup& a, int64_t block, int64_t blocks) {
+    const int64_t first = block * SETUP_THREADS + threadIdx.x, stride = blocks * SETUP_THREADS;
+    for (int64_t i = first; i < a.n; i += stride) {
+        a.logprob[i] = 0.f;
+        if (a.entropy) a.entropy[i] = 0.f;
+        a.lse[i] = 0.f;
     }
-    for (int64_t i = first; i < n_pad / 4; i += stride) unsafe[i] = 0u;
-    for (int64_t i = first; i < queue_words; i += stride) queues[i] = 0u;
+    for (int64_t i = first; i < a.n_pad / 4; i += stride) a.unsafe[i] = 0u;
+    for (int64_t i = first; i < a.queue_words; i += stride) a.queues[i] = 0u;
+    const int64_t row = block * SETUP_ROWS + (threadIdx.x >> 8);
+    if (row >= a.n || row_selected(a.mask, nullptr, row)) return;
+    uint32_t* out = reinterpret_cast<uint32_t*>(a.d_hidden + row * a.hdim);  // hdim is a multiple of 64
+    for (int64_t c = threadIdx.x & 255; c < a.hdim / 2; c += 256) out[c] = 0u;
+}
+inline int64_t setup_blocks(int64_t n) { return (n + SETUP_ROWS - 1) / SETUP_ROWS; }
+__global__ void __launch_bounds__(SETUP_THREADS) slab_setup_kernel(SlabSetup a) { slab_setup(a, blockIdx.x, gridDim.x); }
+
+// The start of a GRPO step in one launch: workgroup 0 selects the rows, plans the slabs and, where one denominator serves
+// all rows, leaves it in row_denoms; the others set up.  A small launch is 5 us of the stream, and a step of few rows is
+// three products and small launches: as five launches this took 23 us of the 1050 of a step of 268 rows.
+struct GrpoStart {
+    int32_t *order, *count;
+    SlabPlanning planning;
+    float* row_denoms;  // null: the denominators are the rows' own
+    int64_t rows;
+    float denominator;
+};
+static_assert(SETUP_THREADS == SELECT_THREADS, "one launch");
+__global__ void __launch_bounds__(SETUP_THREADS) grpo_start_kernel(SlabSetup a, GrpoStart g) {
+    if (blockIdx.x > 0) return slab_setup(a, blockIdx.x - 1, gridDim.x - 1);
+    const int n = select_rows(a.mask, nullptr, a.n, g.order);
+    if (threadIdx.x == 0) *g.count = n;
+    for (int i = threadIdx.x; i < g.planning.n_passes; i += SETUP_THREADS) plan_slab(g.planning, n, i);
+    if (!g.row_denoms) return;
+    const double den = g.denominator > 0.f ? (double)g.denominator : (double)n;
+    const float inv = (float)(den > 0.0 ? 1.0 / den : 0.0);  // as grpo_stats_final_kernel leaves it
+    for (int64_t r = threadIdx.x; r < g.rows; r += SETUP_THREADS) g.row_denoms[r] = inv;
 }
 
 // What a slab-wise step is made of besides the passes themselves
@@ -2710,13 +2792,13 @@ struct SlabStep {
     void *d_hidden, *d_weight;   // d_weight may be null
 };
 
-// Runs the slab passes of `st` over the row index order[0 .. *count) that `plan_rows` leaves in the
-// workspace together with the passes' SlabMeta (it returns a status: reading one clears it).  `upstream()` must enqueue kernels that leave
-// every caller row's d loss / d logprob in the workspace's grad vector, given the logprobs computed
-// so far (the rows of the slabs up to the current one; in the last pass, all rows).
-template <class PlanRows, class Upstream>
-int run_slab_passes(const SlabPlan& p, char* ws, const SlabStep& st, hipStream_t s, PlanRows&& plan_rows,
-                    Upstream&& upstream) {
+// Runs the slab passes of `st` over the row index order[0 .. *count) that `start` leaves in the
+// workspace together with the passes' SlabMeta, once it has set up what SlabSetup says (it returns a status: reading one
+// clears it).  `upstream()` may enqueue kernels and returns, by reference, a status and the upstream gradient as
+// slab_prepare_kernel takes it, given the logprobs computed so far (the rows of the slabs up to the current one; in the
+// last pass, all rows).
+template <class Start, class Upstream>
+int run_slab_passes(const SlabPlan& p, char* ws, const SlabStep& st, hipStream_t s, Start&& start, Upstream&& upstream) {
     const int64_t n = st.n_tokens, hdim = st.hidden_dim, vocab = st.vocab;
     char* ws_fwd = ws + p.off_fwd;
     int32_t* order = reinterpret_cast<int32_t*>(ws + p.off_order);
@@ -2738,13 +2820,10 @@ int run_slab_passes(const SlabPlan& p, char* ws, const SlabStep& st, hipStream_t
     float* parts = p.parts_bytes ? reinterpret_cast<float*>(ws + p.off_parts) : nullptr;
     const uint16_t* hid = static_cast<const uint16_t*>(st.hidden);
 
-    hipLaunchKernelGGL(slab_setup_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, n, p.n_pad,
-                       p.n_passes * SLAB_QUEUE_WORDS, st.logprob, st.entropy, lse, reinterpret_cast<uint32_t*>(unsafe),
-                       queues);
-    const int planned = plan_rows(order, count, meta);
-    if (planned != OI_OK) return planned;
-    hipLaunchKernelGGL(zero_unselected_rows_kernel, dim3((unsigned)n), dim3(256), 0, s, st.mask,
-                       static_cast<const float*>(nullptr), hdim, static_cast<uint16_t*>(st.d_hidden));
+    const SlabSetup setup = {st.mask, n, p.n_pad, p.n_passes * SLAB_QUEUE_WORDS, hdim, st.logprob, st.entropy, lse,
+                             reinterpret_cast<uint32_t*>(unsafe), queues, static_cast<uint16_t*>(st.d_hidden)};
+    const int started = start(setup, order, count, meta);
+    if (started != OI_OK) return started;
     for (int64_t i = 0; i < p.n_passes; ++i) {
         const int32_t* cnt = &meta[i].count;
         uint32_t* pass_queues = queues + i * SLAB_QUEUE_WORDS;
@@ -2758,9 +2837,10 @@ int run_slab_passes(const SlabPlan& p, char* ws, const SlabStep& st, hipStream_t
         fp.off_queue = (size_t)(reinterpret_cast<char*>(pass_queues) - ws_fwd);
         enqueue_fwd(fp, ws_fwd, in, nullptr, st.weight, p.cap, hdim, vocab, st.inv_temperature, st.logprob, st.entropy,
                     lse, keep, s);
-        const int rc = upstream();
+        int rc = OI_OK;
+        const auto gradient = upstream(rc);
         if (rc != OI_OK) return rc;
-        hipLaunchKernelGGL(slab_prepare_kernel, dim3((unsigned)p.cap), dim3(256), 0, s, lse, grad, st.logprob, unsafe,
+        hipLaunchKernelGGL(slab_prepare_kernel, dim3((unsigned)p.cap), dim3(256), 0, s, gradient, lse, grad, st.logprob, unsafe,
                            rows_s, labels_s, xref_s, meta + i, st.inv_temperature, vocab, hdim, keep_buf, p.v_pad,
                            hidden_s, scale_a, scale_b, scaled_hidden);
         enqueue_products_from_exponentials(keep_buf, p.v_pad, p.cap, cnt, rows_s, scale_a, scale_b, scaled_hidden,
@@ -3052,22 +3132,19 @@ int grpo_step_in_slabs(const void* hidden, const void* weight, const int64_t* la
                          d_hidden, d_weight};
     rc = run_slab_passes(
         p, ws, st, s,
-        [&](int32_t* order, int32_t* count, SlabMeta* meta) {
-            hipLaunchKernelGGL(select_rows_kernel, dim3(1), dim3(SELECT_THREADS), 0, s, mask,
-                               static_cast<const float*>(nullptr), n_tokens, order, count,
-                               static_cast<uint32_t*>(nullptr), 0);
+        [&](const SlabSetup& setup, int32_t* order, int32_t* count, SlabMeta* meta) {
             const int64_t h_tiles = (hidden_dim + BN - 1) / BN;
-            hipLaunchKernelGGL(plan_slabs_kernel, dim3((unsigned)((p.n_passes + 63) / 64)), dim3(64), 0, s, count,
-                               (int)p.cap, (int)p.n_passes, (int)h_tiles, (int)resident_grid(p.cap / BM, h_tiles), meta);
+            const SlabPlanning planning = {(int)p.cap, (int)p.n_passes, (int)h_tiles, (int)resident_grid(p.cap / BM, h_tiles), meta};
+            const GrpoStart g = {order, count, planning, axis_mode == 0 ? row_denoms : nullptr, rows, denominator};
+            hipLaunchKernelGGL(grpo_start_kernel, dim3((unsigned)(1 + setup_blocks(n_tokens))), dim3(SETUP_THREADS), 0, s, setup, g);
             // the denominators come from the mask alone
-            return oi_launch_grpo_denoms(mask, count, rows, cols, axis_mode, denominator, row_denoms, s);
+            return axis_mode == 0 ? oi_launch_status()
+                                  : oi_launch_grpo_denoms(mask, rows, cols, denominator, row_denoms, s);
         },
-        [&]() {
-            // every token's d loss / d logprob from its own logprob; tokens of later slabs hold numbers
-            // that nobody reads before their own slab has overwritten them
-            return oi_grpo_fused_bwd(logprob, old_logprobs, ref_logprobs, advantages, mask, rho_weights, rows, cols,
-                                     loss_fn, ratio_lo, ratio_hi, kl_estimator, beta, scale, row_denoms, nullptr, grad,
-                                     stream);
+        // every token's d loss / d logprob from its own logprob
+        [&](int&) {
+            return GrpoUpstream{logprob, old_logprobs, ref_logprobs, advantages, rho_weights, row_denoms, cols,
+                                GrpoCfg{loss_fn, ratio_lo, ratio_hi, kl_estimator}, beta, scale};
         });
     if (rc != OI_OK) return rc;
     // loss and statistics from all logprobs
@@ -3359,18 +3436,19 @@ extern "C" int oi_lmhead_dpo_fwd_bwd(const void* hidden, const void* weight, con
                          nullptr, d_hidden, d_weight};
     // per-sequence sums of the logprobs computed so far, the loss derivative of every pair, and from it
     // every token's d loss / d logprob (right for the pairs whose tokens are all there)
-    auto upstream = [&]() {
-        int r = oi_seq_logp_fwd(per_token_logps, labels, cu_seq_lens, n_seqs, total, average_log_prob, seq_logps, counts,
-                                stream);
-        if (r != OI_OK) return r;
-        r = oi_dpo_sigmoid_bwd(seq_logps, seq_logps + bs, ref_chosen, ref_rejected, nullptr, grad_losses, bs, beta,
-                               label_smoothing, margin, d_seq, d_seq + bs, stream);
-        if (r != OI_OK) return r;
-        return oi_seq_logp_bwd(d_seq, labels, cu_seq_lens, counts, n_seqs, total, average_log_prob, grad, stream);
+    auto upstream = [&](int& r) {
+        r = oi_seq_logp_fwd(per_token_logps, labels, cu_seq_lens, n_seqs, total, average_log_prob, seq_logps, counts, stream);
+        if (r == OI_OK)
+            r = oi_dpo_sigmoid_bwd(seq_logps, seq_logps + bs, ref_chosen, ref_rejected, nullptr, grad_losses, bs, beta,
+                                   label_smoothing, margin, d_seq, d_seq + bs, stream);
+        if (r == OI_OK)
+            r = oi_seq_logp_bwd(d_seq, labels, cu_seq_lens, counts, n_seqs, total, average_log_prob, grad, stream);
+        return StoredUpstream{};
     };
     rc = run_slab_passes(
         p.slabs, ws_slabs, st, s,
-        [&](int32_t* order, int32_t* count, SlabMeta* meta) {
+        [&](const SlabSetup& setup, int32_t* order, int32_t* count, SlabMeta* meta) {
+            hipLaunchKernelGGL(slab_setup_kernel, dim3((unsigned)setup_blocks(n_tokens)), dim3(SETUP_THREADS), 0, s, setup);
             hipLaunchKernelGGL(dpo_plan_kernel, dim3(1), dim3(1), 0, s, cnt, (int)n_seqs, (int)p.slabs.cap,
                                (int)p.slabs.n_passes, off, seq_unsafe, count, meta);
             hipLaunchKernelGGL(dpo_order_kernel, dim3((unsigned)n_seqs), dim3(256), 0, s, mask, cu_seq_lens, n_seqs, total,

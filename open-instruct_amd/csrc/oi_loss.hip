@@ -260,17 +260,10 @@ __global__ void __launch_bounds__(16 * FINAL_SLICES)
     out_stats[q * out_stride] = st;
 }
 
-// row_denoms as grpo_stats_final_kernel leaves them, from the mask alone: with axis_mode 1 one workgroup per row,
-// else workgroup 0 for all rows from `count`, the number of set mask bytes.
+// row_denoms as grpo_stats_final_kernel leaves them with axis_mode 1, from the mask alone; one workgroup per row
 __global__ void __launch_bounds__(256)
-    grpo_denoms_kernel(const uint8_t* __restrict__ mask, const int32_t* __restrict__ count, int64_t rows, int64_t cols,
-                       int axis_mode, float denominator, float* __restrict__ row_denoms) {
-    if (axis_mode == 0) {
-        const double den = denominator > 0.f ? (double)denominator : (double)*count;
-        const float inv = (float)(den > 0.0 ? 1.0 / den : 0.0);
-        for (int64_t r = threadIdx.x; r < rows; r += blockDim.x) row_denoms[r] = inv;
-        return;
-    }
+    grpo_denoms_kernel(const uint8_t* __restrict__ mask, int64_t rows, int64_t cols, float denominator,
+                       float* __restrict__ row_denoms) {
     const int64_t r = blockIdx.x;
     float c = 0.f;  // exact: at most 2^22 columns
     if (!(denominator > 0.f))
@@ -865,7 +858,7 @@ int check_stats_shape(int64_t rows, int64_t cols) {
 }
 }  // namespace
 
-// For the slab-wise step: what oi_grpo_fused_fwd refuses, before anything is launched, and the denominators
+// For the slab-wise step: what oi_grpo_fused_fwd refuses, before anything is launched, and the rows' own denominators
 // before any logprob is there.
 int oi_check_grpo(int64_t rows, int64_t cols, int axis_mode, int loss_fn, int kl_estimator) {
     const int rc = check_stats_shape(rows, cols);
@@ -873,10 +866,8 @@ int oi_check_grpo(int64_t rows, int64_t cols, int axis_mode, int loss_fn, int kl
     OI_RETURN_IF(axis_mode != 0 && axis_mode != 1, OI_EINVAL);
     return check_cfg(loss_fn, kl_estimator);
 }
-int oi_launch_grpo_denoms(const uint8_t* mask, const int32_t* count, int64_t rows, int64_t cols, int axis_mode,
-                          float denominator, float* row_denoms, hipStream_t s) {
-    hipLaunchKernelGGL(grpo_denoms_kernel, dim3((unsigned)(axis_mode == 0 ? 1 : rows)), dim3(256), 0, s, mask, count, rows,
-                       cols, axis_mode, denominator, row_denoms);
+int oi_launch_grpo_denoms(const uint8_t* mask, int64_t rows, int64_t cols, float denominator, float* row_denoms, hipStream_t s) {
+    hipLaunchKernelGGL(grpo_denoms_kernel, dim3((unsigned)rows), dim3(256), 0, s, mask, rows, cols, denominator, row_denoms);
     return oi_launch_status();
 }
 

@@ -740,14 +740,8 @@ int launch_grpo_fused(const void* logits, int64_t rows, int64_t n_inner, int64_t
     return oi_launch_status();
 }
 
-// data[i] *= *scale for a contiguous tensor, skipped altogether when the device scalar is exactly 1
-// (the upstream gradient of a loss that is differentiated directly): every workgroup reads the
-// scalar and leaves, so the host never has to look at it.
 template <typename R>
-__global__ void __launch_bounds__(256) scale_by_scalar_kernel(typename R::elem_t* __restrict__ data, int64_t n,
-                                                              bool vectorised, const float* __restrict__ scale) {
-    const float s = *scale;
-    if (s == 1.f) return;
+__device__ __forceinline__ void scale_tensor(typename R::elem_t* __restrict__ data, int64_t n, bool vectorised, float s) {
     const int64_t stride = (int64_t)gridDim.x * blockDim.x, first = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (vectorised) {
         const int64_t vecs = n / R::VEC;
@@ -776,10 +770,23 @@ __global__ void __launch_bounds__(256) scale_by_scalar_kernel(typename R::elem_t
     }
 }
 
+// data[i] *= *scale for one or two contiguous tensors, skipped altogether when the device scalar is exactly 1
+// (the upstream gradient of a loss that is differentiated directly): every workgroup reads the
+// scalar and leaves, so the host never has to look at it.  Two tensors in one launch: mostly it is nothing else.
 template <typename R>
-int launch_scale(void* data, int64_t n, const float* scale, hipStream_t stream) {
+__global__ void __launch_bounds__(256) scale_by_scalar_kernel(typename R::elem_t* __restrict__ data, int64_t n, bool vectorised,
+                                                              typename R::elem_t* __restrict__ second, int64_t n_second,
+                                                              bool second_vectorised, const float* __restrict__ scale) {
+    const float s = *scale;
+    if (s == 1.f) return;
+    scale_tensor<R>(data, n, vectorised, s);
+    if (n_second > 0) scale_tensor<R>(second, n_second, second_vectorised, s);
+}
+
+template <typename R>
+int launch_scale(void* data, int64_t n, void* second, int64_t n_second, const float* scale, hipStream_t stream) {
     typedef typename R::elem_t E;
-    const int64_t vecs = (n + R::VEC - 1) / R::VEC;
+    const int64_t vecs = ((n > n_second ? n : n_second) + R::VEC - 1) / R::VEC;
     const int64_t want = (vecs + 255) / 256;
     // Few workgroups, since mostly they only read the scalar (16384 of them 4.7 us, three per CU 1.8), and few bytes
     // in flight, since reads and writes share the memory's pages.  bf16 [32768, 4096], [100352, 4096], fp32 [2048,
@@ -788,7 +795,7 @@ int launch_scale(void* data, int64_t n, const float* scale, hipStream_t stream) 
     const int64_t most = 3 * (int64_t)oi_cu_count();
     const unsigned blocks = (unsigned)(want < 1 ? 1 : (want > most ? most : want));
     hipLaunchKernelGGL((scale_by_scalar_kernel<R>), dim3(blocks), dim3(256), 0, stream, static_cast<E*>(data), n,
-                       oi_aligned(data, 16), scale);
+                       oi_aligned(data, 16), static_cast<E*>(second), n_second, oi_aligned(second, 16), scale);
     return oi_launch_status();
 }
 
@@ -902,16 +909,22 @@ extern "C" int oi_lsg_grpo_fwd_bwd(const void* logits, int dtype, int64_t n_oute
     }
 }
 
-extern "C" int oi_scale_by_device_scalar(void* data, int dtype, int64_t n, const float* scale, void* stream) {
-    OI_RETURN_IF(n < 0, OI_EINVAL);
+extern "C" int oi_scale_pair_by_device_scalar(void* data, int64_t n, void* second, int64_t n_second, int dtype,
+                                              const float* scale, void* stream) {
+    OI_RETURN_IF(n < 0 || n_second < 0, OI_EINVAL);
     OI_RETURN_IF(dtype != OI_DTYPE_F32 && dtype != OI_DTYPE_BF16 && dtype != OI_DTYPE_F16, OI_EDTYPE);
-    if (n == 0) return OI_OK;
-    OI_RETURN_IF(!data || !scale, OI_ENULL);
-    OI_RETURN_IF(!oi_aligned(data, dtype == OI_DTYPE_F32 ? 4 : 2), OI_EALIGN);
+    if (n == 0 && n_second == 0) return OI_OK;
+    OI_RETURN_IF((n > 0 && !data) || (n_second > 0 && !second) || !scale, OI_ENULL);
+    const size_t element = dtype == OI_DTYPE_F32 ? 4 : 2;
+    OI_RETURN_IF(!oi_aligned(data, element) || !oi_aligned(second, element), OI_EALIGN);
     hipStream_t s = static_cast<hipStream_t>(stream);
     switch (dtype) {
-        case OI_DTYPE_F32: return launch_scale<F32Row>(data, n, scale, s);
-        case OI_DTYPE_BF16: return launch_scale<BF16Row>(data, n, scale, s);
-        default: return launch_scale<F16Row>(data, n, scale, s);
+        case OI_DTYPE_F32: return launch_scale<F32Row>(data, n, second, n_second, scale, s);
+        case OI_DTYPE_BF16: return launch_scale<BF16Row>(data, n, second, n_second, scale, s);
+        default: return launch_scale<F16Row>(data, n, second, n_second, scale, s);
     }
+}
+
+extern "C" int oi_scale_by_device_scalar(void* data, int dtype, int64_t n, const float* scale, void* stream) {
+    return oi_scale_pair_by_device_scalar(data, n, nullptr, 0, dtype, scale, stream);
 }

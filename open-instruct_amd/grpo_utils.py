@@ -580,12 +580,12 @@ class _AttachHeadGrads(torch.autograd.Function):
         d_hidden, d_weight = ctx.saved_tensors
         _hand_out_once(ctx)
         g = _lib.f32c(grad_loss.detach()).reshape(1)
-        for t in (d_hidden, d_weight):  # nothing is touched when the device scalar is exactly 1
-            if t is not None:
-                _lib.call(
-                    "oi_scale_by_device_scalar", t.data_ptr(), _lib.DTYPE_TAGS[t.dtype], t.numel(), g.data_ptr(),
-                    _lib.stream_of(t),
-                )  # fmt: skip
+        # nothing is touched when the device scalar is exactly 1; both are bf16
+        _lib.call(
+            "oi_scale_pair_by_device_scalar", d_hidden.data_ptr(), d_hidden.numel(), _lib.ptr(d_weight),
+            0 if d_weight is None else d_weight.numel(), _lib.DTYPE_TAGS[d_hidden.dtype], g.data_ptr(),
+            _lib.stream_of(d_hidden),
+        )  # fmt: skip
         need_h, need_w = ctx.needs_input_grad[1], ctx.needs_input_grad[2]
         return None, (d_hidden if need_h else None), (d_weight if need_w else None), None, None
 
