@@ -251,6 +251,11 @@ int oi_pick_values(const float* values, const uint8_t* mask, int64_t n, float* o
 int oi_record_stats(const float* vector, uint32_t row_mask, const float* loss, int loss_row, float* table,
                     int64_t columns, int64_t column, void* stream);
 
+/* Labels as a causal model scores them (open_instruct/padding_free_collator.py:10-16): out[r, c] = labels[r, c + 1] and
+ * `fill` in the last column of each of `rows` contiguous rows; keep (optional): one byte, out != ignored. */
+int oi_shift_labels(const int64_t* labels, int64_t rows, int64_t cols, int64_t fill, int64_t ignored, int64_t* out,
+                    uint8_t* keep, void* stream);
+
 /* Factor of every token's loss in the masked mean of open_instruct/rl_utils.py:426-448:
  * coef = scale / denominator on set mask bytes, 0 elsewhere (and where the denominator is 0).  axis_mode 0: one
  * denominator for all rows, axis_mode 1: one per row (`scale` then holds the 1 / rows of the mean over rows); it is

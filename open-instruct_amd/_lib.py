@@ -54,6 +54,7 @@ SIGNATURES: dict[str, tuple] = {
     "oi_rho_correction": (_I, [_P, _P, _P, _P, _I64, _I64, _I, _I, _F, _F, _F, _F, _P, _P, _P, _P, _P, _P, _P]),
     "oi_pick_values": (_I, [_P, _P, _I64, _P, _P, _P]),
     "oi_record_stats": (_I, [_P, c_uint32, _P, _I, _P, _I64, _I64, _P]),
+    "oi_shift_labels": (_I, [_P, _I64, _I64, _I64, _I64, _P, _P, _P]),
     "oi_grpo_token_coef": (_I, [_P, _I64, _I64, _I, _F, _F, _P, _P]),
     "oi_group_advantages": (_I, [_P, _I64, _I64, _I, _P, _P]),
     "oi_masked_mean_workspace_bytes": (_SZ, [_I64, _I64, _I64]),

@@ -18,7 +18,7 @@ import weakref
 
 import torch
 
-from . import _lib
+from . import _lib, padding_free_collator, rl_utils
 
 
 class _FusedLMHead(torch.autograd.Function):
@@ -277,12 +277,13 @@ def fused_linear_cross_entropy(
     """
     if (labels is None) == (shift_labels is None):
         raise ValueError("pass exactly one of labels / shift_labels")
+    keep = None
     if shift_labels is None:
-        shift_labels = torch.full_like(labels, ignore_index)
-        shift_labels[..., :-1] = labels[..., 1:]
+        shift_labels, keep = padding_free_collator.shifted_and_kept(labels, ignore_index, ignore_index)
     if shift_labels.shape != hidden.shape[:-1]:
         raise ValueError(f"labels {tuple(shift_labels.shape)} do not match hidden {tuple(hidden.shape)}")
-    keep = shift_labels != ignore_index
+    if keep is None:
+        keep = shift_labels != ignore_index
     if token_slabs:
         import types
 
@@ -301,6 +302,8 @@ def fused_linear_cross_entropy(
         )  # fmt: skip
         return loss
     logps, _ = fused_lm_head_logprobs(hidden, weight, shift_labels, mask=keep, keep_logits=keep_logits)
+    if num_items_in_batch is None and logps.numel() > 0:
+        return -rl_utils.masked_mean(logps, keep)
     total = -logps.sum()
     if num_items_in_batch is None:
         return total / keep.sum().clamp(min=1)

@@ -84,8 +84,13 @@ class DPOLMHead(torch.nn.Module):
             self.fused_result = dpo_utils.dpo_loss_on_hidden(h, self.w_out.weight, labels, **self.fused_loss)
             logps = self.fused_result.per_token_logps
             return LMOutputWithLoss(logits=None, loss=logps, ce_loss=logps.clone(), z_loss=None)
-        shifted = padding_free_collator.shift_labels(labels)
-        keep = None if self.score_ignored_positions else shifted != ignore_index
+        if labels.ndim == 2:
+            shifted, keep = padding_free_collator.shifted_and_kept(
+                labels, ignored=ignore_index, want_keep=not self.score_ignored_positions
+            )
+        else:
+            shifted = padding_free_collator.shift_labels(labels)
+            keep = None if self.score_ignored_positions else shifted != ignore_index
         per_token_logps, _ = lm_head.fused_lm_head_logprobs(
             h, self.w_out.weight, shifted, mask=keep, keep_logits=self.keep_logits
         )

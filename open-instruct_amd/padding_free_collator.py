@@ -11,8 +11,28 @@ import torch
 from . import _lib, model_utils
 
 
+def shifted_and_kept(
+    labels: torch.Tensor, fill: int = -100, ignored: int = -100, want_keep: bool = True
+) -> tuple[torch.Tensor, torch.Tensor | None]:
+    """``labels[..., 1:]`` with ``fill`` in the last position, and which of them are not ``ignored``."""
+    if labels.is_cuda and labels.dtype == torch.int64 and labels.ndim > 0 and labels.numel() > 0 and labels.is_contiguous():
+        out = torch.empty_like(labels)
+        keep = torch.empty(labels.shape, dtype=torch.bool, device=labels.device) if want_keep else None
+        cols = labels.shape[-1]
+        _lib.call(
+            "oi_shift_labels", labels.data_ptr(), labels.numel() // cols, cols, fill, ignored, out.data_ptr(), _lib.ptr(keep),
+            _lib.stream_of(labels),
+        )  # fmt: skip
+        return out, keep
+    out = torch.full_like(labels, fill)
+    out[..., :-1] = labels[..., 1:]
+    return out, (out != ignored if want_keep else None)
+
+
 def shift_labels(labels: torch.Tensor) -> torch.Tensor:
     """``out[:, i] = labels[:, i + 1]`` with ``-100`` in the last position (index plumbing, bit-exact)."""
+    if labels.ndim == 2:
+        return shifted_and_kept(labels, want_keep=False)[0]
     out = torch.full_like(labels, -100)
     out[:, :-1] = labels[:, 1:]
     return out
@@ -25,8 +45,8 @@ def calculate_per_token_logps(logits: torch.Tensor, labels: torch.Tensor) -> tor
     (``-100``) and the last position score token 0, exactly as the reference's ``clamp(min=0)``.
     The logits are read once in their own dtype and accumulated in fp32; no fp32 copy is made.
     """
-    safe = shift_labels(labels).clamp(min=0)
-    return model_utils.log_softmax_and_gather(logits, safe)
+    # the kernels score token 0 where the label is negative
+    return model_utils.log_softmax_and_gather(logits, shift_labels(labels))
 
 
 class _SeqLogps(torch.autograd.Function):

@@ -10,7 +10,7 @@ import pytest
 import torch
 
 from conftest import make_grpo_config
-from open_instruct_amd import _lib, grpo_utils, model_utils
+from open_instruct_amd import _lib, grpo_utils, model_utils, padding_free_collator
 from oracle import grpo as o_grpo
 
 pytestmark = pytest.mark.gpu
@@ -137,6 +137,24 @@ def test_statistics_of_few_and_many_rows(rows, cols, axis):
     assert stats["num_response_tokens"].item() == float(mask.sum())
     mean_pg = (e_pg.detach() * mask).sum().item() / mask.sum().item()
     assert abs(stats["loss/policy_avg"].item() - mean_pg) <= 1e-5 * max(1.0, abs(mean_pg))
+
+
+@pytest.mark.parametrize("shape", [(1, 1), (1, 2), (3, 85), (2, 256), (5, 1), (7,)])
+@pytest.mark.parametrize("fill,ignored", [(-100, -100), (-100, 3), (7, 7)])
+def test_shifted_labels(shape, fill, ignored):
+    g = torch.Generator().manual_seed(3)
+    labels = torch.randint(-1, 9, shape, generator=g)
+    labels[labels < 0] = -100
+    want = torch.full_like(labels, fill)
+    want[..., :-1] = labels[..., 1:]
+    # contiguous rows have a kernel, others the general way
+    wide = torch.empty((*shape[:-1], shape[-1] + 2), dtype=torch.int64, device=DEV)
+    wide[..., 1:-1] = labels
+    for given in (labels.to(DEV), wide[..., 1:-1], labels.to(DEV).to(torch.int32)):
+        out, keep = padding_free_collator.shifted_and_kept(given, fill, ignored)
+        assert out.dtype == given.dtype and keep.dtype == torch.bool
+        assert torch.equal(out.cpu().long(), want) and torch.equal(keep.cpu(), want != ignored)
+    assert padding_free_collator.shifted_and_kept(labels.to(DEV), want_keep=False)[1] is None
 
 
 # bytes in front of the first 16-byte boundary and behind the last, one workgroup and as many as count for themselves
