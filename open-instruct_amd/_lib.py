@@ -155,8 +155,14 @@ def ptr(t: torch.Tensor | None) -> int | None:
     return None if t is None else t.data_ptr()
 
 
+# the handle itself; without a stream object around it 0.3 instead of 2.5 us of every call
+_current_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def stream_of(t: torch.Tensor) -> int:
-    return torch.cuda.current_stream(t.device).cuda_stream
+    if _current_stream is None:
+        return torch.cuda.current_stream(t.device).cuda_stream
+    return _current_stream(t.get_device())
 
 
 def require_gpu(*tensors: torch.Tensor | None) -> torch.device:

@@ -60,10 +60,10 @@ class _SigmoidPairLoss(torch.autograd.Function):
         w_c = _lib.f32c(weights).reshape(-1) if weights is not None else None
         n = pc_c.numel()
         out = torch.empty((3, n), dtype=torch.float32, device=dev)
+        at = out.data_ptr()
         _lib.call(
             "oi_dpo_sigmoid_fwd", pc_c.data_ptr(), pr_c.data_ptr(), _lib.ptr(rc_c), _lib.ptr(rr_c), _lib.ptr(w_c), n,
-            beta, label_smoothing, margin, out[0].data_ptr(), out[1].data_ptr(), out[2].data_ptr(),
-            _lib.stream_of(pc_c),
+            beta, label_smoothing, margin, at, at + 4 * n, at + 8 * n, _lib.stream_of(pc_c),
         )  # fmt: skip
         ctx.save_for_backward(pc_c, pr_c, rc_c, rr_c, w_c)
         ctx.meta = (beta, label_smoothing, margin, shape, pc.dtype, pr.dtype)
@@ -81,9 +81,10 @@ class _SigmoidPairLoss(torch.autograd.Function):
         d = torch.empty((2, n), dtype=torch.float32, device=g.device)
         _lib.call(
             "oi_dpo_sigmoid_bwd", pc_c.data_ptr(), pr_c.data_ptr(), _lib.ptr(rc_c), _lib.ptr(rr_c), _lib.ptr(w_c),
-            g.data_ptr(), n, beta, ls, margin, d[0].data_ptr(), d[1].data_ptr(), _lib.stream_of(g),
+            g.data_ptr(), n, beta, ls, margin, d.data_ptr(), d.data_ptr() + 4 * n, _lib.stream_of(g),
         )  # fmt: skip
-        return d[0].reshape(shape).to(dt_c), d[1].reshape(shape).to(dt_r), None, None, None, None, None, None
+        d_c, d_r = d.unbind(0)
+        return d_c.reshape(shape).to(dt_c), d_r.reshape(shape).to(dt_r), None, None, None, None, None, None
 
 
 def dpo_loss(

@@ -123,7 +123,7 @@ def compute_rho_correction(
             int(bool(config.rho_mask_tv_divergence)) if use else 0,
             float(config.rho_mask_lower_bound) if use else 0.0, float(config.rho_mask_upper_bound) if use else 0.0,
             float(config.rho_clamp_lower_bound) if use else 0.0, float(config.rho_clamp_upper_bound) if use else 0.0,
-            *[bufs[k].data_ptr() for k in range(6)], _lib.stream_of(old),
+            *[bufs.data_ptr() + 4 * k * old.numel() for k in range(6)], _lib.stream_of(old),
         )  # fmt: skip
         rho, weights, drop_any, drop_low, drop_high, clipped = bufs.unbind(0)
         hist = {"val/rho_hist": _picked(rho, m)}
@@ -217,10 +217,10 @@ class _GrpoTerms(torch.autograd.Function):
         w = _lib.f32c(rho_weights.expand(shape))
         ref = _lib.f32c(ref_logprobs.expand(shape)) if ref_logprobs is not None else None
         out = torch.empty((3,) + tuple(shape), dtype=torch.float32, device=dev)
-        n = nl.numel()
+        n, at = nl.numel(), out.data_ptr()
         _lib.call(
             "oi_grpo_terms_fwd", nl.data_ptr(), rt.data_ptr(), adv.data_ptr(), _lib.ptr(ref), w.data_ptr(), n, loss_fn,
-            lo, hi, kl_estimator, out[0].data_ptr(), out[1].data_ptr(), out[2].data_ptr(), _lib.stream_of(nl),
+            lo, hi, kl_estimator, at, at + 4 * n, at + 8 * n, _lib.stream_of(nl),
         )  # fmt: skip
         ctx.save_for_backward(nl, rt, adv, ref, w)
         ctx.cfg = (loss_fn, lo, hi, kl_estimator)
