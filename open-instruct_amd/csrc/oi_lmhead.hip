@@ -1236,7 +1236,7 @@ static_assert(2 * GROUP_F32 <= LDS_ELEMS, "the epilogue's regions fit the ring")
 // 128256 x 4096, K = 7680 6000, 6005).
 //
 // Rows and columns past the end read what the last valid ones do, and store nothing.
-template <bool PLAIN, int PIECES>
+template <bool PLAIN, int PIECES, int NJ = WIDE>
 struct GroupRows {
     float a, b;       // factors of the lane's accumulator row
     int dst[PIECES];  // result rows of the thread's pieces
@@ -1246,13 +1246,13 @@ struct GroupRows {
         if constexpr (!PLAIN) {
             const int64_t last = st.m_valid - 1;
             if (st.scale_a) {
-                const int64_t row = group_row(row0, j, srow);
+                const int64_t row = group_row<NJ>(row0, j, srow);
                 a = st.scale_a[row < last ? row : last];
                 b = st.scale_b[row < last ? row : last];
             }
 #pragma unroll
             for (int it = 0; it < PIECES; ++it) {
-                const int64_t row = group_row(row0, j, r_first + it * step);
+                const int64_t row = group_row<NJ>(row0, j, r_first + it * step);
                 dst[it] = (int)row;
                 if (st.mode >= 2 && st.out_rows) dst[it] = st.out_rows[row < last ? row : last];
             }
@@ -1265,7 +1265,7 @@ struct GroupRows {
     }
     // element offset of column col of piece it, group row r
     __device__ __forceinline__ int64_t at(const StoreTo& st, int64_t row0, int64_t col, int j, int r, int it) const {
-        return (PLAIN ? group_row(row0, j, r) : (int64_t)dst[it]) * st.ldo + col;
+        return (PLAIN ? group_row<NJ>(row0, j, r) : (int64_t)dst[it]) * st.ldo + col;
     }
 };
 // mode 2 in whole pieces.  PLAIN results (d_weight) are as large as the head, and who reads them next does so long after
@@ -1305,9 +1305,9 @@ __device__ __forceinline__ void store_group_bf16(const f32x16& z0, const f32x16&
 // Every other mode, any pitch, any alignment of the element type.  ADDS: modes 1 and 3 in whole pieces.
 // Piece `it` of a thread is row (thread / 64) + 8 it of the group, columns 4 (thread mod 64) ..
 constexpr int F32_PIECES = GROUP_ROWS * (BM / 4) / NTHREADS;
-template <bool PLAIN, bool ADDS>
+template <bool PLAIN, bool ADDS, int NJ = WIDE>
 struct F32Rows {
-    GroupRows<PLAIN, F32_PIECES> rows;
+    GroupRows<PLAIN, F32_PIECES, NJ> rows;
     oi_f32x4 sum[F32_PIECES];
 
     __device__ __forceinline__ void request(const StoreTo& st, int64_t row0, int64_t col0, int j, int tid) {
@@ -1321,15 +1321,15 @@ struct F32Rows {
             const uint32_t col = c < last_c ? c : last_c;
 #pragma unroll
             for (int it = 0; it < F32_PIECES; ++it) {
-                const int64_t row = group_row(row0, j, wave + it * (NTHREADS / 64));
+                const int64_t row = group_row<NJ>(row0, j, wave + it * (NTHREADS / 64));
                 sum[it] = *reinterpret_cast<const oi_f32x4*>(st.out_f32 + (row < last ? row : last) * st.ldo + col0 + col);
             }
         }
     }
 };
-template <bool PLAIN, bool ADDS>
+template <bool PLAIN, bool ADDS, int NJ = WIDE>
 __device__ __forceinline__ void store_group_f32(const f32x16& z0, const f32x16& z1, const StoreTo& st, bool pieces,
-                                                const F32Rows<PLAIN, ADDS>& in, int64_t row0, int64_t col0, int j,
+                                                const F32Rows<PLAIN, ADDS, NJ>& in, int64_t row0, int64_t col0, int j,
                                                 uint16_t* stage, int tid) {
     asm volatile("" : "+v"(tid));
     const int lane = tid & 63, wave = tid >> 6, wm = wave & 3, wn = wave >> 2;
@@ -1357,7 +1357,7 @@ __device__ __forceinline__ void store_group_f32(const f32x16& z0, const f32x16& 
     if (mode <= 1 && (ADDS || pieces)) {
 #pragma unroll
         for (int it = 0; it < F32_PIECES; ++it) {
-            const int64_t row = group_row(row0, j, r_first + it * 8);
+            const int64_t row = group_row<NJ>(row0, j, r_first + it * 8);
             const oi_f32x4 v = piece(it);
             if (row < st.m_valid && col < st.N) *reinterpret_cast<oi_f32x4*>(st.out_f32 + row * st.ldo + col) = v;
         }
@@ -1368,7 +1368,7 @@ __device__ __forceinline__ void store_group_f32(const f32x16& z0, const f32x16& 
         for (int it = 0; it < F32_PIECES; ++it) {
             const int r = r_first + it * 8;
             const oi_f32x4 v = piece(it);
-            if (group_row(row0, j, r) >= st.m_valid || col >= st.N) continue;
+            if (group_row<NJ>(row0, j, r) >= st.m_valid || col >= st.N) continue;
             *reinterpret_cast<uint2*>(st.out_bf16 + rows.at(st, row0, col, j, r, it)) =
                 make_uint2(oi_pack_bf16x2(v.x, v.y), oi_pack_bf16x2(v.z, v.w));
         }
@@ -1378,7 +1378,7 @@ __device__ __forceinline__ void store_group_f32(const f32x16& z0, const f32x16& 
     if (col >= st.N) return;
 #pragma unroll 1
     for (int it = 0; it < F32_PIECES; ++it) {
-        const int64_t row = group_row(row0, j, r_first + it * 8);
+        const int64_t row = group_row<NJ>(row0, j, r_first + it * 8);
         if (row >= st.m_valid) break;
         oi_f32x4 v = *reinterpret_cast<const oi_f32x4*>(from + it * 8 * STAGE_F32);
         if (mode == 3) v += *reinterpret_cast<const oi_f32x4*>(st.out_f32 + row * st.ldo + col);
@@ -1487,23 +1487,66 @@ struct DynRows {
 // tiles, 4096, 128256: unchanged (a last round that is 7/8 full is left alone).
 struct TailSplit {
     uint32_t whole, rest, parts;  // tiles [0, whole) in one piece, the `rest` after them in `parts` pieces
+    uint32_t cost;                // of the last round, in 32nds of a k-tile
 };
 constexpr uint32_t SPLIT_MIN_KTILES = 16, SPLIT_MAX_PARTS = 32, SPLIT_MAX_ITEMS = 1024;
-__host__ __device__ inline TailSplit plan_tail(uint32_t tiles, uint32_t grid, uint32_t ktiles) {
-    TailSplit t = {tiles, 0, 1};
+// cost of `parts` pieces, in 32nds of a k-tile (`per_ktile`: what one takes); SPLIT_NEVER: not to be had
+constexpr uint32_t SPLIT_NEVER = 0x3ffffffu;  // costs are below, 32 * 2^16 k-tiles and less than half of that besides
+__host__ __device__ inline uint32_t split_cost(uint32_t rest, uint32_t grid, uint32_t ktiles, uint32_t per_ktile, uint32_t parts) {
+    if (parts == 1) return per_ktile * ktiles + 32 * 4;
+    if (parts > SPLIT_MAX_PARTS || rest * parts > SPLIT_MAX_ITEMS || ktiles < SPLIT_MIN_KTILES * parts) return SPLIT_NEVER;
+    const uint32_t rounds = (rest * parts + grid - 1) / grid;
+    return rounds * (per_ktile * ktiles / parts + 32 * 4) + 3 * rest * parts;
+}
+// Every lane of a wave weighs one number of parts on the device: one after the other, in all waves of a launch, they
+// took as long as two k-tiles.
+__host__ __device__ inline TailSplit plan_tail(uint32_t tiles, uint32_t grid, uint32_t ktiles, uint32_t per_ktile = 32) {
     const uint32_t rest = tiles % grid;
-    if (rest == 0) return t;
-    uint32_t best = 32 * (ktiles + 4);
-    for (uint32_t parts = 2; parts <= SPLIT_MAX_PARTS; ++parts) {
-        if (rest * parts > SPLIT_MAX_ITEMS || ktiles < SPLIT_MIN_KTILES * parts) break;
-        const uint32_t rounds = (rest * parts + grid - 1) / grid;
-        const uint32_t cost = rounds * (32 * ktiles / parts + 32 * 4) + 3 * rest * parts;
-        if (cost < best) {
-            best = cost;
-            t = {tiles - rest, rest, parts};
-        }
+    if (rest == 0) return {tiles, 0, 1, split_cost(grid, grid, ktiles, per_ktile, 1)};
+#ifdef __HIP_DEVICE_COMPILE__
+    const uint32_t mine = 1 + __lane_id();
+    uint32_t best = split_cost(rest, grid, ktiles, per_ktile, mine) * 64 + (mine & 63);
+#pragma unroll
+    for (int d = 32; d > 0; d >>= 1) {
+        const uint32_t other = __shfl_xor(best, d, OI_WAVE);
+        best = other < best ? other : best;
     }
-    return t;
+    best = __builtin_amdgcn_readfirstlane(best);
+#else
+    uint32_t best = ~0u;
+    for (uint32_t parts = 1; parts <= SPLIT_MAX_PARTS; ++parts) {
+        const uint32_t cost = split_cost(rest, grid, ktiles, per_ktile, parts) * 64 + parts;
+        best = cost < best ? cost : best;
+    }
+#endif
+    const uint32_t parts = best & 63;
+    if (parts == 1) return {tiles, 0, 1, best >> 6};
+    return {tiles - rest, rest, parts, best >> 6};
+}
+
+// Rows products of few rows also come in tiles of 192 rows, all of them: 268 rows are then 384 instead of 512 that are
+// multiplied.  (One narrow tile among wide ones has pieces of another length, falls out of step with those that read the
+// same k-tiles of W, and gains nothing.)  A k-tile of theirs takes 26/32 of a wide one's time, and what takes less by the
+// estimate is chosen, where that leaves all tiles in one round and in pieces.  d_hidden, us in tiles of 256 and of 192:
+// 4096 x 100352 268 rows 295, 235; 384 299, 246; 520 448, 365; 1152 743, 735; 8192 x 128256 268 rows 728, 596; 520 1109, 898;
+// 3584 x 151665 268 rows 426, 347; 2048 x 151936 268 rows 266, 211.  Counts in between stay with 256 (4096 x 100352 400
+// rows 294, 600 441).  Kernels of calls with more than 8 tiles of rows have no code for it: their gain would be 6 % at most.
+constexpr int FEWER = 6;
+constexpr uint32_t FEWER_COST = 26, FEWER_ROWS = 32 * FEWER;
+inline bool rows_come_in_widths(int64_t row_tiles) { return row_tiles <= 8; }
+inline int64_t fewer_tiles(int64_t rows) { return (rows + FEWER_ROWS - 1) / FEWER_ROWS; }
+struct RowsPlan {
+    TailSplit split;
+    bool fewer;
+};
+// M: the rows of whole tiles, `rows` what there is of them
+__host__ __device__ inline RowsPlan plan_rows(int64_t M, int64_t rows, uint32_t tiles_c, uint32_t grid, uint32_t ktiles, bool widths) {
+    RowsPlan p = {plan_tail((uint32_t)((M + BN - 1) / BN) * tiles_c, grid, ktiles), false};
+    if (!widths || p.split.whole) return p;
+    const uint32_t tiles = (uint32_t)((rows + FEWER_ROWS - 1) / FEWER_ROWS) * tiles_c;
+    const TailSplit t = plan_tail(tiles, grid, ktiles, FEWER_COST);
+    if (tiles < grid && t.whole == 0 && t.cost < p.split.cost) p = {t, true};
+    return p;
 }
 
 // The sizes of a product that only the device knows, filled in from dyn
@@ -1526,7 +1569,8 @@ __device__ __forceinline__ ProductSizes product_sizes(int64_t M, int64_t K, int6
 
 // `queue` null: one workgroup per tile id (blockIdx); otherwise a launch of resident workgroups
 // that draw their tiles from the queue.  `parts` (with a queue only): scratch for the pieces of split tiles.
-template <bool R_KM, bool C_KM>
+// WIDTHS: rows products (role 1) in tiles of one of two heights, see plan_rows.
+template <bool R_KM, bool C_KM, bool WIDTHS = false>
 __global__ void __launch_bounds__(NTHREADS)
     gemm_store_kernel(Operand R, int64_t M, Operand C, int64_t N, int64_t K, int mode, float* out_f32,
                       uint16_t* out_bf16, int64_t ldo, int64_t m_valid, DynRows dyn, uint32_t* __restrict__ queue,
@@ -1550,10 +1594,14 @@ __global__ void __launch_bounds__(NTHREADS)
         store_no_terms(st);
         return;
     }
-    const uint32_t tiles_r = (uint32_t)((z.M + BN - 1) / BN), tiles_c = (uint32_t)((N + BM - 1) / BM);
-    const uint32_t tiles = tiles_r * tiles_c, ktiles = (uint32_t)(K / BK);
-    TailSplit ts = {tiles, 0, 1};
-    if (parts) ts = plan_tail(tiles, gridDim.x, ktiles);
+    const uint32_t tiles_c = (uint32_t)((N + BM - 1) / BM), ktiles = (uint32_t)(K / BK);
+    RowsPlan rp = {{0, 0, 1, 0}, false};
+    if (parts) rp = plan_rows(z.M, z.m_valid, tiles_c, gridDim.x, ktiles, WIDTHS);
+    const uint32_t height = WIDTHS && rp.fewer ? FEWER_ROWS : BN;
+    const uint32_t tiles_r = (uint32_t)(((WIDTHS && rp.fewer ? z.m_valid : z.M) + height - 1) / height);
+    const uint32_t tiles = tiles_r * tiles_c;
+    TailSplit ts = rp.split;
+    if (!parts) ts.whole = tiles;
     auto tile_at = [&](uint32_t any_item) {
         const uint32_t item = __builtin_amdgcn_readfirstlane(any_item);
         ProductTile t = {R, C, K, nullptr};
@@ -1572,7 +1620,7 @@ __global__ void __launch_bounds__(NTHREADS)
         }
         int64_t tr, tc;
         tile_of_item(tile, tiles_r, tiles_c, &tr, &tc);
-        t.R.r0 = tr * BN;
+        t.R.r0 = tr * height;
         t.C.r0 = tc * BM;
         return t;
     };
@@ -1590,6 +1638,28 @@ __global__ void __launch_bounds__(NTHREADS)
     }
     if (item >= q.items) return;
     ProductTile t = tile_at(item);
+    if constexpr (WIDTHS) {
+        if (rp.fewer) {  // all of them in pieces, which leave without the LDS
+            begin_loads<C_KM, R_KM, FEWER>(t.C, t.R, t.K, lds);
+            for (;;) {
+                AccTile<FEWER> acc;
+                q.request();
+                gemm_loop<C_KM, R_KM>(acc, t.C, t.R, t.K, lds);
+                q.settle();
+                item = q.take_item();
+                float* part = t.part;
+                if (item != ItemQueue::NONE) {
+                    t = tile_at(item);
+                    begin_loads<C_KM, R_KM, FEWER>(t.C, t.R, t.K, lds);
+                }
+                const int tid = opaque_tid();
+#pragma unroll
+                for (int j = 0; j < FEWER / 2; ++j) store_part(tile_columns<FEWER>(acc, j), part, j, tid);
+                if (item == ItemQueue::NONE) return;
+                lds_barrier();  // every wave has read the queue's word, which lies in slot 4
+            }
+        }
+    }
     begin_loads<C_KM, R_KM>(t.C, t.R, t.K, lds);
     for (;;) {
         AccTile<> acc;
@@ -1848,15 +1918,17 @@ __global__ void __launch_bounds__(NTHREADS)
 // bound by reading the pieces once.
 __global__ void __launch_bounds__(NTHREADS)
     gemm_reduce_kernel(const float* __restrict__ parts, uint32_t grid, int64_t M, int64_t N, int64_t K, int mode,
-                       float* out_f32, uint16_t* out_bf16, int64_t ldo, int64_t m_valid, DynRows dyn) {
+                       float* out_f32, uint16_t* out_bf16, int64_t ldo, int64_t m_valid, DynRows dyn, bool widths) {
     __shared__ __align__(16) uint16_t stage[GROUP_F32];
     const ProductSizes z = product_sizes(M, K, m_valid, dyn);
     const StoreTo st = {mode, out_f32, out_bf16, ldo, N, z.m_valid, dyn.out_rows, dyn.scale_a, dyn.scale_b};
-    const int64_t tiles_r = (z.M + BN - 1) / BN, tiles_c = (N + BM - 1) / BM;
-    const TailSplit ts = plan_tail((uint32_t)(tiles_r * tiles_c), grid, (uint32_t)(z.K / BK));
+    const int64_t tiles_c = (N + BM - 1) / BM;
+    const RowsPlan rp = plan_rows(z.M, z.m_valid, (uint32_t)tiles_c, grid, (uint32_t)(z.K / BK), widths);
+    const TailSplit ts = rp.split;
+    const int64_t height = rp.fewer ? FEWER_ROWS : BN, tiles_r = ((rp.fewer ? z.m_valid : z.M) + height - 1) / height;
     const uint32_t tile = blockIdx.x >> 2;
     const int j = blockIdx.x & 3, tid = threadIdx.x;
-    if (tile >= ts.rest) return;
+    if (tile >= ts.rest || j * 2 >= (rp.fewer ? FEWER : WIDE)) return;
     const float* src = parts + (int64_t)tile * PART_FLOATS;
     Columns c = load_part(src, j, tid);
     for (uint32_t p = 1; p < ts.parts; ++p) {
@@ -1870,16 +1942,18 @@ __global__ void __launch_bounds__(NTHREADS)
     int64_t tr, tc;
     tile_of_item(ts.whole + tile, (uint32_t)tiles_r, (uint32_t)tiles_c, &tr, &tc);
     const bool pieces = stores_in_pieces(st);
-    const int64_t row0 = tr * BN, col0 = tc * BM;
-    if (adds_in_pieces(st, pieces)) {
-        F32Rows<false, true> in;
+    const int64_t row0 = tr * height, col0 = tc * BM;
+    auto store = [&](auto adds, auto nj) {
+        F32Rows<false, decltype(adds)::value, decltype(nj)::value> in;
         in.request(st, row0, col0, j, tid);
-        store_group_f32<false, true>(c.z[0], c.z[1], st, pieces, in, row0, col0, j, stage, tid);
-    } else {
-        F32Rows<false, false> in;
-        in.request(st, row0, col0, j, tid);
-        store_group_f32<false, false>(c.z[0], c.z[1], st, pieces, in, row0, col0, j, stage, tid);
-    }
+        store_group_f32<false, decltype(adds)::value, decltype(nj)::value>(c.z[0], c.z[1], st, pieces, in, row0, col0, j, stage, tid);
+    };
+    auto store_rows = [&](auto nj) {
+        if (adds_in_pieces(st, pieces)) store(std::true_type{}, nj);
+        else store(std::false_type{}, nj);
+    };
+    if (rp.fewer) store_rows(std::integral_constant<int, FEWER>{});
+    else store_rows(std::integral_constant<int, WIDE>{});
 }
 
 inline int64_t round_up(int64_t x, int64_t m) { return (x + m - 1) / m * m; }
@@ -2180,10 +2254,14 @@ size_t split_bytes(int64_t row_tiles, int64_t h_tiles, int64_t chunk, int64_t vo
     for (int64_t c : columns) {
         const uint32_t ktiles = (uint32_t)(round_up(c, BK) / BK);
         // what is left of whole rounds repeats after `grid` row tiles
-        for (int64_t r = 1; r <= row_tiles && r <= (int64_t)grid && ktiles >= 2 * SPLIT_MIN_KTILES; ++r) {
-            const TailSplit t = plan_tail((uint32_t)(r * h_tiles), grid, ktiles);
-            if (t.rest * t.parts > most) most = t.rest * t.parts;
-        }
+        auto up_to = [&](int64_t rows, uint32_t per_ktile) {
+            for (int64_t r = 1; r <= rows && r <= (int64_t)grid && ktiles >= 2 * SPLIT_MIN_KTILES; ++r) {
+                const TailSplit t = plan_tail((uint32_t)(r * h_tiles), grid, ktiles, per_ktile);
+                if (t.rest * t.parts > most) most = t.rest * t.parts;
+            }
+        };
+        up_to(row_tiles, 32);
+        if (rows_come_in_widths(row_tiles)) up_to(fewer_tiles(row_tiles * BN), FEWER_COST);
         if (columns[0] == columns[1]) break;
     }
     return (size_t)most * PART_FLOATS * sizeof(float);
@@ -2439,13 +2517,15 @@ void launch_rows_product(unsigned grid, const Operand& a, int64_t M, const Opera
                          float* out_f32, void* out_bf16, int64_t ldo, int64_t m_valid, const DynRows& dyn,
                          uint32_t* queue, float* parts, hipStream_t s) {
     uint16_t* o16 = static_cast<uint16_t*>(out_bf16);
-    hipLaunchKernelGGL((gemm_store_kernel<false, true>), dim3(grid), dim3(NTHREADS), 0, s, a, M, b, N, K, mode, out_f32,
-                       o16, ldo, m_valid, dyn, queue, parts);
+    const bool widths = parts && rows_come_in_widths(M / BM);
+    auto* kernel = widths ? gemm_store_kernel<false, true, true> : gemm_store_kernel<false, true, false>;
+    hipLaunchKernelGGL(kernel, dim3(grid), dim3(NTHREADS), 0, s, a, M, b, N, K, mode, out_f32, o16, ldo, m_valid, dyn, queue,
+                       parts);
     if (!parts) return;
-    const int64_t tiles = (M + BM - 1) / BM * ((N + BN - 1) / BN);
+    const int64_t tiles = (widths ? fewer_tiles(M) : M / BM) * ((N + BN - 1) / BN);
     const int64_t most = tiles < (int64_t)grid ? tiles : (int64_t)grid - 1;  // tiles past the last whole round
     hipLaunchKernelGGL(gemm_reduce_kernel, dim3((unsigned)(most * 4)), dim3(NTHREADS), 0, s, parts, grid, M, N, K, mode,
-                       out_f32, o16, ldo, m_valid, dyn);
+                       out_f32, o16, ldo, m_valid, dyn, widths);
 }
 
 // The forward that also prepares d_hidden.  With x = z c in the log2 domain and a per-token

@@ -359,6 +359,32 @@ def test_row_selection_on_device(keep, want_dw):
             assert not dw.grad.any()
 
 
+@pytest.mark.parametrize("count", [1, 192, 193, 256, 257, 384, 385, 513, 576, 577, 1025, 1152, 1153])
+@pytest.mark.parametrize("h,want_dw", [(128, True), (576, False)])
+def test_selected_rows_in_tiles_of_either_height(count, h, want_dw):
+    """Counts around multiples of 192 and 256, the two heights that tiles of the d_hidden product come in when there are
+    few rows; vocabulary long enough for its tiles to be cut into pieces."""
+    n, v = 1280, 3000
+    hidden, weight, labels = _case(n, h, v, seed=25, w_scale=3.0 / math.sqrt(h))
+    g = torch.Generator().manual_seed(26)
+    mask = torch.zeros(n, dtype=torch.bool)
+    mask[torch.randperm(n, generator=g)[:count]] = True
+    upstream = torch.randn(n, generator=g)
+    rh = hidden.float().requires_grad_(True)
+    rw = weight.float().requires_grad_(True)
+    lp_o, _ = o_lm.lm_head_logprobs(rh, rw, labels, 0.9)
+    (lp_o * mask).backward(upstream)
+    dh = hidden.to(DEV).requires_grad_(True)
+    dw = weight.to(DEV).requires_grad_(want_dw)
+    lp, _ = lm_head.fused_lm_head_logprobs(dh, dw, labels.to(DEV), 0.9, mask=mask.to(DEV))
+    lp.backward(upstream.to(DEV))
+    assert (dh.grad.cpu()[~mask] == 0).all()
+    worst = (dh.grad.float().cpu() - rh.grad).norm(dim=1) / rh.grad.norm(dim=1).clamp(min=1e-30)
+    assert worst[mask].max().item() <= 2e-2
+    if want_dw:
+        assert ((dw.grad.float().cpu() - rw.grad).norm() / rw.grad.norm()).item() <= 2e-2
+
+
 def test_row_selection_with_compact_backward_and_mask():
     """Mask and zero-gradient rows together: the backward selects rows that are in the mask AND carry
     a gradient."""
