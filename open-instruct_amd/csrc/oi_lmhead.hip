@@ -1470,6 +1470,8 @@ struct DynRows {
     const float *scale_a, *scale_b;
     // optional: the store mode comes from device memory (a negative value: the launch does nothing)
     const int32_t* mode_dev;
+    // role 1: pieces of tiles that the scratch holds, where tiles may have either height (plan_rows)
+    uint32_t pieces = 0;
 };
 
 // A launch of resident workgroups computes its tiles in rounds of one per workgroup, and a last round
@@ -1490,22 +1492,25 @@ struct TailSplit {
     uint32_t cost;                // of the last round, in 32nds of a k-tile
 };
 constexpr uint32_t SPLIT_MIN_KTILES = 16, SPLIT_MAX_PARTS = 32, SPLIT_MAX_ITEMS = 1024;
-// cost of `parts` pieces, in 32nds of a k-tile (`per_ktile`: what one takes); SPLIT_NEVER: not to be had
+// cost of `parts` pieces for each tile, in 32nds of a k-tile (`per_ktile`: what one takes), `most` in all; SPLIT_NEVER: not
+// to be had
 constexpr uint32_t SPLIT_NEVER = 0x3ffffffu;  // costs are below, 32 * 2^16 k-tiles and less than half of that besides
-__host__ __device__ inline uint32_t split_cost(uint32_t rest, uint32_t grid, uint32_t ktiles, uint32_t per_ktile, uint32_t parts) {
+__host__ __device__ inline uint32_t split_cost(uint32_t rest, uint32_t grid, uint32_t ktiles, uint32_t per_ktile, uint32_t most,
+                                               uint32_t parts) {
     if (parts == 1) return per_ktile * ktiles + 32 * 4;
-    if (parts > SPLIT_MAX_PARTS || rest * parts > SPLIT_MAX_ITEMS || ktiles < SPLIT_MIN_KTILES * parts) return SPLIT_NEVER;
+    if (parts > SPLIT_MAX_PARTS || rest * parts > most || ktiles < SPLIT_MIN_KTILES * parts) return SPLIT_NEVER;
     const uint32_t rounds = (rest * parts + grid - 1) / grid;
     return rounds * (per_ktile * ktiles / parts + 32 * 4) + 3 * rest * parts;
 }
 // Every lane of a wave weighs one number of parts on the device: one after the other, in all waves of a launch, they
 // took as long as two k-tiles.
-__host__ __device__ inline TailSplit plan_tail(uint32_t tiles, uint32_t grid, uint32_t ktiles, uint32_t per_ktile = 32) {
+__host__ __device__ inline TailSplit plan_tail(uint32_t tiles, uint32_t grid, uint32_t ktiles, uint32_t per_ktile = 32,
+                                               uint32_t most = SPLIT_MAX_ITEMS) {
     const uint32_t rest = tiles % grid;
-    if (rest == 0) return {tiles, 0, 1, split_cost(grid, grid, ktiles, per_ktile, 1)};
+    if (rest == 0) return {tiles, 0, 1, split_cost(grid, grid, ktiles, per_ktile, most, 1)};
 #ifdef __HIP_DEVICE_COMPILE__
     const uint32_t mine = 1 + __lane_id();
-    uint32_t best = split_cost(rest, grid, ktiles, per_ktile, mine) * 64 + (mine & 63);
+    uint32_t best = split_cost(rest, grid, ktiles, per_ktile, most, mine) * 64 + (mine & 63);
 #pragma unroll
     for (int d = 32; d > 0; d >>= 1) {
         const uint32_t other = __shfl_xor(best, d, OI_WAVE);
@@ -1515,7 +1520,7 @@ __host__ __device__ inline TailSplit plan_tail(uint32_t tiles, uint32_t grid, ui
 #else
     uint32_t best = ~0u;
     for (uint32_t parts = 1; parts <= SPLIT_MAX_PARTS; ++parts) {
-        const uint32_t cost = split_cost(rest, grid, ktiles, per_ktile, parts) * 64 + parts;
+        const uint32_t cost = split_cost(rest, grid, ktiles, per_ktile, most, parts) * 64 + parts;
         best = cost < best ? cost : best;
     }
 #endif
@@ -1533,18 +1538,20 @@ __host__ __device__ inline TailSplit plan_tail(uint32_t tiles, uint32_t grid, ui
 // rows 294, 600 441).  Kernels of calls with more than 8 tiles of rows have no code for it: their gain would be 6 % at most.
 constexpr int FEWER = 6;
 constexpr uint32_t FEWER_COST = 26, FEWER_ROWS = 32 * FEWER;
-inline bool rows_come_in_widths(int64_t row_tiles) { return row_tiles <= 8; }
-inline int64_t fewer_tiles(int64_t rows) { return (rows + FEWER_ROWS - 1) / FEWER_ROWS; }
+inline bool either_height(int64_t row_tiles) { return row_tiles <= 8; }
+__host__ __device__ inline uint32_t fewer_tiles(int64_t rows) { return (uint32_t)((rows + FEWER_ROWS - 1) / FEWER_ROWS); }
 struct RowsPlan {
     TailSplit split;
     bool fewer;
 };
-// M: the rows of whole tiles, `rows` what there is of them
-__host__ __device__ inline RowsPlan plan_rows(int64_t M, int64_t rows, uint32_t tiles_c, uint32_t grid, uint32_t ktiles, bool widths) {
+// M: the rows of whole tiles, `rows` what there is of them; `pieces`: what the scratch holds (that of tiles of 256 rows at
+// any count up to the call's), 0 for tiles of 256 only
+__device__ __forceinline__ RowsPlan plan_rows(int64_t M, int64_t rows, uint32_t tiles_c, uint32_t grid, uint32_t ktiles,
+                                              uint32_t pieces) {
     RowsPlan p = {plan_tail((uint32_t)((M + BN - 1) / BN) * tiles_c, grid, ktiles), false};
-    if (!widths || p.split.whole) return p;
-    const uint32_t tiles = (uint32_t)((rows + FEWER_ROWS - 1) / FEWER_ROWS) * tiles_c;
-    const TailSplit t = plan_tail(tiles, grid, ktiles, FEWER_COST);
+    if (pieces == 0 || p.split.whole) return p;
+    const uint32_t tiles = fewer_tiles(rows) * tiles_c;
+    const TailSplit t = plan_tail(tiles, grid, ktiles, FEWER_COST, pieces);
     if (tiles < grid && t.whole == 0 && t.cost < p.split.cost) p = {t, true};
     return p;
 }
@@ -1596,9 +1603,9 @@ __global__ void __launch_bounds__(NTHREADS)
     }
     const uint32_t tiles_c = (uint32_t)((N + BM - 1) / BM), ktiles = (uint32_t)(K / BK);
     RowsPlan rp = {{0, 0, 1, 0}, false};
-    if (parts) rp = plan_rows(z.M, z.m_valid, tiles_c, gridDim.x, ktiles, WIDTHS);
+    if (parts) rp = plan_rows(z.M, z.m_valid, tiles_c, gridDim.x, ktiles, WIDTHS ? dyn.pieces : 0);
     const uint32_t height = WIDTHS && rp.fewer ? FEWER_ROWS : BN;
-    const uint32_t tiles_r = (uint32_t)(((WIDTHS && rp.fewer ? z.m_valid : z.M) + height - 1) / height);
+    const uint32_t tiles_r = WIDTHS && rp.fewer ? fewer_tiles(z.m_valid) : (uint32_t)((z.M + BN - 1) / BN);
     const uint32_t tiles = tiles_r * tiles_c;
     TailSplit ts = rp.split;
     if (!parts) ts.whole = tiles;
@@ -1918,14 +1925,14 @@ __global__ void __launch_bounds__(NTHREADS)
 // bound by reading the pieces once.
 __global__ void __launch_bounds__(NTHREADS)
     gemm_reduce_kernel(const float* __restrict__ parts, uint32_t grid, int64_t M, int64_t N, int64_t K, int mode,
-                       float* out_f32, uint16_t* out_bf16, int64_t ldo, int64_t m_valid, DynRows dyn, bool widths) {
+                       float* out_f32, uint16_t* out_bf16, int64_t ldo, int64_t m_valid, DynRows dyn) {
     __shared__ __align__(16) uint16_t stage[GROUP_F32];
     const ProductSizes z = product_sizes(M, K, m_valid, dyn);
     const StoreTo st = {mode, out_f32, out_bf16, ldo, N, z.m_valid, dyn.out_rows, dyn.scale_a, dyn.scale_b};
     const int64_t tiles_c = (N + BM - 1) / BM;
-    const RowsPlan rp = plan_rows(z.M, z.m_valid, (uint32_t)tiles_c, grid, (uint32_t)(z.K / BK), widths);
+    const RowsPlan rp = plan_rows(z.M, z.m_valid, (uint32_t)tiles_c, grid, (uint32_t)(z.K / BK), dyn.pieces);
     const TailSplit ts = rp.split;
-    const int64_t height = rp.fewer ? FEWER_ROWS : BN, tiles_r = ((rp.fewer ? z.m_valid : z.M) + height - 1) / height;
+    const int64_t height = rp.fewer ? FEWER_ROWS : BN, tiles_r = rp.fewer ? fewer_tiles(z.m_valid) : (z.M + BN - 1) / BN;
     const uint32_t tile = blockIdx.x >> 2;
     const int j = blockIdx.x & 3, tid = threadIdx.x;
     if (tile >= ts.rest || j * 2 >= (rp.fewer ? FEWER : WIDE)) return;
@@ -2254,14 +2261,10 @@ size_t split_bytes(int64_t row_tiles, int64_t h_tiles, int64_t chunk, int64_t vo
     for (int64_t c : columns) {
         const uint32_t ktiles = (uint32_t)(round_up(c, BK) / BK);
         // what is left of whole rounds repeats after `grid` row tiles
-        auto up_to = [&](int64_t rows, uint32_t per_ktile) {
-            for (int64_t r = 1; r <= rows && r <= (int64_t)grid && ktiles >= 2 * SPLIT_MIN_KTILES; ++r) {
-                const TailSplit t = plan_tail((uint32_t)(r * h_tiles), grid, ktiles, per_ktile);
-                if (t.rest * t.parts > most) most = t.rest * t.parts;
-            }
-        };
-        up_to(row_tiles, 32);
-        if (rows_come_in_widths(row_tiles)) up_to(fewer_tiles(row_tiles * BN), FEWER_COST);
+        for (int64_t r = 1; r <= row_tiles && r <= (int64_t)grid && ktiles >= 2 * SPLIT_MIN_KTILES; ++r) {
+            const TailSplit t = plan_tail((uint32_t)(r * h_tiles), grid, ktiles);
+            if (t.rest * t.parts > most) most = t.rest * t.parts;
+        }
         if (columns[0] == columns[1]) break;
     }
     return (size_t)most * PART_FLOATS * sizeof(float);
@@ -2511,21 +2514,31 @@ void enqueue_fwd(const FwdPlan& p, char* ws, const RowInputs& in, const uint8_t*
                        keep.buf ? keep.unsafe : static_cast<uint8_t*>(nullptr));
 }
 
+// scratch for pieces of tiles (none: tiles are not cut)
+struct Pieces {
+    float* at;
+    uint32_t most;
+};
+Pieces pieces_at(char* at, size_t bytes) {
+    return {bytes ? reinterpret_cast<float*>(at) : nullptr, (uint32_t)(bytes / (PART_FLOATS * sizeof(float)))};
+}
+
 // A product of token rows with W (k-contiguous x k-major, rows counted on the device): the tile kernel and,
 // where its tiles may be split along k, the addition of their pieces.
 void launch_rows_product(unsigned grid, const Operand& a, int64_t M, const Operand& b, int64_t N, int64_t K, int mode,
-                         float* out_f32, void* out_bf16, int64_t ldo, int64_t m_valid, const DynRows& dyn,
-                         uint32_t* queue, float* parts, hipStream_t s) {
+                         float* out_f32, void* out_bf16, int64_t ldo, int64_t m_valid, DynRows dyn, uint32_t* queue,
+                         const Pieces& parts, hipStream_t s) {
     uint16_t* o16 = static_cast<uint16_t*>(out_bf16);
-    const bool widths = parts && rows_come_in_widths(M / BM);
-    auto* kernel = widths ? gemm_store_kernel<false, true, true> : gemm_store_kernel<false, true, false>;
+    const bool either = parts.at && either_height(M / BM);
+    dyn.pieces = either ? parts.most : 0;
+    auto* kernel = either ? gemm_store_kernel<false, true, true> : gemm_store_kernel<false, true, false>;
     hipLaunchKernelGGL(kernel, dim3(grid), dim3(NTHREADS), 0, s, a, M, b, N, K, mode, out_f32, o16, ldo, m_valid, dyn, queue,
-                       parts);
-    if (!parts) return;
-    const int64_t tiles = (widths ? fewer_tiles(M) : M / BM) * ((N + BN - 1) / BN);
+                       parts.at);
+    if (!parts.at) return;
+    const int64_t tiles = (either ? fewer_tiles(M) : M / BM) * ((N + BN - 1) / BN);
     const int64_t most = tiles < (int64_t)grid ? tiles : (int64_t)grid - 1;  // tiles past the last whole round
-    hipLaunchKernelGGL(gemm_reduce_kernel, dim3((unsigned)(most * 4)), dim3(NTHREADS), 0, s, parts, grid, M, N, K, mode,
-                       out_f32, o16, ldo, m_valid, dyn, widths);
+    hipLaunchKernelGGL(gemm_reduce_kernel, dim3((unsigned)(most * 4)), dim3(NTHREADS), 0, s, parts.at, grid, M, N, K, mode,
+                       out_f32, o16, ldo, m_valid, dyn);
 }
 
 // The forward that also prepares d_hidden.  With x = z c in the log2 domain and a per-token
@@ -2546,7 +2559,7 @@ void enqueue_fwd_wsum(const FwdPlan& p, char* ws, const RowInputs& in, const uin
     float* zy = reinterpret_cast<float*>(ws + p.off_zy);
     uint32_t* queues = reinterpret_cast<uint32_t*>(ws + p.off_queue);
     uint16_t* chunk_buf = reinterpret_cast<uint16_t*>(ws + p.off_chunk);
-    float* parts = p.parts_bytes ? reinterpret_cast<float*>(ws + p.off_parts) : nullptr;
+    const Pieces parts = pieces_at(ws + p.off_parts, p.parts_bytes);
     const float c = inv_temperature * OI_LOG2E;
     const uint16_t* Wp = static_cast<const uint16_t*>(weight);
     const int64_t h_tiles = (hidden_dim + BN - 1) / BN;
@@ -2636,7 +2649,7 @@ void enqueue_bwd(const BwdPlan& p, char* ws, const RowInputs& in, const void* we
     };
     uint16_t* dz = reinterpret_cast<uint16_t*>(ws + p.off_dz);
     float* dh32 = reinterpret_cast<float*>(ws + p.off_dh32);
-    float* parts = p.parts_bytes ? reinterpret_cast<float*>(ws + p.off_parts) : nullptr;
+    const Pieces parts = pieces_at(ws + p.off_parts, p.parts_bytes);
     uint32_t* queues = reinterpret_cast<uint32_t*>(ws + p.off_queues);
     const uint16_t* Wp = static_cast<const uint16_t*>(weight);
     const float c = inv_temperature * OI_LOG2E;
@@ -2690,7 +2703,7 @@ void enqueue_products_from_exponentials(const uint16_t* ecache, int64_t cache_ld
                                         const int32_t* count, const int32_t* rows_s, const float* scale_a,
                                         const float* scale_b, const uint16_t* scaled_hidden, const void* weight,
                                         int64_t hidden_dim, int64_t vocab, void* d_hidden, void* d_weight,
-                                        const int32_t* dw_mode_dev, float* dw32, uint32_t* queues, float* parts,
+                                        const int32_t* dw_mode_dev, float* dw32, uint32_t* queues, const Pieces& parts,
                                         hipStream_t s) {
     const uint16_t* Wp = static_cast<const uint16_t*>(weight);
     const int64_t h_tiles = (hidden_dim + BN - 1) / BN;
@@ -2927,7 +2940,7 @@ int run_slab_passes(const SlabPlan& p, char* ws, const SlabStep& st, hipStream_t
     float* dw32 = st.d_weight && p.n_passes > 1 ? reinterpret_cast<float*>(ws + p.off_dw32) : nullptr;
     float* lse = reinterpret_cast<float*>(ws + p.off_lse);
     float* grad = reinterpret_cast<float*>(ws + p.off_grad);
-    float* parts = p.parts_bytes ? reinterpret_cast<float*>(ws + p.off_parts) : nullptr;
+    const Pieces parts = pieces_at(ws + p.off_parts, p.parts_bytes);
     const uint16_t* hid = static_cast<const uint16_t*>(st.hidden);
 
     const SlabSetup setup = {st.mask, n, p.n_pad, p.n_passes * SLAB_QUEUE_WORDS, hdim, st.logprob, st.entropy, lse,
