@@ -69,8 +69,9 @@ __device__ __forceinline__ void tile_of_item(uint32_t item, uint32_t tiles_m, ui
     *tm = band * 8 + (in_band - col * rows);
     *tn = col;
 }
-// number of ids to enumerate (whole runs for every XCD, a multiple of 256)
+// number of ids to enumerate (whole runs for every XCD, a multiple of 256), and those of an XCD that may have an item
 __host__ __device__ inline int64_t pids_for_items(int64_t items) { return (items + 255) / 256 * 256; }
+__host__ __device__ inline uint32_t locals_for_items(uint32_t items) { return items / 256 * 32 + (items % 256 + 7) / 8; }
 
 // Work queue.  A launch of the tile kernels is one workgroup per CU (the LDS ring leaves room for
 // no second one) that stays for the whole launch and draws tile ids from a counter, rather than
@@ -111,11 +112,11 @@ struct ItemQueue {
     uint32_t dry, drawn, next;
 
     // begins: the workgroups take the ids of their own numbers first
-    __device__ __forceinline__ ItemQueue(uint32_t* counters_, uint32_t items_, uint16_t* lds, bool begins)
+    __device__ __forceinline__ ItemQueue(uint32_t* counters_, uint32_t items_, uint32_t locals_, uint16_t* lds, bool begins)
         : counters(counters_),
           mailbox(reinterpret_cast<volatile uint32_t*>(lds + 4 * BM * BK)),
           items(items_),
-          locals((uint32_t)(pids_for_items(items_) >> 3)),  // ids per queue
+          locals(locals_),  // ids per queue
           xcd(blockIdx.x & 7),
           begun(begins ? gridDim.x >> 3 : 0),
           dry(counters_ ? 0 : 8),  // without counters there is nothing to draw
@@ -173,10 +174,10 @@ struct ItemQueue {
 // begins: these are the kernel's first items.  (Items that are to fill the end of others' launch time must be drawn: a
 // workgroup that is late would have its own left to do.)
 template <class Body>
-__device__ __forceinline__ void for_each_item(uint32_t* __restrict__ counters, uint32_t items, uint16_t* lds, bool begins,
-                                              Body&& body) {
-    if (items == 0) return;
-    ItemQueue queue(counters, items, lds, begins);
+__device__ __forceinline__ void for_each_id(uint32_t* __restrict__ counters, uint32_t locals, uint16_t* lds, bool begins,
+                                            Body&& body) {
+    if (locals == 0) return;
+    ItemQueue queue(counters, 0, locals, lds, begins);
     uint32_t pid = blockIdx.x;
     if (!begins) {
         queue.request();
@@ -185,8 +186,7 @@ __device__ __forceinline__ void for_each_item(uint32_t* __restrict__ counters, u
     }
     while (pid != ItemQueue::NONE) {
         queue.request();
-        const uint32_t item = item_of_pid(pid, items);
-        if (item < items) body(item);
+        body(pid);
         queue.settle();
         pid = queue.take();
     }
@@ -194,7 +194,10 @@ __device__ __forceinline__ void for_each_item(uint32_t* __restrict__ counters, u
 template <class Body>
 __device__ __forceinline__ void for_each_tile(uint32_t* __restrict__ counters, int64_t tiles_m, int64_t tiles_n,
                                               uint16_t* lds, Body&& body, bool begins = true) {
-    for_each_item(counters, (uint32_t)(tiles_m * tiles_n), lds, begins, [&](uint32_t item) {
+    const uint32_t items = (uint32_t)(tiles_m * tiles_n);
+    for_each_id(counters, locals_for_items(items), lds, begins, [&](uint32_t pid) {
+        const uint32_t item = item_of_pid(pid, items);
+        if (item >= items) return;
         int64_t tm, tn;
         tile_of_item(item, (uint32_t)tiles_m, (uint32_t)tiles_n, &tm, &tn);
         body(tm, tn);
@@ -615,8 +618,8 @@ __device__ __forceinline__ int acc_col(int wn, int j, int lane) { return wn * 16
 // of rows there is little to be shared (300 x 8192 874, 851).  `rows` is all that the call has, selected or not: a
 // choice on the device keeps the other widths' code in every call's kernel (2940 x 8192 0.5 % longer for it).
 //
-// The products behind it have whole tiles only: among them narrow ones gain nothing, as the pieces that tiles are cut
-// into stop being alike (d_hidden of 268 rows 312, so 322).
+// The products behind it have tiles of one height only (plan_rows): among whole ones narrow ones gain nothing, as the
+// pieces that tiles are cut into stop being alike (d_hidden of 268 rows 312, so 322).
 inline bool narrow_tiles(int64_t rows, int64_t hdim) { return rows <= 2 * BN || (rows <= 16 * BN && hdim <= 6144); }
 // What a narrow tile leaves in memory ends with it.  d_weight's k-tiles, the only reader of rows past the last one, do so
 // at the same row or before.
@@ -626,7 +629,8 @@ __device__ __forceinline__ int tile_width(int64_t rows, int64_t row0, bool narro
     if (!narrow || left > 192) return WIDE;
     return left > 128 ? 6 : left > 64 ? 4 : 2;
 }
-// What a call has of token rows: up to one tile (narrow too), tiles of which the last may be narrow, whole tiles.
+// What a call has of token rows: up to one tile (narrow too), tiles of which the last may be narrow, whole tiles.  As a
+// forward kernel, NARROW_LAST is the one that has code for all widths (fwd_tiles).
 enum RowTiles { ONE_TILE, NARROW_LAST, WHOLE_TILES };
 inline RowTiles row_tiles(int64_t rows, int64_t hdim) {
     return rows <= BN ? ONE_TILE : narrow_tiles(rows, hdim) ? NARROW_LAST : WHOLE_TILES;
@@ -796,6 +800,7 @@ struct FwdLaunch {
     const float* xref;  // per token: the exponent that the kept exponentials are relative to (null: 0)
     float* logits;
     int64_t logits_tiles;
+    bool narrow, either;  // the last tile of rows may be narrow; tiles may have either height (see FwdTiles)
 };
 enum FwdKeep { FWD_PLAIN, FWD_EXPONENTIALS, FWD_LOGITS };
 
@@ -902,7 +907,7 @@ __device__ __forceinline__ float4 fwd_merge_waves(const float* red, int columns,
 }
 
 template <FwdKeep KEEP, Walk WALK, int NJ>
-__device__ __forceinline__ void lmhead_fwd_item(const FwdArgs& a, const FwdLaunch& fl, int64_t split, int64_t tt,
+__device__ __forceinline__ void lmhead_fwd_item(const FwdArgs& a, const FwdLaunch& fl, int64_t split, int64_t tt, int64_t n0,
                                                 uint16_t* lds) {
     const int64_t vocab_tiles = (a.vocab + BM - 1) / BM;
     // the first long_splits splits take tiles_per_split vocabulary tiles each, the others one
@@ -913,7 +918,6 @@ __device__ __forceinline__ void lmhead_fwd_item(const FwdArgs& a, const FwdLaunc
     vt_end = vt_end < vocab_tiles ? vt_end : vocab_tiles;
 
     const int tid = opaque_tid(), lane = tid & 63, wave = tid >> 6, wm = wave & 3, wn = wave >> 2;
-    const int64_t n0 = tt * BN;
     const Operand tokens = {a.hidden, a.hdim, n0, a.n_tokens, a.hdim};
     Operand rows = {a.W, a.hdim, vt_begin * BM, a.vocab, a.hdim};
 
@@ -957,24 +961,92 @@ __device__ __forceinline__ void lmhead_fwd_item(const FwdArgs& a, const FwdLaunc
     if (tid < COLUMNS && n0 + tid < a.n_tokens) a.partial[split * a.n_pad + n0 + tid] = fwd_merge_waves(red, COLUMNS, tid);
 }
 
+// Calls of up to 8 tiles of rows may cut them into tiles of 256 or of 192 rows.
+inline bool either_height(int64_t row_tiles) { return row_tiles <= 8; }
+// How a forward of up to 8 tiles of rows cuts them.  A narrow tile among whole ones does not keep step with them, so W's
+// k-tiles come from memory for it once more; tiles that all have 192 rows do.  And a last round that only some workgroups
+// have a tile for is as long as any: where few have, its vocabulary tiles are handed out in tiles of 128 rows, which
+// take about half the time (an XCD's worth of tiles of 4096 with nothing else running: 256 rows 78 us, 192 62, 128 48, 64
+// 50: below 128 the loop waits for its loads).  The estimate takes what its parts take, in 32nds of a whole tile in a
+// full chip.  us before and after: 4096 x 100352 268 rows 335, 312; 384 330, 318; 512 397, 366; 520 471, 424; 1300 893, 865;
+// 4096 x 128256 268 rows 389, 341; 576 569, 542; 8192 x 128256 268 rows 746, 660; 520 1145, 961; 3584 x 151665 384 rows 430,
+// 400.  In alike tiles but without cutting the last round 384 rows take 348 (4096 x 100352, 3.06 rounds).  Where the
+// estimate stays with whole tiles nothing changes (700 rows 494, 492).  The logits that a forward keeps for its backward lie
+// in whole tiles; it takes none of this.
+struct FwdTiles {
+    int height;         // rows of a tile
+    uint32_t row_tiles;
+    uint32_t tail, tail_row_tiles;  // the last `tail` of the short splits come in tiles of TAIL_ROWS
+};
+constexpr int FEWER = 6, FEWER_ROWS = 32 * FEWER, TAIL = 4, TAIL_ROWS = 32 * TAIL;
+__host__ __device__ inline uint32_t fewer_tiles(int64_t rows) { return (uint32_t)((rows + FEWER_ROWS - 1) / FEWER_ROWS); }
+__device__ __forceinline__ FwdTiles fwd_tiles(int64_t rows, uint32_t vocab_tiles, uint32_t short_splits, bool narrow) {
+    // what tiles of the widths 8, 6 and less take, in 32nds of a whole one's time, and what a narrow one among whole
+    // ones costs the others, which read the same k-tiles of W
+    constexpr uint32_t WHOLE_COST = 32, FEWER_COST = 26, TAIL_COST = 18, APART = 8;
+    FwdTiles t = {BN, (uint32_t)((rows + BN - 1) / BN), 0, 0};
+    if (t.row_tiles == 0) return t;
+    const int last = tile_width(rows, (int64_t)(t.row_tiles - 1) * BN, narrow);
+    uint32_t cost = t.row_tiles * WHOLE_COST;
+    if (last != WIDE) cost += (last == FEWER ? FEWER_COST : TAIL_COST) - WHOLE_COST + (t.row_tiles > 1 ? APART : 0);
+    uint32_t one = last == WIDE ? WHOLE_COST : 0;
+    // no rows past those of whole tiles, which is what the buffers hold
+    if (fewer_tiles(rows) * FEWER_COST < cost && fewer_tiles(rows) * FEWER_ROWS <= t.row_tiles * BN) {
+        one = FEWER_COST;
+        t.height = FEWER_ROWS;
+        t.row_tiles = fewer_tiles(rows);
+    }
+    const uint32_t rest = vocab_tiles * t.row_tiles % gridDim.x, tail = (rest + t.row_tiles - 1) / t.row_tiles;
+    const uint32_t tail_row_tiles = (uint32_t)((rows + TAIL_ROWS - 1) / TAIL_ROWS);
+    const uint32_t rounds = (tail * tail_row_tiles + gridDim.x - 1) / gridDim.x;
+    if (tail <= short_splits && rounds * TAIL_COST < one) {
+        t.tail = tail;
+        t.tail_row_tiles = tail_row_tiles;
+    }
+    return t;
+}
+
 template <FwdKeep KEEP, RowTiles TILES>
 __global__ void __launch_bounds__(NTHREADS)
     lmhead_fwd_kernel(FwdArgs a, const int32_t* __restrict__ n_dev, FwdLaunch fl, uint32_t* __restrict__ queue) {
     __shared__ __align__(16) uint16_t lds[LDS_ELEMS];
     if (n_dev) a.n_tokens = device_count(n_dev);  // rows selected on the device: the host only knows an upper bound
-    const int64_t token_tiles = (a.n_tokens + BN - 1) / BN;
+    FwdTiles ft = {BN, (uint32_t)((a.n_tokens + BN - 1) / BN), 0, 0};
+    if (TILES == NARROW_LAST && KEEP != FWD_LOGITS && fl.either)
+        ft = fwd_tiles(a.n_tokens, (uint32_t)(fl.n_first * fl.tiles_per_split + fl.n_second), (uint32_t)fl.n_second, fl.narrow);
     // every long item of every XCD's queue is taken before the first short one: the short items are
     // there to fill the end of the launch
 #pragma unroll 1
     for (int pass = 0; pass < 2; ++pass) {
         const int64_t first = pass ? fl.long_splits : fl.first, splits = pass ? fl.n_second : fl.n_first;
-        for_each_tile(queue + pass * QUEUE_WORDS, splits, token_tiles, lds, [&](int64_t split, int64_t tt) {
+        const uint32_t tail = pass ? ft.tail : 0, head = (uint32_t)splits - tail;
+        const uint32_t items = head * ft.row_tiles, tail_items = tail * ft.tail_row_tiles;
+        const uint32_t locals = locals_for_items(items);
+        for_each_id(queue + pass * QUEUE_WORDS, locals + locals_for_items(tail_items), lds, pass == 0 || fl.n_first == 0,
+                    [&](uint32_t pid) {
+            int64_t split, tt, n0;
+            int width = WIDE;
+            if (TILES == NARROW_LAST && pid >= locals * 8) {
+                const uint32_t item = item_of_pid(pid - locals * 8, tail_items);
+                if (item >= tail_items) return;
+                tile_of_item(item, tail, ft.tail_row_tiles, &split, &tt);
+                split += head;
+                n0 = tt * TAIL_ROWS;
+                width = TAIL;
+            } else {
+                const uint32_t item = item_of_pid(pid, items);
+                if (item >= items) return;
+                tile_of_item(item, head, ft.row_tiles, &split, &tt);
+                n0 = tt * ft.height;
+                if (TILES == NARROW_LAST && ft.height != BN) width = FEWER;
+                else if (TILES != WHOLE_TILES) width = tile_width(a.n_tokens, n0, fl.narrow);
+            }
             auto item = [&](auto nj) {
-                lmhead_fwd_item<KEEP, TILES == ONE_TILE ? ROUND : NEAR, decltype(nj)::value>(a, fl, first + split, tt, lds);
+                lmhead_fwd_item<KEEP, TILES == ONE_TILE ? ROUND : NEAR, decltype(nj)::value>(a, fl, first + split, tt, n0, lds);
             };
-            if constexpr (TILES != WHOLE_TILES) with_width(tile_width(a.n_tokens, tt * BN, true), item);
+            if constexpr (TILES != WHOLE_TILES) with_width(width, item);
             else item(std::integral_constant<int, WIDE>{});
-        }, pass == 0 || fl.n_first == 0);
+        });
     }
 }
 
@@ -1536,10 +1608,7 @@ __host__ __device__ inline TailSplit plan_tail(uint32_t tiles, uint32_t grid, ui
 // 4096 x 100352 268 rows 295, 235; 384 299, 246; 520 448, 365; 1152 743, 735; 8192 x 128256 268 rows 728, 596; 520 1109, 898;
 // 3584 x 151665 268 rows 426, 347; 2048 x 151936 268 rows 266, 211.  Counts in between stay with 256 (4096 x 100352 400
 // rows 294, 600 441).  Kernels of calls with more than 8 tiles of rows have no code for it: their gain would be 6 % at most.
-constexpr int FEWER = 6;
-constexpr uint32_t FEWER_COST = 26, FEWER_ROWS = 32 * FEWER;
-inline bool either_height(int64_t row_tiles) { return row_tiles <= 8; }
-__host__ __device__ inline uint32_t fewer_tiles(int64_t rows) { return (uint32_t)((rows + FEWER_ROWS - 1) / FEWER_ROWS); }
+constexpr uint32_t FEWER_COST = 26;
 struct RowsPlan {
     TailSplit split;
     bool fewer;
@@ -1636,7 +1705,10 @@ __global__ void __launch_bounds__(NTHREADS)
     // The fp32 modes need more LDS than one slot and belong to batches of several slabs, whose tiles are long.
     const bool ahead = mode == 2 && pieces;
     if (tiles == 0) return;
-    ItemQueue q(queue, ts.whole + ts.rest * ts.parts, lds, true);
+    const uint32_t items = ts.whole + ts.rest * ts.parts;
+    // ids without an item among them: the exact number changes the main loop's code, and large d_hidden products take 1.2 %
+    // longer (2950 rows x 8192 4388 us, 4448)
+    ItemQueue q(queue, items, (uint32_t)(pids_for_items(items) >> 3), lds, true);
     uint32_t item = item_of_pid(blockIdx.x, q.items);
     if (item >= q.items && queue) {  // an id without an item
         q.request();
@@ -2475,11 +2547,10 @@ void launch_label_ref(const RowInputs& in, const void* weight, int64_t n_tokens,
 }
 
 template <FwdKeep KEEP>
-auto fwd_kernel(int64_t n_tokens, int64_t hidden_dim) {
-    const RowTiles tiles = row_tiles(n_tokens, hidden_dim);
-    return tiles == ONE_TILE      ? lmhead_fwd_kernel<KEEP, ONE_TILE>
-           : tiles == NARROW_LAST ? lmhead_fwd_kernel<KEEP, NARROW_LAST>
-                                  : lmhead_fwd_kernel<KEEP, WHOLE_TILES>;
+auto fwd_kernel(int64_t n_tokens, const FwdLaunch& fl) {
+    return n_tokens <= BN            ? lmhead_fwd_kernel<KEEP, ONE_TILE>
+           : fl.narrow || fl.either ? lmhead_fwd_kernel<KEEP, NARROW_LAST>
+                                    : lmhead_fwd_kernel<KEEP, WHOLE_TILES>;
 }
 
 // forward launches: tile kernel + merge of the partial statistics.  `queue` must be zeroed.
@@ -2495,9 +2566,10 @@ void enqueue_fwd(const FwdPlan& p, char* ws, const RowInputs& in, const uint8_t*
     const FwdArgs fa = {static_cast<const uint16_t*>(weight), in.hidden, in.labels, n_tokens, hidden_dim, vocab, c,
                         p.n_pad, partial, zy};
     const FwdLaunch fl = {p.tiles_per_split, p.long_splits, 0, p.long_splits, p.n_splits - p.long_splits,
-                          keep.buf, keep.ld, 0, keep.buf ? keep.tiles : 0, 0, keep.xref, keep.logits, p.token_tiles};
+                          keep.buf, keep.ld, 0, keep.buf ? keep.tiles : 0, 0, keep.xref, keep.logits, p.token_tiles,
+                          row_tiles(n_tokens, hidden_dim) != WHOLE_TILES, !keep.logits && either_height(p.token_tiles)};
     auto launch = [&](auto keep_as) {
-        hipLaunchKernelGGL(fwd_kernel<decltype(keep_as)::value>(n_tokens, hidden_dim), grid, dim3(NTHREADS), 0, s, fa, in.n_dev,
+        hipLaunchKernelGGL(fwd_kernel<decltype(keep_as)::value>(n_tokens, fl), grid, dim3(NTHREADS), 0, s, fa, in.n_dev,
                            fl, queue);
     };
     if (keep.buf) {
@@ -2576,8 +2648,9 @@ void enqueue_fwd_wsum(const FwdPlan& p, char* ws, const RowInputs& in, const uin
         const int64_t n_first = p.n_splits - first < splits_per_chunk ? p.n_splits - first : splits_per_chunk;
         uint32_t* q = queues + ci * (FWD_QUEUE_WORDS + QUEUE_WORDS);
         const FwdLaunch fl = {p.tiles_per_split, p.long_splits, first, n_first, 0, chunk_buf, cols, v_begin / BM,
-                              cols / BM, 1, xref, nullptr, 0};
-        hipLaunchKernelGGL(fwd_kernel<FWD_EXPONENTIALS>(n_tokens, hidden_dim),
+                              cols / BM, 1, xref, nullptr, 0, row_tiles(n_tokens, hidden_dim) != WHOLE_TILES,
+                              either_height(p.token_tiles)};
+        hipLaunchKernelGGL(fwd_kernel<FWD_EXPONENTIALS>(n_tokens, fl),
                            dim3(resident_grid(n_first, p.token_tiles)), dim3(NTHREADS), 0, s, fa,
                            in.n_dev, fl, q);
         const Operand a = {chunk_buf, cols, 0, p.n_pad, cols};

@@ -385,6 +385,46 @@ def test_selected_rows_in_tiles_of_either_height(count, h, want_dw):
         assert ((dw.grad.float().cpu() - rw.grad).norm() / rw.grad.norm()).item() <= 2e-2
 
 
+@pytest.mark.parametrize(
+    "rows,vocab",
+    [
+        (257, 33024),  # two tiles of 192, 258 tiles in all: the last vocabulary tile in tiles of 128
+        (384, 35000),  # 274 tiles: the last nine
+        (385, 33000),  # 256 and a narrow one
+        (512, 33000),  # two of 256, the last vocabulary tile in tiles of 128
+        (513, 35000),  # three of 192, no last round worth cutting
+        (576, 22000),  # three of 192, 258 tiles
+        (961, 3000),  # one round that is all last
+        (1281, 33000),  # seven of 192
+    ],
+)  # fmt: skip
+def test_forward_in_tiles_of_either_height(rows, vocab):
+    """Scores, and the step that leaves its exponentials to both products, at row counts on both sides of where the
+    forward changes the height of its tiles, with and without a last round in lower ones."""
+    h = 64
+    hidden, weight, labels = _case(rows + 1, h, vocab, seed=27, w_scale=3.0 / math.sqrt(h))
+    labels[-1], labels[1] = vocab - 1, 0
+    exp_lp, exp_ent = o_lm.lm_head_logprobs(hidden[:rows], weight, labels[1:], 0.9, True)
+    with torch.no_grad():
+        lp, ent = lm_head.fused_lm_head_logprobs(
+            hidden[:rows].to(DEV), weight.to(DEV), labels[1:].to(DEV), 0.9, return_entropy=True
+        )
+    assert (lp.cpu() - exp_lp).abs().max().item() <= TOL
+    assert (ent.cpu() - exp_ent).abs().max().item() <= TOL
+    rh = hidden.float().requires_grad_(True)
+    rw = weight.float().requires_grad_(True)
+    exp = o_lm.linear_cross_entropy(rh[None], rw, labels[None])
+    exp.backward()
+    dh = hidden[None].to(DEV).requires_grad_(True)
+    dw = weight.to(DEV).requires_grad_(True)
+    got = lm_head.fused_linear_cross_entropy(dh, dw, labels[None].to(DEV), token_slabs=True)
+    got.backward()
+    assert abs(got.item() - exp.item()) <= TOL
+    worst = (dh.grad[0, :rows].float().cpu() - rh.grad[:rows]).norm(dim=1) / rh.grad[:rows].norm(dim=1)
+    assert worst.max().item() <= 2e-2
+    assert ((dw.grad.float().cpu() - rw.grad).norm() / rw.grad.norm()).item() <= 2e-2
+
+
 def test_row_selection_with_compact_backward_and_mask():
     """Mask and zero-gradient rows together: the backward selects rows that are in the mask AND carry
     a gradient."""
