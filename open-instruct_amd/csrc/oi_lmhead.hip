@@ -2172,6 +2172,135 @@ __global__ void __launch_bounds__(256)
     if (lane == 0) xref[j] = acc * c;
 }
 
+// Selection without a launch of its own.  Of up to SELECT_AT_ONCE rows every workgroup counts the mask's bytes in front of
+// its rows for itself (8 of a lane at a time, from L2), which tells where those go; it then does what was to be done with
+// them, a wave for each row.  A launch that only makes the row index, and another one each for what goes by it, take 4.6 us
+// of a busy stream whatever they do, and one workgroup takes 18 us for the index of 32768 rows.  Rows selected, gathered and
+// marked, and those left out cleared: 2 launches, 4 with the reference exponents, before; 435 rows x 4096, four 19 us, one
+// 6; 2950 rows x 8192, four 48, one 21.
+constexpr int64_t SELECT_AT_ONCE = 65536;
+constexpr int AT_ONCE_WAVES = 4, AT_ONCE_THREADS = AT_ONCE_WAVES * OI_WAVE;
+// rows of a wave: more where there are many workgroups anyway, so that the mask is not read by too many
+inline int rows_per_wave(int64_t n) { return n > 16384 ? 4 : 1; }
+inline unsigned at_once_grid(int64_t n) {
+    const int64_t rows = AT_ONCE_WAVES * rows_per_wave(n);
+    return (unsigned)((n + rows - 1) / rows);
+}
+__device__ __forceinline__ int nonzero_bytes(uint64_t x) {
+    constexpr uint64_t low = 0x7f7f7f7f7f7f7f7full;
+    return __popcll((((x & low) + low) | x) & ~low);
+}
+// selected rows among [0, b), for every thread of the workgroup
+__device__ __forceinline__ int rows_before(const uint8_t* __restrict__ mask, int64_t b) {
+    const int tid = threadIdx.x;
+    const int64_t to_word = (8 - (reinterpret_cast<uintptr_t>(mask) & 7)) & 7, head = to_word < b ? to_word : b;
+    const int64_t words = (b - head) / 8, tail = head + words * 8;
+    const uint64_t* w = reinterpret_cast<const uint64_t*>(mask + head);
+    int c = 0;
+#pragma unroll 4
+    for (int64_t i = tid; i < words; i += AT_ONCE_THREADS) c += nonzero_bytes(w[i]);
+    if (tid < head) c += mask[tid] != 0;
+    if (tail + tid < b) c += mask[tail + tid] != 0;
+    __shared__ int sum[AT_ONCE_WAVES];
+#pragma unroll
+    for (int d = 32; d > 0; d >>= 1) c += __shfl_xor(c, d, OI_WAVE);
+    if ((tid & 63) == 0) sum[tid >> 6] = c;
+    __syncthreads();
+    int total = 0;
+#pragma unroll
+    for (int k = 0; k < AT_ONCE_WAVES; ++k) total += sum[k];
+    return total;
+}
+// each(row, selected, rank among the selected) for the wave's rows; last(count) for the workgroup that has the last row.
+// Without a mask every row is selected.
+template <class Each, class Last>
+__device__ __forceinline__ void for_selected_rows(const uint8_t* __restrict__ mask, int64_t n, int per_wave, Each&& each,
+                                                  Last&& last) {
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int of_group = AT_ONCE_WAVES * per_wave;  // at most 64
+    const int64_t b = (int64_t)blockIdx.x * of_group;
+    uint64_t set = ~0ull;
+    if (mask) set = __ballot(lane < of_group && b + lane < n && mask[b + lane] != 0);
+    const int before = mask ? rows_before(mask, b) : (int)b;
+#pragma unroll 1
+    for (int k = 0; k < per_wave; ++k) {
+        const int at = wave * per_wave + k;
+        if (b + at >= n) return;
+        const int rank = before + __popcll(set & ((1ull << at) - 1));
+        const bool selected = set >> at & 1;
+        each(b + at, selected, (int64_t)rank);
+        if (b + at == n - 1) last(rank + (selected ? 1 : 0));
+    }
+}
+// What is gathered, and on the way: `zero_words` cleared; with `xref`, the reference exponents (as label_ref_kernel);
+// with `clear`, a byte of every row, selected or not; with `zero_rows`, its rows that were not selected.
+struct GatherRows {
+    const uint16_t* hidden;
+    const int64_t* labels;
+    const float *lse, *grad, *logprob;
+    int64_t hdim;
+    int32_t *rows, *count;
+    uint16_t* hidden_c;
+    int64_t* labels_c;
+    float *lse_c, *grad_c, *logprob_c;
+    uint32_t* zero_words;
+    int n_zero;
+    const uint16_t* W;
+    int64_t vocab;
+    float c;
+    float* xref;
+    uint8_t* clear;
+    uint16_t* zero_rows;
+};
+__global__ void __launch_bounds__(AT_ONCE_THREADS)
+    select_gather_kernel(const uint8_t* __restrict__ mask, int64_t n, int per_wave, GatherRows g) {
+    const int lane = threadIdx.x & 63;
+    if (blockIdx.x == 0)
+        for (int i = threadIdx.x; i < g.n_zero; i += AT_ONCE_THREADS) g.zero_words[i] = 0u;
+    for_selected_rows(
+        mask, n, per_wave,
+        [&](int64_t src, bool selected, int64_t j) {
+            if (g.clear && lane == 0) g.clear[src] = 0;
+            if (!selected) {
+                if (!g.zero_rows) return;
+                uint16_t* row = g.zero_rows + src * g.hdim;  // hdim is a multiple of 64; rows may lie on 4-byte boundaries
+                if ((reinterpret_cast<uintptr_t>(row) & 15) == 0)
+                    for (int64_t p = lane; p < g.hdim / 8; p += OI_WAVE) reinterpret_cast<oi_u32x4*>(row)[p] = oi_u32x4{0u, 0u, 0u, 0u};
+                else
+                    for (int64_t p = lane; p < g.hdim / 2; p += OI_WAVE) reinterpret_cast<uint32_t*>(row)[p] = 0u;
+                return;
+            }
+            const int64_t label = g.labels[src];
+            const oi_u32x4* from = reinterpret_cast<const oi_u32x4*>(g.hidden + src * g.hdim);
+            oi_u32x4* to = reinterpret_cast<oi_u32x4*>(g.hidden_c + j * g.hdim);
+            if (g.xref) {
+                const int64_t y = label < 0 ? 0 : (label >= g.vocab ? g.vocab - 1 : label);
+                const oi_u32x4* wy = reinterpret_cast<const oi_u32x4*>(g.W + y * g.hdim);
+                float acc = 0.f;
+#pragma unroll 8
+                for (int64_t p = lane; p < g.hdim / 8; p += OI_WAVE) {
+                    const oi_u32x4 a = from[p], b = wy[p];
+                    to[p] = a;
+                    acc = dot_bf16x8(a, b, acc);
+                }
+                acc = oi_wave_sum(acc);
+                if (lane == 0) g.xref[j] = acc * g.c;
+            } else {
+#pragma unroll 8
+                for (int64_t p = lane; p < g.hdim / 8; p += OI_WAVE) to[p] = from[p];
+            }
+            if (lane != 0) return;
+            g.rows[j] = (int32_t)src;
+            g.labels_c[j] = label;
+            if (g.lse_c) g.lse_c[j] = g.lse[src];
+            if (g.grad_c) g.grad_c[j] = g.grad[src];
+            if (g.logprob_c) g.logprob_c[j] = g.logprob[src];
+        },
+        [&](int count) {
+            if (lane == 0) *g.count = count;
+        });
+}
+
 // Which rows a slab pass works on: rows order[offset .. offset + count) of a row index that lives
 // on the device.  Written by a planning kernel, read by every kernel of the pass.
 struct SlabMeta {
@@ -2505,11 +2634,21 @@ struct RowInputs {
     const float* logprob;         // the forward's result: the label's entry of dZ is rebuilt from it
 };
 
+// What else a selection does for its rows, all optional: reference exponents of the selected ones (weight, c, xref), a byte
+// of every row cleared, rows of a result that were not selected zeroed.
+struct SelectionExtras {
+    const void* weight;
+    int64_t vocab;
+    float c;
+    float* xref;
+    uint8_t* clear;
+    void* zero_rows;
+};
 // select + gather on `s`; clears `n_zero` queue words on the way
 RowInputs launch_selection(const SelectionPlan& sp, char* ws, const void* hidden, const int64_t* labels,
                            const float* lse, const float* grad, const uint8_t* row_mask, bool skip_zero_grad,
                            int64_t n_tokens, int64_t hdim, uint32_t* zero_words, int n_zero, hipStream_t s,
-                           const float* logprob = nullptr) {
+                           const float* logprob = nullptr, const SelectionExtras& extra = {}) {
     int32_t* rows = reinterpret_cast<int32_t*>(ws + sp.off_rows);
     int32_t* count = reinterpret_cast<int32_t*>(ws + sp.off_count);
     uint16_t* hidden_c = reinterpret_cast<uint16_t*>(ws + sp.off_hidden);
@@ -2517,13 +2656,33 @@ RowInputs launch_selection(const SelectionPlan& sp, char* ws, const void* hidden
     float* lse_c = lse ? reinterpret_cast<float*>(ws + sp.off_lse) : nullptr;
     float* grad_c = grad ? reinterpret_cast<float*>(ws + sp.off_grad) : nullptr;
     float* logprob_c = logprob ? reinterpret_cast<float*>(ws + sp.off_logprob) : nullptr;
-    hipLaunchKernelGGL(select_rows_kernel, dim3(1), dim3(SELECT_THREADS), 0, s, row_mask,
-                       skip_zero_grad ? grad : static_cast<const float*>(nullptr), n_tokens, rows, count, zero_words,
-                       n_zero);
+    const RowInputs in = {hidden_c, labels_c, lse_c, grad_c, rows, count, logprob_c};
+    // rows that a gradient of 0 leaves out have four more bytes each to be counted by everyone
+    if (n_tokens <= SELECT_AT_ONCE && !skip_zero_grad) {
+        const GatherRows g = {static_cast<const uint16_t*>(hidden), labels, lse, grad, logprob, hdim, rows, count, hidden_c,
+                              labels_c, lse_c, grad_c, logprob_c, zero_words, n_zero,
+                              static_cast<const uint16_t*>(extra.weight), extra.vocab, extra.c, extra.xref, extra.clear,
+                              static_cast<uint16_t*>(extra.zero_rows)};
+        hipLaunchKernelGGL(select_gather_kernel, dim3(at_once_grid(n_tokens)), dim3(AT_ONCE_THREADS), 0, s, row_mask, n_tokens,
+                           rows_per_wave(n_tokens), g);
+        return in;
+    }
+    const float* zero_grads = skip_zero_grad ? grad : nullptr;
+    hipLaunchKernelGGL(select_rows_kernel, dim3(1), dim3(SELECT_THREADS), 0, s, row_mask, zero_grads, n_tokens, rows, count,
+                       zero_words, n_zero);
     hipLaunchKernelGGL(gather_rows_kernel, dim3((unsigned)n_tokens), dim3(256), 0, s,
                        static_cast<const uint16_t*>(hidden), labels, lse, grad, logprob, rows, count, hdim, hidden_c,
                        labels_c, lse_c, grad_c, logprob_c);
-    return RowInputs{hidden_c, labels_c, lse_c, grad_c, rows, count, logprob_c};
+    if (extra.clear)
+        hipLaunchKernelGGL(zero_bytes_kernel, dim3((unsigned)((n_tokens + 255) / 256)), dim3(256), 0, s, extra.clear, n_tokens);
+    if (extra.xref)
+        hipLaunchKernelGGL(label_ref_kernel, dim3((unsigned)((n_tokens + 3) / 4)), dim3(256), 0, s, in.hidden,
+                           static_cast<const uint16_t*>(extra.weight), in.labels, in.n_dev, n_tokens, hdim, extra.vocab, extra.c,
+                           extra.xref);
+    if (extra.zero_rows)
+        hipLaunchKernelGGL(zero_unselected_rows_kernel, dim3((unsigned)n_tokens), dim3(256), 0, s, row_mask, zero_grads, hdim,
+                           static_cast<uint16_t*>(extra.zero_rows));
+    return in;
 }
 
 // lse, upstream gradient and logprob of the selected rows (the rows were selected and gathered earlier)
@@ -2537,13 +2696,6 @@ __global__ void gather_f32_kernel(const float* __restrict__ lse, const float* __
     lse_c[j] = lse[src];
     grad_c[j] = grad[src];
     logprob_c[j] = logprob[src];
-}
-
-void launch_label_ref(const RowInputs& in, const void* weight, int64_t n_tokens, int64_t hidden_dim, int64_t vocab,
-                      float inv_temperature, float* xref, hipStream_t s) {
-    hipLaunchKernelGGL(label_ref_kernel, dim3((unsigned)((n_tokens + 3) / 4)), dim3(256), 0, s, in.hidden,
-                       static_cast<const uint16_t*>(weight), in.labels, in.n_dev, n_tokens, hidden_dim, vocab,
-                       inv_temperature * OI_LOG2E, xref);
 }
 
 template <FwdKeep KEEP>
@@ -2638,7 +2790,6 @@ void enqueue_fwd_wsum(const FwdPlan& p, char* ws, const RowInputs& in, const uin
     const int64_t v_pad = p.vocab_tiles * BM;
     const int64_t splits_per_chunk = (p.chunk / BM + p.tiles_per_split - 1) / p.tiles_per_split;
     const FwdArgs fa = {Wp, in.hidden, in.labels, n_tokens, hidden_dim, vocab, c, p.n_pad, partial, zy};
-    launch_label_ref(in, weight, n_tokens, hidden_dim, vocab, inv_temperature, xref, s);
     for (int64_t ci = 0; ci < p.n_chunks; ++ci) {
         const int64_t v_begin = ci * p.chunk;
         const int64_t v_end = v_begin + p.chunk < v_pad ? v_begin + p.chunk : v_pad;
@@ -2665,37 +2816,54 @@ void enqueue_fwd_wsum(const FwdPlan& p, char* ws, const RowInputs& in, const uin
                        entropy, lse, static_cast<const float*>(xref), unsafe);
 }
 
-// d_hidden row of selected token j (caller row rows[j], or j without a selection) from the weighted
-// sum that the forward left behind; one workgroup per selected row.  The factor s is applied in two
-// halves so that neither leaves the fp32 range.  Rows flagged in `unsafe` are left alone (the
-// recomputing backward writes them).
-__global__ void __launch_bounds__(256)
-    dh_from_wsum_kernel(const float* __restrict__ wsum, const float* __restrict__ xref,
-                        const uint8_t* __restrict__ unsafe, const uint16_t* __restrict__ W,
-                        const int64_t* __restrict__ labels, const float* __restrict__ lse,
-                        const float* __restrict__ logprob, const float* __restrict__ grad,
-                        const int32_t* __restrict__ rows, const int32_t* __restrict__ count, int64_t n_tokens,
-                        int64_t hdim, int64_t vocab, float inv_t, uint16_t* __restrict__ d_hidden) {
-    const int64_t j = blockIdx.x;
-    if (j >= (count ? (int64_t)*count : n_tokens)) return;
-    const int64_t n = rows ? (int64_t)rows[j] : j;
-    if (unsafe[n]) return;
-    const float g = grad[n] * inv_t;
-    const float half = __builtin_amdgcn_exp2f(0.5f * (xref[j] - lse[n] * OI_LOG2E));
+// d_hidden row of token n from the weighted sum that the forward left behind for it, row j among the selected; zero where it
+// was not selected.  A wave for each row.  The factor s is applied in two halves so that neither leaves the fp32 range.
+// Rows flagged in `unsafe` are left alone (the recomputing backward writes them).
+struct WsumInputs {
+    const float *wsum, *xref;
+    const uint8_t* unsafe;
+    const uint16_t* W;
+    const int64_t* labels;
+    const float *lse, *logprob, *grad;
+    int64_t hdim, vocab;
+    float inv_t;
+    uint16_t* d_hidden;
+};
+__device__ __forceinline__ void dh_row_from_wsum(const WsumInputs& a, int64_t n, bool selected, int64_t j) {
+    const int lane = threadIdx.x & 63;
+    uint2* dst = reinterpret_cast<uint2*>(a.d_hidden + n * a.hdim);
+    if (!selected) {
+        for (int64_t c = lane; c < a.hdim / 4; c += OI_WAVE) dst[c] = make_uint2(0u, 0u);
+        return;
+    }
+    if (a.unsafe[n]) return;
+    const float g = a.grad[n] * a.inv_t;
+    const float half = __builtin_amdgcn_exp2f(0.5f * (a.xref[j] - a.lse[n] * OI_LOG2E));
     const float sb = -g * half;
-    const float tl = -g * expm1f(logprob[n]);
-    int64_t y = labels[n];
-    y = y < 0 ? 0 : (y >= vocab ? vocab - 1 : y);
-    const float4* src = reinterpret_cast<const float4*>(wsum + j * hdim);
-    const uint2* wy = reinterpret_cast<const uint2*>(W + y * hdim);
-    uint2* dst = reinterpret_cast<uint2*>(d_hidden + n * hdim);
-    for (int64_t c = threadIdx.x; c < hdim / 4; c += blockDim.x) {  // hdim is a multiple of 64
+    const float tl = -g * expm1f(a.logprob[n]);
+    int64_t y = a.labels[n];
+    y = y < 0 ? 0 : (y >= a.vocab ? a.vocab - 1 : y);
+    const float4* src = reinterpret_cast<const float4*>(a.wsum + j * a.hdim);
+    const uint2* wy = reinterpret_cast<const uint2*>(a.W + y * a.hdim);
+#pragma unroll 8
+    for (int64_t c = lane; c < a.hdim / 4; c += OI_WAVE) {  // hdim is a multiple of 64
         const float4 o = src[c];
         const uint2 w = wy[c];
         const float r0 = o.x * half * sb + tl * oi_bf16lo_to_f32(w.x), r1 = o.y * half * sb + tl * oi_bf16hi_to_f32(w.x);
         const float r2 = o.z * half * sb + tl * oi_bf16lo_to_f32(w.y), r3 = o.w * half * sb + tl * oi_bf16hi_to_f32(w.y);
         dst[c] = make_uint2(oi_pack_bf16x2(r0, r1), oi_pack_bf16x2(r2, r3));
     }
+}
+__global__ void __launch_bounds__(AT_ONCE_THREADS)
+    dh_from_wsum_kernel(const uint8_t* __restrict__ mask, int64_t n, int per_wave, WsumInputs a) {
+    for_selected_rows(
+        mask, n, per_wave, [&](int64_t row, bool selected, int64_t j) { dh_row_from_wsum(a, row, selected, j); }, [](int) {});
+}
+// the same by a row index, for more rows than are counted at once
+__global__ void __launch_bounds__(AT_ONCE_THREADS)
+    dh_from_wsum_rows_kernel(const int32_t* __restrict__ rows, const int32_t* __restrict__ count, WsumInputs a) {
+    const int64_t j = (int64_t)blockIdx.x * AT_ONCE_WAVES + (threadIdx.x >> 6);
+    if (j < *count) dh_row_from_wsum(a, rows[j], true, j);
 }
 
 // The recomputing backward.  Per vocabulary chunk: dZ [n_pad, cols] (token-major, bf16, zero in padded
@@ -3152,10 +3320,16 @@ extern "C" int oi_lmhead_logp_fwd_wsum(const void* hidden, const void* weight, c
     if (!select_clears_queues)
         hipLaunchKernelGGL(zero_words_kernel, dim3((unsigned)((n_queue_words + 255) / 256)), dim3(256), 0, s, queues,
                            n_queue_words);
-    if (row_mask)
+    if (row_mask) {
+        const SelectionExtras extra = {weight, vocab, inv_temperature * OI_LOG2E, xref, unsafe, nullptr};
         in = launch_selection(p.sel, ws, hidden, labels, nullptr, nullptr, row_mask, false, n_tokens, hidden_dim, queues,
-                              select_clears_queues ? n_queue_words : 0, s);
-    hipLaunchKernelGGL(zero_bytes_kernel, dim3((unsigned)((n_tokens + 255) / 256)), dim3(256), 0, s, unsafe, n_tokens);
+                              select_clears_queues ? n_queue_words : 0, s, nullptr, extra);
+    } else {
+        hipLaunchKernelGGL(zero_bytes_kernel, dim3((unsigned)((n_tokens + 255) / 256)), dim3(256), 0, s, unsafe, n_tokens);
+        hipLaunchKernelGGL(label_ref_kernel, dim3((unsigned)((n_tokens + 3) / 4)), dim3(256), 0, s, in.hidden,
+                           static_cast<const uint16_t*>(weight), in.labels, in.n_dev, n_tokens, hidden_dim, vocab,
+                           inv_temperature * OI_LOG2E, xref);
+    }
     enqueue_fwd_wsum(p, ws, in, row_mask, weight, n_tokens, hidden_dim, vocab, inv_temperature, logprob, entropy, lse,
                      wsum, xref, unsafe, s);
     return oi_launch_status();
@@ -3199,21 +3373,22 @@ extern "C" int oi_lmhead_dh_from_wsum(const void* hidden, const void* weight, co
     OI_RETURN_IF(workspace_bytes < p.total, OI_EWORKSPACE);
     hipStream_t s = static_cast<hipStream_t>(stream);
     char* ws = static_cast<char*>(workspace);
-    const int32_t *rows = nullptr, *count = nullptr;
-    if (row_mask) {
-        // the same ascending selection as in the forward pass, rebuilt from the same mask
-        int32_t* r = reinterpret_cast<int32_t*>(ws + p.off_rows);
-        int32_t* c = reinterpret_cast<int32_t*>(ws + p.off_count);
+    // the same ascending selection as in the forward pass, from the same mask
+    const WsumInputs wi = {wsum, xref, unsafe, static_cast<const uint16_t*>(weight), labels, lse, logprob, grad_logprob, hidden_dim,
+                           vocab, inv_temperature, static_cast<uint16_t*>(d_hidden)};
+    if (!row_mask || n_tokens <= SELECT_AT_ONCE) {
+        hipLaunchKernelGGL(dh_from_wsum_kernel, dim3(at_once_grid(n_tokens)), dim3(AT_ONCE_THREADS), 0, s, row_mask, n_tokens,
+                           rows_per_wave(n_tokens), wi);
+    } else {
+        int32_t* rows = reinterpret_cast<int32_t*>(ws + p.off_rows);
+        int32_t* count = reinterpret_cast<int32_t*>(ws + p.off_count);
         hipLaunchKernelGGL(select_rows_kernel, dim3(1), dim3(SELECT_THREADS), 0, s, row_mask,
-                           static_cast<const float*>(nullptr), n_tokens, r, c, static_cast<uint32_t*>(nullptr), 0);
+                           static_cast<const float*>(nullptr), n_tokens, rows, count, static_cast<uint32_t*>(nullptr), 0);
         hipLaunchKernelGGL(zero_unselected_rows_kernel, dim3((unsigned)n_tokens), dim3(256), 0, s, row_mask,
                            static_cast<const float*>(nullptr), hidden_dim, static_cast<uint16_t*>(d_hidden));
-        rows = r;
-        count = c;
+        hipLaunchKernelGGL(dh_from_wsum_rows_kernel, dim3((unsigned)((n_tokens + AT_ONCE_WAVES - 1) / AT_ONCE_WAVES)),
+                           dim3(AT_ONCE_THREADS), 0, s, rows, count, wi);
     }
-    hipLaunchKernelGGL(dh_from_wsum_kernel, dim3((unsigned)n_tokens), dim3(256), 0, s, wsum, xref, unsafe,
-                       static_cast<const uint16_t*>(weight), labels, lse, logprob, grad_logprob, rows, count, n_tokens,
-                       hidden_dim, vocab, inv_temperature, static_cast<uint16_t*>(d_hidden));
     // the flagged rows (a subset of the mask's), recomputed; normally none
     char* ws_rep = ws + p.off_repair;
     uint32_t* rq = reinterpret_cast<uint32_t*>(ws_rep + p.repair.off_queues);
@@ -3254,19 +3429,15 @@ int lmhead_backward(const void* hidden, const void* weight, const int64_t* label
     char* ws = static_cast<char*>(workspace);
     uint32_t* queues = reinterpret_cast<uint32_t*>(ws + p.off_queues);
     const int n_queue_words = (int)(3 * p.n_chunks * QUEUE_WORDS);
-    const float* zero_grad_probe = skip_zero_grad_rows ? grad_logprob : nullptr;
     RowInputs in = {static_cast<const uint16_t*>(hidden), labels, lse, grad_logprob, nullptr, nullptr, logprob};
     const bool select_clears_queues = selecting && n_queue_words <= SELECT_THREADS;
     if (!select_clears_queues)
         hipLaunchKernelGGL(zero_words_kernel, dim3((unsigned)((n_queue_words + 255) / 256)), dim3(256), 0, s, queues,
                            n_queue_words);
-    if (selecting) {
+    if (selecting)
         in = launch_selection(p.sel, ws, hidden, labels, lse, grad_logprob, row_mask, skip_zero_grad_rows != 0, n_tokens,
-                              hidden_dim, queues, select_clears_queues ? n_queue_words : 0, s,
-                              logprob);
-        hipLaunchKernelGGL(zero_unselected_rows_kernel, dim3((unsigned)n_tokens), dim3(256), 0, s, row_mask,
-                           zero_grad_probe, hidden_dim, static_cast<uint16_t*>(d_hidden));
-    }
+                              hidden_dim, queues, select_clears_queues ? n_queue_words : 0, s, logprob,
+                              SelectionExtras{nullptr, 0, 0.f, nullptr, nullptr, d_hidden});
     enqueue_bwd(p, ws, in, weight, n_tokens, hidden_dim, vocab, inv_temperature, d_hidden, d_weight, s, false,
                 0, logits);
     return oi_launch_status();
@@ -3391,7 +3562,8 @@ extern "C" int oi_lmhead_grpo_fwd_bwd(const void* hidden, const void* weight, co
         hipLaunchKernelGGL(zero_words_kernel, dim3((unsigned)((n_queue_words + 255) / 256)), dim3(256), 0, s,
                            bwd_queues, n_queue_words);
     RowInputs in = launch_selection(p.bwd.sel, ws_bwd, hidden, labels, nullptr, nullptr, mask, false, n_tokens,
-                                    hidden_dim, bwd_queues, select_clears_queues ? n_queue_words : 0, s);
+                                    hidden_dim, bwd_queues, select_clears_queues ? n_queue_words : 0, s, nullptr,
+                                    SelectionExtras{nullptr, 0, 0.f, nullptr, nullptr, d_hidden});
     enqueue_fwd(p.fwd, ws_fwd, in, mask, weight, n_tokens, hidden_dim, vocab, inv_temperature, logprob, entropy, lse,
                 KeepPlan{}, s);
 
@@ -3413,8 +3585,6 @@ extern "C" int oi_lmhead_grpo_fwd_bwd(const void* hidden, const void* weight, co
     in.lse = lse_c;
     in.grad = grad_c;
     in.logprob = logprob_c;
-    hipLaunchKernelGGL(zero_unselected_rows_kernel, dim3((unsigned)n_tokens), dim3(256), 0, s, mask,
-                       static_cast<const float*>(nullptr), hidden_dim, static_cast<uint16_t*>(d_hidden));
     enqueue_bwd(p.bwd, ws_bwd, in, weight, n_tokens, hidden_dim, vocab, inv_temperature, d_hidden, d_weight, s);
     return oi_launch_status();
 }

@@ -425,6 +425,35 @@ def test_forward_in_tiles_of_either_height(rows, vocab):
     assert ((dw.grad.float().cpu() - rw.grad).norm() / rw.grad.norm()).item() <= 2e-2
 
 
+@pytest.mark.parametrize("n,shift", [(1, 0), (3, 5), (13, 3), (16384, 1), (16385, 0), (65536, 7), (65537, 0)])
+@pytest.mark.parametrize("want_dw", [True, False])
+def test_rows_selected_by_every_workgroup(n, shift, want_dw):
+    """Row counts on both sides of where the selection changes its split and its route, masks off the 8-byte boundaries
+    that their words are read on; the first and the last row on either side of the selection."""
+    h, v = 64, 256
+    hidden, weight, labels = _case(n, h, v, seed=28, w_scale=3.0 / math.sqrt(h))
+    g = torch.Generator().manual_seed(n + shift)
+    mask = torch.rand(n, generator=g) < 0.5
+    mask[0], mask[-1] = shift % 2 == 0, n % 2 == 1
+    upstream = torch.randn(n, generator=g)
+    placed = torch.ones(n + shift, dtype=torch.bool, device=DEV)
+    placed[shift:] = mask.to(DEV)
+    rh = hidden.float().requires_grad_(True)
+    rw = weight.float().requires_grad_(True)
+    lp_o, _ = o_lm.lm_head_logprobs(rh, rw, labels, 0.9)
+    (lp_o * mask).backward(upstream)
+    dh = hidden.to(DEV).requires_grad_(True)
+    dw = weight.to(DEV).requires_grad_(want_dw)
+    lp, _ = lm_head.fused_lm_head_logprobs(dh, dw, labels.to(DEV), 0.9, mask=placed[shift:])
+    lp.backward(upstream.to(DEV))
+    assert ((lp.detach().cpu() - lp_o.detach()) * mask).abs().max().item() <= TOL
+    assert (lp.detach().cpu()[~mask] == 0).all() and (dh.grad.cpu()[~mask] == 0).all()
+    worst = (dh.grad.float().cpu() - rh.grad).norm(dim=1) / rh.grad.norm(dim=1).clamp(min=1e-30)
+    assert not mask.any() or worst[mask].max().item() <= 2e-2
+    if want_dw:
+        assert (dw.grad.float().cpu() - rw.grad).norm().item() <= 2e-2 * rw.grad.norm().item()
+
+
 def test_row_selection_with_compact_backward_and_mask():
     """Mask and zero-gradient rows together: the backward selects rows that are in the mask AND carry
     a gradient."""
