@@ -11,11 +11,21 @@ import torch
 from . import _lib, model_utils
 
 
+def _launchable(labels: torch.Tensor) -> bool:
+    """Whether the shifting kernel takes them.  Wrapped tensors (vmap, fake tensors and other subclasses) have no address,
+    and a tracer sees tensor operations only."""
+    return (
+        type(labels) is torch.Tensor and labels.is_cuda and labels.dtype == torch.int64 and labels.ndim > 0
+        and 0 < labels.numel() < 2**31 and labels.is_contiguous()
+        and torch._C._functorch.maybe_current_level() is None and not torch.compiler.is_compiling()
+    )  # fmt: skip
+
+
 def shifted_and_kept(
     labels: torch.Tensor, fill: int = -100, ignored: int = -100, want_keep: bool = True
 ) -> tuple[torch.Tensor, torch.Tensor | None]:
     """``labels[..., 1:]`` with ``fill`` in the last position, and which of them are not ``ignored``."""
-    if labels.is_cuda and labels.dtype == torch.int64 and labels.ndim > 0 and labels.numel() > 0 and labels.is_contiguous():
+    if _launchable(labels):
         out = torch.empty_like(labels)
         keep = torch.empty(labels.shape, dtype=torch.bool, device=labels.device) if want_keep else None
         cols = labels.shape[-1]

@@ -157,6 +157,15 @@ def test_shifted_labels(shape, fill, ignored):
     assert padding_free_collator.shifted_and_kept(labels.to(DEV), want_keep=False)[1] is None
 
 
+def test_shifted_labels_of_wrapped_tensors():
+    labels = torch.randint(0, 9, (3, 2, 5), device=DEV)
+    want = torch.full_like(labels, -100)
+    want[..., :-1] = labels[..., 1:]
+    assert torch.equal(torch.vmap(padding_free_collator.shift_labels)(labels), want)
+    with torch._subclasses.FakeTensorMode() as mode:
+        assert padding_free_collator.shift_labels(mode.from_tensor(labels)[0]).shape == (2, 5)
+
+
 # bytes in front of the first 16-byte boundary and behind the last, one workgroup and as many as count for themselves
 @pytest.mark.parametrize("rows,cols,shift", [(1, 1, 0), (1, 1, 3), (3, 5, 0), (3, 17, 1), (2, 1000, 13), (16, 1024, 0), (5, 13109, 7)])
 @pytest.mark.parametrize("axis,denominator", [(None, None), (1, None), (None, 37.5), (1, 37.5)])
