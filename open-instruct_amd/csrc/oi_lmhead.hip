@@ -126,7 +126,8 @@ struct ItemQueue {
         // read the previous one's last value before thread 0 writes this one's first
         __syncthreads();
     }
-    // asks for an id; in flight until settle()
+    // asks for an id.  (The addition waits for the counter.  Left to settle(), with the draw in flight until then, it changes
+    // nothing: steps of 268 and 2400 rows 1.001x, frozen-head DPO of 2950 rows 0.990 to 0.994x.)
     __device__ __forceinline__ void request() {
         if (threadIdx.x == 0 && dry < 8) drawn = draw();
     }
@@ -629,21 +630,25 @@ __device__ __forceinline__ int tile_width(int64_t rows, int64_t row0, bool narro
     if (!narrow || left > 192) return WIDE;
     return left > 128 ? 6 : left > 64 ? 4 : 2;
 }
-// What a call has of token rows: up to one tile (narrow too), tiles of which the last may be narrow, whole tiles.  As a
-// forward kernel, NARROW_LAST is the one that has code for all widths (fwd_tiles).
-enum RowTiles { ONE_TILE, NARROW_LAST, WHOLE_TILES };
+// What a call has of token rows: up to one tile (narrow too), tiles of which the last may be narrow, whole tiles.  As
+// forward kernels, NARROW_LAST and TWO_TILES, of up to two tiles whose exponentials are kept, have code for all widths
+// (fwd_tiles).
+enum RowTiles { ONE_TILE, TWO_TILES, NARROW_LAST, WHOLE_TILES };
 inline RowTiles row_tiles(int64_t rows, int64_t hdim) {
     return rows <= BN ? ONE_TILE : narrow_tiles(rows, hdim) ? NARROW_LAST : WHOLE_TILES;
 }
-// The k-tile at which the product of vocabulary tile vt with ONE_TILE begins.  Such a call reads W once and little else,
-// 128 bytes of 256 rows at a time: with all workgroups at the same k-tile those lie hidden_dim * 2 bytes apart, on few of
-// the memory channels.  So each run of 32 vocabulary tiles, the ones that an XCD works on together and that share
-// hidden's k-tiles in its L2, begins at another eighth (vocabulary 128256, us before and after: 100 rows x 2048 160, 134;
-// 100 x 4096 260, 212; 256 x 4096 311, 247; 256 x 8192 560, 444; 30 x 8192 378, 382).  With more
-// tiles of rows W's k-tiles are shared as well and nothing is gained (300 x 4096 350, 360; 2940 x 4096 2205, 2195), while
-// going round costs 0.4 % (scoring pass of 1432 rows, step of 268).
-__device__ __forceinline__ int first_k_tile(int64_t vt, int64_t hdim) {
-    return __builtin_amdgcn_readfirstlane((int)(vt >> 5 & 7) * (int)(hdim / BK) / 8);
+// The k-tile at which the product of vocabulary tile vt with ONE_TILE or TWO_TILES begins.  Such a call reads W once and
+// little else, 128 bytes of 256 rows at a time: with all workgroups at the same k-tile those lie hidden_dim * 2 bytes
+// apart, on few of the memory channels.  So each run of 2^run vocabulary tiles, the ones that an XCD works on together
+// and that share hidden's k-tiles in its L2, begins at another eighth.  One tile (vocabulary 128256, us before and after):
+// 100 rows x 2048 160, 134; 100 x 4096 260, 212; 256 x 4096 311, 247; 256 x 8192 560, 444; 30 x 8192 378, 382.  Two tiles
+// of 192 rows, whose workgroups keep step: steps of 268 rows (4096 x 100352) 979, 967 and 821, 795 (forward 318, 303), of 300 (8192 x
+// 128256) 2244, 2220, frozen-head DPO of 355 rows (8192 x 128256) 1429, 1404; of 256: 500 rows (3584 x 151665) 1577,
+// 1582.  Scoring passes, whose workgroups take several vocabulary tiles one after the other, lose by it (268 rows,
+// 4096 x 128256: 397, 409).  With more tiles of rows W's k-tiles are shared as well and nothing is gained (4096 x 100352
+// 520 rows 418, 420; 2940 x 4096 2205, 2195), while going round costs 0.4 % (scoring pass of 1432 rows).
+__device__ __forceinline__ int first_k_tile(int64_t vt, int run, int64_t hdim) {
+    return __builtin_amdgcn_readfirstlane((int)(vt >> run & 7) * (int)(hdim / BK) / 8);
 }
 template <class Body>
 __device__ __forceinline__ void with_width(int nj, Body&& body) {
@@ -906,7 +911,9 @@ __device__ __forceinline__ float4 fwd_merge_waves(const float* red, int columns,
     return make_float4(m, s, t, 0.f);
 }
 
-template <FwdKeep KEEP, Walk WALK, int NJ>
+// RUN: of first_k_tile, or none
+constexpr int FROM_ZERO = -1;
+template <FwdKeep KEEP, int RUN, int NJ>
 __device__ __forceinline__ void lmhead_fwd_item(const FwdArgs& a, const FwdLaunch& fl, int64_t split, int64_t tt, int64_t n0,
                                                 uint16_t* lds) {
     const int64_t vocab_tiles = (a.vocab + BM - 1) / BM;
@@ -926,7 +933,8 @@ __device__ __forceinline__ void lmhead_fwd_item(const FwdArgs& a, const FwdLaunc
     for (int j = 0; j < NJ / 2; ++j)
         col[j] = fwd_column(a, KEEP == FWD_EXPONENTIALS ? fl.xref : nullptr, n0 + acc_col<NJ>(wn, j, lane));
 
-    auto start_of = [&](int64_t vt) { return WALK == ROUND ? first_k_tile(vt, a.hdim) : 0; };
+    constexpr Walk WALK = RUN == FROM_ZERO ? NEAR : ROUND;
+    auto start_of = [&](int64_t vt) { return WALK == ROUND ? first_k_tile(vt, RUN, a.hdim) : 0; };
     begin_loads<false, false, NJ, WALK>(rows, tokens, a.hdim, lds, start_of(vt_begin));
     for (int64_t vt = vt_begin; vt < vt_end; ++vt) {
         AccTile<NJ> acc;
@@ -1011,8 +1019,10 @@ __global__ void __launch_bounds__(NTHREADS)
     lmhead_fwd_kernel(FwdArgs a, const int32_t* __restrict__ n_dev, FwdLaunch fl, uint32_t* __restrict__ queue) {
     __shared__ __align__(16) uint16_t lds[LDS_ELEMS];
     if (n_dev) a.n_tokens = device_count(n_dev);  // rows selected on the device: the host only knows an upper bound
+    constexpr bool ALL_WIDTHS = TILES == TWO_TILES || TILES == NARROW_LAST;
+    constexpr int RUN = TILES == ONE_TILE ? 5 : TILES == TWO_TILES ? 4 : FROM_ZERO;
     FwdTiles ft = {BN, (uint32_t)((a.n_tokens + BN - 1) / BN), 0, 0};
-    if (TILES == NARROW_LAST && KEEP != FWD_LOGITS && fl.either)
+    if (ALL_WIDTHS && KEEP != FWD_LOGITS && fl.either)
         ft = fwd_tiles(a.n_tokens, (uint32_t)(fl.n_first * fl.tiles_per_split + fl.n_second), (uint32_t)fl.n_second, fl.narrow);
     // every long item of every XCD's queue is taken before the first short one: the short items are
     // there to fill the end of the launch
@@ -1026,7 +1036,7 @@ __global__ void __launch_bounds__(NTHREADS)
                     [&](uint32_t pid) {
             int64_t split, tt, n0;
             int width = WIDE;
-            if (TILES == NARROW_LAST && pid >= locals * 8) {
+            if (ALL_WIDTHS && pid >= locals * 8) {
                 const uint32_t item = item_of_pid(pid - locals * 8, tail_items);
                 if (item >= tail_items) return;
                 tile_of_item(item, tail, ft.tail_row_tiles, &split, &tt);
@@ -1038,11 +1048,11 @@ __global__ void __launch_bounds__(NTHREADS)
                 if (item >= items) return;
                 tile_of_item(item, head, ft.row_tiles, &split, &tt);
                 n0 = tt * ft.height;
-                if (TILES == NARROW_LAST && ft.height != BN) width = FEWER;
+                if (ALL_WIDTHS && ft.height != BN) width = FEWER;
                 else if (TILES != WHOLE_TILES) width = tile_width(a.n_tokens, n0, fl.narrow);
             }
             auto item = [&](auto nj) {
-                lmhead_fwd_item<KEEP, TILES == ONE_TILE ? ROUND : NEAR, decltype(nj)::value>(a, fl, first + split, tt, n0, lds);
+                lmhead_fwd_item<KEEP, RUN, decltype(nj)::value>(a, fl, first + split, tt, n0, lds);
             };
             if constexpr (TILES != WHOLE_TILES) with_width(width, item);
             else item(std::integral_constant<int, WIDE>{});
@@ -1192,7 +1202,7 @@ __device__ __forceinline__ void lmhead_dz_tile(const uint16_t* __restrict__ W, c
     AccTile<> acc;
     // as the forward, so that the logits are its to the bit
     gemm_tile<WALK>(acc, W, hdim, m0, in.vocab, hidden, hdim, n0, in.n_tokens, hdim, lds,
-                    WALK == ROUND ? first_k_tile(m0 / BM, hdim) : 0);
+                    WALK == ROUND ? first_k_tile(m0 / BM, 5, hdim) : 0);
 
     uint16_t* stage = lds;
 #pragma unroll
@@ -2700,6 +2710,8 @@ __global__ void gather_f32_kernel(const float* __restrict__ lse, const float* __
 
 template <FwdKeep KEEP>
 auto fwd_kernel(int64_t n_tokens, const FwdLaunch& fl) {
+    if constexpr (KEEP == FWD_EXPONENTIALS)
+        if (n_tokens > BN && n_tokens <= 2 * BN) return lmhead_fwd_kernel<KEEP, TWO_TILES>;
     return n_tokens <= BN            ? lmhead_fwd_kernel<KEEP, ONE_TILE>
            : fl.narrow || fl.either ? lmhead_fwd_kernel<KEEP, NARROW_LAST>
                                     : lmhead_fwd_kernel<KEEP, WHOLE_TILES>;

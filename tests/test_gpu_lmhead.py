@@ -425,6 +425,40 @@ def test_forward_in_tiles_of_either_height(rows, vocab):
     assert ((dw.grad.float().cpu() - rw.grad).norm() / rw.grad.norm()).item() <= 2e-2
 
 
+@pytest.mark.parametrize("rows,count", [(257, 257), (400, 384), (400, 385), (512, 512), (512, 256), (300, 3)])
+@pytest.mark.parametrize("h", [192, 576])
+def test_forward_of_two_tiles_begins_along_k(rows, count, h):
+    """Up to two tiles of rows begin at k-tiles that differ from vocabulary tile to vocabulary tile (3 k-tiles: eighths that
+    coincide; 9: none of them at a multiple): equal heights, a narrow last tile, whole tiles, and fewer rows than one tile
+    selected on the device."""
+    vocab = 33100
+    hidden, weight, labels = _case(rows, h, vocab, seed=29, w_scale=3.0 / math.sqrt(h))
+    labels[-1], labels[0] = vocab - 1, 0
+    g = torch.Generator().manual_seed(rows + count)
+    mask = torch.zeros(rows, dtype=torch.bool)
+    mask[torch.randperm(rows, generator=g)[:count]] = True
+    exp_lp, exp_ent = o_lm.lm_head_logprobs(hidden, weight, labels, 0.9, True)
+    with torch.no_grad():
+        lp, ent = lm_head.fused_lm_head_logprobs(
+            hidden.to(DEV), weight.to(DEV), labels.to(DEV), 0.9, return_entropy=True, mask=mask.to(DEV)
+        )
+    assert ((lp.cpu() - exp_lp) * mask).abs().max().item() <= TOL
+    assert ((ent.cpu() - exp_ent) * mask).abs().max().item() <= TOL
+    kept = labels.roll(1).masked_fill(~mask.roll(1), -100)  # the row in front of a label is scored against it
+    kept[0] = -100
+    rh = hidden.float().requires_grad_(True)
+    rw = weight.float().requires_grad_(True)
+    exp = o_lm.linear_cross_entropy(rh[None], rw, kept[None])
+    exp.backward()
+    dh = hidden[None].to(DEV).requires_grad_(True)
+    dw = weight.to(DEV).requires_grad_(True)
+    got = lm_head.fused_linear_cross_entropy(dh, dw, kept[None].to(DEV), token_slabs=True)
+    got.backward()
+    assert abs(got.item() - exp.item()) <= TOL
+    assert (dh.grad[0].float().cpu() - rh.grad).norm().item() <= 2e-2 * rh.grad.norm().item()
+    assert ((dw.grad.float().cpu() - rw.grad).norm() / rw.grad.norm()).item() <= 2e-2
+
+
 @pytest.mark.parametrize("n,shift", [(1, 0), (3, 5), (13, 3), (16384, 1), (16385, 0), (65536, 7), (65537, 0)])
 @pytest.mark.parametrize("want_dw", [True, False])
 def test_rows_selected_by_every_workgroup(n, shift, want_dw):
