@@ -11,13 +11,20 @@ import torch
 from . import _lib, model_utils
 
 
-def _launchable(labels: torch.Tensor) -> bool:
-    """Whether the shifting kernel takes them.  Wrapped tensors (vmap, fake tensors and other subclasses) have no address,
-    and a tracer sees tensor operations only."""
+def _recorded() -> bool:
+    """Whether anyone but the device follows this thread's operations: a tracer, a transform, or a mode (``make_fx``, before
+    dispatch too, runs plain tensors under one).  They see tensor operations, and nothing of a launch."""
     return (
-        type(labels) is torch.Tensor and labels.is_cuda and labels.dtype == torch.int64 and labels.ndim > 0
-        and 0 < labels.numel() < 2**31 and labels.is_contiguous()
-        and torch._C._functorch.maybe_current_level() is None and not torch.compiler.is_compiling()
+        torch.compiler.is_compiling() or torch.jit.is_tracing() or torch._C._functorch.maybe_current_level() is not None
+        or torch._C._len_torch_dispatch_stack() > 0 or torch._C._len_torch_function_stack() > 0
+    )  # fmt: skip
+
+
+def _launchable(labels: torch.Tensor) -> bool:
+    """Whether the shifting kernel takes them.  Wrapped tensors (fake tensors and other subclasses) have no address."""
+    return (
+        not _recorded() and type(labels) is torch.Tensor and labels.is_cuda and labels.dtype == torch.int64
+        and labels.ndim > 0 and 0 < labels.numel() < 2**31 and labels.is_contiguous()
     )  # fmt: skip
 
 

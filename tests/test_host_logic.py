@@ -4,6 +4,7 @@ import contextlib
 
 import pytest
 import torch
+from torch.fx.experimental.proxy_tensor import make_fx
 
 from conftest import make_grpo_config
 from open_instruct_amd import dpo_utils, grpo_utils, model_utils, padding_free_collator, rl_utils
@@ -53,6 +54,28 @@ def test_masked_mean_reshape_rules():
 def test_shift_labels_bit_exact():
     labels = torch.tensor([[5, -100, 7, 9], [1, 2, 3, -100]])
     assert padding_free_collator.shift_labels(labels).tolist() == [[-100, 7, 9, -100], [2, 3, -100, -100]]
+
+
+def test_kernels_are_not_launched_behind_a_tracer():
+    """The label shift launches its kernel only where nothing records the calls around it."""
+    seen = []
+
+    def call(x):
+        seen.append(padding_free_collator._recorded())
+        return x + 1
+
+    x = torch.arange(4)
+    call(x)
+    assert seen == [False]
+    make_fx(call)(x)
+    make_fx(call, pre_dispatch=True)(x)
+    torch.jit.trace(call, (x,), check_trace=False)
+    torch.compile(call, fullgraph=True, backend="eager")(x)
+    torch.vmap(call)(x)
+    torch.func.functionalize(call)(x)
+    assert len(seen) == 7 and all(seen[1:])
+    call(x)
+    assert not seen[-1]
 
 
 def test_packed_concatenated_inputs_offsets():
