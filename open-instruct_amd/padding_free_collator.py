@@ -48,8 +48,9 @@ def shifted_and_kept(
 
 def shift_labels(labels: torch.Tensor) -> torch.Tensor:
     """``out[:, i] = labels[:, i + 1]`` with ``-100`` in the last position (index plumbing, bit-exact)."""
-    if labels.ndim == 2:
-        return shifted_and_kept(labels, want_keep=False)[0]
+    if not torch.jit.is_scripting():  # TorchScript compiles the general way alone
+        if labels.ndim == 2:
+            return shifted_and_kept(labels, want_keep=False)[0]
     out = torch.full_like(labels, -100)
     out[:, :-1] = labels[:, 1:]
     return out

@@ -56,6 +56,11 @@ def test_shift_labels_bit_exact():
     assert padding_free_collator.shift_labels(labels).tolist() == [[-100, 7, 9, -100], [2, 3, -100, -100]]
 
 
+def test_shift_labels_is_scriptable():
+    labels = torch.tensor([[5, -100, 7, 9], [1, 2, 3, -100]])
+    assert torch.jit.script(padding_free_collator.shift_labels)(labels).tolist() == [[-100, 7, 9, -100], [2, 3, -100, -100]]
+
+
 def test_kernels_are_not_launched_behind_a_tracer():
     """The label shift launches its kernel only where nothing records the calls around it."""
     seen = []
