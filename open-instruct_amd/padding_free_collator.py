@@ -21,10 +21,12 @@ def _recorded() -> bool:
 
 
 def _launchable(labels: torch.Tensor) -> bool:
-    """Whether the shifting kernel takes them.  Wrapped tensors (fake tensors and other subclasses) have no address."""
+    """Whether the shifting kernel takes them.  Wrapped tensors (fake tensors and other subclasses) have no address, and a
+    launch goes to the current device whichever device its stream belongs to."""
     return (
         not _recorded() and type(labels) is torch.Tensor and labels.is_cuda and labels.dtype == torch.int64
         and labels.ndim > 0 and 0 < labels.numel() < 2**31 and labels.is_contiguous()
+        and labels.get_device() == torch.cuda.current_device()
     )  # fmt: skip
 
 

@@ -167,6 +167,19 @@ def test_shifted_labels_of_wrapped_tensors():
         assert padding_free_collator.shift_labels(mode.from_tensor(labels)[0]).shape == (2, 5)
 
 
+def test_labels_of_another_device_are_shifted_there(monkeypatch):
+    """With another device current, the kernel would run on that one: tensor operations go where the labels are."""
+    labels = torch.randint(0, 9, (2, 5), device=DEV)
+    launched = []
+    monkeypatch.setattr(_lib, "call", lambda name, *args: launched.append(name))
+    padding_free_collator.shift_labels(labels)
+    assert launched == ["oi_shift_labels"]
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: labels.get_device() + 1)
+    want = torch.full_like(labels, -100)
+    want[:, :-1] = labels[:, 1:]
+    assert torch.equal(padding_free_collator.shift_labels(labels), want) and len(launched) == 1
+
+
 @pytest.mark.parametrize("how", ["make_fx", "make_fx before dispatch", "jit.trace", "compile"])
 def test_shifted_labels_of_a_recorded_call(how):
     """What a tracer recorded on some labels shifts others too."""
