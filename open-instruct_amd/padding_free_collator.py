@@ -30,11 +30,16 @@ def _launchable(labels: torch.Tensor) -> bool:
     )  # fmt: skip
 
 
+def _is_int64(value) -> bool:
+    return type(value) is int and -(2**63) <= value < 2**63
+
+
 def shifted_and_kept(
     labels: torch.Tensor, fill: int = -100, ignored: int = -100, want_keep: bool = True
 ) -> tuple[torch.Tensor, torch.Tensor | None]:
     """``labels[..., 1:]`` with ``fill`` in the last position, and which of them are not ``ignored``."""
-    if _launchable(labels):
+    # tensor operations also take numbers of other kinds (numpy's, floats, 0-dim tensors), and refuse what int64 cannot hold
+    if _is_int64(fill) and _is_int64(ignored) and _launchable(labels):
         out = torch.empty_like(labels)
         keep = torch.empty(labels.shape, dtype=torch.bool, device=labels.device) if want_keep else None
         cols = labels.shape[-1]

@@ -6,6 +6,7 @@ either way); a gradient entry is at most |g| and is rounded once to the logits' 
 2**-22 of it, plus 1e-5 for the fp32 exponential.
 """
 
+import numpy as np
 import pytest
 import torch
 from torch.fx.experimental.proxy_tensor import make_fx
@@ -165,6 +166,15 @@ def test_shifted_labels_of_wrapped_tensors():
     assert torch.equal(torch.vmap(padding_free_collator.shift_labels)(labels), want)
     with torch._subclasses.FakeTensorMode() as mode:
         assert padding_free_collator.shift_labels(mode.from_tensor(labels)[0]).shape == (2, 5)
+
+
+@pytest.mark.parametrize("ignore", [np.int64(-100), -100.0, torch.tensor(-100), True])
+def test_ignored_labels_given_as_other_numbers(ignore):
+    labels = torch.tensor([[5, -100, 7, 1]], device=DEV)
+    out, keep = padding_free_collator.shifted_and_kept(labels, ignore, ignore)
+    assert out.tolist() == [[-100, 7, 1, int(ignore)]] and keep.tolist() == [[v != int(ignore) for v in out[0].tolist()]]
+    with pytest.raises(RuntimeError):
+        padding_free_collator.shifted_and_kept(labels, 2**63, 0)
 
 
 def test_labels_of_another_device_are_shifted_there(monkeypatch):
