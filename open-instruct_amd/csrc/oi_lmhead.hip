@@ -2222,16 +2222,14 @@ __device__ __forceinline__ int rows_before(const uint8_t* __restrict__ mask, int
     return total;
 }
 // each(row, selected, rank among the selected) for the wave's rows; last(count) for the workgroup that has the last row.
-// Without a mask every row is selected.
 template <class Each, class Last>
 __device__ __forceinline__ void for_selected_rows(const uint8_t* __restrict__ mask, int64_t n, int per_wave, Each&& each,
                                                   Last&& last) {
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int of_group = AT_ONCE_WAVES * per_wave;  // at most 64
     const int64_t b = (int64_t)blockIdx.x * of_group;
-    uint64_t set = ~0ull;
-    if (mask) set = __ballot(lane < of_group && b + lane < n && mask[b + lane] != 0);
-    const int before = mask ? rows_before(mask, b) : (int)b;
+    const uint64_t set = __ballot(lane < of_group && b + lane < n && mask[b + lane] != 0);
+    const int before = rows_before(mask, b);
 #pragma unroll 1
     for (int k = 0; k < per_wave; ++k) {
         const int at = wave * per_wave + k;
@@ -2829,8 +2827,8 @@ void enqueue_fwd_wsum(const FwdPlan& p, char* ws, const RowInputs& in, const uin
 }
 
 // d_hidden row of token n from the weighted sum that the forward left behind for it, row j among the selected; zero where it
-// was not selected.  A wave for each row.  The factor s is applied in two halves so that neither leaves the fp32 range.
-// Rows flagged in `unsafe` are left alone (the recomputing backward writes them).
+// was not selected.  THREADS threads for each row.  The factor s is applied in two halves so that neither leaves the fp32
+// range.  Rows flagged in `unsafe` are left alone (the recomputing backward writes them).
 struct WsumInputs {
     const float *wsum, *xref;
     const uint8_t* unsafe;
@@ -2841,11 +2839,13 @@ struct WsumInputs {
     float inv_t;
     uint16_t* d_hidden;
 };
+template <int THREADS>
 __device__ __forceinline__ void dh_row_from_wsum(const WsumInputs& a, int64_t n, bool selected, int64_t j) {
-    const int lane = threadIdx.x & 63;
+    constexpr int UNROLL = 8 * OI_WAVE / THREADS;
+    const int lane = threadIdx.x & (THREADS - 1);
     uint2* dst = reinterpret_cast<uint2*>(a.d_hidden + n * a.hdim);
     if (!selected) {
-        for (int64_t c = lane; c < a.hdim / 4; c += OI_WAVE) dst[c] = make_uint2(0u, 0u);
+        for (int64_t c = lane; c < a.hdim / 4; c += THREADS) dst[c] = make_uint2(0u, 0u);
         return;
     }
     if (a.unsafe[n]) return;
@@ -2857,8 +2857,8 @@ __device__ __forceinline__ void dh_row_from_wsum(const WsumInputs& a, int64_t n,
     y = y < 0 ? 0 : (y >= a.vocab ? a.vocab - 1 : y);
     const float4* src = reinterpret_cast<const float4*>(a.wsum + j * a.hdim);
     const uint2* wy = reinterpret_cast<const uint2*>(a.W + y * a.hdim);
-#pragma unroll 8
-    for (int64_t c = lane; c < a.hdim / 4; c += OI_WAVE) {  // hdim is a multiple of 64
+#pragma unroll UNROLL
+    for (int64_t c = lane; c < a.hdim / 4; c += THREADS) {  // hdim is a multiple of 64
         const float4 o = src[c];
         const uint2 w = wy[c];
         const float r0 = o.x * half * sb + tl * oi_bf16lo_to_f32(w.x), r1 = o.y * half * sb + tl * oi_bf16hi_to_f32(w.x);
@@ -2869,13 +2869,18 @@ __device__ __forceinline__ void dh_row_from_wsum(const WsumInputs& a, int64_t n,
 __global__ void __launch_bounds__(AT_ONCE_THREADS)
     dh_from_wsum_kernel(const uint8_t* __restrict__ mask, int64_t n, int per_wave, WsumInputs a) {
     for_selected_rows(
-        mask, n, per_wave, [&](int64_t row, bool selected, int64_t j) { dh_row_from_wsum(a, row, selected, j); }, [](int) {});
+        mask, n, per_wave, [&](int64_t row, bool selected, int64_t j) { dh_row_from_wsum<OI_WAVE>(a, row, selected, j); }, [](int) {});
 }
-// the same by a row index, for more rows than are counted at once
-__global__ void __launch_bounds__(AT_ONCE_THREADS)
+// The same where there is nothing to count: all rows, or those of a row index where there are more than are counted at once.
+// A workgroup for each row: bytes alone bound it then, and a wave for each row (four in turn past 16384) keeps too few under
+// way.  Backward, us, waves and workgroups: all of 32768 rows x 8192 386, 304; of 32768 x 4096 198, 157; of 65600 x 8192 735,
+// 635; of 65600 rows by an index 762, 727, x 4096 443, 419, of 131072 x 2048 678, 710 (70 % of them 597, 615).
+constexpr int ROW_THREADS = 256;
+__global__ void __launch_bounds__(ROW_THREADS)
     dh_from_wsum_rows_kernel(const int32_t* __restrict__ rows, const int32_t* __restrict__ count, WsumInputs a) {
-    const int64_t j = (int64_t)blockIdx.x * AT_ONCE_WAVES + (threadIdx.x >> 6);
-    if (j < *count) dh_row_from_wsum(a, rows[j], true, j);
+    const int64_t j = blockIdx.x;
+    if (count && j >= *count) return;
+    dh_row_from_wsum<ROW_THREADS>(a, rows ? (int64_t)rows[j] : j, true, j);
 }
 
 // The recomputing backward.  Per vocabulary chunk: dZ [n_pad, cols] (token-major, bf16, zero in padded
@@ -3388,18 +3393,22 @@ extern "C" int oi_lmhead_dh_from_wsum(const void* hidden, const void* weight, co
     // the same ascending selection as in the forward pass, from the same mask
     const WsumInputs wi = {wsum, xref, unsafe, static_cast<const uint16_t*>(weight), labels, lse, logprob, grad_logprob, hidden_dim,
                            vocab, inv_temperature, static_cast<uint16_t*>(d_hidden)};
-    if (!row_mask || n_tokens <= SELECT_AT_ONCE) {
+    if (row_mask && n_tokens <= SELECT_AT_ONCE) {
         hipLaunchKernelGGL(dh_from_wsum_kernel, dim3(at_once_grid(n_tokens)), dim3(AT_ONCE_THREADS), 0, s, row_mask, n_tokens,
                            rows_per_wave(n_tokens), wi);
     } else {
-        int32_t* rows = reinterpret_cast<int32_t*>(ws + p.off_rows);
-        int32_t* count = reinterpret_cast<int32_t*>(ws + p.off_count);
-        hipLaunchKernelGGL(select_rows_kernel, dim3(1), dim3(SELECT_THREADS), 0, s, row_mask,
-                           static_cast<const float*>(nullptr), n_tokens, rows, count, static_cast<uint32_t*>(nullptr), 0);
-        hipLaunchKernelGGL(zero_unselected_rows_kernel, dim3((unsigned)n_tokens), dim3(256), 0, s, row_mask,
-                           static_cast<const float*>(nullptr), hidden_dim, static_cast<uint16_t*>(d_hidden));
-        hipLaunchKernelGGL(dh_from_wsum_rows_kernel, dim3((unsigned)((n_tokens + AT_ONCE_WAVES - 1) / AT_ONCE_WAVES)),
-                           dim3(AT_ONCE_THREADS), 0, s, rows, count, wi);
+        const int32_t *rows = nullptr, *count = nullptr;
+        if (row_mask) {
+            int32_t* r = reinterpret_cast<int32_t*>(ws + p.off_rows);
+            int32_t* c = reinterpret_cast<int32_t*>(ws + p.off_count);
+            hipLaunchKernelGGL(select_rows_kernel, dim3(1), dim3(SELECT_THREADS), 0, s, row_mask,
+                               static_cast<const float*>(nullptr), n_tokens, r, c, static_cast<uint32_t*>(nullptr), 0);
+            hipLaunchKernelGGL(zero_unselected_rows_kernel, dim3((unsigned)n_tokens), dim3(256), 0, s, row_mask,
+                               static_cast<const float*>(nullptr), hidden_dim, static_cast<uint16_t*>(d_hidden));
+            rows = r;
+            count = c;
+        }
+        hipLaunchKernelGGL(dh_from_wsum_rows_kernel, dim3((unsigned)n_tokens), dim3(ROW_THREADS), 0, s, rows, count, wi);
     }
     // the flagged rows (a subset of the mask's), recomputed; normally none
     char* ws_rep = ws + p.off_repair;
