@@ -2190,10 +2190,13 @@ __global__ void __launch_bounds__(256)
 // 6; 2950 rows x 8192, four 48, one 21.
 constexpr int64_t SELECT_AT_ONCE = 65536;
 constexpr int AT_ONCE_WAVES = 4, AT_ONCE_THREADS = AT_ONCE_WAVES * OI_WAVE;
-// rows of a wave: more where there are many workgroups anyway, so that the mask is not read by too many
-inline int rows_per_wave(int64_t n) { return n > 16384 ? 4 : 1; }
-inline unsigned at_once_grid(int64_t n) {
-    const int64_t rows = AT_ONCE_WAVES * rows_per_wave(n);
+// Rows of a wave: more where there are many workgroups anyway, so that the mask is not read by too many, and the more the
+// shorter they are.  Forward with the sum and backward, us, one row, two and four: 24576 rows x 2048 155 77, 150 76, 149 75;
+// 32768 x 4096 346 156, 341 158, 341 171; x 8192 614 281, 624 291, 638 318; 65536 x 2048 342 204, 320 174, 314 168; x 4096
+// 561 308, 544 292, 549 298; x 8192 1037 551, 1038 555, 1055 577.
+inline int rows_per_wave(int64_t n, int64_t hdim) { return n <= 16384 ? 1 : hdim <= 2048 ? 4 : 2; }
+inline unsigned at_once_grid(int64_t n, int64_t hdim) {
+    const int64_t rows = AT_ONCE_WAVES * rows_per_wave(n, hdim);
     return (unsigned)((n + rows - 1) / rows);
 }
 __device__ __forceinline__ int nonzero_bytes(uint64_t x) {
@@ -2671,8 +2674,8 @@ RowInputs launch_selection(const SelectionPlan& sp, char* ws, const void* hidden
                               labels_c, lse_c, grad_c, logprob_c, zero_words, n_zero,
                               static_cast<const uint16_t*>(extra.weight), extra.vocab, extra.c, extra.xref, extra.clear,
                               static_cast<uint16_t*>(extra.zero_rows)};
-        hipLaunchKernelGGL(select_gather_kernel, dim3(at_once_grid(n_tokens)), dim3(AT_ONCE_THREADS), 0, s, row_mask, n_tokens,
-                           rows_per_wave(n_tokens), g);
+        hipLaunchKernelGGL(select_gather_kernel, dim3(at_once_grid(n_tokens, hdim)), dim3(AT_ONCE_THREADS), 0, s, row_mask,
+                           n_tokens, rows_per_wave(n_tokens, hdim), g);
         return in;
     }
     const float* zero_grads = skip_zero_grad ? grad : nullptr;
@@ -3394,8 +3397,8 @@ extern "C" int oi_lmhead_dh_from_wsum(const void* hidden, const void* weight, co
     const WsumInputs wi = {wsum, xref, unsafe, static_cast<const uint16_t*>(weight), labels, lse, logprob, grad_logprob, hidden_dim,
                            vocab, inv_temperature, static_cast<uint16_t*>(d_hidden)};
     if (row_mask && n_tokens <= SELECT_AT_ONCE) {
-        hipLaunchKernelGGL(dh_from_wsum_kernel, dim3(at_once_grid(n_tokens)), dim3(AT_ONCE_THREADS), 0, s, row_mask, n_tokens,
-                           rows_per_wave(n_tokens), wi);
+        hipLaunchKernelGGL(dh_from_wsum_kernel, dim3(at_once_grid(n_tokens, hidden_dim)), dim3(AT_ONCE_THREADS), 0, s,
+                           row_mask, n_tokens, rows_per_wave(n_tokens, hidden_dim), wi);
     } else {
         const int32_t *rows = nullptr, *count = nullptr;
         if (row_mask) {

@@ -464,7 +464,17 @@ def test_forward_of_two_tiles_begins_along_k(rows, count, h):
 def test_rows_selected_by_every_workgroup(n, shift, want_dw):
     """Row counts on both sides of where the selection changes its split and its route, masks off the 8-byte boundaries
     that their words are read on; the first and the last row on either side of the selection."""
-    h, v = 64, 256
+    _check_selected_rows(n, shift, 64, want_dw)
+
+
+@pytest.mark.parametrize("n,shift", [(16384, 3), (16385, 0), (16391, 5)])
+def test_long_rows_selected_by_every_workgroup(n, shift):
+    """Rows of more than 2048 have a split of their own past 16384 of them."""
+    _check_selected_rows(n, shift, 2112, False)
+
+
+def _check_selected_rows(n, shift, h, want_dw):
+    v = 256
     hidden, weight, labels = _case(n, h, v, seed=28, w_scale=3.0 / math.sqrt(h))
     g = torch.Generator().manual_seed(n + shift)
     mask = torch.rand(n, generator=g) < 0.5
