@@ -23,6 +23,7 @@
 #include "oi_common.h"
 #include "oi_grpo_math.h"
 #include "oi_ktiles.h"
+#include "oi_queue.h"
 
 #include <type_traits>
 
@@ -44,34 +45,6 @@ static_assert(256 * STAGE_STRIDE <= LDS_ELEMS, "the dZ staging tile must fit");
 constexpr int WIDE = 8;
 template <int NJ = WIDE>
 using AccTile = f32x4[4][NJ];
-
-// XCD-aware tile order.  Consecutive workgroup ids go round-robin to the 8 XCDs, each with its own
-// L2.  The tiles of a launch are numbered in bands of 8 rows, n outermost inside a band, so that 32
-// consecutive numbers are an 8 (m) x 4 (n) super-tile (wider where there are fewer than 8 rows); the ids
-// of an XCD come in runs of 32 such numbers, which its 32 workgroups share operand slabs of in that L2,
-// and the 8 XCDs take neighbouring runs along n.  The sweep over n completes before m advances: the chip
-// as a whole then works on one slab of A (the larger operand: lm_head rows, dZ rows) at a time, which
-// stays in the memory-side cache while every n tile passes over it, instead of streaming all of A from
-// HBM once per n super-tile.  Measured: +4 to +7 % on every shape of the lm_head path (the kernel runs at
-// the chip's power limit, and HBM traffic costs power).  Every number is a tile, whatever the counts, and the
-// numbers past the last whole 256 are dealt out evenly: runs of 32 would leave whole XCDs to take tiles from
-// the others' queues, out of the runs that share slabs.  d_hidden of 7648 rows (480 tiles, 4096 x 128256): 7.03 ms in
-// runs of 32, 6.61 evenly; scoring pass of 1432 rows 1.258 -> 1.223 ms.  Ids without a number give one >= items.
-__device__ __forceinline__ uint32_t item_of_pid(uint32_t pid, uint32_t items) {
-    const uint32_t xcd = pid & 7, local = pid >> 3, first = (local >> 5) * 256, at = local & 31;
-    const uint32_t left = first < items ? items - first : 0, run = left >= 256 ? 32 : (left + 7) / 8;
-    return at < run ? first + xcd * run + at : 0xffffffffu;
-}
-__device__ __forceinline__ void tile_of_item(uint32_t item, uint32_t tiles_m, uint32_t tiles_n, int64_t* tm, int64_t* tn) {
-    const uint32_t band = item / (8 * tiles_n), in_band = item - band * 8 * tiles_n;
-    const uint32_t left = tiles_m - band * 8, rows = left < 8 ? left : 8;
-    const uint32_t col = in_band / rows;
-    *tm = band * 8 + (in_band - col * rows);
-    *tn = col;
-}
-// number of ids to enumerate (whole runs for every XCD, a multiple of 256), and those of an XCD that may have an item
-__host__ __device__ inline int64_t pids_for_items(int64_t items) { return (items + 255) / 256 * 256; }
-__host__ __device__ inline uint32_t locals_for_items(uint32_t items) { return items / 256 * 32 + (items % 256 + 7) / 8; }
 
 // Work queue.  A launch of the tile kernels is one workgroup per CU (the LDS ring leaves room for
 // no second one) that stays for the whole launch and draws tile ids from a counter, rather than
@@ -106,7 +79,7 @@ struct ItemQueue {
     uint32_t* counters;
     // the word sits in the fifth ring slot, which the main loop first writes after its first barrier
     volatile uint32_t* mailbox;
-    uint32_t items, locals, xcd, begun;
+    uint32_t items, locals, xcd, beginners;
     // thread 0 only: the queues of XCDs xcd .. xcd + dry - 1 (mod 8) are known to be empty, `drawn` came from
     // the queue of XCD xcd + dry, `next` is the id it stands for
     uint32_t dry, drawn, next;
@@ -118,7 +91,7 @@ struct ItemQueue {
           items(items_),
           locals(locals_),  // ids per queue
           xcd(blockIdx.x & 7),
-          begun(begins ? gridDim.x >> 3 : 0),
+          beginners(begins ? gridDim.x : 0),
           dry(counters_ ? 0 : 8),  // without counters there is nothing to draw
           drawn(0),
           next(NONE) {
@@ -131,7 +104,10 @@ struct ItemQueue {
     __device__ __forceinline__ void request() {
         if (threadIdx.x == 0 && dry < 8) drawn = draw();
     }
-    __device__ __forceinline__ uint32_t draw() { return begun + atomicAdd(&counters[(xcd + dry) & 7], 1u); }
+    __device__ __forceinline__ uint32_t draw() {
+        const uint32_t q = (xcd + dry) & 7;
+        return ids_begun(beginners, q) + atomicAdd(&counters[q], 1u);
+    }
     __device__ __forceinline__ void settle() {
         if (threadIdx.x != 0) return;
         next = NONE;
@@ -148,7 +124,7 @@ struct ItemQueue {
             uint32_t with_ids = 8;
 #pragma unroll
             for (int q = 7; q > 0; --q)
-                if ((uint32_t)q > dry && begun + at[q] < locals) with_ids = q;
+                if ((uint32_t)q > dry && ids_begun(beginners, (xcd + q) & 7) + at[q] < locals) with_ids = q;
             dry = with_ids;
             if (dry < 8) drawn = draw();
         }
@@ -2897,7 +2873,7 @@ __global__ void __launch_bounds__(ROW_THREADS)
 // without tokens then changes nothing and costs nothing (the rows must be selected on the device).
 // logits: the forward's logits (kept_bytes), read instead of recomputed.
 // max_grid > 0 caps the number of resident workgroups of every launch (the queues work with any
-// number): the launches that serve flagged rows normally find none, and a launch over a few CUs that
+// number, ids_begun): the launches that serve flagged rows normally find none, and a launch over a few CUs that
 // finds nothing costs a fraction of one over all of them.
 constexpr unsigned REPAIR_GRID = 32;
 void enqueue_bwd(const BwdPlan& p, char* ws, const RowInputs& in, const void* weight, int64_t n_tokens,
