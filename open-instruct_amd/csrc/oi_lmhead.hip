@@ -40,8 +40,9 @@ constexpr int STAGE_STRIDE = 256 + 8;           // bf16 per row of the dZ stagin
 constexpr int LDS_ELEMS = 5 * TILE_ELEMS;       // 163840 B: the five-slot operand ring, all of a CU's LDS
 static_assert(256 * STAGE_STRIDE <= LDS_ELEMS, "the dZ staging tile must fit");
 
-// A workgroup's tile is 256 (m) x 32 NJ (n): each wave 64 x 16 NJ, NJ column tiles.  NJ is 8, or less for the last tile
-// of token rows of a forward pass (tile_width).
+// A workgroup's tile is 256 (m) x 32 NJ (n): each wave 64 x 16 NJ, NJ column tiles.  NJ is 8, or less for token rows: for the
+// last tile of a forward (tile_width), for all tiles of a forward or a d_hidden product of few rows (fwd_tiles, plan_rows:
+// 6) and for a forward's last round (4).
 constexpr int WIDE = 8;
 template <int NJ = WIDE>
 using AccTile = f32x4[4][NJ];
@@ -170,9 +171,9 @@ __device__ __forceinline__ void for_each_id(uint32_t* __restrict__ counters, uin
 }
 template <class Body>
 __device__ __forceinline__ void for_each_tile(uint32_t* __restrict__ counters, int64_t tiles_m, int64_t tiles_n,
-                                              uint16_t* lds, Body&& body, bool begins = true) {
+                                              uint16_t* lds, Body&& body) {
     const uint32_t items = (uint32_t)(tiles_m * tiles_n);
-    for_each_id(counters, locals_for_items(items), lds, begins, [&](uint32_t pid) {
+    for_each_id(counters, locals_for_items(items), lds, true, [&](uint32_t pid) {
         const uint32_t item = item_of_pid(pid, items);
         if (item >= items) return;
         int64_t tm, tn;
@@ -618,11 +619,12 @@ inline RowTiles row_tiles(int64_t rows, int64_t hdim) {
 // apart, on few of the memory channels.  So each run of 2^run vocabulary tiles, the ones that an XCD works on together
 // and that share hidden's k-tiles in its L2, begins at another eighth.  One tile (vocabulary 128256, us before and after):
 // 100 rows x 2048 160, 134; 100 x 4096 260, 212; 256 x 4096 311, 247; 256 x 8192 560, 444; 30 x 8192 378, 382.  Two tiles
-// of 192 rows, whose workgroups keep step: steps of 268 rows (4096 x 100352) 979, 967 and 821, 795 (forward 318, 303), of 300 (8192 x
-// 128256) 2244, 2220, frozen-head DPO of 355 rows (8192 x 128256) 1429, 1404; of 256: 500 rows (3584 x 151665) 1577,
-// 1582.  Scoring passes, whose workgroups take several vocabulary tiles one after the other, lose by it (268 rows,
-// 4096 x 128256: 397, 409).  With more tiles of rows W's k-tiles are shared as well and nothing is gained (4096 x 100352
-// 520 rows 418, 420; 2940 x 4096 2205, 2195), while going round costs 0.4 % (scoring pass of 1432 rows).
+// of 192 rows, whose workgroups keep step: steps of 268 rows (4096 x 100352) 979, 967 and on another card 821, 795 (forward 318,
+// 303), of 300 (8192 x 128256) 2244, 2220, frozen-head DPO of 355 rows (8192 x 128256) 1429, 1404.  Two of 256, steps of 500
+// rows: 4096 x 100352 1231, 1221; 8192 x 128256 2850, 2832; 3584 x 151665 1582, 1584; 2048 x 151936 988, 992.  Scoring passes,
+// whose workgroups take several vocabulary tiles one after the other, lose by it (268 rows, 4096 x 128256: 397, 409).  With
+// more tiles of rows W's k-tiles are shared as well and nothing is gained (4096 x 100352 520 rows 418, 420; 2940 x 4096 2205,
+// 2195), while going round costs 0.4 % (scoring pass of 1432 rows).
 __device__ __forceinline__ int first_k_tile(int64_t vt, int run, int64_t hdim) {
     return __builtin_amdgcn_readfirstlane((int)(vt >> run & 7) * (int)(hdim / BK) / 8);
 }
@@ -963,11 +965,12 @@ struct FwdTiles {
     uint32_t tail, tail_row_tiles;  // the last `tail` of the short splits come in tiles of TAIL_ROWS
 };
 constexpr int FEWER = 6, FEWER_ROWS = 32 * FEWER, TAIL = 4, TAIL_ROWS = 32 * TAIL;
+// what a k-tile of tiles of the widths 8, 6 and less takes, in 32nds of a whole one's time
+constexpr uint32_t WHOLE_COST = 32, FEWER_COST = 26, TAIL_COST = 18;
 __host__ __device__ inline uint32_t fewer_tiles(int64_t rows) { return (uint32_t)((rows + FEWER_ROWS - 1) / FEWER_ROWS); }
 __device__ __forceinline__ FwdTiles fwd_tiles(int64_t rows, uint32_t vocab_tiles, uint32_t short_splits, bool narrow) {
-    // what tiles of the widths 8, 6 and less take, in 32nds of a whole one's time, and what a narrow one among whole
-    // ones costs the others, which read the same k-tiles of W
-    constexpr uint32_t WHOLE_COST = 32, FEWER_COST = 26, TAIL_COST = 18, APART = 8;
+    // what a narrow one among whole ones costs the others, which read the same k-tiles of W
+    constexpr uint32_t APART = 8;
     FwdTiles t = {BN, (uint32_t)((rows + BN - 1) / BN), 0, 0};
     if (t.row_tiles == 0) return t;
     const int last = tile_width(rows, (int64_t)(t.row_tiles - 1) * BN, narrow);
@@ -1176,7 +1179,8 @@ __device__ __forceinline__ void lmhead_dz_tile(const uint16_t* __restrict__ W, c
     const int64_t n0 = tt * BN, m0 = v_begin + vt * BM;
 
     AccTile<> acc;
-    // as the forward, so that the logits are its to the bit
+    // As the forward, so that the logits are its to the bit.  (Not where a step of 257 to 512 rows left exponentials, whose
+    // forward may begin elsewhere along k: for the rows that it flagged the logits are its up to the order of their sums.)
     gemm_tile<WALK>(acc, W, hdim, m0, in.vocab, hidden, hdim, n0, in.n_tokens, hdim, lds,
                     WALK == ROUND ? first_k_tile(m0 / BM, 5, hdim) : 0);
 
@@ -1589,12 +1593,11 @@ __host__ __device__ inline TailSplit plan_tail(uint32_t tiles, uint32_t grid, ui
 
 // Rows products of few rows also come in tiles of 192 rows, all of them: 268 rows are then 384 instead of 512 that are
 // multiplied.  (One narrow tile among wide ones has pieces of another length, falls out of step with those that read the
-// same k-tiles of W, and gains nothing.)  A k-tile of theirs takes 26/32 of a wide one's time, and what takes less by the
-// estimate is chosen, where that leaves all tiles in one round and in pieces.  d_hidden, us in tiles of 256 and of 192:
+// same k-tiles of W, and gains nothing.)  What takes less by the estimate
+// (FEWER_COST) is chosen, where that leaves all tiles in one round and in pieces.  d_hidden, us in tiles of 256 and of 192:
 // 4096 x 100352 268 rows 295, 235; 384 299, 246; 520 448, 365; 1152 743, 735; 8192 x 128256 268 rows 728, 596; 520 1109, 898;
 // 3584 x 151665 268 rows 426, 347; 2048 x 151936 268 rows 266, 211.  Counts in between stay with 256 (4096 x 100352 400
 // rows 294, 600 441).  Kernels of calls with more than 8 tiles of rows have no code for it: their gain would be 6 % at most.
-constexpr uint32_t FEWER_COST = 26;
 struct RowsPlan {
     TailSplit split;
     bool fewer;
@@ -2163,7 +2166,11 @@ __global__ void __launch_bounds__(256)
 // them, a wave for each row.  A launch that only makes the row index, and another one each for what goes by it, take 4.6 us
 // of a busy stream whatever they do, and one workgroup takes 18 us for the index of 32768 rows.  Rows selected, gathered and
 // marked, and those left out cleared: 2 launches, 4 with the reference exponents, before; 435 rows x 4096, four 19 us, one
-// 6; 2950 rows x 8192, four 48, one 21.
+// 6; 2950 rows x 8192, four 48, one 29.
+//
+// The bytes counted grow with the square of the rows, so there is a limit, which is as far as the tests go on both sides; it is
+// not where the two ways meet.  Scores, us, at once and by an index: 65600 rows x 2048 157, 206; x 4096 277, 325; x 8192 522,
+// 575; 131072 x 2048 319, 473; x 4096 549, 717.
 constexpr int64_t SELECT_AT_ONCE = 65536;
 constexpr int AT_ONCE_WAVES = 4, AT_ONCE_THREADS = AT_ONCE_WAVES * OI_WAVE;
 // Rows of a wave: more where there are many workgroups anyway, so that the mask is not read by too many, and the more the
