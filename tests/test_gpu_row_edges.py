@@ -86,9 +86,14 @@ def test_rows_read_through_the_caches_and_past_them(rows, vocab, dtype):
     tol = 1e-5 if dtype == torch.float32 else 2e-3
     assert (lp[some].double() - lp_e).abs().max().item() <= tol and (ent[some].double() - ent_e).abs().max().item() <= tol
     assert ((leaf.grad[some].double() - grad_e).abs() - (grad_e.abs() * STEP[dtype] + 1e-5)).max().item() <= 0
-    # a gradient row sums to 0 up to its rounding: every row was written, none twice
+    # a gradient row sums to 0 up to its rounding
     sums = leaf.grad.float().sum(1).abs()
     assert (sums - upstream.abs() * 2e-2 - 1e-3).max().item() <= 0
+    # every row holds its own: the label's entry, upstream (1 - p), is a number that no other row, zeros or memory of an earlier
+    # call would hold there; p is off by the exponential's 1e-5, the product rounded once
+    at_label = leaf.grad.gather(1, index[:, None])[:, 0].double()
+    want = upstream.double() * -torch.expm1(lp.detach().double())
+    assert ((at_label - want).abs() <= want.abs() * STEP[dtype] + 1e-5 * (1 + upstream.abs())).all()
 
 
 @pytest.mark.parametrize("shift_in,shift_out,pitch_out", [(0, 1, 0), (3, 3, 0), (5, 2, 0), (0, 0, 8), (0, 0, 3)])
@@ -250,3 +255,34 @@ def test_scaling_by_a_device_scalar(dtype, shift):
             bound = exp.abs() * (torch.finfo(dtype).eps / 2 + 2**-24) + 2**-25
             assert ((got.double() - exp).abs() <= (bound if value != 1.0 else 0.0)).all()
             assert torch.equal(got[:shift], x[:shift]) and torch.equal(got[shift + n :], x[shift + n :])
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("shift,shift_second", [(0, 0), (0, 1), (1, 0), (1, 1)])
+def test_scaling_two_tensors_by_a_device_scalar(dtype, shift, shift_second):
+    """Each of the two at the ends of its own pieces, whichever is longer and sets the launch, on and off the alignment of whole
+    vectors, one of them empty (and without an address).  The bound is that of one tensor."""
+    vec, threads = 16 // dtype.itemsize, 3 * torch.cuda.get_device_properties(0).multi_processor_count * 256
+    tag = _lib.DTYPE_TAGS[dtype]
+    long = vec * (2 * threads + 1) + 3
+    for n, n_second in ((1, long), (long, 1), (vec - 1, vec + 1), (vec * threads, vec * threads + 1), (0, 5 * vec + 1), (5 * vec + 1, 0), (0, 0)):
+        print("case scale pair", dtype, shift, shift_second, n, n_second, flush=True)
+        tensors = [(torch.randn(m + 2, device=DEV).to(dtype), m, s) for m, s in ((n, shift), (n_second, shift_second))]
+        for value in (1.0, -0.3):
+            scale = torch.tensor([value], device=DEV)
+            got = [x.clone() for x, _, _ in tensors]
+            at = [y[s:].data_ptr() if m else None for y, (_, m, s) in zip(got, tensors)]
+            _lib.call("oi_scale_pair_by_device_scalar", at[0], n, at[1], n_second, tag, scale.data_ptr(), _lib.stream_of(scale))
+            for y, (x, m, s) in zip(got, tensors):
+                exp = x.double()
+                exp[s : s + m] *= scale.double()
+                bound = exp.abs() * (torch.finfo(dtype).eps / 2 + 2**-24) + 2**-25
+                assert ((y.double() - exp).abs() <= (bound if value != 1.0 else 0.0)).all()
+                assert torch.equal(y[:s], x[:s]) and torch.equal(y[s + m :], x[s + m :])
+
+
+def test_scaling_refuses_what_has_no_address():
+    x, scale = torch.randn(8, device=DEV), torch.ones(1, device=DEV)
+    for args in ((None, 8, x.data_ptr(), 8), (x.data_ptr(), 8, None, 8), (x.data_ptr() + 2, 4, None, 0), (x.data_ptr(), -1, None, 0)):
+        with pytest.raises(_lib.KernelError):
+            _lib.call("oi_scale_pair_by_device_scalar", *args, 0, scale.data_ptr(), _lib.stream_of(x))
