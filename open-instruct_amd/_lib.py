@@ -160,6 +160,9 @@ _current_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
 
 
 def stream_of(t: torch.Tensor) -> int:
+    # the last look at a tensor before its address goes to a kernel: one that a saved-tensor hook left on the host ends here
+    if not t.is_cuda:
+        raise ValueError(f"expected a tensor on a GPU, but got one on {t.device}")
     if _current_stream is None:
         return torch.cuda.current_stream(t.device).cuda_stream
     return _current_stream(t.get_device())

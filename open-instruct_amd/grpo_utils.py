@@ -580,6 +580,7 @@ class _AttachHeadGrads(torch.autograd.Function):
         d_hidden, d_weight = ctx.saved_tensors
         _hand_out_once(ctx)
         g = _lib.f32c(grad_loss.detach()).reshape(1)
+        _lib.require_gpu(d_hidden, d_weight, g)  # a saved-tensor hook may have left them on the host
         # nothing is touched when the device scalar is exactly 1; both are bf16
         _lib.call(
             "oi_scale_pair_by_device_scalar", d_hidden.data_ptr(), d_hidden.numel(), _lib.ptr(d_weight),

@@ -286,3 +286,21 @@ def test_scaling_refuses_what_has_no_address():
     for args in ((None, 8, x.data_ptr(), 8), (x.data_ptr(), 8, None, 8), (x.data_ptr() + 2, 4, None, 0), (x.data_ptr(), -1, None, 0)):
         with pytest.raises(_lib.KernelError):
             _lib.call("oi_scale_pair_by_device_scalar", *args, 0, scale.data_ptr(), _lib.stream_of(x))
+
+
+@pytest.mark.parametrize("left", ["logits", "hidden", "weight"])
+def test_gradients_left_on_the_host_are_refused(left):
+    """Saved-tensor hooks that do not bring a stored gradient back: an error, and no kernel sees the address."""
+    hidden = torch.randn(1, 6, 64, device=DEV).bfloat16().requires_grad_(True)
+    weight = torch.randn(320, 64, device=DEV).bfloat16().requires_grad_(True)
+    logits = torch.randn(1, 6, 320, device=DEV).bfloat16().requires_grad_(True)
+    shape = {"logits": logits, "hidden": hidden, "weight": weight}[left].shape
+    labels, mask = torch.randint(0, 320, (1, 6), device=DEV), torch.ones(1, 6, dtype=torch.bool, device=DEV)
+    cfg = make_grpo_config(loss_fn="dapo", beta=0.0)
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: t.cpu() if t.shape == shape else t, lambda t: t):
+        if left == "logits":
+            loss = grpo_utils.grpo_loss_on_logits(logits, labels, None, None, torch.ones(1, 6, device=DEV), mask, cfg)[0]
+        else:
+            loss = grpo_utils.grpo_loss_on_hidden(hidden, weight, labels, None, None, torch.ones(1, 6, device=DEV), mask, cfg)[0]
+    with pytest.raises((ValueError, RuntimeError), match="GPU"):
+        loss.backward()

@@ -7,7 +7,7 @@ import torch
 from torch.fx.experimental.proxy_tensor import make_fx
 
 from conftest import make_grpo_config
-from open_instruct_amd import dpo_utils, grpo_utils, model_utils, padding_free_collator, rl_utils
+from open_instruct_amd import _lib, dpo_utils, grpo_utils, model_utils, padding_free_collator, rl_utils
 
 
 def test_row_layout_contiguous_and_sliced():
@@ -54,6 +54,12 @@ def test_masked_mean_reshape_rules():
 def test_shift_labels_bit_exact():
     labels = torch.tensor([[5, -100, 7, 9], [1, 2, 3, -100]])
     assert padding_free_collator.shift_labels(labels).tolist() == [[-100, 7, 9, -100], [2, 3, -100, -100]]
+
+
+@pytest.mark.parametrize("device", ["cpu", "meta"])
+def test_no_stream_for_tensors_elsewhere(device):
+    with pytest.raises(ValueError, match=device):
+        _lib.stream_of(torch.zeros(1, device=device))
 
 
 def test_shift_labels_is_scriptable():
