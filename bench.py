@@ -55,14 +55,14 @@ PEAK_BF16_TFLOPS = 2500.0
 MEASURED_TRAFFIC_BYTES = {
     # gemm_store_kernel<true, true>, the d_weight product of one slab (average of the launches with rows: two of them
     # write fp32, the last one bf16): L2 misses of the tiled operand re-reads + the result
-    "c3": 18.31e9 + 1.75e9,
-    "c4": 15.57e9 + 1.44e9,
-    "c5-train-head": 37.24e9 + 3.50e9,
+    "c3": 19.57e9 + 1.75e9,
+    "c4": 16.80e9 + 1.44e9,
+    "c5-train-head": 42.47e9 + 3.50e9,
     # lmhead_fwd_kernel: L2 misses of the tiled operand re-reads (1.24 GB of unique operands at c3) + the partials
-    "c3-recompute": 42.56e9 + 0.05e9,
-    "c4-recompute": 44.25e9 + 0.06e9,
+    "c3-recompute": 41.54e9 + 0.05e9,
+    "c4-recompute": 42.03e9 + 0.06e9,
     # oi_lmhead_logp_fwd_wsum: two launches of lmhead_fwd_kernel and two of gemm_store_kernel<false, true>
-    "c5": 2 * (43.27e9 + 2.98e9) + 2 * (36.25e9 + 0.81e9),
+    "c5": 2 * (40.46e9 + 2.98e9) + 2 * (46.55e9 + 0.81e9),
     # lsg_grpo_fused_kernel: one read of the logits (the row waits on the CU for the gradient pass) + one write of
     # dlogits
     "c2": 16.88e9 + 16.94e9,
