@@ -80,7 +80,7 @@ struct ItemQueue {
     uint32_t* counters;
     // the word sits in the fifth ring slot, which the main loop first writes after its first barrier
     volatile uint32_t* mailbox;
-    uint32_t items, locals, xcd, beginners;
+    uint32_t items, locals, xcd, begun;
     // thread 0 only: the queues of XCDs xcd .. xcd + dry - 1 (mod 8) are known to be empty, `drawn` came from
     // the queue of XCD xcd + dry, `next` is the id it stands for
     uint32_t dry, drawn, next;
@@ -92,7 +92,7 @@ struct ItemQueue {
           items(items_),
           locals(locals_),  // ids per queue
           xcd(blockIdx.x & 7),
-          beginners(begins ? gridDim.x : 0),
+          begun(begins ? ids_begun(gridDim.x) : 0),
           dry(counters_ ? 0 : 8),  // without counters there is nothing to draw
           drawn(0),
           next(NONE) {
@@ -105,10 +105,7 @@ struct ItemQueue {
     __device__ __forceinline__ void request() {
         if (threadIdx.x == 0 && dry < 8) drawn = draw();
     }
-    __device__ __forceinline__ uint32_t draw() {
-        const uint32_t q = (xcd + dry) & 7;
-        return ids_begun(beginners, q) + atomicAdd(&counters[q], 1u);
-    }
+    __device__ __forceinline__ uint32_t draw() { return begun + atomicAdd(&counters[(xcd + dry) & 7], 1u); }
     __device__ __forceinline__ void settle() {
         if (threadIdx.x != 0) return;
         next = NONE;
@@ -125,7 +122,7 @@ struct ItemQueue {
             uint32_t with_ids = 8;
 #pragma unroll
             for (int q = 7; q > 0; --q)
-                if ((uint32_t)q > dry && ids_begun(beginners, (xcd + q) & 7) + at[q] < locals) with_ids = q;
+                if ((uint32_t)q > dry && begun + at[q] < locals) with_ids = q;
             dry = with_ids;
             if (dry < 8) drawn = draw();
         }
@@ -2436,13 +2433,9 @@ struct ProbeScope {
     }
 };
 
-// Workgroups of a queue-driven launch: one per CU of the current device (each takes a whole CU's
-// LDS), a multiple of 8 so that every XCD gets the same number, and no more than there are tiles.
-unsigned resident_grid(int64_t tiles_m, int64_t tiles_n) {
-    const int cus = oi_cu_count();
-    const int64_t grid = (cus + 7) / 8 * 8;
-    const int64_t pids = pids_for_items(tiles_m * tiles_n);
-    return (unsigned)(pids < grid ? pids : grid);
+// Workgroups of a queue-driven launch on the current device
+unsigned resident_grid(int64_t tiles_m, int64_t tiles_n, unsigned per_xcd = 0) {
+    return resident_workgroups(tiles_m * tiles_n, oi_cu_count(), per_xcd);
 }
 
 // Scratch for the pieces of the rows products of a call, as launch_rows_product starts them: at most `row_tiles` x
@@ -2879,18 +2872,14 @@ __global__ void __launch_bounds__(ROW_THREADS)
 // dw_adds: the product is added to the bf16 rows of d_weight that an earlier call wrote, instead of stored there; a call
 // without tokens then changes nothing and costs nothing (the rows must be selected on the device).
 // logits: the forward's logits (kept_bytes), read instead of recomputed.
-// max_grid > 0 caps the number of resident workgroups of every launch (the queues work with any
-// number, ids_begun): the launches that serve flagged rows normally find none, and a launch over a few CUs that
-// finds nothing costs a fraction of one over all of them.
-constexpr unsigned REPAIR_GRID = 32;
+// per_xcd > 0 caps the resident workgroups of every launch on each XCD: the launches that serve flagged rows normally find
+// none, and a launch over a few CUs that finds nothing costs a fraction of one over all of them.
+constexpr unsigned REPAIR_PER_XCD = 4;
 void enqueue_bwd(const BwdPlan& p, char* ws, const RowInputs& in, const void* weight, int64_t n_tokens,
                  int64_t hidden_dim, int64_t vocab, float inv_temperature, void* d_hidden, void* d_weight,
-                 hipStream_t s, bool dw_adds = false, unsigned max_grid = 0,
+                 hipStream_t s, bool dw_adds = false, unsigned per_xcd = 0,
                  const float* logits = nullptr) {
-    auto grid_of = [&](int64_t tiles_m, int64_t tiles_n) {
-        const unsigned g = resident_grid(tiles_m, tiles_n);
-        return dim3(max_grid > 0 && g > max_grid ? max_grid : g);
-    };
+    auto grid_of = [&](int64_t tiles_m, int64_t tiles_n) { return dim3(resident_grid(tiles_m, tiles_n, per_xcd)); };
     uint16_t* dz = reinterpret_cast<uint16_t*>(ws + p.off_dz);
     float* dh32 = reinterpret_cast<float*>(ws + p.off_dh32);
     const Pieces parts = pieces_at(ws + p.off_parts, p.parts_bytes);
@@ -3227,7 +3216,7 @@ int run_slab_passes(const SlabPlan& p, char* ws, const SlabStep& st, hipStream_t
         const RowInputs in = launch_selection(p.repair.sel, ws_rep, st.hidden, st.labels, lse, grad, unsafe, false, n,
                                               hdim, rq, select_clears ? n_words : 0, s, st.logprob);
         enqueue_bwd(p.repair, ws_rep, in, st.weight, n, hdim, vocab, st.inv_temperature, st.d_hidden, st.d_weight, s, true,
-                    REPAIR_GRID);
+                    REPAIR_PER_XCD);
     }
     return oi_launch_status();
 }
@@ -3406,7 +3395,7 @@ extern "C" int oi_lmhead_dh_from_wsum(const void* hidden, const void* weight, co
     const RowInputs in = launch_selection(p.repair.sel, ws_rep, hidden, labels, lse, grad_logprob, unsafe, false,
                                           n_tokens, hidden_dim, rq, select_clears ? n_words : 0, s, logprob);
     enqueue_bwd(p.repair, ws_rep, in, weight, n_tokens, hidden_dim, vocab, inv_temperature, d_hidden, nullptr, s, false,
-                REPAIR_GRID);
+                REPAIR_PER_XCD);
     return oi_launch_status();
 }
 

@@ -36,5 +36,15 @@ OI_QUEUE_FN void tile_of_item(uint32_t item, uint32_t tiles_m, uint32_t tiles_n,
 // number of ids to enumerate (whole runs for every XCD, a multiple of 256), and those of an XCD that may have an item
 OI_QUEUE_FN int64_t pids_for_items(int64_t items) { return (items + 255) / 256 * 256; }
 OI_QUEUE_FN uint32_t locals_for_items(uint32_t items) { return items / 256 * 32 + (items % 256 + 7) / 8; }
-// ids of an XCD's queue that the workgroups of a launch begin with, each with that of its own number
-OI_QUEUE_FN uint32_t ids_begun(uint32_t workgroups, uint32_t xcd) { return (workgroups + 7 - xcd) >> 3; }
+// Workgroups of a queue-driven launch on a device of `cus` CUs: one per CU (each takes a whole CU's LDS), at most `per_xcd`
+// (0: any number) on an XCD, no more than there are ids, and always whole eighths, so that every XCD gets the same number.
+inline uint32_t resident_workgroups(int64_t items, int64_t cus, uint32_t per_xcd) {
+    int64_t most = (cus + 7) / 8;
+    if (per_xcd && per_xcd < most) most = per_xcd;
+    const int64_t ids = pids_for_items(items) >> 3;
+    return (uint32_t)((ids < most ? ids : most) * 8);
+}
+// ids of every queue that the workgroups of such a launch begin with, each with that of its own number.  One number for all
+// queues: counted queue by queue, for launches of any number of workgroups, steps and passes of 1400 rows and more take 0.2
+// to 0.4 % longer (22942 rows x 4096 x 128256 53.3 ms, 53.5).
+OI_QUEUE_FN uint32_t ids_begun(uint32_t workgroups) { return workgroups >> 3; }

@@ -1,4 +1,4 @@
-"""Tile ids of the work queues, on the host: whatever the number of workgroups, every tile is handed out once."""
+"""Tile ids of the work queues, on the host: whatever the tiles, the CUs and the cap, every tile is handed out once."""
 
 import os
 import subprocess
@@ -20,7 +20,7 @@ static bool once(uint32_t workgroups, uint32_t items, bool begins) {
     if (begins)
         for (uint32_t b = 0; b < workgroups; ++b) hand_out(b);
     for (uint32_t q = 0; q < 8; ++q)
-        for (uint32_t local = ids_begun(begins ? workgroups : 0, q); local < locals; ++local) hand_out(local * 8 + q);
+        for (uint32_t local = begins ? ids_begun(workgroups) : 0; local < locals; ++local) hand_out(local * 8 + q);
     for (uint32_t i = 0; i < items; ++i)
         if (taken[i] != 1) {
             printf("%u workgroups, %u items, begins %d: item %u taken %d times\n", workgroups, items, (int)begins, i, taken[i]);
@@ -30,8 +30,12 @@ static bool once(uint32_t workgroups, uint32_t items, bool begins) {
 }
 int main() {
     for (uint32_t items = 0; items <= 1100; items = items < 300 ? items + 1 : items + 37)
-        for (uint32_t workgroups = 1; workgroups <= 264; workgroups = workgroups < 40 || workgroups >= 240 ? workgroups + 1 : workgroups + 24)
-            if (!once(workgroups, items, true) || !once(workgroups, items, false)) return 1;
+        for (uint32_t cus = 1; cus <= 310; cus = cus < 40 || cus >= 240 ? cus + 1 : cus + 24)
+            for (uint32_t per_xcd : {0u, 1u, 4u, 64u}) {
+                const uint32_t workgroups = resident_workgroups(items, cus, per_xcd);
+                if ((workgroups == 0) != (items == 0) || (per_xcd && workgroups > per_xcd * 8)) return 2;
+                if (!once(workgroups, items, true) || !once(workgroups, items, false)) return 1;
+            }
     return 0;
 }
 """
