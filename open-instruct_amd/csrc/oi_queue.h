@@ -46,5 +46,5 @@ inline uint32_t resident_workgroups(int64_t items, int64_t cus, uint32_t per_xcd
 }
 // ids of every queue that the workgroups of such a launch begin with, each with that of its own number.  One number for all
 // queues: counted queue by queue, for launches of any number of workgroups, steps and passes of 1400 rows and more take 0.2
-// to 0.4 % longer (22942 rows x 4096 x 128256 53.3 ms, 53.5).
+// to 0.4 % longer (22942 rows x 4096 x 128256 53.10 ms, 53.30).
 OI_QUEUE_FN uint32_t ids_begun(uint32_t workgroups) { return workgroups >> 3; }
